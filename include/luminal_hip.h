@@ -39,6 +39,7 @@ extern "C" {
 #define LMH_F32 0
 #define LMH_F16 1
 #define LMH_BF16 2
+#define LMH_I32 3 /* operands of lmh_map and lmh_matmul only */
 /* out_f32 (a field of both parameter blocks): 0 writes the result in the input element type,
  * 1 writes fp32. A bf16 result carries a rounding error of up to 2^-8 of its magnitude on its
  * own, more than the 2e-3 parity budget of the half-precision configurations, so bf16 callers
@@ -297,6 +298,50 @@ typedef struct lmh_kv_append_params {
   int32_t Hq;
 } lmh_kv_append_params;
 int lmh_kv_append(const lmh_kv_append_params *p);
+
+/* ---- the nodes of a model graph around its attention nodes, so that a whole layer stays on the device ----
+ *
+ * lmh_matmul: MatMul (reference src/Execution.jl:12-90) and Linear (src/NN.jl:11-38), in fp32 whatever the element types,
+ *   c[batch, m, j] = sum_k a[batch, m, k] b[batch, k, j] + bias[j]
+ * for n <= LMH_MATMUL_GROUP independent products in one launch (the projections of a layer). c is contiguous; with
+ * heads > 0 it is [batch M / seq, heads, seq, N / heads] and column h + heads d of row (b, s) lands at [b, h, s, d], the
+ * column-major split of hidden into heads followed by the permute (src/NN.jl:347-353); batch must be 1 then.
+ * c must overlap no operand. */
+#define LMH_MATMUL_GROUP 4
+typedef struct lmh_matmul_params {
+  void *c;
+  const void *a;
+  const void *b;
+  const void *bias;    /* [N], or null */
+  int32_t batch, M, N, K;
+  int64_t a_stride[3]; /* element strides (batch, m, k) */
+  int64_t b_stride[3]; /* element strides (batch, k, column) */
+  int32_t a_dtype, b_dtype, c_dtype, bias_dtype; /* c: LMH_F32 / LMH_F16 / LMH_BF16 */
+  int32_t heads;
+  int32_t seq;
+} lmh_matmul_params;
+int lmh_matmul(const lmh_matmul_params *p, int32_t n, void *stream);
+
+/* lmh_map: Permute, Reshape, Expand and Add (reference src/Execution.jl:207-250) as one affine form,
+ *   out[i0, i1, ...] = a[sum_d i_d a_stride[d]] + b[sum_d i_d b_stride[d]]   (b may be null)
+ * over the index space dims; out is contiguous in it and overlaps no operand. Computed in fp32. */
+#define LMH_MAP_DIMS 8
+typedef struct lmh_map_params {
+  void *out;
+  const void *a;
+  const void *b;
+  int64_t a_stride[8];
+  int64_t b_stride[8];
+  int32_t dims[8];
+  int32_t n_dims;
+  int32_t out_dtype, a_dtype, b_dtype; /* out: LMH_F32 / LMH_F16 / LMH_BF16 */
+} lmh_map_params;
+int lmh_map(const lmh_map_params *p, void *stream);
+
+/* n device-to-device copies in one launch per LMH_COPY_MANY of them (what a compiled graph does with its inputs, reference
+ * src/Compiler.jl:80-96). The ranges must not overlap. */
+#define LMH_COPY_MANY 8
+int lmh_copy_many(void *const *dst, const void *const *src, const size_t *bytes, int32_t n, void *stream);
 
 #ifdef __cplusplus
 }

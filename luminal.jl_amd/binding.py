@@ -11,7 +11,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libluminal_hip.so")
 CALIB_LIB_PATH = os.path.join(HERE, "lib", "libluminal_hip_calib.so")
 
-LMH_F32, LMH_F16, LMH_BF16 = 0, 1, 2
+LMH_F32, LMH_F16, LMH_BF16, LMH_I32 = 0, 1, 2, 3
 HEADMAP_INTERLEAVED, HEADMAP_BLOCKED = 0, 1
 DTYPE_CODES = {"f32": LMH_F32, "f16": LMH_F16, "bf16": LMH_BF16}
 DTYPE_BYTES = {"f32": 4, "f16": 2, "bf16": 2}
@@ -27,7 +27,7 @@ EXPORTS = [
     "lmh_decode_workspace_bytes", "lmh_decode_auto_splits", "lmh_decode_attn", "lmh_flash_attn_plan", "lmh_rope",
     "lmh_kv_append", "lmh_stream_create", "lmh_stream_destroy", "lmh_graph_capture_begin", "lmh_graph_capture_end",
     "lmh_graph_launch", "lmh_graph_destroy", "lmh_static_scratch_bytes", "lmh_decode_static_splits",
-    "lmh_decode_attn_static", "lmh_decode_step_splits", "lmh_decode_step",
+    "lmh_decode_attn_static", "lmh_decode_step_splits", "lmh_decode_step", "lmh_matmul", "lmh_map", "lmh_copy_many",
 ]
 
 
@@ -94,6 +94,26 @@ class KvAppendParams(ctypes.Structure):
         ("q_rope", ctypes.c_void_p), ("Hq", ctypes.c_int32),
     ]
 
+
+class MatmulParams(ctypes.Structure):
+    _fields_ = [
+        ("c", ctypes.c_void_p), ("a", ctypes.c_void_p), ("b", ctypes.c_void_p), ("bias", ctypes.c_void_p),
+        ("batch", ctypes.c_int32), ("M", ctypes.c_int32), ("N", ctypes.c_int32), ("K", ctypes.c_int32),
+        ("a_stride", ctypes.c_int64 * 3), ("b_stride", ctypes.c_int64 * 3),
+        ("a_dtype", ctypes.c_int32), ("b_dtype", ctypes.c_int32), ("c_dtype", ctypes.c_int32), ("bias_dtype", ctypes.c_int32),
+        ("heads", ctypes.c_int32), ("seq", ctypes.c_int32),
+    ]
+
+
+class MapParams(ctypes.Structure):
+    _fields_ = [
+        ("out", ctypes.c_void_p), ("a", ctypes.c_void_p), ("b", ctypes.c_void_p),
+        ("a_stride", ctypes.c_int64 * 8), ("b_stride", ctypes.c_int64 * 8), ("dims", ctypes.c_int32 * 8),
+        ("n_dims", ctypes.c_int32), ("out_dtype", ctypes.c_int32), ("a_dtype", ctypes.c_int32), ("b_dtype", ctypes.c_int32),
+    ]
+
+
+MATMUL_GROUP, MAP_DIMS = 4, 8
 
 # every symbol include/luminal_hip_calib.h declares (libluminal_hip_calib.so: measurement kernels, loaded on demand)
 CALIB_EXPORTS = ["lmh_calib_last_error", "lmh_calib_copy", "lmh_calib_read", "lmh_calib_mfma", "lmh_calib_mfma_xcds",
@@ -162,7 +182,10 @@ def load():
     L.lmh_graph_capture_end.argtypes = [vp, ctypes.POINTER(vp)]
     L.lmh_graph_launch.argtypes = [vp, vp]
     L.lmh_graph_destroy.argtypes = [vp]
-    for name in ("lmh_rope", "lmh_kv_append", "lmh_init", "lmh_device_name", "lmh_malloc", "lmh_free", "lmh_memset", "lmh_memcpy_h2d",
+    L.lmh_matmul.argtypes = [ctypes.POINTER(MatmulParams), ctypes.c_int32, vp]
+    L.lmh_map.argtypes = [ctypes.POINTER(MapParams), vp]
+    L.lmh_copy_many.argtypes = [ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(ctypes.c_size_t), ctypes.c_int32, vp]
+    for name in ("lmh_matmul", "lmh_map", "lmh_copy_many", "lmh_rope", "lmh_kv_append", "lmh_init", "lmh_device_name", "lmh_malloc", "lmh_free", "lmh_memset", "lmh_memcpy_h2d",
                  "lmh_memcpy_d2h", "lmh_memcpy_d2d", "lmh_sync", "lmh_event_create", "lmh_event_destroy",
                  "lmh_event_record", "lmh_event_elapsed_ms", "lmh_flash_attn_fwd", "lmh_decode_attn"):
         getattr(L, name).restype = ctypes.c_int
@@ -304,6 +327,20 @@ def rope(params):
 
 def kv_append(params):
     check(load().lmh_kv_append(ctypes.byref(params)))
+
+
+def matmul(params, n, stream=None):
+    """lmh_matmul of the first n elements of a MatmulParams array."""
+    check(load().lmh_matmul(params, n, stream))
+
+
+def map_op(params, stream=None):
+    check(load().lmh_map(ctypes.byref(params), stream))
+
+
+def copy_many(dst, src, nbytes, n, stream=None):
+    """lmh_copy_many of n ranges; dst, src and nbytes are ctypes arrays."""
+    check(load().lmh_copy_many(dst, src, nbytes, n, stream))
 
 
 def stream_create():

@@ -667,4 +667,81 @@ int lmh_kv_append(const lmh_kv_append_params *p) {
   return launch_kv_append(a, p->dtype, (hipStream_t)p->stream);
 }
 
+// --------------------------------------------------------------------------------------------
+// the nodes around attention
+// --------------------------------------------------------------------------------------------
+static bool graph_dtype(int d) { return d == LMH_F32 || d == LMH_F16 || d == LMH_BF16 || d == LMH_I32; }
+
+int lmh_matmul(const lmh_matmul_params *ps, int32_t n, void *stream) {
+  static_assert(LMH_MATMUL_GROUP == kMatmulGroup, "header and kernel agree");
+  if (!ps) return fail(LMH_E_NULL, "lmh_matmul: null params");
+  if (n < 1 || n > LMH_MATMUL_GROUP) return fail(LMH_E_SHAPE, "lmh_matmul: %d products, 1 to %d fit a launch", n, LMH_MATMUL_GROUP);
+  MatmulArgs args = {};
+  for (int i = 0; i < n; i++) {
+    const lmh_matmul_params &p = ps[i];
+    if (!p.c || !p.a || !p.b) return fail(LMH_E_NULL, "lmh_matmul: null tensor pointer");
+    if (p.batch <= 0 || p.M <= 0 || p.N <= 0 || p.K <= 0)
+      return fail(LMH_E_SHAPE, "lmh_matmul: non-positive dimension (batch=%d M=%d N=%d K=%d)", p.batch, p.M, p.N, p.K);
+    if (!graph_dtype(p.a_dtype) || !graph_dtype(p.b_dtype) || !graph_dtype(p.c_dtype) || p.c_dtype == LMH_I32 ||
+        (p.bias && !graph_dtype(p.bias_dtype)))
+      return fail(LMH_E_UNSUPPORTED, "lmh_matmul: unknown element type");
+    for (int d = 0; d < 3; d++)
+      if (p.a_stride[d] < 0 || p.b_stride[d] < 0) return fail(LMH_E_SHAPE, "lmh_matmul: negative stride");
+    if (p.heads < 0 || (p.heads > 0 && (p.batch != 1 || p.seq <= 0 || p.M % p.seq != 0 || p.N % p.heads != 0)))
+      return fail(LMH_E_SHAPE, "lmh_matmul: %d heads of %d rows do not divide c (batch=%d M=%d N=%d)", p.heads, p.seq, p.batch, p.M, p.N);
+    MatmulProblem &q = args.p[i];
+    q.c = p.c; q.a = p.a; q.b = p.b; q.bias = p.bias;
+    q.batch = p.batch; q.M = p.M; q.N = p.N; q.K = p.K;
+    for (int d = 0; d < 3; d++) { q.as[d] = p.a_stride[d]; q.bs[d] = p.b_stride[d]; }
+    q.a_dtype = p.a_dtype; q.b_dtype = p.b_dtype; q.c_dtype = p.c_dtype; q.bias_dtype = p.bias_dtype;
+    q.heads = p.heads; q.seq = p.heads ? p.seq : 1;
+    // 16-byte chunks along the contraction, addressed with 32-bit byte offsets inside a tile of 64 rows of a / inside b
+    constexpr int64_t kMaxBytes = 0x7ffffff0;
+    q.a_vec = p.a_dtype == LMH_F32 && p.a_stride[2] == 1 && p.K % 4 == 0 && p.a_stride[0] % 4 == 0 && p.a_stride[1] % 4 == 0 && aligned16(p.a) &&
+              (64 * p.a_stride[1] + p.K) * 4 < kMaxBytes;
+    q.b_vec = p.b_dtype == LMH_F32 && p.b_stride[1] == 1 && p.K % 4 == 0 && p.b_stride[0] % 4 == 0 && p.b_stride[2] % 4 == 0 && aligned16(p.b) &&
+              ((int64_t)p.N * p.b_stride[2] + p.K) * 4 < kMaxBytes;
+    q.b_by_column = !q.b_vec && p.b_stride[2] == 1 && p.b_stride[1] != 1;
+  }
+  return launch_matmul(args, n, (hipStream_t)stream);
+}
+
+int lmh_map(const lmh_map_params *p, void *stream) {
+  static_assert(LMH_MAP_DIMS == kMapDims, "header and kernel agree");
+  if (!p) return fail(LMH_E_NULL, "lmh_map: null params");
+  if (!p->out || !p->a) return fail(LMH_E_NULL, "lmh_map: null tensor pointer");
+  if (p->n_dims < 1 || p->n_dims > LMH_MAP_DIMS) return fail(LMH_E_SHAPE, "lmh_map: %d dimensions, 1 to %d are taken", p->n_dims, LMH_MAP_DIMS);
+  if (!graph_dtype(p->out_dtype) || p->out_dtype == LMH_I32 || !graph_dtype(p->a_dtype) || (p->b && !graph_dtype(p->b_dtype)))
+    return fail(LMH_E_UNSUPPORTED, "lmh_map: unknown element type");
+  MapArgs a = {};
+  a.out = p->out; a.a = p->a; a.b = p->b;
+  a.n_dims = p->n_dims;
+  a.out_dtype = p->out_dtype; a.a_dtype = p->a_dtype; a.b_dtype = p->b_dtype;
+  for (int d = 0; d < p->n_dims; d++) {
+    if (p->dims[d] <= 0) return fail(LMH_E_SHAPE, "lmh_map: non-positive dimension");
+    if (p->a_stride[d] < 0 || (p->b && p->b_stride[d] < 0)) return fail(LMH_E_SHAPE, "lmh_map: negative stride");
+    a.dims[d] = p->dims[d];
+    a.as[d] = p->a_stride[d];
+    a.bs[d] = p->b ? p->b_stride[d] : 0;
+  }
+  return launch_map(a, (hipStream_t)stream);
+}
+
+int lmh_copy_many(void *const *dst, const void *const *src, const size_t *bytes, int32_t n, void *stream) {
+  static_assert(LMH_COPY_MANY == kCopyMany, "header and kernel agree");
+  if (n < 0) return fail(LMH_E_SHAPE, "lmh_copy_many: negative count");
+  if (n > 0 && (!dst || !src || !bytes)) return fail(LMH_E_NULL, "lmh_copy_many: null list");
+  for (int32_t first = 0; first < n; first += LMH_COPY_MANY) {
+    CopyManyArgs a = {};
+    const int m = n - first < LMH_COPY_MANY ? n - first : LMH_COPY_MANY;
+    for (int i = 0; i < m; i++) {
+      if (bytes[first + i] && (!dst[first + i] || !src[first + i])) return fail(LMH_E_NULL, "lmh_copy_many: null pointer");
+      a.dst[i] = dst[first + i]; a.src[i] = src[first + i]; a.bytes[i] = (int64_t)bytes[first + i];
+    }
+    const int rc = launch_copy_many(a, m, (hipStream_t)stream);
+    if (rc != LMH_OK) return rc;
+  }
+  return LMH_OK;
+}
+
 }  // extern "C"

@@ -97,6 +97,43 @@ struct KvAppendArgs {
   int32_t Hq;
 };
 
+// Matrix products of one launch (matmul.hip): c[batch, m, j] = sum_k a[batch, m, k] b[batch, k, j] (+ bias[j]).
+constexpr int kMatmulGroup = 4;
+struct MatmulProblem {
+  void *c;
+  const void *a, *b, *bias;  // bias: [N] or null
+  int64_t as[3], bs[3];      // element strides (batch, m, k) and (batch, k, column)
+  int32_t batch, M, N, K;
+  int32_t a_dtype, b_dtype, c_dtype, bias_dtype;
+  int32_t heads, seq;        // heads > 0: c is [M / seq, heads, seq, N / heads], column h + heads d of row (b, s) at [b, h, s, d]
+  int32_t a_vec, b_vec;      // 16-byte loads along the contraction
+  int32_t b_by_column;       // b is contiguous along its columns: neighbouring threads take neighbouring columns
+};
+struct MatmulArgs {
+  MatmulProblem p[kMatmulGroup];
+  int32_t first_tile[kMatmulGroup];
+  int32_t n_tiles;
+};
+
+// out[i] = a[i . as] (+ b[i . bs]) over the index space dims; out is contiguous (map_ops.hip).
+constexpr int kMapDims = 8;
+struct MapArgs {
+  void *out;
+  const void *a, *b;
+  int64_t as[kMapDims], bs[kMapDims];
+  int32_t dims[kMapDims];
+  int32_t n_dims, out_dtype, a_dtype, b_dtype;
+  int32_t tile_dim;
+};
+
+constexpr int kCopyMany = 8;
+struct CopyManyArgs {
+  void *dst[kCopyMany];
+  const void *src[kCopyMany];
+  int64_t bytes[kCopyMany];
+  int32_t first_block[kCopyMany];
+};
+
 // Every field of a launch-argument block, requested from memory in one batch at the kernel's start (a kernel calls this first).
 // Left to the compiler, the scalar loads of these 100 to 230 byte blocks are issued where their values are first needed: in the
 // attention kernels five and more round trips to memory, one after the other, before a wave has issued its first tile load
@@ -149,6 +186,9 @@ int launch_prefill_valu(const PrefillArgs &a, int dtype, hipStream_t stream);
 int launch_decode(const DecodeArgs &a, int dtype, hipStream_t stream);
 int launch_rope(const RopeArgs &a, int dtype, hipStream_t stream);
 int launch_kv_append(const KvAppendArgs &a, int dtype, hipStream_t stream);
+int launch_matmul(MatmulArgs &args, int n, hipStream_t stream);
+int launch_map(MapArgs &a, hipStream_t stream);
+int launch_copy_many(CopyManyArgs &a, int n, hipStream_t stream);
 bool decode_mfma_supported(int dtype, int D, int B);
 bool decode_mfma_rope_ok(int D, int interleaved);
 int launch_decode_mfma_split(const DecodeArgs &a, int dtype, hipStream_t stream);

@@ -1,0 +1,315 @@
+// The matrix products of a model graph's projections in fp32 on the gfx950 matrix cores (v_mfma_f32_32x32x2_f32):
+// c = a b (+ bias), batched, up to kMatmulGroup products in one launch. Semantics: batch_matmul of the reference
+// (src/Execution.jl:12-90) and its Linear layer (src/NN.jl:11-38); operands of any element type are taken to fp32 as they
+// are loaded, sums are fp32, the result is rounded once to c's type.
+//
+// Bound: the fp32 matrix pipe (157 TFLOP/s, 64 flops per cycle and SIMD). A wave owns a 32 x 32 block of c: one 128-bit
+// LDS read of each operand feeds four MFMAs of 64 cycles, so LDS (two reads, 16 of 256 cycles) and the vector ALUs are idle
+// most of the time and what decides is how evenly the blocks fall on the 1024 SIMDs:
+//   * a workgroup is WM x WN blocks, and WK waves share a block by taking every WK-th 32 elements of the contraction
+//     (folded through LDS at the end): the launcher takes the form whose last round is fullest (launch_matmul below);
+//   * several products that run at the same time in a model (the q, k and v projections of a layer, which share a) go into
+//     one launch, so their rounds are filled together;
+//   * blockIdx -> tile hands every XCD a contiguous range of tiles, rows of c fastest: its L2 holds a slice of b's columns.
+// Tiles of 32 contraction elements go to double-buffered LDS rows of eight 16-byte chunks; chunk j of row r lies at
+// j ^ (r & 7), which spreads the eight rows that a fragment read's quarter-wave touches over all banks without padding.
+// fp32 operands that are contiguous along the contraction (VEC) are fetched with buffer loads that write straight into LDS,
+// each lane asking for the chunk whose swizzled place it fills; everything else passes through registers, where any element
+// type and layout becomes fp32.
+// The contraction runs in the order 8 j + e, 8 j + 4 + e (e = 0..3): the MFMA takes its two elements from the two halves
+// of the wave, which read neighbouring chunks.
+#include <limits.h>
+
+#include "common.hpp"
+#include "dtypes.hpp"
+
+namespace lmh {
+namespace {
+
+constexpr int BK = 32;  // contraction elements a wave takes per staged tile
+// Byte offset no operand reaches (the host routes larger ones to the other form): a buffer load there returns zeros.
+constexpr int kOutOfRange = 0x7ffffff0;
+
+__device__ inline float load_as_f32(const void *p, int64_t i, int dtype) {
+  switch (dtype) {
+    case LMH_F16: return (float)reinterpret_cast<const _Float16 *>(p)[i];
+    case LMH_BF16: return bf16_bits_to_f32(reinterpret_cast<const uint16_t *>(p)[i]);
+    case LMH_I32: return (float)reinterpret_cast<const int32_t *>(p)[i];
+    default: return reinterpret_cast<const float *>(p)[i];
+  }
+}
+// VEC: every operand is fp32, contiguous along the contraction and 16-byte aligned, K a multiple of 4.
+template <int WM, int WN, int WK, bool VEC>
+__global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(MatmulArgs args) {
+  constexpr int NT = 64 * WM * WN * WK;
+  constexpr int BM = 32 * WM, BN = 32 * WN, BKT = BK * WK;
+  constexpr int CA = BM * BKT / 4, CB = BN * BKT / 4;  // 16-byte chunks of a tile
+  constexpr int RA = CA / NT, RB = CB / NT;
+  static_assert(CA % NT == 0 && CB % NT == 0, "whole chunks per thread");
+  __shared__ __attribute__((aligned(16))) float As[2][BM * BKT];
+  __shared__ __attribute__((aligned(16))) float Bs[2][BN * BKT];
+
+  // ---- which tile of which product ----
+  const int per_xcd = (args.n_tiles + 7) / 8;
+  int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || t >= args.n_tiles) return;
+  int g = 0;
+#pragma unroll
+  for (int i = 1; i < kMatmulGroup; i++)
+    if (t >= args.first_tile[i]) g = i;
+  const MatmulProblem p = args.p[g];
+  t -= args.first_tile[g];
+  const int m_tiles = (p.M + BM - 1) / BM;
+  const int tm = t % m_tiles;
+  t /= m_tiles;
+  const int n_tiles = (p.N + BN - 1) / BN;
+  const int tn = t % n_tiles, batch = t / n_tiles;
+  const int m0 = tm * BM, n0 = tn * BN;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int n = lane & 31, h = lane >> 5;
+  const int wk = wave / (WM * WN), wm = (wave % (WM * WN)) / WN, wn = wave % WN;
+
+  // Column j of c is column `col` of b: the same, or, where c is split into heads, column h + heads * d for j = h D + d
+  // (the reference's column-major reshape of hidden into (heads, D) makes the head index the fast one).
+  const int D = p.heads ? p.N / p.heads : 1;
+  auto b_col = [&](int j) { return p.heads ? j / D + p.heads * (j % D) : j; };
+
+  floatx16_t acc;
+#pragma unroll
+  for (int i = 0; i < 16; i++) acc[i] = 0.f;
+  const int n_k = (p.K + BKT - 1) / BKT;
+  // Fragments of the wave's block from a staged tile, and their 16 MFMAs. All eight reads are issued first.
+  auto multiply = [&](int buf) {
+    const int arow = 32 * wm + n, brow = 32 * wn + n;
+    const float *Aw = &As[buf][32 * BM * wk], *Bw = &Bs[buf][32 * BN * wk];
+    floatx4_t af[4], bf[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      af[j] = *reinterpret_cast<const floatx4_t *>(&Aw[4 * (arow * 8 + ((2 * j + h) ^ (arow & 7)))]);
+      bf[j] = *reinterpret_cast<const floatx4_t *>(&Bw[4 * (brow * 8 + ((2 * j + h) ^ (brow & 7)))]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[j][e], bf[j][e], acc, 0, 0, 0);
+  };
+
+  if constexpr (VEC) {
+    // A tile of `rows` rows is WK slices of rows / 8 blocks of 1 KB; wave w issues blocks w, w + NW, ... of a, then of b.
+    typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) void lds_void_t;
+    constexpr int NW = WM * WN * WK;
+    constexpr int KA = BM * WK / 8 / NW, KB = BN * WK / 8 / NW;  // blocks per wave
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    auto make_desc = [](const float *base, int64_t elements) {
+      const uint64_t q = (uint64_t)base;
+      i32x4_t d;
+      d[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)q);
+      d[1] = __builtin_amdgcn_readfirstlane((int)((q >> 32) & 0xffff));  // stride 0: raw buffer
+      d[2] = __builtin_amdgcn_readfirstlane((int)(elements * 4));
+      d[3] = 0x00020000;
+      return d;
+    };
+    const i32x4_t a_desc = make_desc(reinterpret_cast<const float *>(p.a) + batch * p.as[0] + m0 * p.as[1], (min(p.M - m0, BM) - 1) * p.as[1] + p.K);
+    const i32x4_t b_desc = make_desc(reinterpret_cast<const float *>(p.b) + batch * p.bs[0], (int64_t)(p.N - 1) * p.bs[2] + p.K);
+    int a_voff[KA], b_voff[KB], a_k[KA], b_k[KB];  // byte offset of the lane's chunk in k-tile 0; its first k
+#pragma unroll
+    for (int j = 0; j < KA; j++) {
+      const int q = wave + NW * j, row = (q % (BM / 8)) * 8 + (lane >> 3);
+      a_k[j] = (q / (BM / 8)) * BK + 4 * ((lane & 7) ^ (row & 7));
+      a_voff[j] = m0 + row < p.M ? (int)((row * p.as[1] + a_k[j]) * 4) : kOutOfRange;
+    }
+#pragma unroll
+    for (int j = 0; j < KB; j++) {
+      const int q = wave + NW * j, row = (q % (BN / 8)) * 8 + (lane >> 3);
+      b_k[j] = (q / (BN / 8)) * BK + 4 * ((lane & 7) ^ (row & 7));
+      b_voff[j] = n0 + row < p.N ? (int)((b_col(n0 + row) * p.bs[2] + b_k[j]) * 4) : kOutOfRange;
+    }
+    const uint32_t a_lds = (uint32_t)(uintptr_t)(lds_void_t *)&As[0][0] + wave_u * 1024;
+    const uint32_t b_lds = (uint32_t)(uintptr_t)(lds_void_t *)&Bs[0][0] + wave_u * 1024;
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is a reserved register; it is only written here
+    // (in asm for the reason prefill_mfma.hip gives: the compiler would wait for the load before the next LDS read)
+    auto load_block = [](i32x4_t desc, uint32_t lds_addr, int voff, int soff) {
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                   :: "s"(lds_addr), "v"(voff), "s"(desc), "s"(soff) : "memory", "m0");
+    };
+#pragma clang diagnostic pop
+    auto load_tile = [&](int kt) {
+      const int buf = kt & 1, k0 = kt * BKT;
+      const bool tail = k0 + BKT > p.K;  // chunks past the contraction's end are fetched out of range: zeros
+#pragma unroll
+      for (int j = 0; j < KA; j++)
+        load_block(a_desc, a_lds + buf * (BM * BKT * 4) + j * (NW * 1024), tail && k0 + a_k[j] >= p.K ? kOutOfRange : a_voff[j], k0 * 4);
+#pragma unroll
+      for (int j = 0; j < KB; j++)
+        load_block(b_desc, b_lds + buf * (BN * BKT * 4) + j * (NW * 1024), tail && k0 + b_k[j] >= p.K ? kOutOfRange : b_voff[j], k0 * 4);
+    };
+    load_tile(0);
+    for (int kt = 0; kt < n_k; kt++) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's blocks of tile kt are in LDS
+      __syncthreads();  // ... and everyone's; tile kt - 1 has been consumed, its buffer is free
+      if (kt + 1 < n_k) load_tile(kt + 1);  // in flight while tile kt is multiplied
+      multiply(kt & 1);
+    }
+  } else {
+    // chunk ch of a tile = row ch / (8 WK), 16-byte chunk ch % (8 WK) of it; where b is contiguous along its columns,
+    // neighbouring threads take neighbouring columns instead
+    const bool b_by_column = p.b_by_column;
+    int64_t a_off[RA], b_off[RB];  // negative: a row past the operand's end
+#pragma unroll
+    for (int r = 0; r < RA; r++) {
+      const int m = m0 + (tid + r * NT) / (8 * WK);
+      a_off[r] = m < p.M ? batch * p.as[0] + m * p.as[1] : -1;
+    }
+#pragma unroll
+    for (int r = 0; r < RB; r++) {
+      const int j = n0 + (b_by_column ? (tid + r * NT) % BN : (tid + r * NT) / (8 * WK));
+      b_off[r] = j < p.N ? batch * p.bs[0] + b_col(j) * p.bs[2] : -1;
+    }
+    floatx4_t a_reg[RA], b_reg[RB];
+    auto fetch = [&](const void *base, int dtype, int64_t off, int64_t ks, int k) {
+      floatx4_t x = {0.f, 0.f, 0.f, 0.f};
+      if (off < 0) return x;
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (k + e < p.K) x[e] = load_as_f32(base, off + (k + e) * ks, dtype);
+      return x;
+    };
+    auto load_tile = [&](int k0) {
+#pragma unroll
+      for (int r = 0; r < RA; r++) a_reg[r] = fetch(p.a, p.a_dtype, a_off[r], p.as[2], k0 + 4 * ((tid + r * NT) % (8 * WK)));
+#pragma unroll
+      for (int r = 0; r < RB; r++) {
+        const int c = b_by_column ? (tid + r * NT) / BN : (tid + r * NT) % (8 * WK);
+        b_reg[r] = fetch(p.b, p.b_dtype, b_off[r], p.bs[1], k0 + 4 * c);
+      }
+    };
+    auto lds_chunk = [](int rows, int row, int c) { return ((c >> 3) * rows + row) * 8 + ((c & 7) ^ (row & 7)); };
+    auto store_tile = [&](int buf) {
+#pragma unroll
+      for (int r = 0; r < RA; r++) {
+        const int ch = tid + r * NT;
+        *reinterpret_cast<floatx4_t *>(&As[buf][4 * lds_chunk(BM, ch / (8 * WK), ch % (8 * WK))]) = a_reg[r];
+      }
+#pragma unroll
+      for (int r = 0; r < RB; r++) {
+        const int ch = tid + r * NT;
+        const int row = b_by_column ? ch % BN : ch / (8 * WK), c = b_by_column ? ch / BN : ch % (8 * WK);
+        *reinterpret_cast<floatx4_t *>(&Bs[buf][4 * lds_chunk(BN, row, c)]) = b_reg[r];
+      }
+    };
+    load_tile(0);
+    store_tile(0);
+    for (int kt = 0; kt < n_k; kt++) {
+      __syncthreads();  // tile kt is in LDS; everyone is done with tile kt - 1, whose buffer is written below
+      if (kt + 1 < n_k) load_tile((kt + 1) * BKT);
+      multiply(kt & 1);
+      if (kt + 1 < n_k) store_tile((kt + 1) & 1);
+    }
+  }
+
+  // ---- fold the WK shares of a block, first share first ----
+  if constexpr (WK > 1) {
+    static_assert((WK - 1) * WM * WN * 16 * 64 <= 2 * BM * BKT, "the folded shares fit the tiles of a");
+    float *xch = &As[0][0];
+    __syncthreads();
+    if (wk > 0) {
+      float *w = xch + ((wk - 1) * (WM * WN) + wave % (WM * WN)) * (16 * 64) + lane;
+#pragma unroll
+      for (int i = 0; i < 16; i++) w[i * 64] = acc[i];
+    }
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int o = 0; o < WK - 1; o++) {
+      const float *r = xch + (o * (WM * WN) + wave) * (16 * 64) + lane;
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[i] += r[i * 64];
+    }
+  }
+
+  // ---- epilogue: lane n holds column n0 + 32 wn + n, register i row 8 (i / 4) + 4 h + i % 4 of the wave's block ----
+  const int j = n0 + 32 * wn + n;
+  if (j >= p.N) return;
+  const float bias = p.bias ? load_as_f32(p.bias, b_col(j), p.bias_dtype) : 0.f;
+  // Offsets by addition: a division per row and lane made the epilogue a tenth of the launch at K = 2048.
+  const int mw = m0 + 32 * wm;
+  int64_t base, wrap = 0;          // offset of row mw; what a step to the next sequence adds beyond a row step
+  int row_step, s0 = 0, seq = INT_MAX;
+  if (p.heads) {  // c[b, head, s, d], rows m = b S + s
+    const int head = j / D, b = mw / p.seq;
+    seq = p.seq;
+    s0 = mw - b * seq;
+    row_step = D;
+    base = (((int64_t)b * p.heads + head) * seq + s0) * D + (j - head * D);
+    wrap = (int64_t)(p.heads - 1) * seq * D;
+  } else {
+    row_step = p.N;
+    base = ((int64_t)batch * p.M + mw) * p.N + j;
+  }
+  auto store_rows = [&](auto store) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int r = 8 * (i >> 2) + 4 * h + (i & 3);
+      if (mw + r >= p.M) break;  // rows ascend with i
+      int64_t off = base + (int64_t)r * row_step;
+      for (int s = s0 + r; s >= seq; s -= seq) off += wrap;
+      store(off, acc[i] + bias);
+    }
+  };
+  if (p.c_dtype == LMH_F32) store_rows([&](int64_t off, float x) { reinterpret_cast<float *>(p.c)[off] = x; });
+  else if (p.c_dtype == LMH_F16) store_rows([&](int64_t off, float x) { reinterpret_cast<_Float16 *>(p.c)[off] = (_Float16)x; });
+  else store_rows([&](int64_t off, float x) { reinterpret_cast<uint16_t *>(p.c)[off] = f32_to_bf16_bits(x); });
+}
+
+template <int WM, int WN, int WK>
+int launch_form(MatmulArgs &args, int n, hipStream_t stream) {
+  int64_t tiles = 0;
+  for (int i = 0; i < kMatmulGroup; i++) {
+    args.first_tile[i] = (int)tiles;
+    if (i < n) {
+      const MatmulProblem &p = args.p[i];
+      tiles += (int64_t)p.batch * ((p.M + 32 * WM - 1) / (32 * WM)) * ((p.N + 32 * WN - 1) / (32 * WN));
+    }
+    if (tiles >= (int64_t(1) << 31) - 8) return fail(LMH_E_UNSUPPORTED, "matmul: too many tiles");
+  }
+  args.n_tiles = (int)tiles;
+  bool vec = true;
+  for (int i = 0; i < n; i++) vec = vec && args.p[i].a_vec && args.p[i].b_vec;
+  const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(64 * WM * WN * WK);
+  if (vec) hipLaunchKernelGGL((matmul_f32_kernel<WM, WN, WK, true>), grid, block, 0, stream, args);
+  else hipLaunchKernelGGL((matmul_f32_kernel<WM, WN, WK, false>), grid, block, 0, stream, args);
+  LMH_HIP_TRY(hipGetLastError());
+  return LMH_OK;
+}
+
+}  // namespace
+
+int launch_matmul(MatmulArgs &args, int n, hipStream_t stream) {
+  // Rounds of the CUs times the 32 x 32 blocks of a workgroup, with a weight for what the smaller workgroups pay in loads and
+  // fixed costs per block. Measured, us for (64 x 64, eight waves) / (32 x 64) / (32 x 32): 700 x 2560 x 2048 82 / 90 / 99,
+  // 700 x 2048 x 2048 73 / 62 / 73, 606 x 1536 x 1536 33 / 35 / 39, 1446 x 768 x 384 18.5 / 16.1 / 19.5,
+  // 690 x 384 x 384 10.9 / 8.5 / 8.5, 164 x 1280 x 1280 26 / 18 / 11.
+  const int64_t cus = device_cu_count();
+  auto rounds = [&](int bm, int bn) {
+    int64_t tiles = 0;
+    for (int i = 0; i < n; i++) tiles += (int64_t)args.p[i].batch * ((args.p[i].M + bm - 1) / bm) * ((args.p[i].N + bn - 1) / bn);
+    return (tiles + cus - 1) / cus;
+  };
+  const int64_t r64 = rounds(64, 64);
+  const double c64 = 4.0 * r64, c32x64 = 2.2 * rounds(32, 64), c32 = 1.5 * rounds(32, 32);
+  if (c64 <= c32x64 && c64 <= c32) {
+    // with several rounds the other workgroups on a CU cover what eight waves on one block cover in a single round
+    // (4096^3: 1062 against 1086 us = 129 TFLOP/s, 82 % of the fp32 matrix peak)
+    if (r64 > 4) return launch_form<2, 2, 1>(args, n, stream);
+    return launch_form<2, 2, 2>(args, n, stream);
+  }
+  if (c32x64 <= c32) return launch_form<1, 2, 2>(args, n, stream);
+  return launch_form<1, 1, 4>(args, n, stream);
+}
+
+}  // namespace lmh

@@ -17,21 +17,22 @@ Additions the reference has only as un-fused subgraphs:
   GQA (Hkv < Hq) inside the fused ops            reference src/NN.jl:305-317, :362-366
 
 Around the attention path, a model graph also holds the nodes of the layer that calls it (projections, reshapes,
-permutes: reference src/NN.jl:343-361, :383-386). Those have no kernel here; they run through a host fallback
-(HostOp: download the inputs, the reference's CPU semantics in numpy, upload the result), so that a whole
-attention layer executes on a HIPDevice with attention itself on the GPU:
+permutes: reference src/NN.jl:343-361, :383-386). lowering.py takes them to lmh_matmul and lmh_map; the few forms those do
+not take (a column-major reshape that is not affine, batch shapes that need a broadcast) run through a host fallback
+(HostOp: download the inputs, the reference's CPU semantics in numpy, upload the result):
   MatMul, Permute, Reshape, Add, Expand          reference src/Execution.jl:216-250, src/HighLevelOps.jl:173-266
   Linear, SelfAttention                          reference src/NN.jl:11-38, :319-387
 
 Arrays here are row-major [B, H, S, D] (numpy order), which is the layout the C ABI takes. There
 is no CPU execution path for the attention ops: running one on host arrays raises.
 """
+import bisect
 import ctypes
 import math
 
 import numpy as np
 
-from . import binding
+from . import binding, lowering
 from .binding import HEADMAP_BLOCKED, HEADMAP_INTERLEAVED, LuminalHipError  # noqa: F401
 
 
@@ -301,11 +302,22 @@ class KVAppendOp(Op):
 
 
 class HostOp(Op):
-    """A node of the reference's graph that has no kernel in libluminal_hip.so. On a HIPDevice it runs through the host:
-    inputs are downloaded, `compute` applies the reference's CPU semantics in fp32 numpy (reference
-    src/Execution.jl:216-250), the result is uploaded in `out_dtype`. The logical meaning is the reference's; where
-    that depends on Julia's column-major element order (Reshape) the numpy form says so."""
+    """A node of the reference's graph around its attention nodes, computed in fp32 and stored in `out_dtype`. `compute` is
+    the reference's CPU semantics in numpy (reference src/Execution.jl:216-250); where that depends on Julia's
+    column-major element order (Reshape) the numpy form says so. On a HIPDevice `launcher` gives the same through
+    lmh_matmul or lmh_map; where it returns None the node runs through the host: inputs are downloaded, `compute`d, the
+    result is uploaded. Nodes that only move elements have `view` (see lowering.py) instead of a launcher of their own."""
     out_dtype = "f32"
+
+    def launcher(self, out, inputs):
+        if not hasattr(self, "view"):
+            return None
+        axes = self.view(lowering.contiguous_view(inputs[0].shape))
+        return None if axes is None else lowering.map_launcher(out, inputs[0], axes)
+
+    def result_shape(self, shapes):
+        axes = self.view(lowering.contiguous_view(shapes[0]))
+        return None if axes is None else tuple(math.prod(f[0] for f in axis) for axis in axes)
 
     def compute(self, *arrays):
         raise NotImplementedError
@@ -319,6 +331,15 @@ class MatMulOp(HostOp):
             raise ValueError("Matmul dimension mismatch: A is %s, B is %s" % (a.shape, b.shape))
         return np.matmul(a, b)
 
+    def launcher(self, out, inputs):
+        return lowering.matmul_launcher(out, *inputs)
+
+    def result_shape(self, shapes):
+        a, b = shapes
+        if len(a) < 2 or len(b) < 2 or not (len(a) == 2 or len(b) == 2 or a[:-2] == b[:-2]):
+            return None
+        return tuple(a[:-1] if len(b) == 2 else b[:-2] + a[-2:-1]) + (b[-1],)
+
 
 class PermuteOp(HostOp):
     """Permute(dims) = permutedims (reference src/Execution.jl:229); dims are 0-based here."""
@@ -328,6 +349,9 @@ class PermuteOp(HostOp):
 
     def compute(self, a):
         return np.transpose(a, self.dims)
+
+    def view(self, axes):
+        return lowering.permute_view(axes, self.dims)
 
 
 class ReshapeOp(HostOp):
@@ -341,12 +365,21 @@ class ReshapeOp(HostOp):
     def compute(self, a):
         return np.reshape(a, self.shape, order="F")
 
+    def view(self, axes):
+        return lowering.reshape_view(axes, self.shape)
+
 
 class AddOp(HostOp):
     """Add with the lower-rank operand given leading singleton axes (reference src/Execution.jl:207-216)."""
 
     def compute(self, a, b):
         return a + b
+
+    def launcher(self, out, inputs):
+        return lowering.add_launcher(out, *inputs)
+
+    def result_shape(self, shapes):
+        return tuple(np.broadcast_shapes(*shapes))
 
 
 class ExpandOp(HostOp):
@@ -357,6 +390,9 @@ class ExpandOp(HostOp):
 
     def compute(self, a):
         return np.repeat(np.expand_dims(a, self.dim), self.size, axis=self.dim)
+
+    def view(self, axes):
+        return lowering.expand_view(axes, self.dim, self.size)
 
 
 class Node:
@@ -379,6 +415,17 @@ class Graph:
         self.shapes = []
         self.dtypes = []
         self.tensors = {}
+        self._lowered = {}
+
+    def lowered(self, wanted, given):
+        """lowering.lower(self, wanted, given), kept while the graph stays as it is."""
+        key = (tuple(wanted), tuple(given))
+        state = [node.op for node in self.nodes]
+        if self._lowered.get("state") != state:
+            self._lowered = {"state": state}
+        if key not in self._lowered:
+            self._lowered[key] = lowering.lower(self, wanted, given)
+        return self._lowered[key]
 
 
 def add_op(graph, op, inputs, output_shape, dtype="f32"):
@@ -694,10 +741,26 @@ def flash_attention_plan(q_shape, kv_shape, dtype, causal=False, scale=None, out
 
 
 def _host_fallback(op, inputs):
-    """The reference's CPU semantics for a node without a kernel: download, compute in fp32 numpy, hand back the host
-    result (the caller uploads it)."""
+    """The reference's CPU semantics for a node that the device does not take: download, compute in fp32 numpy, hand back
+    the host result (the caller uploads it)."""
     host = [x.to_host() if isinstance(x, HipArray) else np.asarray(x, dtype=np.float32) for x in inputs]
     return np.ascontiguousarray(op.compute(*host), dtype=np.float32)
+
+
+def _overlap(a, b):
+    return a.ptr < b.ptr + b.nbytes and b.ptr < a.ptr + a.nbytes
+
+
+def _prepare_host_op(op, out, inputs):
+    """launch(stream) of a HostOp on device arrays, or None where it has to run through the host."""
+    if not all(isinstance(x, HipArray) and x.size and not _overlap(x, out) for x in inputs):
+        return None
+    shape = op.result_shape([x.shape for x in inputs])
+    if shape is None:
+        return None
+    if shape != out.shape:
+        raise ValueError("%s: result shape %s differs from the node's %s" % (type(op).__name__, shape, out.shape))
+    return op.launcher(out, inputs)
 
 
 def _prepare_decode_step(op, out, inputs, workspaces=None):
@@ -748,95 +811,147 @@ def execute_op_inplace(out, op, *inputs, stream=None, workspaces=None):
     is where decode attention takes its split-KV scratch from (default: one buffer shared by all eager calls)."""
     if isinstance(op, HostOp):
         if stream is not None:
-            raise RuntimeError("%s runs through the host and cannot be part of a recorded HIP graph" % type(op).__name__)
+            raise RuntimeError("%s may run through the host and cannot be part of a recorded HIP graph" % type(op).__name__)
         _require_hip(out)
+        launch = _prepare_host_op(op, out, inputs)
+        if launch is not None:
+            launch()
+            return out
         res = _host_fallback(op, inputs)
         if res.shape != out.shape:
             raise ValueError("%s: result shape %s differs from the node's %s" % (type(op).__name__, res.shape, out.shape))
         binding.sync()  # the inputs were produced by kernels on the null stream; the download above waited for them
         return out.copy_from_host(res)
     if isinstance(op, FlashAttentionOp):
-        q, k, v = inputs[:3]
-        rest = list(inputs[3:])
-        if not (op.has_kv_len or op.has_q_pos0) and len(rest) == 1:  # eager callers pass kv_len as a fourth array
-            kv_len, q_pos0 = rest[0], None
-        else:
-            if len(rest) != int(op.has_kv_len) + int(op.has_q_pos0):
-                raise ValueError("FlashAttentionOp takes (q, k, v%s%s); got %d inputs" %
-                                 (", kv_len" if op.has_kv_len else "", ", q_pos0" if op.has_q_pos0 else "", len(inputs)))
-            kv_len = rest.pop(0) if op.has_kv_len else None
-            q_pos0 = rest.pop(0) if op.has_q_pos0 else None
-        _require_hip(out, q, k, v)
-        if len(q.shape) != 4 or len(k.shape) != 4 or k.shape != v.shape:
-            raise ValueError("flash attention expects q (B,H,S,D) and k, v (B,Hkv,Sk,D); got %s %s %s" %
-                             (q.shape, k.shape, v.shape))
-        if out.shape != q.shape:
-            raise ValueError("output shape %s differs from q shape %s" % (out.shape, q.shape))
-        if not (q.dtype == k.dtype == v.dtype) or out.dtype not in (q.dtype, "f32"):
-            raise ValueError("q, k, v must share one element type; out has that type or f32")
-        if k.shape[0] != q.shape[0] or k.shape[3] != q.shape[3]:
-            raise ValueError("k/v batch or head dim differ from q's")
-        p = binding.AttnParams()
-        p.out, p.q, p.k, p.v = out.ptr, q.ptr, k.ptr, v.ptr
-        p.kv_len = kv_len.ptr if kv_len is not None else None
-        p.B, p.Hq, p.Sq, p.D = q.shape
-        p.Hkv, p.Sk = k.shape[1], k.shape[2]
-        p.dtype = binding.DTYPE_CODES[q.dtype]
-        p.scale, p.causal, p.head_map = op.scale, int(op.causal), op.head_map
-        p.out_f32 = int(out.dtype == "f32")
+        p = _attn_params(op, out, inputs)
         p.stream = stream
-        if op.q_rope_base is not None:
-            p.q_rope = 1
-            p.q_rope_pairing = binding.ROPE_INTERLEAVED if op.q_rope_interleaved else binding.ROPE_HALF_SPLIT
-            p.q_pos0 = q_pos0.ptr if q_pos0 is not None else None
-            p.q_prev_seq = op.q_prev_seq
-            p.q_rope_base = op.q_rope_base
         binding.flash_attn_fwd(p)
         return out
     if isinstance(op, DecodeAttentionOp):
-        q, kc, vc = inputs[:3]
-        kv_len = inputs[3] if len(inputs) > 3 else None
-        _require_hip(out, q, kc, vc)
-        if len(q.shape) != 3 or len(kc.shape) != 4 or kc.shape != vc.shape:
-            raise ValueError("decode attention expects q (B,H,D) and caches (B,Hkv,Lmax,D); got %s %s %s" %
-                             (q.shape, kc.shape, vc.shape))
-        if out.shape != q.shape:
-            raise ValueError("output shape %s differs from q shape %s" % (out.shape, q.shape))
-        if not (q.dtype == kc.dtype == vc.dtype) or out.dtype not in (q.dtype, "f32"):
-            raise ValueError("q and the caches must share one element type; out has that type or f32")
-        p = binding.DecodeParams()
-        p.out, p.q, p.k_cache, p.v_cache = out.ptr, q.ptr, kc.ptr, vc.ptr
-        p.kv_len = kv_len.ptr if kv_len is not None else None
-        p.B, p.Hq, p.D = q.shape
-        p.Hkv, p.Lmax = kc.shape[1], kc.shape[2]
-        p.dtype = binding.DTYPE_CODES[q.dtype]
-        p.scale, p.head_map = op.scale, op.head_map
-        p.out_f32 = int(out.dtype == "f32")
-        p.num_splits = op.num_splits or binding.decode_auto_splits(p.B, p.Hkv, p.Lmax)
-        need = binding.decode_workspace_bytes(p.B, p.Hq, p.Hkv, p.Lmax, p.D, p.num_splits)
-        p.workspace, p.workspace_bytes = (workspaces or _workspaces).get(need, q.device)
+        p, need = _decode_params(op, out, inputs)
+        p.workspace, p.workspace_bytes = (workspaces or _workspaces).get(need, inputs[0].device)
         p.stream = stream
         binding.decode_attn(p)
         return out
     if isinstance(op, DecodeStepOp):
         return _prepare_decode_step(op, out, inputs, workspaces)(stream)
     if isinstance(op, RotaryEmbeddingOp):
-        x = inputs[0]
-        pos0 = inputs[1] if len(inputs) > 1 else None
-        return apply_rotary_embeddings(x, op.prev_seq, op.base, pos0=pos0, out=out, interleaved=op.interleaved,
-                                       stream=stream)
+        binding.rope(_rope_op_params(op, out, inputs, stream))
+        return out
     if isinstance(op, KVAppendOp):
-        if len(inputs) != (6 if op.rope_q else 5):
-            raise ValueError("KVAppendOp takes (k_cache, v_cache, k_new, v_new, pos%s)" % (", q" if op.rope_q else ""))
-        kc, vc, k_new, v_new, pos = inputs[:5]
-        q = inputs[5] if op.rope_q else None
-        if out is not None and not (isinstance(out, tuple) and out[0] is kc and out[1] is vc and
-                                    (q is None or out[2] is q)):
-            raise ValueError("KVAppendOp works in place: its outputs are its cache (and query) inputs")
-        kv_append(kc, vc, k_new, v_new, pos, rope_k=op.rope_k, base=op.base, interleaved=op.interleaved, q=q,
-                  stream=stream)
-        return (kc, vc) if q is None else (kc, vc, q)
+        binding.kv_append(_kv_append_op_params(op, out, inputs, stream))
+        return tuple(inputs[:2]) if not op.rope_q else (inputs[0], inputs[1], inputs[5])
     raise TypeError("no HIP kernel for op %s" % type(op).__name__)
+
+
+def _attn_params(op, out, inputs):
+    """Validates a FlashAttentionOp call; the parameter block without its stream."""
+    q, k, v = inputs[:3]
+    rest = list(inputs[3:])
+    if not (op.has_kv_len or op.has_q_pos0) and len(rest) == 1:  # eager callers pass kv_len as a fourth array
+        kv_len, q_pos0 = rest[0], None
+    else:
+        if len(rest) != int(op.has_kv_len) + int(op.has_q_pos0):
+            raise ValueError("FlashAttentionOp takes (q, k, v%s%s); got %d inputs" %
+                             (", kv_len" if op.has_kv_len else "", ", q_pos0" if op.has_q_pos0 else "", len(inputs)))
+        kv_len = rest.pop(0) if op.has_kv_len else None
+        q_pos0 = rest.pop(0) if op.has_q_pos0 else None
+    _require_hip(out, q, k, v)
+    if len(q.shape) != 4 or len(k.shape) != 4 or k.shape != v.shape:
+        raise ValueError("flash attention expects q (B,H,S,D) and k, v (B,Hkv,Sk,D); got %s %s %s" %
+                         (q.shape, k.shape, v.shape))
+    if out.shape != q.shape:
+        raise ValueError("output shape %s differs from q shape %s" % (out.shape, q.shape))
+    if not (q.dtype == k.dtype == v.dtype) or out.dtype not in (q.dtype, "f32"):
+        raise ValueError("q, k, v must share one element type; out has that type or f32")
+    if k.shape[0] != q.shape[0] or k.shape[3] != q.shape[3]:
+        raise ValueError("k/v batch or head dim differ from q's")
+    p = binding.AttnParams()
+    p.out, p.q, p.k, p.v = out.ptr, q.ptr, k.ptr, v.ptr
+    p.kv_len = kv_len.ptr if kv_len is not None else None
+    p.B, p.Hq, p.Sq, p.D = q.shape
+    p.Hkv, p.Sk = k.shape[1], k.shape[2]
+    p.dtype = binding.DTYPE_CODES[q.dtype]
+    p.scale, p.causal, p.head_map = op.scale, int(op.causal), op.head_map
+    p.out_f32 = int(out.dtype == "f32")
+    if op.q_rope_base is not None:
+        p.q_rope = 1
+        p.q_rope_pairing = binding.ROPE_INTERLEAVED if op.q_rope_interleaved else binding.ROPE_HALF_SPLIT
+        p.q_pos0 = q_pos0.ptr if q_pos0 is not None else None
+        p.q_prev_seq = op.q_prev_seq
+        p.q_rope_base = op.q_rope_base
+    return p
+
+
+def _decode_params(op, out, inputs):
+    """Validates a DecodeAttentionOp call; (the parameter block without workspace and stream, workspace bytes)."""
+    q, kc, vc = inputs[:3]
+    kv_len = inputs[3] if len(inputs) > 3 else None
+    _require_hip(out, q, kc, vc)
+    if len(q.shape) != 3 or len(kc.shape) != 4 or kc.shape != vc.shape:
+        raise ValueError("decode attention expects q (B,H,D) and caches (B,Hkv,Lmax,D); got %s %s %s" %
+                         (q.shape, kc.shape, vc.shape))
+    if out.shape != q.shape:
+        raise ValueError("output shape %s differs from q shape %s" % (out.shape, q.shape))
+    if not (q.dtype == kc.dtype == vc.dtype) or out.dtype not in (q.dtype, "f32"):
+        raise ValueError("q and the caches must share one element type; out has that type or f32")
+    p = binding.DecodeParams()
+    p.out, p.q, p.k_cache, p.v_cache = out.ptr, q.ptr, kc.ptr, vc.ptr
+    p.kv_len = kv_len.ptr if kv_len is not None else None
+    p.B, p.Hq, p.D = q.shape
+    p.Hkv, p.Lmax = kc.shape[1], kc.shape[2]
+    p.dtype = binding.DTYPE_CODES[q.dtype]
+    p.scale, p.head_map = op.scale, op.head_map
+    p.out_f32 = int(out.dtype == "f32")
+    p.num_splits = op.num_splits or binding.decode_auto_splits(p.B, p.Hkv, p.Lmax)
+    return p, binding.decode_workspace_bytes(p.B, p.Hq, p.Hkv, p.Lmax, p.D, p.num_splits)
+
+
+def _rope_op_params(op, out, inputs, stream=None):
+    return _rope_params(inputs[0], out, op.prev_seq, op.base, inputs[1] if len(inputs) > 1 else None, op.interleaved, stream)
+
+
+def _kv_append_op_params(op, out, inputs, stream=None):
+    if len(inputs) != (6 if op.rope_q else 5):
+        raise ValueError("KVAppendOp takes (k_cache, v_cache, k_new, v_new, pos%s)" % (", q" if op.rope_q else ""))
+    kc, vc, k_new, v_new, pos = inputs[:5]
+    q = inputs[5] if op.rope_q else None
+    if out is not None and not (isinstance(out, tuple) and out[0] is kc and out[1] is vc and (q is None or out[2] is q)):
+        raise ValueError("KVAppendOp works in place: its outputs are its cache (and query) inputs")
+    return _kv_append_params(kc, vc, k_new, v_new, pos, op.rope_k, op.base, op.interleaved, q, stream)
+
+
+def _prepare(op, out, inputs, workspaces):
+    """launch(stream) of an op on buffers that never move: validated and its parameter block filled once, so that a
+    compiled graph's step costs the host one call of the library."""
+    if isinstance(op, HostOp):
+        launch = _prepare_host_op(op, out, inputs)
+        if launch is None:
+            return lambda stream=None: execute_op_inplace(out, op, *inputs, stream=stream)
+        return launch
+    if isinstance(op, DecodeStepOp):
+        return _prepare_decode_step(op, out, inputs, workspaces)
+    if isinstance(op, FlashAttentionOp):
+        p, call = _attn_params(op, out, inputs), binding.flash_attn_fwd
+    elif isinstance(op, RotaryEmbeddingOp):
+        p, call = _rope_op_params(op, out, inputs), binding.rope
+    elif isinstance(op, KVAppendOp):
+        p, call = _kv_append_op_params(op, out, inputs), binding.kv_append
+    elif isinstance(op, DecodeAttentionOp):
+        p, need = _decode_params(op, out, inputs)
+        device = inputs[0].device
+
+        def call(p):
+            p.workspace, p.workspace_bytes = workspaces.get(need, device)
+            binding.decode_attn(p)
+    else:
+        raise TypeError("no HIP kernel for op %s" % type(op).__name__)
+
+    def launch(stream=None):
+        p.stream = stream
+        call(p)
+
+    return launch
 
 
 def execute_op(op, *inputs):
@@ -845,6 +960,14 @@ def execute_op(op, *inputs):
         dev = next((x.device for x in inputs if isinstance(x, HipArray)), None)
         if dev is None:
             raise TypeError("%s: no input is on a HIP device" % type(op).__name__)
+        if all(isinstance(x, HipArray) and x.size for x in inputs):
+            shape = op.result_shape([x.shape for x in inputs])
+            if shape is not None:
+                out = HipArray(shape, op.out_dtype, dev)
+                launch = op.launcher(out, inputs)
+                if launch is not None:
+                    launch()
+                    return out
         res = _host_fallback(op, inputs)
         return HipArray(res.shape, op.out_dtype, dev).copy_from_host(res)
     q = inputs[0]
@@ -880,11 +1003,16 @@ def execute(graph, output_ids, initial_inputs, device=None, dtype=None):
         if node_id not in results and out_idx == 0:
             results[node_id] = to_device(data, device, graph.dtypes[node_id])
     for node_id, node in enumerate(graph.nodes):
-        if node_id in results:
-            continue
-        if isinstance(node.op, InputTensor):
+        if isinstance(node.op, InputTensor) and node_id not in results:
             raise KeyError("no value given for input tensor %d" % node_id)
-        results[node_id] = execute_op(node.op, *[_pick(results, ref) for ref in node.inputs])
+    for step in graph.lowered(ids, results)[0]:
+        args = [_pick(results, ref) for ref in step.inputs]
+        if isinstance(step, lowering.NodeOp):
+            results[step.nodes[0]] = execute_op(graph.nodes[step.nodes[0]].op, *args)
+        else:
+            outs = [HipArray(graph.shapes[i], graph.dtypes[i], device) for i in step.nodes]
+            step.prepare(outs, args)()
+            results.update(zip(step.nodes, outs))
     final = {i: from_device(results[i][0] if isinstance(results[i], tuple) else results[i]) for i in ids}
     return final[ids[0]] if single else final
 
@@ -936,34 +1064,55 @@ def release_capture(cache):
     cache.pop("hip_warm", None)
 
 
+class _Results(list):
+    """The node buffers of a compiled graph. A node that disappeared into another node's launch has none until somebody
+    asks for it: then it is computed from its operands, and by every later call as well."""
+
+    def __init__(self, buffers, materialise):
+        super().__init__(buffers)
+        self._materialise = materialise
+
+    def __getitem__(self, i):
+        if isinstance(i, slice):
+            return [self[j] for j in range(*i.indices(len(self)))]
+        value = super().__getitem__(i)
+        return self._materialise(self, i if i >= 0 else i + len(self)) if value is None else value
+
+    def __iter__(self):
+        return (self[i] for i in range(len(self)))
+
+
 class CompiledGraph:
     """Pre-allocated node buffers + a step list (reference src/Compiler.jl:75-100). Calling it copies the
     inputs into their buffers, runs the steps in place and returns the buffer list; nothing is
     allocated per call. After capture() the steps go through execute_with_capture: one HIP graph launch."""
 
     def __init__(self, steps, results, workspaces=None, device=None, host_steps=0):
-        self.host_steps = host_steps  # nodes served by the host fallback
+        self.host_steps = host_steps  # nodes of the classes that may run through the host
         self.steps = steps
         self.results = results
         self.workspaces = workspaces  # decode scratch owned by this graph: its address never changes
         self.device = device
         self.cache = {}
         self.use_capture = False
+        self._copies = {}
 
     def _run(self, stream):
         for step in self.steps:
             step(stream)
 
     def __call__(self, inputs, device=None):
-        for k, v in inputs.items():
-            if k >= len(self.results) or self.results[k] is None:
-                raise KeyError("Input node %d not found in compiled graph results." % k)
-            if isinstance(v, HipArray):
-                if v.nbytes != self.results[k].nbytes:
-                    raise ValueError("Input length mismatch for node %d" % k)
-                binding.memcpy_d2d(self.results[k].ptr, v.ptr, v.nbytes)
-            else:
-                self.results[k].copy_from_host(v)
+        try:  # device arrays: one launch copies them all; its ranges are kept with the addresses they hold for (a program
+            # feeds the same few arrays again and again)
+            key = (*inputs, *[v.ptr for v in inputs.values()], *[v.nbytes for v in inputs.values()])
+            copies = self._copies.get(key)
+            if copies is None:
+                copies = self._plan_copies(key, inputs)
+            if copies:
+                copies.launch()
+        except AttributeError:  # host arrays among them
+            for k, v in inputs.items():
+                self._copy_one(k, v)
         if self.use_capture:
             execute_with_capture(self.device, self._run, self.cache)
         else:
@@ -971,12 +1120,43 @@ class CompiledGraph:
             self.cache["hip_warm"] = True
         return self.results
 
+    def _buffer(self, k):
+        if k >= len(self.results) or self.results[k] is None:
+            raise KeyError("Input node %d not found in compiled graph results." % k)
+        return self.results[k]
+
+    def _copy_one(self, k, v):
+        buffer = self._buffer(k)
+        if isinstance(v, HipArray):
+            if v.nbytes != buffer.nbytes:
+                raise ValueError("Input length mismatch for node %d" % k)
+            binding.memcpy_d2d(buffer.ptr, v.ptr, v.nbytes)
+        else:
+            buffer.copy_from_host(v)
+
+    def _plan_copies(self, key, inputs):
+        pairs = []
+        for k, v in inputs.items():
+            buffer = self._buffer(k)
+            if v.nbytes != buffer.nbytes:
+                raise ValueError("Input length mismatch for node %d" % k)
+            if v.ptr != buffer.ptr:
+                pairs.append((buffer.ptr, v.ptr, v.nbytes))
+        if lowering.copies_overlap(pairs):  # one after the other
+            for k, v in inputs.items():
+                self._copy_one(k, v)
+            return None
+        if len(self._copies) >= 64:
+            self._copies.clear()
+        self._copies[key] = copies = lowering.CopyList(pairs) if pairs else False
+        return copies
+
     def capture(self):
         """From the next call on, run the step list as one recorded HIP graph. Buffer addresses are fixed and
         per-step values (positions, lengths) are device tensors, so one recording is valid for every call."""
         if self.host_steps:
-            raise RuntimeError("this graph has %d nodes that run through the host (projections, reshapes): only graphs "
-                               "of device ops can be recorded" % self.host_steps)
+            raise RuntimeError("this graph has %d nodes of kinds that may run through the host (projections, reshapes): only "
+                               "graphs without them can be recorded" % self.host_steps)
         self.use_capture = True
         return self
 
@@ -993,28 +1173,41 @@ def compile(graph, device=None):
     device = device or get_device()
     if not isinstance(device, HIPDevice):
         raise RuntimeError("compile: no HIP device available and this backend has no CPU path")
+    lowered, virtual = graph.lowered((), ())
     results = []
+
+    def buffer(node_id):
+        return HipArray(graph.shapes[node_id], graph.dtypes[node_id], device).fill_bytes(0)
+
     for node_id, node in enumerate(graph.nodes):
         if isinstance(node.op, KVAppendOp):  # in place: the node's outputs are its cache (and query) inputs
             refs = [node.inputs[0], node.inputs[1]] + ([node.inputs[5]] if node.op.rope_q else [])
             results.append(tuple(_pick(results, r) for r in refs))
-            continue
-        if isinstance(node.op, DecodeStepOp):  # output 0 is a buffer of its own, outputs 1 and 2 are the cache inputs
-            results.append((HipArray(graph.shapes[node_id], graph.dtypes[node_id], device).fill_bytes(0),
-                            _pick(results, node.inputs[1]), _pick(results, node.inputs[2])))
-            continue
-        results.append(HipArray(graph.shapes[node_id], graph.dtypes[node_id], device).fill_bytes(0))
-    steps = []
+        elif isinstance(node.op, DecodeStepOp):  # output 0 is a buffer of its own, outputs 1 and 2 are the cache inputs
+            results.append((buffer(node_id), _pick(results, node.inputs[1]), _pick(results, node.inputs[2])))
+        else:
+            results.append(None if node_id in virtual else buffer(node_id))
+    steps, at = [], []  # at: the first node of each step, ascending
     workspaces = _Workspaces()
-    for node_id, node in enumerate(graph.nodes):
-        if isinstance(node.op, InputTensor):
-            continue
-        args = [_pick(results, ref) for ref in node.inputs]
-        if isinstance(node.op, DecodeStepOp):
-            steps.append(_prepare_decode_step(node.op, results[node_id], args, workspaces))
-            continue
-        steps.append(lambda stream, out=results[node_id], op=node.op, args=args:
-                     execute_op_inplace(out, op, *args, stream=stream, workspaces=workspaces))
+
+    def materialise(results, node_id):  # (given the list, not holding it: a dropped graph frees its buffers at once)
+        node = graph.nodes[node_id]
+        out = buffer(node_id)
+        list.__setitem__(results, node_id, out)
+        launch = _prepare(node.op, out, [_pick(results, ref) for ref in node.inputs], workspaces)
+        where = bisect.bisect_left(at, node_id)
+        steps.insert(where, launch)
+        at.insert(where, node_id)
+        launch()
+        return out
+
+    results = _Results(results, materialise)
+    for step in lowered:
+        args = [_pick(results, ref) for ref in step.inputs]
+        outs = [list.__getitem__(results, i) for i in step.nodes]
+        steps.append(step.prepare(outs, args) if not isinstance(step, lowering.NodeOp) else
+                     _prepare(graph.nodes[step.nodes[0]].op, outs[0], args, workspaces))
+        at.append(min(step.nodes))
     host_steps = sum(isinstance(node.op, HostOp) for node in graph.nodes)
     return CompiledGraph(steps, results, workspaces, device, host_steps)
 
@@ -1027,9 +1220,15 @@ def apply_rotary_embeddings(x, prev_seq=0, base=10000.0, pos0=None, out=None, in
     (apply_rotary_embeddings(input, prev_seq; base), reference src/NN.jl:253-303). `pos0` (HipArray
     int32[B]) gives per-sequence start positions instead of the scalar prev_seq; `out` may be x."""
     _require_hip(x)
+    out = out if out is not None else HipArray(x.shape, x.dtype, x.device)
+    binding.rope(_rope_params(x, out, prev_seq, base, pos0, interleaved, stream))
+    return out
+
+
+def _rope_params(x, out, prev_seq, base, pos0, interleaved, stream):
+    _require_hip(x)
     if len(x.shape) != 4:
         raise ValueError("rotary embedding expects (B,H,S,D); got %s" % (x.shape,))
-    out = out if out is not None else HipArray(x.shape, x.dtype, x.device)
     if out.shape != x.shape or out.dtype != x.dtype:
         raise ValueError("rotary embedding: out must match x in shape and element type")
     p = binding.RopeParams()
@@ -1041,8 +1240,7 @@ def apply_rotary_embeddings(x, prev_seq=0, base=10000.0, pos0=None, out=None, in
     p.base = float(base)
     p.pairing = binding.ROPE_INTERLEAVED if interleaved else binding.ROPE_HALF_SPLIT
     p.stream = stream
-    binding.rope(p)
-    return out
+    return p
 
 
 def kv_append(k_cache, v_cache, k_new, v_new, pos, rope_k=False, base=10000.0, interleaved=False, q=None,
@@ -1050,6 +1248,10 @@ def kv_append(k_cache, v_cache, k_new, v_new, pos, rope_k=False, base=10000.0, i
     """In-place cache update cache[b,h,pos[b]+t,:] = new[b,h,t,:] (the reference rebuilds the whole cache
     with _kv_scatter, reference src/Whisper.jl:552-570). `pos` is a HipArray int32[B] or an int. `q`
     (B,Hq,T,D), if given, is rotated in place at the same positions by the same launch."""
+    binding.kv_append(_kv_append_params(k_cache, v_cache, k_new, v_new, pos, rope_k, base, interleaved, q, stream))
+
+
+def _kv_append_params(k_cache, v_cache, k_new, v_new, pos, rope_k, base, interleaved, q, stream):
     _require_hip(k_cache, v_cache, k_new, v_new)
     if k_cache.shape != v_cache.shape or k_new.shape != v_new.shape or len(k_cache.shape) != 4:
         raise ValueError("kv_append expects caches (B,Hkv,Lmax,D) and new rows (B,Hkv,T,D)")
@@ -1076,7 +1278,7 @@ def kv_append(k_cache, v_cache, k_new, v_new, pos, rope_k=False, base=10000.0, i
             raise ValueError("kv_append: q %s (%s) does not match new rows %s (%s)" %
                              (q.shape, q.dtype, k_new.shape, k_cache.dtype))
         p.q_rope, p.Hq = q.ptr, q.shape[1]
-    binding.kv_append(p)
+    return p
 
 
 class KVCacheState:

@@ -1,0 +1,390 @@
+"""How the nodes around attention reach the device: the reference's Permute, Reshape, Expand, Add and MatMul nodes
+(reference src/Execution.jl:12-90, :207-250) as launches of lmh_map and lmh_matmul, and the chains of them that an
+attention layer is made of as one launch each.
+
+Permute, Reshape and Expand move elements and change none, so a chain of them is an affine map from the index space of
+its last node to the memory of its first operand, and runs as one lmh_map however long it is. Around a MatMul:
+
+  x W^T (+ bias)                     one product that reads W as it lies (no transposed copy of the weights)
+  ... split into heads and permuted  the same product, storing where the permute would have put the element
+  several of these on the same x     one launch
+
+The nodes in between are then not computed: `lower` returns them as `virtual`, and whoever asks for such a node gets it
+from its own operands (host.CompiledGraph, host.execute).
+"""
+import ctypes
+
+from . import binding
+
+_CODES = dict(binding.DTYPE_CODES, i32=binding.LMH_I32)
+
+
+# ---------------------------------------------------------------------------------------------
+# affine views
+# ---------------------------------------------------------------------------------------------
+def contiguous_view(shape):
+    """A view is a list of axes, each a list of (size, element stride) factors, the slowest first."""
+    axes, stride = [], 1
+    for n in reversed(shape):
+        axes.append([(n, stride)])
+        stride *= n
+    return axes[::-1]
+
+
+def permute_view(axes, dims):
+    order = [d + len(axes) if d < 0 else d for d in dims]
+    return [axes[d] for d in order] if sorted(order) == list(range(len(axes))) else None
+
+
+def expand_view(axes, dim, size):
+    dim = dim + len(axes) + 1 if dim < 0 else dim
+    return axes[:dim] + [[(size, 0)]] + axes[dim:] if 0 <= dim <= len(axes) and size > 0 else None
+
+
+def reshape_view(axes, shape):
+    """Column-major reshape (Base.reshape): the elements keep their order with the FIRST axis the fastest one. None where
+    a new axis would cut an old one at a place that does not divide it (then the map is not affine)."""
+    pending = [f for axis in axes for f in reversed(axis) if f[0] != 1]  # fastest first
+    pending.reverse()  # the fastest at the end
+    out = []
+    if any(n < 1 for n in shape):
+        return None
+    for n in shape:
+        axis = []
+        while n > 1:
+            if not pending:
+                return None
+            size, stride = pending.pop()
+            if size > n:
+                if size % n:
+                    return None
+                pending.append((size // n, stride * n))
+                size = n
+            elif n % size:
+                return None
+            axis.append((size, stride))
+            n //= size
+        out.append(axis[::-1])
+    return None if pending else out
+
+
+def view_dims(axes):
+    """(dims, strides) of a view, the slowest first, neighbours that walk memory together merged."""
+    dims = []
+    for n, s in (f for axis in axes for f in axis if f[0] != 1):
+        if dims and dims[-1][1] == s * n:
+            dims[-1] = (dims[-1][0] * n, s)
+        else:
+            dims.append((n, s))
+    dims = dims or [(1, 0)]
+    return [d[0] for d in dims], [d[1] for d in dims]
+
+
+def broadcast_dims(shape, a_shape, b_shape):
+    """(dims, a strides, b strides) of an elementwise sum with numpy's broadcasting."""
+    def strides(own):
+        view = contiguous_view(own)
+        own = (1,) * (len(shape) - len(own)) + tuple(own)
+        view = [[(1, 0)]] * (len(shape) - len(view)) + view
+        return [0 if n == 1 else v[0][1] for n, v in zip(own, view)]
+
+    out = []
+    for n, sa, sb in zip(shape, strides(a_shape), strides(b_shape)):
+        if n == 1:
+            continue
+        if out and out[-1][1] == sa * n and out[-1][2] == sb * n:
+            out[-1] = (out[-1][0] * n, sa, sb)
+        else:
+            out.append((n, sa, sb))
+    out = out or [(1, 0, 0)]
+    return [d[0] for d in out], [d[1] for d in out], [d[2] for d in out]
+
+
+# ---------------------------------------------------------------------------------------------
+# launchers: parameter blocks filled once, launch(stream) as often as the buffers stand
+# ---------------------------------------------------------------------------------------------
+def map_launcher(out, a, axes):
+    """out = the elements of `a` seen through `axes`; None where lmh_map does not take it."""
+    dims, strides = view_dims(axes)
+    if len(dims) > binding.MAP_DIMS or max(dims) >= 1 << 31:
+        return None
+    p = binding.MapParams()
+    p.out, p.a, p.out_dtype, p.a_dtype = out.ptr, a.ptr, _CODES[out.dtype], _CODES[a.dtype]
+    p.n_dims = len(dims)
+    p.dims[:len(dims)], p.a_stride[:len(dims)] = dims, strides
+    return lambda stream=None: binding.map_op(p, stream)
+
+
+def add_launcher(out, a, b):
+    dims, sa, sb = broadcast_dims(out.shape, a.shape, b.shape)
+    if len(dims) > binding.MAP_DIMS or max(dims) >= 1 << 31:
+        return None
+    p = binding.MapParams()
+    p.out, p.a, p.b = out.ptr, a.ptr, b.ptr
+    p.out_dtype, p.a_dtype, p.b_dtype = _CODES[out.dtype], _CODES[a.dtype], _CODES[b.dtype]
+    p.n_dims = len(dims)
+    p.dims[:len(dims)], p.a_stride[:len(dims)], p.b_stride[:len(dims)] = dims, sa, sb
+    return lambda stream=None: binding.map_op(p, stream)
+
+
+def _product(n):
+    r = 1
+    for x in n:
+        r *= x
+    return r
+
+
+def fill_matmul(p, out, a, b, transposed=False, bias=None, heads=0):
+    """Fill one lmh_matmul_params; `transposed`: b is (N, K). False where the batch shapes need a broadcast that one
+    batch stride does not express."""
+    M, K = a.shape[-2:]
+    N = b.shape[-2] if transposed else b.shape[-1]
+    if (b.shape[-1] if transposed else b.shape[-2]) != K:
+        raise ValueError("Matmul dimension mismatch: A is %s, B is %s" % (a.shape, b.shape))
+    batch, a_batch, b_batch = 1, 0, 0
+    if len(b.shape) == 2:
+        M = _product(a.shape[:-1])
+    elif a.shape[:-2] == b.shape[:-2] or len(a.shape) == 2:
+        batch, b_batch = _product(b.shape[:-2]), N * K
+        a_batch = 0 if len(a.shape) == 2 else M * K
+    else:
+        return False
+    if max(batch, M, N, K) >= 1 << 31:
+        return False
+    p.c, p.a, p.b, p.batch, p.M, p.N, p.K = out.ptr, a.ptr, b.ptr, batch, M, N, K
+    p.a_stride[:] = [a_batch, K, 1]
+    p.b_stride[:] = [b_batch, 1, K] if transposed else [b_batch, N, 1]
+    p.a_dtype, p.b_dtype, p.c_dtype = _CODES[a.dtype], _CODES[b.dtype], _CODES[out.dtype]
+    if bias is not None:
+        p.bias, p.bias_dtype = bias.ptr, _CODES[bias.dtype]
+    if heads:
+        p.heads, p.seq = heads, a.shape[-2]
+    return True
+
+
+def matmul_launcher(out, a, b):
+    p = (binding.MatmulParams * 1)()
+    if len(a.shape) < 2 or len(b.shape) < 2 or not fill_matmul(p[0], out, a, b):
+        return None
+    return lambda stream=None: binding.matmul(p, 1, stream)
+
+
+class Projection:
+    """One product of a ProjectionOp: the node whose value it is, x W^T (+ bias), heads > 0 where it is split."""
+
+    def __init__(self, node, weight, bias, heads):
+        self.node, self.weight, self.bias, self.heads = node, weight, bias, heads
+
+
+class ProjectionOp:
+    """x W^T (+ bias) for up to MATMUL_GROUP weights in one launch, each written where its chain's last node wants it."""
+
+    def __init__(self, x, items):
+        self.items = items
+        self.inputs = [x]  # (node, output index, shape) references, like a graph node's
+        self.nodes = [i.node for i in items]
+        for i in items:
+            self.inputs += [i.weight] + ([i.bias] if i.bias is not None else [])
+
+    def prepare(self, outs, arrays):
+        p = (binding.MatmulParams * len(self.items))()
+        x, rest = arrays[0], list(arrays[1:])
+        for q, item, out in zip(p, self.items, outs):
+            w = rest.pop(0)
+            fill_matmul(q, out, x, w, transposed=True, bias=rest.pop(0) if item.bias is not None else None, heads=item.heads)
+        return lambda stream=None: binding.matmul(p, len(self.items), stream)
+
+
+class ViewOp:
+    """A chain of Permute, Reshape and Expand as one lmh_map."""
+
+    def __init__(self, node, base, axes):
+        self.nodes, self.inputs, self.axes = [node], [base], axes
+
+    def prepare(self, outs, arrays):
+        return map_launcher(outs[0], arrays[0], self.axes)
+
+
+class NodeOp:
+    """A graph node that runs as itself."""
+
+    def __init__(self, node, inputs):
+        self.nodes, self.inputs = [node], inputs
+
+
+# ---------------------------------------------------------------------------------------------
+# from a graph to steps
+# ---------------------------------------------------------------------------------------------
+class _Lowering:
+    def __init__(self, graph, wanted, given):
+        self.graph, self.given = graph, given
+        self.users = [[] for _ in graph.nodes]
+        for i, node in enumerate(graph.nodes):
+            for ref in node.inputs:
+                self.users[ref[0]].append(i)
+        # a node may disappear into its only user; nodes without users are results
+        self.private = [len(u) == 1 and i not in wanted and i not in given for i, u in enumerate(self.users)]
+        self.virtual = set()
+
+    def op(self, i):
+        return self.graph.nodes[i].op
+
+    def plain(self, i):
+        """Node i is private and fp32, so that computing it in passing rounds nothing less than before."""
+        return self.private[i] and self.graph.dtypes[i] == "f32"
+
+    def base_view(self, ref, inside):
+        """Follow a chain of view nodes from `ref` back to an operand that stays: (base reference, axes). `inside`
+        collects the nodes passed through."""
+        node, index, shape = ref[0], ref[1], tuple(ref[2])
+        chain = []
+        while index == 0 and node not in self.given and self.private[node] and hasattr(self.op(node), "view") and \
+                shape == tuple(self.graph.shapes[node]) and \
+                self.graph.dtypes[node] in ("f32", self.graph.dtypes[self.graph.nodes[node].inputs[0][0]]):
+            chain.append(node)
+            node, index, shape = self.graph.nodes[node].inputs[0][:2] + (tuple(self.graph.nodes[node].inputs[0][2]),)
+        base, axes = (node, index, shape), contiguous_view(shape)
+        for n in reversed(chain):
+            axes = self.op(n).view(axes)
+            if axes is None:
+                return ref, contiguous_view(ref[2])
+        inside.update(chain)
+        return base, axes
+
+    def weight(self, ref):
+        """The (N, K) tensor whose transpose `ref` is, and the transpose's node; None where it is something else."""
+        node = ref[0]
+        if not self.private[node] or type(self.op(node)).__name__ != "PermuteOp" or self.op(node).dims != (1, 0):
+            return None
+        base = self.graph.nodes[node].inputs[0]
+        same_type = self.graph.dtypes[node] in ("f32", self.graph.dtypes[base[0]])
+        return (base, node) if same_type and self.is_input(base) else None
+
+    def is_input(self, ref):
+        return type(self.op(ref[0])).__name__ == "InputTensor" or ref[0] in self.given
+
+    def bias(self, ref, width):
+        """The [width] tensor that `ref` repeats along leading axes; None where it is something else."""
+        inside = set()
+        base, axes = self.base_view(ref, inside)
+        flat = [f for axis in axes for f in axis if f[0] != 1 and f[1] != 0]
+        if tuple(base[2]) == (width,) and axes and axes[-1] == [(width, 1)] and flat in ([(width, 1)], []) and self.is_input(base):
+            return base, inside
+        return None
+
+    def projection(self, i):
+        """A Projection that starts at MatMul node i, its x and the nodes it swallows."""
+        x, b = ((r[0], r[1], tuple(r[2])) for r in self.graph.nodes[i].inputs)
+        w = self.weight(b) if len(x[2]) == 3 and len(b[2]) == 2 else None
+        if w is None:
+            return None
+        weight, inside = w[0], {w[1]}
+        node, bias, heads = i, None, 0
+        batch, seq, width = self.graph.shapes[i]
+        if self.plain(node):
+            user = self.users[node][0]
+            if type(self.op(user)).__name__ == "AddOp" and self.graph.shapes[user] == (batch, seq, width) and user not in self.given:
+                other = [r for r in self.graph.nodes[user].inputs if r[0] != node]
+                found = self.bias(other[0], width) if other else None
+                if found:
+                    bias = found[0]
+                    inside |= found[1] | {node}
+                    node = user
+        if self.plain(node):
+            split = self.users[node][0]
+            if type(self.op(split)).__name__ == "ReshapeOp" and len(self.op(split).shape) == 4 and split not in self.given and self.plain(split):
+                shape, last = self.op(split).shape, self.users[split][0]
+                if shape[:2] == (batch, seq) and type(self.op(last)).__name__ == "PermuteOp" and self.op(last).dims == (0, 2, 1, 3) and \
+                        last not in self.given:
+                    inside |= {node, split}
+                    node, heads = last, shape[2]
+        if self.graph.dtypes[node] == "i32":
+            return None
+        return Projection(node, weight, bias, heads), x, inside
+
+    def steps(self):
+        steps, by_x = [], {}
+        products = {i: self.projection(i) for i, n in enumerate(self.graph.nodes) if type(n.op).__name__ == "MatMulOp" and i not in self.given}
+        products = {i: found for i, found in products.items() if found}
+        for item, _, inside in products.values():
+            self.virtual |= inside
+        tails = {found[0].node for i, found in products.items() if found[0].node != i}
+        in_place = [i for i, n in enumerate(self.graph.nodes) if type(n.op).__name__ in ("KVAppendOp", "DecodeStepOp")]
+        for i, node in enumerate(self.graph.nodes):
+            name = type(node.op).__name__
+            if i in products:
+                item, x, _ = products[i]
+                # products on the same x join the first one's launch (their weights are inputs: nothing they read is
+                # computed in between, unless a node in between writes into its own inputs)
+                first = by_x.get(x)
+                if first and len(first[1].items) < binding.MATMUL_GROUP and not any(first[0] < p < i for p in in_place):
+                    step = ProjectionOp(x, first[1].items + [item])
+                    steps[steps.index(first[1])] = step
+                    by_x[x] = (first[0], step)
+                else:
+                    step = ProjectionOp(x, [item])
+                    steps.append(step)
+                    by_x[x] = (i, step)
+                continue
+            if i in self.virtual or i in self.given or i in tails or name == "InputTensor":
+                continue
+            if hasattr(node.op, "view"):
+                # the longest chain that ends here; a node that its own user will swallow waits for that user
+                user = self.users[i][0] if self.private[i] else None
+                if user is not None and hasattr(self.op(user), "view") and user not in self.given and self.swallows(i, user):
+                    continue
+                inside = set()
+                base, axes = self.base_view(node.inputs[0], inside)
+                axes = node.op.view(axes)
+                if axes is None:  # not affine over the whole chain: this node alone
+                    inside = set()
+                    base, axes = node.inputs[0], node.op.view(contiguous_view(node.inputs[0][2]))
+                if axes is not None and len(view_dims(axes)[0]) <= binding.MAP_DIMS:
+                    self.virtual |= inside
+                    steps.append(ViewOp(i, base, axes))
+                    continue
+            steps.append(NodeOp(i, node.inputs))
+        return steps
+
+    def swallows(self, i, user):
+        """Whether the chain of view nodes up to and including `user` is affine with node i inside it."""
+        inside = set()
+        base, axes = self.base_view(self.graph.nodes[user].inputs[0], inside)
+        return i in inside and self.op(user).view(axes) is not None
+
+
+def lower(graph, wanted=(), given=()):
+    """(steps, virtual): the launches that compute every node of `graph` that is `wanted` or has no or several users, in
+    order, and the nodes that disappeared into one of them. `given` nodes have values already."""
+    given = set(given)
+    if not any(hasattr(node.op, "compute") for node in graph.nodes):  # nothing around the attention nodes
+        return [NodeOp(i, node.inputs) for i, node in enumerate(graph.nodes)
+                if i not in given and type(node.op).__name__ != "InputTensor"], set()
+    work = _Lowering(graph, set(wanted), given)
+    steps = work.steps()
+    return steps, work.virtual
+
+
+class CopyList:
+    """The device-to-device copies of one call's inputs, as the ctypes arrays lmh_copy_many takes."""
+
+    def __init__(self, pairs):
+        n = len(pairs)
+        self.n = n
+        self.dst = (ctypes.c_void_p * n)(*[p[0] for p in pairs])
+        self.src = (ctypes.c_void_p * n)(*[p[1] for p in pairs])
+        self.nbytes = (ctypes.c_size_t * n)(*[p[2] for p in pairs])
+
+    def launch(self, stream=None):
+        binding.copy_many(self.dst, self.src, self.nbytes, self.n, stream)
+
+
+def copies_overlap(pairs):
+    """Whether any source range meets any destination range, or two destinations meet (then the copies need their order)."""
+    for i, (d, _, n) in enumerate(pairs):
+        for j, (d2, s2, n2) in enumerate(pairs):
+            if s2 < d + n and d < s2 + n2:
+                return True
+            if i != j and d2 < d + n and d < d2 + n2:
+                return True
+    return False

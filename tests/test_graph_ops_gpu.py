@@ -1,0 +1,111 @@
+"""The nodes around attention on the device: lmh_matmul, lmh_map and lmh_copy_many at the edges of their tiles, against
+float64 numpy and the reference's CPU semantics (HostOp.compute); and what a compiled graph does with nodes that
+disappeared into another node's launch."""
+import numpy as np
+import pytest
+
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _low(lm):
+    return lm.host.lowering
+
+
+# one case per form of the kernel (64 x 64, 32 x 64 and 32 x 32 tiles), each with remainders in every direction; the heads
+# split with rows that cross sequences inside a tile; operands that take the register path (K % 4, 16-bit types)
+@pytest.mark.parametrize("B,S,K,N,heads,dtype,bias", [
+    (1, 1, 4, 1, 0, "f32", False), (1, 33, 36, 65, 0, "f32", True), (1, 700, 132, 1024, 0, "f32", False),
+    (2, 1100, 64, 2100, 0, "f32", True), (3, 37, 68, 120, 5, "f32", True), (5, 7, 128, 64, 2, "f16", False),
+    (2, 129, 256, 320, 5, "bf16", True), (1, 50, 30, 70, 0, "f32", True), (1, 63, 2050, 33, 3, "f32", False),
+])
+def test_projection_matches_float64(lm, hip, oracle, B, S, K, N, heads, dtype, bias):
+    x, w = oracle.gen_normal((B, S, K), 31000 + S), oracle.gen_normal((N, K), 31100 + N, 1.0 / np.sqrt(K))
+    bv = oracle.gen_normal((N,), 31200)
+    dx, dw, db = (lm.to_device(a, hip) for a in (x, w, bv))
+    out = lm.HipArray((B, heads, S, N // heads) if heads else (B, S, N), dtype, hip)
+    p = (lm.binding.MatmulParams * 1)()
+    assert _low(lm).fill_matmul(p[0], out, dx, dw, transposed=True, bias=db if bias else None, heads=heads)
+    lm.binding.matmul(p, 1)
+    want = x.astype(np.float64) @ w.astype(np.float64).T + (bv if bias else 0)
+    if heads:
+        want = np.transpose(np.reshape(want, (B, S, heads, N // heads), order="F"), (0, 2, 1, 3))
+    assert rel_err(out.to_host(), want) <= {"f32": 2e-6, "f16": 5e-4, "bf16": 4e-3}[dtype]
+
+
+@pytest.mark.parametrize("a_shape,b_shape,dtypes", [
+    ((3, 40, 72), (3, 72, 50), ("f32", "f32")), ((40, 72), (5, 72, 64), ("f32", "f16")), ((2, 3, 33, 20), (20, 100), ("bf16", "f32")),
+])
+def test_batched_products_of_any_type(lm, hip, oracle, a_shape, b_shape, dtypes):
+    a, b = (oracle.round_to(oracle.gen_normal(s, 31300 + i), d) for i, (s, d) in enumerate(zip((a_shape, b_shape), dtypes)))
+    got = lm.execute_op(lm.MatMulOp(), lm.to_device(a, hip, dtypes[0]), lm.to_device(b, hip, dtypes[1])).to_host()
+    assert rel_err(got, np.matmul(a.astype(np.float64), b.astype(np.float64))) <= 2e-6
+
+
+@pytest.mark.parametrize("shape,ops", [
+    ((5,), [("expand", 0, 3)]), ((2, 70, 130), [("permute", 0, 2, 1)]), ((3, 65, 8, 9), [("permute", 0, 2, 1, 3), ("reshape", 3, 8, 585)]),
+    ((2, 6, 40), [("reshape", 2, 6, 8, 5), ("permute", 0, 2, 1, 3), ("permute", 0, 2, 1, 3), ("reshape", 2, 6, 40)]),
+    ((7, 11), [("reshape", 11, 7)]), ((1, 1, 64), [("permute", 2, 0, 1), ("expand", 3, 64)]),
+])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_chains_of_moved_elements(lm, hip, oracle, shape, ops, dtype):
+    g = lm.Graph()
+    x = lm.tensor(g, shape, dtype)
+    a = oracle.round_to(oracle.gen_normal(shape, 31400), dtype)
+    node, want = x, a
+    for kind, *args in ops:
+        node = {"permute": lambda: lm.permute(node, args), "reshape": lambda: lm.reshape(node, args), "expand": lambda: lm.expand(node, *args)}[kind]()
+        want = g.nodes[node.id].op.compute(want)
+    np.testing.assert_array_equal(lm.execute(g, node.id, {x.id: a}, hip), want)
+    b = oracle.gen_normal(want.shape[-1:], 31401)
+    got = lm.execute_op(lm.AddOp(), lm.to_device(want, hip), lm.to_device(b, hip)).to_host()
+    np.testing.assert_array_equal(got, want + b)
+
+
+@pytest.mark.parametrize("offset", [0, 4])
+def test_copies_of_every_length_in_one_launch(lm, hip, offset):
+    lengths = [1, 15, 16, 17, 16383, 16384, 16385, 40000, 3, 100]  # more than one launch's worth
+    rng = np.random.default_rng(5)
+    src = [rng.integers(0, 1 << 30, n + 8, dtype=np.int32) for n in lengths]
+    dev = [lm.to_device(s, hip) for s in src]
+    out = [lm.to_device(np.full(n + 8, -1, np.int32), hip) for n in lengths]
+    copies = _low(lm).CopyList([(o.ptr + offset, d.ptr + offset, n * 4 - (1 if n > 1 else 0)) for o, d, n in zip(out, dev, lengths)])
+    copies.launch()
+    for s, o, n in zip(src, out, lengths):
+        got, nbytes = o.to_host().view(np.uint8), n * 4 - (1 if n > 1 else 0)
+        want = np.full((n + 8) * 4, 255, np.uint8)
+        want[offset:offset + nbytes] = s.view(np.uint8)[offset:offset + nbytes]
+        np.testing.assert_array_equal(got, want)
+
+
+def test_a_node_inside_a_launch_is_computed_once_it_is_asked_for(lm, hip, oracle):
+    B, S, hidden, heads = 2, 20, 64, 4
+    g = lm.Graph()
+    x = lm.tensor(g, (B, S, hidden))
+    layer = lm.SelfAttention(hidden, heads, heads, g)
+    out = layer(x)
+    product = next(i for i, n in enumerate(g.nodes) if isinstance(n.op, lm.MatMulOp))
+    cg = lm.compile(g, hip)
+    ws = {p.weight.id: oracle.gen_normal((hidden, hidden), 31500 + i, 0.1) for i, p in
+          enumerate((layer.q_proj, layer.k_proj, layer.v_proj, layer.o_proj))}
+    first = cg({x.id: oracle.gen_normal((B, S, hidden), 31600), **ws})[out.id].to_host()
+    buffer = cg.results[product]  # handed out: kept up to date from here on
+    for seed in (31601, 31602):
+        xs = oracle.gen_normal((B, S, hidden), seed)
+        res = cg({x.id: lm.to_device(xs, hip)})
+        want = xs.astype(np.float64) @ ws[layer.q_proj.weight.id].astype(np.float64).T
+        assert rel_err(buffer.to_host(), want) <= 2e-6 and res[product] is buffer
+        np.testing.assert_array_equal(res[out.id].to_host(), lm.execute(g, out.id, {x.id: xs, **ws}, hip))
+    np.testing.assert_array_equal(cg({x.id: oracle.gen_normal((B, S, hidden), 31600)})[out.id].to_host(), first)
+
+
+def test_inputs_that_overlap_are_copied_in_their_order(lm, hip, oracle):
+    g = lm.Graph()
+    a, b = lm.tensor(g, (64,)), lm.tensor(g, (64,))
+    out = lm.add(a, b)
+    cg = lm.compile(g, hip)
+    va, vb = oracle.gen_normal((64,), 1), oracle.gen_normal((64,), 2)
+    cg({a.id: va, b.id: vb})
+    res = cg({a.id: cg.results[b.id], b.id: cg.results[a.id]})  # a takes b's values, then b takes a's new ones
+    np.testing.assert_array_equal(res[out.id].to_host(), vb + vb)
