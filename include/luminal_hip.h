@@ -122,8 +122,8 @@ int lmh_graph_destroy(void *graph_exec);
  * out[b,hq,i,:] = sum_j softmax_j(scale * q[b,hq,i,:] . k[b,kvh,j,:]) v[b,kvh,j,:]
  * with j restricted to j <= i when causal != 0 (the reference skips j > i,
  * src/Execution.jl:462), and to j < kv_len[b] when kv_len is non-null.
- * Head dims up to 256, like decode. The matrix-core kernels take multiples of 8 up to 128 (with 16-byte
- * aligned pointers and strides, scale > 0); everything else runs on a vector-ALU kernel with the same
+ * Head dims up to 256, like decode. The matrix-core kernels take multiples of 8 up to 128 and of 16 above (with
+ * 16-byte aligned pointers and strides, scale > 0); everything else runs on a vector-ALU kernel with the same
  * results at a fraction of the speed. ---- */
 typedef struct lmh_attn_params {
   void *out;          /* [B,Hq,Sq,D] device */
@@ -146,8 +146,8 @@ typedef struct lmh_attn_params {
    * (reference src/NN.jl:357, apply_rotary_embeddings :253-303), done on the rows as the kernel loads them instead of
    * by a launch of lmh_rope on q: row i of sequence b is rotated at position (q_pos0 ? q_pos0[b] : q_prev_seq) + i and
    * rounded to `dtype`, exactly what lmh_rope would have stored; q itself is not modified. K is not rotated here
-   * (lmh_kv_append rotates it on its way into a cache, lmh_rope anywhere else). D must be even; head dims 64, 96 and
-   * 128 keep the matrix-core kernels, any other runs on the vector-ALU kernel. Last in the struct so that
+   * (lmh_kv_append rotates it on its way into a cache, lmh_rope anywhere else). D must be even; head dims 64, 96,
+   * 128, 192 and 256 keep the matrix-core kernels, any other runs on the vector-ALU kernel. Last in the struct so that
    * zero-initialised params of earlier callers keep their meaning. */
   int32_t q_rope;         /* 0 / 1 */
   int32_t q_rope_pairing; /* LMH_ROPE_* */

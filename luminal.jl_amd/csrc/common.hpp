@@ -171,8 +171,8 @@ __host__ __device__ inline int q_head_of(int kvh, int g, int Hq, int Hkv, int he
 // Launchers: validate nothing (api.hip already did), pick an instantiation, enqueue on `stream`.
 // Return LMH_OK or LMH_E_UNSUPPORTED / LMH_E_HIP.
 // The matrix-core kernels rotate Q in registers, which needs the partner of every element in the same lane: head dims
-// that fill a tiling exactly (64, 96, 128).
-inline bool prefill_mfma_rope_ok(int D) { return D == 64 || D == 96 || D == 128; }
+// that fill a tiling exactly.
+inline bool prefill_mfma_rope_ok(int D) { return D == 64 || D == 96 || D == 128 || D == 192 || D == 256; }
 bool prefill_mfma_supported(int dtype, int D);
 int launch_prefill_mfma(const PrefillArgs &a, int dtype, hipStream_t stream);
 #ifdef LMH_W64_KERNEL

@@ -23,6 +23,10 @@ typedef short shortx4_t __attribute__((ext_vector_type(4)));
 __device__ inline void swap_wave_halves(float &a, float &b) {
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32_e32 %0, %1" : "+v"(a), "+v"(b));
 }
+// The same between neighbouring rows of 16 lanes: afterwards a holds the even rows' values and b the odd rows', on both rows.
+__device__ inline void swap_wave_rows(float &a, float &b) {
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32_e32 %0, %1" : "+v"(a), "+v"(b));
+}
 __device__ inline float max_over_wave_halves(float x) {
   float a = x, b = x;
   swap_wave_halves(a, b);  // a = the lower half's x on all lanes, b = the upper half's
@@ -34,15 +38,23 @@ __device__ inline float sum_over_wave_halves(float x) {
   return a + b;  // lower + upper on every lane: both halves get the same bits
 }
 
+// max / sum over the four lanes n, n + 16, n + 32, n + 48 (every one of them gets it)
+__device__ inline float max_over_wave_rows(float x) {
+  float a = x, b = x;
+  swap_wave_rows(a, b);
+  return max_over_wave_halves(fmaxf(a, b));
+}
+__device__ inline float sum_over_wave_rows(float x) {
+  float a = x, b = x;
+  swap_wave_rows(a, b);
+  return sum_over_wave_halves(a + b);
+}
+
 __device__ inline float bf16_bits_to_f32(uint32_t bits16) { return __uint_as_float(bits16 << 16); }
 
-// round-to-nearest-even, NaN kept quiet
-__device__ inline uint16_t f32_to_bf16_bits(float x) {
-  uint32_t u = __float_as_uint(x);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
+// round-to-nearest-even, NaN kept quiet: v_cvt_pk_bf16_f32, the same bits as the integer rounding it replaces for every
+// fp32 pattern (seven instructions per value there, half of one here)
+__device__ inline uint16_t f32_to_bf16_bits(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
 
 struct F32 {
   static constexpr const char *kName = "f32";

@@ -97,7 +97,7 @@ __device__ inline void rotate_q_fragments_with_table(typename MT::vec8 (&qreg)[D
 // and a wave's share of a tile is half as long.
 // The second launch bound is waves per SIMD.
 // WPS: waves per SIMD the register budget is set for (3 x 4 waves, 2 x 8 waves or 1 x 8 waves per CU).
-template <int D, int NW> constexpr int default_wps() { return D > 96 ? 2 : NW == 8 ? 4 : 3; }
+template <int D, int NW> constexpr int default_wps() { return D > 128 ? 1 : D > 96 ? 2 : NW == 8 ? 4 : 3; }
 template <typename MT, int D, bool CAUSAL, int KSPLIT, int NW, int WPS>
 __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(PrefillArgs a, int n_q_tiles, int n_bh_groups) {
   request_args(a);
@@ -1362,9 +1362,23 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
   return launch_split<MT, V16, D, 1, 4>(a, stream);
 }
 
+// Head dims above 128: Q and the accumulators of 32 rows take up to 192 registers and a tile buffer pair up to 141 KB, so a
+// workgroup of four waves, one per SIMD with all 512 registers, has the CU to itself; the long rows leave the softmax a
+// small share of a tile. Measured at D = 256 (the vector-ALU kernel that took these launches reaches 8 TFLOP/s): B=1 H=32
+// S=4096 causal fp16 332 us = 827 TFLOP/s, bf16 408 us = 674; B=1 H=16 S=1500 causal bf16 2310 -> 55 us, in 64-row
+// workgroups with two key groups, which small launches take as they do at the other head dims. bf16 keeps head + remainder
+// weights at every length: the registers of the fp16 rewrite of V spill here (S=4096: 633 us; D = 192, where they do not,
+// S=2048 200 against 187 us). The head dims that are odd multiples of 8 stay on the vector-ALU kernel.
+template <typename MT, int D>
+int launch_wide_heads(const PrefillArgs &a, hipStream_t stream) {
+  const int64_t wgs = (int64_t)((a.B * a.Hq + 7) / 8) * 8 * ((a.Sq + 127) / 128);
+  if (wgs <= device_cu_count() && a.Sk >= 4 * BN) return launch_split<MT, false, D, 2, 4>(a, stream);
+  return launch_split<MT, false, D, 1, 4>(a, stream);
+}
+
 template <typename MT>
 int launch_for_type(const PrefillArgs &a, hipStream_t stream) {
-  if (a.D > 128) return fail(LMH_E_UNSUPPORTED, "MFMA flash attention: head dim %d not tiled", a.D);
+  if (a.D > 256) return fail(LMH_E_UNSUPPORTED, "MFMA flash attention: head dim %d not tiled", a.D);
 #ifndef LMH_BF16_SPLIT_P
   if constexpr (MT::kSplitP) {
     // bf16: V as fp16 pays from about 512 keys per query row on. Its prologue (the first V tile through registers before
@@ -1373,7 +1387,7 @@ int launch_for_type(const PrefillArgs &a, hipStream_t stream) {
     // -13 ... 0 %; without a mask S=128 0 ... +30 %, S=256 -7 ... -1 %, S=512 -13 ... +5 %, S=1024 -5 ... -19 %. (The
     // D = 96 tiling, one workgroup per CU in this form, is the one that ties or loses at 512 keys per row: 1024 there.)
     const int64_t keys_per_row = a.causal ? (a.Sq < a.Sk ? a.Sq : a.Sk) / 2 : a.Sk;
-    if (keys_per_row >= (a.D > 64 && a.D <= 96 ? 1024 : 512)) {
+    if (a.D <= 128 && keys_per_row >= (a.D > 64 && a.D <= 96 ? 1024 : 512)) {
       if (a.D <= 64) return launch_for_d<MT, 64, true>(a, stream);
       if (a.D <= 96) return launch_for_d<MT, 96, true>(a, stream);
       return launch_for_d<MT, 128, true>(a, stream);
@@ -1383,13 +1397,15 @@ int launch_for_type(const PrefillArgs &a, hipStream_t stream) {
   // the smallest tiling that holds the head dim; the padding costs its share of the MFMAs
   if (a.D <= 64) return launch_for_d<MT, 64, false>(a, stream);
   if (a.D <= 96) return launch_for_d<MT, 96, false>(a, stream);
-  return launch_for_d<MT, 128, false>(a, stream);
+  if (a.D <= 128) return launch_for_d<MT, 128, false>(a, stream);
+  if (a.D <= 192) return launch_wide_heads<MT, 192>(a, stream);
+  return launch_wide_heads<MT, 256>(a, stream);
 }
 
 }  // namespace
 
 bool prefill_mfma_supported(int dtype, int D) {
-  return (dtype == LMH_F16 || dtype == LMH_BF16) && D >= 8 && D <= 128 && D % 8 == 0;
+  return (dtype == LMH_F16 || dtype == LMH_BF16) && D >= 8 && (D <= 128 ? D % 8 == 0 : D <= 256 && D % 16 == 0);
 }
 
 int launch_prefill_mfma(const PrefillArgs &a, int dtype, hipStream_t stream) {

@@ -16,7 +16,7 @@ constexpr int BN = 64;   // keys per staged tile (twice that in one instantiatio
 // 128, 8 at D + 8, 16 at a multiple of 128 bytes), in the kernel D = 64 measures the same with 0, 8,
 // 16 or 32 elements of padding, and 0 lets a fourth workgroup fit on a CU.
 constexpr int kPadK = 8;
-template <int D> constexpr int pad_v() { return D == 128 ? 32 : 0; }
+template <int D> constexpr int pad_v() { return D >= 128 ? 32 : 0; }
 constexpr float kLog2e = 1.4426950408889634f;
 // The running max is only raised (and the output rescaled) when a row's scores outgrow it by more
 // than this many powers of two; until then P is computed against the stale max and may reach

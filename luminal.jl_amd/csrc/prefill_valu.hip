@@ -1,6 +1,5 @@
-// Flash attention forward on the vector ALUs: the fp32 path (parity budget 1e-5, which rules
-// out half-precision matrix cores) and the fallback for head dims the MFMA kernels do not tile
-// (anything that is not a multiple of 8, and 129 .. 256, the range decode attention accepts too).
+// Flash attention forward on the vector ALUs: the fallback for what the MFMA kernels do not take (head dims that are not a
+// multiple of 8, above 128 of 16; unaligned tensors; scales that are not positive; slices beyond 2 GB).
 //
 // Same recurrence as flash_attn_cpu (reference src/Execution.jl:453-479), evaluated a tile of
 // 32 keys at a time: m' = max(m, tile max), o = o*exp(m-m') + sum_j exp(s_j-m') v_j,
