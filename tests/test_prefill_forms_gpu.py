@@ -1,0 +1,58 @@
+"""Flash attention at the edges of the fp32 kernel's forms and of the head dims above 128: every form is reached (the
+plan says so) with remainders of its row and key tiles, grouped heads and ragged keys, against the oracle."""
+import numpy as np
+import pytest
+
+from conftest import TOL, rel_err
+from test_fused_rope_gpu import inputs, plan, rotated_on_device, run
+
+pytestmark = pytest.mark.gpu
+
+NT = 16
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,form", [
+    (1, 2, 1, 33, 65, 16, False, "D=32, full, key groups=4> rows=16"), (1, 3, 3, 129, 70, 40, False, "D=48, full, key groups=4> rows=16"),
+    (2, 32, 8, 135, 131, 64, True, "D=64, causal, key groups=2> rows=32"), (2, 40, 8, 100, 65, 72, True, "D=80, causal, key groups=2> rows=32"),
+    (3, 32, 8, 500, 17, 80, False, "D=80, full, key groups=1> rows=64"), (3, 24, 24, 260, 100, 112, False, "D=112, full, key groups=1> rows=128"),
+    (8, 48, 16, 257, 33, 128, True, "D=128, causal, key groups=1> rows=128"), (1, 16, 4, 1100, 1100, 96, True, "D=96, causal, key groups=2> rows=32"), (1, 48, 4, 1100, 1100, 64, True, "D=64, causal, key groups=1> rows=64"),
+    (2, 20, 4, 637, 29, 256, False, "D=256, full, key groups=1> rows=64"),
+    (1, 4, 2, 100, 300, 144, True, "D=160, causal, key groups=2> rows=32"), (1, 2, 2, 1, 1, 192, False, "D=192, full, key groups=1> rows=64"),
+])
+def test_fp32_forms(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causal, form):
+    q, k, v = inputs(oracle, (B, Hq, Sq, D), (B, Hkv, Sk, D), "f32", 32000 + Sq + D)
+    assert "prefill_f32_kernel<" + form in plan(lm, q, k, "f32", causal, False)
+    lens = [max(1, Sk - 3 * i) for i in range(B)]
+    for kv_len in (None, lens):
+        got = run(lm, hip, q, k, v, "f32", causal, kv_len=kv_len)
+        want = oracle.flash_attn(q, k, v, causal=causal, kv_len=None if kv_len is None else np.array(lens, np.int32), nthreads=NT)
+        assert rel_err(got, want) <= TOL["f32"]
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("D", [144, 192, 208, 256])
+@pytest.mark.parametrize("Sq,Sk", [(1, 1), (33, 63), (64, 65), (129, 300), (300, 129)])
+def test_head_dims_above_128_on_the_matrix_cores(lm, hip, oracle, dtype, D, Sq, Sk):
+    q, k, v = inputs(oracle, (2, 6, Sq, D), (2, 2, Sk, D), dtype, 32500 + Sq + D)
+    lens = np.array([Sk, (Sk + 1) // 2], np.int32)
+    for causal in (False, True):
+        assert "prefill_valu_kernel" not in plan(lm, q, k, dtype, causal, False)
+        got = run(lm, hip, q, k, v, dtype, causal, kv_len=lens)
+        assert rel_err(got, oracle.flash_attn(q, k, v, causal=causal, kv_len=lens, nthreads=NT)) <= TOL[dtype]
+
+
+def test_large_launch_of_wide_heads(lm, hip, oracle):
+    # more 128-row workgroups than compute units: one key group
+    q, k, v = inputs(oracle, (3, 48, 260, 256), (3, 2, 300, 256), "bf16", 32900)
+    assert "key groups=1" in plan(lm, q, k, "bf16", True, False)
+    assert rel_err(run(lm, hip, q, k, v, "bf16", True), oracle.flash_attn(q, k, v, causal=True, nthreads=NT)) <= TOL["bf16"]
+
+
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("dtype,D", [("f16", 192), ("bf16", 256), ("f32", 192), ("f32", 256), ("f32", 64)])
+def test_wide_heads_rotate_their_queries_in_registers(lm, hip, oracle, dtype, D, interleaved):
+    q, k, v = inputs(oracle, (1, 4, 90, D), (1, 2, 90, D), dtype, 32950 + D)
+    assert plan(lm, q, k, dtype, True, True) == plan(lm, q, k, dtype, True, False)
+    got = run(lm, hip, q, k, v, dtype, True, rope=(7, interleaved))
+    q_rot = rotated_on_device(lm, hip, q, dtype, prev_seq=7, interleaved=interleaved)
+    np.testing.assert_array_equal(got, run(lm, hip, q_rot, k, v, dtype, True))
