@@ -86,6 +86,23 @@ int lmh_memcpy_h2d(void *dst_dev, const void *src_host, size_t bytes, void *stre
 int lmh_memcpy_d2h(void *dst_host, const void *src_dev, size_t bytes, void *stream);
 int lmh_memcpy_d2d(void *dst_dev, const void *src_dev, size_t bytes, void *stream);
 int lmh_sync(void *stream);
+/* Pinned host memory, and what it is for: host arrays to the device and back at the rate of PCIe, converted on the GPU.
+ * lmh_upload takes up to LMH_UPLOAD_ITEMS host arrays (pageable or not): with `convert` n fp32 values stored as `dtype`,
+ * otherwise n bytes as they are. The host memory may be reused when it returns; the device memory is written in the order of
+ * `stream` (lmh_memcpy_h2d waits for it, this does not). lmh_download enqueues n elements of type `dtype` -> fp32 in memory
+ * of lmh_host_alloc; lmh_sync says when they are there. Nothing of either may be recorded into a HIP graph. */
+#define LMH_UPLOAD_ITEMS 16
+typedef struct lmh_upload_item {
+  void *dst;
+  const void *src;
+  int64_t n;
+  int32_t dtype;
+  int32_t convert;
+} lmh_upload_item;
+int lmh_host_alloc(void **ptr, size_t bytes);
+int lmh_host_free(void *ptr);
+int lmh_upload(const lmh_upload_item *items, int32_t n, void *stream);
+int lmh_download(void *dst_pinned, const void *src_dev, int64_t n, int32_t dtype, void *stream);
 /* HIP-event timing on a stream (for benchmarks) */
 int lmh_event_create(void **event);
 int lmh_event_destroy(void *event);

@@ -28,6 +28,7 @@ EXPORTS = [
     "lmh_kv_append", "lmh_stream_create", "lmh_stream_destroy", "lmh_graph_capture_begin", "lmh_graph_capture_end",
     "lmh_graph_launch", "lmh_graph_destroy", "lmh_static_scratch_bytes", "lmh_decode_static_splits",
     "lmh_decode_attn_static", "lmh_decode_step_splits", "lmh_decode_step", "lmh_matmul", "lmh_map", "lmh_copy_many",
+    "lmh_host_alloc", "lmh_host_free", "lmh_upload", "lmh_download",
 ]
 
 
@@ -113,7 +114,11 @@ class MapParams(ctypes.Structure):
     ]
 
 
-MATMUL_GROUP, MAP_DIMS = 4, 8
+class UploadItem(ctypes.Structure):
+    _fields_ = [("dst", ctypes.c_void_p), ("src", ctypes.c_void_p), ("n", ctypes.c_int64), ("dtype", ctypes.c_int32), ("convert", ctypes.c_int32)]
+
+
+MATMUL_GROUP, MAP_DIMS, UPLOAD_ITEMS = 4, 8, 16
 
 # every symbol include/luminal_hip_calib.h declares (libluminal_hip_calib.so: measurement kernels, loaded on demand)
 CALIB_EXPORTS = ["lmh_calib_last_error", "lmh_calib_copy", "lmh_calib_read", "lmh_calib_mfma", "lmh_calib_mfma_xcds",
@@ -185,7 +190,11 @@ def load():
     L.lmh_matmul.argtypes = [ctypes.POINTER(MatmulParams), ctypes.c_int32, vp]
     L.lmh_map.argtypes = [ctypes.POINTER(MapParams), vp]
     L.lmh_copy_many.argtypes = [ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(ctypes.c_size_t), ctypes.c_int32, vp]
-    for name in ("lmh_matmul", "lmh_map", "lmh_copy_many", "lmh_rope", "lmh_kv_append", "lmh_init", "lmh_device_name", "lmh_malloc", "lmh_free", "lmh_memset", "lmh_memcpy_h2d",
+    L.lmh_host_alloc.argtypes = [ctypes.POINTER(vp), ctypes.c_size_t]
+    L.lmh_host_free.argtypes = [vp]
+    L.lmh_upload.argtypes = [ctypes.POINTER(UploadItem), ctypes.c_int32, vp]
+    L.lmh_download.argtypes = [vp, vp, ctypes.c_int64, ctypes.c_int32, vp]
+    for name in ("lmh_host_alloc", "lmh_host_free", "lmh_upload", "lmh_download", "lmh_matmul", "lmh_map", "lmh_copy_many", "lmh_rope", "lmh_kv_append", "lmh_init", "lmh_device_name", "lmh_malloc", "lmh_free", "lmh_memset", "lmh_memcpy_h2d",
                  "lmh_memcpy_d2h", "lmh_memcpy_d2d", "lmh_sync", "lmh_event_create", "lmh_event_destroy",
                  "lmh_event_record", "lmh_event_elapsed_ms", "lmh_flash_attn_fwd", "lmh_decode_attn"):
         getattr(L, name).restype = ctypes.c_int
@@ -259,6 +268,28 @@ def memcpy_h2d(dst, src_host_ptr, nbytes, stream=None):
 
 def memcpy_d2h(dst_host_ptr, src, nbytes, stream=None):
     check(load().lmh_memcpy_d2h(dst_host_ptr, src, nbytes, stream))
+
+
+def host_alloc(nbytes):
+    """Pinned host memory; the address."""
+    p = ctypes.c_void_p()
+    check(load().lmh_host_alloc(ctypes.byref(p), nbytes))
+    return p.value or 0
+
+
+def host_free(ptr):
+    check(load().lmh_host_free(ptr))
+
+
+def upload(items, stream=None):
+    """items: (device address, host address, n, dtype code, convert) per host array; see lmh_upload."""
+    for first in range(0, len(items), UPLOAD_ITEMS):
+        part = items[first:first + UPLOAD_ITEMS]
+        check(load().lmh_upload((UploadItem * len(part))(*part), len(part), stream))
+
+
+def download(dst_pinned, src, n, dtype_code, stream=None):
+    check(load().lmh_download(dst_pinned, src, n, dtype_code, stream))
 
 
 def memcpy_d2d(dst, src, nbytes, stream=None):

@@ -20,7 +20,7 @@ LIBNAME = "libluminal_hip.so"
 CALIB_LIBNAME = "libluminal_hip_calib.so"
 LIBRARIES = {
     LIBNAME: ["api.hip", "prefill_valu.hip", "prefill_mfma.hip", "prefill_f32.hip", "decode.hip",
-              "decode_mfma.hip", "cache_ops.hip", "matmul.hip", "map_ops.hip"],
+              "decode_mfma.hip", "cache_ops.hip", "matmul.hip", "map_ops.hip", "staging.hip"],
     CALIB_LIBNAME: ["calib.hip"],
 }
 

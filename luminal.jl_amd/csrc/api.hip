@@ -271,6 +271,45 @@ int lmh_sync(void *stream) {
   return LMH_OK;
 }
 
+int lmh_host_alloc(void **ptr, size_t bytes) {
+  if (!ptr) return fail(LMH_E_NULL, "lmh_host_alloc: null result pointer");
+  *ptr = nullptr;
+  if (bytes == 0) return LMH_OK;
+  LMH_HIP_TRY(hipHostMalloc(ptr, bytes, hipHostMallocDefault));
+  return LMH_OK;
+}
+
+int lmh_host_free(void *ptr) {
+  if (!ptr) return LMH_OK;
+  LMH_HIP_TRY(hipHostFree(ptr));
+  return LMH_OK;
+}
+
+int lmh_upload(const lmh_upload_item *items, int32_t n, void *stream) {
+  if (n < 0 || n > LMH_UPLOAD_ITEMS) return fail(LMH_E_SHAPE, "lmh_upload: %d arrays, up to %d fit a call", n, LMH_UPLOAD_ITEMS);
+  if (n > 0 && !items) return fail(LMH_E_NULL, "lmh_upload: null list");
+  UploadItem out[LMH_UPLOAD_ITEMS];
+  for (int i = 0; i < n; i++) {
+    if (items[i].n < 0) return fail(LMH_E_SHAPE, "lmh_upload: negative length");
+    if (items[i].n > 0 && (!items[i].dst || !items[i].src)) return fail(LMH_E_NULL, "lmh_upload: null pointer");
+    if (items[i].convert && items[i].dtype != LMH_F32 && items[i].dtype != LMH_F16 && items[i].dtype != LMH_BF16)
+      return fail(LMH_E_UNSUPPORTED, "lmh_upload: unknown element type %d", items[i].dtype);
+    out[i].dst = items[i].dst;
+    out[i].src = items[i].src;
+    out[i].bytes = (size_t)items[i].n * (items[i].convert ? 4 : 1);
+    out[i].dtype = items[i].convert && items[i].dtype != LMH_F32 ? items[i].dtype : -1;
+  }
+  return launch_upload(out, n, (hipStream_t)stream);
+}
+
+int lmh_download(void *dst_pinned, const void *src_dev, int64_t n, int32_t dtype, void *stream) {
+  if (n < 0) return fail(LMH_E_SHAPE, "lmh_download: negative length");
+  if (n == 0) return LMH_OK;
+  if (!dst_pinned || !src_dev) return fail(LMH_E_NULL, "lmh_download: null pointer");
+  if (dtype != LMH_F32 && dtype != LMH_F16 && dtype != LMH_BF16) return fail(LMH_E_UNSUPPORTED, "lmh_download: unknown element type %d", dtype);
+  return launch_download(reinterpret_cast<float *>(dst_pinned), src_dev, n, dtype, (hipStream_t)stream);
+}
+
 int lmh_stream_create(void **stream) {
   if (!stream) return fail(LMH_E_NULL, "lmh_stream_create: null result pointer");
   hipStream_t s;

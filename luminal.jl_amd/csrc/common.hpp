@@ -134,6 +134,15 @@ struct CopyManyArgs {
   int32_t first_block[kCopyMany];
 };
 
+// One host array of an upload (staging.hip): `bytes` source bytes; dtype -1 moves them as they are, an element type makes it
+// of fp32 values.
+struct UploadItem {
+  void *dst;
+  const void *src;
+  size_t bytes;
+  int dtype;
+};
+
 // Every field of a launch-argument block, requested from memory in one batch at the kernel's start (a kernel calls this first).
 // Left to the compiler, the scalar loads of these 100 to 230 byte blocks are issued where their values are first needed: in the
 // attention kernels five and more round trips to memory, one after the other, before a wave has issued its first tile load
@@ -189,6 +198,8 @@ int launch_kv_append(const KvAppendArgs &a, int dtype, hipStream_t stream);
 int launch_matmul(MatmulArgs &args, int n, hipStream_t stream);
 int launch_map(MapArgs &a, hipStream_t stream);
 int launch_copy_many(CopyManyArgs &a, int n, hipStream_t stream);
+int launch_upload(const UploadItem *items, int n, hipStream_t stream);
+int launch_download(float *dst_pinned, const void *src, int64_t n, int dtype, hipStream_t stream);
 bool decode_mfma_supported(int dtype, int D, int B);
 bool decode_mfma_rope_ok(int D, int interleaved);
 int launch_decode_mfma_split(const DecodeArgs &a, int dtype, hipStream_t stream);
