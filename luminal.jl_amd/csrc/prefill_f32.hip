@@ -37,14 +37,11 @@ constexpr int kOutOfRange = 0x7ffffff0;   // byte offset no K/V slice reaches: a
 constexpr float kLazyRescale = 8.0f;      // the running max is raised only when outgrown by 2^8 (see prefill_mfma.hpp)
 
 // RW waves own 16 rows each, KG waves share 16 rows by taking the kg-th 16 NK keys of every staged tile of 16 NK KG keys.
-// snake: see launch_form.
 template <int D, int RW, int KG, int NK> constexpr int tile_blocks() { return (16 * NK * KG * (D / 4 + 1) + 63) / 64; }  // 1 KB blocks
 template <int D, bool CAUSAL, int RW, int KG, int NK>
-__global__ __launch_bounds__(64 * RW * KG, 1) void prefill_f32_kernel(PrefillArgs a, int n_q_tiles, int n_bh_groups, int snake) {
+__global__ __launch_bounds__(64 * RW * KG, 1) void prefill_f32_kernel(PrefillArgs a, Deal deal) {
   request_args(a);
-  request_arg(n_q_tiles);
-  request_arg(n_bh_groups);
-  request_arg(snake);
+  request_args(deal);
   constexpr int NW = RW * KG;
   constexpr int BM = 16 * RW;            // query rows per workgroup
   constexpr int BW = 16 * NK;            // keys a wave takes per tile
@@ -57,19 +54,11 @@ __global__ __launch_bounds__(64 * RW * KG, 1) void prefill_f32_kernel(PrefillArg
   __shared__ __attribute__((aligned(16))) float Vs2[2][BLOCKS * 256];
 
   // ---- which (b, hq, query tile): a head's tiles on one XCD, causal tiles heaviest first (see prefill_mfma.hip) ----
-  const int bid = blockIdx.x;
-  const int xcd = bid & 7;
-  int idx = bid >> 3;
-  if (snake && (idx / snake) & 1) {
-    const int first = idx / snake * snake, last = min(first + snake, n_q_tiles * n_bh_groups) - 1;
-    idx = first + last - idx;
-  }
-  const int tile_rank = idx / n_bh_groups;
-  const int bh = (idx % n_bh_groups) * 8 + xcd;
-  if (bh >= a.B * a.Hq) return;
-  const int b = bh / a.Hq, hq = bh % a.Hq;
+  int bh, tile_rank;
+  if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3, &bh, &tile_rank)) return;
+  const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
-  const int q_tile = CAUSAL ? (n_q_tiles - 1 - tile_rank) : tile_rank;
+  const int q_tile = CAUSAL ? (deal.tiles - 1 - tile_rank) : tile_rank;
   const int q0 = q_tile * BM;
 
   const int tid = threadIdx.x;
@@ -321,21 +310,16 @@ template <int D, int RW, int KG, int NK> constexpr int resident() {  // workgrou
   return by_lds < 1 ? 1 : by_lds < by_waves ? by_lds : by_waves;
 }
 
-// Causal workgroups are issued heaviest first. Where all of them are resident at once nothing balances them afterwards: a CU
-// keeps the ones it was dealt, the k-th of every round. Such launches deal every other round in the opposite order (`snake`
-// = CUs of an XCD), so that the heaviest shares its CU with the lightest. B=1 H=16 S=2048 D=128 in 64-row workgroups 218 ->
-// 179 us, H=32 in 128-row ones 368 -> 283 us.
+// (dealing backwards: B=1 H=16 S=2048 D=128 causal in 64-row workgroups 218 -> 179 us, H=32 in 128-row ones 368 -> 283 us)
 template <int D, int RW, int KG, int NK>
 int launch_form(const PrefillArgs &a, hipStream_t stream) {
   const int n_q_tiles = (a.Sq + 16 * RW - 1) / (16 * RW);
-  const int n_bh_groups = (a.B * a.Hq + 7) / 8;
-  dim3 grid(8 * n_bh_groups * n_q_tiles), block(64 * RW * KG);
+  dim3 grid(deal_grid(a.B * a.Hq, n_q_tiles)), block(64 * RW * KG);
   if (plan_only("prefill_f32_kernel<D=%d, %s, key groups=%d> rows=%d, workgroups=%u", D, a.causal ? "causal" : "full", KG, 16 * RW, grid.x))
     return LMH_OK;
-  const int n_cus = device_cu_count();
-  const int snake = (int)grid.x <= resident<D, RW, KG, NK>() * n_cus ? n_cus / 8 : 0;
-  if (a.causal) hipLaunchKernelGGL((prefill_f32_kernel<D, true, RW, KG, NK>), grid, block, 0, stream, a, n_q_tiles, n_bh_groups, snake);
-  else hipLaunchKernelGGL((prefill_f32_kernel<D, false, RW, KG, NK>), grid, block, 0, stream, a, n_q_tiles, n_bh_groups, 0);
+  const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? resident<D, RW, KG, NK>() : 0);
+  if (a.causal) hipLaunchKernelGGL((prefill_f32_kernel<D, true, RW, KG, NK>), grid, block, 0, stream, a, deal);
+  else hipLaunchKernelGGL((prefill_f32_kernel<D, false, RW, KG, NK>), grid, block, 0, stream, a, deal);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }

@@ -99,10 +99,9 @@ __device__ inline void rotate_q_fragments_with_table(typename MT::vec8 (&qreg)[D
 // WPS: waves per SIMD the register budget is set for (3 x 4 waves, 2 x 8 waves or 1 x 8 waves per CU).
 template <int D, int NW> constexpr int default_wps() { return D > 128 ? 1 : D > 96 ? 2 : NW == 8 ? 4 : 3; }
 template <typename MT, int D, bool CAUSAL, int KSPLIT, int NW, int WPS>
-__global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(PrefillArgs a, int n_q_tiles, int n_bh_groups) {
+__global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(PrefillArgs a, Deal deal) {
   request_args(a);
-  request_arg(n_q_tiles);
-  request_arg(n_bh_groups);
+  request_args(deal);
   using vec8 = typename MT::vec8;
   constexpr int BM = 32 * NW / KSPLIT;  // query rows per workgroup
   // keys per staged tile: 64; 128 where one workgroup has the CU to itself and LDS and registers allow (half the
@@ -130,18 +129,14 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(PrefillArgs 
   if ((blockIdx.x & 7) >= LMH_ONLY_XCDS) return;
 #endif
   // ---- which (b, hq, query tile) this workgroup owns ----
-  const int bid = blockIdx.x;
-  const int xcd = bid & 7;
-  const int idx = bid >> 3;
-  const int tile_rank = idx / n_bh_groups;
-  const int bh = (idx % n_bh_groups) * 8 + xcd;
-  if (bh >= a.B * a.Hq) return;
-  const int b = bh / a.Hq, hq = bh % a.Hq;
+  int bh, tile_rank;
+  if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3, &bh, &tile_rank)) return;
+  const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
   // Causal rows grow with the query index: long rows are issued first so that the short ones fill
   // the tail of the launch. (Pairing tile r with tile n-1-r in one workgroup equalises the work but
   // halves the number of workgroups; measured 15 % slower on the S = 4096 workload.)
-  const int q_tile = CAUSAL ? (n_q_tiles - 1 - tile_rank) : tile_rank;
+  const int q_tile = CAUSAL ? (deal.tiles - 1 - tile_rank) : tile_rank;
   const int q0 = q_tile * BM;
 
   const int tid = threadIdx.x;
@@ -583,10 +578,10 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(PrefillArgs 
 // 37.4 us on the 64-row workgroups -> 32.7 us here).
 constexpr int kWideMaxKeyGroups = 6;  // tiles of up to 192 keys: two buffers of them fit the LDS at D = 96
 template <typename MT, int D>
-__global__ __launch_bounds__(1024, 4) void prefill_mfma_wide_kernel(PrefillArgs a, int wgs_per_head, int n_bh_groups, int mixed) {
+__global__ __launch_bounds__(1024, 4) void prefill_mfma_wide_kernel(PrefillArgs a, int wgs_per_head, int n_whole, int mixed) {
   request_args(a);
   request_arg(wgs_per_head);
-  request_arg(n_bh_groups);
+  request_arg(n_whole);
   request_arg(mixed);
   using vec8 = typename MT::vec8;
   constexpr int KS = D / 16, DB = D / 32;
@@ -604,11 +599,8 @@ __global__ __launch_bounds__(1024, 4) void prefill_mfma_wide_kernel(PrefillArgs 
   static_assert(sizeof(lds) <= 160 * 1024, "LDS of a CU");
 
   const int cpr = a.D / 8;
-  const int bid = blockIdx.x;
-  const int xcd = bid & 7, idx = bid >> 3;
-  const int j_wg = idx % wgs_per_head;
-  const int bh = (idx / wgs_per_head) * 8 + xcd;
-  if (bh >= a.B * a.Hq) return;
+  int bh, j_wg;
+  if (!deal_tile_by_head(a.B * a.Hq, wgs_per_head, n_whole, blockIdx.x & 7, blockIdx.x >> 3, &bh, &j_wg)) return;
   const int b = bh / a.Hq, hq = bh % a.Hq;
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
   // row blocks of this workgroup: the head's ceil(Sq / 32) blocks dealt evenly to its workgroups
@@ -846,10 +838,10 @@ __global__ __launch_bounds__(1024, 4) void prefill_mfma_wide_kernel(PrefillArgs 
 // Without a mask (CAUSAL = false) the two tiles are neighbours — a 512-row tile — and share every fragment to the end.
 // ---------------------------------------------------------------------------------------------------------------
 template <typename MT, int D, bool CAUSAL>
-__global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a, int n_q_tiles, int n_bh_groups) {
+__global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a, Deal deal, int n_q_tiles) {
   request_args(a);
+  request_args(deal);
   request_arg(n_q_tiles);
-  request_arg(n_bh_groups);
   using vec8 = typename MT::vec8;
   static_assert(!MT::kSplitP && !MT::kConvertV, "one weight fragment per V fragment, V tiles staged as they are: fp16");
   constexpr int NW = 8, BM = 256;
@@ -862,12 +854,9 @@ __global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a
   __shared__ __attribute__((aligned(16))) uint16_t Ks2[2][BT * LDK];
   __shared__ __attribute__((aligned(16))) uint16_t Vs2[2][BT * LDV];
 
-  const int bid = blockIdx.x;
-  const int xcd = bid & 7, idx = bid >> 3;
-  const int pair = idx / n_bh_groups;
-  const int bh = (idx % n_bh_groups) * 8 + xcd;
-  if (bh >= a.B * a.Hq) return;
-  const int b = bh / a.Hq, hq = bh % a.Hq;
+  int bh, pair;
+  if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3, &bh, &pair)) return;
+  const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
   // tile p with tile n - 1 - p; with an odd number of tiles the middle one is alone (its workgroup has no early tile)
   // (without a mask: two neighbouring tiles; the second one, row block 0 here, is missing at an odd end)
@@ -1206,13 +1195,13 @@ template <typename MT, int D>
 int launch_pair(const PrefillArgs &a, hipStream_t stream) {
   const int n_q_tiles = (a.Sq + 255) / 256;
   const int n_pairs = (n_q_tiles + 1) / 2;
-  const int n_bh_groups = (a.B * a.Hq + 7) / 8;
-  dim3 grid(8 * n_bh_groups * n_pairs), block(512);
+  dim3 grid(deal_grid(a.B * a.Hq, n_pairs)), block(512);
   if (plan_only("prefill_mfma_pair_kernel<%s, D=%d, %s> query tiles=%d, workgroups=%u", MT::kName, D, a.causal ? "causal" : "full", n_q_tiles, grid.x)) return LMH_OK;
+  const Deal deal = make_deal(a.B, a.Hq, n_pairs, 0);
   if (a.causal)
-    hipLaunchKernelGGL((prefill_mfma_pair_kernel<MT, D, true>), grid, block, 0, stream, a, n_q_tiles, n_bh_groups);
+    hipLaunchKernelGGL((prefill_mfma_pair_kernel<MT, D, true>), grid, block, 0, stream, a, deal, n_q_tiles);
   else
-    hipLaunchKernelGGL((prefill_mfma_pair_kernel<MT, D, false>), grid, block, 0, stream, a, n_q_tiles, n_bh_groups);
+    hipLaunchKernelGGL((prefill_mfma_pair_kernel<MT, D, false>), grid, block, 0, stream, a, deal, n_q_tiles);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }
@@ -1229,15 +1218,15 @@ int launch_split(const PrefillArgs &a, hipStream_t stream) {
   using MT = typename base_policy<MT0, V16, KSPLIT>::type;
   constexpr int BM = 32 * NW / KSPLIT;
   const int n_q_tiles = (a.Sq + BM - 1) / BM;
-  const int n_bh_groups = (a.B * a.Hq + 7) / 8;
-  dim3 grid(8 * n_bh_groups * n_q_tiles), block(64 * NW);
+  dim3 grid(deal_grid(a.B * a.Hq, n_q_tiles)), block(64 * NW);
   if (plan_only("prefill_mfma_kernel<%s, D=%d, %s, key groups=%d, waves=%d, waves per SIMD=%d> workgroups=%u%s", MT::kName, D,
                 a.causal ? "causal" : "full", KSPLIT, NW, WPS, grid.x, MT::kConvertV ? ", V as fp16" : ""))
     return LMH_OK;
+  const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? 4 * WPS / NW : 0);
   if (a.causal)
-    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS>), grid, block, 0, stream, a, n_q_tiles, n_bh_groups);
+    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS>), grid, block, 0, stream, a, deal);
   else
-    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, false, KSPLIT, NW, WPS>), grid, block, 0, stream, a, n_q_tiles, n_bh_groups);
+    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, false, KSPLIT, NW, WPS>), grid, block, 0, stream, a, deal);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }
@@ -1248,10 +1237,10 @@ int launch_split(const PrefillArgs &a, hipStream_t stream) {
 // wide against 64-row workgroups): load 1.33 vs 1.5 -12 % (D = 64), -14 % (D = 96); 0.75 vs 1.0 -7 ... -12 %; equal loads
 // +-2 %, and +7 % at 1024 keys; under about 500 keys the single prologue per CU costs more than the balance wins.
 inline bool wide_plan(const PrefillArgs &a, int n_cus, int *wgs_per_head, int *n_waves, int *mixed) {
-  const int heads = a.B * a.Hq, heads8 = (heads + 7) / 8 * 8;
+  const int heads = a.B * a.Hq;
   const int n_blocks = (a.Sq + 31) / 32;
-  if (a.causal || heads8 > n_cus || n_blocks < 2 || a.Sk < 640) return false;
-  const int w = max(1, min(n_cus / heads8, n_blocks / 2));
+  if (a.causal || heads > n_cus || n_blocks < 2 || a.Sk < 640) return false;
+  const int w = max(1, min(n_cus / heads, n_blocks / 2));
   const int r_max = (n_blocks + w - 1) / w;
   if (r_max > 8) return false;
   int best_kg = 0;
@@ -1269,7 +1258,7 @@ inline bool wide_plan(const PrefillArgs &a, int n_cus, int *wgs_per_head, int *n
 #endif
   if (!best_kg && !*mixed) return false;
   // the equal 64-row workgroups, wave pairs splitting the keys: up to three resident on a CU, half a block's keys a wave
-  const int64_t n64 = (int64_t)heads8 * ((a.Sq + 63) / 64);
+  const int64_t n64 = (int64_t)heads * ((a.Sq + 63) / 64);
   const double load_now = 0.5 * (double)((n64 + n_cus - 1) / n_cus);
   if (best > LMH_WIDE_MARGIN * load_now) return false;
   *wgs_per_head = w;
@@ -1279,12 +1268,11 @@ inline bool wide_plan(const PrefillArgs &a, int n_cus, int *wgs_per_head, int *n
 
 template <typename MT, int D>
 int launch_wide(const PrefillArgs &a, int wgs_per_head, int n_waves, int mixed, hipStream_t stream) {
-  const int n_bh_groups = (a.B * a.Hq + 7) / 8;
-  dim3 grid(8 * n_bh_groups * wgs_per_head), block(64 * n_waves);
+  dim3 grid(deal_grid(a.B * a.Hq, wgs_per_head)), block(64 * n_waves);
   if (plan_only("prefill_mfma_wide_kernel<%s, D=%d> workgroups per head=%d, waves=%d, workgroups=%u%s", MT::kName, D, wgs_per_head,
                 n_waves, grid.x, mixed ? ", two and four key groups" : ""))
     return LMH_OK;
-  hipLaunchKernelGGL((prefill_mfma_wide_kernel<MT, D>), grid, block, 0, stream, a, wgs_per_head, n_bh_groups, mixed);
+  hipLaunchKernelGGL((prefill_mfma_wide_kernel<MT, D>), grid, block, 0, stream, a, wgs_per_head, a.B * a.Hq / 8 * wgs_per_head, mixed);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }
@@ -1309,18 +1297,18 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
   // plus the rewrite's registers do not fit; this kernel is built for fp16 only.
 #ifndef LMH_NO_PAIR_KERNEL  // (measurement builds can keep these launches on the kernels below, for comparisons with them)
   if constexpr (D <= 96 && !MT::kSplitP) {
-    const int64_t wgs_pair = (int64_t)((a.B * a.Hq + 7) / 8) * 8 * (((a.Sq + 255) / 256 + 1) / 2);
+    const int64_t wgs_pair = (int64_t)a.B * a.Hq * (((a.Sq + 255) / 256 + 1) / 2);
     if (a.causal && a.Sq > 256 && wgs_pair <= n_cus && 16 * wgs_pair >= 15 * n_cus) return launch_pair<MT, D>(a, stream);
     // Without a mask the same kernel takes two neighbouring tiles (512 rows, every fragment read shared all the way);
     // its workgroups are equal, so it wants whole rounds: B=1 H=32 S=4096 D=96 (one round) -5.9 %, S=8192 (two) -3.5 %,
     // B=4 (four) -1.1 %; D=64 one round -2.4 %, two rounds +2.5 %; 1.25 rounds +20 %.
-    if (!a.causal && a.Sq > 256 && wgs_pair >= n_cus) {
+    if (!a.causal && a.Sq > 256) {
       const int64_t rounds = (wgs_pair + n_cus - 1) / n_cus, last = wgs_pair - (rounds - 1) * n_cus;
       if (16 * last >= 15 * n_cus && (rounds == 1 || (D > 64 && rounds <= 2))) return launch_pair<MT, D>(a, stream);
     }
   }
 #endif
-  const int64_t wgs = (int64_t)((a.B * a.Hq + 7) / 8) * 8 * ((a.Sq + 127) / 128);
+  const int64_t wgs = (int64_t)a.B * a.Hq * ((a.Sq + 127) / 128);
   const int64_t limit = a.causal ? 2 * n_cus : 2 * n_cus - 1;
   if (wgs <= limit && a.Sk >= 4 * BN) {
     if constexpr (D <= 96) {
@@ -1336,7 +1324,7 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
   // which turns over in rounds and balances earlier. fp16: non-causal 256 / 512 / 2048 workgroups +5 / +3 / +6 %,
   // causal 256 / 384 -8 / -5 %, 512 / 1024 / 2048 +8 / +3 / +4 %; bf16 (V rewritten as fp16) 512 workgroups causal
   // +8 %, without a mask +5 %, 2048 causal +5 %.
-  const int64_t wgs256 = (int64_t)((a.B * a.Hq + 7) / 8) * 8 * ((a.Sq + 255) / 256);
+  const int64_t wgs256 = (int64_t)a.B * a.Hq * ((a.Sq + 255) / 256);
   if (a.Sq <= 128) return launch_split<MT, V16, D, 1, 4>(a, stream);  // nothing for waves 4-7 to own
   if constexpr (D <= 96) {
     // Causal launches of 1.5 to 3 rounds of one 256-row workgroup per CU (the Phi-3 prompt, 32 heads x 4096 rows,
@@ -1371,7 +1359,7 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
 // S=2048 200 against 187 us). The head dims that are odd multiples of 8 stay on the vector-ALU kernel.
 template <typename MT, int D>
 int launch_wide_heads(const PrefillArgs &a, hipStream_t stream) {
-  const int64_t wgs = (int64_t)((a.B * a.Hq + 7) / 8) * 8 * ((a.Sq + 127) / 128);
+  const int64_t wgs = (int64_t)a.B * a.Hq * ((a.Sq + 127) / 128);
   if (wgs <= device_cu_count() && a.Sk >= 4 * BN) return launch_split<MT, false, D, 2, 4>(a, stream);
   return launch_split<MT, false, D, 1, 4>(a, stream);
 }

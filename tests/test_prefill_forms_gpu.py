@@ -56,3 +56,16 @@ def test_wide_heads_rotate_their_queries_in_registers(lm, hip, oracle, dtype, D,
     got = run(lm, hip, q, k, v, dtype, True, rope=(7, interleaved))
     q_rot = rotated_on_device(lm, hip, q, dtype, prev_seq=7, interleaved=interleaved)
     np.testing.assert_array_equal(got, run(lm, hip, q_rot, k, v, dtype, True))
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,dtype,kernel", [
+    (1, 1, 1, 1000, 1000, 64, True, "f16", "key groups=2"), (1, 11, 11, 4096, 4096, 64, True, "f16", "prefill_mfma_kernel"),
+    (1, 42, 42, 3000, 3000, 96, True, "f16", "prefill_mfma_pair_kernel"), (1, 50, 50, 448, 704, 64, False, "bf16", "prefill_mfma_wide_kernel"),
+    (3, 7, 7, 700, 700, 128, True, "bf16", "prefill_mfma_kernel"), (1, 15, 5, 900, 900, 64, True, "f32", "prefill_f32_kernel"),
+])
+def test_head_counts_that_are_no_multiple_of_the_xcds(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causal, dtype, kernel):
+    """The tiles of the heads beyond a multiple of eight go round the XCDs: every tile of every head is computed, also in
+    launches that deal every other round backwards."""
+    q, k, v = inputs(oracle, (B, Hq, Sq, D), (B, Hkv, Sk, D), dtype, 33000 + Sq + Hq)
+    assert kernel in plan(lm, q, k, dtype, causal, False)
+    assert rel_err(run(lm, hip, q, k, v, dtype, causal), oracle.flash_attn(q, k, v, causal=causal, nthreads=NT)) <= TOL[dtype]
