@@ -24,6 +24,7 @@
 //     lie entirely above its diagonal, and only diagonal tiles pay for masking;
 //   * blockIdx -> work mapping keeps all query tiles of a head on one XCD (private L2) and, for
 //     causal, issues the long rows first.
+#include <algorithm>
 #include <type_traits>
 
 #include "prefill_mfma.hpp"
@@ -94,7 +95,8 @@ __device__ inline void rotate_q_fragments_with_table(typename MT::vec8 (&qreg)[D
 // KSPLIT = 2: for launches too small to fill the chip. The workgroup owns 64 query rows; waves 0-1
 // take them against the first 32 keys of every tile, waves 2-3 against the second 32, each pair
 // with its own running max / sum / output, merged through LDS at the end. Twice the workgroups,
-// and a wave's share of a tile is half as long.
+// and a wave's share of a tile is half as long. With NW = 8 (head dims above 128) the workgroup owns 128 rows: the two
+// waves of a SIMD hide each other's LDS latency.
 // The second launch bound is waves per SIMD.
 // WPS: waves per SIMD the register budget is set for (3 x 4 waves, 2 x 8 waves or 1 x 8 waves per CU).
 template <int D, int NW> constexpr int default_wps() { return D > 128 ? 1 : D > 96 ? 2 : NW == 8 ? 4 : 3; }
@@ -388,16 +390,22 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(PrefillArgs 
 #pragma unroll
       for (int i = 0; i < 16; i++) sacc[kb][i] = 0.f;
     constexpr int KBG = NKB < 2 ? NKB : 2;  // key blocks whose fragments are fetched together
+    constexpr int KSG = D <= 128 ? KS : WPS == 2 ? 4 : KS / 2;  // ... and k-steps (long rows: what the registers hold)
 #pragma unroll
-    for (int kb0 = 0; kb0 < NKB; kb0 += KBG) {
+    for (int kb0 = 0; kb0 < NKB; kb0 += KBG)
+#pragma unroll
+    for (int ks0 = 0; ks0 < KS; ks0 += KSG) {
       vec8 kf[KBG][KS];
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++)
+      for (int ks = ks0; ks < ks0 + KSG; ks++)
 #pragma unroll
         for (int kb = 0; kb < KBG; kb++)
           kf[kb][ks] = *reinterpret_cast<const vec8 *>(&Ks[k_frag_off + (kb0 + kb) * 32 * LDK + 16 * ks]);
+      // (with one wave per SIMD the compiler sinks every read to its MFMA and waits for it there: B=1 H=16/8 S=1500 D=256
+      // causal bf16 54.2 -> 52.8 us; all sixteen reads at once spill and measure the same)
+      if constexpr (D > 128 && WPS == 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++)
+      for (int ks = ks0; ks < ks0 + KSG; ks++)
 #pragma unroll
         for (int kb = 0; kb < KBG; kb++) {
 #ifdef LMH_FOLD_SCALE
@@ -526,7 +534,44 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(PrefillArgs 
       for (int i = 0; i < 16; i++) oacc[db][i] *= f;
   }
   // ---- key groups: fold group 1's (m, l, O) into group 0's; lane for lane the same layout ----
-  if (KSPLIT > 1) {
+  if constexpr (KSPLIT > 1 && RG * (DB * 16 + 2) * 64 * 4 > (int)sizeof(Ks2)) {
+    // in two halves of the head dim: the K tiles hold one at a time
+    constexpr int PARTS = 2, PB = (DB + 1) / 2;
+    constexpr int NF = PB * 16 + 2;  // floats per lane
+    static_assert(RG * NF * 64 * 4 <= (int)sizeof(Ks2), "merge buffer must fit in the K tiles");
+    float *xch = reinterpret_cast<float *>(&Ks2[0][0]) + (wave % RG) * (NF * 64) + lane;  // [NF][64 lanes]
+    float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+    for (int part = 0; part < PARTS; part++) {
+      const int db0 = part * PB, db1 = db0 + PB < DB ? db0 + PB : DB;
+      __syncthreads();  // every wave has read its last tile, or the part before
+      if (kg == 1) {
+        xch[0] = m_i;
+        xch[64] = l_i;
+#pragma unroll
+        for (int db = db0; db < db1; db++)
+#pragma unroll
+          for (int i = 0; i < 16; i++) xch[(2 + (db - db0) * 16 + i) * 64] = oacc[db][i];
+      }
+      __syncthreads();
+      if (kg == 1) {
+        if (part == PARTS - 1) return;
+        continue;
+      }
+      if (part == 0) {
+        const float m1 = xch[0], l1 = xch[64];
+        const float m_new = fmaxf(m_i, m1);
+        // a group that saw no key has m = -inf, l = 0, O = 0
+        a0 = m_i == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_i - m_new) * c);
+        a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m1 - m_new) * c);
+        l_i = l_i * a0 + l1 * a1;
+      }
+#pragma unroll
+      for (int db = db0; db < db1; db++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) oacc[db][i] = oacc[db][i] * a0 + xch[(2 + (db - db0) * 16 + i) * 64] * a1;
+    }
+  } else if (KSPLIT > 1) {
     constexpr int NF = DB * 16 + 2;  // floats per lane
     static_assert(KSPLIT == 1 || RG * NF * 64 * 4 <= (int)sizeof(Ks2), "merge buffer must fit in the K tiles");
     float *xch = reinterpret_cast<float *>(&Ks2[0][0]) + (wave % RG) * (NF * 64) + lane;  // [NF][64 lanes]
@@ -1351,17 +1396,36 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
 }
 
 // Head dims above 128: Q and the accumulators of 32 rows take up to 192 registers and a tile buffer pair up to 141 KB, so a
-// workgroup of four waves, one per SIMD with all 512 registers, has the CU to itself; the long rows leave the softmax a
-// small share of a tile. Measured at D = 256 (the vector-ALU kernel that took these launches reaches 8 TFLOP/s): B=1 H=32
-// S=4096 causal fp16 332 us = 827 TFLOP/s, bf16 408 us = 674; B=1 H=16 S=1500 causal bf16 2310 -> 55 us, in 64-row
-// workgroups with two key groups, which small launches take as they do at the other head dims. bf16 keeps head + remainder
-// weights at every length: the registers of the fp16 rewrite of V spill here (S=4096: 633 us; D = 192, where they do not,
-// S=2048 200 against 187 us). The head dims that are odd multiples of 8 stay on the vector-ALU kernel.
+// workgroup has the CU to itself. The vector-ALU kernel that took these launches reaches 8 TFLOP/s. Three forms:
+//   64 rows, four waves in two key groups: one wave per SIMD, as many workgroups as there can be;
+//   128 rows, eight waves in two key groups: two waves per SIMD, which fit with 256 registers each when K fragments are
+//     fetched four k-steps at a time. The second wave computes while the first waits for LDS: a staged tile takes 0.95
+//     (fp16) to 1.13 times (bf16) as long as in the first form and serves twice the rows;
+//   128 rows, four waves: no fold at the end, one wave per SIMD.
+// The first two are compared by the tiles that the busiest CU walks: its longest workgroup or the mean over the CUs
+// (causal, heaviest first), whole rounds without a mask. Where 128 rows need fewer, they are 20 to 47 % faster; where both
+// need the same, the 64-row form is up to 27 % ahead (fp16 from 12 tiles on 0 to 7 % behind). The third is ahead of the
+// second where a row has no more than about four tiles, five with the causal mask's short ones (D=256 bf16 448 workgroups
+// of 104 keys 32.4 against 34.4 us; 1344 of 673 keys 171.0 against 167.5) and was the only 128-row form before: B=1 H=32 S=4096 D=256 causal fp16 363 -> 292 us = 940
+// TFLOP/s, bf16 432 -> 378; B=1 H=32 S=2048 102 -> 86; B=1 H=4 S=6000 without a mask, on 64 rows before, 333 -> 167.
+// bf16 keeps head + remainder weights at every length: the registers of the fp16 rewrite of V spill here (S=4096: 633 us).
+// The head dims that are odd multiples of 8 stay on the vector-ALU kernel.
 template <typename MT, int D>
 int launch_wide_heads(const PrefillArgs &a, hipStream_t stream) {
-  const int64_t wgs = (int64_t)a.B * a.Hq * ((a.Sq + 127) / 128);
-  if (wgs <= device_cu_count() && a.Sk >= 4 * BN) return launch_split<MT, false, D, 2, 4>(a, stream);
-  return launch_split<MT, false, D, 1, 4>(a, stream);
+  const int64_t heads = (int64_t)a.B * a.Hq, cus = device_cu_count();
+  const int64_t row_tiles = (a.Sk + BN - 1) / BN;  // key tiles of a whole row
+  auto steps = [&](int rows) -> double {           // key tiles the busiest CU walks in workgroups of `rows` query rows
+    const int64_t n = (a.Sq + rows - 1) / rows, s = rows / BN;
+    if (!a.causal) return (double)((heads * n + cus - 1) / cus * row_tiles);
+    const int64_t ramp = std::min(n, row_tiles / s);  // workgroups r < ramp walk (r + 1) s tiles, the others all of them
+    const double longest = (double)std::min(row_tiles, n * s);
+    return std::max(longest, (double)heads * (s * ramp * (ramp + 1) / 2 + (n - ramp) * row_tiles) / cus);
+  };
+  const double s64 = steps(64), s128 = steps(128);
+  const bool even_wins = !MT::kSplitP && s128 >= 12;
+  if (s128 > 0.9 * s64 && !even_wins) return launch_split<MT, false, D, 2, 4>(a, stream);
+  if (row_tiles <= (a.causal ? 5 : 4)) return launch_split<MT, false, D, 1, 4>(a, stream);
+  return launch_split<MT, false, D, 2, 8, 2>(a, stream);
 }
 
 template <typename MT>

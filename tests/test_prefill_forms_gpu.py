@@ -48,6 +48,23 @@ def test_large_launch_of_wide_heads(lm, hip, oracle):
     assert rel_err(run(lm, hip, q, k, v, "bf16", True), oracle.flash_attn(q, k, v, causal=True, nthreads=NT)) <= TOL["bf16"]
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,dtype", [
+    (2, 40, 8, 385, 385, 256, True, "f16"), (3, 40, 4, 257, 330, 256, False, "bf16"), (1, 80, 8, 513, 481, 144, True, "bf16"),
+    (5, 32, 8, 129, 321, 192, False, "f16"), (1, 2, 1, 1537, 1537, 208, True, "f16"), (4, 33, 3, 300, 511, 256, True, "bf16"),
+])
+def test_eight_waves_on_wide_heads(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causal, dtype):
+    q, k, v = inputs(oracle, (B, Hq, Sq, D), (B, Hkv, Sk, D), dtype, 32970 + Sq + D)
+    assert "key groups=2, waves=8, waves per SIMD=2>" in plan(lm, q, k, dtype, causal, False)
+    # a last tile with keys for both key groups, for one, and a sequence without a key (zeros; the oracle wants one)
+    lens = np.array([(Sk, Sk - 30, 33, 0, 64)[i] for i in range(B)], np.int32)
+    for kv_len in (None, lens):
+        got = run(lm, hip, q, k, v, dtype, causal, kv_len=None if kv_len is None else list(kv_len))
+        want = oracle.flash_attn(q, k, v, causal=causal, kv_len=None if kv_len is None else np.maximum(kv_len, 1), nthreads=NT)
+        if kv_len is not None:
+            want[kv_len == 0] = 0
+        assert rel_err(got, want) <= TOL[dtype]
+
+
 @pytest.mark.parametrize("interleaved", [False, True])
 @pytest.mark.parametrize("dtype,D", [("f16", 192), ("bf16", 256), ("f32", 192), ("f32", 256), ("f32", 64)])
 def test_wide_heads_rotate_their_queries_in_registers(lm, hip, oracle, dtype, D, interleaved):
