@@ -161,7 +161,7 @@ def test_glue_defines_every_array_method_the_reference_call_paths_use():
     for pattern in EXTRA_METHODS:
         assert re.search(pattern, text, flags=re.M), pattern
     # where a checkout of the reference is at hand, the cited lines must say what this table says they do
-    if os.path.isdir(REFERENCE):
+    if os.path.isdir(os.path.join(REFERENCE, "src")):
         for what, ref_file, ref_line, ref_text, _ in ARRAY_PROTOCOL:
             lines = open(os.path.join(REFERENCE, ref_file)).read().split("\n")
             window = "\n".join(lines[max(ref_line - 3, 0):ref_line + 2])
@@ -345,11 +345,11 @@ def test_glue_host_fallback_and_layer_builder():
     for piece in ("layer.q_proj, x", "layer.k_proj, keys_from", "layer.v_proj, values_from", "layer.o_proj(out)",
                   "[b, s, n_heads, head_dim]", "[1, 3, 2, 4]", "Luminal.flash_attention(", "causal=mask", "[batch, seq, hidden]"):
         assert piece in wh, piece
-    if os.path.isdir(REFERENCE):
+    if os.path.isdir(os.path.join(REFERENCE, "src")):
         w = open(os.path.join(REFERENCE, "src/Whisper.jl")).read()
         assert "Luminal.permute(Luminal.reshape(sa.q_proj(x) * scale, [batch, seq, HEADS, HEAD_DIM]), [1, 3, 2, 4])" in w
         assert "scale = (Float32(hidden) / Float32(HEADS)) ^ -0.25f0" in w
-    if os.path.isdir(REFERENCE):  # the layer's own lines in the reference say the same
+    if os.path.isdir(os.path.join(REFERENCE, "src")):  # the layer's own lines in the reference say the same
         nn = open(os.path.join(REFERENCE, "src/NN.jl")).read()
         assert "Luminal.reshape(sa.q_proj(x), [batch, seq, sa.n_heads, sa.head_dim])" in nn
         assert "Luminal.permute(queries, [1, 3, 2, 4])" in nn and "Luminal.reshape(out, [batch, seq, hidden])" in nn
@@ -375,6 +375,6 @@ def test_glue_device_cache_mirrors_the_reference_cache_holder():
             assert re.search(r"\b%s(::\w+)?=" % kw, keywords), (fn, kw)
     begin = re.search(r"^function begin_step!\(.*?^end$", text, flags=re.M | re.S).group(0)
     assert "copyto!(c.pos, c.kv_len_host)" in begin and "c.kv_len_host .+ Int32(n_new)" in begin and "error(" in begin
-    if os.path.isdir(REFERENCE):
+    if os.path.isdir(os.path.join(REFERENCE, "src")):
         wh = open(os.path.join(REFERENCE, "src/Whisper.jl")).read()
         assert "self_cache::Vector{Tuple{Array{Float32,4}, Array{Float32,4}}}" in wh and "cache.step_pos += 1" in wh
