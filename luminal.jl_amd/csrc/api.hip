@@ -31,6 +31,11 @@ int device_cu_count() {
   return n;
 }
 
+int check_grid(int64_t workgroups, int threads) {
+  if (workgroups * threads <= 0xffffffffll) return LMH_OK;
+  return fail(LMH_E_UNSUPPORTED, "%lld workgroups of %d threads are more than a launch can number", (long long)workgroups, threads);
+}
+
 int fail(int code, const char *fmt, ...) {
   va_list ap;
   va_start(ap, fmt);

@@ -314,10 +314,13 @@ template <int D, int RW, int KG, int NK> constexpr int resident() {  // workgrou
 template <int D, int RW, int KG, int NK>
 int launch_form(const PrefillArgs &a, hipStream_t stream) {
   const int n_q_tiles = (a.Sq + 16 * RW - 1) / (16 * RW);
-  dim3 grid(deal_grid(a.B * a.Hq, n_q_tiles)), block(64 * RW * KG);
+  const int64_t wgs = deal_grid((int64_t)a.B * a.Hq, n_q_tiles);
+  const int rc = check_grid(wgs, 64 * RW * KG);
+  if (rc != LMH_OK) return rc;
+  dim3 grid((uint32_t)wgs), block(64 * RW * KG);
   if (plan_only("prefill_f32_kernel<D=%d, %s, key groups=%d> rows=%d, workgroups=%u", D, a.causal ? "causal" : "full", KG, 16 * RW, grid.x))
     return LMH_OK;
-  const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? resident<D, RW, KG, NK>() : 0);
+  const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? resident<D, RW, KG, NK>() : 0, device_cu_count());
   if (a.causal) hipLaunchKernelGGL((prefill_f32_kernel<D, true, RW, KG, NK>), grid, block, 0, stream, a, deal);
   else hipLaunchKernelGGL((prefill_f32_kernel<D, false, RW, KG, NK>), grid, block, 0, stream, a, deal);
   LMH_HIP_TRY(hipGetLastError());

@@ -1240,9 +1240,12 @@ template <typename MT, int D>
 int launch_pair(const PrefillArgs &a, hipStream_t stream) {
   const int n_q_tiles = (a.Sq + 255) / 256;
   const int n_pairs = (n_q_tiles + 1) / 2;
-  dim3 grid(deal_grid(a.B * a.Hq, n_pairs)), block(512);
+  const int64_t wgs = deal_grid((int64_t)a.B * a.Hq, n_pairs);
+  const int rc = check_grid(wgs, 512);
+  if (rc != LMH_OK) return rc;
+  dim3 grid((uint32_t)wgs), block(512);
   if (plan_only("prefill_mfma_pair_kernel<%s, D=%d, %s> query tiles=%d, workgroups=%u", MT::kName, D, a.causal ? "causal" : "full", n_q_tiles, grid.x)) return LMH_OK;
-  const Deal deal = make_deal(a.B, a.Hq, n_pairs, 0);
+  const Deal deal = make_deal(a.B, a.Hq, n_pairs, 0, device_cu_count());
   if (a.causal)
     hipLaunchKernelGGL((prefill_mfma_pair_kernel<MT, D, true>), grid, block, 0, stream, a, deal, n_q_tiles);
   else
@@ -1263,11 +1266,14 @@ int launch_split(const PrefillArgs &a, hipStream_t stream) {
   using MT = typename base_policy<MT0, V16, KSPLIT>::type;
   constexpr int BM = 32 * NW / KSPLIT;
   const int n_q_tiles = (a.Sq + BM - 1) / BM;
-  dim3 grid(deal_grid(a.B * a.Hq, n_q_tiles)), block(64 * NW);
+  const int64_t wgs = deal_grid((int64_t)a.B * a.Hq, n_q_tiles);
+  const int rc = check_grid(wgs, 64 * NW);
+  if (rc != LMH_OK) return rc;
+  dim3 grid((uint32_t)wgs), block(64 * NW);
   if (plan_only("prefill_mfma_kernel<%s, D=%d, %s, key groups=%d, waves=%d, waves per SIMD=%d> workgroups=%u%s", MT::kName, D,
                 a.causal ? "causal" : "full", KSPLIT, NW, WPS, grid.x, MT::kConvertV ? ", V as fp16" : ""))
     return LMH_OK;
-  const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? 4 * WPS / NW : 0);
+  const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? 4 * WPS / NW : 0, device_cu_count());
   if (a.causal)
     hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS>), grid, block, 0, stream, a, deal);
   else
@@ -1282,9 +1288,10 @@ int launch_split(const PrefillArgs &a, hipStream_t stream) {
 // wide against 64-row workgroups): load 1.33 vs 1.5 -12 % (D = 64), -14 % (D = 96); 0.75 vs 1.0 -7 ... -12 %; equal loads
 // +-2 %, and +7 % at 1024 keys; under about 500 keys the single prologue per CU costs more than the balance wins.
 inline bool wide_plan(const PrefillArgs &a, int n_cus, int *wgs_per_head, int *n_waves, int *mixed) {
+  if ((int64_t)a.B * a.Hq > n_cus) return false;
   const int heads = a.B * a.Hq;
   const int n_blocks = (a.Sq + 31) / 32;
-  if (a.causal || heads > n_cus || n_blocks < 2 || a.Sk < 640) return false;
+  if (a.causal || n_blocks < 2 || a.Sk < 640) return false;
   const int w = max(1, min(n_cus / heads, n_blocks / 2));
   const int r_max = (n_blocks + w - 1) / w;
   if (r_max > 8) return false;
@@ -1313,7 +1320,7 @@ inline bool wide_plan(const PrefillArgs &a, int n_cus, int *wgs_per_head, int *n
 
 template <typename MT, int D>
 int launch_wide(const PrefillArgs &a, int wgs_per_head, int n_waves, int mixed, hipStream_t stream) {
-  dim3 grid(deal_grid(a.B * a.Hq, wgs_per_head)), block(64 * n_waves);
+  dim3 grid((uint32_t)deal_grid(a.B * a.Hq, wgs_per_head)), block(64 * n_waves);
   if (plan_only("prefill_mfma_wide_kernel<%s, D=%d> workgroups per head=%d, waves=%d, workgroups=%u%s", MT::kName, D, wgs_per_head,
                 n_waves, grid.x, mixed ? ", two and four key groups" : ""))
     return LMH_OK;
