@@ -68,6 +68,10 @@ def reshape_view(axes, shape):
     return None if pending else out
 
 
+def view_shape(axes):
+    return tuple(_product(f[0] for f in axis) for axis in axes)
+
+
 def view_dims(axes):
     """(dims, strides) of a view, the slowest first, neighbours that walk memory together merged."""
     dims = []
@@ -216,6 +220,9 @@ class NodeOp:
 # from a graph to steps
 # ---------------------------------------------------------------------------------------------
 class _Lowering:
+    """Nodes carry the shape they were declared with (add_op takes any), while a node that runs as itself has the shape its op
+    gives. A node therefore joins a launch only where the two agree, and where the next node reads it under that shape."""
+
     def __init__(self, graph, wanted, given):
         self.graph, self.given = graph, given
         self.users = [[] for _ in graph.nodes]
@@ -229,24 +236,35 @@ class _Lowering:
     def op(self, i):
         return self.graph.nodes[i].op
 
+    def reads(self, i, operand):
+        """Node i reads `operand` as it was declared."""
+        return all(self.as_declared(r) for r in self.graph.nodes[i].inputs if r[0] == operand)
+
     def plain(self, i):
         """Node i is private and fp32, so that computing it in passing rounds nothing less than before."""
         return self.private[i] and self.graph.dtypes[i] == "f32"
+
+    def shape(self, i):
+        return tuple(self.graph.shapes[i])
+
+    def as_declared(self, ref):
+        """`ref` is its node's own result in the shape the node was declared with."""
+        return ref[1] == 0 and tuple(ref[2]) == self.shape(ref[0])
 
     def base_view(self, ref, inside):
         """Follow a chain of view nodes from `ref` back to an operand that stays: (base reference, axes). `inside`
         collects the nodes passed through."""
         node, index, shape = ref[0], ref[1], tuple(ref[2])
         chain = []
-        while index == 0 and node not in self.given and self.private[node] and hasattr(self.op(node), "view") and \
-                shape == tuple(self.graph.shapes[node]) and \
+        while node not in self.given and self.private[node] and hasattr(self.op(node), "view") and \
+                self.as_declared((node, index, shape)) and \
                 self.graph.dtypes[node] in ("f32", self.graph.dtypes[self.graph.nodes[node].inputs[0][0]]):
             chain.append(node)
             node, index, shape = self.graph.nodes[node].inputs[0][:2] + (tuple(self.graph.nodes[node].inputs[0][2]),)
         base, axes = (node, index, shape), contiguous_view(shape)
         for n in reversed(chain):
             axes = self.op(n).view(axes)
-            if axes is None:
+            if axes is None or view_shape(axes) != self.shape(n):
                 return ref, contiguous_view(ref[2])
         inside.update(chain)
         return base, axes
@@ -257,6 +275,8 @@ class _Lowering:
         if not self.private[node] or type(self.op(node)).__name__ != "PermuteOp" or self.op(node).dims != (1, 0):
             return None
         base = self.graph.nodes[node].inputs[0]
+        if not self.as_declared(ref) or self.shape(node) != tuple(base[2])[::-1]:
+            return None
         same_type = self.graph.dtypes[node] in ("f32", self.graph.dtypes[base[0]])
         return (base, node) if same_type and self.is_input(base) else None
 
@@ -280,10 +300,14 @@ class _Lowering:
             return None
         weight, inside = w[0], {w[1]}
         node, bias, heads = i, None, 0
-        batch, seq, width = self.graph.shapes[i]
+        batch, seq, _ = x[2]
+        width = weight[2][0]
+        if weight[2][1] != x[2][2] or self.shape(i) != (batch, seq, width):
+            return None
         if self.plain(node):
             user = self.users[node][0]
-            if type(self.op(user)).__name__ == "AddOp" and self.graph.shapes[user] == (batch, seq, width) and user not in self.given:
+            if type(self.op(user)).__name__ == "AddOp" and self.shape(user) == (batch, seq, width) and user not in self.given and \
+                    self.reads(user, node):
                 other = [r for r in self.graph.nodes[user].inputs if r[0] != node]
                 found = self.bias(other[0], width) if other else None
                 if found:
@@ -292,9 +316,11 @@ class _Lowering:
                     node = user
         if self.plain(node):
             split = self.users[node][0]
-            if type(self.op(split)).__name__ == "ReshapeOp" and len(self.op(split).shape) == 4 and split not in self.given and self.plain(split):
+            if type(self.op(split)).__name__ == "ReshapeOp" and len(self.op(split).shape) == 4 and split not in self.given and self.plain(split) and \
+                    self.reads(split, node):
                 shape, last = self.op(split).shape, self.users[split][0]
-                if shape[:2] == (batch, seq) and type(self.op(last)).__name__ == "PermuteOp" and self.op(last).dims == (0, 2, 1, 3) and \
+                if shape[:2] == (batch, seq) and shape[2] > 0 and shape[2] * shape[3] == width and self.shape(split) == shape and \
+                        self.reads(last, split) and self.shape(last) == (batch, shape[2], seq, shape[3]) and type(self.op(last)).__name__ == "PermuteOp" and self.op(last).dims == (0, 2, 1, 3) and \
                         last not in self.given:
                     inside |= {node, split}
                     node, heads = last, shape[2]
@@ -339,7 +365,7 @@ class _Lowering:
                 if axes is None:  # not affine over the whole chain: this node alone
                     inside = set()
                     base, axes = node.inputs[0], node.op.view(contiguous_view(node.inputs[0][2]))
-                if axes is not None and len(view_dims(axes)[0]) <= binding.MAP_DIMS:
+                if axes is not None and view_shape(axes) == self.shape(i) and len(view_dims(axes)[0]) <= binding.MAP_DIMS:
                     self.virtual |= inside
                     steps.append(ViewOp(i, base, axes))
                     continue
@@ -350,7 +376,8 @@ class _Lowering:
         """Whether the chain of view nodes up to and including `user` is affine with node i inside it."""
         inside = set()
         base, axes = self.base_view(self.graph.nodes[user].inputs[0], inside)
-        return i in inside and self.op(user).view(axes) is not None
+        axes = self.op(user).view(axes)
+        return i in inside and axes is not None and view_shape(axes) == self.shape(user)
 
 
 def lower(graph, wanted=(), given=()):

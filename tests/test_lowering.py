@@ -1,0 +1,80 @@
+"""What compile() and execute() make of the nodes around attention, on host memory (host_device.py)."""
+import gc
+
+import numpy as np
+import pytest
+
+from host_device import HostDevice
+
+
+@pytest.fixture
+def mem(lm, monkeypatch):
+    device = HostDevice(lm)
+    device.hip = device.install(monkeypatch)
+    yield device
+    gc.collect()
+
+
+def normal(shape, seed):
+    return np.random.default_rng(seed).standard_normal(shape).astype(np.float32)
+
+
+def close(got, want):
+    np.testing.assert_allclose(got, want, rtol=2e-6, atol=2e-6)
+
+
+# ---- declared shapes -------------------------------------------------------------------------
+def test_a_fed_array_of_another_size_is_refused(lm, mem):
+    g = lm.Graph()
+    x = lm.tensor(g, (1, 16, 64))
+    layer = lm.Linear(64, 32, g, bias=False)
+    out = layer(x)
+    y = lm.tensor(g, (4, 8))
+    moved = lm.permute(y, (1, 0))
+    w = normal((32, 64), 1)
+    with pytest.raises(ValueError):
+        lm.execute(g, out.id, {x.id: normal((1, 32, 64), 2), layer.weight.id: w, y.id: normal((4, 8), 3)}, mem.hip)
+    with pytest.raises(ValueError):
+        lm.execute(g, moved.id, {x.id: normal((1, 16, 64), 2), layer.weight.id: w, y.id: normal((2, 3), 3)}, mem.hip)
+    # the same elements under another shape are taken as they lie
+    a = normal((8, 4), 4)
+    got = lm.execute(g, moved.id, {x.id: normal((16, 64), 2), layer.weight.id: w, y.id: a}, mem.hip)
+    np.testing.assert_array_equal(got, a.reshape(4, 8).T)
+
+
+def test_a_node_declared_in_another_shape_than_its_op_gives_stays_out_of_launches(lm, mem):
+    # add_op takes any shape: the op's own result decides, as it does for a node that runs alone
+    def graph(shape):
+        g = lm.Graph()
+        x, w = lm.tensor(g, (2, 6, 8)), lm.tensor(g, (5, 8))
+        product = lm.matmul(x, lm.permute(w, (1, 0)))
+        g.shapes[product.id] = shape
+        return g, x, w, product
+
+    a, b = normal((2, 6, 8), 1), normal((5, 8), 2)
+    for shape in ((2, 3, 5), (2, 6, 4), (1, 1, 1)):
+        g, x, w, product = graph(shape)
+        close(lm.execute(g, product.id, {x.id: a, w.id: b}, mem.hip), a @ b.T)
+        with pytest.raises(ValueError):
+            lm.compile(g, mem.hip)({x.id: a, w.id: b})
+    for shape in ((2, 2), (8, 4, 2)):
+        g = lm.Graph()
+        x = lm.tensor(g, (4, 8))
+        y = lm.add_op(g, lm.PermuteOp((1, 0)), [(x.id, 0, (4, 8))], shape)
+        c = normal((4, 8), 3)
+        np.testing.assert_array_equal(lm.execute(g, y.id, {x.id: c}, mem.hip), c.T)
+        with pytest.raises(ValueError):
+            lm.compile(g, mem.hip)({x.id: c})
+
+
+def test_weights_read_under_another_shape(lm, mem):
+    # W^T's elements as a (16, 4) matrix: not a product with W as it lies
+    g = lm.Graph()
+    x, w = lm.tensor(g, (1, 3, 16)), lm.tensor(g, (8, 8))
+    wt = lm.permute(w, (1, 0))
+    wt.shape = (16, 4)
+    out = lm.matmul(x, wt)
+    a, b = normal((1, 3, 16), 1), normal((8, 8), 2)
+    close(lm.execute(g, out.id, {x.id: a, w.id: b}, mem.hip), a @ np.ascontiguousarray(b.T).reshape(16, 4))
+    cg = lm.compile(g, mem.hip)
+    close(cg({x.id: a, w.id: b})[out.id].to_host(), a @ np.ascontiguousarray(b.T).reshape(16, 4))
