@@ -357,27 +357,27 @@ class _Lowering:
             if hasattr(node.op, "view"):
                 # the longest chain that ends here; a node that its own user will swallow waits for that user
                 user = self.users[i][0] if self.private[i] else None
-                if user is not None and hasattr(self.op(user), "view") and user not in self.given and self.swallows(i, user):
+                if user is not None and hasattr(self.op(user), "view") and user not in self.given and i in self.moved(user)[2]:
                     continue
-                inside = set()
-                base, axes = self.base_view(node.inputs[0], inside)
-                axes = node.op.view(axes)
-                if axes is None:  # not affine over the whole chain: this node alone
-                    inside = set()
-                    base, axes = node.inputs[0], node.op.view(contiguous_view(node.inputs[0][2]))
-                if axes is not None and view_shape(axes) == self.shape(i) and len(view_dims(axes)[0]) <= binding.MAP_DIMS:
+                base, axes, inside = self.moved(i)
+                if axes is not None:
                     self.virtual |= inside
                     steps.append(ViewOp(i, base, axes))
                     continue
             steps.append(NodeOp(i, node.inputs))
         return steps
 
-    def swallows(self, i, user):
-        """Whether the chain of view nodes up to and including `user` is affine with node i inside it."""
-        inside = set()
-        base, axes = self.base_view(self.graph.nodes[user].inputs[0], inside)
-        axes = self.op(user).view(axes)
-        return i in inside and axes is not None and view_shape(axes) == self.shape(user)
+    def moved(self, i):
+        """View node i as one launch: (base reference, axes, the nodes it swallows), over the whole chain that ends here or, if
+        that is not one affine map, over node i alone. axes None: the node runs as itself."""
+        node, inside = self.graph.nodes[i], set()
+        chain = self.base_view(node.inputs[0], inside)
+        for base, axes in (chain, (node.inputs[0], contiguous_view(node.inputs[0][2]))):
+            axes = node.op.view(axes)
+            if axes is not None and view_shape(axes) == self.shape(i) and len(view_dims(axes)[0]) <= binding.MAP_DIMS:
+                return base, axes, inside
+            inside = set()
+        return None, None, inside
 
 
 def lower(graph, wanted=(), given=()):

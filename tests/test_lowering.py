@@ -78,3 +78,14 @@ def test_weights_read_under_another_shape(lm, mem):
     close(lm.execute(g, out.id, {x.id: a, w.id: b}, mem.hip), a @ np.ascontiguousarray(b.T).reshape(16, 4))
     cg = lm.compile(g, mem.hip)
     close(cg({x.id: a, w.id: b})[out.id].to_host(), a @ np.ascontiguousarray(b.T).reshape(16, 4))
+
+
+def test_a_chain_of_more_dimensions_than_a_launch_takes(lm, mem):
+    g = lm.Graph()
+    x = lm.tensor(g, (512,))
+    split = lm.reshape(x, (2,) * 9)
+    out = lm.permute(split, (1, 0, 3, 2, 5, 4, 7, 6, 8)[::-1])
+    a = normal((512,), 1)
+    want = g.nodes[out.id].op.compute(g.nodes[split.id].op.compute(a))
+    np.testing.assert_array_equal(lm.execute(g, out.id, {x.id: a}, mem.hip), want)
+    np.testing.assert_array_equal(lm.compile(g, mem.hip)({x.id: a})[out.id].to_host(), want)
