@@ -232,9 +232,31 @@ class _Lowering:
         # a node may disappear into its only user; nodes without users are results
         self.private = [len(u) == 1 and i not in wanted and i not in given for i, u in enumerate(self.users)]
         self.virtual = set()
+        self.in_place = [i for i in range(len(graph.nodes)) if self.aliases(i)]
+        self.last_write = {}  # the last node that writes into an operand's memory
+        for i in self.in_place:
+            for k in self.aliases(i).values():
+                self.last_write[self.memory(graph.nodes[i].inputs[k])] = i
 
     def op(self, i):
         return self.graph.nodes[i].op
+
+    def aliases(self, i):
+        """{output index: input} of a node that writes into its inputs."""
+        return {"KVAppendOp": {0: 0, 1: 1, 2: 5} if getattr(self.op(i), "rope_q", False) else {0: 0, 1: 1},
+                "DecodeStepOp": {1: 1, 2: 2}}.get(type(self.op(i)).__name__, {})
+
+    def memory(self, ref):
+        """The (node, output index) whose buffer `ref` is."""
+        node, index = ref[0], ref[1]
+        while node not in self.given and index in self.aliases(node):
+            node, index = self.graph.nodes[node].inputs[self.aliases(node)[index]][:2]
+        return node, index
+
+    def settled(self, ref, i):
+        """Nothing writes into `ref` after node i. Otherwise node i has to run at its own place and keep its value: a launch
+        that reads `ref` for a later node, or for whoever asks for node i after the call, would find what was written since."""
+        return self.last_write.get(self.memory(ref), -1) < i
 
     def reads(self, i, operand):
         """Node i reads `operand` as it was declared."""
@@ -262,6 +284,8 @@ class _Lowering:
             chain.append(node)
             node, index, shape = self.graph.nodes[node].inputs[0][:2] + (tuple(self.graph.nodes[node].inputs[0][2]),)
         base, axes = (node, index, shape), contiguous_view(shape)
+        if chain and not self.settled(base, chain[-1]):
+            return ref, contiguous_view(ref[2])
         for n in reversed(chain):
             axes = self.op(n).view(axes)
             if axes is None or view_shape(axes) != self.shape(n):
@@ -275,7 +299,7 @@ class _Lowering:
         if not self.private[node] or type(self.op(node)).__name__ != "PermuteOp" or self.op(node).dims != (1, 0):
             return None
         base = self.graph.nodes[node].inputs[0]
-        if not self.as_declared(ref) or self.shape(node) != tuple(base[2])[::-1]:
+        if not self.as_declared(ref) or not self.settled(base, node) or self.shape(node) != tuple(base[2])[::-1]:
             return None
         same_type = self.graph.dtypes[node] in ("f32", self.graph.dtypes[base[0]])
         return (base, node) if same_type and self.is_input(base) else None
@@ -288,7 +312,8 @@ class _Lowering:
         inside = set()
         base, axes = self.base_view(ref, inside)
         flat = [f for axis in axes for f in axis if f[0] != 1 and f[1] != 0]
-        if tuple(base[2]) == (width,) and axes and axes[-1] == [(width, 1)] and flat in ([(width, 1)], []) and self.is_input(base):
+        if tuple(base[2]) == (width,) and axes and axes[-1] == [(width, 1)] and flat in ([(width, 1)], []) and self.is_input(base) and \
+                self.last_write.get(self.memory(base)) is None:
             return base, inside
         return None
 
@@ -302,7 +327,7 @@ class _Lowering:
         node, bias, heads = i, None, 0
         batch, seq, _ = x[2]
         width = weight[2][0]
-        if weight[2][1] != x[2][2] or self.shape(i) != (batch, seq, width):
+        if weight[2][1] != x[2][2] or self.shape(i) != (batch, seq, width) or not self.settled(x, i):
             return None
         if self.plain(node):
             user = self.users[node][0]
@@ -335,7 +360,6 @@ class _Lowering:
         for item, _, inside in products.values():
             self.virtual |= inside
         tails = {found[0].node for i, found in products.items() if found[0].node != i}
-        in_place = [i for i, n in enumerate(self.graph.nodes) if type(n.op).__name__ in ("KVAppendOp", "DecodeStepOp")]
         for i, node in enumerate(self.graph.nodes):
             name = type(node.op).__name__
             if i in products:
@@ -343,7 +367,7 @@ class _Lowering:
                 # products on the same x join the first one's launch (their weights are inputs: nothing they read is
                 # computed in between, unless a node in between writes into its own inputs)
                 first = by_x.get(x)
-                if first and len(first[1].items) < binding.MATMUL_GROUP and not any(first[0] < p < i for p in in_place):
+                if first and len(first[1].items) < binding.MATMUL_GROUP and not any(first[0] < p < i for p in self.in_place):
                     step = ProjectionOp(x, first[1].items + [item])
                     steps[steps.index(first[1])] = step
                     by_x[x] = (first[0], step)

@@ -89,3 +89,53 @@ def test_a_chain_of_more_dimensions_than_a_launch_takes(lm, mem):
     want = g.nodes[out.id].op.compute(g.nodes[split.id].op.compute(a))
     np.testing.assert_array_equal(lm.execute(g, out.id, {x.id: a}, mem.hip), want)
     np.testing.assert_array_equal(lm.compile(g, mem.hip)({x.id: a})[out.id].to_host(), want)
+
+
+# ---- nodes that write into their inputs ------------------------------------------------------
+def cache_graph(lm, before, after):
+    """before(k cache) -> append a row -> after(what before gave); (graph, feeds, tensors by name)."""
+    g = lm.Graph()
+    kc, vc = lm.tensor(g, (2, 1, 4, 6)), lm.tensor(g, (2, 1, 4, 6))
+    kn, vn, pos = lm.tensor(g, (2, 1, 1, 6)), lm.tensor(g, (2, 1, 1, 6)), lm.tensor(g, (2,), "i32")
+    first = before(kc)
+    k2, v2 = lm.kv_cache_append(kc, vc, kn, vn, pos)
+    last = after(first, k2)
+    feeds = {kc.id: normal((2, 1, 4, 6), 1), vc.id: normal((2, 1, 4, 6), 2), kn.id: normal((2, 1, 1, 6), 3), vn.id: normal((2, 1, 1, 6), 4),
+             pos.id: np.array([3, 1], np.int32)}
+    return g, feeds, kc.id, first.id, last.id
+
+
+def test_a_chain_reads_its_operand_before_it_is_written(lm, mem):
+    g, feeds, kc, first, last = cache_graph(lm, lambda k: lm.permute(k, (0, 1, 3, 2)), lambda x, k2: lm.permute(x, (2, 3, 0, 1)))
+    want = feeds[kc].transpose(0, 1, 3, 2).transpose(2, 3, 0, 1)
+    np.testing.assert_array_equal(lm.execute(g, last, feeds, mem.hip), want)
+    cg = lm.compile(g, mem.hip)
+    for _ in range(2):
+        np.testing.assert_array_equal(cg(feeds)[last].to_host(), want)
+
+
+def test_a_node_asked_for_has_the_value_from_before_a_later_write(lm, mem):
+    g, feeds, kc, first, last = cache_graph(lm, lambda k: lm.permute(lm.permute(k, (0, 1, 3, 2)), (2, 3, 0, 1)), lambda x, k2: lm.permute(k2, (0, 2, 1, 3)))
+    cg = lm.compile(g, mem.hip)
+    for _ in range(2):
+        res = cg(feeds)
+        np.testing.assert_array_equal(res[first].to_host(), feeds[kc].transpose(0, 1, 3, 2).transpose(2, 3, 0, 1))
+        np.testing.assert_array_equal(res[first - 1].to_host(), feeds[kc].transpose(0, 1, 3, 2))
+
+
+def test_products_with_weights_that_are_written_later(lm, mem):
+    g = lm.Graph()
+    kc, vc = lm.tensor(g, (1, 1, 4, 6)), lm.tensor(g, (1, 1, 4, 6))
+    kn, vn, pos, x = lm.tensor(g, (1, 1, 1, 6)), lm.tensor(g, (1, 1, 1, 6)), lm.tensor(g, (1,), "i32"), lm.tensor(g, (1, 3, 6))
+    w = lm.GraphTensor(kc.id, (4, 6), g)
+    wt = lm.permute(w, (1, 0))
+    lm.kv_cache_append(kc, vc, kn, vn, pos)
+    out = lm.matmul(x, wt)
+    feeds = {kc.id: normal((1, 1, 4, 6), 1), vc.id: normal((1, 1, 4, 6), 2), kn.id: normal((1, 1, 1, 6), 3), vn.id: normal((1, 1, 1, 6), 4),
+             pos.id: np.array([2], np.int32), x.id: normal((1, 3, 6), 5)}
+    want = feeds[x.id] @ feeds[kc.id][0, 0].T
+    close(lm.execute(g, out.id, feeds, mem.hip), want)
+    cg = lm.compile(g, mem.hip)
+    for _ in range(2):
+        close(cg(feeds)[out.id].to_host(), want)
+        np.testing.assert_array_equal(cg.results[wt.id].to_host(), feeds[kc.id][0, 0].T)
