@@ -26,7 +26,6 @@ not take (a column-major reshape that is not affine, batch shapes that need a br
 Arrays here are row-major [B, H, S, D] (numpy order), which is the layout the C ABI takes. There
 is no CPU execution path for the attention ops: running one on host arrays raises.
 """
-import bisect
 import ctypes
 import math
 import threading
@@ -1347,7 +1346,7 @@ def compile(graph, device=None):
             results.append((buffer(node_id), _pick(results, node.inputs[1]), _pick(results, node.inputs[2])))
         else:
             results.append(None if node_id in virtual else buffer(node_id))
-    steps, at = [], []  # at: the first node of each step, ascending
+    steps = []
     workspaces = _Workspaces()
 
     def materialise(results, node_id):  # (given the list, not holding it: a dropped graph frees its buffers at once)
@@ -1355,9 +1354,9 @@ def compile(graph, device=None):
         out = buffer(node_id)
         list.__setitem__(results, node_id, out)
         launch = _prepare(node.op, out, [_pick(results, ref) for ref in node.inputs], workspaces)
-        where = bisect.bisect_left(at, node_id)
-        steps.insert(where, launch)
-        at.insert(where, node_id)
+        # at the end: its operands (those that had disappeared as well were asked for in the line above) are made by earlier
+        # steps, and nothing writes into them after the node's own place (lowering's `settled`)
+        steps.append(launch)
         launch()
         return out
 
@@ -1367,7 +1366,6 @@ def compile(graph, device=None):
         outs = [list.__getitem__(results, i) for i in step.nodes]
         steps.append(step.prepare(outs, args) if not isinstance(step, lowering.NodeOp) else
                      _prepare(graph.nodes[step.nodes[0]].op, outs[0], args, workspaces))
-        at.append(min(step.nodes))
     host_steps = sum(isinstance(node.op, HostOp) for node in graph.nodes)
     return CompiledGraph(steps, results, workspaces, device, host_steps)
 

@@ -139,3 +139,102 @@ def test_products_with_weights_that_are_written_later(lm, mem):
     for _ in range(2):
         close(cg(feeds)[out.id].to_host(), want)
         np.testing.assert_array_equal(cg.results[wt.id].to_host(), feeds[kc.id][0, 0].T)
+
+
+# ---- nodes computed when they are asked for --------------------------------------------------
+def test_a_node_asked_for_comes_after_its_operand(lm, mem):
+    g = lm.Graph()
+    x, c, w, bias = lm.tensor(g, (2, 3, 4)), lm.tensor(g, (4,)), lm.tensor(g, (4, 4)), lm.tensor(g, (4,))
+    lm.add(x, c)
+    product = lm.matmul(x, lm.permute(w, (1, 0)))
+    plus = lm.add(x, c)
+    inner = lm.permute(plus, (0, 2, 1))
+    outer = lm.permute(inner, (2, 1, 0))
+    for _ in range(3):
+        outer = lm.add(outer, lm.tensor(g, (1,)))
+    # the product's launch stands for its last node, the one with the highest number
+    out = lm.add(product, lm.expand(lm.expand(bias, 0, 3), 0, 2))
+    values = {i: normal(g.shapes[i], 50 + i) for i, n in enumerate(g.nodes) if isinstance(n.op, lm.host.InputTensor)}
+    cg = lm.compile(g, mem.hip)
+    cg(values)
+    handed = cg.results[inner.id]
+    for seed in (1, 2):
+        values[x.id] = normal((2, 3, 4), seed)
+        res = cg(values)
+        np.testing.assert_array_equal(handed.to_host(), (values[x.id] + values[c.id]).transpose(0, 2, 1))
+        assert res[inner.id] is handed
+        close(res[out.id].to_host(), values[x.id] @ values[w.id].T + values[bias.id])
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_every_node_of_random_graphs(lm, mem, seed):
+    """Views, sums, products and cache appends in random order: the value of every node, asked for in random order, after each
+    of several calls, is what the nodes one by one give."""
+    rng = np.random.default_rng(seed)
+    g = lm.Graph()
+    B, S, W = 2, 4, 6
+    shape = (B, S, W)
+    pool = [lm.tensor(g, shape) for _ in range(2)]
+    caches = [lm.tensor(g, (B, 1, S, W)) for _ in range(2)]
+    pos, weights, bias = lm.tensor(g, (B,), "i32"), [lm.tensor(g, (W, W)) for _ in range(2)], lm.tensor(g, (W,))
+    for _ in range(12):
+        a = pool[rng.integers(len(pool))]
+        kind = rng.integers(7)
+        if kind <= 1:
+            a = lm.permute(a, tuple(int(d) for d in rng.permutation(3)))
+        elif kind == 2:
+            a = lm.reshape(a, [(B, S, W), (S, B, W), (W, S, B), (B, W, S)][rng.integers(4)])
+        elif kind == 3 and a.shape == shape:
+            a = lm.add(a, pool[0])
+        elif kind == 4 and a.shape == shape:
+            a = lm.matmul(a, lm.permute(weights[rng.integers(2)], (1, 0)))
+            if rng.integers(2):
+                a = lm.add(a, lm.expand(lm.expand(bias, 0, S), 0, B))
+            if rng.integers(2):
+                a = lm.permute(lm.reshape(a, (B, S, 3, 2)), (0, 2, 1, 3))
+                a = lm.reshape(a, shape)
+        elif kind == 5:
+            new = [lm.GraphTensor(t.id, (B, 1, 2, W), g, t.index) for t in (lm.tensor(g, (B, 2, W)), lm.tensor(g, (B, 2, W)))]
+            lm.kv_cache_append(caches[0], caches[1], new[0], new[1], pos)
+            continue
+        else:
+            cache = caches[rng.integers(2)]
+            a = lm.GraphTensor(cache.id, shape, g)
+        pool.append(a)
+    inputs = [i for i, n in enumerate(g.nodes) if isinstance(n.op, lm.host.InputTensor)]
+
+    def feeds():
+        return {i: rng.integers(0, S - 1, B).astype(np.int32) if i == pos.id else rng.standard_normal(g.shapes[i]).astype(np.float32) for i in inputs}
+
+    def one_by_one(values):
+        got = {i: v.copy() for i, v in values.items()}
+        pick = lambda r: np.ascontiguousarray(got[r[0]]).reshape(r[2])
+        for i, n in enumerate(g.nodes):
+            if i in got:
+                continue
+            if isinstance(n.op, lm.KVAppendOp):
+                for b, p in enumerate(values[pos.id]):
+                    for cache, new in zip(n.inputs[:2], n.inputs[2:4]):
+                        got[cache[0]][b, :, p:p + 2] = pick(new)[b]
+            else:
+                got[i] = np.array(n.op.compute(*[pick(r) for r in n.inputs]), np.float32)
+        return got
+
+    def same(got, want):  # up to 12 nodes in fp32, each within a few roundings of its largest term
+        np.testing.assert_allclose(got, want, rtol=0, atol=12 * 6 * 2.0 ** -24 * max(1.0, float(np.abs(want).max())) * W)
+
+    cg = lm.compile(g, mem.hip)
+    asked = []
+    nodes = [i for i, n in enumerate(g.nodes) if not isinstance(n.op, lm.KVAppendOp)]
+    for _ in range(3):
+        values = feeds()
+        want = one_by_one(values)
+        res = cg(values)
+        for i in asked:
+            same(res[i].to_host(), want[i])
+        asked = [int(i) for i in rng.permutation(nodes)[:6]]
+        for i in asked:
+            same(res[i].to_host(), want[i])
+    for i in nodes[-3:]:
+        if i not in inputs:
+            same(lm.execute(g, i, values, mem.hip), want[i])
