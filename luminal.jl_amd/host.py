@@ -18,7 +18,7 @@ Additions the reference has only as un-fused subgraphs:
 
 Around the attention path, a model graph also holds the nodes of the layer that calls it (projections, reshapes,
 permutes: reference src/NN.jl:343-361, :383-386). lowering.py takes them to lmh_matmul and lmh_map; the few forms those do
-not take (a column-major reshape that is not affine, batch shapes that need a broadcast) run through a host fallback
+not take (a column-major reshape that is not affine, batch shapes that need a broadcast, results of whole numbers) run through a host fallback
 (HostOp: download the inputs, the reference's CPU semantics in numpy, upload the result):
   MatMul, Permute, Reshape, Add, Expand          reference src/Execution.jl:216-250, src/HighLevelOps.jl:173-266
   Linear, SelfAttention                          reference src/NN.jl:11-38, :319-387

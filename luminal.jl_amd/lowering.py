@@ -110,7 +110,7 @@ def broadcast_dims(shape, a_shape, b_shape):
 def map_launcher(out, a, axes):
     """out = the elements of `a` seen through `axes`; None where lmh_map does not take it."""
     dims, strides = view_dims(axes)
-    if len(dims) > binding.MAP_DIMS or max(dims) >= 1 << 31:
+    if out.dtype == "i32" or len(dims) > binding.MAP_DIMS or max(dims) >= 1 << 31:
         return None
     p = binding.MapParams()
     p.out, p.a, p.out_dtype, p.a_dtype = out.ptr, a.ptr, _CODES[out.dtype], _CODES[a.dtype]
@@ -121,7 +121,7 @@ def map_launcher(out, a, axes):
 
 def add_launcher(out, a, b):
     dims, sa, sb = broadcast_dims(out.shape, a.shape, b.shape)
-    if len(dims) > binding.MAP_DIMS or max(dims) >= 1 << 31:
+    if out.dtype == "i32" or len(dims) > binding.MAP_DIMS or max(dims) >= 1 << 31:
         return None
     p = binding.MapParams()
     p.out, p.a, p.b = out.ptr, a.ptr, b.ptr
@@ -139,8 +139,8 @@ def _product(n):
 
 
 def fill_matmul(p, out, a, b, transposed=False, bias=None, heads=0):
-    """Fill one lmh_matmul_params; `transposed`: b is (N, K). False where the batch shapes need a broadcast that one
-    batch stride does not express."""
+    """Fill one lmh_matmul_params; `transposed`: b is (N, K). False where lmh_matmul does not take it: a result of whole
+    numbers, or batch shapes that need a broadcast which one batch stride does not express."""
     M, K = a.shape[-2:]
     N = b.shape[-2] if transposed else b.shape[-1]
     if (b.shape[-1] if transposed else b.shape[-2]) != K:
@@ -153,7 +153,7 @@ def fill_matmul(p, out, a, b, transposed=False, bias=None, heads=0):
         a_batch = 0 if len(a.shape) == 2 else M * K
     else:
         return False
-    if max(batch, M, N, K) >= 1 << 31:
+    if out.dtype == "i32" or max(batch, M, N, K) >= 1 << 31:
         return False
     p.c, p.a, p.b, p.batch, p.M, p.N, p.K = out.ptr, a.ptr, b.ptr, batch, M, N, K
     p.a_stride[:] = [a_batch, K, 1]
@@ -393,8 +393,10 @@ class _Lowering:
 
     def moved(self, i):
         """View node i as one launch: (base reference, axes, the nodes it swallows), over the whole chain that ends here or, if
-        that is not one affine map, over node i alone. axes None: the node runs as itself."""
+        that is not one affine map, over node i alone. axes None: the node runs as itself (whole numbers: lmh_map gives none)."""
         node, inside = self.graph.nodes[i], set()
+        if self.graph.dtypes[i] == "i32":
+            return None, None, inside
         chain = self.base_view(node.inputs[0], inside)
         for base, axes in (chain, (node.inputs[0], contiguous_view(node.inputs[0][2]))):
             axes = node.op.view(axes)

@@ -238,3 +238,25 @@ def test_every_node_of_random_graphs(lm, mem, seed):
     for i in nodes[-3:]:
         if i not in inputs:
             same(lm.execute(g, i, values, mem.hip), want[i])
+
+
+def test_whole_numbers_are_moved_and_multiplied(lm, mem):
+    g = lm.Graph()
+    x, a, b = lm.tensor(g, (2, 6), "i32"), lm.tensor(g, (3, 4)), lm.tensor(g, (5, 4))
+    moved = lm.permute(lm.reshape(lm.expand(x, 0, 2), (4, 6)), (1, 0))
+    product = lm.matmul(a, lm.permute(b, (1, 0)), dtype="i32")
+    one = lm.reshape(x, (3, 4))
+    values = {x.id: np.arange(12, dtype=np.int32).reshape(2, 6) * 1000003 % 16777213, a.id: np.arange(12, dtype=np.float32).reshape(3, 4),
+              b.id: np.arange(20, dtype=np.float32).reshape(5, 4) - 7}
+    want = {moved.id: np.reshape(np.repeat(values[x.id][None], 2, 0), (4, 6), order="F").T, product.id: values[a.id] @ values[b.id].T,
+            one.id: np.reshape(values[x.id], (3, 4), order="F")}
+    res = lm.compile(g, mem.hip)(values)
+    for i, w in want.items():
+        got = lm.execute(g, i, values, mem.hip)
+        assert got.dtype == np.int32
+        np.testing.assert_array_equal(got, w)
+        np.testing.assert_array_equal(res[i].to_host(), w)
+    x_dev = lm.to_device(values[x.id], mem.hip)
+    op = lm.PermuteOp((1, 0))
+    op.out_dtype = "i32"
+    np.testing.assert_array_equal(lm.execute_op(op, x_dev).to_host(), values[x.id].T)
