@@ -775,17 +775,38 @@ int lmh_copy_many(void *const *dst, const void *const *src, const size_t *bytes,
   static_assert(LMH_COPY_MANY == kCopyMany, "header and kernel agree");
   if (n < 0) return fail(LMH_E_SHAPE, "lmh_copy_many: negative count");
   if (n > 0 && (!dst || !src || !bytes)) return fail(LMH_E_NULL, "lmh_copy_many: null list");
-  for (int32_t first = 0; first < n; first += LMH_COPY_MANY) {
-    CopyManyArgs a = {};
-    const int m = n - first < LMH_COPY_MANY ? n - first : LMH_COPY_MANY;
-    for (int i = 0; i < m; i++) {
-      if (bytes[first + i] && (!dst[first + i] || !src[first + i])) return fail(LMH_E_NULL, "lmh_copy_many: null pointer");
-      a.dst[i] = dst[first + i]; a.src[i] = src[first + i]; a.bytes[i] = (int64_t)bytes[first + i];
+  for (int32_t i = 0; i < n; i++)
+    if (bytes[i] && (!dst[i] || !src[i])) return fail(LMH_E_NULL, "lmh_copy_many: null pointer");
+  auto meet = [](const void *x, size_t nx, const void *y, size_t ny) {
+    return (uintptr_t)x < (uintptr_t)y + ny && (uintptr_t)y < (uintptr_t)x + nx;
+  };
+  CopyManyArgs a = {};
+  int m = 0;  // ranges of the launch that is being put together
+  auto launch = [&]() {
+    const int count = m;
+    m = 0;
+    return count ? launch_copy_many(a, count, (hipStream_t)stream) : LMH_OK;
+  };
+  for (int32_t i = 0; i < n; i++) {
+    const size_t len = bytes[i];
+    if (!len || dst[i] == src[i]) continue;
+    // a range that meets one of the launch waits for it
+    bool wait = m == LMH_COPY_MANY;
+    for (int j = 0; j < m && !wait; j++)
+      wait = meet(dst[i], len, a.dst[j], a.bytes[j]) || meet(dst[i], len, a.src[j], a.bytes[j]) || meet(src[i], len, a.dst[j], a.bytes[j]);
+    const bool itself = meet(dst[i], len, src[i], len);
+    if (wait || itself) {
+      const int rc = launch();
+      if (rc != LMH_OK) return rc;
     }
-    const int rc = launch_copy_many(a, m, (hipStream_t)stream);
-    if (rc != LMH_OK) return rc;
+    if (itself) {  // the runtime's copy, as lmh_memcpy_d2d
+      LMH_HIP_TRY(hipMemcpyAsync(dst[i], src[i], len, hipMemcpyDeviceToDevice, (hipStream_t)stream));
+      continue;
+    }
+    a.dst[m] = dst[i]; a.src[m] = src[i]; a.bytes[m] = (int64_t)len;
+    m++;
   }
-  return LMH_OK;
+  return launch();
 }
 
 }  // extern "C"

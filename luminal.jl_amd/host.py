@@ -1254,22 +1254,20 @@ class CompiledGraph:
         self.device = device
         self.cache = {}
         self.use_capture = False
-        self._copies = {}
+        self._copies = None  # of the last call's nodes
 
     def _run(self, stream):
         for step in self.steps:
             step(stream)
 
     def __call__(self, inputs, device=None):
-        try:  # device arrays: one launch copies them all; its ranges are kept with the addresses they hold for (a program
-            # feeds the same few arrays again and again)
-            key = (*inputs, *[v.ptr for v in inputs.values()], *[v.nbytes for v in inputs.values()])
-            copies = self._copies.get(key)
-            if copies is None:
-                copies = self._plan_copies(key, inputs)
-            if copies:
-                copies.launch()
-        except AttributeError:  # host arrays among them
+        copies, nodes = self._copies, [*inputs]
+        if copies is None or copies.nodes != nodes:  # a program feeds the same nodes again and again
+            copies = self._copies = lowering.InputCopies(nodes, [self._buffer(k) for k in nodes])
+        arrays = inputs.values()
+        if all(isinstance(v, HipArray) for v in arrays):  # one launch copies them all
+            copies.launch(arrays)
+        else:
             for k, v in inputs.items():
                 self._copy_one(k, v)
         if self.use_capture:
@@ -1292,23 +1290,6 @@ class CompiledGraph:
             binding.memcpy_d2d(buffer.ptr, v.ptr, v.nbytes)
         else:
             buffer.copy_from_host(v)
-
-    def _plan_copies(self, key, inputs):
-        pairs = []
-        for k, v in inputs.items():
-            buffer = self._buffer(k)
-            if v.nbytes != buffer.nbytes:
-                raise ValueError("Input length mismatch for node %d" % k)
-            if v.ptr != buffer.ptr:
-                pairs.append((buffer.ptr, v.ptr, v.nbytes))
-        if lowering.copies_overlap(pairs):  # one after the other
-            for k, v in inputs.items():
-                self._copy_one(k, v)
-            return None
-        if len(self._copies) >= 64:
-            self._copies.clear()
-        self._copies[key] = copies = lowering.CopyList(pairs) if pairs else False
-        return copies
 
     def capture(self):
         """From the next call on, run the step list as one recorded HIP graph. Buffer addresses are fixed and

@@ -419,11 +419,10 @@ def lower(graph, wanted=(), given=()):
 
 
 class CopyList:
-    """The device-to-device copies of one call's inputs, as the ctypes arrays lmh_copy_many takes."""
+    """Device-to-device copies, as the ctypes arrays lmh_copy_many takes: (destination, source, bytes) each."""
 
     def __init__(self, pairs):
-        n = len(pairs)
-        self.n = n
+        n = self.n = len(pairs)
         self.dst = (ctypes.c_void_p * n)(*[p[0] for p in pairs])
         self.src = (ctypes.c_void_p * n)(*[p[1] for p in pairs])
         self.nbytes = (ctypes.c_size_t * n)(*[p[2] for p in pairs])
@@ -432,12 +431,20 @@ class CopyList:
         binding.copy_many(self.dst, self.src, self.nbytes, self.n, stream)
 
 
-def copies_overlap(pairs):
-    """Whether any source range meets any destination range, or two destinations meet (then the copies need their order)."""
-    for i, (d, _, n) in enumerate(pairs):
-        for j, (d2, s2, n2) in enumerate(pairs):
-            if s2 < d + n and d < s2 + n2:
-                return True
-            if i != j and d2 < d + n and d < d2 + n2:
-                return True
-    return False
+class InputCopies:
+    """The copies of a call's input arrays into a compiled graph's buffers. Buffers stand for as long as the graph; the arrays
+    are each call's own, so that nothing is kept of them."""
+
+    def __init__(self, nodes, buffers):
+        n = len(nodes)
+        self.nodes, self.lengths = nodes, [b.nbytes for b in buffers]
+        self.dst = (ctypes.c_void_p * n)(*[b.ptr for b in buffers])
+        self.nbytes = (ctypes.c_size_t * n)(*self.lengths)
+        self.sources = ctypes.c_void_p * n
+
+    def launch(self, arrays):
+        src = self.sources(*[a.ptr for a in arrays])
+        if [a.nbytes for a in arrays] != self.lengths:
+            raise ValueError("Input length mismatch for node %d" %
+                             next(i for i, a, n in zip(self.nodes, arrays, self.lengths) if a.nbytes != n))
+        binding.copy_many(self.dst, src, self.nbytes, len(self.nodes))

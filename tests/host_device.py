@@ -105,9 +105,8 @@ class HostDevice:
 
     def copy_many(self, dst, src, nbytes, n, stream=None):
         self.calls.append("copy_many %d" % n)
-        data = [self.bytes(src[i], nbytes[i]).copy() for i in range(n)]
         for i in range(n):
-            self.bytes(dst[i], nbytes[i])[:] = data[i]
+            self.bytes(dst[i], nbytes[i])[:] = self.bytes(src[i], nbytes[i]).copy()
 
     def install(self, monkeypatch):
         binding, host = self.lm.binding, self.lm.host

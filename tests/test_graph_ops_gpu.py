@@ -109,3 +109,21 @@ def test_inputs_that_overlap_are_copied_in_their_order(lm, hip, oracle):
     cg({a.id: va, b.id: vb})
     res = cg({a.id: cg.results[b.id], b.id: cg.results[a.id]})  # a takes b's values, then b takes a's new ones
     np.testing.assert_array_equal(res[out.id].to_host(), vb + vb)
+
+
+def test_copies_that_meet_keep_their_order(lm, hip):
+    rng = np.random.default_rng(6)
+    n = 30000
+    host = rng.integers(0, 1 << 30, 8 * n, dtype=np.int32)
+    for _ in range(20):
+        dev, want = lm.to_device(host, hip), host.copy()
+        ranges = []
+        for _ in range(int(rng.integers(2, 20))):
+            length = int(rng.integers(0, n))
+            dst, src = (int(x) for x in rng.integers(0, 8 * n - length, 2))
+            if abs(dst - src) < length:  # (a range that meets itself is the runtime's copy, whose order is its own)
+                dst = src
+            ranges.append((dst, src, length))
+            want[dst:dst + length] = want[src:src + length].copy()
+        _low(lm).CopyList([(dev.ptr + 4 * d, dev.ptr + 4 * s, 4 * k) for d, s, k in ranges]).launch()
+        np.testing.assert_array_equal(dev.to_host(), want)

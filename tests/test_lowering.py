@@ -260,3 +260,29 @@ def test_whole_numbers_are_moved_and_multiplied(lm, mem):
     op = lm.PermuteOp((1, 0))
     op.out_dtype = "i32"
     np.testing.assert_array_equal(lm.execute_op(op, x_dev).to_host(), values[x.id].T)
+
+
+# ---- inputs ----------------------------------------------------------------------------------
+def test_nothing_is_kept_of_the_arrays_a_call_is_fed(lm, mem):
+    g = lm.Graph()
+    a, b = lm.tensor(g, (8,)), lm.tensor(g, (8,))
+    out = lm.add(a, b)
+    cg = lm.compile(g, mem.hip)
+    state = set()
+    for seed in range(200):
+        va, vb = normal((8,), seed), normal((8,), seed + 1000)
+        fed = {a.id: lm.to_device(va, mem.hip), b.id: lm.to_device(vb, mem.hip)}
+        mem.calls.clear()
+        np.testing.assert_array_equal(cg(fed)[out.id].to_host(), va + vb)
+        assert mem.calls == ["copy_many 2", "map"]
+        state.add(repr({k: sorted(map(str, v)) if isinstance(v, dict) else str(v) for k, v in vars(cg).items()}))
+    assert len(state) == 1  # the graph after 200 calls with arrays of their own is the graph after one
+    assert all(addr not in repr([list(cg._copies.dst), cg._copies.nodes]) for addr in (str(x.ptr) for x in fed.values()))
+    # other nodes than before, another order, host arrays among them, a wrong length
+    np.testing.assert_array_equal(cg({b.id: lm.to_device(va, mem.hip)})[out.id].to_host(), va + va)
+    np.testing.assert_array_equal(cg({b.id: lm.to_device(vb, mem.hip), a.id: va})[out.id].to_host(), va + vb)
+    with pytest.raises(ValueError, match="node %d" % b.id):
+        cg({a.id: lm.to_device(va, mem.hip), b.id: lm.to_device(normal((9,), 1), mem.hip)})
+    with pytest.raises(KeyError):
+        cg({17: lm.to_device(va, mem.hip)})
+    np.testing.assert_array_equal(cg({})[out.id].to_host(), va + vb)
