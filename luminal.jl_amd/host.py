@@ -541,17 +541,25 @@ class Graph:
         self.shapes = []
         self.dtypes = []
         self.tensors = {}
-        self._lowered = {}
+        self._lowered = None
 
     def lowered(self, wanted, given):
-        """lowering.lower(self, wanted, given), kept while the graph stays as it is."""
+        """lowering.lower(self, wanted, given), kept while the graph stays as it is: its ops and what they hold, what they read,
+        shapes and types. Safe between threads: (graph as it was, {question: answer}) is replaced as a whole."""
+        state = ([(node.op, *vars(node.op).values()) for node in self.nodes], [[*node.inputs] for node in self.nodes],
+                 [*self.shapes], [*self.dtypes])
+        kept = self._lowered
+        if kept is None or kept[0] != state:
+            kept = (state, {})
         key = (tuple(wanted), tuple(given))
-        state = [node.op for node in self.nodes]
-        if self._lowered.get("state") != state:
-            self._lowered = {"state": state}
-        if key not in self._lowered:
-            self._lowered[key] = lowering.lower(self, wanted, given)
-        return self._lowered[key]
+        found = kept[1].get(key)
+        if found is None:
+            found = lowering.lower(self, wanted, given)
+            if len(kept[1]) >= 64:
+                kept[1].clear()
+            kept[1][key] = found
+        self._lowered = kept
+        return found
 
 
 def add_op(graph, op, inputs, output_shape, dtype="f32"):

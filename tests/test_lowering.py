@@ -286,3 +286,65 @@ def test_nothing_is_kept_of_the_arrays_a_call_is_fed(lm, mem):
     with pytest.raises(KeyError):
         cg({17: lm.to_device(va, mem.hip)})
     np.testing.assert_array_equal(cg({})[out.id].to_host(), va + vb)
+
+
+# ---- the kept lowering -----------------------------------------------------------------------
+def test_a_changed_graph_is_lowered_again(lm, mem):
+    g = lm.Graph()
+    x, y = lm.tensor(g, (4, 8)), lm.tensor(g, (4, 8))
+    moved = lm.permute(lm.permute(x, (1, 0)), (1, 0))
+    out = lm.permute(moved, (1, 0))
+    feeds = {x.id: normal((4, 8), 1), y.id: normal((4, 8), 2)}
+
+    def value():
+        return lm.execute(g, out.id, feeds, mem.hip)
+
+    np.testing.assert_array_equal(value(), feeds[x.id].T)
+    g.nodes[moved.id - 1].inputs = [(y.id, 0, (4, 8))]  # another operand
+    np.testing.assert_array_equal(value(), feeds[y.id].T)
+    g.nodes[out.id].op.dims = (0, 1)  # another op
+    g.shapes[out.id] = (4, 8)
+    np.testing.assert_array_equal(value(), feeds[y.id])
+    g.dtypes[out.id] = g.nodes[out.id].op.out_dtype = "f16"  # another type
+    np.testing.assert_array_equal(value(), feeds[y.id].astype(np.float16).astype(np.float32))
+    kept = g.lowered([out.id], feeds)
+    assert g.lowered([out.id], feeds) is kept
+
+
+def test_threads_lower_a_new_graph_at_the_same_time(lm, mem):
+    import random
+    import threading
+    import time
+
+    class SlowGraph(lm.Graph):  # every access to what is kept takes its time
+        def __init__(self):
+            self.kept = None
+            super().__init__()
+
+        @property
+        def _lowered(self):
+            time.sleep(random.uniform(0, 2e-4))
+            return self.kept
+
+        @_lowered.setter
+        def _lowered(self, value):
+            time.sleep(random.uniform(0, 4e-4))
+            self.kept = value
+
+    wrong = []
+    for _ in range(60):
+        g = SlowGraph()
+        nodes = [lm.tensor(g, (2, 3))]
+        for _ in range(4):
+            nodes.append(lm.permute(nodes[-1], (1, 0)))
+
+        def work(wanted):
+            try:
+                assert g.lowered([wanted], [0])[0][-1].nodes
+            except Exception as e:
+                wrong.append(repr(e))
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(1, 5)]
+        [t.start() for t in threads]
+        [t.join() for t in threads]
+    assert not wrong, wrong[:3]
