@@ -356,7 +356,8 @@ typedef struct lmh_map_params {
 int lmh_map(const lmh_map_params *p, void *stream);
 
 /* n device-to-device copies in one launch per LMH_COPY_MANY of them (what a compiled graph does with its inputs, reference
- * src/Compiler.jl:80-96). Ranges that meet are copied in their order, by launches of their own. */
+ * src/Compiler.jl:80-96). Ranges that meet are copied in their order, by launches of their own.
+ * Memory of the current GPU (lmh_memcpy_d2d takes another GPU's as well). */
 #define LMH_COPY_MANY 8
 int lmh_copy_many(void *const *dst, const void *const *src, const size_t *bytes, int32_t n, void *stream);
 

@@ -245,6 +245,10 @@ class HipArray:
         binding.sync()  # whoever uses the array next may do so on any stream
         return self
 
+    def copy_from_device(self, array):
+        binding.memcpy_d2d(self.ptr, array.ptr, self.nbytes)
+        return self
+
     def to_host_raw(self):
         raw = np.empty(self.shape, dtype=_NP_STORAGE[self.dtype])
         binding.memcpy_d2h(raw.ctypes.data, self.ptr, self.nbytes)
@@ -881,13 +885,18 @@ def _host_fallback(op, inputs):
     return np.ascontiguousarray(op.compute(*host), dtype=np.float32)
 
 
+def _on(device, x):
+    """x is an array that kernels of `device` can reach (another GPU's takes peer access, which nobody arranges)."""
+    return isinstance(x, HipArray) and x.device.index == device.index
+
+
 def _overlap(a, b):
     return a.ptr < b.ptr + b.nbytes and b.ptr < a.ptr + a.nbytes
 
 
 def _prepare_host_op(op, out, inputs):
     """launch(stream) of a HostOp on device arrays, or None where it has to run through the host."""
-    if not all(isinstance(x, HipArray) and x.size and not _overlap(x, out) for x in inputs):
+    if not all(_on(out.device, x) and x.size and not _overlap(x, out) for x in inputs):
         return None
     shape = op.result_shape([x.shape for x in inputs])
     if shape is None:
@@ -1094,7 +1103,7 @@ def execute_op(op, *inputs):
         dev = next((x.device for x in inputs if isinstance(x, HipArray)), None)
         if dev is None:
             raise TypeError("%s: no input is on a HIP device" % type(op).__name__)
-        if all(isinstance(x, HipArray) and x.size for x in inputs):
+        if all(_on(dev, x) and x.size for x in inputs):
             shape = op.result_shape([x.shape for x in inputs])
             if shape is not None:
                 out = HipArray(shape, op.out_dtype, dev)
@@ -1164,6 +1173,7 @@ def execute(graph, output_ids, initial_inputs, device=None, dtype=None):
             args = [_pick(results, ref) for ref in step.inputs]
             op = graph.nodes[step.nodes[0]].op
             if not isinstance(step, lowering.NodeOp):
+                args = [x if _on(device, x) else new(x.shape, x.dtype).copy_from_device(x) for x in args]
                 outs = [new(graph.shapes[i], graph.dtypes[i]) for i in step.nodes]
                 step.prepare(outs, args)()
                 results.update(zip(step.nodes, outs))
@@ -1273,7 +1283,9 @@ class CompiledGraph:
         if copies is None or copies.nodes != nodes:  # a program feeds the same nodes again and again
             copies = self._copies = lowering.InputCopies(nodes, [self._buffer(k) for k in nodes])
         arrays = inputs.values()
-        if all(isinstance(v, HipArray) for v in arrays):  # one launch copies them all
+        # one launch copies them all; a kernel does not reach into another GPU's memory without the peer access that the
+        # runtime's copy arranges for itself
+        if all(isinstance(v, HipArray) and v.device.index == copies.device for v in arrays):
             copies.launch(arrays)
         else:
             for k, v in inputs.items():

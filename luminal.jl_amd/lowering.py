@@ -438,6 +438,7 @@ class InputCopies:
     def __init__(self, nodes, buffers):
         n = len(nodes)
         self.nodes, self.lengths = nodes, [b.nbytes for b in buffers]
+        self.device = buffers[0].device.index if buffers else None  # the graph's, and so every buffer's
         self.dst = (ctypes.c_void_p * n)(*[b.ptr for b in buffers])
         self.nbytes = (ctypes.c_size_t * n)(*self.lengths)
         self.sources = ctypes.c_void_p * n

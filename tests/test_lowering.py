@@ -348,3 +348,23 @@ def test_threads_lower_a_new_graph_at_the_same_time(lm, mem):
         [t.start() for t in threads]
         [t.join() for t in threads]
     assert not wrong, wrong[:3]
+
+
+def test_arrays_of_another_gpu_take_the_runtimes_copy(lm, mem):
+    g = lm.Graph()
+    a, b = lm.tensor(g, (8,)), lm.tensor(g, (8,))
+    out = lm.add(a, b)
+    cg = lm.compile(g, mem.hip)
+    va, vb = normal((8,), 1), normal((8,), 2)
+    fed = {a.id: lm.to_device(va, mem.hip), b.id: lm.to_device(vb, lm.HIPDevice(1))}
+    mem.calls.clear()
+    np.testing.assert_array_equal(cg(fed)[out.id].to_host(), va + vb)
+    assert mem.calls == ["memcpy_d2d", "memcpy_d2d", "map"]
+    mem.calls.clear()
+    np.testing.assert_array_equal(lm.execute_op(lm.AddOp(), *fed.values()).to_host(), va + vb)  # through the host
+    assert mem.calls == []
+    h = lm.Graph()
+    x = lm.tensor(h, (2, 4))
+    moved = lm.permute(x, (1, 0))
+    np.testing.assert_array_equal(lm.execute(h, moved.id, {x.id: fed[b.id].view((2, 4))}, mem.hip), vb.reshape(2, 4).T)
+    assert mem.calls == ["memcpy_d2d", "map"]
