@@ -1169,7 +1169,8 @@ def execute(graph, output_ids, initial_inputs, device=None, dtype=None):
                 raise KeyError("no value given for input tensor %d" % node_id)
         if uploads:
             binding.upload(uploads)
-        for step in graph.lowered(ids, results)[0]:
+        steps = graph.lowered(ids, results)[0] if isinstance(device, HIPDevice) else lowering.one_by_one(graph, results)
+        for step in steps:
             args = [_pick(results, ref) for ref in step.inputs]
             op = graph.nodes[step.nodes[0]].op
             if not isinstance(step, lowering.NodeOp):
@@ -1177,7 +1178,7 @@ def execute(graph, output_ids, initial_inputs, device=None, dtype=None):
                 outs = [new(graph.shapes[i], graph.dtypes[i]) for i in step.nodes]
                 step.prepare(outs, args)()
                 results.update(zip(step.nodes, outs))
-            elif isinstance(op, (FlashAttentionOp, DecodeAttentionOp, RotaryEmbeddingOp)) and isinstance(args[0], HipArray):
+            elif isinstance(op, (FlashAttentionOp, DecodeAttentionOp, RotaryEmbeddingOp)) and isinstance(device, HIPDevice) and _on(device, args[0]):
                 results[step.nodes[0]] = execute_op_inplace(new(args[0].shape, getattr(op, "out_dtype", None) or args[0].dtype), op, *args)
             else:
                 results[step.nodes[0]] = execute_op(op, *args)

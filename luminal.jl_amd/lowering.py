@@ -406,13 +406,16 @@ class _Lowering:
         return None, None, inside
 
 
+def one_by_one(graph, given):
+    return [NodeOp(i, node.inputs) for i, node in enumerate(graph.nodes) if i not in given and type(node.op).__name__ != "InputTensor"]
+
+
 def lower(graph, wanted=(), given=()):
     """(steps, virtual): the launches that compute every node of `graph` that is `wanted` or has no or several users, in
     order, and the nodes that disappeared into one of them. `given` nodes have values already."""
     given = set(given)
     if not any(hasattr(node.op, "compute") for node in graph.nodes):  # nothing around the attention nodes
-        return [NodeOp(i, node.inputs) for i, node in enumerate(graph.nodes)
-                if i not in given and type(node.op).__name__ != "InputTensor"], set()
+        return one_by_one(graph, given), set()
     work = _Lowering(graph, set(wanted), given)
     steps = work.steps()
     return steps, work.virtual

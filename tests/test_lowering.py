@@ -368,3 +368,19 @@ def test_arrays_of_another_gpu_take_the_runtimes_copy(lm, mem):
     moved = lm.permute(x, (1, 0))
     np.testing.assert_array_equal(lm.execute(h, moved.id, {x.id: fed[b.id].view((2, 4))}, mem.hip), vb.reshape(2, 4).T)
     assert mem.calls == ["memcpy_d2d", "map"]
+
+
+def test_without_a_device_nodes_are_refused_by_name(lm):
+    g = lm.Graph()
+    x = lm.tensor(g, (2, 4))
+    moved = lm.permute(x, (1, 0))
+    with pytest.raises(TypeError, match="PermuteOp: no input is on a HIP device"):
+        lm.execute(g, moved.id, {x.id: normal((2, 4), 1)}, lm.CPUDevice())
+
+
+def test_device_arrays_run_where_they_are(lm, mem):
+    g = lm.Graph()
+    x = lm.tensor(g, (2, 4))
+    moved = lm.permute(lm.permute(x, (1, 0)), (1, 0))
+    a = normal((2, 4), 1)
+    np.testing.assert_array_equal(lm.execute(g, moved.id, {x.id: lm.to_device(a, mem.hip)}, lm.CPUDevice()), a)
