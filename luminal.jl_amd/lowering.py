@@ -232,6 +232,7 @@ class _Lowering:
         # a node may disappear into its only user; nodes without users are results
         self.private = [len(u) == 1 and i not in wanted and i not in given for i, u in enumerate(self.users)]
         self.virtual = set()
+        self.tails = set()  # nodes whose value a product's launch writes
         self.in_place = [i for i in range(len(graph.nodes)) if self.aliases(i)]
         self.last_write = {}  # the last node that writes into an operand's memory
         for i in self.in_place:
@@ -278,7 +279,7 @@ class _Lowering:
         collects the nodes passed through."""
         node, index, shape = ref[0], ref[1], tuple(ref[2])
         chain = []
-        while node not in self.given and self.private[node] and hasattr(self.op(node), "view") and \
+        while node not in self.given and node not in self.tails and self.private[node] and hasattr(self.op(node), "view") and \
                 self.as_declared((node, index, shape)) and \
                 self.graph.dtypes[node] in ("f32", self.graph.dtypes[self.graph.nodes[node].inputs[0][0]]):
             chain.append(node)
@@ -359,7 +360,7 @@ class _Lowering:
         products = {i: found for i, found in products.items() if found}
         for item, _, inside in products.values():
             self.virtual |= inside
-        tails = {found[0].node for i, found in products.items() if found[0].node != i}
+        self.tails = {found[0].node for i, found in products.items() if found[0].node != i}
         for i, node in enumerate(self.graph.nodes):
             name = type(node.op).__name__
             if i in products:
@@ -376,7 +377,7 @@ class _Lowering:
                     steps.append(step)
                     by_x[x] = (i, step)
                 continue
-            if i in self.virtual or i in self.given or i in tails or name == "InputTensor":
+            if i in self.virtual or i in self.given or i in self.tails or name == "InputTensor":
                 continue
             if hasattr(node.op, "view"):
                 # the longest chain that ends here; a node that its own user will swallow waits for that user

@@ -192,7 +192,7 @@ def test_every_node_of_random_graphs(lm, mem, seed):
                 a = lm.add(a, lm.expand(lm.expand(bias, 0, S), 0, B))
             if rng.integers(2):
                 a = lm.permute(lm.reshape(a, (B, S, 3, 2)), (0, 2, 1, 3))
-                a = lm.reshape(a, shape)
+                a = lm.reshape(lm.permute(a, (0, 2, 1, 3)) if rng.integers(2) else a, shape)
         elif kind == 5:
             new = [lm.GraphTensor(t.id, (B, 1, 2, W), g, t.index) for t in (lm.tensor(g, (B, 2, W)), lm.tensor(g, (B, 2, W)))]
             lm.kv_cache_append(caches[0], caches[1], new[0], new[1], pos)
@@ -384,3 +384,19 @@ def test_device_arrays_run_where_they_are(lm, mem):
     moved = lm.permute(lm.permute(x, (1, 0)), (1, 0))
     a = normal((2, 4), 1)
     np.testing.assert_array_equal(lm.execute(g, moved.id, {x.id: lm.to_device(a, mem.hip)}, lm.CPUDevice()), a)
+
+
+def test_views_behind_a_product_that_is_split_into_heads(lm, mem):
+    g = lm.Graph()
+    x, w = lm.tensor(g, (2, 3, 4)), lm.tensor(g, (8, 4))
+    product = lm.matmul(x, lm.permute(w, (1, 0)))
+    heads = lm.permute(lm.reshape(product, (2, 3, 2, 4)), (0, 2, 1, 3))
+    moved = lm.permute(heads, (3, 0, 1, 2))
+    values = {x.id: normal(x.shape, 1), w.id: normal(w.shape, 2)}
+    split = np.reshape(values[x.id] @ values[w.id].T, (2, 3, 2, 4), order="F").transpose(0, 2, 1, 3)
+    cg = lm.compile(g, mem.hip)
+    for _ in range(2):
+        res = cg(values)
+        close(res[moved.id].to_host(), split.transpose(3, 0, 1, 2))
+        close(res[heads.id].to_host(), split)
+    close(lm.execute(g, moved.id, values, mem.hip), split.transpose(3, 0, 1, 2))
