@@ -29,6 +29,7 @@ is no CPU execution path for the attention ops: running one on host arrays raise
 import ctypes
 import math
 import threading
+import weakref
 
 import numpy as np
 
@@ -1126,7 +1127,10 @@ def execute_op(op, *inputs):
 
 def _pick(results, ref):
     """Value of input triple (node_id, output_index, shape): multi-output nodes store a tuple."""
-    r = results[ref[0]]
+    return _view(results[ref[0]], ref)
+
+
+def _view(r, ref):
     r = r[ref[1]] if isinstance(r, tuple) else r
     if isinstance(r, HipArray) and tuple(ref[2]) != r.shape:
         r = r.view(ref[2])
@@ -1242,22 +1246,54 @@ def release_capture(cache):
     cache.pop("hip_warm", None)
 
 
+class _AskedStep:
+    """The launch of a node that had disappeared, for as long as somebody holds its buffer."""
+
+    def __init__(self, out, launch, operands):
+        self.out, self.launch, self.operands = weakref.ref(out), launch, operands
+
+    def __call__(self, stream):
+        out = self.out()  # held until the launch is enqueued
+        if out is not None:
+            self.launch(stream)
+
+
 class _Results(list):
     """The node buffers of a compiled graph. A node that disappeared into another node's launch has none until somebody
-    asks for it: then it is computed from its operands, and by every later call as well."""
+    asks for it: then it is computed from its operands, and by every later call as well. The graph itself holds what was asked
+    for by number; what a walk over all nodes handed out is computed for as long as its holder keeps it."""
 
     def __init__(self, buffers, materialise):
         super().__init__(buffers)
         self._materialise = materialise
+        self._walked = {}  # node -> weak reference
 
     def __getitem__(self, i):
         if isinstance(i, slice):
-            return [self[j] for j in range(*i.indices(len(self)))]
+            return [self._look(j) for j in range(*i.indices(len(self)))]
         value = super().__getitem__(i)
-        return self._materialise(self, i if i >= 0 else i + len(self)) if value is None else value
+        if value is None:
+            value = self._look(i if i >= 0 else i + len(self))
+            self[i] = value
+        return value
+
+    def _look(self, i):
+        value = super().__getitem__(i)
+        if value is None and i in self._walked:
+            value = self._walked[i]()
+        if value is None:
+            value = self._materialise(self, i)
+            self._walked[i] = weakref.ref(value)
+        return value
 
     def __iter__(self):
-        return (self[i] for i in range(len(self)))
+        return (self._look(i) for i in range(len(self)))
+
+    def __reversed__(self):
+        return (self._look(i) for i in reversed(range(len(self))))
+
+    def copy(self):
+        return [*self]
 
 
 class CompiledGraph:
@@ -1265,9 +1301,10 @@ class CompiledGraph:
     inputs into their buffers, runs the steps in place and returns the buffer list; nothing is
     allocated per call. After capture() the steps go through execute_with_capture: one HIP graph launch."""
 
-    def __init__(self, steps, results, workspaces=None, device=None, host_steps=0):
+    def __init__(self, steps, results, workspaces=None, device=None, host_steps=0, asked=None):
         self.host_steps = host_steps  # nodes of the classes that may run through the host
         self.steps = steps
+        self.asked = [] if asked is None else asked  # _AskedSteps, after the others
         self.results = results
         self.workspaces = workspaces  # decode scratch owned by this graph: its address never changes
         self.device = device
@@ -1278,6 +1315,12 @@ class CompiledGraph:
     def _run(self, stream):
         for step in self.steps:
             step(stream)
+        if self.asked:
+            for i in reversed(range(len(self.asked))):  # a step holds its operands, which earlier ones make
+                if self.asked[i].out() is None:
+                    del self.asked[i]
+            for step in self.asked:
+                step(stream)
 
     def __call__(self, inputs, device=None):
         copies, nodes = self._copies, [*inputs]
@@ -1348,17 +1391,16 @@ def compile(graph, device=None):
             results.append((buffer(node_id), _pick(results, node.inputs[1]), _pick(results, node.inputs[2])))
         else:
             results.append(None if node_id in virtual else buffer(node_id))
-    steps = []
+    steps, asked = [], []
     workspaces = _Workspaces()
 
     def materialise(results, node_id):  # (given the list, not holding it: a dropped graph frees its buffers at once)
         node = graph.nodes[node_id]
-        out = buffer(node_id)
-        list.__setitem__(results, node_id, out)
-        launch = _prepare(node.op, out, [_pick(results, ref) for ref in node.inputs], workspaces)
-        # at the end: its operands (those that had disappeared as well were asked for in the line above) are made by earlier
-        # steps, and nothing writes into them after the node's own place (lowering's `settled`)
-        steps.append(launch)
+        out, operands = buffer(node_id), [results._look(ref[0]) for ref in node.inputs]
+        launch = _prepare(node.op, out, [_view(x, ref) for x, ref in zip(operands, node.inputs)], workspaces)
+        # behind all steps: its operands (those that had disappeared as well were asked for in the line above) are made by
+        # earlier ones, and nothing writes into them after the node's own place (lowering's `settled`)
+        asked.append(_AskedStep(out, launch, operands))
         launch()
         return out
 
@@ -1369,7 +1411,7 @@ def compile(graph, device=None):
         steps.append(step.prepare(outs, args) if not isinstance(step, lowering.NodeOp) else
                      _prepare(graph.nodes[step.nodes[0]].op, outs[0], args, workspaces))
     host_steps = sum(isinstance(node.op, HostOp) for node in graph.nodes)
-    return CompiledGraph(steps, results, workspaces, device, host_steps)
+    return CompiledGraph(steps, results, workspaces, device, host_steps, asked)
 
 
 # ---------------------------------------------------------------------------------------------

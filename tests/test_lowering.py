@@ -400,3 +400,40 @@ def test_views_behind_a_product_that_is_split_into_heads(lm, mem):
         close(res[moved.id].to_host(), split.transpose(3, 0, 1, 2))
         close(res[heads.id].to_host(), split)
     close(lm.execute(g, moved.id, values, mem.hip), split.transpose(3, 0, 1, 2))
+
+
+def test_a_walk_over_all_results_leaves_the_graph_as_it_was(lm, mem):
+    g = lm.Graph()
+    x, w, b = lm.tensor(g, (2, 3, 4)), lm.tensor(g, (8, 4)), lm.tensor(g, (8,))
+    product = lm.matmul(x, lm.permute(w, (1, 0)))
+    biased = lm.add(product, lm.expand(lm.expand(b, 0, 3), 0, 2))
+    out = lm.permute(lm.reshape(biased, (2, 3, 2, 4)), (0, 2, 1, 3))
+    moved = lm.permute(lm.permute(out, (3, 0, 1, 2)), (1, 0, 2, 3))
+    cg = lm.compile(g, mem.hip)
+
+    def call(seed):
+        values = {t.id: normal(t.shape, seed + t.id) for t in (x, w, b)}
+        mem.calls.clear()
+        return values, cg(values)
+
+    values, res = call(1)
+    assert mem.calls == ["matmul 1", "map"]
+    for walk in (list, tuple, lambda r: r[:], lambda r: [*reversed(r)], lambda r: r.copy(), lambda r: [y for y in r]):
+        buffers = walk(res)
+        assert len(buffers) == len(g.nodes) and all(isinstance(y, lm.HipArray) for y in buffers)
+        del buffers
+        call(2)
+        gc.collect()
+        assert mem.calls == ["matmul 1", "map"]
+    blocks = len(mem.blocks)
+    held = list(res)[biased.id]  # one of them is kept: it is up to date in every later call, and what it reads as well
+    for seed in (3, 4):
+        values, _ = call(seed)
+        close(held.to_host(), values[x.id] @ values[w.id].T + values[b.id])
+    assert res[biased.id] is held
+    del held
+    again = res[biased.id]  # asked for by number: the graph's from now on
+    values, _ = call(6)
+    close(again.to_host(), values[x.id] @ values[w.id].T + values[b.id])
+    close(res[product.id].to_host(), values[x.id] @ values[w.id].T)
+    assert len(mem.blocks) > blocks
