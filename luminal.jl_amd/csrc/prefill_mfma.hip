@@ -390,30 +390,52 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(PrefillArgs 
 #pragma unroll
       for (int i = 0; i < 16; i++) sacc[kb][i] = 0.f;
     constexpr int KBG = NKB < 2 ? NKB : 2;  // key blocks whose fragments are fetched together
-    constexpr int KSG = D <= 128 ? KS : WPS == 2 ? 4 : KS / 2;  // ... and k-steps (long rows: what the registers hold)
 #pragma unroll
-    for (int kb0 = 0; kb0 < NKB; kb0 += KBG)
+    for (int kb0 = 0; kb0 < NKB; kb0 += KBG) {
+      if constexpr (D <= 128) {
+        // (as one turn of the loop below the same instructions come in another order: B=1 H=32 S=512 D=64 causal fp16 7.9
+        // -> 8.2 us, B=2 H=16 S=256 D=128 8.0 -> 8.2, B=8 H=32/8 S=512 D=128 causal bf16 40.3 -> 42.4)
+        vec8 kf[KBG][KS];
 #pragma unroll
-    for (int ks0 = 0; ks0 < KS; ks0 += KSG) {
-      vec8 kf[KBG][KS];
+        for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-      for (int ks = ks0; ks < ks0 + KSG; ks++)
+          for (int kb = 0; kb < KBG; kb++)
+            kf[kb][ks] = *reinterpret_cast<const vec8 *>(&Ks[k_frag_off + (kb0 + kb) * 32 * LDK + 16 * ks]);
 #pragma unroll
-        for (int kb = 0; kb < KBG; kb++)
-          kf[kb][ks] = *reinterpret_cast<const vec8 *>(&Ks[k_frag_off + (kb0 + kb) * 32 * LDK + 16 * ks]);
-      // (with one wave per SIMD the compiler sinks every read to its MFMA and waits for it there: B=1 H=16/8 S=1500 D=256
-      // causal bf16 54.2 -> 52.8 us; all sixteen reads at once spill and measure the same)
-      if constexpr (D > 128 && WPS == 1) __builtin_amdgcn_sched_barrier(0);
+        for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-      for (int ks = ks0; ks < ks0 + KSG; ks++)
-#pragma unroll
-        for (int kb = 0; kb < KBG; kb++) {
+          for (int kb = 0; kb < KBG; kb++) {
 #ifdef LMH_FOLD_SCALE
-          sacc[kb0 + kb] = MT::mfma(kf[kb][ks], qreg[ks], ks == 0 ? neg_mc16 : sacc[kb0 + kb]);
+            sacc[kb0 + kb] = MT::mfma(kf[kb][ks], qreg[ks], ks == 0 ? neg_mc16 : sacc[kb0 + kb]);
 #else
-          sacc[kb0 + kb] = MT::mfma(kf[kb][ks], qreg[ks], sacc[kb0 + kb]);
+            sacc[kb0 + kb] = MT::mfma(kf[kb][ks], qreg[ks], sacc[kb0 + kb]);
 #endif
+          }
+      } else {
+        constexpr int KSG = WPS == 2 ? 4 : KS / 2;  // long rows: as many k-steps at a time as the registers hold
+#pragma unroll
+        for (int ks0 = 0; ks0 < KS; ks0 += KSG) {
+          vec8 kf[KBG][KS];
+#pragma unroll
+          for (int ks = ks0; ks < ks0 + KSG; ks++)
+#pragma unroll
+            for (int kb = 0; kb < KBG; kb++)
+              kf[kb][ks] = *reinterpret_cast<const vec8 *>(&Ks[k_frag_off + (kb0 + kb) * 32 * LDK + 16 * ks]);
+          // (with one wave per SIMD the compiler sinks every read to its MFMA and waits for it there: B=1 H=16/8 S=1500
+          // D=256 causal bf16 54.2 -> 52.8 us; all sixteen reads at once spill and measure the same)
+          if constexpr (WPS == 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int ks = ks0; ks < ks0 + KSG; ks++)
+#pragma unroll
+            for (int kb = 0; kb < KBG; kb++) {
+#ifdef LMH_FOLD_SCALE
+              sacc[kb0 + kb] = MT::mfma(kf[kb][ks], qreg[ks], ks == 0 ? neg_mc16 : sacc[kb0 + kb]);
+#else
+              sacc[kb0 + kb] = MT::mfma(kf[kb][ks], qreg[ks], sacc[kb0 + kb]);
+#endif
+            }
         }
+      }
     }
 
     // The next V tile is rewritten here, in the shadow of the MFMAs just issued. (After the last tile this rewrites
