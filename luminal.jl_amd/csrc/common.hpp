@@ -181,7 +181,7 @@ __host__ __device__ inline int q_head_of(int kvh, int g, int Hq, int Hkv, int he
 }
 
 __device__ __forceinline__ void request_args(const Deal &t) {
-  asm volatile("" ::"s"(t.heads), "s"(t.tiles), "s"(t.snake), "s"(t.whole.m), "s"(t.whole.s), "s"(t.all.m), "s"(t.all.s), "s"(t.hq.m), "s"(t.hq.s), "s"(t.cus.m), "s"(t.cus.s));
+  asm volatile("" ::"s"(t.heads), "s"(t.tiles), "s"(t.n_per_xcd), "s"(t.snake), "s"(t.all.m), "s"(t.all.s), "s"(t.hq.m), "s"(t.hq.s), "s"(t.cus.m), "s"(t.cus.s));
 }
 
 // Launchers: validate nothing (api.hip already did), pick an instantiation, enqueue on `stream`.

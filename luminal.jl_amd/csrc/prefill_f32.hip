@@ -55,7 +55,7 @@ __global__ __launch_bounds__(64 * RW * KG, 1) void prefill_f32_kernel(PrefillArg
 
   // ---- which (b, hq, query tile): a head's tiles on one XCD, causal tiles heaviest first (see prefill_mfma.hip) ----
   int bh, tile_rank;
-  if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3, &bh, &tile_rank)) return;
+  if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, &bh, &tile_rank)) return;
   const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
   const int q_tile = CAUSAL ? (deal.tiles - 1 - tile_rank) : tile_rank;

@@ -132,7 +132,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(PrefillArgs 
 #endif
   // ---- which (b, hq, query tile) this workgroup owns ----
   int bh, tile_rank;
-  if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3, &bh, &tile_rank)) return;
+  if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, &bh, &tile_rank)) return;
   const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
   // Causal rows grow with the query index: long rows are issued first so that the short ones fill
@@ -922,7 +922,7 @@ __global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a
   __shared__ __attribute__((aligned(16))) uint16_t Vs2[2][BT * LDV];
 
   int bh, pair;
-  if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3, &bh, &pair)) return;
+  if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, &bh, &pair)) return;
   const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
   // tile p with tile n - 1 - p; with an odd number of tiles the middle one is alone (its workgroup has no early tile)

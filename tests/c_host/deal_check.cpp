@@ -14,15 +14,15 @@ using namespace lmh;
 static void launch(int B, int Hq, int tiles, int resident, int cus) {
   const Deal t = make_deal(B, Hq, tiles, resident, cus);
   const int64_t heads = (int64_t)B * Hq, grid = deal_grid(heads, tiles);
-  const int n_per_xcd = (int)(grid >> 3);
   std::vector<uint8_t> seen(heads * tiles, 0), by_head(heads * tiles, 0);
-  int64_t out = 0, twice = 0, split = 0, missing = 0;
+  int64_t out = 0, twice = 0, split = 0, moved = 0, missing = 0;
   for (int64_t bid = 0; bid < grid; bid++) {
     int head = -1, rank = -1;
-    if (deal_tile(t, (int)(bid & 7), (int)(bid >> 3), n_per_xcd, &head, &rank)) {
+    if (deal_tile(t, (int)(bid & 7), (int)(bid >> 3), &head, &rank)) {
       if (head < 0 || head >= heads || rank < 0 || rank >= tiles) out++;
       else if (seen[(int64_t)head * tiles + rank]++) twice++;
       else if ((int)((uint32_t)head / t.hq) != head / Hq) split++;
+      else if (head < (heads & ~7) && (head & 7) != (bid & 7)) moved++;
     }
     if (deal_tile_by_head((int)heads, tiles, (int)(heads / 8 * tiles), (int)(bid & 7), (int)(bid >> 3), &head, &rank)) {
       if (head < 0 || head >= heads || rank < 0 || rank >= tiles) out++;
@@ -31,9 +31,9 @@ static void launch(int B, int Hq, int tiles, int resident, int cus) {
   }
   for (auto *v : {&seen, &by_head})
     for (uint8_t x : *v) missing += x == 0;
-  if (out || twice || split || missing)
-    printf("wrong B=%d Hq=%d tiles=%d: %lld out of range, %lld twice, %lld missing, %lld of the wrong sequence\n", B, Hq, tiles,
-           (long long)out, (long long)twice, (long long)missing, (long long)split);
+  if (out || twice || split || moved || missing)
+    printf("wrong B=%d Hq=%d tiles=%d: %lld out of range, %lld twice, %lld missing, %lld of the wrong sequence, %lld on the wrong XCD\n", B, Hq, tiles,
+           (long long)out, (long long)twice, (long long)missing, (long long)split, (long long)moved);
   else printf("ok\n");
 }
 
