@@ -198,6 +198,7 @@ int launch_prefill_w64(const PrefillArgs &a, hipStream_t stream);
 #endif
 bool prefill_f32_mfma_supported(int dtype, int D);
 int launch_prefill_f32_mfma(const PrefillArgs &a, hipStream_t stream);
+int launch_prefill_f32_full(const PrefillArgs &a, int key_groups, hipStream_t stream);  // no mask, head dim <= 128
 int launch_prefill_valu(const PrefillArgs &a, int dtype, hipStream_t stream);
 int launch_decode(const DecodeArgs &a, int dtype, hipStream_t stream);
 int launch_rope(const RopeArgs &a, int dtype, hipStream_t stream);

@@ -16,7 +16,8 @@
 //   * registers: 64 for Q and 64 for O at head dim 256, which the larger blocks cannot hold.
 // Measured, us, with 32 x 32 blocks -> now: B=1 H=8 S=128 D=64 causal 7.3 -> 5.5, B=2 H=12 S=1023 D=80 103 -> 77, B=1 H=16
 // S=2048 D=64 causal 143 -> 95, B=1 H=8 S=1000 D=128 causal 76 -> 38, B=4 H=20 448 x 1500 D=64 194 -> 148, B=1 H=32 S=4096
-// D=96 causal 822 -> 803 (128 TFLOP/s, 82 % of the peak); B=2 H=16 S=1024 D=128 without a mask 136 -> 141.
+// D=96 causal 822 -> 803 (128 TFLOP/s, 82 % of the peak). Without a mask, where all workgroups are equally long and fill the
+// chip, the 32 x 32 blocks stay ahead by 1 to 13 %: prefill_f32_full.hip.
 //
 // Layout of the 16 x 16 x 4 product: lane (n = lane % 16, g = lane / 16); A and B give element k = g of row / column n, the
 // result register i is row 4 g + i of column n. The head dim is contracted in the order d = 16 j + 4 g + e, so a 128-bit K
@@ -330,7 +331,9 @@ int launch_form(const PrefillArgs &a, hipStream_t stream) {
 // Expected time of a form: the walk of the busiest SIMD, in keys of one wave, times a weight for what the form pays per key
 // (64-row workgroups = 1). Without a mask the workgroups are equal and go round in whole rounds of the CUs; causal ones end
 // up near the mean of their lengths, a little above it where every one is resident from the start and by a quarter of the
-// longest where they turn over. Fewer than three waves per SIMD leave some of the LDS latency in sight.
+// longest where they turn over. Causal launches with fewer than three waves per SIMD leave some of the LDS latency in sight,
+// the equally long ones up to head dim 128 with fewer than two (D=96, B=1 H=16 S=1024: 64 rows, one wave, 70 us, 32 rows x 2 key groups, two,
+// 68; B=1 H=32 S=1024: two waves in 128 rows 113, in 64 rows 116, four in 32 rows 122).
 template <int D, int RW, int KG, int NK>
 double form_cost(const PrefillArgs &a, double weight) {
   constexpr int tile = 16 * NK * KG;
@@ -339,7 +342,7 @@ double form_cost(const PrefillArgs &a, double weight) {
   const double wgs = (double)a.B * a.Hq * ((a.Sq + 16 * RW - 1) / (16 * RW));
   const double walk = (double)((keys + tile - 1) / tile) * tile / KG * (RW * KG / 4);
   const double occupancy = fmin(wgs / n_cus, resident<D, RW, KG, NK>()) * (RW * KG / 4);
-  if (keys >= 256 && occupancy < 3.0) weight *= 1.15;
+  if (keys >= 256 && occupancy < (a.causal || D > 128 ? 3.0 : 2.0)) weight *= 1.15;
   if (!a.causal) return weight * walk * ceil(wgs / n_cus);
   const double mean = 0.5 * walk * wgs / n_cus;
   if (wgs <= n_cus) return weight * walk;
@@ -358,11 +361,24 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
     if (form_cost<D, 2, 2, 1>(a, w32) < form_cost<D, 4, 1, 1>(a, 1.0)) return launch_form<D, 2, 2, 1>(a, stream);
     return launch_form<D, 4, 1, 1>(a, stream);
   } else {
-    if (tiles(128) >= 4 * n_cus) return launch_form<D, 8, 1, 2>(a, stream);
+    // Without a mask, in blocks of 32 x 32 (prefill_f32_full.hip), where the head dim needs no more padding for it: a wave walks
+    // twice the rows per key. Weights from launches that fill the chip (D=96, B=1 H=32 S=1024: 106 us against 113 for the
+    // 128-row form here, two key groups on B=1 H=16 S=1024 61 against 68).
+    constexpr bool kFull = D == 64 || D == 96 || D == 128;
+    double f128 = INFINITY, f64 = INFINITY;
+    if (kFull && !a.causal) {
+      auto cost = [&](int rows, int tile, double weight) {
+        return weight * (double)((a.Sk + tile - 1) / tile) * tile * (rows / 64) * ceil((double)tiles(rows) / n_cus);
+      };
+      f128 = cost(128, 32, 0.92);
+      f64 = cost(64, 64, tiles(64) <= n_cus ? 1.07 : INFINITY);
+    }
+    if (tiles(128) >= 4 * n_cus) return kFull && !a.causal ? launch_prefill_f32_full(a, 1, stream) : launch_form<D, 8, 1, 2>(a, stream);
     const bool few32 = tiles(32) <= (a.causal ? 2 : 1) * n_cus, few16 = tiles(16) <= 2 * n_cus;
     const double c128 = form_cost<D, 8, 1, 2>(a, 0.96), c64 = form_cost<D, 4, 1, 2>(a, 1.0), c32 = form_cost<D, 2, 2, 1>(a, w32),
                  c32x2 = form_cost<D, 2, 2, 2>(a, few32 ? 1.0 : D <= 64 ? 1.15 : 1.4), c16 = form_cost<D, 1, 4, 1>(a, few16 ? 1.2 : D <= 64 ? 1.5 : 1.8);
     const double best = fmin(fmin(c128, c64), fmin(fmin(c32, c32x2), c16));
+    if (fmin(f128, f64) < best) return launch_prefill_f32_full(a, f64 < f128 ? 2 : 1, stream);
     if (best == c128) return launch_form<D, 8, 1, 2>(a, stream);
     if (best == c64) return launch_form<D, 4, 1, 2>(a, stream);
     if (best == c32) return launch_form<D, 2, 2, 1>(a, stream);

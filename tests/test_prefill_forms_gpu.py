@@ -86,3 +86,33 @@ def test_head_counts_that_are_no_multiple_of_the_xcds(lm, hip, oracle, B, Hq, Hk
     q, k, v = inputs(oracle, (B, Hq, Sq, D), (B, Hkv, Sk, D), dtype, 33000 + Sq + Hq)
     assert kernel in plan(lm, q, k, dtype, causal, False)
     assert rel_err(run(lm, hip, q, k, v, dtype, causal), oracle.flash_attn(q, k, v, causal=causal, nthreads=NT)) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,form", [
+    (1, 32, 8, 1000, 40, 64, "D=64, key groups=1> rows=128"), (2, 15, 15, 970, 65, 56, "D=64, key groups=1> rows=128"),
+    (4, 16, 4, 500, 33, 96, "D=96, key groups=1> rows=128"), (1, 31, 1, 1024, 97, 88, "D=96, key groups=1> rows=128"),
+    (8, 32, 32, 127, 64, 128, "D=128, key groups=1> rows=128"), (3, 10, 5, 1001, 95, 120, "D=128, key groups=1> rows=128"),
+    (2, 8, 2, 1000, 320, 64, "D=64, key groups=2> rows=64"), (1, 16, 8, 993, 319, 96, "D=96, key groups=2> rows=64"),
+    (3, 7, 7, 640, 320, 128, "D=128, key groups=2> rows=64"),
+])
+def test_fp32_without_a_mask_in_blocks_of_32(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, form):
+    q, k, v = inputs(oracle, (B, Hq, Sq, D), (B, Hkv, Sk, D), "f32", 33500 + Sq + D)
+    assert "prefill_f32_full_kernel<" + form in plan(lm, q, k, "f32", False, False)
+    # a last tile with keys for both key groups, for one, and a sequence without a key (zeros; the oracle wants one)
+    lens = np.array([(Sk - 30, 0, 32, Sk)[i % 4] for i in range(B)] if B > 1 else [(Sk + 1) // 2], np.int32)
+    for kv_len in (None, lens):
+        got = run(lm, hip, q, k, v, "f32", False, kv_len=None if kv_len is None else list(kv_len))
+        want = oracle.flash_attn(q, k, v, kv_len=None if kv_len is None else np.maximum(kv_len, 1), nthreads=NT)
+        if kv_len is not None:
+            want[kv_len == 0] = 0
+        assert rel_err(got, want) <= TOL["f32"]
+
+
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("Hq,Sk,D", [(32, 64, 64), (32, 64, 96), (16, 320, 128)])
+def test_blocks_of_32_rotate_their_queries_in_registers(lm, hip, oracle, Hq, Sk, D, interleaved):
+    q, k, v = inputs(oracle, (1, Hq, 1000, D), (1, Hq, Sk, D), "f32", 33600 + D)
+    assert "prefill_f32_full_kernel" in plan(lm, q, k, "f32", False, True)
+    got = run(lm, hip, q, k, v, "f32", False, rope=(7, interleaved))
+    q_rot = rotated_on_device(lm, hip, q, "f32", prev_seq=7, interleaved=interleaved)
+    np.testing.assert_array_equal(got, run(lm, hip, q_rot, k, v, "f32", False))
