@@ -15,7 +15,7 @@
 //   * padding: head dims go in steps of 16, where 32 x 32 blocks of O^T pad 80 to 96 and 112 to 128;
 //   * registers: 64 for Q and 64 for O at head dim 256, which the larger blocks cannot hold.
 // Measured, us, with 32 x 32 blocks -> now: B=1 H=8 S=128 D=64 causal 7.3 -> 5.5, B=2 H=12 S=1023 D=80 103 -> 77, B=1 H=16
-// S=2048 D=64 causal 143 -> 95, B=1 H=8 S=1000 D=128 causal 76 -> 38, B=4 H=20 448 x 1500 D=64 194 -> 148, B=1 H=32 S=4096
+// S=2048 D=64 causal 143 -> 85, B=1 H=8 S=1000 D=128 causal 76 -> 38, B=4 H=20 448 x 1500 D=64 194 -> 148, B=1 H=32 S=4096
 // D=96 causal 822 -> 803 (128 TFLOP/s, 82 % of the peak). Without a mask, where all workgroups are equally long and fill the
 // chip, the 32 x 32 blocks stay ahead by 1 to 13 %: prefill_f32_full.hip.
 //

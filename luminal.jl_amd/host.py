@@ -551,6 +551,14 @@ class Graph:
     def lowered(self, wanted, given):
         """lowering.lower(self, wanted, given), kept while the graph stays as it is: its ops and what they hold, what they read,
         shapes and types. Safe between threads: (graph as it was, {question: answer}) is replaced as a whole."""
+        steps = []
+        for i, node in enumerate(self.nodes):
+            if isinstance(node.op, HostOp):
+                break
+            if i not in given and not isinstance(node.op, InputTensor):
+                steps.append(lowering.NodeOp(i, node.inputs))
+        else:  # nothing around the attention nodes: one by one, and no reason to keep it
+            return steps, set()
         state = ([(node.op, *vars(node.op).values()) for node in self.nodes], [[*node.inputs] for node in self.nodes],
                  [*self.shapes], [*self.dtypes])
         kept = self._lowered
@@ -640,7 +648,7 @@ class SelfAttention:
     into heads (a column-major reshape, so the head index is the fast one), the permutes — and everything between them
     (rotary embedding of Q and K, repeat_kv, scaled causal softmax attention, src/NN.jl:356-382) replaced by
     self_attention_core: GQA without copies of K/V, the queries rotated inside the attention kernel. `attn_dtype` is
-    the element type attention runs in (the reference is fp32 only); the projections stay fp32 on the host."""
+    the element type attention runs in (the reference is fp32 only); the projections are fp32 products on the device."""
 
     def __init__(self, hidden, n_heads, n_kv_heads, graph, attn_dtype="f32"):
         if hidden % n_heads or n_heads % n_kv_heads:
@@ -656,7 +664,7 @@ class SelfAttention:
         batch, seq, hidden = x.shape
         dt = self.attn_dtype
 
-        def heads(proj, n):  # (B, S, n*D) -> (B, n, S, D), uploaded in the element type attention reads
+        def heads(proj, n):  # (B, S, n*D) -> (B, n, S, D), in the element type attention reads
             return permute(reshape(proj(x), (batch, seq, n, self.head_dim)), (0, 2, 1, 3), dtype=dt)
 
         queries, keys, values = heads(self.q_proj, self.n_heads), heads(self.k_proj, self.n_kv_heads), heads(self.v_proj, self.n_kv_heads)
@@ -688,7 +696,7 @@ class WhisperAttention:
         k_in = x if keys_from is None else keys_from
         v_in = x if values_from is None else values_from
 
-        def heads(proj, t):  # (B, S, H*D) -> (B, H, S, D), uploaded in the element type attention reads
+        def heads(proj, t):  # (B, S, H*D) -> (B, H, S, D), in the element type attention reads
             return permute(reshape(proj(t), (t.shape[0], t.shape[1], self.n_heads, self.head_dim)), (0, 2, 1, 3),
                            dtype=self.attn_dtype)
 

@@ -415,8 +415,6 @@ def lower(graph, wanted=(), given=()):
     """(steps, virtual): the launches that compute every node of `graph` that is `wanted` or has no or several users, in
     order, and the nodes that disappeared into one of them. `given` nodes have values already."""
     given = set(given)
-    if not any(hasattr(node.op, "compute") for node in graph.nodes):  # nothing around the attention nodes
-        return one_by_one(graph, given), set()
     work = _Lowering(graph, set(wanted), given)
     steps = work.steps()
     return steps, work.virtual
