@@ -18,7 +18,11 @@ inline FastDiv fast_div(uint32_t d) {
 }
 __host__ __device__ inline uint32_t operator/(uint32_t n, FastDiv f) { return (uint32_t)(((uint64_t)(2 * n) * f.m) >> 32) >> f.s; }
 
-// How a flash attention launch deals its (b, hq) pairs ("heads") and their query tiles to workgroups.
+// How a flash attention launch deals its (b, hq) pairs ("heads") and their query tiles to workgroups. The kernels take it in front
+// of their other arguments: a workgroup reads its argument block as one batch of scalar loads in the order of the block, and
+// waits for all of it. Behind PrefillArgs the same block took launches of less than 10 us 0.1 to 0.2 us longer when the host
+// enqueued them one by one (B=1 H=8 S=128 D=64 causal fp16 5.87 us, in front 5.67; B=1 H=32 S=512 8.08 and 7.89; the number of
+// words makes no difference, nor does either in a recorded graph).
 struct Deal {
   int32_t heads, tiles;
   int32_t n_per_xcd;     // workgroups of an XCD

@@ -40,7 +40,7 @@ constexpr float kLazyRescale = 8.0f;      // the running max is raised only when
 // RW waves own 16 rows each, KG waves share 16 rows by taking the kg-th 16 NK keys of every staged tile of 16 NK KG keys.
 template <int D, int RW, int KG, int NK> constexpr int tile_blocks() { return (16 * NK * KG * (D / 4 + 1) + 63) / 64; }  // 1 KB blocks
 template <int D, bool CAUSAL, int RW, int KG, int NK>
-__global__ __launch_bounds__(64 * RW * KG, 1) void prefill_f32_kernel(PrefillArgs a, Deal deal) {
+__global__ __launch_bounds__(64 * RW * KG, 1) void prefill_f32_kernel(Deal deal, PrefillArgs a) {
   request_args(a);
   request_args(deal);
   constexpr int NW = RW * KG;
@@ -322,8 +322,8 @@ int launch_form(const PrefillArgs &a, hipStream_t stream) {
   if (plan_only("prefill_f32_kernel<D=%d, %s, key groups=%d> rows=%d, workgroups=%u", D, a.causal ? "causal" : "full", KG, 16 * RW, grid.x))
     return LMH_OK;
   const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? resident<D, RW, KG, NK>() : 0, device_cu_count());
-  if (a.causal) hipLaunchKernelGGL((prefill_f32_kernel<D, true, RW, KG, NK>), grid, block, 0, stream, a, deal);
-  else hipLaunchKernelGGL((prefill_f32_kernel<D, false, RW, KG, NK>), grid, block, 0, stream, a, deal);
+  if (a.causal) hipLaunchKernelGGL((prefill_f32_kernel<D, true, RW, KG, NK>), grid, block, 0, stream, deal, a);
+  else hipLaunchKernelGGL((prefill_f32_kernel<D, false, RW, KG, NK>), grid, block, 0, stream, deal, a);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }

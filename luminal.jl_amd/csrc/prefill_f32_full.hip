@@ -32,7 +32,7 @@ typedef float floatx4_t __attribute__((ext_vector_type(4)));
 // 64 rows per CU: the waves own 2 x 32 rows, tiles have 64 keys, and each half of the waves takes 32 of them with a running max,
 // sum and output of its own, folded through LDS at the end.
 template <int D, int KG>
-__global__ __launch_bounds__(256, (KG > 1 ? 1 : D <= 96 ? 3 : 2)) void prefill_f32_full_kernel(PrefillArgs a, Deal deal) {
+__global__ __launch_bounds__(256, (KG > 1 ? 1 : D <= 96 ? 3 : 2)) void prefill_f32_full_kernel(Deal deal, PrefillArgs a) {
   request_args(a);
   request_args(deal);
   constexpr int BM = 128 / KG;      // query rows per workgroup
@@ -297,7 +297,7 @@ int launch_form(const PrefillArgs &a, hipStream_t stream) {
   dim3 grid((uint32_t)wgs), block(256);
   if (plan_only("prefill_f32_full_kernel<D=%d, key groups=%d> rows=%d, workgroups=%u", D, KG, 128 / KG, grid.x)) return LMH_OK;
   const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, 0, device_cu_count());
-  hipLaunchKernelGGL((prefill_f32_full_kernel<D, KG>), grid, block, 0, stream, a, deal);
+  hipLaunchKernelGGL((prefill_f32_full_kernel<D, KG>), grid, block, 0, stream, deal, a);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }

@@ -101,7 +101,7 @@ __device__ inline void rotate_q_fragments_with_table(typename MT::vec8 (&qreg)[D
 // WPS: waves per SIMD the register budget is set for (3 x 4 waves, 2 x 8 waves or 1 x 8 waves per CU).
 template <int D, int NW> constexpr int default_wps() { return D > 128 ? 1 : D > 96 ? 2 : NW == 8 ? 4 : 3; }
 template <typename MT, int D, bool CAUSAL, int KSPLIT, int NW, int WPS>
-__global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(PrefillArgs a, Deal deal) {
+__global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, PrefillArgs a) {
   request_args(a);
   request_args(deal);
   using vec8 = typename MT::vec8;
@@ -1297,9 +1297,9 @@ int launch_split(const PrefillArgs &a, hipStream_t stream) {
     return LMH_OK;
   const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? 4 * WPS / NW : 0, device_cu_count());
   if (a.causal)
-    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS>), grid, block, 0, stream, a, deal);
+    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS>), grid, block, 0, stream, deal, a);
   else
-    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, false, KSPLIT, NW, WPS>), grid, block, 0, stream, a, deal);
+    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, false, KSPLIT, NW, WPS>), grid, block, 0, stream, deal, a);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }

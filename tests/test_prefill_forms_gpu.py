@@ -116,3 +116,13 @@ def test_blocks_of_32_rotate_their_queries_in_registers(lm, hip, oracle, Hq, Sk,
     got = run(lm, hip, q, k, v, "f32", False, rope=(7, interleaved))
     q_rot = rotated_on_device(lm, hip, q, "f32", prev_seq=7, interleaved=interleaved)
     np.testing.assert_array_equal(got, run(lm, hip, q_rot, k, v, "f32", False))
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+def test_launches_with_very_many_heads(lm, hip, oracle, dtype):
+    """More heads than a 32-bit reciprocal divides exactly: every one of them is computed."""
+    B, H, Sk, D = 16384, 32, 2, 8
+    q, k, v = inputs(oracle, (B, H, 1, D), (B, H, Sk, D), dtype, 34000)
+    w = np.exp((q.astype(np.float64) * k).sum(-1, keepdims=True) * lm.default_scale(D))
+    want = (w * v).sum(2, keepdims=True) / w.sum(2, keepdims=True)
+    assert rel_err(run(lm, hip, q, k, v, dtype, False), want) <= TOL[dtype]
