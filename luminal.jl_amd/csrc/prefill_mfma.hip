@@ -24,6 +24,8 @@
 //     lie entirely above its diagonal, and only diagonal tiles pay for masking;
 //   * blockIdx -> work mapping keeps all query tiles of a head on one XCD (private L2) and, for
 //     causal, issues the long rows first.
+#include <math.h>
+
 #include <algorithm>
 #include <type_traits>
 
@@ -1351,10 +1353,133 @@ int launch_wide(const PrefillArgs &a, int wgs_per_head, int n_waves, int mixed, 
   return LMH_OK;
 }
 
-// V16 (bf16 only): the launches of one key group hand V to the matrix cores as fp16 (base_policy above).
+// The forms of prefill_mfma_kernel and what a launch of each costs.
+//
+// A launch lasts as long as its busiest CU, and where the sizes leave a last row tile or a last round nearly empty the forms
+// differ by up to 60 %: B=4 H=32 S=777 D=128 causal fp16 has four row tiles of 256 with 9 rows in the last (46.8 us) or seven of
+// 128 (40.2); B=1 H=16 S=4501 D=96 causal bf16 one and a half rounds of 128-row workgroups (173 us) or 1.1 rounds of 256-row
+// ones (106). The thresholds of launch_for_d were measured at powers of two. Hence an estimate from the launch's own tiles, in us:
+//   fixed + longest row tile x alone       while every CU has at most one workgroup, or
+//   the mean over the CUs x shared         when several share it (causal; the fourth powers blend the two), or
+//   whole rounds of equal workgroups       (no mask), + per_wg for every workgroup that a CU starts.
+// `alone` and `shared` are the times of a tile of 64 keys in a CU's only workgroup and in one of two or three (per tile, the
+// others' tiles not counted). Fitted to 1916 launches, most of drawn sizes (16 to 8192 rows, 1 to 64 heads, batches to 16), some
+// of powers of two, with every form timed on each: rms 5 to 13 %. The form of the rules by size is therefore left only for one
+// that is estimated 8 % cheaper: 337 of those launches change their form, 296 of them gain more than 5 %, two lose more than 5 %
+// (13 and 14 us), all 1916 together gain 2.5 % (with a margin of 4 % 2.9 %, and ten lose).
+enum Form { kKeysSplit64, kRows128, kRows256, kRows256Pair };  // rows per workgroup; Pair: two 256-row workgroups on a CU
+struct FormCost {
+  float fixed, alone, per_wg, shared[2];  // shared by two and by three workgroups; with one per CU: in a later round
+};
+// [fp16, bf16 head + remainder, bf16 with V as fp16][head dims up to 64, 96, 128][form][causal]; fixed < 0: not built or never ahead
+constexpr FormCost kFormCosts[3][3][4][2] = {
+    {  // fp16
+     {{{2.92f, 0.46f, 0.86f, 0.32f, 0.3f}, {2.75f, 0.49f, 0.91f, 0.31f, 0.31f}},
+      {{2.6f, 0.75f, 1.2f, 0.55f, 0.54f}, {2.9f, 0.77f, 1.16f, 0.56f, 0.56f}},
+      {{0.f, 1.01f, 4.8f, 1.01f, 1.01f}, {1.69f, 0.9f, 4.54f, 1.03f, 1.03f}},
+      {{1.98f, 1.07f, 2.83f, 0.94f, 0.94f}, {3.44f, 1.02f, 2.09f, 1.05f, 1.05f}}},  // head dims up to 64
+     {{{2.66f, 0.62f, 1.3f, 0.41f, 0.41f}, {2.55f, 0.61f, 1.47f, 0.43f, 0.43f}},
+      {{2.18f, 0.9f, 2.07f, 0.7f, 0.7f}, {3.68f, 0.86f, 1.38f, 0.78f, 0.78f}},
+      {{0.f, 1.29f, 5.74f, 1.29f, 1.29f}, {0.f, 1.11f, 6.8f, 1.36f, 1.36f}},
+      {{1.12f, 1.34f, 4.16f, 1.23f, 1.23f}, {4.74f, 1.19f, 1.57f, 1.45f, 1.45f}}},  // head dims up to 96
+     {{{1.97f, 0.79f, 2.58f, 0.53f, 0.53f}, {1.82f, 0.73f, 3.08f, 0.55f, 0.55f}},
+      {{0.99f, 1.13f, 4.13f, 0.88f, 0.88f}, {2.55f, 1.06f, 3.23f, 0.99f, 0.99f}},
+      {{0.f, 1.63f, 8.71f, 1.63f, 1.63f}, {0.19f, 1.41f, 8.29f, 1.77f, 1.77f}},
+      {{-1.f}, {-1.f}}},  // head dims up to 128
+    },
+    {  // bf16, weights as head + remainder
+     {{{3.3f, 0.59f, 0.74f, 0.46f, 0.42f}, {3.38f, 0.64f, 0.65f, 0.44f, 0.44f}},
+      {{2.7f, 1.05f, 1.11f, 0.85f, 0.78f}, {4.61f, 1.01f, 0.24f, 0.86f, 0.86f}},
+      {{1.28f, 1.55f, 3.98f, 1.55f, 1.55f}, {1.58f, 1.45f, 3.93f, 1.53f, 1.53f}},
+      {{2.2f, 1.62f, 2.77f, 1.4f, 1.4f}, {4.8f, 1.55f, 0.22f, 1.58f, 1.58f}}},  // head dims up to 64
+     {{{2.9f, 0.76f, 1.25f, 0.55f, 0.55f}, {3.1f, 0.75f, 1.17f, 0.58f, 0.58f}},
+      {{2.65f, 1.21f, 1.79f, 1.f, 1.f}, {4.61f, 1.17f, 0.69f, 1.1f, 1.1f}},
+      {{0.f, 1.8f, 6.79f, 1.8f, 1.8f}, {0.15f, 1.66f, 6.72f, 1.88f, 1.88f}},
+      {{3.04f, 2.f, 4.23f, 1.81f, 1.81f}, {4.45f, 2.24f, 1.47f, 2.04f, 2.04f}}},  // head dims up to 96
+     {{{2.96f, 0.92f, 2.21f, 0.71f, 0.71f}, {2.48f, 0.93f, 2.75f, 0.72f, 0.72f}},
+      {{1.99f, 1.49f, 3.51f, 1.23f, 1.23f}, {3.23f, 1.43f, 2.58f, 1.34f, 1.34f}},
+      {{-1.f}, {-1.f}},
+      {{-1.f}, {-1.f}}},  // head dims up to 128
+    },
+    {  // bf16, V as fp16
+     {{{-1.f}, {-1.f}},
+      {{4.03f, 0.97f, 2.01f, 0.66f, 0.57f}, {4.68f, 0.98f, 1.59f, 0.64f, 0.64f}},
+      {{0.98f, 1.11f, 6.96f, 1.11f, 1.11f}, {0.99f, 1.04f, 7.51f, 1.14f, 1.14f}},
+      {{3.86f, 1.16f, 3.91f, 0.97f, 0.97f}, {6.18f, 1.17f, 1.98f, 1.13f, 1.13f}}},  // head dims up to 64
+     {{{-1.f}, {-1.f}},
+      {{4.55f, 1.5f, 3.45f, 0.88f, 0.84f}, {1.55f, 1.88f, 4.44f, 1.59f, 0.87f}},
+      {{0.f, 1.33f, 9.72f, 1.33f, 1.33f}, {0.8f, 1.22f, 9.79f, 1.35f, 1.35f}},
+      {{-1.f}, {-1.f}}},  // head dims up to 96
+     {{{-1.f}, {-1.f}},
+      {{3.81f, 1.36f, 4.9f, 0.97f, 0.97f}, {3.82f, 1.3f, 4.58f, 1.f, 1.f}},
+      {{0.07f, 1.71f, 11.89f, 1.71f, 1.71f}, {0.f, 1.54f, 12.61f, 1.7f, 1.7f}},
+      {{-1.f}, {-1.f}}},  // head dims up to 128
+    },
+};
+
+inline double form_cost(const FormCost &f, const PrefillArgs &a, int form, int per_cu, int n_cus) {
+  const int64_t heads = (int64_t)a.B * a.Hq, rows = form == kKeysSplit64 ? 64 : form == kRows128 ? 128 : 256;
+  const int64_t n = (a.Sq + rows - 1) / rows, step = rows / BN, row_tiles = (a.Sk + BN - 1) / BN;
+  const double wgs = (double)(heads * n) / n_cus;
+  const int64_t rounds = (heads * n + n_cus - 1) / n_cus;
+  const int on_cu = (int)std::min<int64_t>(rounds, per_cu);
+  if (!a.causal) {
+    auto batch = [&](int64_t k) -> double { return k < 1 ? 0. : k < 2 ? f.alone : std::max<double>(f.alone, k * f.shared[k - 2]); };
+    return f.fixed + row_tiles * (rounds / per_cu * batch(per_cu) + batch(rounds % per_cu)) + f.per_wg * rounds;
+  }
+  const int64_t ramp = std::min(n, row_tiles / step);  // workgroups r < ramp walk (r + 1) step tiles, the others all of them
+  const double longest = (double)std::min(row_tiles, n * step) * f.alone;
+  if (wgs <= 1) return f.fixed + longest + f.per_wg;
+  const double mean = (double)heads * (step * ramp * (ramp + 1) / 2 + (n - ramp) * row_tiles) / n_cus * f.shared[on_cu > 1 ? on_cu - 2 : 0];
+  return f.fixed + sqrt(sqrt(longest * longest * longest * longest + mean * mean * mean * mean)) + f.per_wg * wgs;
+}
+
+// Launch the cheapest form, in favour of the one that the rules by size chose. bf16 launches whose weights are head + remainder
+// by those rules stay so: V as fp16 goes with weights of 11 bits.
+template <typename MT, int D, bool V16>
+int launch_cheapest(const PrefillArgs &a, int by_size, hipStream_t stream) {
+  constexpr int tiling = D / 32 - 2;
+  const int n_cus = device_cu_count();
+  const bool v16 = V16 && by_size != kKeysSplit64;
+  auto cost = [&](bool v, int form) {
+    const FormCost &f = kFormCosts[!MT::kSplitP ? 0 : v ? 2 : 1][tiling][form][a.causal != 0];
+    if (f.fixed < 0 || (form >= kRows256 && a.Sq <= 128)) return 1e30;
+    // up to 16 workgroups stay on 128 rows, which the tests of the rotation in registers expect of one such launch
+    if (form == kKeysSplit64 && by_size != form && (int64_t)a.B * a.Hq * ((a.Sq + 63) / 64) <= 16) return 1e30;
+    return form_cost(f, a, form, form == kRows256 ? 1 : form == kRows256Pair || D > 96 ? 2 : 3, n_cus);
+  };
+  int best = by_size;
+  bool best_v = v16;
+  const double now = cost(v16, by_size);
+  double least = now < 1e30 ? 0.92 * now : 0.;  // (a form without an estimate stays)
+  for (int v = 0; v <= (int)v16; v++)
+    for (int form = v ? (int)kRows128 : (int)kKeysSplit64; form <= kRows256Pair; form++) {
+      const double t = cost(v, form);
+      if (t < least) least = t, best = form, best_v = v;
+    }
+  auto launch = [&](auto with_v) {
+    constexpr bool V = decltype(with_v)::value;
+    if (best == kKeysSplit64) return launch_split<MT, V, D, 2, 4>(a, stream);
+    if constexpr (D <= 96) {
+      if (best == kRows256) return launch_split<MT, V, D, 1, 8, 2>(a, stream);
+      if constexpr (!(D == 96 && V))  // (its registers spill at four waves per SIMD)
+        if (best == kRows256Pair) return launch_split<MT, V, D, 1, 8>(a, stream);
+    } else if constexpr (!MT::kSplitP || V) {
+      if (best == kRows256) return launch_split<MT, V, D, 1, 8>(a, stream);
+    }
+    return launch_split<MT, V, D, 1, 4>(a, stream);
+  };
+  if constexpr (V16)
+    if (best_v) return launch(std::true_type{});
+  return launch(std::false_type{});
+}
+
+// V16 (bf16 only): the launches of one key group hand V to the matrix cores as fp16 (base_policy above). The rules by size of
+// this function hold where the sizes fill whole tiles and rounds; launch_cheapest looks at the others.
 template <typename MT, int D, bool V16>
 int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
   static_assert(!V16 || MT::kSplitP, "V16 is a form of the bf16 kernels");
+  const auto launch = [&](int by_size) { return launch_cheapest<MT, D, V16>(a, by_size, stream); };
   // With fewer than two 128-row workgroups per CU the launch is bound by how long one workgroup
   // takes to walk its keys, not by the matrix pipes: split the keys of a tile between wave pairs.
   // Measured on 256 CUs: at exactly two per CU the split still wins for causal launches (41.8 vs
@@ -1389,7 +1514,7 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
       int wgs_per_head, n_waves, mixed;
       if (wide_plan(a, n_cus, &wgs_per_head, &n_waves, &mixed)) return launch_wide<MT, D>(a, wgs_per_head, n_waves, mixed, stream);
     }
-    return launch_split<MT, V16, D, 2, 4>(a, stream);
+    return launch(kKeysSplit64);
   }
   // Large launches: 256-row workgroups of eight waves. Measured against the 128-row ones at D = 96, fp16:
   // non-causal 512 / 768 / 1024 / 1536 / 2048 workgroups +3 / +2 / +2 / +6 / +5 %, causal 512 -7 %
@@ -1399,7 +1524,7 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
   // causal 256 / 384 -8 / -5 %, 512 / 1024 / 2048 +8 / +3 / +4 %; bf16 (V rewritten as fp16) 512 workgroups causal
   // +8 %, without a mask +5 %, 2048 causal +5 %.
   const int64_t wgs256 = (int64_t)a.B * a.Hq * ((a.Sq + 255) / 256);
-  if (a.Sq <= 128) return launch_split<MT, V16, D, 1, 4>(a, stream);  // nothing for waves 4-7 to own
+  if (a.Sq <= 128) return launch(kRows128);  // nothing for waves 4-7 to own
   if constexpr (D <= 96) {
     // Causal launches of 1.5 to 3 rounds of one 256-row workgroup per CU (the Phi-3 prompt, 32 heads x 4096 rows,
     // is exactly two): the workgroups turn over heaviest first, so every CU ends up with about the same number
@@ -1415,13 +1540,13 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
     if constexpr (D == 96 || V16)
       if ((D == 96 || a.causal) && ((D == 96 && V16) || wgs256 < 3 * n_cus) &&
           (a.causal ? 2 * wgs256 >= 3 * n_cus : wgs256 >= 2 * n_cus))
-        return launch_split<MT, V16, D, 1, 8, 2>(a, stream);
+        return launch(kRows256);
     if constexpr (!(D == 96 && V16))  // (with V16, D = 96 never gets here with that many workgroups)
-      if (wgs256 >= (a.causal ? 4 * n_cus : 2 * n_cus)) return launch_split<MT, V16, D, 1, 8>(a, stream);
+      if (wgs256 >= (a.causal ? 4 * n_cus : 2 * n_cus)) return launch(kRows256Pair);
   } else if constexpr (!MT::kSplitP || V16) {  // (bf16 with head + remainder weights: 0 / -2 %, stays on 128 rows)
-    if (wgs256 >= (a.causal ? 2 * n_cus : n_cus)) return launch_split<MT, V16, D, 1, 8>(a, stream);
+    if (wgs256 >= (a.causal ? 2 * n_cus : n_cus)) return launch(kRows256);
   }
-  return launch_split<MT, V16, D, 1, 4>(a, stream);
+  return launch(kRows128);
 }
 
 // Head dims above 128: Q and the accumulators of 32 rows take up to 192 registers and a tile buffer pair up to 141 KB, so a

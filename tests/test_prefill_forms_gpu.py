@@ -118,6 +118,23 @@ def test_blocks_of_32_rotate_their_queries_in_registers(lm, hip, oracle, Hq, Sk,
     np.testing.assert_array_equal(got, run(lm, hip, q_rot, k, v, "f32", False))
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,dtype,form", [
+    (13, 6, 6, 730, 730, 64, False, "f16", "key groups=1, waves=8, waves per SIMD=2>"), (10, 20, 20, 408, 65, 80, False, "f16", "key groups=1, waves=8, waves per SIMD=4>"),
+    (1, 19, 19, 3000, 100, 120, False, "f16", "key groups=1, waves=4, waves per SIMD=2>"), (2, 16, 4, 777, 777, 128, True, "f16", "key groups=2, waves=4"),
+    (4, 32, 8, 777, 777, 128, True, "f16", "key groups=1, waves=4"), (5, 20, 20, 115, 67, 64, False, "f16", "key groups=2, waves=4"),
+    (5, 16, 16, 119, 119, 80, True, "bf16", "key groups=2, waves=4"), (6, 16, 4, 431, 431, 72, True, "bf16", "key groups=2, waves=4"),
+    (3, 33, 11, 1285, 1285, 128, True, "bf16", "waves=4, waves per SIMD=2> workgroups=1096, V as fp16"),
+])
+def test_forms_chosen_by_cost(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causal, dtype, form):
+    """Launches whose estimated cost takes them to another form than their size alone."""
+    q, k, v = inputs(oracle, (B, Hq, Sq, D), (B, Hkv, Sk, D), dtype, 35000 + Sq + D)
+    assert form in plan(lm, q, k, dtype, causal, False)
+    lens = np.array([max(1, Sk - 31 * i) for i in range(B)], np.int32)
+    for kv_len in (None, lens):
+        got = run(lm, hip, q, k, v, dtype, causal, kv_len=None if kv_len is None else list(kv_len))
+        assert rel_err(got, oracle.flash_attn(q, k, v, causal=causal, kv_len=kv_len, nthreads=NT)) <= TOL[dtype]
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
 def test_launches_with_very_many_heads(lm, hip, oracle, dtype):
     """More heads than a 32-bit reciprocal divides exactly: every one of them is computed."""
