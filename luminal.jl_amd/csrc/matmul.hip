@@ -20,6 +20,8 @@
 // of the wave, which read neighbouring chunks.
 #include <limits.h>
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "dtypes.hpp"
 
@@ -38,6 +40,46 @@ __device__ inline float load_as_f32(const void *p, int64_t i, int dtype) {
     default: return reinterpret_cast<const float *>(p)[i];
   }
 }
+// Column j of c is column `b_column` of b: the same, or, where c is split into heads, column h + heads * d for j = h D + d
+// (the reference's column-major reshape of hidden into (heads, D) makes the head index the fast one).
+__device__ inline int b_column(const MatmulProblem &p, int D, int j) { return p.heads ? j / D + p.heads * (j % D) : j; }
+
+// Store R registers a lane of a wave's 32 x 32 block, R / 4 rows of it in fours: lane (n, h) holds column j, register i row
+// mw + 8 (i / 4) + 4 h + i % 4.
+template <int R, typename Acc>
+__device__ inline void store_block(const MatmulProblem &p, const Acc &acc, int mw, int j, int h, int batch) {
+  if (j >= p.N || mw >= p.M) return;
+  const int D = p.heads ? p.N / p.heads : 1;
+  const float bias = p.bias ? load_as_f32(p.bias, b_column(p, D, j), p.bias_dtype) : 0.f;
+  // Offsets by addition: a division per row and lane made the epilogue a tenth of the launch at K = 2048.
+  int64_t base, wrap = 0;          // offset of row mw; what a step to the next sequence adds beyond a row step
+  int row_step, s0 = 0, seq = INT_MAX;
+  if (p.heads) {  // c[b, head, s, d], rows m = b S + s
+    const int head = j / D, b = mw / p.seq;
+    seq = p.seq;
+    s0 = mw - b * seq;
+    row_step = D;
+    base = (((int64_t)b * p.heads + head) * seq + s0) * D + (j - head * D);
+    wrap = (int64_t)(p.heads - 1) * seq * D;
+  } else {
+    row_step = p.N;
+    base = ((int64_t)batch * p.M + mw) * p.N + j;
+  }
+  auto store_rows = [&](auto store) {
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      const int r = 8 * (i >> 2) + 4 * h + (i & 3);
+      if (mw + r >= p.M) break;  // rows ascend with i
+      int64_t off = base + (int64_t)r * row_step;
+      for (int s = s0 + r; s >= seq; s -= seq) off += wrap;
+      store(off, acc[i] + bias);
+    }
+  };
+  if (p.c_dtype == LMH_F32) store_rows([&](int64_t off, float x) { reinterpret_cast<float *>(p.c)[off] = x; });
+  else if (p.c_dtype == LMH_F16) store_rows([&](int64_t off, float x) { reinterpret_cast<_Float16 *>(p.c)[off] = (_Float16)x; });
+  else store_rows([&](int64_t off, float x) { reinterpret_cast<uint16_t *>(p.c)[off] = f32_to_bf16_bits(x); });
+}
+
 // VEC: every operand is fp32, contiguous along the contraction and 16-byte aligned, K a multiple of 4.
 template <int WM, int WN, int WK, bool VEC>
 __global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(MatmulArgs args) {
@@ -71,10 +113,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(Matmul
   const int n = lane & 31, h = lane >> 5;
   const int wk = wave / (WM * WN), wm = (wave % (WM * WN)) / WN, wn = wave % WN;
 
-  // Column j of c is column `col` of b: the same, or, where c is split into heads, column h + heads * d for j = h D + d
-  // (the reference's column-major reshape of hidden into (heads, D) makes the head index the fast one).
   const int D = p.heads ? p.N / p.heads : 1;
-  auto b_col = [&](int j) { return p.heads ? j / D + p.heads * (j % D) : j; };
+  auto b_col = [&](int j) { return b_column(p, D, j); };
 
   floatx16_t acc;
 #pragma unroll
@@ -232,52 +272,278 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(Matmul
     }
   }
 
-  // ---- epilogue: lane n holds column n0 + 32 wn + n, register i row 8 (i / 4) + 4 h + i % 4 of the wave's block ----
-  const int j = n0 + 32 * wn + n;
-  if (j >= p.N) return;
-  const float bias = p.bias ? load_as_f32(p.bias, b_col(j), p.bias_dtype) : 0.f;
-  // Offsets by addition: a division per row and lane made the epilogue a tenth of the launch at K = 2048.
-  const int mw = m0 + 32 * wm;
-  int64_t base, wrap = 0;          // offset of row mw; what a step to the next sequence adds beyond a row step
-  int row_step, s0 = 0, seq = INT_MAX;
-  if (p.heads) {  // c[b, head, s, d], rows m = b S + s
-    const int head = j / D, b = mw / p.seq;
-    seq = p.seq;
-    s0 = mw - b * seq;
-    row_step = D;
-    base = (((int64_t)b * p.heads + head) * seq + s0) * D + (j - head * D);
-    wrap = (int64_t)(p.heads - 1) * seq * D;
-  } else {
-    row_step = p.N;
-    base = ((int64_t)batch * p.M + mw) * p.N + j;
-  }
-  auto store_rows = [&](auto store) {
+  store_block<16>(p, acc, m0 + 32 * wm, n0 + 32 * wn + n, h, batch);
+}
+
+// The same products for fp32 operands that are contiguous along the contraction, on the bf16 matrix pipe (16 times the rate).
+// x = x1 + x2 + x3 in bf16, each the rest rounded to nearest: 8 bits and a sign a piece hold all 24 bits of x. Of the nine
+// products of pieces the six with x_i y_j, i + j <= 4, are summed; the other three are below 2^-25 of x y. Error against 64 bits
+// (2-norm): 3.6e-7 where the fp32 product has 5.7e-7 (K = 2048; fewer roundings), 9.2e-8 and 1.07e-7 (K = 64).
+// Where the pieces do not hold the values a wave takes its share again with the fp32 product: an infinity, a NaN or a value that
+// rounds up to an infinity makes every sum it enters not finite, and rows below 2^-95 are told by their bits (pieces below 2^-126
+// lose some).
+//
+// Bound: the vector ALUs beside the matrix pipe. Splitting takes 5.5 instructions an element, 5.5 a MFMA at 64 x 128 and 7.3 at
+// 64 x 64, where the chip holds 1590 TFLOP/s of bare MFMAs and 1280 with six vector instructions each. So:
+//   * a wave multiplies blocks as large as its registers hold (MB x NB of 32 x 32: 64 rows with 64 or 128 columns), and the four
+//     waves of a workgroup each take all of its tile for every fourth 16 elements of the contraction; the shares are folded
+//     through LDS at the end;
+//   * a wave fetches its own operands and shares nothing until then, so there is no barrier in the loop: buffer loads write fp32
+//     rows of 64 bytes straight into the wave's two stages in LDS, the wave reads them in the MFMA's layout (chunk j of row r
+//     lies at j ^ f(r): all banks) and splits them in registers one step ahead of the MFMAs, five to ten instructions between
+//     every two of those. (Planes of pieces in LDS, split once per workgroup with a barrier per 64 elements, take 50 us in place
+//     of 46.5 on 700 x 2560 x 2048: the waves of a SIMD then do the same thing at the same time.)
+__device__ inline void split_bf16x2(float a, float b, uint32_t *p1, uint32_t *p2, uint32_t *p3) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  auto round2 = [](float x, float y) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x, y}, bf16x2)); };
+  const uint32_t h1 = round2(a, b);
+  const float ra = a - __uint_as_float(h1 << 16), rb = b - __uint_as_float(h1 & 0xffff0000u);
+  const uint32_t h2 = round2(ra, rb);
+  *p1 = h1;
+  *p2 = h2;
+  *p3 = round2(ra - __uint_as_float(h2 << 16), rb - __uint_as_float(h2 & 0xffff0000u));
+}
+__device__ inline int swizzle16(int row) { return ((row >> 1 ^ row >> 3) & 1) | (row >> 1 & 2); }
+
+template <int MB, int NB>
+__global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args) {
+  constexpr int BM = 32 * MB, BN = 32 * NB, WK = 4;
+  constexpr int L = 2 * (MB + NB);              // loads of 1 KB (16 rows) per stage: a, then b
+  constexpr int kStage = 16 * 16 * L;           // floats
+  constexpr int kShare = MB * NB * 1024;        // floats of a wave's sums
+  __shared__ __attribute__((aligned(16))) float lds[WK * (2 * kStage > kShare ? 2 * kStage : kShare)];
+
+  const int per_xcd = (args.n_tiles + 7) / 8;
+  int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || t >= args.n_tiles) return;
+  int g = 0;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const int r = 8 * (i >> 2) + 4 * h + (i & 3);
-      if (mw + r >= p.M) break;  // rows ascend with i
-      int64_t off = base + (int64_t)r * row_step;
-      for (int s = s0 + r; s >= seq; s -= seq) off += wrap;
-      store(off, acc[i] + bias);
+  for (int i = 1; i < kMatmulGroup; i++)
+    if (t >= args.first_tile[i]) g = i;
+  const MatmulProblem p = args.p[g];
+  t -= args.first_tile[g];
+  const int m_tiles = (p.M + BM - 1) / BM;
+  const int tm = t % m_tiles;
+  t /= m_tiles;
+  const int n_tiles = (p.N + BN - 1) / BN;
+  const int tn = t % n_tiles, batch = t / n_tiles;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int wk = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+  const int lane = threadIdx.x & 63;
+  const int n = lane & 31, h = lane >> 5;
+  const int D = p.heads ? p.N / p.heads : 1;
+  const int steps = ((p.K + 15) / 16 - wk + WK - 1) / WK;  // of this wave (may be none)
+
+  typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) void lds_void_t;
+  auto make_desc = [](const float *base, int64_t elements) {
+    const uint64_t q = (uint64_t)base;
+    i32x4_t d;
+    d[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)q);
+    d[1] = __builtin_amdgcn_readfirstlane((int)((q >> 32) & 0xffff));  // stride 0: raw buffer
+    d[2] = __builtin_amdgcn_readfirstlane((int)(elements * 4));
+    d[3] = 0x00020000;
+    return d;
+  };
+  const float *a_base = reinterpret_cast<const float *>(p.a) + batch * p.as[0] + m0 * p.as[1];
+  const float *b_base = reinterpret_cast<const float *>(p.b) + batch * p.bs[0];
+  const i32x4_t a_desc = make_desc(a_base, (min(p.M - m0, BM) - 1) * p.as[1] + p.K);
+  const i32x4_t b_desc = make_desc(b_base, (int64_t)(p.N - 1) * p.bs[2] + p.K);
+  int voff[L], k_of[2];  // byte offset of the lane's chunk of each load at k = 0; its first k, by the parity of the load
+#pragma unroll
+  for (int l = 0; l < L; l++) {
+    const int row = 16 * l + (lane >> 2), chunk = (lane & 3) ^ swizzle16(row), col = n0 + row - BM;
+    if (l < 2) k_of[l] = 4 * chunk;
+    if (l < 2 * MB) voff[l] = m0 + row < p.M ? (int)((row * p.as[1] + 4 * chunk) * 4) : kOutOfRange;
+    else voff[l] = col < p.N ? (int)((b_column(p, D, col) * p.bs[2] + 4 * chunk) * 4) : kOutOfRange;
+  }
+  const uint32_t ring = (uint32_t)(uintptr_t)(lds_void_t *)&lds[wk * 2 * kStage];
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is a reserved register; it is only written here
+  auto load_block = [](i32x4_t desc, uint32_t lds_addr, int off, int soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(lds_addr), "v"(off), "s"(desc), "s"(soff) : "memory", "m0");
+  };
+#pragma clang diagnostic pop
+  // Past the wave's last step every lane is out of range and zeros arrive; the scalar offset stays inside the operand (one beyond
+  // its end would defeat the range check).
+  auto load_stage = [&](int i) {
+    const int k0 = 16 * (wk + WK * i), soff = min(k0, p.K - 4) * 4;
+    const bool tail = k0 + 16 > p.K;
+#pragma unroll
+    for (int l = 0; l < L; l++)
+      load_block(l < 2 * MB ? a_desc : b_desc, ring + (i & 1) * (kStage * 4) + l * 1024, tail && k0 + k_of[l & 1] >= p.K ? kOutOfRange : voff[l], soff);
+  };
+
+  // 32 rows of a stage in the MFMA's layout: lane (n, h) takes elements 8 h .. 8 h + 7 of row n. Blocks: MB of a, then NB of b.
+  const int frag0 = n * 16 + 4 * ((2 * h) ^ swizzle16(n)), frag1 = n * 16 + 4 * ((2 * h + 1) ^ swizzle16(n));
+  const float *own = &lds[wk * 2 * kStage];
+  struct Raw { floatx4_t lo, hi; };
+  struct Frag { bf16x8_t p[3]; };
+  uint32_t bits[MB + NB];  // every first piece of the lane's rows, or-ed
+#pragma unroll
+  for (int i = 0; i < MB + NB; i++) bits[i] = 0;
+  auto split = [&](const Raw &r, int block) {
+    uint32_t w[3][4];
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      split_bf16x2(e < 2 ? r.lo[2 * e] : r.hi[2 * e - 4], e < 2 ? r.lo[2 * e + 1] : r.hi[2 * e - 3], &w[0][e], &w[1][e], &w[2][e]);
+    bits[block] |= w[0][0] | w[0][1];
+    bits[block] |= w[0][2] | w[0][3];
+    Frag f;
+#pragma unroll
+    for (int i = 0; i < 3; i++) f.p[i] = __builtin_bit_cast(bf16x8_t, make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]));
+    return f;
+  };
+  auto read_stage = [&](int i, Raw (&raw)[MB + NB]) {
+#pragma unroll
+    for (int b = 0; b < MB + NB; b++) {
+      const float *q = own + (i & 1) * kStage + b * 512;
+      raw[b].lo = *reinterpret_cast<const floatx4_t *>(q + frag0);
+      raw[b].hi = *reinterpret_cast<const floatx4_t *>(q + frag1);
     }
   };
-  if (p.c_dtype == LMH_F32) store_rows([&](int64_t off, float x) { reinterpret_cast<float *>(p.c)[off] = x; });
-  else if (p.c_dtype == LMH_F16) store_rows([&](int64_t off, float x) { reinterpret_cast<_Float16 *>(p.c)[off] = (_Float16)x; });
-  else store_rows([&](int64_t off, float x) { reinterpret_cast<uint16_t *>(p.c)[off] = f32_to_bf16_bits(x); });
+
+  floatx16_t acc[MB][NB];
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
+  };
+  clear();
+
+  // Step i multiplies stage i while stage i + 1 is split and stages i + 2 and i + 3 are on their way.
+  Frag even[MB + NB], odd[MB + NB];
+  Raw raw[MB + NB];
+  load_stage(0);
+  load_stage(1);
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(L) : "memory");
+  read_stage(0, raw);
+#pragma unroll
+  for (int b = 0; b < MB + NB; b++) even[b] = split(raw[b], b);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  load_stage(2);
+  constexpr int kA[6] = {0, 0, 1, 1, 0, 2}, kB[6] = {0, 1, 0, 1, 2, 0};
+  auto step = [&](int i, const Frag (&cur)[MB + NB], Frag (&nxt)[MB + NB]) {
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(L) : "memory");  // stage i + 1 has landed
+    read_stage(i + 1, raw);
+#pragma unroll
+    for (int r = 0; r < MB; r++)
+#pragma unroll
+      for (int j = 0; j < NB; j++) acc[r][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur[r].p[0], cur[MB + j].p[0], acc[r][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every read of that stage has returned
+    load_stage(i + 3);
+#pragma unroll
+    for (int b = 0; b < MB + NB; b++) nxt[b] = split(raw[b], b);  // (past the last step: zeros)
+#pragma unroll
+    for (int q = 1; q < 6; q++)
+#pragma unroll
+      for (int r = 0; r < MB; r++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) acc[r][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur[r].p[kA[q]], cur[MB + j].p[kB[q]], acc[r][j], 0, 0, 0);
+    constexpr int kValu = (46 * (MB + NB) + 5 * MB * NB) / (5 * MB * NB);
+#pragma unroll
+    for (int q = 0; q < 5 * MB * NB; q++) {
+      __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    }
+  };
+  int i = 0;
+  for (; i + 1 < steps; i += 2) {  // (two steps a turn: no copies of the fragments)
+    step(i, even, odd);
+    step(i + 1, odd, even);
+  }
+  if (i < steps) step(i, even, odd);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing arrives in the ring any more
+  bool exact = true;
+#pragma unroll
+  for (int i = 0; i < MB + NB; i++) exact = exact && ((bits[i] & 0x70007000u) != 0 || (bits[i] & 0x7fff7fffu) == 0);
+  bool again = __builtin_amdgcn_ballot_w64(!exact) != 0;
+
+  // ---- fold the shares: each wave takes MB NB / WK blocks (or a part of one), and looks whether their sums are finite ----
+  constexpr int kRegs = 16 * MB * NB / WK;  // registers a lane of a wave folds
+  static_assert(kRegs % 4 == 0 && (kRegs < 16 ? 16 % kRegs : kRegs % 16) == 0, "quarters of a block, or blocks");
+  float sum[kRegs];
+  for (int pass = 0;; pass++) {
+    if (again) {
+      // this wave's share again with the fp32 product, its operands straight from memory
+      clear();
+      const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a_base), 0, a_desc[2], 0x00020000);
+      const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(b_base), 0, b_desc[2], 0x00020000);
+      int off[MB + NB];
+#pragma unroll
+      for (int i = 0; i < MB + NB; i++) {
+        const int row = 32 * i + n, col = n0 + row - BM;
+        if (i < MB) off[i] = m0 + row < p.M ? (int)(row * p.as[1] * 4) : -1;
+        else off[i] = col < p.N ? (int)(b_column(p, D, col) * p.bs[2] * 4) : -1;
+      }
+      for (int i = 0; i < 2 * steps; i++) {
+        const int k = 16 * (wk + WK * (i >> 1)) + 8 * (i & 1) + 4 * h;
+        floatx4_t x[MB + NB];
+#pragma unroll
+        for (int r = 0; r < MB + NB; r++)
+          x[r] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(r < MB ? a_rsrc : b_rsrc, k < p.K && off[r] >= 0 ? off[r] + 4 * k : kOutOfRange, 0, 0));
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int r = 0; r < MB; r++)
+#pragma unroll
+            for (int j = 0; j < NB; j++) acc[r][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[r][e], x[MB + j][e], acc[r][j], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4 * MB * NB; q++) {
+      const floatx16_t &x = acc[q / 4 / NB][q / 4 % NB];
+      *reinterpret_cast<floatx4_t *>(&lds[wk * kShare + q * 256 + 4 * lane]) = (floatx4_t){x[4 * (q & 3)], x[4 * (q & 3) + 1], x[4 * (q & 3) + 2], x[4 * (q & 3) + 3]};
+    }
+    __syncthreads();
+    float finite = 0.f;
+#pragma unroll
+    for (int q = 0; q < kRegs / 4; q++) {
+      const float *s = &lds[(wk * (kRegs / 4) + q) * 256 + 4 * lane];
+      floatx4_t x = *reinterpret_cast<const floatx4_t *>(s);
+#pragma unroll
+      for (int w = 1; w < WK; w++) x += *reinterpret_cast<const floatx4_t *>(s + w * kShare);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        sum[4 * q + e] = x[e];
+        finite = fmaf(x[e], 0.f, finite);
+      }
+    }
+    if (pass == 1 || !__syncthreads_or(finite != 0.f || finite != finite)) break;
+    again = true;
+  }
+  constexpr int kPart = kRegs < 16 ? kRegs : 16;
+#pragma unroll
+  for (int r = 0; r < kRegs; r += kPart) {
+    const int block = (wk * kRegs + r) / 16;
+    store_block<kPart>(p, sum + r, m0 + 32 * (block / NB) + wk * kRegs % 16 * 2, n0 + 32 * (block % NB) + n, h, batch);
+  }
+}
+
+// The tiles of the products of a launch, numbered one product after the other; negative where there are too many.
+int64_t number_tiles(MatmulArgs &args, int n, int bm, int bn) {
+  int64_t tiles = 0;
+  for (int i = 0; i < kMatmulGroup; i++) {
+    args.first_tile[i] = (int)tiles;
+    if (i < n) tiles += (int64_t)args.p[i].batch * ((args.p[i].M + bm - 1) / bm) * ((args.p[i].N + bn - 1) / bn);
+    if (tiles >= (int64_t(1) << 31) - 8) return -1;
+  }
+  args.n_tiles = (int)tiles;
+  return tiles;
 }
 
 template <int WM, int WN, int WK>
 int launch_form(MatmulArgs &args, int n, hipStream_t stream) {
-  int64_t tiles = 0;
-  for (int i = 0; i < kMatmulGroup; i++) {
-    args.first_tile[i] = (int)tiles;
-    if (i < n) {
-      const MatmulProblem &p = args.p[i];
-      tiles += (int64_t)p.batch * ((p.M + 32 * WM - 1) / (32 * WM)) * ((p.N + 32 * WN - 1) / (32 * WN));
-    }
-    if (tiles >= (int64_t(1) << 31) - 8) return fail(LMH_E_UNSUPPORTED, "matmul: too many tiles");
-  }
-  args.n_tiles = (int)tiles;
+  const int64_t tiles = number_tiles(args, n, 32 * WM, 32 * WN);
+  if (tiles < 0) return fail(LMH_E_UNSUPPORTED, "matmul: too many tiles");
   bool vec = true;
   for (int i = 0; i < n; i++) vec = vec && args.p[i].a_vec && args.p[i].b_vec;
   const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(64 * WM * WN * WK);
@@ -287,10 +553,21 @@ int launch_form(MatmulArgs &args, int n, hipStream_t stream) {
   return LMH_OK;
 }
 
+template <int MB, int NB>
+int launch_split_form(MatmulArgs &args, int n, hipStream_t stream) {
+  const int64_t tiles = number_tiles(args, n, 32 * MB, 32 * NB);
+  if (tiles < 0) return fail(LMH_E_UNSUPPORTED, "matmul: too many tiles");
+  hipLaunchKernelGGL((matmul_split_kernel<MB, NB>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, stream, args);
+  LMH_HIP_TRY(hipGetLastError());
+  return LMH_OK;
+}
+
 }  // namespace
 
 int launch_matmul(MatmulArgs &args, int n, hipStream_t stream) {
-  // Rounds of the CUs times the 32 x 32 blocks of a workgroup, with a weight for what the smaller workgroups pay in loads and
+  // Both kernels by what their forms cost, in us: a part per launch, a part per round of the CUs, and one per round and
+  // contraction element.
+  // fp32 product: rounds times the 32 x 32 blocks of a workgroup, with a weight for what the smaller workgroups pay in loads and
   // fixed costs per block. Measured, us for (64 x 64, eight waves) / (32 x 64) / (32 x 32): 700 x 2560 x 2048 82 / 90 / 99,
   // 700 x 2048 x 2048 73 / 62 / 73, 606 x 1536 x 1536 33 / 35 / 39, 1446 x 768 x 384 18.5 / 16.1 / 19.5,
   // 690 x 384 x 384 10.9 / 8.5 / 8.5, 164 x 1280 x 1280 26 / 18 / 11.
@@ -302,6 +579,27 @@ int launch_matmul(MatmulArgs &args, int n, hipStream_t stream) {
   };
   const int64_t r64 = rounds(64, 64);
   const double c64 = 4.0 * r64, c32x64 = 2.2 * rounds(32, 64), c32 = 1.5 * rounds(32, 32);
+  // Split product, us fp32 product -> 64 x 128 / 64 x 64 / 32 x 64: 700 x 2560 x 2048 75 -> 46.5 / 49.6 / 63.4, 700 x 2048 x 2048
+  // 57.8 -> 42.7 / 46.0 / 50.1, 4096^3 1039 -> 754 / 848 / 1073, 1792 x 1280 x 1280 69 -> 60 / 50 / 56, 590 x 1152 x 576 14.0 ->
+  // 16.2 / 10.9 / 11.8, 2048 x 768 x 256 12.7 -> 12.5 / 11.8 / 11.0, 16 x 12288 x 4096 48 -> 68 / 41 / 33. A launch of few tiles
+  // stays with the fp32 product, whose waves share the contraction of smaller blocks (100 x 768 x 768 8.1 -> 18.6 / 12.3 / 9.6).
+  bool vec = true;
+  int64_t K = 0;
+  for (int i = 0; i < n; i++) {
+    vec = vec && args.p[i].a_vec && args.p[i].b_vec;
+    K = std::max<int64_t>(K, args.p[i].K);
+  }
+  if (vec) {
+    const double fp32 = 0.95 * (3.3 + 0.0045 * K * std::min(c64, std::min(c32x64, c32)));
+    const double s64x128 = 2.0 + rounds(64, 128) * (6.0 + 0.0205 * K), s64 = 2.5 + r64 * (3.5 + 0.0105 * K);
+    const double s32x64 = 3.0 + rounds(32, 64) * (1.3 + 0.0067 * K);
+    const double split = std::min(s64x128, std::min(s64, s32x64));
+    if (split < fp32) {
+      if (split == s64) return launch_split_form<2, 2>(args, n, stream);
+      if (split == s64x128) return launch_split_form<2, 4>(args, n, stream);
+      return launch_split_form<1, 2>(args, n, stream);
+    }
+  }
   if (c64 <= c32x64 && c64 <= c32) {
     // with several rounds the other workgroups on a CU cover what eight waves on one block cover in a single round
     // (4096^3: 1062 against 1086 us = 129 TFLOP/s, 82 % of the fp32 matrix peak)

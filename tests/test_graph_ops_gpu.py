@@ -34,6 +34,47 @@ def test_projection_matches_float64(lm, hip, oracle, B, S, K, N, heads, dtype, b
     assert rel_err(out.to_host(), want) <= {"f32": 2e-6, "f16": 5e-4, "bf16": 4e-3}[dtype]
 
 
+# Large products of fp32 operands run on bf16 pieces: every tile (64 x 128, 64 x 64, 32 x 64) with remainders in every direction,
+# heads whose rows cross sequences, 16-bit results. Against float64 with the bound of the fp32 product (its error is smaller).
+@pytest.mark.parametrize("B,S,K,N,heads,dtype,bias", [
+    (1, 701, 2052, 2500, 0, "f32", True), (2, 350, 2048, 2560, 20, "bf16", False), (1, 590, 580, 1150, 0, "f32", True),
+    (3, 197, 576, 1152, 9, "f16", True), (1, 33, 772, 5000, 0, "f32", False), (1, 31, 1540, 9000, 10, "f32", True),
+])
+def test_products_on_pieces_match_float64(lm, hip, oracle, B, S, K, N, heads, dtype, bias):
+    test_projection_matches_float64(lm, hip, oracle, B, S, K, N, heads, dtype, bias)
+
+
+@pytest.mark.parametrize("M,K,N", [(590, 580, 1150), (33, 772, 5000), (701, 2052, 2500)])
+def test_values_that_pieces_do_not_hold(lm, hip, oracle, M, K, N):
+    """Infinities, NaN, values next to the largest and rows far below the smallest normal bf16 piece: what fp32 gives."""
+    x, w = oracle.gen_normal((M, K), 36000 + M), oracle.gen_normal((N, K), 36100 + N)
+    x[0, 3], x[1, 5], x[2, 7], x[3, 9], w[4, 11] = np.inf, np.nan, -np.inf, 3.4e38, np.inf
+    w[:, 9] *= 0.01
+    x[:, 11] = np.where(np.arange(M) % 7 == 0, 0, x[:, 11])  # infinity times zero
+    x[10:13] *= np.float32(2.0 ** -122)
+    w[20:23] *= np.float32(2.0 ** -100)
+    x[14] *= np.float32(2.0 ** 110)
+    out = lm.HipArray((1, M, N), "f32", hip)
+    p = (lm.binding.MatmulParams * 1)()
+    dx, dw = lm.to_device(x[None], hip), lm.to_device(w, hip)
+    assert _low(lm).fill_matmul(p[0], out, dx, dw, transposed=True)
+    lm.binding.matmul(p, 1)
+    got = out.to_host()[0]
+    with np.errstate(all="ignore"):
+        want = x.astype(np.float64) @ w.astype(np.float64).T
+        top = np.abs(np.where(np.isfinite(x), x, 0)).astype(np.float64) @ np.abs(np.where(np.isfinite(w), w, 0)).astype(np.float64).T
+    finite = np.abs(want) < 3e38
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    # fp32 sums of K products, each within K 2^-24 of the sum of their magnitudes (and within the smallest subnormal)
+    assert (np.abs(got[finite] - want[finite]) <= K * 2.0 ** -24 * top[finite] + K * 2.0 ** -149).all()
+    # rows of one magnitude each, as exact as any other row
+    for rows in (slice(10, 13), slice(14, 15)):
+        ok = np.r_[0:4, 5:20, 23:N]
+        g, v = got[rows][:, ok].astype(np.float64), want[rows][:, ok]
+        assert np.linalg.norm(g - v) <= 2e-6 * np.linalg.norm(v)
+
+
 @pytest.mark.parametrize("a_shape,b_shape,dtypes", [
     ((3, 40, 72), (3, 72, 50), ("f32", "f32")), ((40, 72), (5, 72, 64), ("f32", "f16")), ((2, 3, 33, 20), (20, 100), ("bf16", "f32")),
 ])
