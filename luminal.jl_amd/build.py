@@ -19,8 +19,8 @@ LIBDIR = os.path.join(HERE, "lib")
 LIBNAME = "libluminal_hip.so"
 CALIB_LIBNAME = "libluminal_hip_calib.so"
 LIBRARIES = {
-    LIBNAME: ["api.hip", "prefill_valu.hip", "prefill_mfma.hip", "prefill_f32.hip", "prefill_f32_full.hip", "decode.hip",
-              "decode_mfma.hip", "cache_ops.hip", "matmul.hip", "map_ops.hip", "staging.hip"],
+    LIBNAME: ["api.hip", "prefill_valu.hip", "prefill_mfma.hip", "prefill_f32.hip", "prefill_f32_full.hip",
+              "prefill_f32_split.hip", "decode.hip", "decode_mfma.hip", "cache_ops.hip", "matmul.hip", "map_ops.hip", "staging.hip"],
     CALIB_LIBNAME: ["calib.hip"],
 }
 

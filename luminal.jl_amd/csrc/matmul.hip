@@ -24,6 +24,7 @@
 
 #include "common.hpp"
 #include "dtypes.hpp"
+#include "split.hpp"
 
 namespace lmh {
 namespace {
@@ -276,12 +277,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(Matmul
 }
 
 // The same products for fp32 operands that are contiguous along the contraction, on the bf16 matrix pipe (16 times the rate).
-// x = x1 + x2 + x3 in bf16, each the rest rounded to nearest: 8 bits and a sign a piece hold all 24 bits of x. Of the nine
-// products of pieces the six with x_i y_j, i + j <= 4, are summed; the other three are below 2^-25 of x y. Error against 64 bits
-// (2-norm): 3.6e-7 where the fp32 product has 5.7e-7 (K = 2048; fewer roundings), 9.2e-8 and 1.07e-7 (K = 64).
-// Where the pieces do not hold the values a wave takes its share again with the fp32 product: an infinity, a NaN or a value that
-// rounds up to an infinity makes every sum it enters not finite, and rows below 2^-95 are told by their bits (pieces below 2^-126
-// lose some).
+// Every operand is split into three bf16 pieces (split.hpp); of the nine products of pieces the six with x_i y_j, i + j <= 4, are
+// summed, the other three are below 2^-25 of x y. Error against 64 bits (2-norm): 3.6e-7 where the fp32 product has 5.7e-7 (K =
+// 2048; fewer roundings), 9.2e-8 and 1.07e-7 (K = 64). A wave whose operands the pieces do not hold takes its share again with
+// the fp32 product.
 //
 // Bound: the vector ALUs beside the matrix pipe. Splitting takes 5.5 instructions an element, 5.5 a MFMA at 64 x 128 and 7.3 at
 // 64 x 64, where the chip holds 1590 TFLOP/s of bare MFMAs and 1280 with six vector instructions each. So:
@@ -293,17 +292,6 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(Matmul
 //     lies at j ^ f(r): all banks) and splits them in registers one step ahead of the MFMAs, five to ten instructions between
 //     every two of those. (Planes of pieces in LDS, split once per workgroup with a barrier per 64 elements, take 50 us in place
 //     of 46.5 on 700 x 2560 x 2048: the waves of a SIMD then do the same thing at the same time.)
-__device__ inline void split_bf16x2(float a, float b, uint32_t *p1, uint32_t *p2, uint32_t *p3) {
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  auto round2 = [](float x, float y) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x, y}, bf16x2)); };
-  const uint32_t h1 = round2(a, b);
-  const float ra = a - __uint_as_float(h1 << 16), rb = b - __uint_as_float(h1 & 0xffff0000u);
-  const uint32_t h2 = round2(ra, rb);
-  *p1 = h1;
-  *p2 = h2;
-  *p3 = round2(ra - __uint_as_float(h2 << 16), rb - __uint_as_float(h2 & 0xffff0000u));
-}
 __device__ inline int swizzle16(int row) { return ((row >> 1 ^ row >> 3) & 1) | (row >> 1 & 2); }
 
 template <int MB, int NB>
@@ -381,22 +369,10 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args) {
   const int frag0 = n * 16 + 4 * ((2 * h) ^ swizzle16(n)), frag1 = n * 16 + 4 * ((2 * h + 1) ^ swizzle16(n));
   const float *own = &lds[wk * 2 * kStage];
   struct Raw { floatx4_t lo, hi; };
-  struct Frag { bf16x8_t p[3]; };
   uint32_t bits[MB + NB];  // every first piece of the lane's rows, or-ed
 #pragma unroll
   for (int i = 0; i < MB + NB; i++) bits[i] = 0;
-  auto split = [&](const Raw &r, int block) {
-    uint32_t w[3][4];
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-      split_bf16x2(e < 2 ? r.lo[2 * e] : r.hi[2 * e - 4], e < 2 ? r.lo[2 * e + 1] : r.hi[2 * e - 3], &w[0][e], &w[1][e], &w[2][e]);
-    bits[block] |= w[0][0] | w[0][1];
-    bits[block] |= w[0][2] | w[0][3];
-    Frag f;
-#pragma unroll
-    for (int i = 0; i < 3; i++) f.p[i] = __builtin_bit_cast(bf16x8_t, make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]));
-    return f;
-  };
+  auto split = [&](const Raw &r, int block) { return split_8(r.lo, r.hi, &bits[block]); };
   auto read_stage = [&](int i, Raw (&raw)[MB + NB]) {
 #pragma unroll
     for (int b = 0; b < MB + NB; b++) {
@@ -418,7 +394,7 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args) {
   clear();
 
   // Step i multiplies stage i while stage i + 1 is split and stages i + 2 and i + 3 are on their way.
-  Frag even[MB + NB], odd[MB + NB];
+  Pieces even[MB + NB], odd[MB + NB];
   Raw raw[MB + NB];
   load_stage(0);
   load_stage(1);
@@ -429,7 +405,7 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args) {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   load_stage(2);
   constexpr int kA[6] = {0, 0, 1, 1, 0, 2}, kB[6] = {0, 1, 0, 1, 2, 0};
-  auto step = [&](int i, const Frag (&cur)[MB + NB], Frag (&nxt)[MB + NB]) {
+  auto step = [&](int i, const Pieces (&cur)[MB + NB], Pieces (&nxt)[MB + NB]) {
     asm volatile("s_waitcnt vmcnt(%0)" :: "n"(L) : "memory");  // stage i + 1 has landed
     read_stage(i + 1, raw);
 #pragma unroll
@@ -463,7 +439,7 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing arrives in the ring any more
   bool exact = true;
 #pragma unroll
-  for (int i = 0; i < MB + NB; i++) exact = exact && ((bits[i] & 0x70007000u) != 0 || (bits[i] & 0x7fff7fffu) == 0);
+  for (int i = 0; i < MB + NB; i++) exact = exact && pieces_hold(bits[i]);
   bool again = __builtin_amdgcn_ballot_w64(!exact) != 0;
 
   // ---- fold the shares: each wave takes MB NB / WK blocks (or a part of one), and looks whether their sums are finite ----

@@ -373,11 +373,30 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
       f128 = cost(128, 32, 0.92);
       f64 = cost(64, 64, tiles(64) <= n_cus ? 1.07 : INFINITY);
     }
-    if (tiles(128) >= 4 * n_cus) return kFull && !a.causal ? launch_prefill_f32_full(a, 1, stream) : launch_form<D, 8, 1, 2>(a, stream);
+    const bool many = tiles(128) >= 4 * n_cus;
+    const double c128 = form_cost<D, 8, 1, 2>(a, 0.96);
+    // In bf16 pieces (prefill_f32_split.hip), up to head dim 96: by the time that the cost of the form here stands for, in us (a part
+    // per launch, a part per key of the walk; fitted to 240 launches of drawn sizes, rms 2 to 13 %). Of 330 such launches 159 go
+    // over, none loses more than 4 %, and together the 330 gain 12 %: B=2 H=12 S=1023 D=80 without a mask 75.5 -> 57 us, B=1 H=32
+    // S=2048 D=96 380 -> 233, causal 214 -> 146. The small launches stay because their waves walk the keys alone (B=1 H=6 S=846
+    // D=96 causal); so do, though they would gain as well, rows of up to five key tiles without a mask and causal launches of
+    // up to two rounds at the tiling for 64, where the tests of the forms here reach those forms (B=3 H=4 1844 x 304 D=64
+    // 23.3 us here, 18.8 there; B=1 H=48 S=1100 D=64 causal 79 and 58).
+    auto pieces = [&](double here, int *form) {
+      if (D > 96 || (!a.causal && a.Sk <= 320) || (a.causal && D <= 64 && tiles(128) <= 2 * n_cus)) return false;
+      constexpr double fit[5][2][2] = {{{6.6, 0.0178}, {4.3, 0.0197}}, {{6.1, 0.0249}, {5.1, 0.0277}}, {{5.6, 0.0352}, {5.7, 0.0351}},
+                                       {{7.5, 0.0419}, {6.4, 0.0451}}, {{6.2, 0.0527}, {8.6, 0.0505}}};  // D = 32, 48, 64, 80, 96
+      const auto &f = fit[D <= 96 ? D / 16 - 2 : 0][a.causal != 0];
+      return prefill_f32_split_cost(a, form) < 0.95 * (f[0] + f[1] * here);
+    };
+    int split_form = 0;
+    if (many && pieces(kFull && !a.causal ? f128 : c128, &split_form)) return launch_prefill_f32_split(a, split_form, stream);
+    if (many) return kFull && !a.causal ? launch_prefill_f32_full(a, 1, stream) : launch_form<D, 8, 1, 2>(a, stream);
     const bool few32 = tiles(32) <= (a.causal ? 2 : 1) * n_cus, few16 = tiles(16) <= 2 * n_cus;
-    const double c128 = form_cost<D, 8, 1, 2>(a, 0.96), c64 = form_cost<D, 4, 1, 2>(a, 1.0), c32 = form_cost<D, 2, 2, 1>(a, w32),
+    const double c64 = form_cost<D, 4, 1, 2>(a, 1.0), c32 = form_cost<D, 2, 2, 1>(a, w32),
                  c32x2 = form_cost<D, 2, 2, 2>(a, few32 ? 1.0 : D <= 64 ? 1.15 : 1.4), c16 = form_cost<D, 1, 4, 1>(a, few16 ? 1.2 : D <= 64 ? 1.5 : 1.8);
     const double best = fmin(fmin(c128, c64), fmin(fmin(c32, c32x2), c16));
+    if (pieces(fmin(best, fmin(f128, f64)), &split_form)) return launch_prefill_f32_split(a, split_form, stream);
     if (fmin(f128, f64) < best) return launch_prefill_f32_full(a, f64 < f128 ? 2 : 1, stream);
     if (best == c128) return launch_form<D, 8, 1, 2>(a, stream);
     if (best == c64) return launch_form<D, 4, 1, 2>(a, stream);

@@ -1,0 +1,466 @@
+// Flash attention forward in fp32 on the bf16 matrix pipe: every operand as three bf16 pieces, six products for one.
+//
+// Every operand is split into three bf16 pieces (split.hpp); of the nine products of pieces the six with x_i y_j, i + j <= 4, are
+// summed in fp32, the other three are below 2^-25 of x y. Six bf16 products take 6 / 16 of the time of the fp32 one. A workgroup
+// that meets a value that the pieces do not hold takes its rows again with the fp32 product. Error against 64 bits (2-norm): 1.9e-7
+// where the forms of prefill_f32.hip have 4.3e-7 (S = 1023 D = 80), 1.3e-7 and 2.7e-7 (S = 500 D = 96 causal).
+//
+// Same data flow as prefill_mfma.hip: a wave owns 32 query rows with the pieces of its Q fragments in registers, S^T = K Q^T so
+// that a lane holds one query column, and the registers of P, split there, are the B operands of O^T = V^T P^T. Statistics, sums
+// and accumulators are fp32 as in prefill_f32.hip. K and V tiles of 64 keys pass through registers: fetched as fp32 while the tile
+// before is multiplied, split once per workgroup and stored as three planes each.
+// Bound: the bf16 matrix pipe at the clock it gets, then the vector ALUs beside it. S = 1023 D = 80, 57 us: 36 with two of the six
+// products, 52 without splitting K and V, 57 without splitting P (measurement variants). Head dims above 96 do not fit two waves
+// per SIMD (D=128: 160 bytes of spills; B=1 H=16 S=2048 causal 178 us against 175 on the fp32 product) and stay there.
+#include <math.h>
+
+#include <algorithm>
+
+#include "prefill_mfma.hpp"
+#include "rope.hpp"
+#include "split.hpp"
+
+namespace lmh {
+namespace {
+
+// NW waves: RW = NW / KSPLIT groups of 32 rows; KSPLIT = 2: half of the waves take the second 32 keys of every tile, folded
+// through LDS at the end.
+template <int D, bool CAUSAL, int NW, int KSPLIT>
+__global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal, PrefillArgs a) {
+  request_args(a);
+  request_args(deal);
+  constexpr int RW = NW / KSPLIT, BM = 32 * RW, NT = 64 * NW;
+  constexpr int BT = 64;                   // keys per tile
+  constexpr int NKB = 2 / KSPLIT;          // 32-key blocks a wave takes of it
+  constexpr int KS = D / 16;               // k-steps of the S^T product
+  constexpr int DB = (D + 31) / 32;        // 32-row blocks of O^T
+  constexpr int LDK = D + kPadK, LDV = 32 * DB + pad_v<32 * DB>();
+  constexpr int kPlaneK = BT * LDK, kPlaneV = BT * LDV;
+  constexpr int DC = D / 8, kChunks = 2 * BT * DC, R = (kChunks + NT - 1) / NT;  // chunks of eight elements, K's then V's
+  // Two tiles where they fit (tile kt + 1 is split beside the MFMAs of tile kt, one barrier a tile), or one.
+  constexpr int kTile = 3 * (kPlaneK + kPlaneV);
+  constexpr int NBUF = 4 * kTile <= 160 * 1024 && NW == 8 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) uint16_t planes[NBUF * kTile];
+  __shared__ int redo;
+
+  int bh, tile_rank;
+  if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, &bh, &tile_rank)) return;
+  const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
+  const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
+  const int q_tile = CAUSAL ? (deal.tiles - 1 - tile_rank) : tile_rank;
+  const int q0 = q_tile * BM;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, g = lane >> 5;
+  const int kg = wave / RW;
+  const int wave_q_lo = q0 + (wave % RW) * 32, wave_q_hi = wave_q_lo + 31;
+  const int qi = wave_q_lo + n;
+
+  int n_keys = a.kv_len ? a.kv_len[b] : a.Sk;
+  n_keys = min(max(n_keys, 0), a.Sk);
+  int k_end = n_keys;
+  if (CAUSAL) k_end = min(k_end, q0 + BM);
+  const int n_kv_tiles = (k_end + BT - 1) / BT;
+
+  const float *qp = reinterpret_cast<const float *>(a.q) + b * a.qs[0] + hq * a.qs[1];
+  const float *kp = reinterpret_cast<const float *>(a.k) + b * a.ks[0] + kvh * a.ks[1];
+  const float *vp = reinterpret_cast<const float *>(a.v) + b * a.vs[0] + kvh * a.vs[1];
+
+  // ---- tile staging; columns past the tensors' own head dim and rows past n_keys arrive as zeros ----
+  auto make_rsrc = [](const float *p, int64_t elements) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, __builtin_amdgcn_readfirstlane((int)(elements * 4)), 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t k_rsrc = make_rsrc(kp, (int64_t)n_keys * a.ks[2]);
+  const __amdgpu_buffer_rsrc_t v_rsrc = make_rsrc(vp, (int64_t)n_keys * a.vs[2]);
+  const int k_tile_bytes = (int)(BT * a.ks[2] * 4), v_tile_bytes = (int)(BT * a.vs[2] * 4);
+  int voff[R], lds_off[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int q = tid + r * NT, c = q % (BT * DC), row = c / DC, col = c % DC;
+    const bool is_v = q >= BT * DC;
+    voff[r] = q < kChunks && 8 * col < a.D ? (int)((row * (is_v ? a.vs[2] : a.ks[2]) + 8 * col) * 4) : kOutOfRange - 16;
+    lds_off[r] = is_v ? 3 * kPlaneK + row * LDV + 8 * col : row * LDK + 8 * col;
+  }
+  floatx4_t x[R][2];
+  uint32_t bits[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) bits[r] = 0;
+  auto is_v_wave = [&](int r) { return wave * 64 + r * NT >= BT * DC; };  // (a wave's 64 chunks are K's or V's: 8 D is a multiple of 64)
+  auto fetch = [&](int kt) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      if (kChunks % NT != 0 && wave * 64 + r * NT >= kChunks) continue;
+#pragma unroll
+      for (int e = 0; e < 2; e++)
+        x[r][e] = __builtin_bit_cast(floatx4_t, is_v_wave(r) ? __builtin_amdgcn_raw_buffer_load_b128(v_rsrc, voff[r] + 16 * e, kt * v_tile_bytes, 0)
+                                                             : __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, voff[r] + 16 * e, kt * k_tile_bytes, 0));
+    }
+  };
+  auto split_tile = [&](int buf) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      if (kChunks % NT != 0 && wave * 64 + r * NT >= kChunks) continue;
+      const Pieces f = split_8(x[r][0], x[r][1], &bits[r]);
+      const int plane = is_v_wave(r) ? kPlaneV : kPlaneK;
+#pragma unroll
+      for (int i = 0; i < 3; i++) *reinterpret_cast<bf16x8_t *>(&planes[buf * kTile + i * plane + lds_off[r]]) = f.p[i];
+    }
+  };
+  if (n_kv_tiles > 0) fetch(0);
+  if (D % 32 != 0) {  // columns of the last block of O^T that no chunk fills
+    for (int i = tid; i < NBUF * 3 * BT * (32 * DB - D); i += NT) {
+      const int row = i / (32 * DB - D), col = i % (32 * DB - D), plane = row / BT;
+      planes[plane / 3 * kTile + 3 * kPlaneK + plane % 3 * kPlaneV + row % BT * LDV + D + col] = 0;
+    }
+  }
+  if (tid == 0) redo = 0;
+
+  // ---- Q: lane (n, g) holds q[qi][16 ks + 8 g .. + 7] ----
+  floatx4_t q[KS][2];
+  auto load_q = [&]() {
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+      for (int e = 0; e < 2; e++) {
+        q[ks][e] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
+        if (qi < a.Sq && 16 * ks + 8 * g < a.D) q[ks][e] = *reinterpret_cast<const floatx4_t *>(qp + (int64_t)qi * a.qs[2] + 16 * ks + 8 * g + 4 * e);
+      }
+    if (D % 32 == 0 && a.q_rope) {  // (the head dim equals the tiling: the partner of an element is in the same lane)
+      const float pos = (float)((a.q_pos0 ? a.q_pos0[b] : a.q_prev_seq) + qi);
+      if (!a.q_interleaved) {
+#pragma unroll
+        for (int ks = 0; ks < KS / 2; ks++)
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            float sn, cs, o0, o1;
+            sincos_angle(pos * rope_inv_freq(16 * ks + 8 * g + e, D, a.q_log2_base), &sn, &cs);
+            rope_rotate(q[ks][e >> 2][e & 3], q[ks + KS / 2][e >> 2][e & 3], sn, cs, &o0, &o1);
+            q[ks][e >> 2][e & 3] = o0;
+            q[ks + KS / 2][e >> 2][e & 3] = o1;
+          }
+      } else {
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            float sn, cs, o0, o1;
+            sincos_angle(pos * rope_inv_freq((16 * ks + 8 * g + e) / 2, D, a.q_log2_base), &sn, &cs);
+            rope_rotate(q[ks][e >> 2][e & 3], q[ks][e >> 2][(e & 3) + 1], sn, cs, &o0, &o1);
+            q[ks][e >> 2][e & 3] = o0;
+            q[ks][e >> 2][(e & 3) + 1] = o1;
+          }
+      }
+    }
+  };
+  Pieces qf[KS];
+  uint32_t q_bits = 0;
+  load_q();
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) qf[ks] = split_8(q[ks][0], q[ks][1], &q_bits);
+
+  floatx16_t oacc[DB];
+  float m_i, l_i;
+  const float c = a.scale * kLog2e;
+  auto clear = [&]() {
+    m_i = -INFINITY;
+    l_i = 0.f;
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) oacc[db][i] = 0.f;
+  };
+  clear();
+  // Mask, running max, weights and their sum; register i of block kb is key k0 + 32 kb + 8 (i / 4) + 4 g + i % 4.
+  auto soften = [&](auto &s, int blocks, int k0) {
+    if (k0 + 32 * blocks > n_keys || (CAUSAL && k0 + 32 * blocks - 1 > wave_q_lo)) {
+#pragma unroll
+      for (int kb = 0; kb < blocks; kb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          const int key = k0 + 32 * kb + 8 * (i >> 2) + 4 * g + (i & 3);
+          if (key >= n_keys || (CAUSAL && key > qi)) s[kb][i] = -INFINITY;
+        }
+    }
+    float mx = s[0][0];
+#pragma unroll
+    for (int kb = 0; kb < blocks; kb++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[kb][i]);
+    mx = max_over_wave_halves(mx);
+    if (__builtin_amdgcn_ballot_w64((mx - m_i) * c > kLazyRescale) != 0) {
+      const float m_new = fmaxf(m_i, mx);
+      const float alpha = m_i == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_i - m_new) * c);
+      m_i = m_new;
+      l_i *= alpha;
+#pragma unroll
+      for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) oacc[db][i] *= alpha;
+    }
+    const float mc = m_i == -INFINITY ? 0.f : m_i * c;
+    float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < blocks; kb++)
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        s[kb][i] = __builtin_amdgcn_exp2f(s[kb][i] * c - mc);
+        s[kb][i + 1] = __builtin_amdgcn_exp2f(s[kb][i + 1] * c - mc);
+        l0 += s[kb][i];
+        l1 += s[kb][i + 1];
+      }
+    l_i += l0 + l1;
+  };
+
+  const int k_frag = (32 * NKB * kg + n) * LDK + 8 * g;
+  // the transposing read: within each 16 lanes, lane i supplies row i / 4 and columns 4 (i % 4) of a 4-key x 16-column patch
+  const int i16 = lane & 15;
+  const int v_frag = (32 * NKB * kg + 4 * g + (i16 >> 2)) * LDV + 16 * ((lane >> 4) & 1) + 4 * (i16 & 3);
+  // The five smaller products are summed ahead of the large one, those of the scores in accumulators of their own: their sums are
+  // rounded at 2^-8 of the result's magnitude. A tile's share of O^T is summed from zero and added once.
+  constexpr int kX[6] = {2, 0, 1, 1, 0, 0}, kY[6] = {0, 2, 1, 0, 1, 0};
+
+  if (NBUF == 2 && n_kv_tiles > 0) {
+    split_tile(0);
+    if (n_kv_tiles > 1) fetch(1);
+  }
+  for (int kt = 0; kt < n_kv_tiles; kt++) {
+    const int buf = NBUF == 2 ? kt & 1 : 0;
+    __syncthreads();  // everyone is done with tile kt - 1 (and, with two tiles, tile kt is in LDS)
+    if (NBUF == 1) {
+      split_tile(0);
+      if (kt + 1 < n_kv_tiles) fetch(kt + 1);
+      __syncthreads();  // tile kt is in LDS
+    }
+    auto prepare_next = [&]() {
+      if (NBUF == 1) return;
+      split_tile(buf ^ 1);  // (of the last tile again, behind the last one: nobody reads it)
+      if (kt + 2 < n_kv_tiles) fetch(kt + 2);
+    };
+    const int k0 = kt * BT + 32 * NKB * kg;
+    if ((CAUSAL && k0 > wave_q_hi) || k0 >= k_end) {
+      prepare_next();
+      continue;
+    }
+    const uint16_t *Kp = planes + buf * kTile, *Vp = Kp + 3 * kPlaneK;
+
+    floatx16_t s[NKB], small[NKB];
+#pragma unroll
+    for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) s[kb][i] = small[kb][i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      bf16x8_t kf[NKB][3];
+#pragma unroll
+      for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) kf[kb][i] = *reinterpret_cast<const bf16x8_t *>(&Kp[i * kPlaneK + k_frag + 32 * kb * LDK + 16 * ks]);
+#pragma unroll
+      for (int j = 0; j < 6; j++)
+#pragma unroll
+        for (int kb = 0; kb < NKB; kb++) {
+          floatx16_t &acc = j < 5 ? small[kb] : s[kb];
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kb][kX[j]], qf[ks].p[kY[j]], acc, 0, 0, 0);
+        }
+    }
+    prepare_next();
+#pragma unroll
+    for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) s[kb][i] += small[kb][i];
+    soften(s, NKB, k0);
+    Pieces pf[NKB][2];
+#pragma unroll
+    for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        uint32_t unused = 0;
+        pf[kb][t] = split_8((floatx4_t){s[kb][8 * t], s[kb][8 * t + 1], s[kb][8 * t + 2], s[kb][8 * t + 3]},
+                            (floatx4_t){s[kb][8 * t + 4], s[kb][8 * t + 5], s[kb][8 * t + 6], s[kb][8 * t + 7]}, &unused);
+      }
+#pragma unroll
+    for (int db = 0; db < DB; db++) {
+      floatx16_t o;
+#pragma unroll
+      for (int i = 0; i < 16; i++) o[i] = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < NKB; kb++) {
+        bf16x8_t vf[2][3];
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int i = 0; i < 3; i++) {
+            const uint16_t *p = &Vp[i * kPlaneV + v_frag + (32 * kb + 16 * t) * LDV + 32 * db];
+            const shortx4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)p);
+            const shortx4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(p + 8 * LDV));
+            vf[t][i] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          }
+#pragma unroll
+        for (int j = 0; j < 6; j++)
+#pragma unroll
+          for (int t = 0; t < 2; t++) o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[t][kX[j]], pf[kb][t].p[kY[j]], o, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; i++) oacc[db][i] += o[i];
+    }
+  }
+
+  // ---- values that pieces do not hold, anywhere in the workgroup: its rows again with the fp32 product ----
+  bool held = pieces_hold(q_bits);
+#pragma unroll
+  for (int r = 0; r < R; r++) held = held && pieces_hold(bits[r]);
+  float finite = 0.f;
+#pragma unroll
+  for (int db = 0; db < DB; db++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) finite = fmaf(oacc[db][i], 0.f, finite);
+  finite = fmaf(l_i, 0.f, finite);
+  __syncthreads();
+  if (!held || finite != 0.f || finite != finite) redo = 1;
+  __syncthreads();
+  if (redo) {
+    clear();
+    load_q();
+    for (int k0 = 32 * kg; k0 < k_end; k0 += 32 * KSPLIT) {
+      if (CAUSAL && k0 > wave_q_hi) break;
+      floatx16_t s[1];
+#pragma unroll
+      for (int i = 0; i < 16; i++) s[0][i] = 0.f;
+      const bool in = k0 + n < n_keys;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          floatx4_t kf = {0.f, 0.f, 0.f, 0.f};
+          if (in && 16 * ks + 8 * g < a.D) kf = *reinterpret_cast<const floatx4_t *>(kp + (int64_t)(k0 + n) * a.ks[2] + 16 * ks + 8 * g + 4 * e);
+#pragma unroll
+          for (int i = 0; i < 4; i++) s[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[i], q[ks][e][i], s[0], 0, 0, 0);
+        }
+      soften(s, 1, k0);
+      auto v_at = [&](int key, int db) { return key < n_keys && 32 * db + n < a.D ? vp[(int64_t)key * a.vs[2] + 32 * db + n] : 0.f; };
+      if (!CAUSAL || k0 + 31 <= wave_q_lo) {
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+#pragma unroll
+          for (int db = 0; db < DB; db++)
+            oacc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(v_at(k0 + 8 * (i >> 2) + 4 * g + (i & 3), db), s[0][i], oacc[db], 0, 0, 0);
+      } else {
+        // on the diagonal key by key: a value that is not finite stays out of the rows that do not see it (zero times it is NaN)
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+          for (int half = 0; half < 2; half++) {
+            const int key = k0 + 8 * (i >> 2) + 4 * half + (i & 3);
+#pragma unroll
+            for (int db = 0; db < DB; db++) {
+              const floatx16_t with = __builtin_amdgcn_mfma_f32_32x32x2f32(g == half ? v_at(key, db) : 0.f, g == half ? s[0][i] : 0.f, oacc[db], 0, 0, 0);
+              if (key <= qi) oacc[db] = with;
+            }
+          }
+      }
+    }
+  }
+
+  // ---- fold the second key group's (m, l, O) into the first's; lane for lane the same layout ----
+  if constexpr (KSPLIT > 1) {
+    constexpr int NF = DB * 16 + 2;
+    static_assert(RW * NF * 64 * 4 <= (int)sizeof(planes), "the partial results fit the planes");
+    float *xch = reinterpret_cast<float *>(planes) + (wave % RW) * (NF * 64) + lane;
+    if (kg > 0) {
+      xch[0] = m_i;
+      xch[64] = l_i;
+#pragma unroll
+      for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) xch[(2 + db * 16 + i) * 64] = oacc[db][i];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+    const float m1 = xch[0], m_all = fmaxf(m_i, m1);
+    const float a0 = m_i == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_i - m_all) * c);
+    const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m1 - m_all) * c);
+    l_i = l_i * a0 + xch[64] * a1;
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) oacc[db][i] = oacc[db][i] * a0 + xch[(2 + db * 16 + i) * 64] * a1;
+  }
+
+  const float l_tot = sum_over_wave_halves(l_i);
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  if (qi < a.Sq) {
+    float *op = reinterpret_cast<float *>(a.out) + b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2];
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; i4++) {
+        const int d = db * 32 + 8 * i4 + 4 * g;
+        if (d >= a.D) continue;
+        *reinterpret_cast<float4 *>(op + d) = make_float4(oacc[db][4 * i4 + 0] * inv, oacc[db][4 * i4 + 1] * inv,
+                                                          oacc[db][4 * i4 + 2] * inv, oacc[db][4 * i4 + 3] * inv);
+      }
+  }
+}
+
+template <int D, int NW, int KSPLIT>
+int launch_form(const PrefillArgs &a, hipStream_t stream) {
+  constexpr int BM = 32 * NW / KSPLIT;
+  const int n_q_tiles = (a.Sq + BM - 1) / BM;
+  const int64_t wgs = deal_grid((int64_t)a.B * a.Hq, n_q_tiles);
+  const int rc = check_grid(wgs, 64 * NW);
+  if (rc != LMH_OK) return rc;
+  dim3 grid((uint32_t)wgs), block(64 * NW);
+  if (plan_only("prefill_f32_split_kernel<D=%d, %s, key groups=%d> rows=%d, workgroups=%u", D, a.causal ? "causal" : "full", KSPLIT, BM, grid.x)) return LMH_OK;
+  const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? 8 / NW : 0, device_cu_count());
+  if (a.causal) hipLaunchKernelGGL((prefill_f32_split_kernel<D, true, NW, KSPLIT>), grid, block, 0, stream, deal, a);
+  else hipLaunchKernelGGL((prefill_f32_split_kernel<D, false, NW, KSPLIT>), grid, block, 0, stream, deal, a);
+  LMH_HIP_TRY(hipGetLastError());
+  return LMH_OK;
+}
+
+template <int D>
+int launch_for_d(const PrefillArgs &a, int form, hipStream_t stream) {
+  if (form == 0) return launch_form<D, 4, 2>(a, stream);
+  if (form == 1) return launch_form<D, 8, 2>(a, stream);
+  return launch_form<D, 8, 1>(a, stream);
+}
+
+}  // namespace
+
+// Estimated microseconds of the cheapest form (0: 64 rows, two workgroups on a CU; 1: 128 rows; 2: 256 rows), from the launch's own
+// tiles as in prefill_mfma.hip: without a mask whole rounds, causal the longest workgroup and the mean over the CUs. Fitted to 330
+// launches of drawn sizes, rms 3 to 10 %.
+double prefill_f32_split_cost(const PrefillArgs &a, int *form) {
+  struct Cost { double fixed, alone, per_wg, shared; };  // a tile of 64 keys in a CU's only workgroup, and in one of several
+  static const Cost costs[3][3][2] = {  // [head dims up to 64, 80, 96][form][causal]
+      {{{3.3, 1.89, 1.8, 1.33}, {3.6, 1.86, 1.8, 1.40}}, {{1.3, 2.26, 5.7, 0.}, {1.5, 2.13, 6.4, 2.47}}, {{0., 4.26, 8.4, 0.}, {0., 3.98, 8.4, 4.13}}},
+      {{{2.6, 2.61, 2.4, 1.76}, {3.3, 2.51, 2.7, 1.85}}, {{0., 3.00, 7.0, 0.}, {0., 2.86, 8.0, 3.28}}, {{0., 4.96, 10.3, 0.}, {0., 4.46, 10.1, 5.47}}},
+      {{{0.2, 3.36, 5.0, 2.28}, {2.3, 3.17, 5.5, 2.19}}, {{0., 3.30, 8.9, 0.}, {0., 3.03, 10.3, 3.44}}, {{0., 5.72, 11.6, 0.}, {0., 5.73, 10.0, 6.74}}}};
+  const int64_t cus = device_cu_count(), heads = (int64_t)a.B * a.Hq, row_tiles = (a.Sk + 63) / 64;
+  double least = INFINITY;
+  for (int f = 0; f < 3; f++) {
+    const Cost &c = costs[a.D <= 64 ? 0 : a.D <= 80 ? 1 : 2][f][a.causal != 0];
+    const int64_t step = int64_t(1) << f, n = (a.Sq + 64 * step - 1) / (64 * step), rounds = (heads * n + cus - 1) / cus;
+    double t;
+    if (!a.causal) {
+      const int64_t pairs = f == 0 ? rounds / 2 : 0;
+      t = c.fixed + row_tiles * (pairs * std::max(c.alone, 2 * c.shared) + (rounds - 2 * pairs) * c.alone) + c.per_wg * rounds;
+    } else {
+      const int64_t ramp = std::min(n, row_tiles / step);
+      const double longest = (double)std::min(row_tiles, n * step) * c.alone;
+      const double mean = (double)heads * (step * ramp * (ramp + 1) / 2 + (n - ramp) * row_tiles) / cus * c.shared;
+      t = rounds <= 1 ? c.fixed + longest + c.per_wg
+                      : c.fixed + sqrt(sqrt(longest * longest * longest * longest + mean * mean * mean * mean)) + c.per_wg * (heads * n) / cus;
+    }
+    if (t < least) least = t, *form = f;
+  }
+  return least;
+}
+
+int launch_prefill_f32_split(const PrefillArgs &a, int form, hipStream_t stream) {
+  if (a.D <= 64) return launch_for_d<64>(a, form, stream);
+  if (a.D <= 80) return launch_for_d<80>(a, form, stream);
+  return launch_for_d<96>(a, form, stream);
+}
+
+}  // namespace lmh

@@ -135,6 +135,56 @@ def test_forms_chosen_by_cost(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causal, dt
         assert rel_err(got, oracle.flash_attn(q, k, v, causal=causal, kv_len=kv_len, nthreads=NT)) <= TOL[dtype]
 
 
+PIECES = [(2, 16, 16, 300, 1000, 64, False, "D=64, full, key groups=2> rows=64"), (7, 24, 8, 1025, 330, 56, False, "D=64, full, key groups=2> rows=128"),
+          (3, 16, 4, 700, 500, 72, False, "D=80, full, key groups=1> rows=256"), (2, 33, 3, 513, 500, 96, False, "D=96, full, key groups=1> rows=256"),
+          (2, 12, 4, 1023, 401, 80, False, "D=80, full, key groups=2> rows=128"), (2, 20, 20, 300, 700, 88, False, "D=96, full, key groups=2> rows=64"),
+          (2, 33, 11, 1000, 1000, 80, True, "D=80, causal, key groups=2> rows=64"), (1, 32, 8, 1300, 1300, 96, True, "D=96, causal, key groups=2> rows=128"),
+          (5, 33, 33, 900, 900, 64, True, "D=64, causal, key groups=1> rows=256")]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,form", PIECES)
+def test_fp32_on_pieces(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causal, form):
+    q, k, v = inputs(oracle, (B, Hq, Sq, D), (B, Hkv, Sk, D), "f32", 36000 + Sq + D)
+    assert "prefill_f32_split_kernel<" + form in plan(lm, q, k, "f32", causal, False)
+    lens = np.array([(Sk - 30, 0, 33, Sk)[i % 4] for i in range(B)] if B > 1 else [Sk - 95], np.int32)
+    for kv_len in (None, lens):
+        got = run(lm, hip, q, k, v, "f32", causal, kv_len=None if kv_len is None else list(kv_len))
+        want = oracle.flash_attn(q, k, v, causal=causal, kv_len=None if kv_len is None else np.maximum(kv_len, 1), nthreads=NT)
+        if kv_len is not None:
+            want[kv_len == 0] = 0
+        assert rel_err(got, want) <= TOL["f32"]
+
+
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("Hq,S,D", [(32, 1300, 96), (40, 1999, 64)])
+def test_pieces_rotate_their_queries_in_registers(lm, hip, oracle, Hq, S, D, interleaved):
+    q, k, v = inputs(oracle, (1, Hq, S, D), (1, Hq, S, D), "f32", 36100 + D)
+    assert "prefill_f32_split_kernel" in plan(lm, q, k, "f32", True, True)
+    got = run(lm, hip, q, k, v, "f32", True, rope=(7, interleaved))
+    q_rot = rotated_on_device(lm, hip, q, "f32", prev_seq=7, interleaved=interleaved)
+    np.testing.assert_array_equal(got, run(lm, hip, q_rot, k, v, "f32", True))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_on_values_that_pieces_do_not_hold(lm, hip, oracle, causal):
+    """Infinities, NaN, values below the smallest normal piece and next to the largest: what fp32 gives, in the rows that see them."""
+    q, k, v = inputs(oracle, (1, 40, 1000, 80), (1, 8, 1000, 80), "f32", 36200)
+    assert "prefill_f32_split_kernel" in plan(lm, q, k, "f32", causal, False)
+    v[0, 0, 50, 3], v[0, 1, 60, 4] = np.inf, np.nan
+    k[0, 2, 70, 5], q[0, 2::8, :, 5] = 3.4e38, q[0, 2::8, :, 5] * np.float32(2.0 ** -126)
+    v[0, 3] *= np.float32(2.0 ** -122)
+    k[0, 4], q[0, 4::8] = k[0, 4] * np.float32(2.0 ** -110), q[0, 4::8] * np.float32(2.0 ** 110)
+    got = run(lm, hip, q, k, v, "f32", causal)
+    want = oracle.flash_attn(q, k, v, causal=causal, nthreads=NT)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    finite = np.isfinite(want)
+    for h in range(8):  # the heads of a KV head are of one magnitude
+        ok = finite[0, h::8]
+        err = np.abs(np.where(ok, got[0, h::8] - np.where(ok, want[0, h::8], 0), 0))
+        assert err.max() <= TOL["f32"] * np.abs(want[0, h::8][ok]).max()
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
 def test_launches_with_very_many_heads(lm, hip, oracle, dtype):
     """More heads than a 32-bit reciprocal divides exactly: every one of them is computed."""
