@@ -9,6 +9,7 @@
 #include <mutex>
 
 #include "common.hpp"
+#include "copy.hpp"
 
 // Split-KV partial storage of lmh_decode_attn_static, for callers that cannot allocate device memory.
 // One copy per GPU, held from the moment the code object is loaded on that GPU until the process ends.
@@ -392,7 +393,7 @@ int lmh_event_elapsed_ms(float *ms, void *start, void *stop) {
 // --------------------------------------------------------------------------------------------
 // flash attention forward
 // --------------------------------------------------------------------------------------------
-int lmh_flash_attn_fwd(const lmh_attn_params *p) {
+static int attn_args(const lmh_attn_params *p, PrefillArgs &a, bool &mfma_ok) {
   if (!p) return fail(LMH_E_NULL, "lmh_flash_attn_fwd: null params");
   if (!p->out || !p->q || !p->k || !p->v) return fail(LMH_E_NULL, "lmh_flash_attn_fwd: null tensor pointer");
   if (p->B <= 0 || p->Hq <= 0 || p->Hkv <= 0 || p->Sq <= 0 || p->Sk <= 0 || p->D <= 0)
@@ -413,7 +414,6 @@ int lmh_flash_attn_fwd(const lmh_attn_params *p) {
     if (!(p->q_rope_base > 0.f)) return fail(LMH_E_SHAPE, "lmh_flash_attn_fwd: q_rope_base must be positive");
   }
 
-  PrefillArgs a;
   a.out = p->out; a.q = p->q; a.k = p->k; a.v = p->v; a.kv_len = p->kv_len;
   a.B = p->B; a.Hq = p->Hq; a.Hkv = p->Hkv; a.Sq = p->Sq; a.Sk = p->Sk; a.D = p->D;
   a.scale = p->scale; a.causal = p->causal ? 1 : 0; a.head_map = p->head_map;
@@ -443,7 +443,7 @@ int lmh_flash_attn_fwd(const lmh_attn_params *p) {
   // The matrix-core kernels do 128-bit accesses, track the max on raw scores (needs scale > 0) and fetch
   // K/V tiles with 32-bit buffer offsets inside one (b, kv head) slice.
   const int64_t esz = (int64_t)elem_bytes(p->dtype), vec = 16 / esz;
-  bool mfma_ok = (prefill_mfma_supported(p->dtype, p->D) || prefill_f32_mfma_supported(p->dtype, p->D)) && p->scale > 0.f &&
+  mfma_ok = (prefill_mfma_supported(p->dtype, p->D) || prefill_f32_mfma_supported(p->dtype, p->D)) && p->scale > 0.f &&
                  aligned16(p->q) && aligned16(p->k) && aligned16(p->v) && aligned16(p->out);
   // (offsets from 0x7ffffff0 up are what the half-precision kernel uses as "out of range")
   constexpr int64_t kMaxSliceBytes = 0x7ffffff0;
@@ -451,9 +451,20 @@ int lmh_flash_attn_fwd(const lmh_attn_params *p) {
   mfma_ok = mfma_ok && (!p->q_rope || prefill_mfma_rope_ok(p->D));  // the rotation in registers needs a head dim that fills its tiling
   for (int i = 0; i < 3 && mfma_ok; i++)
     mfma_ok = (a.qs[i] % vec == 0) && (a.ks[i] % vec == 0) && (a.vs[i] % vec == 0) && (a.os[i] % vec == 0);
-  if (mfma_ok && p->dtype == LMH_F32) return launch_prefill_f32_mfma(a, (hipStream_t)p->stream);
-  if (mfma_ok) return launch_prefill_mfma(a, p->dtype, (hipStream_t)p->stream);
-  return launch_prefill_valu(a, p->dtype, (hipStream_t)p->stream);
+  return LMH_OK;
+}
+
+static int launch_attn(const PrefillArgs &a, int dtype, bool mfma_ok, hipStream_t stream) {
+  if (mfma_ok && dtype == LMH_F32) return launch_prefill_f32_mfma(a, stream);
+  if (mfma_ok) return launch_prefill_mfma(a, dtype, stream);
+  return launch_prefill_valu(a, dtype, stream);
+}
+
+int lmh_flash_attn_fwd(const lmh_attn_params *p) {
+  PrefillArgs a;
+  bool mfma_ok;
+  const int rc = attn_args(p, a, mfma_ok);
+  return rc != LMH_OK ? rc : launch_attn(a, p->dtype, mfma_ok, (hipStream_t)p->stream);
 }
 
 int lmh_flash_attn_plan(const lmh_attn_params *p, char *plan, size_t plan_bytes) {
@@ -493,9 +504,8 @@ size_t lmh_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lm
 
 // Validation and launch shared by lmh_decode_attn (caller-owned workspace) and lmh_decode_attn_static (the
 // library's static scratch): `ws` / `ws_bytes` is the split-KV partial storage, `num_splits` already resolved.
-static int decode_launch(const lmh_decode_params *p, const char *fn, int32_t num_splits, void *ws, size_t ws_bytes,
-                         const lmh_decode_step_extra *step = nullptr) {
-  DecodeArgs a;
+static int decode_args(const lmh_decode_params *p, const char *fn, int32_t num_splits, void *ws, size_t ws_bytes,
+                       const lmh_decode_step_extra *step, DecodeArgs &a) {
   a.step = step ? 1 : 0;
   a.q_rope = (step && step->rope) ? 1 : 0;
   a.rope_interleaved = (step && step->pairing == LMH_ROPE_INTERLEAVED) ? 1 : 0;
@@ -557,7 +567,13 @@ static int decode_launch(const lmh_decode_params *p, const char *fn, int32_t num
       return fail(LMH_E_UNSUPPORTED, "%s: head dim %d with the half-split pairing cannot be rotated in registers; use lmh_kv_append + "
                   "lmh_decode_attn", fn, p->D);
   }
-  return launch_decode(a, p->dtype, (hipStream_t)p->stream);
+  return LMH_OK;
+}
+
+static int decode_launch(const lmh_decode_params *p, const char *fn, int32_t num_splits, void *ws, size_t ws_bytes) {
+  DecodeArgs a;
+  const int rc = decode_args(p, fn, num_splits, ws, ws_bytes, nullptr, a);
+  return rc != LMH_OK ? rc : launch_decode(a, p->dtype, (hipStream_t)p->stream);
 }
 
 static int decode_check(const lmh_decode_params *p, const char *fn) {
@@ -591,7 +607,7 @@ int32_t lmh_decode_step_splits(int32_t B, int32_t Hkv, int32_t Lmax) {
   return s == 0 ? 0 : (s < 2 ? 2 : s);  // the merge launch always runs: it is what adds the new row
 }
 
-int lmh_decode_step(const lmh_decode_params *p, const lmh_decode_step_extra *x) {
+static int decode_step_args(const lmh_decode_params *p, const lmh_decode_step_extra *x, DecodeArgs &a) {
   const char *fn = "lmh_decode_step";
   const int rc = decode_check(p, fn);
   if (rc != LMH_OK) return rc;
@@ -603,7 +619,13 @@ int lmh_decode_step(const lmh_decode_params *p, const lmh_decode_step_extra *x) 
   if (x->rope && !(x->rope_base > 1.f)) return fail(LMH_E_SHAPE, "%s: rope base must be > 1", fn);
   if (p->num_splits == 1) return fail(LMH_E_SHAPE, "%s: num_splits must be 0 or >= 2", fn);
   const int32_t splits = p->num_splits == 0 ? lmh_decode_step_splits(p->B, p->Hkv, p->Lmax) : p->num_splits;
-  return decode_launch(p, fn, splits, p->workspace, p->workspace_bytes, x);
+  return decode_args(p, fn, splits, p->workspace, p->workspace_bytes, x, a);
+}
+
+int lmh_decode_step(const lmh_decode_params *p, const lmh_decode_step_extra *x) {
+  DecodeArgs a;
+  const int rc = decode_step_args(p, x, a);
+  return rc != LMH_OK ? rc : launch_decode(a, p->dtype, (hipStream_t)p->stream);
 }
 
 // --------------------------------------------------------------------------------------------
@@ -675,7 +697,7 @@ int lmh_rope(const lmh_rope_params *p) {
   return launch_rope(a, p->dtype, (hipStream_t)p->stream);
 }
 
-int lmh_kv_append(const lmh_kv_append_params *p) {
+static int append_args(const lmh_kv_append_params *p, KvAppendArgs &a) {
   if (!p) return fail(LMH_E_NULL, "lmh_kv_append: null params");
   if (!p->k_cache || !p->v_cache || !p->k_new || !p->v_new) return fail(LMH_E_NULL, "lmh_kv_append: null tensor pointer");
   if (p->B <= 0 || p->Hkv <= 0 || p->T <= 0 || p->D <= 0 || p->Lmax <= 0)
@@ -690,7 +712,6 @@ int lmh_kv_append(const lmh_kv_append_params *p) {
       return fail(LMH_E_UNSUPPORTED, "lmh_kv_append: unknown pairing %d", p->pairing);
     if (!(p->base > 0.f)) return fail(LMH_E_SHAPE, "lmh_kv_append: base must be positive");
   }
-  KvAppendArgs a;
   a.k_cache = p->k_cache; a.v_cache = p->v_cache; a.k_new = p->k_new; a.v_new = p->v_new;
   a.pos = p->pos; a.pos_all = p->pos_all;
   a.B = p->B; a.Hkv = p->Hkv; a.T = p->T; a.D = p->D; a.Lmax = p->Lmax;
@@ -708,7 +729,13 @@ int lmh_kv_append(const lmh_kv_append_params *p) {
   a.log2_base = (p->rope_k || p->q_rope) ? log2f(p->base) : 0.f;
   a.q = p->q_rope;
   a.Hq = p->q_rope ? p->Hq : 0;
-  return launch_kv_append(a, p->dtype, (hipStream_t)p->stream);
+  return LMH_OK;
+}
+
+int lmh_kv_append(const lmh_kv_append_params *p) {
+  KvAppendArgs a;
+  const int rc = append_args(p, a);
+  return rc != LMH_OK ? rc : launch_kv_append(a, p->dtype, (hipStream_t)p->stream);
 }
 
 // --------------------------------------------------------------------------------------------
@@ -771,15 +798,16 @@ int lmh_map(const lmh_map_params *p, void *stream) {
   return launch_map(a, (hipStream_t)stream);
 }
 
+static bool meet(const void *x, size_t nx, const void *y, size_t ny) {
+  return (uintptr_t)x < (uintptr_t)y + ny && (uintptr_t)y < (uintptr_t)x + nx;
+}
+
 int lmh_copy_many(void *const *dst, const void *const *src, const size_t *bytes, int32_t n, void *stream) {
   static_assert(LMH_COPY_MANY == kCopyMany, "header and kernel agree");
   if (n < 0) return fail(LMH_E_SHAPE, "lmh_copy_many: negative count");
   if (n > 0 && (!dst || !src || !bytes)) return fail(LMH_E_NULL, "lmh_copy_many: null list");
   for (int32_t i = 0; i < n; i++)
     if (bytes[i] && (!dst[i] || !src[i])) return fail(LMH_E_NULL, "lmh_copy_many: null pointer");
-  auto meet = [](const void *x, size_t nx, const void *y, size_t ny) {
-    return (uintptr_t)x < (uintptr_t)y + ny && (uintptr_t)y < (uintptr_t)x + nx;
-  };
   CopyManyArgs a = {};
   int m = 0;  // ranges of the launch that is being put together
   auto launch = [&]() {
@@ -807,6 +835,156 @@ int lmh_copy_many(void *const *dst, const void *const *src, const size_t *bytes,
     m++;
   }
   return launch();
+}
+
+}  // extern "C"
+
+// --------------------------------------------------------------------------------------------
+// launches that take their operands from the caller's arrays and copy those into the graph's buffers on the side
+// --------------------------------------------------------------------------------------------
+namespace {
+
+// The bytes from the first element to the last one of a tensor.
+template <int N>
+int64_t extent(const int64_t (&stride)[N], std::initializer_list<int64_t> dims, int64_t D, int64_t esz) {
+  int64_t last = D - 1;
+  int i = 0;
+  for (int64_t n : dims) last += (n - 1) * stride[i++];
+  return (last + 1) * esz;
+}
+
+// Copies whose order among themselves and against the launch that carries them does not matter.
+struct Feed {
+  CopyManyArgs a = {};
+  int n = 0;
+
+  // Whether the copies may all run at once; from then on `a` holds those that move something.
+  bool apart(void *const *dst, const void *const *src, const size_t *bytes, int32_t count) {
+    if (count < 0 || (count > 0 && (!dst || !src || !bytes))) return false;
+    for (int32_t i = 0; i < count; i++) {
+      if (!bytes[i] || dst[i] == src[i]) continue;
+      if (!dst[i] || !src[i] || n == kCopyMany || touches(dst[i], bytes[i]) || writes(src[i], bytes[i]) || meet(dst[i], bytes[i], src[i], bytes[i]))
+        return false;
+      a.dst[n] = dst[i]; a.src[n] = src[i]; a.bytes[n] = (int64_t)bytes[i];
+      n++;
+    }
+    return true;
+  }
+  bool writes(const void *p, int64_t bytes) const {
+    for (int j = 0; j < n; j++)
+      if (meet(p, bytes, a.dst[j], a.bytes[j])) return true;
+    return false;
+  }
+  bool touches(const void *p, int64_t bytes) const {
+    for (int j = 0; j < n; j++)
+      if (meet(p, bytes, a.src[j], a.bytes[j])) return true;
+    return writes(p, bytes);
+  }
+  // Sends an operand inside one of the destinations to where its values come from, which has to be as aligned as the
+  // destination is; false for one that lies across an end.
+  template <typename T>
+  bool redirect(T *&p, int64_t bytes) const {
+    for (int j = 0; j < n; j++) {
+      if (!meet(p, bytes, a.dst[j], a.bytes[j])) continue;
+      const intptr_t at = (intptr_t)p - (intptr_t)a.dst[j];
+      if (at < 0 || at + bytes > a.bytes[j] || !aligned16(a.src[j]) || !aligned16(a.dst[j])) return false;
+      p = (T *)((const char *)a.src[j] + at);
+      return true;
+    }
+    return true;
+  }
+  // Copies that a launch has workgroups for, beside its own.
+  bool some() {
+    const int64_t blocks = number_copy_blocks(a, n);
+    return blocks > 0 && blocks <= 32768;
+  }
+  // The copy that fills exactly this tensor, both ends 16-byte aligned; -1: there is none.
+  int of(const void *p, int64_t bytes) const {
+    for (int j = 0; j < n; j++)
+      if (p == a.dst[j] && bytes == a.bytes[j] && aligned16(a.dst[j]) && aligned16(a.src[j])) return j;
+    return -1;
+  }
+  void drop(int j) {
+    n--;
+    a.dst[j] = a.dst[n]; a.src[j] = a.src[n]; a.bytes[j] = a.bytes[n];
+  }
+};
+
+}  // namespace
+
+extern "C" {
+
+int lmh_decode_step_fed(const lmh_decode_params *p, const lmh_decode_step_extra *x, void *const *dst, const void *const *src,
+                        const size_t *bytes, int32_t n) {
+  DecodeArgs a;
+  Feed feed;
+  if (feed.apart(dst, src, bytes, n) && feed.n && decode_step_args(p, x, a) == LMH_OK) {
+    const int64_t esz = (int64_t)elem_bytes(p->dtype), rows = (int64_t)p->B * p->Hkv * p->D * esz;
+    bool ok = feed.some() && !feed.touches(a.out, extent(a.os, {p->B, p->Hq}, p->D, a.out_f32 ? 4 : esz)) &&
+              !feed.touches(a.k, extent(a.ks, {p->B, p->Hkv, p->Lmax}, p->D, esz)) &&
+              !feed.touches(a.v, extent(a.vs, {p->B, p->Hkv, p->Lmax}, p->D, esz)) &&
+              !feed.touches(a.ws_o, (int64_t)lmh_decode_workspace_bytes(p->B, p->Hq, p->Hkv, p->Lmax, p->D, a.num_splits));
+    ok = ok && feed.redirect(a.q, extent(a.qs, {p->B, p->Hq}, p->D, esz)) && feed.redirect(a.k_new, rows) &&
+         feed.redirect(a.v_new, rows) && feed.redirect(a.kv_len, (int64_t)p->B * 4);
+    if (ok) return launch_decode(a, p->dtype, (hipStream_t)p->stream, &feed.a, feed.n);
+  }
+  const int rc = lmh_copy_many(dst, src, bytes, n, p ? p->stream : nullptr);
+  return rc != LMH_OK ? rc : lmh_decode_step(p, x);
+}
+
+// Lets an attention launch read its queries from the caller's array and store them itself: under a causal mask on the
+// 16-bit matrix-core kernels up to head dim 128, whole contiguous tensors that nothing of this launch or the append in front of it lies in.
+static void attention_stores_queries(const lmh_kv_append_params *p, Feed &feed, PrefillArgs &f, int dtype, bool mfma_ok, QueryCopy &queries) {
+#ifdef LMH_W64_KERNEL
+  return;
+#endif
+  const int64_t esz = (int64_t)elem_bytes(dtype), bytes = (int64_t)f.B * f.Hq * f.Sq * f.D * esz;
+  if (!mfma_ok || dtype == LMH_F32 || !f.causal || f.D > 128 || f.qs[2] != f.D || f.qs[1] != (int64_t)f.Sq * f.D || f.qs[0] != (int64_t)f.Hq * f.Sq * f.D)
+    return;
+  const int j = feed.of(f.q, bytes);
+  if (j < 0) return;
+  const int64_t rows = (int64_t)p->B * p->Hkv * p->T * p->D * (int64_t)elem_bytes(p->dtype);
+  const struct { const void *at; int64_t bytes; } others[] = {
+      {f.out, extent(f.os, {f.B, f.Hq, f.Sq}, f.D, f.out_f32 ? 4 : esz)}, {f.k, extent(f.ks, {f.B, f.Hkv, f.Sk}, f.D, esz)},
+      {f.v, extent(f.vs, {f.B, f.Hkv, f.Sk}, f.D, esz)}, {f.kv_len, (int64_t)f.B * 4}, {f.q_pos0, (int64_t)f.B * 4},
+      {p->k_new, rows}, {p->v_new, rows}, {p->pos, (int64_t)p->B * 4}};
+  for (const auto &o : others)
+    if (o.at && (meet(o.at, o.bytes, feed.a.dst[j], bytes) || meet(o.at, o.bytes, feed.a.src[j], bytes))) return;
+  f.q = queries.src = feed.a.src[j];
+  queries.dst = feed.a.dst[j];
+  feed.drop(j);
+}
+
+int lmh_kv_append_fed(const lmh_kv_append_params *p, const lmh_attn_params *attn, void *const *dst, const void *const *src,
+                      const size_t *bytes, int32_t n) {
+  KvAppendArgs a;
+  PrefillArgs f;
+  bool mfma_ok = false;
+  Feed feed;
+  if (feed.apart(dst, src, bytes, n) && append_args(p, a) == LMH_OK &&
+      (!attn || (attn->stream == p->stream && attn_args(attn, f, mfma_ok) == LMH_OK))) {
+    const int64_t esz = (int64_t)elem_bytes(p->dtype), rows = (int64_t)p->B * p->Hkv * p->T * p->D * esz;
+    bool ok = feed.some() && !feed.touches(a.k_cache, extent(a.ks, {p->B, p->Hkv, p->Lmax}, p->D, esz)) &&
+              !feed.touches(a.v_cache, extent(a.vs, {p->B, p->Hkv, p->Lmax}, p->D, esz));
+    if (ok && a.q) {  // rotated on the way from the caller's array, where that is all that is made of it
+      const int64_t q_bytes = (int64_t)p->B * p->Hq * p->T * p->D * esz;
+      const int j = feed.of(a.q, q_bytes);
+      ok = j >= 0 && !meet(a.q, q_bytes, p->k_new, rows) && !meet(a.q, q_bytes, p->v_new, rows) &&
+           !(p->pos && meet(a.q, q_bytes, p->pos, (int64_t)p->B * 4));
+      if (ok) a.q_from = feed.a.src[j], feed.drop(j);
+    }
+    ok = ok && feed.redirect(a.k_new, rows) && feed.redirect(a.v_new, rows) && (!a.pos || feed.redirect(a.pos, (int64_t)p->B * 4));
+    if (ok) {
+      QueryCopy queries;
+      if (attn) attention_stores_queries(p, feed, f, attn->dtype, mfma_ok, queries);
+      const int rc = launch_kv_append(a, p->dtype, (hipStream_t)p->stream, &feed.a, feed.n);
+      if (rc != LMH_OK || !attn) return rc;
+      return queries.dst ? launch_prefill_mfma(f, attn->dtype, (hipStream_t)p->stream, queries) : launch_attn(f, attn->dtype, mfma_ok, (hipStream_t)p->stream);
+    }
+  }
+  int rc = lmh_copy_many(dst, src, bytes, n, p ? p->stream : nullptr);
+  if (rc == LMH_OK) rc = lmh_kv_append(p);
+  return rc != LMH_OK || !attn ? rc : lmh_flash_attn_fwd(attn);
 }
 
 }  // extern "C"

@@ -49,6 +49,13 @@ struct PrefillArgs {
   float q_log2_base;
 };
 
+// A causal launch of prefill_mfma.hip that stores its queries, whole and contiguous, as they are. Not a part of PrefillArgs: what
+// request_args asks for occupies registers from the start.
+struct QueryCopy {
+  void *dst = nullptr;  // null: no copy
+  const void *src = nullptr;
+};
+
 // Decode launch arguments.
 struct DecodeArgs {
   void *out;
@@ -98,6 +105,8 @@ struct KvAppendArgs {
   float log2_base;
   void *q;         // optional [B, Hq, T, D], contiguous: rotated in place at the same positions
   int32_t Hq;
+  const void *q_from = nullptr;  // where q comes from if not from itself
+  void *k_copy = nullptr, *v_copy = nullptr;  // where k_new and v_new are to be stored as they are, or null (16-byte chunks only)
 };
 
 // Matrix products of one launch (matmul.hip): c[batch, m, j] = sum_k a[batch, m, k] b[batch, k, j] (+ bias[j]).
@@ -166,7 +175,7 @@ __device__ __forceinline__ void request_args(const RopeArgs &a) {
 }
 __device__ __forceinline__ void request_args(const KvAppendArgs &a) {
   asm volatile("" ::"s"(a.k_cache), "s"(a.v_cache), "s"(a.k_new), "s"(a.v_new), "s"(a.pos), "s"(a.pos_all), "s"(a.B), "s"(a.Hkv), "s"(a.T), "s"(a.D), "s"(a.Lmax));
-  asm volatile("" ::"s"(a.ks[0]), "s"(a.ks[1]), "s"(a.ks[2]), "s"(a.vs[0]), "s"(a.vs[1]), "s"(a.vs[2]), "s"(a.rope_k), "s"(a.interleaved), "s"(a.log2_base), "s"(a.q), "s"(a.Hq));
+  asm volatile("" ::"s"(a.ks[0]), "s"(a.ks[1]), "s"(a.ks[2]), "s"(a.vs[0]), "s"(a.vs[1]), "s"(a.vs[2]), "s"(a.rope_k), "s"(a.interleaved), "s"(a.log2_base), "s"(a.q), "s"(a.Hq), "s"(a.q_from), "s"(a.k_copy), "s"(a.v_copy));
 }
 
 __host__ __device__ inline int kv_head_of(int hq, int Hq, int Hkv, int head_map) {
@@ -190,7 +199,7 @@ __device__ __forceinline__ void request_args(const Deal &t) {
 // that fill a tiling exactly.
 inline bool prefill_mfma_rope_ok(int D) { return D == 64 || D == 96 || D == 128 || D == 192 || D == 256; }
 bool prefill_mfma_supported(int dtype, int D);
-int launch_prefill_mfma(const PrefillArgs &a, int dtype, hipStream_t stream);
+int launch_prefill_mfma(const PrefillArgs &a, int dtype, hipStream_t stream, const QueryCopy &queries = {});
 #ifdef LMH_W64_KERNEL
 // measurement builds only (prefill_mfma_w64.hip): the hand-pipelined 64-columns-per-wave kernel and the launches it takes
 bool prefill_w64_takes(const PrefillArgs &a, int dtype);
@@ -202,9 +211,10 @@ int launch_prefill_f32_full(const PrefillArgs &a, int key_groups, hipStream_t st
 double prefill_f32_split_cost(const PrefillArgs &a, int *form);  // head dim <= 96: microseconds of its cheapest form
 int launch_prefill_f32_split(const PrefillArgs &a, int form, hipStream_t stream);
 int launch_prefill_valu(const PrefillArgs &a, int dtype, hipStream_t stream);
-int launch_decode(const DecodeArgs &a, int dtype, hipStream_t stream);
+// n_fed copies beside the launch (copy.hpp; 2^31 workgroups hold them): by workgroups of its last kernel
+int launch_decode(const DecodeArgs &a, int dtype, hipStream_t stream, CopyManyArgs *fed = nullptr, int n_fed = 0);
 int launch_rope(const RopeArgs &a, int dtype, hipStream_t stream);
-int launch_kv_append(const KvAppendArgs &a, int dtype, hipStream_t stream);
+int launch_kv_append(KvAppendArgs a, int dtype, hipStream_t stream, CopyManyArgs *fed = nullptr, int n_fed = 0);  // ... of its first
 int launch_matmul(MatmulArgs &args, int n, hipStream_t stream);
 int launch_map(MapArgs &a, hipStream_t stream);
 int launch_copy_many(CopyManyArgs &a, int n, hipStream_t stream);

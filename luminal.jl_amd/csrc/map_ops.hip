@@ -8,6 +8,7 @@
 //   * tiles: where an operand's contiguous dimension is another one than out's (a transpose), 64 x 64 tiles of those two
 //     dimensions pass through LDS, so that both sides move whole lines.
 #include "common.hpp"
+#include "copy.hpp"
 #include "dtypes.hpp"
 
 namespace lmh {
@@ -120,29 +121,7 @@ __global__ __launch_bounds__(256) void map_tiles_kernel(MapArgs a, int tiles_in,
 
 // Up to kCopyMany byte ranges in one launch: the inputs of a compiled graph's call are a handful of small tensors, and a
 // runtime copy of each costs the host 3.4 us (a decode step's five: 17.8 us of its 26 us). A workgroup moves 16 KB.
-constexpr int kCopyChunk = 16384;
-__global__ __launch_bounds__(256) void copy_many_kernel(CopyManyArgs a) {
-  int j = 0;
-#pragma unroll
-  for (int i = 1; i < kCopyMany; i++)
-    if (blockIdx.x >= (unsigned)a.first_block[i]) j = i;
-  const int64_t begin = (int64_t)(blockIdx.x - a.first_block[j]) * kCopyChunk;
-  const int64_t end = min(begin + kCopyChunk, a.bytes[j]);
-  char *dst = reinterpret_cast<char *>(a.dst[j]);
-  const char *src = reinterpret_cast<const char *>(a.src[j]);
-  if (((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) == 0) {
-    const int64_t whole = end & ~(int64_t)15;
-#pragma unroll
-    for (int r = 0; r < kCopyChunk / (256 * 16); r++) {
-      const int64_t i = begin + (r * 256 + threadIdx.x) * 16;
-      if (i < whole) *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(src + i);
-    }
-    const int64_t i = max(whole, begin) + threadIdx.x;
-    if (i < end) dst[i] = src[i];
-  } else {
-    for (int64_t i = begin + threadIdx.x; i < end; i += 256) dst[i] = src[i];
-  }
-}
+__global__ __launch_bounds__(256) void copy_many_kernel(CopyManyArgs a) { copy_block<256>(a, blockIdx.x); }
 
 }  // namespace
 
@@ -178,12 +157,8 @@ int launch_map(MapArgs &a, hipStream_t stream) {
 }
 
 int launch_copy_many(CopyManyArgs &a, int n, hipStream_t stream) {
-  int64_t blocks = 0;
-  for (int i = 0; i < kCopyMany; i++) {
-    a.first_block[i] = (int32_t)blocks;
-    if (i < n) blocks += (a.bytes[i] + kCopyChunk - 1) / kCopyChunk;
-    if (blocks >= (int64_t(1) << 31)) return fail(LMH_E_UNSUPPORTED, "copy: too many bytes in one call");
-  }
+  const int64_t blocks = number_copy_blocks(a, n);
+  if (blocks < 0) return fail(LMH_E_UNSUPPORTED, "copy: too many bytes in one call");
   if (blocks == 0) return LMH_OK;
   hipLaunchKernelGGL(copy_many_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, a);
   LMH_HIP_TRY(hipGetLastError());

@@ -103,7 +103,7 @@ __device__ inline void rotate_q_fragments_with_table(typename MT::vec8 (&qreg)[D
 // WPS: waves per SIMD the register budget is set for (3 x 4 waves, 2 x 8 waves or 1 x 8 waves per CU).
 template <int D, int NW> constexpr int default_wps() { return D > 128 ? 1 : D > 96 ? 2 : NW == 8 ? 4 : 3; }
 template <typename MT, int D, bool CAUSAL, int KSPLIT, int NW, int WPS>
-__global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, PrefillArgs a) {
+__global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, PrefillArgs a, QueryCopy queries) {
   request_args(a);
   request_args(deal);
   using vec8 = typename MT::vec8;
@@ -557,6 +557,16 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
 #pragma unroll
       for (int i = 0; i < 16; i++) oacc[db][i] *= f;
   }
+  // ---- the queries' copy, where the workgroups of a CU are at different places of their tiles: beside the loads of Q all
+  // workgroups would store at once (B=4 H=32/8 T=777 D=128 fp16: 53.4 us, here 51.2, without a copy 46.0; a launch for the copy
+  // 8). Workgroups of their own for it, between or behind the others, took 67 and 56 us. Not above head dim 128, where one
+  // workgroup has the CU (D=256, 1500 rows: 1 % slower without a copy to make). ----
+  auto store_queries = [&]() {
+    const int64_t at = ((int64_t)(b * a.Hq + hq) * a.Sq + q0) * a.D * 2;
+    copy_span<64 * NW, (D / 16 + KSPLIT - 1) / KSPLIT>((char *)queries.dst + at, (const char *)queries.src + at, min(BM, a.Sq - q0) * a.D * 2, wave_u);
+  };
+  if (CAUSAL && KSPLIT > 1 && D <= 128 && queries.dst) store_queries();  // (before its second key group's waves end)
+
   // ---- key groups: fold group 1's (m, l, O) into group 0's; lane for lane the same layout ----
   if constexpr (KSPLIT > 1 && RG * (DB * 16 + 2) * 64 * 4 > (int)sizeof(Ks2)) {
     // in two halves of the head dim: the K tiles hold one at a time
@@ -629,6 +639,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
     const int64_t off = b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2];
     store_out_rows<MT, DB, false>(oacc, inv, a.out, off, g, a.D, a.out_f32);
   }
+  if (CAUSAL && KSPLIT == 1 && D <= 128 && queries.dst) store_queries();
 }
 
 // One workgroup per CU for non-causal launches with too few query rows to go round: the workgroup owns R
@@ -907,7 +918,7 @@ __global__ __launch_bounds__(1024, 4) void prefill_mfma_wide_kernel(PrefillArgs 
 // Without a mask (CAUSAL = false) the two tiles are neighbours — a 512-row tile — and share every fragment to the end.
 // ---------------------------------------------------------------------------------------------------------------
 template <typename MT, int D, bool CAUSAL>
-__global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a, Deal deal, int n_q_tiles) {
+__global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a, Deal deal, int n_q_tiles, QueryCopy queries) {
   request_args(a);
   request_args(deal);
   request_arg(n_q_tiles);
@@ -1258,10 +1269,17 @@ __global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a
     }
   }
   store_rows(1);
+  if (CAUSAL && queries.dst) {
+    for (int t = has_early ? 0 : 1; t < 2; t++) {
+      const int q0 = (t ? t_late : t_early) * BM;
+      const int64_t at = ((int64_t)(b * a.Hq + hq) * a.Sq + q0) * a.D * 2;
+      copy_span<64 * NW, D / 16>((char *)queries.dst + at, (const char *)queries.src + at, min(BM, a.Sq - q0) * a.D * 2, wave_u);
+    }
+  }
 }
 
 template <typename MT, int D>
-int launch_pair(const PrefillArgs &a, hipStream_t stream) {
+int launch_pair(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream) {
   const int n_q_tiles = (a.Sq + 255) / 256;
   const int n_pairs = (n_q_tiles + 1) / 2;
   const int64_t wgs = deal_grid((int64_t)a.B * a.Hq, n_pairs);
@@ -1271,9 +1289,9 @@ int launch_pair(const PrefillArgs &a, hipStream_t stream) {
   if (plan_only("prefill_mfma_pair_kernel<%s, D=%d, %s> query tiles=%d, workgroups=%u", MT::kName, D, a.causal ? "causal" : "full", n_q_tiles, grid.x)) return LMH_OK;
   const Deal deal = make_deal(a.B, a.Hq, n_pairs, 0, device_cu_count());
   if (a.causal)
-    hipLaunchKernelGGL((prefill_mfma_pair_kernel<MT, D, true>), grid, block, 0, stream, a, deal, n_q_tiles);
+    hipLaunchKernelGGL((prefill_mfma_pair_kernel<MT, D, true>), grid, block, 0, stream, a, deal, n_q_tiles, queries);
   else
-    hipLaunchKernelGGL((prefill_mfma_pair_kernel<MT, D, false>), grid, block, 0, stream, a, deal, n_q_tiles);
+    hipLaunchKernelGGL((prefill_mfma_pair_kernel<MT, D, false>), grid, block, 0, stream, a, deal, n_q_tiles, queries);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }
@@ -1286,7 +1304,7 @@ template <typename MT, bool V16, int KSPLIT> struct base_policy { using type = M
 template <> struct base_policy<MfmaBF16, true, 1> { using type = MfmaBF16V16; };
 
 template <typename MT0, bool V16, int D, int KSPLIT, int NW, int WPS = default_wps<D, NW>()>
-int launch_split(const PrefillArgs &a, hipStream_t stream) {
+int launch_split(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream) {
   using MT = typename base_policy<MT0, V16, KSPLIT>::type;
   constexpr int BM = 32 * NW / KSPLIT;
   const int n_q_tiles = (a.Sq + BM - 1) / BM;
@@ -1299,9 +1317,9 @@ int launch_split(const PrefillArgs &a, hipStream_t stream) {
     return LMH_OK;
   const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? 4 * WPS / NW : 0, device_cu_count());
   if (a.causal)
-    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS>), grid, block, 0, stream, deal, a);
+    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS>), grid, block, 0, stream, deal, a, queries);
   else
-    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, false, KSPLIT, NW, WPS>), grid, block, 0, stream, deal, a);
+    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, false, KSPLIT, NW, WPS>), grid, block, 0, stream, deal, a, queries);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }
@@ -1437,7 +1455,7 @@ inline double form_cost(const FormCost &f, const PrefillArgs &a, int form, int p
 // Launch the cheapest form, in favour of the one that the rules by size chose. bf16 launches whose weights are head + remainder
 // by those rules stay so: V as fp16 goes with weights of 11 bits.
 template <typename MT, int D, bool V16>
-int launch_cheapest(const PrefillArgs &a, int by_size, hipStream_t stream) {
+int launch_cheapest(const PrefillArgs &a, const QueryCopy &queries, int by_size, hipStream_t stream) {
   constexpr int tiling = D / 32 - 2;
   const int n_cus = device_cu_count();
   const bool v16 = V16 && by_size != kKeysSplit64;
@@ -1459,15 +1477,15 @@ int launch_cheapest(const PrefillArgs &a, int by_size, hipStream_t stream) {
     }
   auto launch = [&](auto with_v) {
     constexpr bool V = decltype(with_v)::value;
-    if (best == kKeysSplit64) return launch_split<MT, V, D, 2, 4>(a, stream);
+    if (best == kKeysSplit64) return launch_split<MT, V, D, 2, 4>(a, queries, stream);
     if constexpr (D <= 96) {
-      if (best == kRows256) return launch_split<MT, V, D, 1, 8, 2>(a, stream);
+      if (best == kRows256) return launch_split<MT, V, D, 1, 8, 2>(a, queries, stream);
       if constexpr (!(D == 96 && V))  // (its registers spill at four waves per SIMD)
-        if (best == kRows256Pair) return launch_split<MT, V, D, 1, 8>(a, stream);
+        if (best == kRows256Pair) return launch_split<MT, V, D, 1, 8>(a, queries, stream);
     } else if constexpr (!MT::kSplitP || V) {
-      if (best == kRows256) return launch_split<MT, V, D, 1, 8>(a, stream);
+      if (best == kRows256) return launch_split<MT, V, D, 1, 8>(a, queries, stream);
     }
-    return launch_split<MT, V, D, 1, 4>(a, stream);
+    return launch_split<MT, V, D, 1, 4>(a, queries, stream);
   };
   if constexpr (V16)
     if (best_v) return launch(std::true_type{});
@@ -1477,9 +1495,9 @@ int launch_cheapest(const PrefillArgs &a, int by_size, hipStream_t stream) {
 // V16 (bf16 only): the launches of one key group hand V to the matrix cores as fp16 (base_policy above). The rules by size of
 // this function hold where the sizes fill whole tiles and rounds; launch_cheapest looks at the others.
 template <typename MT, int D, bool V16>
-int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
+int launch_for_d(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream) {
   static_assert(!V16 || MT::kSplitP, "V16 is a form of the bf16 kernels");
-  const auto launch = [&](int by_size) { return launch_cheapest<MT, D, V16>(a, by_size, stream); };
+  const auto launch = [&](int by_size) { return launch_cheapest<MT, D, V16>(a, queries, by_size, stream); };
   // With fewer than two 128-row workgroups per CU the launch is bound by how long one workgroup
   // takes to walk its keys, not by the matrix pipes: split the keys of a tile between wave pairs.
   // Measured on 256 CUs: at exactly two per CU the split still wins for causal launches (41.8 vs
@@ -1497,13 +1515,13 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
 #ifndef LMH_NO_PAIR_KERNEL  // (measurement builds can keep these launches on the kernels below, for comparisons with them)
   if constexpr (D <= 96 && !MT::kSplitP) {
     const int64_t wgs_pair = (int64_t)a.B * a.Hq * (((a.Sq + 255) / 256 + 1) / 2);
-    if (a.causal && a.Sq > 256 && wgs_pair <= n_cus && 16 * wgs_pair >= 15 * n_cus) return launch_pair<MT, D>(a, stream);
+    if (a.causal && a.Sq > 256 && wgs_pair <= n_cus && 16 * wgs_pair >= 15 * n_cus) return launch_pair<MT, D>(a, queries, stream);
     // Without a mask the same kernel takes two neighbouring tiles (512 rows, every fragment read shared all the way);
     // its workgroups are equal, so it wants whole rounds: B=1 H=32 S=4096 D=96 (one round) -5.9 %, S=8192 (two) -3.5 %,
     // B=4 (four) -1.1 %; D=64 one round -2.4 %, two rounds +2.5 %; 1.25 rounds +20 %.
     if (!a.causal && a.Sq > 256) {
       const int64_t rounds = (wgs_pair + n_cus - 1) / n_cus, last = wgs_pair - (rounds - 1) * n_cus;
-      if (16 * last >= 15 * n_cus && (rounds == 1 || (D > 64 && rounds <= 2))) return launch_pair<MT, D>(a, stream);
+      if (16 * last >= 15 * n_cus && (rounds == 1 || (D > 64 && rounds <= 2))) return launch_pair<MT, D>(a, queries, stream);
     }
   }
 #endif
@@ -1565,7 +1583,7 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
 // bf16 keeps head + remainder weights at every length: the registers of the fp16 rewrite of V spill here (S=4096: 633 us).
 // The head dims that are odd multiples of 8 stay on the vector-ALU kernel.
 template <typename MT, int D>
-int launch_wide_heads(const PrefillArgs &a, hipStream_t stream) {
+int launch_wide_heads(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream) {
   const int64_t heads = (int64_t)a.B * a.Hq, cus = device_cu_count();
   const int64_t row_tiles = (a.Sk + BN - 1) / BN;  // key tiles of a whole row
   auto steps = [&](int rows) -> double {           // key tiles the busiest CU walks in workgroups of `rows` query rows
@@ -1577,13 +1595,13 @@ int launch_wide_heads(const PrefillArgs &a, hipStream_t stream) {
   };
   const double s64 = steps(64), s128 = steps(128);
   const bool even_wins = !MT::kSplitP && s128 >= 12;
-  if (s128 > 0.9 * s64 && !even_wins) return launch_split<MT, false, D, 2, 4>(a, stream);
-  if (row_tiles <= (a.causal ? 5 : 4)) return launch_split<MT, false, D, 1, 4>(a, stream);
-  return launch_split<MT, false, D, 2, 8, 2>(a, stream);
+  if (s128 > 0.9 * s64 && !even_wins) return launch_split<MT, false, D, 2, 4>(a, queries, stream);
+  if (row_tiles <= (a.causal ? 5 : 4)) return launch_split<MT, false, D, 1, 4>(a, queries, stream);
+  return launch_split<MT, false, D, 2, 8, 2>(a, queries, stream);
 }
 
 template <typename MT>
-int launch_for_type(const PrefillArgs &a, hipStream_t stream) {
+int launch_for_type(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream) {
   if (a.D > 256) return fail(LMH_E_UNSUPPORTED, "MFMA flash attention: head dim %d not tiled", a.D);
 #ifndef LMH_BF16_SPLIT_P
   if constexpr (MT::kSplitP) {
@@ -1594,18 +1612,18 @@ int launch_for_type(const PrefillArgs &a, hipStream_t stream) {
     // D = 96 tiling, one workgroup per CU in this form, is the one that ties or loses at 512 keys per row: 1024 there.)
     const int64_t keys_per_row = a.causal ? (a.Sq < a.Sk ? a.Sq : a.Sk) / 2 : a.Sk;
     if (a.D <= 128 && keys_per_row >= (a.D > 64 && a.D <= 96 ? 1024 : 512)) {
-      if (a.D <= 64) return launch_for_d<MT, 64, true>(a, stream);
-      if (a.D <= 96) return launch_for_d<MT, 96, true>(a, stream);
-      return launch_for_d<MT, 128, true>(a, stream);
+      if (a.D <= 64) return launch_for_d<MT, 64, true>(a, queries, stream);
+      if (a.D <= 96) return launch_for_d<MT, 96, true>(a, queries, stream);
+      return launch_for_d<MT, 128, true>(a, queries, stream);
     }
   }
 #endif
   // the smallest tiling that holds the head dim; the padding costs its share of the MFMAs
-  if (a.D <= 64) return launch_for_d<MT, 64, false>(a, stream);
-  if (a.D <= 96) return launch_for_d<MT, 96, false>(a, stream);
-  if (a.D <= 128) return launch_for_d<MT, 128, false>(a, stream);
-  if (a.D <= 192) return launch_wide_heads<MT, 192>(a, stream);
-  return launch_wide_heads<MT, 256>(a, stream);
+  if (a.D <= 64) return launch_for_d<MT, 64, false>(a, queries, stream);
+  if (a.D <= 96) return launch_for_d<MT, 96, false>(a, queries, stream);
+  if (a.D <= 128) return launch_for_d<MT, 128, false>(a, queries, stream);
+  if (a.D <= 192) return launch_wide_heads<MT, 192>(a, queries, stream);
+  return launch_wide_heads<MT, 256>(a, queries, stream);
 }
 
 }  // namespace
@@ -1614,12 +1632,12 @@ bool prefill_mfma_supported(int dtype, int D) {
   return (dtype == LMH_F16 || dtype == LMH_BF16) && D >= 8 && (D <= 128 ? D % 8 == 0 : D <= 256 && D % 16 == 0);
 }
 
-int launch_prefill_mfma(const PrefillArgs &a, int dtype, hipStream_t stream) {
+int launch_prefill_mfma(const PrefillArgs &a, int dtype, hipStream_t stream, const QueryCopy &queries) {
 #ifdef LMH_W64_KERNEL
   if (prefill_w64_takes(a, dtype)) return launch_prefill_w64(a, stream);
 #endif
-  if (dtype == LMH_F16) return launch_for_type<MfmaF16>(a, stream);
-  if (dtype == LMH_BF16) return launch_for_type<MfmaBF16>(a, stream);
+  if (dtype == LMH_F16) return launch_for_type<MfmaF16>(a, queries, stream);
+  if (dtype == LMH_BF16) return launch_for_type<MfmaBF16>(a, queries, stream);
   return fail(LMH_E_UNSUPPORTED, "MFMA flash attention: dtype %d has no matrix-core path", dtype);
 }
 

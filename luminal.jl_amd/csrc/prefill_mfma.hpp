@@ -3,6 +3,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "copy.hpp"
 #include "dtypes.hpp"
 
 namespace lmh {

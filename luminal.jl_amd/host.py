@@ -955,6 +955,12 @@ def _prepare_decode_step(op, out, inputs, workspaces=None):
         binding.decode_step(p, x)
         return result
 
+    def fed(*copies):
+        p.workspace, p.workspace_bytes = pool.get(need, q.device)
+        p.stream = None
+        binding.decode_step_fed(p, x, *copies)
+
+    launch.fed = fed
     return launch
 
 
@@ -1103,7 +1109,28 @@ def _prepare(op, out, inputs, workspaces):
         p.stream = stream
         call(p)
 
+    launch.op, launch.params = op, p
     return launch
+
+
+def _fed_start(steps):
+    """(number of steps, call) for a graph that begins with a decode step or a cache append: `call` of the inputs' copies makes
+    these and runs the steps. (A copy in front of such steps is a launch as long as theirs.) (0, None) for others."""
+    if steps and hasattr(steps[0], "fed"):
+        return 1, steps[0].fed
+    ops = [getattr(step, "op", None) for step in steps[:2]]
+    if not ops or not isinstance(ops[0], KVAppendOp):
+        return 0, None
+    append = steps[0].params
+    attn = steps[1].params if len(ops) > 1 and isinstance(ops[1], FlashAttentionOp) else None
+
+    def fed(*copies):
+        append.stream = None
+        if attn is not None:
+            attn.stream = None
+        binding.kv_append_fed(append, attn, *copies)
+
+    return 1 if attn is None else 2, fed
 
 
 def execute_op(op, *inputs):
@@ -1319,9 +1346,10 @@ class CompiledGraph:
         self.cache = {}
         self.use_capture = False
         self._copies = None  # of the last call's nodes
+        self._fed_steps, self._fed = _fed_start(steps)
 
-    def _run(self, stream):
-        for step in self.steps:
+    def _run(self, stream, first=0):
+        for step in self.steps[first:]:
             step(stream)
         if self.asked:
             for i in reversed(range(len(self.asked))):  # a step holds its operands, which earlier ones make
@@ -1337,15 +1365,20 @@ class CompiledGraph:
         arrays = inputs.values()
         # one launch copies them all; a kernel does not reach into another GPU's memory without the peer access that the
         # runtime's copy arranges for itself
+        first = 0  # step that is still to run
         if all(isinstance(v, HipArray) and v.device.index == copies.device for v in arrays):
-            copies.launch(arrays)
+            if self._fed and nodes and not self.use_capture:
+                copies.launch(arrays, self._fed)
+                first = self._fed_steps
+            else:
+                copies.launch(arrays)
         else:
             for k, v in inputs.items():
                 self._copy_one(k, v)
         if self.use_capture:
             execute_with_capture(self.device, self._run, self.cache)
         else:
-            self._run(None)
+            self._run(None, first)
             self.cache["hip_warm"] = True
         return self.results
 

@@ -445,9 +445,10 @@ class InputCopies:
         self.nbytes = (ctypes.c_size_t * n)(*self.lengths)
         self.sources = ctypes.c_void_p * n
 
-    def launch(self, arrays):
+    def launch(self, arrays, call=None):
+        """lmh_copy_many, or another `call` of destinations, sources, sizes and their number."""
         src = self.sources(*[a.ptr for a in arrays])
         if [a.nbytes for a in arrays] != self.lengths:
             raise ValueError("Input length mismatch for node %d" %
                              next(i for i, a, n in zip(self.nodes, arrays, self.lengths) if a.nbytes != n))
-        binding.copy_many(self.dst, src, self.nbytes, len(self.nodes))
+        (call or binding.copy_many)(self.dst, src, self.nbytes, len(self.nodes))

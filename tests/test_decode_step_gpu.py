@@ -148,3 +148,59 @@ def test_decode_step_refuses_what_it_cannot_take(lm, hip, oracle):
     tpos, tlen = lm.tensor(g, (B,), "i32"), lm.tensor(g, (B,), "i32")
     out, _, _ = lm.cached_self_attention_core(tq, tkn, tvn, tkc, tvc, tpos, tlen, rope_base=10000.0, fused=True)
     assert isinstance(g.nodes[out.id].op, lm.DecodeAttentionOp)
+
+
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,T,L,D,rope", [
+    ("bf16", 1, 4, 4, 1, 64, 64, True), ("f16", 5, 32, 2, 1, 700, 128, True), ("f16", 2, 12, 4, 1, 300, 96, True),  # steps; the last in two nodes
+    ("f32", 3, 6, 2, 1, 130, 64, True),  # ... that rotates the queries in place
+    ("f16", 2, 8, 2, 33, 64, 128, True), ("bf16", 1, 6, 3, 777, 800, 64, True), ("f16", 1, 8, 2, 300, 333, 256, False),  # prompts
+    ("f16", 3, 16, 16, 513, 600, 96, True), ("bf16", 2, 4, 1, 130, 200, 80, False), ("f16", 2, 4, 4, 16, 40, 80, True),
+    ("f32", 2, 4, 2, 257, 300, 64, False)])
+def test_operands_taken_from_the_callers_arrays(lm, hip, dtype, B, Hq, Hkv, T, L, D, rope):
+    """A call of a compiled graph leaves the same memory behind whether its inputs are copied in front of the launches or read
+    where they lie: the result, the caches and the graph's copies of the inputs, bit for bit. Also with inputs that rule
+    the second out (a misaligned array, the graph's own result or cache as input) and with some left out."""
+    g = lm.Graph()
+    tq, tkn, tvn = lm.tensor(g, (B, Hq, T, D), dtype), lm.tensor(g, (B, Hkv, T, D), dtype), lm.tensor(g, (B, Hkv, T, D), dtype)
+    tkc, tvc = lm.tensor(g, (B, Hkv, L, D), dtype), lm.tensor(g, (B, Hkv, L, D), dtype)
+    tpos, tlen = lm.tensor(g, (B,), "i32"), lm.tensor(g, (B,), "i32")
+    core = lm.prompt_self_attention_core if T > 1 else lm.cached_self_attention_core
+    out = core(tq, tkn, tvn, tkc, tvc, tpos, tlen, rope_base=10000.0 if rope else None, **({} if T > 1 else {"fused": True}))[0]
+    fed, plain = lm.compile(g, hip), lm.compile(g, hip)
+    assert fed._fed is not None
+    plain._fed = None
+    rng = np.random.default_rng(16800)
+
+    def array(t, skip=0):
+        values = rng.standard_normal(t.shape).astype(np.float32)
+        whole = lm.to_device(np.concatenate([np.zeros(skip, np.float32), values.reshape(-1)]), hip, dtype)
+        part = whole.view(whole.shape)
+        part.shape, part.nbytes = t.shape, whole.nbytes - skip * whole.nbytes // whole.size
+        part.ptr += whole.nbytes - part.nbytes
+        return part
+
+    def result(cg):
+        r = cg.results[out.id]
+        return r[0] if isinstance(r, tuple) else r
+
+    def call(feeds):
+        for cg in (fed, plain):
+            cg({k: v(cg) if callable(v) else v for k, v in feeds.items()})
+        lm.binding.sync()
+        for t in (tq, tkn, tvn, tkc, tvc, tpos, tlen):
+            np.testing.assert_array_equal(fed.results[t.id].to_host_raw(), plain.results[t.id].to_host_raw())
+        got = result(fed).to_host()
+        np.testing.assert_array_equal(got, result(plain).to_host())
+        assert np.isfinite(got).all() and np.abs(got).max() > 0
+
+    pos = rng.integers(0, L, B) if T == 1 else np.zeros(B)
+    at = {tpos.id: lm.to_device(pos.astype(np.int32), hip), tlen.id: lm.to_device(pos.astype(np.int32) + T, hip)}
+    call({tq.id: array(tq), tkn.id: array(tkn), tvn.id: array(tvn), **at})
+    call({tvn.id: array(tvn), tq.id: array(tq)})
+    call({tkn.id: array(tkn, 1), tvn.id: array(tvn), tq.id: array(tq, 3), **at})
+    same = array(tkn)
+    call({tkn.id: same, tvn.id: same, tq.id: lambda cg: result(cg).view(tq.shape)})
+    call({tkc.id: array(tkc), tvn.id: array(tvn), tkn.id: lambda cg: cg.results[tvn.id]})
+    if Hq * T <= Hkv * L:
+        inside = lambda cg: (lambda v: (setattr(v, "shape", tq.shape), setattr(v, "nbytes", cg.results[tq.id].nbytes), v)[2])(cg.results[tvc.id].view(tvc.shape))
+        call({tq.id: inside, tkn.id: array(tkn)})
