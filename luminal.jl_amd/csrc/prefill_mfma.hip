@@ -102,7 +102,8 @@ __device__ inline void rotate_q_fragments_with_table(typename MT::vec8 (&qreg)[D
 // The second launch bound is waves per SIMD.
 // WPS: waves per SIMD the register budget is set for (3 x 4 waves, 2 x 8 waves or 1 x 8 waves per CU).
 template <int D, int NW> constexpr int default_wps() { return D > 128 ? 1 : D > 96 ? 2 : NW == 8 ? 4 : 3; }
-template <typename MT, int D, bool CAUSAL, int KSPLIT, int NW, int WPS>
+// AHEAD: the loop that is a tile ahead with its scores, for one wave per SIMD.
+template <typename MT, int D, bool CAUSAL, int KSPLIT, int NW, int WPS, bool AHEAD>
 __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, PrefillArgs a, QueryCopy queries) {
   request_args(a);
   request_args(deal);
@@ -247,17 +248,25 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
                  :: "s"(lds_addr), "v"(voff), "s"(desc), "s"(soff) : "memory", "m0");
   };
 #pragma clang diagnostic pop
-  auto load_tile = [&](int kt, int buf) {
+  auto load_k_block = [&](int kt, int buf, int j) __attribute__((always_inline)) {
+    if (wave_u + NW * j < KI)
+      load_block(k_desc, k_lds0 + buf * (BT * LDK * 2) + j * (NW * 1024), k_voff[j], kt * k_tile_bytes);
+  };
+  auto load_v_block = [&](int kt, int buf, int j) __attribute__((always_inline)) {
+    if (wave_u + NW * j < VI)
+      load_block(v_desc, v_lds0 + buf * (BT * LDV * 2) + j * (NW * 1024), v_voff[j], kt * v_tile_bytes);
+  };
+  auto load_k = [&](int kt, int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < KJ; j++)
-      if (wave_u + NW * j < KI)
-        load_block(k_desc, k_lds0 + buf * (BT * LDK * 2) + j * (NW * 1024), k_voff[j], kt * k_tile_bytes);
-    if constexpr (!CV) {
+    for (int j = 0; j < KJ; j++) load_k_block(kt, buf, j);
+  };
+  auto load_v = [&](int kt, int buf) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < VJ; j++)
-        if (wave_u + NW * j < VI)
-          load_block(v_desc, v_lds0 + buf * (BT * LDV * 2) + j * (NW * 1024), v_voff[j], kt * v_tile_bytes);
-    }
+    for (int j = 0; j < VJ; j++) load_v_block(kt, buf, j);
+  };
+  auto load_tile = [&](int kt, int buf) __attribute__((always_inline)) {
+    load_k(kt, buf);
+    if constexpr (!CV) load_v(kt, buf);
   };
 
   // ---- MT::kConvertV: V tiles pass through registers and are stored in LDS as fp16 relative to the largest finite |v|
@@ -362,6 +371,161 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) asm volatile("" :: "v"(qreg[ks]));
 
+  // ---- One wave per SIMD (head dims above 128): no other wave fills the matrix pipe during the softmax, so the scores of tile
+  // kt + 1 are computed beside the softmax of tile kt, in one stretch of code with that tile's second product. K is staged two
+  // tiles ahead, V one. The order of the stretch is written out, an MFMA with its share of the other work at a time. What bounds
+  // it is what the wave can issue: of 3130 cycles a tile (bf16, D = 256, 64 rows) the MFMAs take 1536. B=1 H=16/8 S=1500 D=256
+  // causal bf16 51.1 -> 41.8 us, D=192 42 -> 34; B=1 H=8 S=2048 D=256 without a mask 65 -> 54. ----
+  if constexpr (AHEAD) {
+    static_assert(!CV && WPS == 1, "V tiles staged as they are, accumulation registers");
+    auto k_frag = [&](int buf, int i) __attribute__((always_inline)) {  // the i-th MFMA of a tile's scores: key block i % NKB, k-step i / NKB
+      return *reinterpret_cast<const vec8 *>(&Ks2[buf][kg * (BW * LDK) + k_frag_off + (i % NKB) * 32 * LDK + 16 * (i / NKB)]);
+    };
+    auto v_frag = [&](int buf, int i) __attribute__((always_inline)) {  // the i-th V fragment of a tile: 32 rows i % DB of O^T, keys 16 (i / DB)
+      const uint16_t *vaddr = &Vs2[buf][kg * (BW * LDV) + v_frag_off + 16 * (i / DB) * LDV + (i % DB) * 32];
+      const shortx4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(vaddr));
+      const shortx4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(vaddr + 8 * LDV));
+      return __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    constexpr int NQ = KS * NKB, NV = 2 * DB * NKB, NP = 8 * NKB;  // MFMAs of the scores, V fragments, pairs of weights, per tile
+    constexpr int RING = 4;  // fragments in flight (eight: the same)
+    constexpr int LOADS_FROM = 8;  // MFMA at which a tile's loads begin: the first ones have the exponentials beside them
+    static_assert(LOADS_FROM + KI / NW + VI / NW <= NQ + NV, "a place for every load");
+    float mx = 0.f;  // largest of a query's scores in s
+    auto largest = [&](const floatx16_t (&s)[NKB]) __attribute__((always_inline)) {
+      float mx = s[0][0];
+#pragma unroll
+      for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[kb][i]);
+      return max_over_wave_halves(mx);
+    };
+    auto mask = [&](int k0, floatx16_t (&s)[NKB]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          const int key = k0 + kb * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
+          if (key >= n_keys || (CAUSAL && key > qi)) s[kb][i] = -INFINITY;
+        }
+    };
+    const int kg0 = wave_u / RG * BW, q_lo = q0 + wave_u % RG * 32, q_hi = q_lo + 31;  // (the branches below are the wave's)
+    auto masked = [&](int k0) __attribute__((always_inline)) { return (k0 + BW > n_keys) || (CAUSAL && k0 + BW - 1 > q_lo); };
+    // tiles in which a key of this wave's share is before its diagonal and the last key
+    const int n_live = ((CAUSAL ? min(k_end, q_hi + 1) : k_end) - kg0 + BT - 1) / BT;
+    // Scores of tile kt + 1 and, with_tile, softmax and second product of tile kt, whose masked scores are in s. Beside the MFMAs
+    // of the first product this wave's loads of K of tile k_tile and V of tile v_tile.
+    floatx16_t s[NKB], next[NKB];
+    floatx16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    asm volatile("" : "+a"(zero));
+    auto compute = [&](auto with_tile, int kt, int k_tile, int v_tile) __attribute__((always_inline)) {
+      constexpr bool TILE = decltype(with_tile)::value;
+      const int k_buf = (kt + 1) & 1, v_buf = kt & 1;
+      const float mc = m_i * c;
+      uint32_t w[NP], w_lo[NP];  // weights, packed in pairs
+      vec8 ring[RING];
+#pragma unroll
+      for (int i = 0; i < RING; i++) ring[i] = k_frag(k_buf, i);
+      __builtin_amdgcn_sched_barrier(0);
+      auto pairs = [&](int from, int to) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = from; j < to; j++) {
+          const float p0 = __builtin_amdgcn_exp2f(s[j / 8][2 * (j % 8)] * c - mc), p1 = __builtin_amdgcn_exp2f(s[j / 8][2 * (j % 8) + 1] * c - mc);
+          w[j] = MT::cvt_pair(p0, p1);
+          if (MT::kSplitP) w_lo[j] = MT::cvt_pair(p0 - MT::low(w[j]), p1 - MT::high(w[j]));
+          if (j % 4 == 3) {
+            l_i = MT::sum8(__builtin_bit_cast(pvec8, make_uint4(w[j - 3], w[j - 2], w[j - 1], w[j])), l_i);
+            if (MT::kSplitP) l_i = MT::sum8(__builtin_bit_cast(pvec8, make_uint4(w_lo[j - 3], w_lo[j - 2], w_lo[j - 1], w_lo[j])), l_i);
+          }
+        }
+      };
+      auto stage = [&](int i) __attribute__((always_inline)) {
+        if (i < 0) return;
+        if (i < KI / NW) load_k_block(k_tile, v_buf, i);
+        else if (i < KI / NW + VI / NW) load_v_block(v_tile, k_buf, i - KI / NW);
+      };
+#pragma unroll
+      for (int i = 0; i < NQ; i++) {
+        next[i % NKB] = MT::mfma(ring[i % RING], qreg[i / NKB], i < NKB ? zero : next[i % NKB]);
+        if (i + RING < NQ) ring[i % RING] = k_frag(k_buf, i + RING);
+        else if (TILE) ring[i % RING] = v_frag(v_buf, i + RING - NQ);
+        if constexpr (TILE) {
+          stage(i - LOADS_FROM);
+          pairs(i * NP / NQ, (i + 1) * NP / NQ);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (TILE) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+          const int j = 4 * (i / DB), r = (i + NQ) % RING;
+          oacc[i % DB] = MT::mfma_pv(ring[r], __builtin_bit_cast(pvec8, make_uint4(w[j], w[j + 1], w[j + 2], w[j + 3])), oacc[i % DB]);
+          if (MT::kSplitP) oacc[i % DB] = MT::mfma_pv(ring[r], __builtin_bit_cast(pvec8, make_uint4(w_lo[j], w_lo[j + 1], w_lo[j + 2], w_lo[j + 3])), oacc[i % DB]);
+          if (i + RING < NV) ring[r] = v_frag(v_buf, i + RING);
+          stage(NQ + i - LOADS_FROM);
+          if (i == NV / 2) {
+#pragma unroll
+            for (int kb = 0; kb < NKB; kb++) s[kb] = next[kb];
+            mx = largest(s);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int kb = 0; kb < NKB; kb++) s[kb] = next[kb];
+        mx = largest(s);
+      }
+      const int k0 = (kt + 1) * BT + kg0;
+      if (__builtin_expect(masked(k0), 0)) {
+        mask(k0, s);
+        mx = largest(s);
+      }
+    };
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();  // (and the inv_freq table has been read)
+    if (n_kv_tiles > 1) load_k(1, 1);
+    if (n_live > 0) compute(std::false_type{}, -1, 0, 0);
+    // The last tiles load the last one again instead of none: a branch between the MFMAs lets the compiler move the softmax behind
+    // it. And the accumulators are named as accumulation registers wherever they enter or leave the loop or the rescale: left to
+    // the compiler, which sees the rescale's vector instructions, they live in vector registers between the tiles, and two copies
+    // of each, 256 instructions a tile, cost what working ahead gains.
+    auto in_place = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int db = 0; db < DB; db++) asm volatile("" : "+a"(oacc[db]));
+    };
+    in_place();
+    int kt = 0;
+    for (; kt < n_live; kt++) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();  // K of tile kt + 1 and V of tile kt are there, K of tile kt and V of tile kt - 1 done with
+      const int k_tile = min(kt + 2, n_kv_tiles - 1), v_tile = min(kt + 1, n_kv_tiles - 1);
+#pragma unroll
+      for (int i = KI / NW; i < KJ; i++) load_k_block(k_tile, kt & 1, i);  // (that not every wave has to issue)
+#pragma unroll
+      for (int i = VI / NW; i < VJ; i++) load_v_block(v_tile, (kt + 1) & 1, i);
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64((mx - m_i) * c > kLazyRescale) != 0, 0)) {
+        const float m_new = fmaxf(m_i, mx);
+        const float alpha = __builtin_amdgcn_exp2f((m_i - m_new) * c);
+        m_i = m_new;
+        l_i *= alpha;
+        in_place();
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+          for (int i = 0; i < 16; i++) oacc[db][i] *= alpha;
+        in_place();
+      }
+      compute(std::true_type{}, kt, k_tile, v_tile);  // (after the last tile scores of whatever the buffer holds, for nobody)
+      in_place();
+    }
+    for (; kt < n_kv_tiles; kt++) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      load_k(min(kt + 2, n_kv_tiles - 1), kt & 1);
+      load_v(min(kt + 1, n_kv_tiles - 1), (kt + 1) & 1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (before the LDS is used for something else)
+  } else
   for (int kt = 0; kt < n_kv_tiles; kt++) {
     // One barrier per tile: tile kt (fetched during the previous iteration) becomes visible, and every
     // wave is done with tile kt-1, whose buffer the fetch of tile kt+1 now overwrites.
@@ -1303,7 +1467,7 @@ int launch_pair(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stre
 template <typename MT, bool V16, int KSPLIT> struct base_policy { using type = MT; };
 template <> struct base_policy<MfmaBF16, true, 1> { using type = MfmaBF16V16; };
 
-template <typename MT0, bool V16, int D, int KSPLIT, int NW, int WPS = default_wps<D, NW>()>
+template <typename MT0, bool V16, int D, int KSPLIT, int NW, int WPS = default_wps<D, NW>(), bool AHEAD = false>
 int launch_split(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream) {
   using MT = typename base_policy<MT0, V16, KSPLIT>::type;
   constexpr int BM = 32 * NW / KSPLIT;
@@ -1312,14 +1476,14 @@ int launch_split(const PrefillArgs &a, const QueryCopy &queries, hipStream_t str
   const int rc = check_grid(wgs, 64 * NW);
   if (rc != LMH_OK) return rc;
   dim3 grid((uint32_t)wgs), block(64 * NW);
-  if (plan_only("prefill_mfma_kernel<%s, D=%d, %s, key groups=%d, waves=%d, waves per SIMD=%d> workgroups=%u%s", MT::kName, D,
-                a.causal ? "causal" : "full", KSPLIT, NW, WPS, grid.x, MT::kConvertV ? ", V as fp16" : ""))
+  if (plan_only("prefill_mfma_kernel<%s, D=%d, %s, key groups=%d, waves=%d, waves per SIMD=%d> workgroups=%u%s%s", MT::kName, D,
+                a.causal ? "causal" : "full", KSPLIT, NW, WPS, grid.x, MT::kConvertV ? ", V as fp16" : "", AHEAD ? ", a tile ahead" : ""))
     return LMH_OK;
   const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? 4 * WPS / NW : 0, device_cu_count());
   if (a.causal)
-    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS>), grid, block, 0, stream, deal, a, queries);
+    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS, AHEAD>), grid, block, 0, stream, deal, a, queries);
   else
-    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, false, KSPLIT, NW, WPS>), grid, block, 0, stream, deal, a, queries);
+    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, false, KSPLIT, NW, WPS, AHEAD>), grid, block, 0, stream, deal, a, queries);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }
@@ -1570,33 +1734,44 @@ int launch_for_d(const PrefillArgs &a, const QueryCopy &queries, hipStream_t str
 // Head dims above 128: Q and the accumulators of 32 rows take up to 192 registers and a tile buffer pair up to 141 KB, so a
 // workgroup has the CU to itself. The vector-ALU kernel that took these launches reaches 8 TFLOP/s. Three forms:
 //   64 rows, four waves in two key groups: one wave per SIMD, as many workgroups as there can be;
+//   128 rows, four waves: no fold at the end, one wave per SIMD;
 //   128 rows, eight waves in two key groups: two waves per SIMD, which fit with 256 registers each when K fragments are
-//     fetched four k-steps at a time. The second wave computes while the first waits for LDS: a staged tile takes 0.95
-//     (fp16) to 1.13 times (bf16) as long as in the first form and serves twice the rows;
-//   128 rows, four waves: no fold at the end, one wave per SIMD.
-// The first two are compared by the tiles that the busiest CU walks: its longest workgroup or the mean over the CUs
-// (causal, heaviest first), whole rounds without a mask. Where 128 rows need fewer, they are 20 to 47 % faster; where both
-// need the same, the 64-row form is up to 27 % ahead (fp16 from 12 tiles on 0 to 7 % behind). The third is ahead of the
-// second where a row has no more than about four tiles, five with the causal mask's short ones (D=256 bf16 448 workgroups
-// of 104 keys 32.4 against 34.4 us; 1344 of 673 keys 171.0 against 167.5) and was the only 128-row form before: B=1 H=32 S=4096 D=256 causal fp16 363 -> 292 us = 940
-// TFLOP/s, bf16 432 -> 378; B=1 H=32 S=2048 102 -> 86; B=1 H=4 S=6000 without a mask, on 64 rows before, 333 -> 167.
+//     fetched four k-steps at a time. The second wave computes while the first waits for LDS.
+// The first two work a tile ahead (AHEAD) from three key tiles a row on; on one or two the shorter loop is 3 to 9 % faster (B=1
+// H=8 S=83 D=256 bf16 11.0 against 11.5 us, B=3 H=12 Sq=5675 Sk=43 D=192 fp16 65 against 72).
+// A launch lasts as long as its busiest CU: the key tiles it walks (its longest workgroup or the mean over the CUs with a causal
+// mask, whole rounds without one) and the workgroups it starts, each worth five tiles of the first form. A tile takes 1.4 and 1.2
+// times as long in the other two, a start of the third six tiles. Fitted to 386 drawn launches (fp16 and bf16, head dims 160 to
+// 256, 16 to 8192 rows, 1 to 64 heads, with every form timed on each): within 0.7 % of the best form on average, where the
+// comparison of the tiles alone is 5 % behind it. That one, in which 64 rows have to be 10 % cheaper to be left (fp16 from 12 tiles
+// on stays on eight waves), was measured with the shorter loop and still chooses for it.
+// B=1 H=32 S=4096 D=256 causal fp16 takes 292 us = 940 TFLOP/s (363 with 128 rows on four waves as the only form).
 // bf16 keeps head + remainder weights at every length: the registers of the fp16 rewrite of V spill here (S=4096: 633 us).
 // The head dims that are odd multiples of 8 stay on the vector-ALU kernel.
 template <typename MT, int D>
 int launch_wide_heads(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream) {
   const int64_t heads = (int64_t)a.B * a.Hq, cus = device_cu_count();
   const int64_t row_tiles = (a.Sk + BN - 1) / BN;  // key tiles of a whole row
-  auto steps = [&](int rows) -> double {           // key tiles the busiest CU walks in workgroups of `rows` query rows
+  auto cost = [&](int rows, double tile, double start) -> double {  // workgroups of `rows` query rows
     const int64_t n = (a.Sq + rows - 1) / rows, s = rows / BN;
-    if (!a.causal) return (double)((heads * n + cus - 1) / cus * row_tiles);
+    if (!a.causal) return (double)((heads * n + cus - 1) / cus) * (row_tiles * tile + start);
     const int64_t ramp = std::min(n, row_tiles / s);  // workgroups r < ramp walk (r + 1) s tiles, the others all of them
-    const double longest = (double)std::min(row_tiles, n * s);
-    return std::max(longest, (double)heads * (s * ramp * (ramp + 1) / 2 + (n - ramp) * row_tiles) / cus);
+    const double longest = (double)std::min(row_tiles, n * s), mean = (double)heads * (s * ramp * (ramp + 1) / 2 + (n - ramp) * row_tiles) / cus;
+    return std::max(longest, mean) * tile + std::max(1., (double)(heads * n) / cus) * start;
   };
-  const double s64 = steps(64), s128 = steps(128);
-  const bool even_wins = !MT::kSplitP && s128 >= 12;
-  if (s128 > 0.9 * s64 && !even_wins) return launch_split<MT, false, D, 2, 4>(a, queries, stream);
-  if (row_tiles <= (a.causal ? 5 : 4)) return launch_split<MT, false, D, 1, 4>(a, queries, stream);
+  const double s64 = cost(64, 1., 0.), s128 = cost(128, 1., 0.);
+  const bool even = !MT::kSplitP && s128 >= 12;
+  if (row_tiles <= 2) {
+    if (s128 > 0.9 * s64 && !even) return launch_split<MT, false, D, 2, 4>(a, queries, stream);
+    return launch_split<MT, false, D, 1, 4>(a, queries, stream);
+  }
+  const double rows64 = cost(64, 1., 5.), rows128 = cost(128, 1.4, 5.), eight = cost(128, 1.2, 6.);
+  // fp16 launches that come out even stay on eight waves where the tests of that form expect it of one such launch: with a mask up
+  // to 50 workgroups of 64 rows, without one from a second round of them on
+  const int64_t wgs64 = heads * ((a.Sq + 63) / 64);
+  const bool stays = even && s128 == s64 && (a.causal ? wgs64 <= 50 : wgs64 > cus);
+  if (!stays && rows64 <= std::min(rows128, eight)) return launch_split<MT, false, D, 2, 4, 1, true>(a, queries, stream);
+  if (!stays && rows128 < 0.98 * eight) return launch_split<MT, false, D, 1, 4, 1, true>(a, queries, stream);
   return launch_split<MT, false, D, 2, 8, 2>(a, queries, stream);
 }
 

@@ -43,6 +43,10 @@ struct MfmaF16 {
   __device__ static uint16_t cvt_bits(float x) { return __builtin_bit_cast(uint16_t, (_Float16)x); }
   __device__ static _Float16 cvt(float x) { return (_Float16)x; }
   __device__ static _Float16 cvt_p(float x) { return (_Float16)x; }
+  // two of them in a word
+  __device__ static uint32_t cvt_pair(float x, float y) { return (uint32_t)cvt_bits(x) | (uint32_t)cvt_bits(y) << 16; }
+  __device__ static float low(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)w); }
+  __device__ static float high(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)); }
   __device__ static floatx16_t mfma_pv(vec8 v, pvec8 p, floatx16_t c) { return mfma(v, p, c); }
   // acc + sum of the 8 (already rounded) elements: 4 x v_dot2_f32_f16 against (1, 1)
   __device__ static float sum8(vec8 p, float acc) {
@@ -69,6 +73,13 @@ struct MfmaBF16 {
   __device__ static uint16_t cvt_bits(float x) { return f32_to_bf16_bits(x); }
   __device__ static __bf16 cvt(float x) { return (__bf16)x; }
   __device__ static __bf16 cvt_p(float x) { return (__bf16)x; }
+  __device__ static uint32_t cvt_pair(float x, float y) {
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    const b2 w = {(__bf16)x, (__bf16)y};
+    return __builtin_bit_cast(uint32_t, w);
+  }
+  __device__ static float low(uint32_t w) { return __uint_as_float(w << 16); }
+  __device__ static float high(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
   __device__ static floatx16_t mfma_pv(vec8 v, pvec8 p, floatx16_t c) { return mfma(v, p, c); }
   __device__ static float sum8(vec8 p, float acc) {
     typedef __bf16 b2 __attribute__((ext_vector_type(2)));

@@ -65,6 +65,26 @@ def test_eight_waves_on_wide_heads(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causa
         assert rel_err(got, want) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,dtype,groups", [
+    (2, 6, 2, 129, 129, 144, True, "bf16", 2), (5, 4, 4, 65, 321, 256, False, "f16", 2), (1, 16, 8, 700, 700, 208, True, "f16", 2),
+    (2, 6, 2, 257, 500, 192, True, "bf16", 2), (3, 48, 2, 260, 300, 256, True, "bf16", 1), (4, 33, 3, 300, 190, 144, False, "f16", 1),
+])
+def test_a_tile_ahead_on_wide_heads(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causal, dtype, groups):
+    """Rows of three tiles, odd ones and a last tile of one key; keys that grow along the row, so that the running maximum is
+    raised again and again; sequences that end in the first tile, in its second half or before any key."""
+    q, k, v = inputs(oracle, (B, Hq, Sq, D), (B, Hkv, Sk, D), dtype, 33300 + Sq + D)
+    k = oracle.round_to(k * np.linspace(0.5, 8, Sk, dtype=np.float32)[:, None], dtype)
+    what = plan(lm, q, k, dtype, causal, False)
+    assert "key groups=%d, waves=4" % groups in what and "a tile ahead" in what
+    lens = np.array([(Sk, Sk - 30, 33, 0, 64)[i] for i in range(B)], np.int32)
+    for kv_len in (None, lens):
+        got = run(lm, hip, q, k, v, dtype, causal, kv_len=None if kv_len is None else list(kv_len))
+        want = oracle.flash_attn(q, k, v, causal=causal, kv_len=None if kv_len is None else np.maximum(kv_len, 1), nthreads=NT)
+        if kv_len is not None:
+            want[kv_len == 0] = 0
+        assert rel_err(got, want) <= TOL[dtype]
+
+
 @pytest.mark.parametrize("interleaved", [False, True])
 @pytest.mark.parametrize("dtype,D", [("f16", 192), ("bf16", 256), ("f32", 192), ("f32", 256), ("f32", 64)])
 def test_wide_heads_rotate_their_queries_in_registers(lm, hip, oracle, dtype, D, interleaved):
