@@ -284,7 +284,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(Matmul
 //
 // Bound: the vector ALUs beside the matrix pipe. Splitting takes 5.5 instructions an element, 5.5 a MFMA at 64 x 128 and 7.3 at
 // 64 x 64, where the chip holds 1590 TFLOP/s of bare MFMAs and 1280 with six vector instructions each. So:
-//   * a wave multiplies blocks as large as its registers hold (MB x NB of 32 x 32: 64 rows with 64 or 128 columns), and the four
+//   * a wave multiplies blocks as large as its registers hold (MB x NB of 32 x 32, up to nine or eight), and the four
 //     waves of a workgroup each take all of its tile for every fourth 16 elements of the contraction; the shares are folded
 //     through LDS at the end;
 //   * a wave fetches its own operands and shares nothing until then, so there is no barrier in the loop: buffer loads write fp32
@@ -444,7 +444,8 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args) {
 
   // ---- fold the shares: each wave takes MB NB / WK blocks (or a part of one), and looks whether their sums are finite ----
   constexpr int kRegs = 16 * MB * NB / WK;  // registers a lane of a wave folds
-  static_assert(kRegs % 4 == 0 && (kRegs < 16 ? 16 % kRegs : kRegs % 16) == 0, "quarters of a block, or blocks");
+  constexpr int kPart = kRegs % 16 == 0 ? 16 : kRegs % 8 == 0 ? 8 : 4;  // ... in parts that lie in one block
+  static_assert(kRegs % kPart == 0, "whole parts");
   float sum[kRegs];
   for (int pass = 0;; pass++) {
     if (again) {
@@ -496,11 +497,10 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args) {
     if (pass == 1 || !__syncthreads_or(finite != 0.f || finite != finite)) break;
     again = true;
   }
-  constexpr int kPart = kRegs < 16 ? kRegs : 16;
 #pragma unroll
   for (int r = 0; r < kRegs; r += kPart) {
     const int block = (wk * kRegs + r) / 16;
-    store_block<kPart>(p, sum + r, m0 + 32 * (block / NB) + wk * kRegs % 16 * 2, n0 + 32 * (block % NB) + n, h, batch);
+    store_block<kPart>(p, sum + r, m0 + 32 * (block / NB) + (wk * kRegs + r) % 16 * 2, n0 + 32 * (block % NB) + n, h, batch);
   }
 }
 
@@ -555,10 +555,12 @@ int launch_matmul(MatmulArgs &args, int n, hipStream_t stream) {
   };
   const int64_t r64 = rounds(64, 64);
   const double c64 = 4.0 * r64, c32x64 = 2.2 * rounds(32, 64), c32 = 1.5 * rounds(32, 32);
-  // Split product, us fp32 product -> 64 x 128 / 64 x 64 / 32 x 64: 700 x 2560 x 2048 75 -> 46.5 / 49.6 / 63.4, 700 x 2048 x 2048
-  // 57.8 -> 42.7 / 46.0 / 50.1, 4096^3 1039 -> 754 / 848 / 1073, 1792 x 1280 x 1280 69 -> 60 / 50 / 56, 590 x 1152 x 576 14.0 ->
-  // 16.2 / 10.9 / 11.8, 2048 x 768 x 256 12.7 -> 12.5 / 11.8 / 11.0, 16 x 12288 x 4096 48 -> 68 / 41 / 33. A launch of few tiles
-  // stays with the fp32 product, whose waves share the contraction of smaller blocks (100 x 768 x 768 8.1 -> 18.6 / 12.3 / 9.6).
+  // Split product: fitted to 160 launches of drawn projections (16 to 4000 rows, 256 to 4096 columns and elements, one to three
+  // products, every form timed on each); the choice is 0.8 % from the best form on average (three forms, of 64 x 128, 64 x 64 and
+  // 32 x 64, with constants from nine sizes: 4 %). us fp32 product / 96 x 96 / 64 x 128 / 64 x 96 / 64 x 64 / 32 x 64:
+  // 700 x 2048 x 2048 67 / 44 / 46 / 40 / 47 / 51, 1374 x 1536 x 1536 80 / 42 / 69 / 56 / 56 / 62, 700 x 2560 x 2048 70 / 49 / 48 /
+  // 69 / 49 / 63, 1248 x 1024 x 512 19 / 19 / 17 / 15 / 17 / 16. A launch of few tiles stays with the fp32 product, whose waves
+  // share the contraction of smaller blocks (100 x 768 x 768 8.1 -> 18.6 on 64 x 128, 9.6 on 32 x 64).
   bool vec = true;
   int64_t K = 0;
   for (int i = 0; i < n; i++) {
@@ -567,13 +569,15 @@ int launch_matmul(MatmulArgs &args, int n, hipStream_t stream) {
   }
   if (vec) {
     const double fp32 = 0.95 * (3.3 + 0.0045 * K * std::min(c64, std::min(c32x64, c32)));
-    const double s64x128 = 2.0 + rounds(64, 128) * (6.0 + 0.0205 * K), s64 = 2.5 + r64 * (3.5 + 0.0105 * K);
-    const double s32x64 = 3.0 + rounds(32, 64) * (1.3 + 0.0067 * K);
-    const double split = std::min(s64x128, std::min(s64, s32x64));
+    const double s96 = rounds(96, 96) * (10.0 + 0.0160 * K), s64x128 = rounds(64, 128) * (7.5 + 0.0165 * K);
+    const double s64x96 = rounds(64, 96) * (7.0 + 0.0129 * K), s64 = 2.9 + r64 * (2.6 + 0.0096 * K), s32x64 = 3.7 + rounds(32, 64) * (0.9 + 0.0068 * K);
+    const double split = std::min({s96, s64x128, s64x96, s64, s32x64});
     if (split < fp32) {
       if (split == s64) return launch_split_form<2, 2>(args, n, stream);
+      if (split == s32x64) return launch_split_form<1, 2>(args, n, stream);
+      if (split == s64x96) return launch_split_form<2, 3>(args, n, stream);
       if (split == s64x128) return launch_split_form<2, 4>(args, n, stream);
-      return launch_split_form<1, 2>(args, n, stream);
+      return launch_split_form<3, 3>(args, n, stream);
     }
   }
   if (c64 <= c32x64 && c64 <= c32) {

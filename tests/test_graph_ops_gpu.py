@@ -44,6 +44,14 @@ def test_products_on_pieces_match_float64(lm, hip, oracle, B, S, K, N, heads, dt
     test_projection_matches_float64(lm, hip, oracle, B, S, K, N, heads, dtype, bias)
 
 
+# ... and the tiles of 96 columns: 64 x 96 and 96 x 96
+@pytest.mark.parametrize("B,S,K,N,heads,dtype,bias", [(1, 701, 2052, 2000, 0, "f32", True), (2, 351, 2048, 1940, 20, "bf16", False), (3, 458, 1540, 1530, 9, "f16", True), (1, 1390, 1028, 1450, 0, "f32", False)])
+def test_products_on_pieces_of_96_columns(lm, hip, oracle, B, S, K, N, heads, dtype, bias):
+    test_projection_matches_float64(lm, hip, oracle, B, S, K, N, heads, dtype, bias)
+    if not heads:
+        test_values_that_pieces_do_not_hold(lm, hip, oracle, S, K, N)
+
+
 @pytest.mark.parametrize("M,K,N", [(590, 580, 1150), (33, 772, 5000), (701, 2052, 2500)])
 def test_values_that_pieces_do_not_hold(lm, hip, oracle, M, K, N):
     """Infinities, NaN, values next to the largest and rows far below the smallest normal bf16 piece: what fp32 gives."""
