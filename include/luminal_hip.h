@@ -363,13 +363,16 @@ int lmh_copy_many(void *const *dst, const void *const *src, const size_t *bytes,
 
 /* The same copies together with the launches that a compiled graph begins with: results and memory are as after
  *   lmh_copy_many(dst, src, bytes, n, p->stream), then lmh_decode_step(p, x)
- *   lmh_copy_many(dst, src, bytes, n, p->stream), then lmh_kv_append(p), then lmh_flash_attn_fwd(attn) unless attn is null.
+ *   lmh_copy_many(dst, src, bytes, n, p->stream), then lmh_kv_append(p), then lmh_flash_attn_fwd(attn) unless attn is null
+ *   lmh_copy_many(dst, src, bytes, n_copies, stream), then lmh_matmul(p, n, stream).
  * Where no copy depends on another or meets what the launches write, these take their operands from src and the copies run
  * beside them; anything else is done in that order. `attn` has the stream of `p`. */
 int lmh_decode_step_fed(const lmh_decode_params *p, const lmh_decode_step_extra *x, void *const *dst, const void *const *src,
                         const size_t *bytes, int32_t n);
 int lmh_kv_append_fed(const lmh_kv_append_params *p, const lmh_attn_params *attn, void *const *dst, const void *const *src,
                       const size_t *bytes, int32_t n);
+int lmh_matmul_fed(const lmh_matmul_params *p, int32_t n, void *stream, void *const *dst, const void *const *src, const size_t *bytes,
+                   int32_t n_copies);
 
 #ifdef __cplusplus
 }

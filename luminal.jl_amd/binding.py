@@ -27,7 +27,7 @@ EXPORTS = [
     "lmh_decode_workspace_bytes", "lmh_decode_auto_splits", "lmh_decode_attn", "lmh_flash_attn_plan", "lmh_rope",
     "lmh_kv_append", "lmh_stream_create", "lmh_stream_destroy", "lmh_graph_capture_begin", "lmh_graph_capture_end",
     "lmh_graph_launch", "lmh_graph_destroy", "lmh_static_scratch_bytes", "lmh_decode_static_splits",
-    "lmh_decode_attn_static", "lmh_decode_step_splits", "lmh_decode_step", "lmh_matmul", "lmh_map", "lmh_copy_many", "lmh_decode_step_fed", "lmh_kv_append_fed",
+    "lmh_decode_attn_static", "lmh_decode_step_splits", "lmh_decode_step", "lmh_matmul", "lmh_map", "lmh_copy_many", "lmh_decode_step_fed", "lmh_kv_append_fed", "lmh_matmul_fed",
     "lmh_host_alloc", "lmh_host_free", "lmh_upload", "lmh_download",
 ]
 
@@ -193,6 +193,7 @@ def load():
     lists = L.lmh_copy_many.argtypes[:4]
     L.lmh_decode_step_fed.argtypes = [ctypes.POINTER(DecodeParams), ctypes.POINTER(DecodeStepExtra)] + lists
     L.lmh_kv_append_fed.argtypes = [ctypes.POINTER(KvAppendParams), ctypes.POINTER(AttnParams)] + lists
+    L.lmh_matmul_fed.argtypes = L.lmh_matmul.argtypes + lists
     L.lmh_host_alloc.argtypes = [ctypes.POINTER(vp), ctypes.c_size_t]
     L.lmh_host_free.argtypes = [vp]
     L.lmh_upload.argtypes = [ctypes.POINTER(UploadItem), ctypes.c_int32, vp]
@@ -385,6 +386,11 @@ def decode_step_fed(params, extra, dst, src, nbytes, n):
 def kv_append_fed(params, attn, dst, src, nbytes, n):
     """lmh_copy_many, lmh_kv_append and, unless `attn` is None, lmh_flash_attn_fwd in one call."""
     check(load().lmh_kv_append_fed(ctypes.byref(params), None if attn is None else ctypes.byref(attn), dst, src, nbytes, n))
+
+
+def matmul_fed(params, n, dst, src, nbytes, n_copies):
+    """lmh_copy_many and lmh_matmul in one call."""
+    check(load().lmh_matmul_fed(params, n, None, dst, src, nbytes, n_copies))
 
 
 def stream_create():

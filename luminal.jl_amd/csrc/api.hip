@@ -743,11 +743,10 @@ int lmh_kv_append(const lmh_kv_append_params *p) {
 // --------------------------------------------------------------------------------------------
 static bool graph_dtype(int d) { return d == LMH_F32 || d == LMH_F16 || d == LMH_BF16 || d == LMH_I32; }
 
-int lmh_matmul(const lmh_matmul_params *ps, int32_t n, void *stream) {
+static int matmul_args(const lmh_matmul_params *ps, int32_t n, MatmulArgs &args) {
   static_assert(LMH_MATMUL_GROUP == kMatmulGroup, "header and kernel agree");
   if (!ps) return fail(LMH_E_NULL, "lmh_matmul: null params");
   if (n < 1 || n > LMH_MATMUL_GROUP) return fail(LMH_E_SHAPE, "lmh_matmul: %d products, 1 to %d fit a launch", n, LMH_MATMUL_GROUP);
-  MatmulArgs args = {};
   for (int i = 0; i < n; i++) {
     const lmh_matmul_params &p = ps[i];
     if (!p.c || !p.a || !p.b) return fail(LMH_E_NULL, "lmh_matmul: null tensor pointer");
@@ -774,7 +773,13 @@ int lmh_matmul(const lmh_matmul_params *ps, int32_t n, void *stream) {
               ((int64_t)p.N * p.b_stride[2] + p.K) * 4 < kMaxBytes;
     q.b_by_column = !q.b_vec && p.b_stride[2] == 1 && p.b_stride[1] != 1;
   }
-  return launch_matmul(args, n, (hipStream_t)stream);
+  return LMH_OK;
+}
+
+int lmh_matmul(const lmh_matmul_params *ps, int32_t n, void *stream) {
+  MatmulArgs args = {};
+  const int rc = matmul_args(ps, n, args);
+  return rc != LMH_OK ? rc : launch_matmul(args, n, (hipStream_t)stream);
 }
 
 int lmh_map(const lmh_map_params *p, void *stream) {
@@ -985,6 +990,26 @@ int lmh_kv_append_fed(const lmh_kv_append_params *p, const lmh_attn_params *attn
   int rc = lmh_copy_many(dst, src, bytes, n, p ? p->stream : nullptr);
   if (rc == LMH_OK) rc = lmh_kv_append(p);
   return rc != LMH_OK || !attn ? rc : lmh_flash_attn_fwd(attn);
+}
+
+int lmh_matmul_fed(const lmh_matmul_params *ps, int32_t n, void *stream, void *const *dst, const void *const *src, const size_t *bytes,
+                   int32_t n_copies) {
+  MatmulArgs args = {};
+  Feed feed;
+  if (feed.apart(dst, src, bytes, n_copies) && matmul_args(ps, n, args) == LMH_OK && feed.some()) {
+    bool ok = true;
+    for (int i = 0; i < n && ok; i++) {
+      MatmulProblem &q = args.p[i];
+      auto size = [](int dtype) -> int64_t { return dtype == LMH_F32 || dtype == LMH_I32 ? 4 : 2; };
+      ok = !feed.touches(q.c, (int64_t)q.batch * q.M * q.N * size(q.c_dtype)) &&
+           feed.redirect(q.a, ((q.batch - 1) * q.as[0] + (q.M - 1) * q.as[1] + (q.K - 1) * q.as[2] + 1) * size(q.a_dtype)) &&
+           feed.redirect(q.b, ((q.batch - 1) * q.bs[0] + (q.K - 1) * q.bs[1] + (q.N - 1) * q.bs[2] + 1) * size(q.b_dtype)) &&
+           (!q.bias || feed.redirect(q.bias, q.N * size(q.bias_dtype)));
+    }
+    if (ok) return launch_matmul(args, n, (hipStream_t)stream, &feed.a, feed.n);
+  }
+  const int rc = lmh_copy_many(dst, src, bytes, n_copies, stream);
+  return rc != LMH_OK ? rc : lmh_matmul(ps, n, stream);
 }
 
 }  // extern "C"

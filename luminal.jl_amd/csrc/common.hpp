@@ -215,7 +215,7 @@ int launch_prefill_valu(const PrefillArgs &a, int dtype, hipStream_t stream);
 int launch_decode(const DecodeArgs &a, int dtype, hipStream_t stream, CopyManyArgs *fed = nullptr, int n_fed = 0);
 int launch_rope(const RopeArgs &a, int dtype, hipStream_t stream);
 int launch_kv_append(KvAppendArgs a, int dtype, hipStream_t stream, CopyManyArgs *fed = nullptr, int n_fed = 0);  // ... of its first
-int launch_matmul(MatmulArgs &args, int n, hipStream_t stream);
+int launch_matmul(MatmulArgs &args, int n, hipStream_t stream, CopyManyArgs *fed = nullptr, int n_fed = 0);
 int launch_map(MapArgs &a, hipStream_t stream);
 int launch_copy_many(CopyManyArgs &a, int n, hipStream_t stream);
 int launch_upload(const UploadItem *items, int n, hipStream_t stream);

@@ -23,6 +23,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "copy.hpp"
 #include "dtypes.hpp"
 #include "split.hpp"
 
@@ -83,7 +84,7 @@ __device__ inline void store_block(const MatmulProblem &p, const Acc &acc, int m
 
 // VEC: every operand is fp32, contiguous along the contraction and 16-byte aligned, K a multiple of 4.
 template <int WM, int WN, int WK, bool VEC>
-__global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(MatmulArgs args) {
+__global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(MatmulArgs args, CopyManyArgs fed, int n_copies) {
   constexpr int NT = 64 * WM * WN * WK;
   constexpr int BM = 32 * WM, BN = 32 * WN, BKT = BK * WK;
   constexpr int CA = BM * BKT / 4, CB = BN * BKT / 4;  // 16-byte chunks of a tile
@@ -95,7 +96,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(Matmul
   // ---- which tile of which product ----
   const int per_xcd = (args.n_tiles + 7) / 8;
   int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per_xcd || t >= args.n_tiles) return;
+  if ((int)(blockIdx.x >> 3) >= per_xcd) {  // copies beside the products
+    if ((int)blockIdx.x - 8 * per_xcd < n_copies) copy_block<64 * WM * WN * WK>(fed, blockIdx.x - 8 * per_xcd);
+    return;
+  }
+  if (t >= args.n_tiles) return;
   int g = 0;
 #pragma unroll
   for (int i = 1; i < kMatmulGroup; i++)
@@ -295,7 +300,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(Matmul
 __device__ inline int swizzle16(int row) { return ((row >> 1 ^ row >> 3) & 1) | (row >> 1 & 2); }
 
 template <int MB, int NB>
-__global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args) {
+__global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, CopyManyArgs fed, int n_copies) {
   constexpr int BM = 32 * MB, BN = 32 * NB, WK = 4;
   constexpr int L = 2 * (MB + NB);              // loads of 1 KB (16 rows) per stage: a, then b
   constexpr int kStage = 16 * 16 * L;           // floats
@@ -304,7 +309,11 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args) {
 
   const int per_xcd = (args.n_tiles + 7) / 8;
   int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per_xcd || t >= args.n_tiles) return;
+  if ((int)(blockIdx.x >> 3) >= per_xcd) {
+    if ((int)blockIdx.x - 8 * per_xcd < n_copies) copy_block<256>(fed, blockIdx.x - 8 * per_xcd);
+    return;
+  }
+  if (t >= args.n_tiles) return;
   int g = 0;
 #pragma unroll
   for (int i = 1; i < kMatmulGroup; i++)
@@ -510,37 +519,39 @@ int64_t number_tiles(MatmulArgs &args, int n, int bm, int bn) {
   for (int i = 0; i < kMatmulGroup; i++) {
     args.first_tile[i] = (int)tiles;
     if (i < n) tiles += (int64_t)args.p[i].batch * ((args.p[i].M + bm - 1) / bm) * ((args.p[i].N + bn - 1) / bn);
-    if (tiles >= (int64_t(1) << 31) - 8) return -1;
+    if (tiles >= (int64_t(1) << 31) - 65536) return -1;  // (with room for the copies)
   }
   args.n_tiles = (int)tiles;
   return tiles;
 }
 
 template <int WM, int WN, int WK>
-int launch_form(MatmulArgs &args, int n, hipStream_t stream) {
+int launch_form(MatmulArgs &args, int n, hipStream_t stream, const CopyManyArgs &fed, int n_copies) {
   const int64_t tiles = number_tiles(args, n, 32 * WM, 32 * WN);
   if (tiles < 0) return fail(LMH_E_UNSUPPORTED, "matmul: too many tiles");
   bool vec = true;
   for (int i = 0; i < n; i++) vec = vec && args.p[i].a_vec && args.p[i].b_vec;
-  const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(64 * WM * WN * WK);
-  if (vec) hipLaunchKernelGGL((matmul_f32_kernel<WM, WN, WK, true>), grid, block, 0, stream, args);
-  else hipLaunchKernelGGL((matmul_f32_kernel<WM, WN, WK, false>), grid, block, 0, stream, args);
+  const dim3 grid((unsigned)((tiles + 7) / 8 * 8 + n_copies)), block(64 * WM * WN * WK);
+  if (vec) hipLaunchKernelGGL((matmul_f32_kernel<WM, WN, WK, true>), grid, block, 0, stream, args, fed, n_copies);
+  else hipLaunchKernelGGL((matmul_f32_kernel<WM, WN, WK, false>), grid, block, 0, stream, args, fed, n_copies);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }
 
 template <int MB, int NB>
-int launch_split_form(MatmulArgs &args, int n, hipStream_t stream) {
+int launch_split_form(MatmulArgs &args, int n, hipStream_t stream, const CopyManyArgs &fed, int n_copies) {
   const int64_t tiles = number_tiles(args, n, 32 * MB, 32 * NB);
   if (tiles < 0) return fail(LMH_E_UNSUPPORTED, "matmul: too many tiles");
-  hipLaunchKernelGGL((matmul_split_kernel<MB, NB>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, stream, args);
+  hipLaunchKernelGGL((matmul_split_kernel<MB, NB>), dim3((unsigned)((tiles + 7) / 8 * 8 + n_copies)), dim3(256), 0, stream, args, fed, n_copies);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }
 
 }  // namespace
 
-int launch_matmul(MatmulArgs &args, int n, hipStream_t stream) {
+int launch_matmul(MatmulArgs &args, int n, hipStream_t stream, CopyManyArgs *fed, int n_fed) {
+  const int n_copies = n_fed ? (int)number_copy_blocks(*fed, n_fed) : 0;
+  const CopyManyArgs copies = n_copies ? *fed : CopyManyArgs{};
   // Both kernels by what their forms cost, in us: a part per launch, a part per round of the CUs, and one per round and
   // contraction element.
   // fp32 product: rounds times the 32 x 32 blocks of a workgroup, with a weight for what the smaller workgroups pay in loads and
@@ -573,21 +584,21 @@ int launch_matmul(MatmulArgs &args, int n, hipStream_t stream) {
     const double s64x96 = rounds(64, 96) * (7.0 + 0.0129 * K), s64 = 2.9 + r64 * (2.6 + 0.0096 * K), s32x64 = 3.7 + rounds(32, 64) * (0.9 + 0.0068 * K);
     const double split = std::min({s96, s64x128, s64x96, s64, s32x64});
     if (split < fp32) {
-      if (split == s64) return launch_split_form<2, 2>(args, n, stream);
-      if (split == s32x64) return launch_split_form<1, 2>(args, n, stream);
-      if (split == s64x96) return launch_split_form<2, 3>(args, n, stream);
-      if (split == s64x128) return launch_split_form<2, 4>(args, n, stream);
-      return launch_split_form<3, 3>(args, n, stream);
+      if (split == s64) return launch_split_form<2, 2>(args, n, stream, copies, n_copies);
+      if (split == s32x64) return launch_split_form<1, 2>(args, n, stream, copies, n_copies);
+      if (split == s64x96) return launch_split_form<2, 3>(args, n, stream, copies, n_copies);
+      if (split == s64x128) return launch_split_form<2, 4>(args, n, stream, copies, n_copies);
+      return launch_split_form<3, 3>(args, n, stream, copies, n_copies);
     }
   }
   if (c64 <= c32x64 && c64 <= c32) {
     // with several rounds the other workgroups on a CU cover what eight waves on one block cover in a single round
     // (4096^3: 1062 against 1086 us = 129 TFLOP/s, 82 % of the fp32 matrix peak)
-    if (r64 > 4) return launch_form<2, 2, 1>(args, n, stream);
-    return launch_form<2, 2, 2>(args, n, stream);
+    if (r64 > 4) return launch_form<2, 2, 1>(args, n, stream, copies, n_copies);
+    return launch_form<2, 2, 2>(args, n, stream, copies, n_copies);
   }
-  if (c32x64 <= c32) return launch_form<1, 2, 2>(args, n, stream);
-  return launch_form<1, 1, 4>(args, n, stream);
+  if (c32x64 <= c32) return launch_form<1, 2, 2>(args, n, stream, copies, n_copies);
+  return launch_form<1, 1, 4>(args, n, stream, copies, n_copies);
 }
 
 }  // namespace lmh

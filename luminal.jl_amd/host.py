@@ -1114,7 +1114,7 @@ def _prepare(op, out, inputs, workspaces):
 
 
 def _fed_start(steps):
-    """(number of steps, call) for a graph that begins with a decode step or a cache append: `call` of the inputs' copies makes
+    """(number of steps, call) for a graph that begins with products, a decode step or a cache append: `call` of the inputs' copies makes
     these and runs the steps. (A copy in front of such steps is a launch as long as theirs.) (0, None) for others."""
     if steps and hasattr(steps[0], "fed"):
         return 1, steps[0].fed

@@ -166,11 +166,19 @@ def fill_matmul(p, out, a, b, transposed=False, bias=None, heads=0):
     return True
 
 
+def _matmul_launch(p):
+    def launch(stream=None):
+        binding.matmul(p, len(p), stream)
+
+    launch.fed = lambda *copies: binding.matmul_fed(p, len(p), *copies)
+    return launch
+
+
 def matmul_launcher(out, a, b):
     p = (binding.MatmulParams * 1)()
     if len(a.shape) < 2 or len(b.shape) < 2 or not fill_matmul(p[0], out, a, b):
         return None
-    return lambda stream=None: binding.matmul(p, 1, stream)
+    return _matmul_launch(p)
 
 
 class Projection:
@@ -196,7 +204,7 @@ class ProjectionOp:
         for q, item, out in zip(p, self.items, outs):
             w = rest.pop(0)
             fill_matmul(q, out, x, w, transposed=True, bias=rest.pop(0) if item.bias is not None else None, heads=item.heads)
-        return lambda stream=None: binding.matmul(p, len(self.items), stream)
+        return _matmul_launch(p)
 
 
 class ViewOp:
