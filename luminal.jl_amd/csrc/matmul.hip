@@ -572,15 +572,16 @@ int launch_matmul(MatmulArgs &args, int n, hipStream_t stream, CopyManyArgs *fed
   // 700 x 2048 x 2048 67 / 44 / 46 / 40 / 47 / 51, 1374 x 1536 x 1536 80 / 42 / 69 / 56 / 56 / 62, 700 x 2560 x 2048 70 / 49 / 48 /
   // 69 / 49 / 63, 1248 x 1024 x 512 19 / 19 / 17 / 15 / 17 / 16. A launch of few tiles stays with the fp32 product, whose waves
   // share the contraction of smaller blocks (100 x 768 x 768 8.1 -> 18.6 on 64 x 128, 9.6 on 32 x 64).
-  bool vec = true;
+  bool vec = true, near96 = true;  // 96 rows of every a within 32-bit offsets; a_vec has looked at 64
   int64_t K = 0;
   for (int i = 0; i < n; i++) {
     vec = vec && args.p[i].a_vec && args.p[i].b_vec;
+    near96 = near96 && (96 * args.p[i].as[1] + args.p[i].K) * 4 < kOutOfRange;
     K = std::max<int64_t>(K, args.p[i].K);
   }
   if (vec) {
     const double fp32 = 0.95 * (3.3 + 0.0045 * K * std::min(c64, std::min(c32x64, c32)));
-    const double s96 = rounds(96, 96) * (10.0 + 0.0160 * K), s64x128 = rounds(64, 128) * (7.5 + 0.0165 * K);
+    const double s96 = near96 ? rounds(96, 96) * (10.0 + 0.0160 * K) : INFINITY, s64x128 = rounds(64, 128) * (7.5 + 0.0165 * K);
     const double s64x96 = rounds(64, 96) * (7.0 + 0.0129 * K), s64 = 2.9 + r64 * (2.6 + 0.0096 * K), s32x64 = 3.7 + rounds(32, 64) * (0.9 + 0.0068 * K);
     const double split = std::min({s96, s64x128, s64x96, s64, s32x64});
     if (split < fp32) {

@@ -52,6 +52,24 @@ def test_products_on_pieces_of_96_columns(lm, hip, oracle, B, S, K, N, heads, dt
         test_values_that_pieces_do_not_hold(lm, hip, oracle, S, K, N)
 
 
+def test_products_of_rows_far_apart(lm, hip, oracle):
+    """96 rows so far apart that the last one's byte offset takes more than 31 bits (64 rows' does not), beside a remainder of K."""
+    M, K, N, step = 96, 1540, 24576, 5_800_000
+    x, w = oracle.gen_normal((M, K), 37000), oracle.gen_normal((N, K), 37100)
+    spread = np.ones(((M - 1) * step + K,), np.float32)
+    for m in range(M):
+        spread[m * step:m * step + K] = x[m]
+    dx, dw, out = lm.to_device(spread, hip), lm.to_device(w, hip), lm.HipArray((1, M, N), "f32", hip)
+    p = (lm.binding.MatmulParams * 1)()
+    assert _low(lm).fill_matmul(p[0], out, lm.HipArray((1, M, K), "f32", hip), dw, transposed=True)
+    p[0].a, p[0].a_stride[1] = dx.ptr, step
+    lm.binding.matmul(p, 1)
+    got = out.to_host()[0]
+    # fp32 sums of K products, each within K 2^-24 of the sum of their magnitudes
+    want, top = x.astype(np.float64) @ w.astype(np.float64).T, np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    assert (np.abs(got - want) <= K * 2.0 ** -24 * top).all()
+
+
 @pytest.mark.parametrize("M,K,N", [(590, 580, 1150), (33, 772, 5000), (701, 2052, 2500)])
 def test_values_that_pieces_do_not_hold(lm, hip, oracle, M, K, N):
     """Infinities, NaN, values next to the largest and rows far below the smallest normal bf16 piece: what fp32 gives."""
