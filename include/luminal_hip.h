@@ -211,7 +211,7 @@ typedef struct lmh_decode_params {
 /* bytes of split-KV partial storage lmh_decode_attn needs for these sizes (0 on bad input) */
 size_t lmh_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lmax, int32_t D,
                                   int32_t num_splits);
-/* the split count lmh_decode_attn uses when num_splits == 0 */
+/* the most splits lmh_decode_attn uses when num_splits == 0, and those its workspace has to hold; fewer where that is faster */
 int32_t lmh_decode_auto_splits(int32_t B, int32_t Hkv, int32_t Lmax);
 int lmh_decode_attn(const lmh_decode_params *p);
 
@@ -224,7 +224,7 @@ int lmh_decode_attn(const lmh_decode_params *p);
  *     (a sequence whose cache is full attends its old rows only and writes nothing);
  *   - k_cache / v_cache are written: row kv_len[b] of every KV head receives x->k_new (rotated when x->rope)
  *     and x->v_new; out = attention of q over rows 0 .. kv_len[b] inclusive. q itself is not modified.
- *   - num_splits == 0 takes lmh_decode_step_splits(); an explicit count must be >= 2; the workspace is
+ *   - num_splits == 0 takes up to lmh_decode_step_splits(); an explicit count must be >= 2; the workspace is
  *     lmh_decode_workspace_bytes(..., that count).
  * The first launch is the split kernel of lmh_decode_attn over the old rows, rotating q as it loads it; the second
  * merges the partials, adds the new row from k_new / v_new and stores it into the caches, so the separate append
@@ -246,7 +246,7 @@ int lmh_decode_step(const lmh_decode_params *p, const lmh_decode_step_extra *x);
  * loops, harnesses that forbid allocation). Same parameter block, same kernels, same results; `workspace`
  * and `workspace_bytes` are ignored. The split-KV partials go to a static device array of
  * LMH_STATIC_SCRATCH_BYTES that each GPU the library runs on holds until the process ends.
- *   - num_splits == 0 takes lmh_decode_static_splits(): the split count of lmh_decode_attn, halved until
+ *   - num_splits == 0 takes lmh_decode_static_splits(): lmh_decode_auto_splits(), halved until
  *     the partials fit. An explicit num_splits whose partials (lmh_decode_workspace_bytes) exceed the
  *     array is rejected with LMH_E_WORKSPACE.
  *   - Every call on one GPU shares that GPU's array, which keeps the last call's contents. Nothing in it

@@ -6,6 +6,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "common.hpp"
@@ -502,10 +503,34 @@ size_t lmh_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lm
   return (size_t)B * Hq * num_splits * (size_t)(D + 2) * sizeof(float);
 }
 
+// Where the caller leaves the split count to the library, the matrix-core kernel takes fewer than lmh_decode_auto_splits where
+// that is faster (us with that count and with this one, D = 128 bf16 unless named; 190 sizes timed):
+//   * one, so that the merge launch and the partials drop out, where a workgroup walks a whole sequence in the time of that
+//     launch, or where the pairs fill the CUs and the walk is short beside the whole launch: B=1 Hkv=8 L=200 12.8 -> 9.2 and
+//     L=512 11.8 -> 11.2 (L=1024 12.1 -> 15.7; D=64 L=512 9.4 -> 7.9, L=1000 9.4 -> 10.5, with 96 pairs 13.4 -> 11.8), B=16
+//     L=1024 20.8 -> 18.7 (L=2100 33.5 -> 32.3, ragged 26.0 -> 28.8), B=64 L=512 ragged 35.1 -> 24.0, L=2100 92 -> 90 (L=4096
+//     169.6 -> 167.6, ragged 121.0 -> 120.6: within what boxes differ by); the longer walks only where the last round of pairs
+//     is nearly full (B=81 Hkv=4 L=3522 D=64 54.5 -> 58.6);
+//   * one unit per CU for few pairs, in chunks long enough for the merge: B=4 Hkv=8 L=2100 19.3 -> 16.0, L=8192 ragged
+//     28.4 -> 24.0, B=1 L=8192 19.0 -> 16.4, L=32768 41.4 -> 29.9. From 128 pairs on more units balance ragged batches better
+//     (B=16 L=4096 ragged 38.5 with 16, 39.9 with 2).
+// A step keeps its two launches and with them two splits at least; there, few are no better than more.
+static int32_t decode_splits(const DecodeArgs &a, int32_t most) {
+  const int64_t cus = device_cu_count(), pairs = (int64_t)a.B * a.Hkv * ((a.Hq / a.Hkv + 15) / 16), walk = (int64_t)a.Lmax * a.D;
+  const bool full = pairs * 20 >= (pairs + cus - 1) / cus * cus * 17;
+  const bool one = (walk <= 65536 && (a.Lmax <= 512 || pairs * 8 >= cus * 3)) || (walk <= 131072 && pairs >= cus / 2) || (walk <= 262144 && pairs >= cus && full);
+  if (one && !a.step) return 1;
+  const int64_t per_pair = cus / pairs;
+  if (per_pair < 4 || per_pair * pairs * 8 < cus * 7) return most;
+  const int64_t chunk = std::min(std::max(a.Lmax / 1024 * 64, 128), 512);
+  const int64_t chunks = std::max<int64_t>((a.Lmax + chunk - 1) / chunk, a.step ? 2 : 1);
+  return (int32_t)std::min({per_pair, chunks, (int64_t)most});
+}
+
 // Validation and launch shared by lmh_decode_attn (caller-owned workspace) and lmh_decode_attn_static (the
-// library's static scratch): `ws` / `ws_bytes` is the split-KV partial storage, `num_splits` already resolved.
+// library's static scratch): `ws` / `ws_bytes` is the split-KV partial storage, enough for `num_splits`; `choose`: fewer will do.
 static int decode_args(const lmh_decode_params *p, const char *fn, int32_t num_splits, void *ws, size_t ws_bytes,
-                       const lmh_decode_step_extra *step, DecodeArgs &a) {
+                       const lmh_decode_step_extra *step, DecodeArgs &a, bool choose) {
   a.step = step ? 1 : 0;
   a.q_rope = (step && step->rope) ? 1 : 0;
   a.rope_interleaved = (step && step->pairing == LMH_ROPE_INTERLEAVED) ? 1 : 0;
@@ -546,15 +571,18 @@ static int decode_args(const lmh_decode_params *p, const char *fn, int32_t num_s
   const bool slice_fits = rows * a.ks[2] * 2 < 0x7ffffff0 && rows * a.vs[2] * 2 < 0x7ffffff0;
   a.mfma_ok = (p->scale > 0.f && aligned16(p->q) && a.qs[0] % 8 == 0 && a.qs[1] % 8 == 0 && slice_fits) ? 1 : 0;
   a.num_splits = num_splits;
-  a.chunk = decode_chunk_for(p->Lmax, a.num_splits);
   a.ws_o = nullptr;
   a.ws_ml = nullptr;
-  if (a.num_splits > 1) {
-    const size_t need = lmh_decode_workspace_bytes(p->B, p->Hq, p->Hkv, p->Lmax, p->D, a.num_splits);
+  if (num_splits > 1) {
+    const size_t need = lmh_decode_workspace_bytes(p->B, p->Hq, p->Hkv, p->Lmax, p->D, num_splits);
     if (!ws || ws_bytes < need)
       return fail(LMH_E_WORKSPACE, "%s: workspace of %zu bytes needed for %d splits, got %zu", fn, need,
-                  a.num_splits, ws ? ws_bytes : (size_t)0);
+                  num_splits, ws ? ws_bytes : (size_t)0);
     if (!aligned16(ws)) return fail(LMH_E_WORKSPACE, "%s: workspace must be 16-byte aligned", fn);
+    if (choose && a.mfma_ok && decode_mfma_supported(p->dtype, p->D, p->B)) a.num_splits = decode_splits(a, num_splits);
+  }
+  a.chunk = decode_chunk_for(p->Lmax, a.num_splits);
+  if (a.num_splits > 1) {
     a.ws_o = reinterpret_cast<float *>(ws);
     a.ws_ml = a.ws_o + (size_t)p->B * p->Hq * a.num_splits * p->D;
   }
@@ -570,9 +598,9 @@ static int decode_args(const lmh_decode_params *p, const char *fn, int32_t num_s
   return LMH_OK;
 }
 
-static int decode_launch(const lmh_decode_params *p, const char *fn, int32_t num_splits, void *ws, size_t ws_bytes) {
+static int decode_launch(const lmh_decode_params *p, const char *fn, int32_t num_splits, void *ws, size_t ws_bytes, bool choose) {
   DecodeArgs a;
-  const int rc = decode_args(p, fn, num_splits, ws, ws_bytes, nullptr, a);
+  const int rc = decode_args(p, fn, num_splits, ws, ws_bytes, nullptr, a, choose);
   return rc != LMH_OK ? rc : launch_decode(a, p->dtype, (hipStream_t)p->stream);
 }
 
@@ -599,7 +627,7 @@ int lmh_decode_attn(const lmh_decode_params *p) {
   const int rc = decode_check(p, "lmh_decode_attn");
   if (rc != LMH_OK) return rc;
   const int32_t splits = p->num_splits == 0 ? lmh_decode_auto_splits(p->B, p->Hkv, p->Lmax) : p->num_splits;
-  return decode_launch(p, "lmh_decode_attn", splits, p->workspace, p->workspace_bytes);
+  return decode_launch(p, "lmh_decode_attn", splits, p->workspace, p->workspace_bytes, p->num_splits == 0);
 }
 
 int32_t lmh_decode_step_splits(int32_t B, int32_t Hkv, int32_t Lmax) {
@@ -619,7 +647,7 @@ static int decode_step_args(const lmh_decode_params *p, const lmh_decode_step_ex
   if (x->rope && !(x->rope_base > 1.f)) return fail(LMH_E_SHAPE, "%s: rope base must be > 1", fn);
   if (p->num_splits == 1) return fail(LMH_E_SHAPE, "%s: num_splits must be 0 or >= 2", fn);
   const int32_t splits = p->num_splits == 0 ? lmh_decode_step_splits(p->B, p->Hkv, p->Lmax) : p->num_splits;
-  return decode_args(p, fn, splits, p->workspace, p->workspace_bytes, x, a);
+  return decode_args(p, fn, splits, p->workspace, p->workspace_bytes, x, a, p->num_splits == 0);
 }
 
 int lmh_decode_step(const lmh_decode_params *p, const lmh_decode_step_extra *x) {
@@ -662,7 +690,7 @@ int lmh_decode_attn_static(const lmh_decode_params *p) {
   }
   // Nothing in the scratch has to start at zero: every partial slot the merge kernel reads was written by
   // the split kernel of the same call (a result, or the "empty" marker), so no clearing is enqueued.
-  const int rc_launch = decode_launch(p, fn, splits, ws, LMH_STATIC_SCRATCH_BYTES);
+  const int rc_launch = decode_launch(p, fn, splits, ws, LMH_STATIC_SCRATCH_BYTES, false);
   if (rc_launch == LMH_OK && splits > 1) static_scratch_mark((hipStream_t)p->stream);
   return rc_launch;
 }

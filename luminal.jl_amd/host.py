@@ -940,8 +940,8 @@ def _prepare_decode_step(op, out, inputs, workspaces=None):
     p.dtype = binding.DTYPE_CODES[q.dtype]
     p.scale, p.head_map = op.scale, op.head_map
     p.out_f32 = int(res.dtype == "f32")
-    p.num_splits = op.num_splits or binding.decode_step_splits(p.B, p.Hkv, p.Lmax)
-    need = binding.decode_workspace_bytes(p.B, p.Hq, p.Hkv, p.Lmax, p.D, p.num_splits)
+    p.num_splits = op.num_splits
+    need = binding.decode_workspace_bytes(p.B, p.Hq, p.Hkv, p.Lmax, p.D, op.num_splits or binding.decode_step_splits(p.B, p.Hkv, p.Lmax))
     x = binding.DecodeStepExtra()
     x.k_new, x.v_new = k_new.ptr, v_new.ptr
     x.rope = int(op.rope_base is not None)
@@ -1061,8 +1061,8 @@ def _decode_params(op, out, inputs):
     p.dtype = binding.DTYPE_CODES[q.dtype]
     p.scale, p.head_map = op.scale, op.head_map
     p.out_f32 = int(out.dtype == "f32")
-    p.num_splits = op.num_splits or binding.decode_auto_splits(p.B, p.Hkv, p.Lmax)
-    return p, binding.decode_workspace_bytes(p.B, p.Hq, p.Hkv, p.Lmax, p.D, p.num_splits)
+    p.num_splits = op.num_splits
+    return p, binding.decode_workspace_bytes(p.B, p.Hq, p.Hkv, p.Lmax, p.D, op.num_splits)
 
 
 def _rope_op_params(op, out, inputs, stream=None):

@@ -445,6 +445,23 @@ def test_whisper_split_scale_equals_single_scale(lm, hip, oracle):
     assert rel_err(split, fused) <= 1e-5
 
 
+# the library's own split counts on both sides of each line of its rule: a walk of 65536, 131072 and 262144 elements, pairs that
+# fill the CUs once and half, few pairs in one unit per CU (chunks of 128, of Lmax / 16 and of 512 keys), groups of two slices
+@pytest.mark.parametrize("B,Hq,Hkv,L,D", [
+    (1, 8, 2, 512, 128), (1, 8, 2, 513, 128), (1, 2, 2, 513, 64), (12, 8, 8, 1024, 64), (2, 2, 1, 257, 256), (16, 16, 8, 1024, 128), (16, 16, 8, 1025, 128),
+    (15, 16, 8, 1024, 128), (32, 8, 8, 2048, 128), (32, 8, 8, 2049, 128), (33, 8, 8, 1500, 128), (1, 8, 8, 9000, 64), (8, 32, 4, 2100, 96), (1, 40, 2, 1100, 128),
+    (6, 8, 8, 1500, 128), (1, 4, 1, 33000, 64),
+])
+def test_decode_split_counts_of_the_library(lm, hip, oracle, B, Hq, Hkv, L, D):
+    q, k, v = inputs(oracle, (B, Hq, D), (B, Hkv, L, D), "bf16", 7650 + L)
+    lens = np.maximum(1, L - np.arange(B, dtype=np.int32) * (L // B))
+    for kv_len in (None, lens):
+        got = run_decode(lm, hip, q, k, v, "bf16", kv_len=kv_len, out_dtype="f32")
+        assert rel_err(got, oracle.decode_attn(q, k, v, kv_len=kv_len)) <= TOL["bf16"]
+        # the partial sums are fp32 and the weights of each split are exact to 1e-5 (as for every explicit count)
+        assert rel_err(got, run_decode(lm, hip, q, k, v, "bf16", kv_len=kv_len, num_splits=4, out_dtype="f32")) <= 2e-5
+
+
 @pytest.mark.parametrize("dtype,D", [("f32", 64), ("f32", 128), ("f16", 64), ("f16", 96), ("bf16", 128), ("bf16", 256), ("f16", 8)])
 @pytest.mark.parametrize("Hq,Hkv", [(4, 4), (8, 4), (8, 2), (8, 1), (12, 2), (16, 1)])
 def test_decode_group_sizes_and_dims(lm, hip, oracle, dtype, D, Hq, Hkv):
