@@ -301,7 +301,7 @@ function execute_op!(out::HipArray{TO,3}, op::DecodeAttentionOp, q::HipArray{T,3
                  B, Hq, Hkv, Lmax, D, splits)
     ws = workspace(need)
     p = Ref(DecodeParams(out.ptr, q.ptr, kc.ptr, vc.ptr, Ptr{Int32}(kv_len.ptr), B, Hq, Hkv, Lmax, D, Z2, Z2, Z3, Z3,
-                         dtype_code(T), op.scale, op.head_map, out_f32, splits,
+                         dtype_code(T), op.scale, op.head_map, out_f32, Int32(0),
                          ws === nothing ? C_NULL : ws.ptr, need, current_stream()))
     check(ccall((:lmh_decode_attn, libluminal_hip), Cint, (Ref{DecodeParams},), p))
     return out
@@ -359,7 +359,7 @@ function execute_op!(out::HipArray{TO,3}, op::DecodeStepOp, q::HipArray{T,3}, kc
                  B, Hq, Hkv, Lmax, D, splits)
     ws = workspace(need)
     p = Ref(DecodeParams(out.ptr, q.ptr, kc.ptr, vc.ptr, Ptr{Int32}(pos.ptr), B, Hq, Hkv, Lmax, D, Z2, Z2, Z3, Z3,
-                         dtype_code(T), op.scale, op.head_map, out_f32, splits,
+                         dtype_code(T), op.scale, op.head_map, out_f32, Int32(0),
                          ws === nothing ? C_NULL : ws.ptr, need, current_stream()))
     x = Ref(DecodeStepExtra(k_new.ptr, v_new.ptr, Int32(op.rope_base > 0), Int32(0), op.rope_base > 0 ? op.rope_base : 10000.0f0))
     check(ccall((:lmh_decode_step, libluminal_hip), Cint, (Ref{DecodeParams}, Ref{DecodeStepExtra}), p, x))
