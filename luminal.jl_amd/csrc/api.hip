@@ -509,7 +509,7 @@ size_t lmh_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lm
 //     launch, or where the pairs fill the CUs and the walk is short beside the whole launch: B=1 Hkv=8 L=200 12.8 -> 9.2 and
 //     L=512 11.8 -> 11.2 (L=1024 12.1 -> 15.7; D=64 L=512 9.4 -> 7.9, L=1000 9.4 -> 10.5, with 96 pairs 13.4 -> 11.8), B=16
 //     L=1024 20.8 -> 18.7 (L=2100 33.5 -> 32.3, ragged 26.0 -> 28.8), B=64 L=512 ragged 35.1 -> 24.0, L=2100 92 -> 90 (L=4096
-//     169.6 -> 167.6, ragged 121.0 -> 120.6: within what boxes differ by); the longer walks only where the last round of pairs
+//     169.6 -> 167.6, ragged 121.0 -> 120.6: within what cards differ by); the longer walks only where the last round of pairs
 //     is nearly full (B=81 Hkv=4 L=3522 D=64 54.5 -> 58.6);
 //   * one unit per CU for few pairs, in chunks long enough for the merge: B=4 Hkv=8 L=2100 19.3 -> 16.0, L=8192 ragged
 //     28.4 -> 24.0, B=1 L=8192 19.0 -> 16.4, L=32768 41.4 -> 29.9. From 128 pairs on more units balance ragged batches better
