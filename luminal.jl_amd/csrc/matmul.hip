@@ -284,10 +284,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(Matmul
 // The same products for fp32 operands that are contiguous along the contraction, on the bf16 matrix pipe (16 times the rate).
 // Every operand is split into three bf16 pieces (split.hpp); of the nine products of pieces the six with x_i y_j, i + j <= 4, are
 // summed, the other three are below 2^-25 of x y. Error against 64 bits (2-norm): 3.6e-7 where the fp32 product has 5.7e-7 (K =
-// 2048; fewer roundings), 9.2e-8 and 1.07e-7 (K = 64). A wave whose operands the pieces do not hold takes its share again with
-// the fp32 product.
+// 2048; fewer roundings), 9.2e-8 and 1.07e-7 (K = 64). A workgroup with a sum that is not finite (an operand that the pieces do not
+// hold, or a sum beyond 2^80 before the scale comes off) takes its block again with the fp32 product; a launch all of whose blocks are
+// repeated takes twice as long (700 x 2048 x 2048: 44 and 103 us).
 //
-// Bound: the vector ALUs beside the matrix pipe. Splitting takes 5.5 instructions an element, 5.5 a MFMA at 64 x 128 and 7.3 at
+// Bound: the vector ALUs beside the matrix pipe. Splitting takes 6.5 instructions an element, 6.5 a MFMA at 64 x 128 and 8.7 at
 // 64 x 64, where the chip holds 1590 TFLOP/s of bare MFMAs and 1280 with six vector instructions each. So:
 //   * a wave multiplies blocks as large as its registers hold (MB x NB of 32 x 32, up to nine or eight), and the four
 //     waves of a workgroup each take all of its tile for every fourth 16 elements of the contraction; the shares are folded
@@ -378,10 +379,7 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
   const int frag0 = n * 16 + 4 * ((2 * h) ^ swizzle16(n)), frag1 = n * 16 + 4 * ((2 * h + 1) ^ swizzle16(n));
   const float *own = &lds[wk * 2 * kStage];
   struct Raw { floatx4_t lo, hi; };
-  uint32_t bits[MB + NB];  // every first piece of the lane's rows, or-ed
-#pragma unroll
-  for (int i = 0; i < MB + NB; i++) bits[i] = 0;
-  auto split = [&](const Raw &r, int block) { return split_8(r.lo, r.hi, &bits[block]); };
+  auto split = [](const Raw &r) { return split_8(r.lo * kPieceScale, r.hi * kPieceScale); };
   auto read_stage = [&](int i, Raw (&raw)[MB + NB]) {
 #pragma unroll
     for (int b = 0; b < MB + NB; b++) {
@@ -410,7 +408,7 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
   asm volatile("s_waitcnt vmcnt(%0)" :: "n"(L) : "memory");
   read_stage(0, raw);
 #pragma unroll
-  for (int b = 0; b < MB + NB; b++) even[b] = split(raw[b], b);
+  for (int b = 0; b < MB + NB; b++) even[b] = split(raw[b]);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   load_stage(2);
   constexpr int kA[6] = {0, 0, 1, 1, 0, 2}, kB[6] = {0, 1, 0, 1, 2, 0};
@@ -425,14 +423,14 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every read of that stage has returned
     load_stage(i + 3);
 #pragma unroll
-    for (int b = 0; b < MB + NB; b++) nxt[b] = split(raw[b], b);  // (past the last step: zeros)
+    for (int b = 0; b < MB + NB; b++) nxt[b] = split(raw[b]);  // (past the last step: zeros)
 #pragma unroll
     for (int q = 1; q < 6; q++)
 #pragma unroll
       for (int r = 0; r < MB; r++)
 #pragma unroll
         for (int j = 0; j < NB; j++) acc[r][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur[r].p[kA[q]], cur[MB + j].p[kB[q]], acc[r][j], 0, 0, 0);
-    constexpr int kValu = (46 * (MB + NB) + 5 * MB * NB) / (5 * MB * NB);
+    constexpr int kValu = (52 * (MB + NB) + 5 * MB * NB) / (5 * MB * NB);
 #pragma unroll
     for (int q = 0; q < 5 * MB * NB; q++) {
       __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
@@ -446,10 +444,6 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
   }
   if (i < steps) step(i, even, odd);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing arrives in the ring any more
-  bool exact = true;
-#pragma unroll
-  for (int i = 0; i < MB + NB; i++) exact = exact && pieces_hold(bits[i]);
-  bool again = __builtin_amdgcn_ballot_w64(!exact) != 0;
 
   // ---- fold the shares: each wave takes MB NB / WK blocks (or a part of one), and looks whether their sums are finite ----
   constexpr int kRegs = 16 * MB * NB / WK;  // registers a lane of a wave folds
@@ -457,8 +451,9 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
   static_assert(kRegs % kPart == 0, "whole parts");
   float sum[kRegs];
   for (int pass = 0;; pass++) {
-    if (again) {
-      // this wave's share again with the fp32 product, its operands straight from memory
+    const float unscale = pass ? 1.f : kPieceUnscale * kPieceUnscale;
+    if (pass) {
+      // the workgroup's block again with the fp32 product, the operands straight from memory
       clear();
       const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a_base), 0, a_desc[2], 0x00020000);
       const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(b_base), 0, b_desc[2], 0x00020000);
@@ -499,12 +494,11 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
       for (int w = 1; w < WK; w++) x += *reinterpret_cast<const floatx4_t *>(s + w * kShare);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        sum[4 * q + e] = x[e];
+        sum[4 * q + e] = x[e] * unscale;
         finite = fmaf(x[e], 0.f, finite);
       }
     }
-    if (pass == 1 || !__syncthreads_or(finite != 0.f || finite != finite)) break;
-    again = true;
+    if (pass || !__syncthreads_or(finite != 0.f || finite != finite)) break;
   }
 #pragma unroll
   for (int r = 0; r < kRegs; r += kPart) {

@@ -1,9 +1,12 @@
 // Flash attention forward in fp32 on the bf16 matrix pipe: every operand as three bf16 pieces, six products for one.
 //
 // Every operand is split into three bf16 pieces (split.hpp); of the nine products of pieces the six with x_i y_j, i + j <= 4, are
-// summed in fp32, the other three are below 2^-25 of x y. Six bf16 products take 6 / 16 of the time of the fp32 one. A workgroup
-// that meets a value that the pieces do not hold takes its rows again with the fp32 product. Error against 64 bits (2-norm): 1.9e-7
-// where the forms of prefill_f32.hip have 4.3e-7 (S = 1023 D = 80), 1.3e-7 and 2.7e-7 (S = 500 D = 96 causal).
+// summed in fp32, the other three are below 2^-25 of x y. Six bf16 products take 6 / 16 of the time of the fp32 one. Error against
+// 64 bits (2-norm): 1.9e-7 where the forms of prefill_f32.hip have 4.3e-7 (S = 1023 D = 80), 1.3e-7 and 2.7e-7 (S = 500 D = 96 causal).
+// V's pieces are scaled, so that a result that is left to a small value has all its bits. Q and K come as they are: what counts of
+// a score is its absolute error, and the bits that their pieces lose lie below 2^-126. A workgroup that meets an infinity, a NaN,
+// queries or keys so large that those bits would count, or an overflow takes its rows again with the fp32 product, straight from
+// memory: a launch all of whose workgroups do takes about five times as long (S = 1023 D = 80, 62 and 297 us).
 //
 // Same data flow as prefill_mfma.hip: a wave owns 32 query rows with the pieces of its Q fragments in registers, S^T = K Q^T so
 // that a lane holds one query column, and the registers of P, split there, are the B operands of O^T = V^T P^T. Statistics, sums
@@ -83,9 +86,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
     lds_off[r] = is_v ? 3 * kPlaneK + row * LDV + 8 * col : row * LDK + 8 * col;
   }
   floatx4_t x[R][2];
-  uint32_t bits[R];
-#pragma unroll
-  for (int r = 0; r < R; r++) bits[r] = 0;
+  float top = 0.f;  // the largest magnitude among this thread's values of Q and K (and a part of V's)
   auto is_v_wave = [&](int r) { return wave * 64 + r * NT >= BT * DC; };  // (a wave's 64 chunks are K's or V's: 8 D is a multiple of 64)
   auto fetch = [&](int kt) {
 #pragma unroll
@@ -97,12 +98,20 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
                                                              : __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, voff[r] + 16 * e, kt * k_tile_bytes, 0));
     }
   };
+  auto top_of = [](const floatx4_t &lo, const floatx4_t &hi, float so_far) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) so_far = fmaxf(fmaxf(fabsf(lo[e]), fabsf(hi[e])), so_far);
+    return so_far;
+  };
   auto split_tile = [&](int buf) {
 #pragma unroll
     for (int r = 0; r < R; r++) {
       if (kChunks % NT != 0 && wave * 64 + r * NT >= kChunks) continue;
-      const Pieces f = split_8(x[r][0], x[r][1], &bits[r]);
       const int plane = is_v_wave(r) ? kPlaneV : kPlaneK;
+      // V is scaled, K is not; a round of chunks that are all K's or all V's spares the other one's part
+      if (r * NT < BT * DC) top = top_of(x[r][0], x[r][1], top);
+      const float scale = (r + 1) * NT > BT * DC && is_v_wave(r) ? kPieceScale : 1.f;
+      const Pieces f = split_8(x[r][0] * scale, x[r][1] * scale);
 #pragma unroll
       for (int i = 0; i < 3; i++) *reinterpret_cast<bf16x8_t *>(&planes[buf * kTile + i * plane + lds_off[r]]) = f.p[i];
     }
@@ -154,10 +163,12 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
     }
   };
   Pieces qf[KS];
-  uint32_t q_bits = 0;
   load_q();
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) qf[ks] = split_8(q[ks][0], q[ks][1], &q_bits);
+  for (int ks = 0; ks < KS; ks++) {
+    top = top_of(q[ks][0], q[ks][1], top);
+    qf[ks] = split_8(q[ks][0], q[ks][1]);
+  }
 
   floatx16_t oacc[DB];
   float m_i, l_i;
@@ -275,9 +286,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
     for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
       for (int t = 0; t < 2; t++) {
-        uint32_t unused = 0;
         pf[kb][t] = split_8((floatx4_t){s[kb][8 * t], s[kb][8 * t + 1], s[kb][8 * t + 2], s[kb][8 * t + 3]},
-                            (floatx4_t){s[kb][8 * t + 4], s[kb][8 * t + 5], s[kb][8 * t + 6], s[kb][8 * t + 7]}, &unused);
+                            (floatx4_t){s[kb][8 * t + 4], s[kb][8 * t + 5], s[kb][8 * t + 6], s[kb][8 * t + 7]});
       }
 #pragma unroll
     for (int db = 0; db < DB; db++) {
@@ -307,9 +317,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   }
 
   // ---- values that pieces do not hold, anywhere in the workgroup: its rows again with the fp32 product ----
-  bool held = pieces_hold(q_bits);
-#pragma unroll
-  for (int r = 0; r < R; r++) held = held && pieces_hold(bits[r]);
+  // (up to here the lost bits of Q and K move a scaled score by less than 2^-37)
+  const bool held = fmaxf(top, 1.f) * a.scale <= 0x1p80f;
   float finite = 0.f;
 #pragma unroll
   for (int db = 0; db < DB; db++)
@@ -319,7 +328,9 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   __syncthreads();
   if (!held || finite != 0.f || finite != finite) redo = 1;
   __syncthreads();
+  float unscale = kPieceUnscale;
   if (redo) {
+    unscale = 1.f;
     clear();
     load_q();
     for (int k0 = 32 * kg; k0 < k_end; k0 += 32 * KSPLIT) {
@@ -387,7 +398,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   }
 
   const float l_tot = sum_over_wave_halves(l_i);
-  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  const float inv = l_tot > 0.f ? unscale / l_tot : 0.f;
   if (qi < a.Sq) {
     float *op = reinterpret_cast<float *>(a.out) + b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2];
 #pragma unroll
@@ -435,7 +446,7 @@ double prefill_f32_split_cost(const PrefillArgs &a, int *form) {
   static const Cost costs[3][3][2] = {  // [head dims up to 64, 80, 96][form][causal]
       {{{3.3, 1.89, 1.8, 1.33}, {3.6, 1.86, 1.8, 1.40}}, {{1.3, 2.26, 5.7, 0.}, {1.5, 2.13, 6.4, 2.47}}, {{0., 4.26, 8.4, 0.}, {0., 3.98, 8.4, 4.13}}},
       {{{2.6, 2.61, 2.4, 1.76}, {3.3, 2.51, 2.7, 1.85}}, {{0., 3.00, 7.0, 0.}, {0., 2.86, 8.0, 3.28}}, {{0., 4.96, 10.3, 0.}, {0., 4.46, 10.1, 5.47}}},
-      {{{0.2, 3.36, 5.0, 2.28}, {2.3, 3.17, 5.5, 2.19}}, {{0., 3.30, 8.9, 0.}, {0., 3.03, 10.3, 3.44}}, {{0., 5.72, 11.6, 0.}, {0., 5.73, 10.0, 6.74}}}};
+      {{{0.2, 3.36, 5.0, 2.28}, {2.3, 3.17, 5.5, 2.19}}, {{0., 3.30, 8.9, 0.}, {0., 3.03, 10.3, 3.44}}, {{0., 6.3, 11.6, 0.}, {0., 5.73, 10.0, 6.74}}}};
   const int64_t cus = device_cu_count(), heads = (int64_t)a.B * a.Hq, row_tiles = (a.Sk + 63) / 64;
   double least = INFINITY;
   for (int f = 0; f < 3; f++) {

@@ -229,3 +229,32 @@ def test_products_of_operands_in_the_callers_arrays(lm, hip, oracle, M, K, N):
         for t in (x, w, other, out):
             np.testing.assert_array_equal(fed.results[t.id].to_host(), plain.results[t.id].to_host())
         assert np.abs(fed.results[out.id].to_host()).max() > 0
+
+
+@pytest.mark.parametrize("M,K,N", [(590, 580, 1150), (33, 772, 5000), (701, 2052, 2500), (701, 2052, 2000), (1390, 1028, 1450)])
+def test_a_product_left_to_a_small_element(lm, hip, oracle, M, K, N):
+    """One element of a row far below the others of it, and the only one that meets something: its product with all its bits, on
+    every tile that takes bf16 pieces."""
+    x, w = oracle.gen_normal((M, K), 38000 + M), oracle.gen_normal((N, K), 38100 + N)
+    small = [2.0 ** -e for e in (100, 104, 108, 112, 116, 120, 124)]
+    # the column where the rows meet; large values of x's and of w's row in front of it that meet zeros (64 columns apart: a lane
+    # of the kernel reads them all)
+    k, at_x, at_w = 64 * 5 + 9, slice(72, 77), slice(136, 141)
+    x[:, k], w[:, k] = 1 + np.abs(x[:, k]), 1 + np.abs(w[:, k])
+    x[:, at_w], w[:, at_x] = 0, 0
+    for i, e in enumerate(small):
+        x[3 * i], x[3 * i, at_x], x[3 * i, k] = 0, 1.5, 1.2345678 * e
+        w[40 + i], w[40 + i, at_w], w[40 + i, k] = 0, 1.5, -1.1234567 * e
+    out = lm.HipArray((1, M, N), "f32", hip)
+    p = (lm.binding.MatmulParams * 1)()
+    dx, dw = lm.to_device(x[None], hip), lm.to_device(w, hip)
+    assert _low(lm).fill_matmul(p[0], out, dx, dw, transposed=True)
+    lm.binding.matmul(p, 1)
+    got = out.to_host()[0].astype(np.float64)
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    others = np.r_[0:40, 47:N]
+    for i in range(len(small)):  # one product each: its rounding, and that of the pieces left out
+        a, b = got[3 * i, others], want[3 * i, others]
+        assert (np.abs(a - b) <= 2.0 ** -22 * np.abs(b)).all(), small[i]
+        a, b = got[21:, 40 + i], want[21:, 40 + i]
+        assert (np.abs(a - b) <= 2.0 ** -22 * np.abs(b)).all(), small[i]

@@ -205,6 +205,22 @@ def test_attention_on_values_that_pieces_do_not_hold(lm, hip, oracle, causal):
         assert err.max() <= TOL["f32"] * np.abs(want[0, h::8][ok]).max()
 
 
+@pytest.mark.parametrize("Sq,D", [(1000, 80), (1999, 64), (1300, 96)])
+def test_a_result_left_to_a_small_value_on_pieces(lm, hip, oracle, Sq, D):
+    """The first row of a causal launch sees one key: its result is that key's value with all its bits, however far below the other
+    values it lies. Keys and queries as small, beside large ones, change no weight."""
+    q, k, v = inputs(oracle, (1, 40, Sq, D), (1, 8, Sq, D), "f32", 36300)
+    assert "prefill_f32_split_kernel" in plan(lm, q, k, "f32", True, False)
+    for d, e in enumerate((100, 104, 108, 112, 116, 120, 124)):
+        v[0, :, 0, d] *= np.float32(2.0 ** -e)
+        k[0, :, 5 + d::11, d] *= np.float32(2.0 ** -e)
+        q[0, ::3, d::13, d] *= np.float32(2.0 ** -e)
+    got = run(lm, hip, q, k, v, "f32", True)
+    for h in range(40):
+        assert (np.abs(got[0, h, 0] - v[0, h % 8, 0]) <= 2.0 ** -22 * np.abs(v[0, h % 8, 0])).all()
+    assert rel_err(got, oracle.flash_attn(q, k, v, causal=True, nthreads=NT)) <= TOL["f32"]
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
 def test_launches_with_very_many_heads(lm, hip, oracle, dtype):
     """More heads than a 32-bit reciprocal divides exactly: every one of them is computed."""
