@@ -3,10 +3,11 @@
 // Every operand is split into three bf16 pieces (split.hpp); of the nine products of pieces the six with x_i y_j, i + j <= 4, are
 // summed in fp32, the other three are below 2^-25 of x y. Six bf16 products take 6 / 16 of the time of the fp32 one. Error against
 // 64 bits (2-norm): 1.9e-7 where the forms of prefill_f32.hip have 4.3e-7 (S = 1023 D = 80), 1.3e-7 and 2.7e-7 (S = 500 D = 96 causal).
-// V's pieces are scaled, so that a result that is left to a small value has all its bits. Q and K come as they are: what counts of
-// a score is its absolute error, and the bits that their pieces lose lie below 2^-126. A workgroup that meets an infinity, a NaN,
-// queries or keys so large that those bits would count, or an overflow takes its rows again with the fp32 product, straight from
-// memory: a launch all of whose workgroups do takes about five times as long (S = 1023 D = 80, 62 and 297 us).
+// The pieces of V and of the weights are scaled, so that a result that is left to a small value or to small weights has all its
+// bits (not through the exponent of the weights, which is rounded at its own magnitude: 2^-21 of a weight at 24). Q and K come as
+// they are: what counts of a score is its absolute error, and the bits that their pieces lose lie below 2^-126. A workgroup that
+// meets an infinity, a NaN, queries or keys so large that those bits would count, or an overflow takes its rows again with the fp32
+// product, straight from memory: a launch all of whose workgroups do takes about five times as long (S = 1023 D = 80, 62 and 297 us).
 //
 // Same data flow as prefill_mfma.hip: a wave owns 32 query rows with the pieces of its Q fragments in registers, S^T = K Q^T so
 // that a lane holds one query column, and the registers of P, split there, are the B operands of O^T = V^T P^T. Statistics, sums
@@ -286,8 +287,13 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
     for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
       for (int t = 0; t < 2; t++) {
-        pf[kb][t] = split_8((floatx4_t){s[kb][8 * t], s[kb][8 * t + 1], s[kb][8 * t + 2], s[kb][8 * t + 3]},
-                            (floatx4_t){s[kb][8 * t + 4], s[kb][8 * t + 5], s[kb][8 * t + 6], s[kb][8 * t + 7]});
+        floatx4_t lo, hi;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          lo[e] = s[kb][8 * t + e] * kPieceScale;
+          hi[e] = s[kb][8 * t + 4 + e] * kPieceScale;
+        }
+        pf[kb][t] = split_8(lo, hi);
       }
 #pragma unroll
     for (int db = 0; db < DB; db++) {
@@ -328,7 +334,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   __syncthreads();
   if (!held || finite != 0.f || finite != finite) redo = 1;
   __syncthreads();
-  float unscale = kPieceUnscale;
+  float unscale = kPieceUnscale * kPieceUnscale;
   if (redo) {
     unscale = 1.f;
     clear();

@@ -221,6 +221,22 @@ def test_a_result_left_to_a_small_value_on_pieces(lm, hip, oracle, Sq, D):
     assert rel_err(got, oracle.flash_attn(q, k, v, causal=True, nthreads=NT)) <= TOL["f32"]
 
 
+@pytest.mark.parametrize("Sq,D", [(1000, 80), (1999, 64), (1300, 96)])
+def test_a_result_left_to_small_weights_on_pieces(lm, hip, oracle, Sq, D):
+    """One key far ahead of all others whose value is zero: the result is the others', with weights of about 2^-121."""
+    q, k, v = (np.zeros((1, n, Sq, D), np.float32) for n in (40, 8, 8))
+    assert "prefill_f32_split_kernel" in plan(lm, q, k, "f32", False, False)
+    q[..., 0], q[..., 1] = 1, oracle.gen_normal((1, 40, Sq), 36400)
+    k[0, :, 0, 0], k[0, :, 1:, 1] = 84 * np.sqrt(D), oracle.gen_normal((8, Sq - 1), 36401)
+    v[:, :, 1:] = oracle.gen_normal((1, 8, Sq - 1, D), 36402)
+    got = run(lm, hip, q, k, v, "f32", False)
+    s = (k[0].astype(np.float64) @ np.swapaxes(q[0, :8].astype(np.float64), 1, 2)).swapaxes(1, 2) * np.float64(np.float32(lm.default_scale(D)))
+    w = np.exp(s - s.max(-1, keepdims=True))
+    want = (w / w.sum(-1, keepdims=True)) @ v[0].astype(np.float64)
+    # an exponent of 121 comes with an error of 2^-18 relative to one of them
+    assert np.linalg.norm(got[0, :8] - want) <= 2.0 ** -17 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
 def test_launches_with_very_many_heads(lm, hip, oracle, dtype):
     """More heads than a 32-bit reciprocal divides exactly: every one of them is computed."""
