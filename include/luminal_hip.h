@@ -202,7 +202,8 @@ typedef struct lmh_decode_params {
   float scale;
   int32_t head_map;
   int32_t out_f32;       /* 0: out has element type `dtype`; 1: out is fp32 */
-  int32_t num_splits;    /* KV splits per (b, kv head); 0 = choose */
+  int32_t num_splits;    /* KV splits per (b, kv head); 0 = choose, by the sizes and the device's compute units: the sums
+                          * of another count or on another device are the same to fp32 rounding, not bit for bit */
   void *workspace;       /* device, 16-byte aligned, >= lmh_decode_workspace_bytes(...) */
   size_t workspace_bytes;
   void *stream;

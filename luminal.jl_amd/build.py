@@ -24,6 +24,12 @@ LIBRARIES = {
     CALIB_LIBNAME: ["calib.hip"],
 }
 
+# Flags of single files. -amdgpu-mfma-vgpr-form: the compiler otherwise leaves the products in the accumulation registers and
+# moves them out one by one, a quarter of the instructions of a block of 32 keys.
+FILE_FLAGS = {
+    "decode_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+}
+
 # Sources that only a measurement build contains: switch in LMH_EXTRA_FLAGS -> (source, flags for that file alone).
 # -amdgpu-mfma-vgpr-form: with one wave per SIMD the compiler otherwise keeps every MFMA result in the accumulation
 # registers and moves the scores out of them one by one.
@@ -70,7 +76,7 @@ def build_library(verbose=True):
     objdir = os.path.join(LIBDIR, "obj")
     os.makedirs(objdir, exist_ok=True)
     procs = []
-    file_flags = {}
+    file_flags = dict(FILE_FLAGS)
     libraries = {name: list(sources) for name, sources in LIBRARIES.items()}
     for switch, (src, src_flags) in MEASUREMENT_SOURCES.items():
         if switch in flags:

@@ -4,9 +4,9 @@
 // On the vector ALUs the 2*G flops per cache element (plus 16-bit unpacking and the cross-lane
 // dot-product reductions) keep the VALUs ~60 % busy at 5 TB/s, which caps the kernel below the
 // memory roofline. The matrix cores are otherwise idle, so the G query heads of a KV head are
-// padded to a 16-wide MFMA operand and both products run as v_mfma_f32_16x16x32: per 32 keys a
-// wave then issues 16 MFMAs and ~100 VALU instructions instead of ~900, and the kernel is left
-// waiting on memory only. (Same semantics as decode.hip: reference src/Whisper.jl:584-620 with the
+// padded to a 16-wide MFMA operand and both products run as v_mfma_f32_16x16x32: per 32 keys of
+// head dim 128 a wave then issues 16 MFMAs and ~200 VALU instructions instead of ~900, and the
+// kernel is left waiting on memory only. (Same semantics as decode.hip: reference src/Whisper.jl:584-620 with the
 // GQA head sharing of src/NN.jl:305-317.)
 //
 // Data flow per wave, 32 keys at a time (each wave owns a private LDS region, so the loop has no
@@ -17,8 +17,11 @@
 //   online softmax on the accumulator: lane (head n, g) holds keys 4g..4g+3 of each 16-key half; the
 //   4 lanes of a head agree on the max through two lane exchanges
 //   O^T[d, head] += V^T P^T : A = V^T fragment via the transposing LDS read ds_read_b64_tr_b16,
-//   B = P^T = the softmax registers converted to 16 bit (never leaves the register file), as a
-//   head + remainder pair so that P keeps ~16 significant bits
+//   B = P^T = the softmax registers converted to 16 bit (never leaves the register file), as two (fp16)
+//   or three (bf16) pieces so that P keeps 22 or 24 significant bits. Up to 8 (5) query heads per KV head
+//   the pieces are columns of one product (COLUMNS); as products of their own the third took a walk of 512
+//   keys from 10.5 to 11.2 us. Error of fp32 results against 64 bits (2-norm), L = 512 D = 128: bf16
+//   1.6e-7 (two pieces: 1.9e-6), fp16 1.9e-7
 //
 // Scheduling: a rectangular (split, kv head, batch) grid wastes a ragged batch twice — workgroups
 // whose split lies past kv_len[b] still have to be dispatched (≈40 % of the grid for lengths spread
@@ -29,6 +32,8 @@
 // one (b, kv head) with a single softmax state, so partials are written once per run, not once per
 // chunk (the other chunk slots of the run get an "empty" marker the merge kernel skips).
 // Split-KV partial layout and the merge kernel are shared with decode.hip.
+#include <algorithm>
+
 #include "common.hpp"
 #include "dtypes.hpp"
 #include "rope.hpp"
@@ -44,6 +49,8 @@ typedef short shortx8_t __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) shortx4_t lds_shortx4_t;
 
 struct Mfma16F16 {
+  static constexpr int kPieces = 2;
+  static constexpr float kScale = 16384.f;  // of the weights: the second piece of one below 2^-3 would be subnormal
   using vec8 = half8_t;
   __device__ static floatx4_t mfma(vec8 a, vec8 b, floatx4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -52,6 +59,8 @@ struct Mfma16F16 {
   __device__ static uint16_t cvt_bits(float x) { return __builtin_bit_cast(uint16_t, (_Float16)x); }
 };
 struct Mfma16BF16 {
+  static constexpr int kPieces = 3;
+  static constexpr float kScale = 1.f;
   using vec8 = bf16x8_t;
   __device__ static floatx4_t mfma(vec8 a, vec8 b, floatx4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -70,7 +79,9 @@ __device__ inline void wave_lds_fence() {
 
 constexpr int kMaxBatchPersistent = 1024;  // prefix sums live in LDS
 
-template <typename MT, int D>
+// COLUMNS: the pieces of a head's weights are columns of one product. The 16 columns hold the heads of a slice kPieces times, so
+// that their scores come out once per copy; the lanes of copy x take piece x, and the copies of O are added where the waves' are.
+template <typename MT, int D, bool COLUMNS>
 __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, int g_chunks) {
   request_args(a);
   request_arg(g_chunks);
@@ -168,9 +179,11 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
 
   // Q^T fragments (B operand): lane (head n, g) holds q[head][32*ks + 8*g .. +7]; zero for padding heads
   vec8 qreg[KS];
+  const int copy = COLUMNS ? n / n_heads : 0;
   {
-    const bool head_ok = n < n_heads;
-    const int hq = q_head_of(kvh, head_ok ? g0 + n : 0, a.Hq, a.Hkv, a.head_map);
+    const int head = n - copy * n_heads;
+    const bool head_ok = COLUMNS ? copy < MT::kPieces : n < n_heads;
+    const int hq = q_head_of(kvh, head_ok ? g0 + head : 0, a.Hq, a.Hkv, a.head_map);
     const uint16_t *qp = reinterpret_cast<const uint16_t *>(a.q) + b * a.qs[0] + hq * a.qs[1];
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
@@ -186,7 +199,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
   floatx4_t oacc[DB];
 #pragma unroll
   for (int db = 0; db < DB; db++) oacc[db] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-  float m_i = -INFINITY;  // running max of the raw scores of head n (same in the 4 lanes of a head)
+  float m_i = -INFINITY;  // running max of the scores of head n in log2 units, as the weights have it (same in the 4 lanes of a head)
   float l_i = 0.f;        // this lane's share of the running sum
 
   // Raw buffer descriptors over the valid rows [0, end) of this (b, kv head) slice: a load past `end` returns zeros
@@ -284,37 +297,56 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
                      fmaxf(fmaxf(sacc[1][0], sacc[1][1]), fmaxf(sacc[1][2], sacc[1][3])));
     mx = fmaxf(mx, __shfl_xor(mx, 16));
     mx = fmaxf(mx, __shfl_xor(mx, 32));
-    const float m_new = fmaxf(m_i, mx);  // finite: key0 < end, so every head sees a key in this block
-    const float alpha = __builtin_amdgcn_exp2f((m_i - m_new) * c);
-    const float mc = m_new * c;
-    m_i = m_new;
-    // P is split into a 16-bit head and a 16-bit remainder (p = hi + lo to ~16 significant bits) and
-    // both are multiplied with V: the matrix cores have time to spare here, and it keeps the result
-    // independent of where the split boundaries fall to ~1e-5 instead of the 2^-9 of a single bf16 P.
+    // (finite: key0 < end, so every head sees a key in this block.) The product is rounded before anything is subtracted from it:
+    // old and new weights then differ by exactly the factor alpha, whatever the rounding
+    const float mc = fmaxf(m_i, mx * c);
+    const float alpha = __builtin_amdgcn_exp2f(m_i - mc);
+    m_i = mc;
+    // P is split into 16-bit pieces that hold all of it that fp32 sums see (two of fp16, 22 bits, or three of bf16, 24), and each is
+    // multiplied with V: the matrix cores have time to spare here, and the result depends on where the split boundaries fall by
+    // fp32 roundings only.
     float psum = 0.f;
-    vec8 pf, pf_lo;
+    vec8 pf[COLUMNS ? 1 : MT::kPieces];
 #pragma unroll
     for (int hb = 0; hb < 2; hb++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const float p = __builtin_amdgcn_exp2f(sacc[hb][i] * c - mc);
         psum += p;
-        pf[4 * hb + i] = MT::cvt(p);
-        pf_lo[4 * hb + i] = MT::cvt(p - (float)pf[4 * hb + i]);
+        float rest = p * MT::kScale;
+#pragma unroll
+        for (int x = 0; x < MT::kPieces; x++) {
+          const auto piece = MT::cvt(rest);
+          rest -= (float)piece;
+          if (!COLUMNS || x == 0 || copy >= x) pf[COLUMNS ? 0 : x][4 * hb + i] = piece;
+        }
       }
     l_i = l_i * alpha + psum;
 #pragma unroll
     for (int db = 0; db < DB; db++) oacc[db] *= alpha;
 
-    // ---- O^T += V^T P^T ----
+    // ---- O^T += V^T P^T: a block's share from zero, the first pieces apart from the others, added once ----
+    constexpr int GB = DB % 8 == 0 ? 8 : DB;  // row blocks whose products are on their way together
 #pragma unroll
-    for (int db = 0; db < DB; db++) {
-      const uint16_t *vaddr = &Vs[v_frag_off + 16 * db];
-      const shortx4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(vaddr));
-      const shortx4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(vaddr + 16 * LDV));
-      const shortx8_t v8 = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-      oacc[db] = MT::mfma(__builtin_bit_cast(vec8, v8), pf, oacc[db]);
-      oacc[db] = MT::mfma(__builtin_bit_cast(vec8, v8), pf_lo, oacc[db]);
+    for (int b0 = 0; b0 < DB; b0 += GB) {
+      floatx4_t o[GB], rest[GB];
+#pragma unroll
+      for (int i = 0; i < GB; i++) {
+        const uint16_t *vaddr = &Vs[v_frag_off + 16 * (b0 + i)];
+        const shortx4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(vaddr));
+        const shortx4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(vaddr + 16 * LDV));
+        const vec8 v8 = __builtin_bit_cast(vec8, (shortx8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        o[i] = MT::mfma(v8, pf[0], floatx4_t{0.f, 0.f, 0.f, 0.f});
+        if constexpr (!COLUMNS) {
+          rest[i] = MT::mfma(v8, pf[MT::kPieces - 1], floatx4_t{0.f, 0.f, 0.f, 0.f});
+          if (MT::kPieces == 3) rest[i] = MT::mfma(v8, pf[1], rest[i]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < GB; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) oacc[b0 + i][e] += COLUMNS ? o[i][e] : o[i][e] + rest[i][e];
     }
   }
 
@@ -328,9 +360,9 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
 #pragma unroll
   for (int db = 0; db < DB; db++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) sm_o[(wave * 16 + n) * D + 16 * db + 4 * g + i] = oacc[db][i];
+    for (int i = 0; i < 4; i++) sm_o[(wave * 16 + n) * D + 16 * db + 4 * g + i] = oacc[db][i] * (1.f / MT::kScale);
   if (g == 0) {
-    sm_m[wave * 16 + n] = m_i * c;  // log2 units, like the vector kernel's partials
+    sm_m[wave * 16 + n] = m_i;
     sm_l[wave * 16 + n] = l_i;
   }
   __syncthreads();
@@ -346,7 +378,13 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
       const float mw = sm_m[w * 16 + h];
       const float f = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - M);
       lsum += sm_l[w * 16 + h] * f;
-      o += sm_o[(w * 16 + h) * D + d] * f;
+      float x = sm_o[(w * 16 + h) * D + d];
+      if constexpr (COLUMNS) {
+        float rest = sm_o[(w * 16 + (MT::kPieces - 1) * n_heads + h) * D + d];
+        if (MT::kPieces == 3) rest += sm_o[(w * 16 + n_heads + h) * D + d];
+        x += rest;
+      }
+      o += x * f;
     }
     const int hq = q_head_of(kvh, g0 + h, a.Hq, a.Hkv, a.head_map);
     if (a.num_splits == 1) {
@@ -389,28 +427,35 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
   }
 }
 
-template <typename MT, int D>
-int launch_for_d(const DecodeArgs &a, hipStream_t stream) {
-  // Persistent launch: as many workgroups as the chip holds at once (never more than there are units).
-  // Same for every device this library runs on (gfx950 only); initialised once, thread-safely.
-  static const int wgs_per_device = [] {
-    int dev = 0, per_cu = 0;
-    hipDeviceProp_t prop;
-    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_mfma_kernel<MT, D>, kWaves * 64, 0) != hipSuccess) {
+template <typename MT, int D, bool COLUMNS>
+int launch_form(const DecodeArgs &a, hipStream_t stream) {
+  // Persistent launch: as many workgroups as the chip holds at once (never more than there are units). Same for every device this
+  // library runs on (gfx950 only); initialised once, thread-safely.
+  static const int per_cu = [] {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, decode_mfma_kernel<MT, D, COLUMNS>, kWaves * 64, 0) != hipSuccess) {
       (void)hipGetLastError();
-      return 256;  // one workgroup per CU: correct for any value, only the balance changes
+      return 1;  // correct for any value, only the balance changes
     }
-    return (per_cu < 1 ? 1 : per_cu) * prop.multiProcessorCount;
+    return n < 1 ? 1 : n;
   }();
+  // With several splits every further workgroup is a further partial row for the merge to read: one per CU, two up to head dim 96
+  // (bf16 steps D = 128 B=32 L=1024: 30.8 us, 32.2 with two). With one split, as many as fit (fp16 B=64 L=512 ragged 20.1 and 22.4).
+  const int wgs_per_device = device_cu_count() * (a.num_splits > 1 ? std::min(per_cu, D > 96 ? 1 : 2) : per_cu);
   const int group = a.Hq / a.Hkv;
   const int g_chunks = (group + 15) / 16;
   const int64_t max_units = (int64_t)a.B * a.Hkv * g_chunks * a.num_splits;
   if (max_units >= (int64_t(1) << 31)) return fail(LMH_E_UNSUPPORTED, "MFMA decode: %lld units do not fit 32 bits", (long long)max_units);
   const int n_wgs = (int)(max_units < wgs_per_device ? max_units : wgs_per_device);
-  hipLaunchKernelGGL((decode_mfma_kernel<MT, D>), dim3(n_wgs), dim3(kWaves * 64), 0, stream, a, g_chunks);
+  hipLaunchKernelGGL((decode_mfma_kernel<MT, D, COLUMNS>), dim3(n_wgs), dim3(kWaves * 64), 0, stream, a, g_chunks);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
+}
+
+template <typename MT, int D>
+int launch_for_d(const DecodeArgs &a, hipStream_t stream) {
+  if (a.Hq / a.Hkv * MT::kPieces <= 16) return launch_form<MT, D, true>(a, stream);
+  return launch_form<MT, D, false>(a, stream);
 }
 
 template <typename MT>

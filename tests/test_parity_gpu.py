@@ -1033,3 +1033,26 @@ def test_decode_random_shapes_and_options(lm, hip, oracle, seed):
     want = oracle.decode_attn(q, k, v, kv_len=lens, head_map=head_map, nthreads=NT)
     assert rel_err(got, want) <= TOL[dtype], dict(dtype=dtype, D=D, B=B, Hq=Hq, Hkv=Hkv, L=L, head_map=head_map, splits=splits,
                                                    lens=None if lens is None else lens.tolist())
+
+
+@pytest.mark.parametrize("dtype,D,group,L", [
+    ("bf16", 128, 1, 512), ("bf16", 128, 4, 200), ("bf16", 64, 5, 512), ("bf16", 96, 6, 500), ("bf16", 256, 17, 300),
+    ("f16", 64, 1, 512), ("f16", 128, 3, 200), ("f16", 96, 8, 500), ("f16", 64, 9, 512), ("f16", 256, 33, 300), ("f16", 64, 4, 20000),
+])
+def test_decode_is_no_less_exact_where_the_library_chooses_the_splits(lm, hip, oracle, dtype, D, group, L):
+    """fp32 results of both split counts against 64 bits, with the pieces of the weights as columns of one product and not. A score,
+    a weight and a sum are rounded to fp32, each by up to 2^-24 of itself: 2^-21 of the result for all of them."""
+    B, Hkv = 4, 4
+    err = {}
+    for seed in range(3):
+        q, k, v = (oracle.round_to(oracle.gen_normal(s, 9600 + 3 * seed + i), dtype)
+                   for i, s in enumerate(((B, Hkv * group, D), (B, Hkv, L, D), (B, Hkv, L, D))))
+        heads = np.arange(Hkv * group) % Hkv
+        s = np.matmul(k.astype(np.float64)[:, heads], q.astype(np.float64)[..., None])[..., 0] * np.float64(np.float32(lm.default_scale(D)))
+        w = np.exp(s - s.max(-1, keepdims=True))
+        want = np.matmul((w / w.sum(-1, keepdims=True))[:, :, None], v.astype(np.float64)[:, heads])[:, :, 0]
+        for splits in (0, lm.binding.decode_auto_splits(B, Hkv, L)):
+            got = run_decode(lm, hip, q, k, v, dtype, num_splits=splits, out_dtype="f32")
+            err[splits] = err.get(splits, 0) + np.linalg.norm(got - want) / np.linalg.norm(want) / 3
+    few, many = err.values()
+    assert many <= 2.0 ** -21 and few <= 1.05 * many, err
