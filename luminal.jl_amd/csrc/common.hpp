@@ -207,7 +207,7 @@ int launch_prefill_w64(const PrefillArgs &a, hipStream_t stream);
 #endif
 bool prefill_f32_mfma_supported(int dtype, int D);
 int launch_prefill_f32_mfma(const PrefillArgs &a, hipStream_t stream);
-int launch_prefill_f32_full(const PrefillArgs &a, int key_groups, hipStream_t stream);  // no mask, head dim <= 128
+int launch_prefill_f32_full(const PrefillArgs &a, int key_groups, hipStream_t stream);  // no mask, head dim <= 128; two groups above 96
 double prefill_f32_split_cost(const PrefillArgs &a, int *form);  // head dim <= 96: microseconds of its cheapest form
 int launch_prefill_f32_split(const PrefillArgs &a, int form, hipStream_t stream);
 int launch_prefill_valu(const PrefillArgs &a, int dtype, hipStream_t stream);

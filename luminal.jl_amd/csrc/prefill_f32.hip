@@ -363,7 +363,7 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
   } else {
     // Without a mask, in blocks of 32 x 32 (prefill_f32_full.hip), where the head dim needs no more padding for it: a wave walks
     // twice the rows per key. Weights from launches that fill the chip (D=96, B=1 H=32 S=1024: 106 us against 113 for the
-    // 128-row form here, two key groups on B=1 H=16 S=1024 61 against 68).
+    // 128-row form here; D=128, two key groups on B=1 H=16 S=1024 78 against 89).
     constexpr bool kFull = D == 64 || D == 96 || D == 128;
     double f128 = INFINITY, f64 = INFINITY;
     if (kFull && !a.causal) {
@@ -371,23 +371,25 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
         return weight * (double)((a.Sk + tile - 1) / tile) * tile * (rows / 64) * ceil((double)tiles(rows) / n_cus);
       };
       f128 = cost(128, 32, 0.92);
-      f64 = cost(64, 64, tiles(64) <= n_cus ? 1.07 : INFINITY);
+      if (D == 128 && tiles(64) <= n_cus) f64 = cost(64, 64, 1.07);  // (narrower ones of more than 256 keys go over to the pieces)
     }
     const bool many = tiles(128) >= 4 * n_cus;
     const double c128 = form_cost<D, 8, 1, 2>(a, 0.96);
     // In bf16 pieces (prefill_f32_split.hip), up to head dim 96: by the time that the cost of the form here stands for, in us (a part
     // per launch, a part per key of the walk; fitted to 240 launches of drawn sizes, rms 2 to 13 %). Of 330 such launches 159 go
-    // over, none loses more than 4 %, and together the 330 gain 12 %: B=2 H=12 S=1023 D=80 without a mask 75.5 -> 57 us, B=1 H=32
-    // S=2048 D=96 380 -> 233, causal 214 -> 146. The small launches stay because their waves walk the keys alone (B=1 H=6 S=846
-    // D=96 causal); so do, though they would gain as well, rows of up to five key tiles without a mask and causal launches of
-    // up to two rounds at the tiling for 64, where the tests of the forms here reach those forms (B=3 H=4 1844 x 304 D=64
-    // 23.3 us here, 18.8 there; B=1 H=48 S=1100 D=64 causal 79 and 58).
+    // over, none loses more than 4 %, and together the 330 gain 12 %: B=2 H=12 S=1023 D=80 without a mask 76 -> 57 us, B=1 H=32
+    // S=2048 D=96 380 -> 255, causal 214 -> 150, B=1 H=48 S=1100 D=64 causal 79 -> 58. The small launches stay because their waves
+    // walk the keys alone (B=1 H=6 S=846 D=96 causal), and without a mask what the pieces would take less than 14.5 us for, where
+    // the fit overrates the forms here: D=72 to 96 on up to 170 keys 4 to 14 us here, up to 2 times that there (H=12 502 x 167
+    // D=72 13.5 and 14.0), while above it 55 of 60 drawn launches of up to 340 keys gain (20 x 300 x 119 D=80, B=4, 28.9 -> 21.2) and
+    // the worst loses 7 % (H=4 1981 x 163 D=96, B=2, 16.3 and 17.5).
     auto pieces = [&](double here, int *form) {
-      if (D > 96 || (!a.causal && a.Sk <= 320) || (a.causal && D <= 64 && tiles(128) <= 2 * n_cus)) return false;
+      if (D > 96) return false;
       constexpr double fit[5][2][2] = {{{6.6, 0.0178}, {4.3, 0.0197}}, {{6.1, 0.0249}, {5.1, 0.0277}}, {{5.6, 0.0352}, {5.7, 0.0351}},
                                        {{7.5, 0.0419}, {6.4, 0.0451}}, {{6.2, 0.0527}, {8.6, 0.0505}}};  // D = 32, 48, 64, 80, 96
       const auto &f = fit[D <= 96 ? D / 16 - 2 : 0][a.causal != 0];
-      return prefill_f32_split_cost(a, form) < 0.95 * (f[0] + f[1] * here);
+      const double split = prefill_f32_split_cost(a, form);
+      return (a.causal || split >= 14.5) && split < 0.95 * (f[0] + f[1] * here);
     };
     int split_form = 0;
     if (many && pieces(kFull && !a.causal ? f128 : c128, &split_form)) return launch_prefill_f32_split(a, split_form, stream);

@@ -4,7 +4,7 @@
 // round of workgroups fills the chip, the larger block wins, because it reads half as much from LDS per product (a 128-bit K
 // fragment feeds 32 rows instead of 16, a V fragment as well) at the same rate of the matrix pipe. Measured, us, the best of the
 // 16 x 16 forms against this file: B=1 H=32 S=1024 D=64 86 -> 76, D=96 113 -> 106, D=128 146 -> 136; H=8 S=4096 D=96 410 -> 404,
-// D=128 537 -> 519; B=1 H=16 S=1024 (two key groups) D=96 68 -> 61, D=128 89 -> 78. Where the rows or the head dim do not fill
+// D=128 537 -> 519; B=1 H=16 S=1024 (two key groups) D=128 89 -> 78. Where the rows or the head dim do not fill
 // the blocks the smaller ones stay ahead (B=2 H=12 S=1023 D=96 105 here, 92 there; D=80 padded to 96 104 here, 94 there), and so
 // they do under the causal mask; launch_for_d in prefill_f32.hip compares the two. Error against 64 bits: that of the 16 x 16 forms
 // with as many key groups (0.99 to 1.00 of it over drawn shapes), 5 to 8e-7 in the 2-norm at 1000 to 2000 keys.
@@ -305,8 +305,8 @@ int launch_form(const PrefillArgs &a, hipStream_t stream) {
 }  // namespace
 
 int launch_prefill_f32_full(const PrefillArgs &a, int key_groups, hipStream_t stream) {
-  if (a.D <= 64) return key_groups == 2 ? launch_form<64, 2>(a, stream) : launch_form<64, 1>(a, stream);
-  if (a.D <= 96) return key_groups == 2 ? launch_form<96, 2>(a, stream) : launch_form<96, 1>(a, stream);
+  if (a.D <= 64) return launch_form<64, 1>(a, stream);
+  if (a.D <= 96) return launch_form<96, 1>(a, stream);
   return key_groups == 2 ? launch_form<128, 2>(a, stream) : launch_form<128, 1>(a, stream);
 }
 

@@ -15,7 +15,7 @@ NT = 16
     (1, 2, 1, 33, 65, 16, False, "D=32, full, key groups=4> rows=16"), (1, 3, 3, 129, 70, 40, False, "D=48, full, key groups=4> rows=16"),
     (2, 32, 8, 135, 131, 64, True, "D=64, causal, key groups=2> rows=32"), (2, 40, 8, 100, 65, 72, True, "D=80, causal, key groups=2> rows=32"),
     (3, 32, 8, 500, 17, 80, False, "D=80, full, key groups=1> rows=64"), (3, 24, 24, 260, 100, 112, False, "D=112, full, key groups=1> rows=128"),
-    (8, 48, 16, 257, 33, 128, True, "D=128, causal, key groups=1> rows=128"), (1, 16, 4, 1100, 1100, 96, True, "D=96, causal, key groups=2> rows=32"), (1, 48, 4, 1100, 1100, 64, True, "D=64, causal, key groups=1> rows=64"),
+    (8, 48, 16, 257, 33, 128, True, "D=128, causal, key groups=1> rows=128"), (1, 16, 4, 1100, 1100, 96, True, "D=96, causal, key groups=2> rows=32"), (5, 30, 10, 244, 244, 64, True, "D=64, causal, key groups=1> rows=64"),
     (2, 20, 4, 637, 29, 256, False, "D=256, full, key groups=1> rows=64"),
     (1, 4, 2, 100, 300, 144, True, "D=160, causal, key groups=2> rows=32"), (1, 2, 2, 1, 1, 192, False, "D=192, full, key groups=1> rows=64"),
 ])
@@ -110,9 +110,8 @@ def test_head_counts_that_are_no_multiple_of_the_xcds(lm, hip, oracle, B, Hq, Hk
 
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,form", [
     (1, 32, 8, 1000, 40, 64, "D=64, key groups=1> rows=128"), (2, 15, 15, 970, 65, 56, "D=64, key groups=1> rows=128"),
-    (4, 16, 4, 500, 33, 96, "D=96, key groups=1> rows=128"), (1, 31, 1, 1024, 97, 88, "D=96, key groups=1> rows=128"),
+    (4, 16, 4, 500, 33, 96, "D=96, key groups=1> rows=128"), (1, 31, 1, 1024, 65, 88, "D=96, key groups=1> rows=128"),
     (8, 32, 32, 127, 64, 128, "D=128, key groups=1> rows=128"), (3, 10, 5, 1001, 95, 120, "D=128, key groups=1> rows=128"),
-    (2, 8, 2, 1000, 320, 64, "D=64, key groups=2> rows=64"), (1, 16, 8, 993, 319, 96, "D=96, key groups=2> rows=64"),
     (3, 7, 7, 640, 320, 128, "D=128, key groups=2> rows=64"),
 ])
 def test_fp32_without_a_mask_in_blocks_of_32(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, form):
@@ -159,7 +158,9 @@ PIECES = [(2, 16, 16, 300, 1000, 64, False, "D=64, full, key groups=2> rows=64")
           (3, 16, 4, 700, 500, 72, False, "D=80, full, key groups=1> rows=256"), (2, 33, 3, 513, 500, 96, False, "D=96, full, key groups=1> rows=256"),
           (2, 12, 4, 1023, 401, 80, False, "D=80, full, key groups=2> rows=128"), (2, 20, 20, 300, 700, 88, False, "D=96, full, key groups=2> rows=64"),
           (2, 33, 11, 1000, 1000, 80, True, "D=80, causal, key groups=2> rows=64"), (1, 32, 8, 1300, 1300, 96, True, "D=96, causal, key groups=2> rows=128"),
-          (5, 33, 33, 900, 900, 64, True, "D=64, causal, key groups=1> rows=256")]
+          (5, 33, 33, 900, 900, 64, True, "D=64, causal, key groups=1> rows=256"), (1, 48, 4, 1100, 1100, 64, True, "D=64, causal, key groups=2> rows=64"),
+          (2, 8, 2, 1000, 320, 64, False, "D=64, full, key groups=2> rows=64"), (1, 16, 8, 993, 319, 96, False, "D=96, full, key groups=2> rows=64"),
+          (1, 31, 1, 1024, 97, 88, False, "D=96, full, key groups=2> rows=128")]
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,form", PIECES)
