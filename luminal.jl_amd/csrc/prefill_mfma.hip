@@ -1626,10 +1626,9 @@ int launch_cheapest(const PrefillArgs &a, const QueryCopy &queries, int by_size,
   auto cost = [&](bool v, int form) {
     const FormCost &f = kFormCosts[!MT::kSplitP ? 0 : v ? 2 : 1][tiling][form][a.causal != 0];
     if (f.fixed < 0 || (form >= kRows256 && a.Sq <= 128)) return 1e30;
-    // up to 16 workgroups stay on 128 rows, which the tests of the rotation in registers expect of one such launch; so do up to 64
-    // rows of one or two key tiles, which are as many workgroups either way (B=3 H=20 Sq=35 Sk=112 D=40 fp16 4.56 against 4.74 us)
-    if (form == kKeysSplit64 && by_size != form &&
-        ((int64_t)a.B * a.Hq * ((a.Sq + 63) / 64) <= 16 || (a.Sq <= 64 && a.Sk <= 2 * BN))) return 1e30;
+    // one row tile and one key tile in fp16 are as many workgroups either way, and no fold (recorded back to back, H=2 S=45 D=128
+    // 5.15 against 5.34 us, D=64 3.68 and 3.72; on two key tiles 64 rows are ahead, 5.08 and 5.27)
+    if (form == kKeysSplit64 && by_size != form && !MT::kSplitP && a.Sq <= 64 && a.Sk <= BN) return 1e30;
     return form_cost(f, a, form, form == kRows256 ? 1 : form == kRows256Pair || D > 96 ? 2 : 3, n_cus);
   };
   int best = by_size;

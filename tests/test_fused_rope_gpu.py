@@ -60,7 +60,8 @@ def inputs(oracle, shape_q, shape_kv, dtype, seed, mul=1.0):
 
 # (B, Hq, Hkv, Sq, Sk, D, causal, dtype, part of the kernel name the launch must reach)
 CASES = [
-    (1, 8, 2, 96, 96, 64, True, "f16", "prefill_mfma_kernel<f16, D=64, causal, key groups=1"),
+    (1, 8, 2, 61, 61, 64, True, "f16", "prefill_mfma_kernel<f16, D=64, causal, key groups=1"),
+    (1, 8, 2, 96, 96, 64, True, "f16", "prefill_mfma_kernel<f16, D=64, causal, key groups=2"),
     (1, 4, 4, 300, 300, 96, True, "f16", "prefill_mfma_kernel<f16, D=96, causal, key groups=2"),
     (2, 4, 2, 200, 333, 128, False, "bf16", "prefill_mfma_kernel<bf16, D=128, full"),
     (1, 48, 8, 2048, 2048, 96, True, "f16", "waves=8"),
