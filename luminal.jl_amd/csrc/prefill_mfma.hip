@@ -1744,8 +1744,10 @@ int launch_for_d(const PrefillArgs &a, const QueryCopy &queries, hipStream_t str
 // mask, whole rounds without one) and the workgroups it starts, each worth five tiles of the first form. A tile takes 1.4 and 1.2
 // times as long in the other two, a start of the third six tiles. Fitted to 386 drawn launches (fp16 and bf16, head dims 160 to
 // 256, 16 to 8192 rows, 1 to 64 heads, with every form timed on each): within 0.7 % of the best form on average, where the
-// comparison of the tiles alone is 5 % behind it. That one, in which 64 rows have to be 10 % cheaper to be left (fp16 from 12 tiles
-// on stays on eight waves), was measured with the shorter loop and still chooses for it.
+// comparison of the tiles alone is 5 % behind it. (fp16 launches whose 64-row and 128-row workgroups walk the same 12 tiles or more are
+// in it too: of 60 such the 46 with a mask, up to 50 workgroups, take 19 to 37 % less time in the 64-row form than on eight waves, H=2/1
+// S=1537 D=208 44.4 and 31.2 us; the 14 without one from -5 to +11 %.) That comparison, in which 64 rows have to be 10 % cheaper to be
+// left (fp16 from 12 tiles on takes 128), was measured with the shorter loop and still chooses for it.
 // B=1 H=32 S=4096 D=256 causal fp16 takes 292 us = 940 TFLOP/s (363 with 128 rows on four waves as the only form).
 // bf16 keeps head + remainder weights at every length: the registers of the fp16 rewrite of V spill here (S=4096: 633 us).
 // The head dims that are odd multiples of 8 stay on the vector-ALU kernel.
@@ -1760,19 +1762,14 @@ int launch_wide_heads(const PrefillArgs &a, const QueryCopy &queries, hipStream_
     const double longest = (double)std::min(row_tiles, n * s), mean = (double)heads * (s * ramp * (ramp + 1) / 2 + (n - ramp) * row_tiles) / cus;
     return std::max(longest, mean) * tile + std::max(1., (double)(heads * n) / cus) * start;
   };
-  const double s64 = cost(64, 1., 0.), s128 = cost(128, 1., 0.);
-  const bool even = !MT::kSplitP && s128 >= 12;
   if (row_tiles <= 2) {
-    if (s128 > 0.9 * s64 && !even) return launch_split<MT, false, D, 2, 4>(a, queries, stream);
+    const double s64 = cost(64, 1., 0.), s128 = cost(128, 1., 0.);
+    if (s128 > 0.9 * s64 && (MT::kSplitP || s128 < 12)) return launch_split<MT, false, D, 2, 4>(a, queries, stream);
     return launch_split<MT, false, D, 1, 4>(a, queries, stream);
   }
   const double rows64 = cost(64, 1., 5.), rows128 = cost(128, 1.4, 5.), eight = cost(128, 1.2, 6.);
-  // fp16 launches that come out even stay on eight waves where the tests of that form expect it of one such launch: with a mask up
-  // to 50 workgroups of 64 rows, without one from a second round of them on
-  const int64_t wgs64 = heads * ((a.Sq + 63) / 64);
-  const bool stays = even && s128 == s64 && (a.causal ? wgs64 <= 50 : wgs64 > cus);
-  if (!stays && rows64 <= std::min(rows128, eight)) return launch_split<MT, false, D, 2, 4, 1, true>(a, queries, stream);
-  if (!stays && rows128 < 0.98 * eight) return launch_split<MT, false, D, 1, 4, 1, true>(a, queries, stream);
+  if (rows64 <= std::min(rows128, eight)) return launch_split<MT, false, D, 2, 4, 1, true>(a, queries, stream);
+  if (rows128 < 0.98 * eight) return launch_split<MT, false, D, 1, 4, 1, true>(a, queries, stream);
   return launch_split<MT, false, D, 2, 8, 2>(a, queries, stream);
 }
 

@@ -50,7 +50,7 @@ def test_large_launch_of_wide_heads(lm, hip, oracle):
 
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,dtype", [
     (2, 40, 8, 385, 385, 256, True, "f16"), (3, 40, 4, 257, 330, 256, False, "bf16"), (1, 80, 8, 513, 481, 144, True, "bf16"),
-    (5, 32, 8, 129, 321, 192, False, "f16"), (1, 2, 1, 1537, 1537, 208, True, "f16"), (4, 33, 3, 300, 511, 256, True, "bf16"),
+    (5, 40, 8, 127, 321, 192, False, "f16"), (1, 40, 8, 1025, 1025, 208, True, "f16"), (4, 33, 3, 300, 511, 256, True, "bf16"),
 ])
 def test_eight_waves_on_wide_heads(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causal, dtype):
     q, k, v = inputs(oracle, (B, Hq, Sq, D), (B, Hkv, Sk, D), dtype, 32970 + Sq + D)
@@ -68,6 +68,7 @@ def test_eight_waves_on_wide_heads(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causa
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,dtype,groups", [
     (2, 6, 2, 129, 129, 144, True, "bf16", 2), (5, 4, 4, 65, 321, 256, False, "f16", 2), (1, 16, 8, 700, 700, 208, True, "f16", 2),
     (2, 6, 2, 257, 500, 192, True, "bf16", 2), (3, 48, 2, 260, 300, 256, True, "bf16", 1), (4, 33, 3, 300, 190, 144, False, "f16", 1),
+    (5, 32, 8, 129, 321, 192, False, "f16", 2), (1, 2, 1, 1537, 1537, 208, True, "f16", 2),  # as many key tiles in 64 rows as in 128
 ])
 def test_a_tile_ahead_on_wide_heads(lm, hip, oracle, B, Hq, Hkv, Sq, Sk, D, causal, dtype, groups):
     """Rows of three tiles, odd ones and a last tile of one key; keys that grow along the row, so that the running maximum is
