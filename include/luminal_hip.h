@@ -244,11 +244,12 @@ int lmh_decode_step(const lmh_decode_params *p, const lmh_decode_step_extra *x);
 
 /* ---- decode attention that allocates nothing and takes no workspace. No counterpart in the reference: it
  * is lmh_decode_attn for callers that cannot call hipMalloc (code under HIP graph capture, tight serving
- * loops, harnesses that forbid allocation). Same parameter block, same kernels, same results; `workspace`
- * and `workspace_bytes` are ignored. The split-KV partials go to a static device array of
+ * loops, harnesses that forbid allocation). Same parameter block, same kernels, and bit for bit the results of
+ * lmh_decode_attn with the same explicit num_splits; `workspace` and `workspace_bytes` are ignored. The split-KV partials go to a static device array of
  * LMH_STATIC_SCRATCH_BYTES that each GPU the library runs on holds until the process ends.
- *   - num_splits == 0 takes lmh_decode_static_splits(): lmh_decode_auto_splits(), halved until
- *     the partials fit. An explicit num_splits whose partials (lmh_decode_workspace_bytes) exceed the
+ *   - num_splits == 0 takes lmh_decode_static_splits(), whatever the device: lmh_decode_auto_splits(), halved until
+ *     the partials fit. (lmh_decode_attn takes fewer splits there where that is faster; its results differ from these
+ *     by fp32 rounding, and a caller that wants that count here passes it.) An explicit num_splits whose partials (lmh_decode_workspace_bytes) exceed the
  *     array is rejected with LMH_E_WORKSPACE.
  *   - Every call on one GPU shares that GPU's array, which keeps the last call's contents. Nothing in it
  *     has to start at zero (each call writes every slot it later reads), so none is cleared; calls that
