@@ -204,3 +204,38 @@ def test_operands_taken_from_the_callers_arrays(lm, hip, dtype, B, Hq, Hkv, T, L
     if Hq * T <= Hkv * L:
         inside = lambda cg: (lambda v: (setattr(v, "shape", tq.shape), setattr(v, "nbytes", cg.results[tq.id].nbytes), v)[2])(cg.results[tvc.id].view(tvc.shape))
         call({tq.id: inside, tkn.id: array(tkn)})
+
+
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,T,L,D,form", [
+    ("f16", 1, 50, 10, 2059, 2100, 96, "prefill_mfma_pair_kernel<f16, D=96, causal> query tiles=9,"),  # the odd tile has a workgroup of its own
+    ("f16", 1, 42, 6, 2999, 3003, 96, "prefill_mfma_pair_kernel<f16, D=96, causal> query tiles=12,"),
+    ("f16", 1, 84, 12, 1301, 1400, 80, "prefill_mfma_pair_kernel<f16, D=96, causal> query tiles=6,"),
+    ("f16", 1, 48, 8, 2305, 2400, 64, "prefill_mfma_pair_kernel<f16, D=64, causal> query tiles=10,"),
+    ("f16", 1, 48, 8, 3009, 3100, 96, "D=96, causal, key groups=1, waves=8, waves per SIMD=2>"),
+    ("f16", 4, 64, 8, 1001, 1100, 64, "D=64, causal, key groups=1, waves=8, waves per SIMD=4>"),
+    ("f16", 4, 64, 8, 1003, 1100, 96, "D=96, causal, key groups=1, waves=8, waves per SIMD=4>"),
+    ("f16", 4, 64, 8, 897, 900, 128, "D=128, causal, key groups=1, waves=8, waves per SIMD=2>"),
+    ("bf16", 2, 64, 8, 2101, 2200, 64, "D=64, causal, key groups=1, waves=8, waves per SIMD=4>"),
+    ("bf16", 1, 64, 8, 2100, 2100, 96, "D=96, causal, key groups=1, waves=8, waves per SIMD=2>"),
+    ("bf16", 2, 64, 8, 2177, 2300, 128, "D=128, causal, key groups=1, waves=8, waves per SIMD=2>")])
+def test_queries_stored_by_the_forms_of_large_prompts(lm, hip, dtype, B, Hq, Hkv, T, L, D, form):
+    """The attention launch of a prompt stores the graph's copy of the queries: every row of it in the 256-row and paired-tile forms
+    too, whose last tile is partly filled, and the result is the one of queries that were copied in front of the launch."""
+    assert form in lm.flash_attention_plan((B, Hq, T, D), (B, Hkv, L, D), dtype, causal=True)
+    g = lm.Graph()
+    tq, tkn, tvn = lm.tensor(g, (B, Hq, T, D), dtype), lm.tensor(g, (B, Hkv, T, D), dtype), lm.tensor(g, (B, Hkv, T, D), dtype)
+    tkc, tvc = lm.tensor(g, (B, Hkv, L, D), dtype), lm.tensor(g, (B, Hkv, L, D), dtype)
+    tpos, tlen = lm.tensor(g, (B,), "i32"), lm.tensor(g, (B,), "i32")
+    out = lm.prompt_self_attention_core(tq, tkn, tvn, tkc, tvc, tpos, tlen, rope_base=10000.0 if D != 80 else None)[0]
+    fed, plain = lm.compile(g, hip), lm.compile(g, hip)
+    assert fed._fed is not None and fed._fed_steps == 2
+    plain._fed = None
+    rng = np.random.default_rng(16900)
+    feeds = {t.id: lm.to_device(rng.standard_normal(t.shape, dtype=np.float32), hip, dtype) for t in (tq, tkn, tvn)}
+    feeds.update({tpos.id: lm.to_device(np.zeros(B, np.int32), hip), tlen.id: lm.to_device(np.full(B, T, np.int32), hip)})
+    fed(feeds)
+    plain(feeds)
+    lm.binding.sync()
+    np.testing.assert_array_equal(fed.results[tq.id].to_host_raw(), feeds[tq.id].to_host_raw())
+    for t in (tkn, tvn, tkc, tvc, out):
+        np.testing.assert_array_equal(fed.results[t.id].to_host_raw(), plain.results[t.id].to_host_raw())
