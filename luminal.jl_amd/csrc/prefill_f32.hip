@@ -60,7 +60,7 @@ __global__ __launch_bounds__(64 * RW * KG, 1) void prefill_f32_kernel(Deal deal,
   const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
   const int q_tile = CAUSAL ? (deal.tiles - 1 - tile_rank) : tile_rank;
-  const int q0 = q_tile * BM;
+  const int q0 = q_tile * BM - (CAUSAL ? causal_shift(deal.tiles, BM, a.Sq, BT) : 0);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(64 * RW * KG, 1) void prefill_f32_kernel(Deal deal,
 #pragma unroll
   for (int j = 0; j < J; j++) {
     float4 raw = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (qi < a.Sq && 16 * j + 4 * g < a.D) raw = *reinterpret_cast<const float4 *>(qp + (int64_t)qi * a.qs[2] + 16 * j + 4 * g);
+    if ((uint32_t)qi < (uint32_t)a.Sq && 16 * j + 4 * g < a.D) raw = *reinterpret_cast<const float4 *>(qp + (int64_t)qi * a.qs[2] + 16 * j + 4 * g);
     qf[j] = (floatx4_t){raw.x, raw.y, raw.z, raw.w};
   }
   if (n_kv_tiles > 0) load_tile(0, 0);
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(64 * RW * KG, 1) void prefill_f32_kernel(Deal deal,
   // ---- epilogue: out[qi][16 db + 4 g + i] = O^T / l ----
   const float l_tot = sum_over_wave_rows(l_i);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if (qi < a.Sq) {
+  if ((uint32_t)qi < (uint32_t)a.Sq) {
     float *op = reinterpret_cast<float *>(a.out) + b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2];
 #pragma unroll
     for (int db = 0; db < J; db++) {

@@ -52,7 +52,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
   const int q_tile = CAUSAL ? (deal.tiles - 1 - tile_rank) : tile_rank;
-  const int q0 = q_tile * BM;
+  const int q0 = q_tile * BM - (CAUSAL ? causal_shift(deal.tiles, BM, a.Sq, BT) : 0);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
 #pragma unroll
       for (int e = 0; e < 2; e++) {
         q[ks][e] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
-        if (qi < a.Sq && 16 * ks + 8 * g < a.D) q[ks][e] = *reinterpret_cast<const floatx4_t *>(qp + (int64_t)qi * a.qs[2] + 16 * ks + 8 * g + 4 * e);
+        if ((uint32_t)qi < (uint32_t)a.Sq && 16 * ks + 8 * g < a.D) q[ks][e] = *reinterpret_cast<const floatx4_t *>(qp + (int64_t)qi * a.qs[2] + 16 * ks + 8 * g + 4 * e);
       }
     if (D % 32 == 0 && a.q_rope) {  // (the head dim equals the tiling: the partner of an element is in the same lane)
       const float pos = (float)((a.q_pos0 ? a.q_pos0[b] : a.q_prev_seq) + qi);
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
 
   const float l_tot = sum_over_wave_halves(l_i);
   const float inv = l_tot > 0.f ? unscale / l_tot : 0.f;
-  if (qi < a.Sq) {
+  if ((uint32_t)qi < (uint32_t)a.Sq) {
     float *op = reinterpret_cast<float *>(a.out) + b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2];
 #pragma unroll
     for (int db = 0; db < DB; db++)

@@ -142,7 +142,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   // the tail of the launch. (Pairing tile r with tile n-1-r in one workgroup equalises the work but
   // halves the number of workgroups; measured 15 % slower on the S = 4096 workload.)
   const int q_tile = CAUSAL ? (deal.tiles - 1 - tile_rank) : tile_rank;
-  const int q0 = q_tile * BM;
+  const int q0 = q_tile * BM - (CAUSAL ? causal_shift(deal.tiles, BM, a.Sq, BT) : 0);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) {
     uint4 raw = make_uint4(0, 0, 0, 0);
-    if (qi < a.Sq && 16 * ks + 8 * g < a.D) raw = *reinterpret_cast<const uint4 *>(qp + (int64_t)qi * a.qs[2] + 16 * ks + 8 * g);
+    if ((uint32_t)qi < (uint32_t)a.Sq && 16 * ks + 8 * g < a.D) raw = *reinterpret_cast<const uint4 *>(qp + (int64_t)qi * a.qs[2] + 16 * ks + 8 * g);
     qreg[ks] = __builtin_bit_cast(vec8, raw);
 #ifdef LMH_FOLD_SCALE
     // Measurement build, not the shipped path: scale * log2(e) multiplied into the Q fragments (rounded to the element
@@ -726,8 +726,9 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   // 8). Workgroups of their own for it, between or behind the others, took 67 and 56 us. Not above head dim 128, where one
   // workgroup has the CU (D=256, 1500 rows: 1 % slower without a copy to make). ----
   auto store_queries = [&]() {
-    const int64_t at = ((int64_t)(b * a.Hq + hq) * a.Sq + q0) * a.D * 2;
-    copy_span<64 * NW, (D / 16 + KSPLIT - 1) / KSPLIT>((char *)queries.dst + at, (const char *)queries.src + at, min(BM, a.Sq - q0) * a.D * 2, wave_u);
+    const int first = max(q0, 0);
+    const int64_t at = ((int64_t)(b * a.Hq + hq) * a.Sq + first) * a.D * 2;
+    copy_span<64 * NW, (D / 16 + KSPLIT - 1) / KSPLIT>((char *)queries.dst + at, (const char *)queries.src + at, (min(q0 + BM, a.Sq) - first) * a.D * 2, wave_u);
   };
   if (CAUSAL && KSPLIT > 1 && D <= 128 && queries.dst) store_queries();  // (before its second key group's waves end)
 
@@ -799,7 +800,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   // ---- epilogue: out[qi][d] = O^T[d][qi] / l ----
   const float l_tot = sum_over_wave_halves(l_i);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if (qi < a.Sq) {
+  if ((uint32_t)qi < (uint32_t)a.Sq) {
     const int64_t off = b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2];
     store_out_rows<MT, DB, false>(oacc, inv, a.out, off, g, a.D, a.out_f32);
   }
@@ -1111,14 +1112,16 @@ __global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a
   const int lane = tid & 63, wave = tid >> 6;
   const int n = lane & 31, g = lane >> 5;
   // rows of this wave: qlo[rb] .. qlo[rb] + 31; without an early tile row block 0 lies past the last query
+  const int shift = CAUSAL ? causal_shift(n_q_tiles, BM, a.Sq, BT) : 0;
+  const int q0_early = t_early * BM - shift, q0_late = t_late * BM - shift;
   int qlo[2];
-  qlo[0] = has_early ? t_early * BM + 32 * wave : a.Sq + 64;
-  qlo[1] = t_late * BM + 32 * wave;
+  qlo[0] = has_early ? q0_early + 32 * wave : a.Sq + 64;
+  qlo[1] = q0_late + 32 * wave;
 
   int n_keys = a.kv_len ? a.kv_len[b] : a.Sk;
   n_keys = min(max(n_keys, 0), a.Sk);
-  const int k_end_early = !has_early ? 0 : CAUSAL ? min(n_keys, (t_early + 1) * BM) : n_keys;   // keys the early tile can see
-  const int k_end_late = CAUSAL ? min(n_keys, (t_late + 1) * BM) : n_keys;
+  const int k_end_early = !has_early ? 0 : CAUSAL ? min(n_keys, q0_early + BM) : n_keys;   // keys the early tile can see
+  const int k_end_late = CAUSAL ? min(n_keys, q0_late + BM) : n_keys;
   const int n_tiles_early = (k_end_early + BT - 1) / BT;
   const int n_tiles_late = (k_end_late + BT - 1) / BT;
 
@@ -1133,7 +1136,7 @@ __global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
       uint4 raw = make_uint4(0, 0, 0, 0);
-      if (qi < a.Sq && 16 * ks + 8 * g < a.D) raw = *reinterpret_cast<const uint4 *>(qp + (int64_t)qi * a.qs[2] + 16 * ks + 8 * g);
+      if ((uint32_t)qi < (uint32_t)a.Sq && 16 * ks + 8 * g < a.D) raw = *reinterpret_cast<const uint4 *>(qp + (int64_t)qi * a.qs[2] + 16 * ks + 8 * g);
       qreg[rb][ks] = __builtin_bit_cast(vec8, raw);
     }
   }
@@ -1301,7 +1304,7 @@ __global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a
     const int qi = qlo[rb] + n;
     const float l_tot = sum_over_wave_halves(l_i[rb]);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    if (qi < a.Sq)
+    if ((uint32_t)qi < (uint32_t)a.Sq)
       store_out_rows<MT, DB, false>(oacc[rb], inv, a.out, b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2], g, a.D, a.out_f32);
   };
   // A whole 128-key tile for the late row block alone: the loop body of prefill_mfma_kernel (four 32-key blocks at a
@@ -1435,9 +1438,9 @@ __global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a
   store_rows(1);
   if (CAUSAL && queries.dst) {
     for (int t = has_early ? 0 : 1; t < 2; t++) {
-      const int q0 = (t ? t_late : t_early) * BM;
-      const int64_t at = ((int64_t)(b * a.Hq + hq) * a.Sq + q0) * a.D * 2;
-      copy_span<64 * NW, D / 16>((char *)queries.dst + at, (const char *)queries.src + at, min(BM, a.Sq - q0) * a.D * 2, wave_u);
+      const int q0 = t ? q0_late : q0_early, first = max(q0, 0);
+      const int64_t at = ((int64_t)(b * a.Hq + hq) * a.Sq + first) * a.D * 2;
+      copy_span<64 * NW, D / 16>((char *)queries.dst + at, (const char *)queries.src + at, (min(q0 + BM, a.Sq) - first) * a.D * 2, wave_u);
     }
   }
 }
