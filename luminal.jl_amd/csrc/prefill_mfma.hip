@@ -802,7 +802,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if ((uint32_t)qi < (uint32_t)a.Sq) {
     const int64_t off = b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2];
-    store_out_rows<MT, DB, false>(oacc, inv, a.out, off, g, a.D, a.out_f32);
+    store_out_rows<MT, DB>(oacc, inv, a.out, off, g, a.D, a.out_f32);
   }
   if (CAUSAL && KSPLIT == 1 && D <= 128 && queries.dst) store_queries();
 }
@@ -1068,7 +1068,7 @@ __global__ __launch_bounds__(1024, 4) void prefill_mfma_wide_kernel(PrefillArgs 
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (qi < a.Sq) {
     const int64_t off = b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2];
-    store_out_rows<MT, DB, true>(oacc, inv, a.out, off, g, a.D, a.out_f32);
+    store_out_rows<MT, DB>(oacc, inv, a.out, off, g, a.D, a.out_f32);
   }
 }
 
@@ -1305,7 +1305,7 @@ __global__ __launch_bounds__(512, 2) void prefill_mfma_pair_kernel(PrefillArgs a
     const float l_tot = sum_over_wave_halves(l_i[rb]);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     if ((uint32_t)qi < (uint32_t)a.Sq)
-      store_out_rows<MT, DB, false>(oacc[rb], inv, a.out, b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2], g, a.D, a.out_f32);
+      store_out_rows<MT, DB>(oacc[rb], inv, a.out, b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2], g, a.D, a.out_f32);
   };
   // A whole 128-key tile for the late row block alone: the loop body of prefill_mfma_kernel (four 32-key blocks at a
   // time, their QK^T chains alternating two by two, one softmax pass over all 64 scores of a lane).
