@@ -311,6 +311,7 @@ template <typename E, bool STEP>
 __device__ __forceinline__ void merge_row(const DecodeArgs &a, int hq, int b) {
   using raw = typename E::raw;
   __shared__ float w_s[kMergeMaxSlots];
+  __shared__ uint16_t full_s[kMergeMaxSlots];  // slots behind the prefetched ones that hold something
   __shared__ float red_m[kMergeThreads / 64], red_l[kMergeThreads / 64], red_s[kMergeThreads / 64];
   const int tid = threadIdx.x;
   const int64_t off = b * a.os[0] + hq * a.os[1];
@@ -395,6 +396,18 @@ __device__ __forceinline__ void merge_row(const DecodeArgs &a, int hq, int b) {
   lsum = 0.f;
 #pragma unroll
   for (int w = 0; w < kMergeThreads / 64; w++) lsum += red_l[w];
+  // Most slots behind the prefetched ones are empty where a workgroup walks several chunks of a sequence (a slot per chunk, one
+  // row per run of them): their rows are not read (B=64 H=32/8 up to 32768 keys D=128, 64 slots: the whole call 849.7 -> 842.2 us). Up to
+  // twice as many slots as are prefetched, all of them are fetched as they come (B=1 L=32768, 32 slots, none empty: 29.0, skipping 30.4).
+  const int n_lds = min(n, kMergeMaxSlots), n_p = min(n_lds, n_pre) & ~3;
+  const bool skip = n_lds > 2 * kMergePrefetch;
+  int n_full = 0;
+  for (int base = n_p; skip && base < n_lds; base += 64) {  // (every wave finds the same ones)
+    const int s = base + (tid & 63);
+    const uint64_t full = __builtin_amdgcn_ballot_w64(s < n_lds && w_s[s] != 0.f);
+    if (full >> (tid & 63) & 1) full_s[n_full + __builtin_popcountll(full & ((uint64_t(1) << (tid & 63)) - 1))] = (uint16_t)s;
+    n_full += __builtin_popcountll(full);
+  }
   const float w_new = (STEP && v_new_row) ? __builtin_amdgcn_exp2f(m_new - M) : 0.f;  // the new row's sum is 1
   lsum += w_new;
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
@@ -415,7 +428,7 @@ __device__ __forceinline__ void merge_row(const DecodeArgs &a, int hq, int b) {
       }
       s = n_p;
     }
-    for (; s + 4 <= n_lds; s += 4) {
+    for (const int end = skip ? n_p : n_lds; s + 4 <= end; s += 4) {
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const float w = w_s[s + u];
@@ -423,7 +436,20 @@ __device__ __forceinline__ void merge_row(const DecodeArgs &a, int hq, int b) {
         acc[u] += w != 0.f ? x * w : 0.f;
       }
     }
-    for (; s < n; s++) {
+    for (int f = 0; f < n_full; f += 8) {
+      float x[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) x[u] = f + u < n_full ? po[(int64_t)full_s[f + u] * a.D + d] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        if (f + u >= n_full) break;
+        const int slot = full_s[f + u];
+        const float y = x[u] * w_s[slot];
+#pragma unroll
+        for (int q = 0; q < 4; q++) acc[q] += (slot & 3) == q ? y : 0.f;
+      }
+    }
+    for (s = skip ? n_lds : s; s < n; s++) {
       const float w = s < kMergeMaxSlots ? w_s[s] : (ml[s].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[s].x - M));
       const float x = po[(int64_t)s * a.D + d];
       acc[0] += w != 0.f ? x * w : 0.f;
