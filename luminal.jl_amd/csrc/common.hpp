@@ -222,7 +222,8 @@ int launch_upload(const UploadItem *items, int n, hipStream_t stream);
 int launch_download(float *dst_pinned, const void *src, int64_t n, int dtype, hipStream_t stream);
 bool decode_mfma_supported(int dtype, int D, int B);
 bool decode_mfma_rope_ok(int D, int interleaved);
-int launch_decode_mfma_split(const DecodeArgs &a, int dtype, hipStream_t stream);
+bool decode_by_pairs(const DecodeArgs &a);
+int launch_decode_mfma_split(const DecodeArgs &a, int dtype, hipStream_t stream, const CopyManyArgs *fed, int n_copies);
 
 // Keys per split used for a given (Lmax, num_splits); always a multiple of 64.
 int decode_chunk_for(int Lmax, int num_splits);

@@ -415,9 +415,7 @@ __device__ __forceinline__ void merge_row(const DecodeArgs &a, int hq, int b) {
   for (int d = tid; d < a.D; d += kMergeThreads) {
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     int s = 0;
-    const int n_lds = min(n, kMergeMaxSlots);
     if (d == tid) {  // the prefetched rows (same summation order as below: slot s adds to acc[s % 4])
-      const int n_p = min(n_lds, n_pre) & ~3;
 #pragma unroll
       for (int u = 0; u < kMergePrefetch; u++) {
         if (u < n_p) {
@@ -485,7 +483,7 @@ int launch_merge(const DecodeArgs &a, hipStream_t stream, const CopyManyArgs *fe
   if (a.step && n_copies > 0) {
     hipLaunchKernelGGL((decode_merge_fed_kernel<E>), dim3(a.Hq, a.B + (n_copies + a.Hq - 1) / a.Hq), dim3(kMergeThreads), 0, stream, a, *fed, n_copies);
     LMH_HIP_TRY(hipGetLastError());
-  } else if (a.step) {  // (always with partials: lmh_decode_step asks for two splits or more)
+  } else if (a.step) {  // (with partials: a step of one split is one launch)
     hipLaunchKernelGGL((decode_merge_kernel<E, true>), dim3(a.Hq, a.B), dim3(kMergeThreads), 0, stream, a);
     LMH_HIP_TRY(hipGetLastError());
   } else if (a.num_splits > 1) {
@@ -538,9 +536,9 @@ int launch_decode(const DecodeArgs &a, int dtype, hipStream_t stream, CopyManyAr
   // (the matrix-core kernel deals its (b, kv head slice, chunk) units in 32-bit arithmetic)
   const int64_t mfma_units = (int64_t)a.B * a.Hkv * ((a.Hq / a.Hkv + 15) / 16) * a.num_splits;
   if (a.mfma_ok && decode_mfma_supported(dtype, a.D, a.B) && mfma_units < (int64_t(1) << 31)) {
-    const int rc = launch_decode_mfma_split(a, dtype, stream);
-    if (rc != LMH_OK) return rc;
     const int n_copies = n_fed ? (int)number_copy_blocks(*fed, n_fed) : 0;
+    const int rc = launch_decode_mfma_split(a, dtype, stream, fed, n_copies);
+    if (rc != LMH_OK || a.num_splits == 1) return rc;
     return dtype == LMH_F16 ? launch_merge<F16>(a, stream, fed, n_copies) : launch_merge<BF16>(a, stream, fed, n_copies);
   }
   if (a.step) return fail(LMH_E_UNSUPPORTED, "decode step: only the matrix-core decode kernel rotates q as it loads it");

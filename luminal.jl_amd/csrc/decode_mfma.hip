@@ -35,6 +35,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "copy.hpp"
 #include "dtypes.hpp"
 #include "rope.hpp"
 
@@ -52,6 +53,7 @@ struct Mfma16F16 {
   static constexpr int kPieces = 2;
   static constexpr float kScale = 16384.f;  // of the weights: the second piece of one below 2^-3 would be subnormal
   using vec8 = half8_t;
+  using elem = F16;
   __device__ static floatx4_t mfma(vec8 a, vec8 b, floatx4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
@@ -62,6 +64,7 @@ struct Mfma16BF16 {
   static constexpr int kPieces = 3;
   static constexpr float kScale = 1.f;
   using vec8 = bf16x8_t;
+  using elem = BF16;
   __device__ static floatx4_t mfma(vec8 a, vec8 b, floatx4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
@@ -81,6 +84,78 @@ constexpr int kMaxBatchPersistent = 1024;  // prefix sums live in LDS
 
 // COLUMNS: the pieces of a head's weights are columns of one product. The 16 columns hold the heads of a slice kPieces times, so
 // that their scores come out once per copy; the lanes of copy x take piece x, and the copies of O are added where the waves' are.
+// Softmax and second product of a wave's 32 keys from key0 on, whose raw scores of head n are in sacc: lane (n, g) holds keys
+// 4 g .. 4 g + 3 of each 16. `end`: the first key that does not exist; v_xor: how the lane's rows of V are swizzled; GB: row blocks
+// whose products are on their way together.
+template <typename MT, int D, bool COLUMNS, int GB, int LDV>
+__device__ __forceinline__ void attend_block(floatx4_t (&sacc)[2], int key0, int end, int g, int copy, float c, const uint16_t *v_frag, int v_xor, float &m_i,
+                                             float &l_i, floatx4_t (&oacc)[D / 16]) {
+  using vec8 = typename MT::vec8;
+  constexpr int DB = D / 16;
+  if (key0 + kBlk > end) {  // ragged last block
+#pragma unroll
+    for (int hb = 0; hb < 2; hb++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (key0 + 16 * hb + 4 * g + i >= end) sacc[hb][i] = -INFINITY;
+  }
+
+  // ---- online softmax; lane (n, g) owns head n ----
+  float mx = fmaxf(fmaxf(fmaxf(sacc[0][0], sacc[0][1]), fmaxf(sacc[0][2], sacc[0][3])),
+                   fmaxf(fmaxf(sacc[1][0], sacc[1][1]), fmaxf(sacc[1][2], sacc[1][3])));
+  mx = max_over_wave_rows(mx);
+  // (finite: key0 < end, so every head sees a key in this block.) The product is rounded before anything is subtracted from it:
+  // old and new weights then differ by exactly the factor alpha, whatever the rounding
+  const float mc = fmaxf(m_i, mx * c);
+  const float alpha = __builtin_amdgcn_exp2f(m_i - mc);
+  m_i = mc;
+  // P is split into 16-bit pieces that hold all of it that fp32 sums see (two of fp16, 22 bits, or three of bf16, 24), and each is
+  // multiplied with V: the matrix cores have time to spare here, and the result depends on where the split boundaries fall by
+  // fp32 roundings only.
+  float psum = 0.f;
+  vec8 pf[COLUMNS ? 1 : MT::kPieces];
+#pragma unroll
+  for (int hb = 0; hb < 2; hb++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float p = __builtin_amdgcn_exp2f(sacc[hb][i] * c - mc);
+      psum += p;
+      float rest = p * MT::kScale;
+#pragma unroll
+      for (int x = 0; x < MT::kPieces; x++) {
+        const auto piece = MT::cvt(rest);
+        rest -= (float)piece;
+        if (!COLUMNS || x == 0 || copy >= x) pf[COLUMNS ? 0 : x][4 * hb + i] = piece;
+      }
+    }
+  l_i = l_i * alpha + psum;
+#pragma unroll
+  for (int db = 0; db < DB; db++) oacc[db] *= alpha;
+
+  // ---- O^T += V^T P^T: a block's share from zero, the first pieces apart from the others, added once ----
+#pragma unroll
+  for (int b0 = 0; b0 < DB; b0 += GB) {
+    floatx4_t o[GB], rest[GB];
+#pragma unroll
+    for (int i = 0; i < GB; i++) {
+      const uint16_t *vaddr = v_frag + ((16 * (b0 + i)) ^ v_xor);
+      const shortx4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(vaddr));
+      const shortx4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(vaddr + 16 * LDV));
+      const vec8 v8 = __builtin_bit_cast(vec8, (shortx8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      o[i] = MT::mfma(v8, pf[0], floatx4_t{0.f, 0.f, 0.f, 0.f});
+      if constexpr (!COLUMNS) {
+        rest[i] = MT::mfma(v8, pf[MT::kPieces - 1], floatx4_t{0.f, 0.f, 0.f, 0.f});
+        if (MT::kPieces == 3) rest[i] = MT::mfma(v8, pf[1], rest[i]);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < GB; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) oacc[b0 + i][e] += COLUMNS ? o[i][e] : o[i][e] + rest[i][e];
+  }
+}
+
 template <typename MT, int D, bool COLUMNS>
 __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, int g_chunks) {
   request_args(a);
@@ -93,7 +168,10 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
   constexpr int LDK = D + 8;             // LDS row strides (elements): chosen so that the 16 rows a
   constexpr int LDV = D + 16;            // fragment read touches fall on different banks
   constexpr int kTileBytes = kBlk * (LDK + LDV) * 2;
-  constexpr int kMergeBytes = kWaves * 16 * (D + 2) * 4;
+  // rows of the waves' sums, in floats: as rows of D the sixteen heads fall on the same banks (D=256 B=2 Hkv=2 L=3000 fp16 20.8 -> 19.2
+  // us, D=128 B=64 Hkv=8 L=512 ragged 19.4 -> 18.6, B=16 L=4096 49.4 -> 48.8)
+  constexpr int LDO = D + 4;
+  constexpr int kMergeBytes = kWaves * 16 * (LDO + 2) * 4;
   constexpr int kSmemBytes = kWaves * kTileBytes > kMergeBytes ? kWaves * kTileBytes : kMergeBytes;
   __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytes];
   __shared__ int s_pref[kMaxBatchPersistent + 1];  // s_pref[b] = chunks of sequences 0..b-1
@@ -284,83 +362,19 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
         sacc[hb] = MT::mfma(kf, qreg[ks], sacc[hb]);
       }
     }
-    if (key0 + kBlk > end) {  // ragged last block
-#pragma unroll
-      for (int hb = 0; hb < 2; hb++)
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-          if (key0 + 16 * hb + 4 * g + i >= end) sacc[hb][i] = -INFINITY;
-    }
-
-    // ---- online softmax; lane (n, g) owns head n ----
-    float mx = fmaxf(fmaxf(fmaxf(sacc[0][0], sacc[0][1]), fmaxf(sacc[0][2], sacc[0][3])),
-                     fmaxf(fmaxf(sacc[1][0], sacc[1][1]), fmaxf(sacc[1][2], sacc[1][3])));
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    // (finite: key0 < end, so every head sees a key in this block.) The product is rounded before anything is subtracted from it:
-    // old and new weights then differ by exactly the factor alpha, whatever the rounding
-    const float mc = fmaxf(m_i, mx * c);
-    const float alpha = __builtin_amdgcn_exp2f(m_i - mc);
-    m_i = mc;
-    // P is split into 16-bit pieces that hold all of it that fp32 sums see (two of fp16, 22 bits, or three of bf16, 24), and each is
-    // multiplied with V: the matrix cores have time to spare here, and the result depends on where the split boundaries fall by
-    // fp32 roundings only.
-    float psum = 0.f;
-    vec8 pf[COLUMNS ? 1 : MT::kPieces];
-#pragma unroll
-    for (int hb = 0; hb < 2; hb++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float p = __builtin_amdgcn_exp2f(sacc[hb][i] * c - mc);
-        psum += p;
-        float rest = p * MT::kScale;
-#pragma unroll
-        for (int x = 0; x < MT::kPieces; x++) {
-          const auto piece = MT::cvt(rest);
-          rest -= (float)piece;
-          if (!COLUMNS || x == 0 || copy >= x) pf[COLUMNS ? 0 : x][4 * hb + i] = piece;
-        }
-      }
-    l_i = l_i * alpha + psum;
-#pragma unroll
-    for (int db = 0; db < DB; db++) oacc[db] *= alpha;
-
-    // ---- O^T += V^T P^T: a block's share from zero, the first pieces apart from the others, added once ----
-    constexpr int GB = DB % 8 == 0 ? 8 : DB;  // row blocks whose products are on their way together
-#pragma unroll
-    for (int b0 = 0; b0 < DB; b0 += GB) {
-      floatx4_t o[GB], rest[GB];
-#pragma unroll
-      for (int i = 0; i < GB; i++) {
-        const uint16_t *vaddr = &Vs[v_frag_off + 16 * (b0 + i)];
-        const shortx4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(vaddr));
-        const shortx4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4_t *)(vaddr + 16 * LDV));
-        const vec8 v8 = __builtin_bit_cast(vec8, (shortx8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        o[i] = MT::mfma(v8, pf[0], floatx4_t{0.f, 0.f, 0.f, 0.f});
-        if constexpr (!COLUMNS) {
-          rest[i] = MT::mfma(v8, pf[MT::kPieces - 1], floatx4_t{0.f, 0.f, 0.f, 0.f});
-          if (MT::kPieces == 3) rest[i] = MT::mfma(v8, pf[1], rest[i]);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < GB; i++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) oacc[b0 + i][e] += COLUMNS ? o[i][e] : o[i][e] + rest[i][e];
-    }
+    attend_block<MT, D, COLUMNS, DB % 8 == 0 ? 8 : DB, LDV>(sacc, key0, end, g, copy, c, Vs + v_frag_off, 0, m_i, l_i, oacc);
   }
 
   // ---- merge the 4 waves, then write the split partial (or the final output) ----
-  l_i += __shfl_xor(l_i, 16);
-  l_i += __shfl_xor(l_i, 32);
+  l_i = sum_over_wave_rows(l_i);
   __syncthreads();  // all waves are done with their tiles: the memory is reused for the merge
-  float *sm_o = reinterpret_cast<float *>(smem);              // [kWaves][16][D]
-  float *sm_m = sm_o + kWaves * 16 * D;                       // [kWaves][16]
+  float *sm_o = reinterpret_cast<float *>(smem);              // [kWaves][16][LDO]
+  float *sm_m = sm_o + kWaves * 16 * LDO;                       // [kWaves][16]
   float *sm_l = sm_m + kWaves * 16;                           // [kWaves][16]
 #pragma unroll
   for (int db = 0; db < DB; db++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) sm_o[(wave * 16 + n) * D + 16 * db + 4 * g + i] = oacc[db][i] * (1.f / MT::kScale);
+    for (int i = 0; i < 4; i++) sm_o[(wave * 16 + n) * LDO + 16 * db + 4 * g + i] = oacc[db][i] * (1.f / MT::kScale);
   if (g == 0) {
     sm_m[wave * 16 + n] = m_i;
     sm_l[wave * 16 + n] = l_i;
@@ -378,10 +392,10 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
       const float mw = sm_m[w * 16 + h];
       const float f = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - M);
       lsum += sm_l[w * 16 + h] * f;
-      float x = sm_o[(w * 16 + h) * D + d];
+      float x = sm_o[(w * 16 + h) * LDO + d];
       if constexpr (COLUMNS) {
-        float rest = sm_o[(w * 16 + (MT::kPieces - 1) * n_heads + h) * D + d];
-        if (MT::kPieces == 3) rest += sm_o[(w * 16 + n_heads + h) * D + d];
+        float rest = sm_o[(w * 16 + (MT::kPieces - 1) * n_heads + h) * LDO + d];
+        if (MT::kPieces == 3) rest += sm_o[(w * 16 + n_heads + h) * LDO + d];
         x += rest;
       }
       o += x * f;
@@ -427,6 +441,227 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
   }
 }
 
+// A (b, kv head slice) pair's whole walk in one workgroup, for launches of few keys and at most about one pair per CU: no partials
+// in memory and no second launch. What bounds these launches is latency: the kernel's chain of round trips and barriers, and the start
+// of a second kernel behind it. So as many waves as LDS holds take a 32-key block each (256 keys at once at D = 128), straight into LDS
+// in whole rows (K into the MFMA's layout, 16 rows x 64 bytes a load, reads every line twice: a step of 512 keys 12.6 us, 10.5 this
+// way), and q, which every wave needs, is rotated once by the whole workgroup. Bank conflicts of the sums' rows and of V's transposing
+// read were 2.4 of those 10.5 us. A step's new row is one more partial of the merge of the waves, as in decode_merge_kernel, and the
+// copies of a fed step are further workgroups.
+template <int D> constexpr int pair_waves() { return D > 128 ? 4 : D > 96 ? 8 : D > 64 ? 12 : 16; }
+template <typename MT, int D, bool COLUMNS>
+__global__ __launch_bounds__(64 * pair_waves<D>()) void decode_pair_kernel(DecodeArgs a, int group, CopyManyArgs fed, int n_copies) {
+  constexpr int NW = pair_waves<D>(), NT = 64 * NW;
+  if ((int)blockIdx.z >= a.B) {
+    constexpr int CT = NT >= 1024 ? 1024 : NT >= 512 ? 512 : 256;  // threads that divide a chunk of the copies
+    const int block = ((blockIdx.z - a.B) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    if (block < n_copies && threadIdx.x < CT) copy_block<CT>(fed, block);
+    return;
+  }
+  request_args(a);
+  request_arg(group);
+  using vec8 = typename MT::vec8;
+  using E = typename MT::elem;
+  using raw = typename E::raw;
+  constexpr int KS = D / 32, DB = D / 16, CPR = D / 8, NL = kBlk * CPR / 64;
+  constexpr int LDQ = D + 8;
+  constexpr int kTile = NW * 2 * kBlk * D * 2, LDO = D + 4, kMerge = NW * 16 * LDO * 4;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kTile > kMerge ? kTile : kMerge];  // K and V tiles, then the waves' sums
+  __shared__ __attribute__((aligned(16))) raw q_s[16 * LDQ], k_s[D];
+  __shared__ float sm_m[NW * 16], sm_l[NW * 16], sm_f[NW * 16], new_s[16], total_s[16], new_w[16];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const int b = blockIdx.z, kvh = blockIdx.x, g0 = 16 * blockIdx.y, n_heads = min(16, group - g0);
+
+  // ---- tiles: global memory -> LDS directly, in whole rows (see prefill_mfma.hip for the asm). Load r of a block fetches its chunks
+  // r * 64 .. + 63; the descriptor ends with the cache, past it zeros arrive. The first block is fetched without waiting for kv_len:
+  // rows past it are masked (K) and cleared (V) below. Chunk j of row i of K lies at j ^ (i % 16) (of a
+  // row of 8 or 16 chunks or more), so that a fragment read, 16 rows x 64 bytes, falls on all banks; V's likewise in pairs. ----
+  typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) void lds_void_t;
+  constexpr int kSwizzle = CPR == 8 ? 7 : CPR % 16 == 0 ? 15 : 0, kSwizzleV = kSwizzle & ~1;
+  const int k_row_bytes = (int)(a.ks[2] * 2), v_row_bytes = (int)(a.vs[2] * 2);
+  auto make_desc = [&](const void *base, int64_t offset, int row_bytes) {
+    const uint64_t p = (uint64_t)base + 2 * offset;
+    i32x4_t d;
+    d[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)p);
+    d[1] = __builtin_amdgcn_readfirstlane((int)((p >> 32) & 0xffff));
+    d[2] = __builtin_amdgcn_readfirstlane(a.Lmax * row_bytes);
+    d[3] = 0x00020000;
+    return d;
+  };
+  const i32x4_t k_desc = make_desc(a.k, b * a.ks[0] + kvh * a.ks[1], k_row_bytes), v_desc = make_desc(a.v, b * a.vs[0] + kvh * a.vs[1], v_row_bytes);
+  int k_voff[NL], v_voff[NL];
+#pragma unroll
+  for (int r = 0; r < NL; r++) {
+    const int id = r * 64 + lane, row = id / CPR, col = id % CPR;
+    k_voff[r] = (int)((row * a.ks[2] + (col ^ (row & kSwizzle)) * 8) * 2);
+    v_voff[r] = (int)((row * a.vs[2] + (col ^ (2 * row & kSwizzleV)) * 8) * 2);
+  }
+  const uint32_t k_lds = (uint32_t)(uintptr_t)(lds_void_t *)smem + wave * (2 * kBlk * D * 2), v_lds = k_lds + kBlk * D * 2;
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is a reserved register; it is only written here
+  auto load = [](i32x4_t desc, uint32_t lds, const int (&voff)[NL], int soff) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < NL; r++)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                   :: "s"(lds + r * 1024), "v"(voff[r]), "s"(desc), "s"(soff) : "memory", "m0");
+  };
+#pragma clang diagnostic pop
+  auto load_k = [&](int key0) __attribute__((always_inline)) { load(k_desc, k_lds, k_voff, key0 * k_row_bytes); };
+  auto load_v = [&](int key0) __attribute__((always_inline)) { load(v_desc, v_lds, v_voff, key0 * v_row_bytes); };
+  if (wave * kBlk < a.Lmax) {
+    load_k(wave * kBlk);
+    load_v(wave * kBlk);
+  }
+  int L = a.kv_len ? a.kv_len[b] : a.Lmax;
+  L = min(max(L, 0), a.Lmax);
+  const int n_blocks = (L + kBlk - 1) / kBlk;
+
+  // ---- q and, for a step, its new row, rotated at position L and rounded to the element type, through LDS ----
+  const bool append = a.step && L < a.Lmax;
+  const raw *v_new = reinterpret_cast<const raw *>(a.v_new) + ((int64_t)b * a.Hkv + kvh) * D;
+  {
+    const raw *k_new = reinterpret_cast<const raw *>(a.k_new) + ((int64_t)b * a.Hkv + kvh) * D;
+    raw *k_dst = const_cast<raw *>(reinterpret_cast<const raw *>(a.k)) + b * a.ks[0] + kvh * a.ks[1] + (int64_t)L * a.ks[2];
+    raw *v_dst = const_cast<raw *>(reinterpret_cast<const raw *>(a.v)) + b * a.vs[0] + kvh * a.vs[1] + (int64_t)L * a.vs[2];
+    const bool writer = g0 == 0;
+    for (int i = tid; i < (n_heads + (append ? 1 : 0)) * (D / 2); i += NT) {
+      const int h = i / (D / 2), j = i % (D / 2);
+      const int d0 = a.rope_interleaved ? 2 * j : j, d1 = a.rope_interleaved ? 2 * j + 1 : j + D / 2;
+      const bool is_q = h < n_heads;
+      const raw *src = is_q ? reinterpret_cast<const raw *>(a.q) + b * a.qs[0] + q_head_of(kvh, g0 + (is_q ? h : 0), a.Hq, a.Hkv, a.head_map) * a.qs[1] : k_new;
+      raw x0 = src[d0], x1 = src[d1];
+      if (a.q_rope) {
+        float o0, o1;
+        rope_pair(E::ld(x0), E::ld(x1), (float)L, j, D, a.rope_log2_base, &o0, &o1);
+        x0 = E::st(o0);
+        x1 = E::st(o1);
+      }
+      raw *dst = is_q ? q_s + h * LDQ : k_s;
+      dst[d0] = x0;
+      dst[d1] = x1;
+      if (!is_q && writer) {
+        k_dst[d0] = x0;
+        k_dst[d1] = x1;
+        v_dst[d0] = v_new[d0];
+        v_dst[d1] = v_new[d1];
+      }
+    }
+  }
+  __syncthreads();
+  const int copy = !COLUMNS ? 0 : (n >= n_heads) + (n >= 2 * n_heads) + (MT::kPieces > 2 && n >= 3 * n_heads), head = n - copy * n_heads;
+  const bool head_ok = COLUMNS ? copy < MT::kPieces : n < n_heads;
+  vec8 qreg[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) {
+    uint4 x = make_uint4(0, 0, 0, 0);
+    if (head_ok) x = *reinterpret_cast<const uint4 *>(&q_s[head * LDQ + 32 * ks + 8 * g]);
+    qreg[ks] = __builtin_bit_cast(vec8, x);
+  }
+  const float c = a.scale * kLog2e;
+  if (append) {  // the new row's scores, a head per wave
+    for (int h = wave; h < n_heads; h += NW) {
+      float dot = 0.f;
+      for (int d = lane; d < D; d += 64) dot += E::ld(q_s[h * LDQ + d]) * E::ld(k_s[d]);
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) dot += __shfl_xor(dot, o);
+      if (lane == 0) new_s[h] = dot * a.scale * kLog2e;
+    }
+  }
+
+  floatx4_t oacc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; db++) oacc[db] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  float m_i = -INFINITY, l_i = 0.f;
+  uint16_t *const k_tile = reinterpret_cast<uint16_t *>(smem) + wave * (2 * kBlk * D);
+  const int v_row = 4 * g + (n >> 2), v_xor = (2 * v_row & kSwizzleV) * 8;  // (and row v_row + 16)
+  const uint16_t *v_frag = k_tile + kBlk * D + v_row * D + 4 * (n & 3);
+  for (int blk = wave; blk < n_blocks; blk += NW) {
+    const int key0 = blk * kBlk;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the block is in LDS
+    floatx4_t sacc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+      for (int hb = 0; hb < 2; hb++) {
+        const vec8 kf = *reinterpret_cast<const vec8 *>(k_tile + (16 * hb + n) * D + ((4 * ks + g) ^ (n & kSwizzle)) * 8);
+        sacc[hb] = MT::mfma(kf, qreg[ks], sacc[hb]);
+      }
+    if (blk + NW < n_blocks) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every read of this block's K has returned
+      load_k(key0 + NW * kBlk);
+    }
+    if (key0 + kBlk > L) {  // (zero times what lies past the last row could be NaN)
+#pragma unroll
+      for (int r = 0; r < NL; r++)
+        if (r * 64 + lane >= (L - key0) * CPR) *reinterpret_cast<uint4 *>(k_tile + kBlk * D + (r * 64 + lane) * 8) = make_uint4(0, 0, 0, 0);
+      wave_lds_fence();
+    }
+    attend_block<MT, D, COLUMNS, DB % 4 == 0 ? 4 : DB, D>(sacc, key0, L, g, copy, c, v_frag, v_xor, m_i, l_i, oacc);
+    if (blk + NW < n_blocks) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every read of this block's V has returned
+      load_v(key0 + NW * kBlk);
+    }
+  }
+
+  // ---- merge the waves and the new row: the waves' factors against the common maximum first ----
+  l_i = sum_over_wave_rows(l_i);
+  if (g == 0) {
+    sm_m[wave * 16 + n] = m_i;
+    sm_l[wave * 16 + n] = l_i;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (blocks fetched for nobody)
+  __syncthreads();  // all waves are done with their tiles: the memory is reused for the merge
+  float *sm_o = reinterpret_cast<float *>(smem);  // [NW][16][LDO]
+  const int used = min(NW, n_blocks);
+  {
+    const float m_new = append && head_ok ? new_s[head] : -INFINITY;
+    float M = m_new;
+#pragma unroll
+    for (int w = 0; w < NW; w++) M = fmaxf(M, sm_m[w * 16 + n]);
+    if (wave < used) {
+      if (g == 0) sm_f[wave * 16 + n] = __builtin_amdgcn_exp2f(m_i - M);
+#pragma unroll
+      for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) sm_o[(wave * 16 + n) * LDO + 16 * db + 4 * g + i] = oacc[db][i] * (1.f / MT::kScale);
+    }
+    if (wave == NW - 1 && g == 0 && n < n_heads) {
+      const float w_new = append ? __builtin_amdgcn_exp2f(m_new - M) : 0.f;  // the new row's sum is 1
+      float part[4] = {0.f, 0.f, 0.f, 0.f};  // (four shorter sums are rounded less than one)
+#pragma unroll
+      for (int w = 0; w < NW; w++)
+        if (w < used) part[w & 3] += sm_l[w * 16 + n] * __builtin_amdgcn_exp2f(sm_m[w * 16 + n] - M);
+      total_s[n] = used == 0 && !append ? 1.f : (part[0] + part[1]) + (part[2] + part[3]) + w_new;  // no key: zeros
+      new_w[n] = w_new;
+    }
+  }
+  __syncthreads();
+  for (int idx = tid; idx < n_heads * D; idx += NT) {
+    const int h = idx / D, d = idx % D;
+    float part[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      if (w >= used) break;
+      float x = sm_o[(w * 16 + h) * LDO + d];
+      if constexpr (COLUMNS) {
+        float rest = sm_o[(w * 16 + (MT::kPieces - 1) * n_heads + h) * LDO + d];
+        if (MT::kPieces == 3) rest += sm_o[(w * 16 + n_heads + h) * LDO + d];
+        x += rest;
+      }
+      part[w & 3] += x * sm_f[w * 16 + h];
+    }
+    float o = (part[0] + part[1]) + (part[2] + part[3]);
+    if (append) o += new_w[h] * E::ld(v_new[d]);
+    const float out = o / total_s[h];
+    const int64_t off = b * a.os[0] + q_head_of(kvh, g0 + h, a.Hq, a.Hkv, a.head_map) * a.os[1] + d;
+    if (a.out_f32) reinterpret_cast<float *>(a.out)[off] = out;
+    else reinterpret_cast<uint16_t *>(a.out)[off] = MT::cvt_bits(out);
+  }
+}
+
 template <typename MT, int D, bool COLUMNS>
 int launch_form(const DecodeArgs &a, hipStream_t stream) {
   // Persistent launch: as many workgroups as the chip holds at once (never more than there are units). Same for every device this
@@ -452,19 +687,30 @@ int launch_form(const DecodeArgs &a, hipStream_t stream) {
   return LMH_OK;
 }
 
+template <typename MT, int D, bool COLUMNS>
+int launch_pair(const DecodeArgs &a, const CopyManyArgs *fed, int n_copies, hipStream_t stream) {
+  const int group = a.Hq / a.Hkv, g_chunks = (group + 15) / 16, per = a.Hkv * g_chunks;
+  const CopyManyArgs copies = n_copies ? *fed : CopyManyArgs{};
+  hipLaunchKernelGGL((decode_pair_kernel<MT, D, COLUMNS>), dim3(a.Hkv, g_chunks, a.B + (n_copies + per - 1) / per), dim3(64 * pair_waves<D>()), 0,
+                     stream, a, group, copies, n_copies);
+  LMH_HIP_TRY(hipGetLastError());
+  return LMH_OK;
+}
+
 template <typename MT, int D>
-int launch_for_d(const DecodeArgs &a, hipStream_t stream) {
-  if (a.Hq / a.Hkv * MT::kPieces <= 16) return launch_form<MT, D, true>(a, stream);
-  return launch_form<MT, D, false>(a, stream);
+int launch_for_d(const DecodeArgs &a, const CopyManyArgs *fed, int n_copies, hipStream_t stream) {
+  const bool columns = a.Hq / a.Hkv * MT::kPieces <= 16;
+  if (a.num_splits == 1 && (a.step || decode_by_pairs(a))) return columns ? launch_pair<MT, D, true>(a, fed, n_copies, stream) : launch_pair<MT, D, false>(a, fed, n_copies, stream);
+  return columns ? launch_form<MT, D, true>(a, stream) : launch_form<MT, D, false>(a, stream);
 }
 
 template <typename MT>
-int launch_for_type(const DecodeArgs &a, hipStream_t stream) {
+int launch_for_type(const DecodeArgs &a, const CopyManyArgs *fed, int n_copies, hipStream_t stream) {
   switch (a.D) {
-    case 64: return launch_for_d<MT, 64>(a, stream);
-    case 96: return launch_for_d<MT, 96>(a, stream);
-    case 128: return launch_for_d<MT, 128>(a, stream);
-    case 256: return launch_for_d<MT, 256>(a, stream);
+    case 64: return launch_for_d<MT, 64>(a, fed, n_copies, stream);
+    case 96: return launch_for_d<MT, 96>(a, fed, n_copies, stream);
+    case 128: return launch_for_d<MT, 128>(a, fed, n_copies, stream);
+    case 256: return launch_for_d<MT, 256>(a, fed, n_copies, stream);
   }
   return fail(LMH_E_UNSUPPORTED, "MFMA decode: head dim %d not tiled", a.D);
 }
@@ -474,15 +720,32 @@ int launch_for_type(const DecodeArgs &a, hipStream_t stream) {
 // The query rotation of lmh_decode_step happens in registers: the partner of every element must be in the same lane.
 bool decode_mfma_rope_ok(int D, int interleaved) { return interleaved || (D / 32) % 2 == 0; }
 
+// Whether a pair's whole walk in one workgroup (decode_pair_kernel, with one split) is the fastest form. By 12 000 launches, both ways
+// timed on each (1 to 640 pairs, 64 to 4096 keys, D = 64 to 256): where it is taken steps take 0.66 of the two launches' time and
+// decodes 0.85 of the split kernel's, on average; the worst 1.06 (steps) and 1.1 (ragged decodes of 128 pairs). us, steps, D = 128 bf16,
+// H=32/8: L=128 12.8 -> 6.2 (what the host takes for a call), L=512 12.8 -> 8.0, L=1024 13.0 -> 10.3 (L=1500 13.6 -> 15), B=16 L=512 16.1
+// -> 10.8, B=32 L=512 20.7 -> 14.5; decodes L=512 10.6 -> 7.3 (L=1024 11.9 -> 12.1), D=64 B=1 L=700 9.1 -> 6.7 (L=1500 9.5 -> 10.2). Few pairs:
+// as long as one CU's walk is not longer than the merge launch and what more CUs gain. From 112 pairs on the CUs are at work either way,
+// and the walk may be longer: D=128 128 pairs L=2048 a step 0.95, a decode 0.98, ragged 1.1. More pairs than CUs go round in rounds.
+bool decode_by_pairs(const DecodeArgs &a) {
+  const int64_t cus = device_cu_count(), pairs = (int64_t)a.B * a.Hkv * ((a.Hq / a.Hkv + 15) / 16), walk = (int64_t)a.Lmax * a.D;
+  const bool many = pairs * 16 >= cus * 7;
+  if (!many) return walk <= (a.step ? (a.D > 96 ? 110000 : 90000) : (a.D > 96 ? 95000 : 78000));
+  if (!a.step) return walk <= 160000 && pairs <= cus && (a.D > 64 || pairs * 5 <= cus * 4);
+  const int64_t rounds = (pairs + cus - 1) / cus;
+  return walk <= (rounds == 1 || pairs * 20 >= rounds * cus * 17 ? 262144 : 50000);
+}
+
 bool decode_mfma_supported(int dtype, int D, int B) {
   return (dtype == LMH_F16 || dtype == LMH_BF16) && (D == 64 || D == 96 || D == 128 || D == 256) &&
          B <= kMaxBatchPersistent;
 }
 
-// Enqueues only the split kernel; the caller adds the merge kernel when num_splits > 1.
-int launch_decode_mfma_split(const DecodeArgs &a, int dtype, hipStream_t stream) {
-  if (dtype == LMH_F16) return launch_for_type<Mfma16F16>(a, stream);
-  if (dtype == LMH_BF16) return launch_for_type<Mfma16BF16>(a, stream);
+// Enqueues only the split kernel; the caller adds the merge kernel when num_splits > 1. With one split, everything (the copies
+// only of a step).
+int launch_decode_mfma_split(const DecodeArgs &a, int dtype, hipStream_t stream, const CopyManyArgs *fed, int n_copies) {
+  if (dtype == LMH_F16) return launch_for_type<Mfma16F16>(a, fed, n_copies, stream);
+  if (dtype == LMH_BF16) return launch_for_type<Mfma16BF16>(a, fed, n_copies, stream);
   return fail(LMH_E_UNSUPPORTED, "MFMA decode: dtype %d has no matrix-core path", dtype);
 }
 
