@@ -120,6 +120,8 @@ struct MatmulProblem {
   int32_t heads, seq;        // heads > 0: c is [M / seq, heads, seq, N / heads], column h + heads d of row (b, s) at [b, h, s, d]
   int32_t a_vec, b_vec;      // 16-byte loads along the contraction
   int32_t b_by_column;       // b is contiguous along its columns: neighbouring threads take neighbouring columns
+  int32_t c_vec;             // four neighbouring columns are one aligned store
+  FastDiv by_m_tiles, by_n_tiles, by_D, by_seq;  // (matmul_split_kernel; D = N / heads)
 };
 struct MatmulArgs {
   MatmulProblem p[kMatmulGroup];

@@ -305,7 +305,9 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
   constexpr int BM = 32 * MB, BN = 32 * NB, WK = 4;
   constexpr int L = 2 * (MB + NB);              // loads of 1 KB (16 rows) per stage: a, then b
   constexpr int kStage = 16 * 16 * L;           // floats
-  constexpr int kShare = MB * NB * 1024;        // floats of a wave's sums
+  constexpr int LDC = BN + 8;                   // row of a wave's sums: the rows r and r + 4 of a store fall on different banks
+  constexpr int kShare = BM * LDC;              // floats of a wave's sums
+  __shared__ __attribute__((aligned(16))) float bias_s[BN];
   __shared__ __attribute__((aligned(16))) float lds[WK * (2 * kStage > kShare ? 2 * kStage : kShare)];
 
   const int per_xcd = (args.n_tiles + 7) / 8;
@@ -321,17 +323,21 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
     if (t >= args.first_tile[i]) g = i;
   const MatmulProblem p = args.p[g];
   t -= args.first_tile[g];
-  const int m_tiles = (p.M + BM - 1) / BM;
-  const int tm = t % m_tiles;
-  t /= m_tiles;
-  const int n_tiles = (p.N + BN - 1) / BN;
-  const int tn = t % n_tiles, batch = t / n_tiles;
+  const int m_tiles = (p.M + BM - 1) / BM, n_tiles = (p.N + BN - 1) / BN;
+  const int tm_row = (uint32_t)t / p.by_m_tiles, tm = t - tm_row * m_tiles;
+  const int batch = (uint32_t)tm_row / p.by_n_tiles, tn = tm_row - batch * n_tiles;
   const int m0 = tm * BM, n0 = tn * BN;
   const int wk = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
   const int lane = threadIdx.x & 63;
   const int n = lane & 31, h = lane >> 5;
   const int D = p.heads ? p.N / p.heads : 1;
+  auto b_col = [&](int j) {  // b_column
+    const int head = (uint32_t)j / p.by_D;
+    return p.heads ? head + p.heads * (j - head * D) : j;
+  };
+  // the bias of column n0 + thread, fetched ahead of everything
+  const float bias = p.bias && (int)threadIdx.x < BN && n0 + (int)threadIdx.x < p.N ? load_as_f32(p.bias, b_col(n0 + threadIdx.x), p.bias_dtype) : 0.f;
   const int steps = ((p.K + 15) / 16 - wk + WK - 1) / WK;  // of this wave (may be none)
 
   typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
@@ -355,7 +361,7 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
     const int row = 16 * l + (lane >> 2), chunk = (lane & 3) ^ swizzle16(row), col = n0 + row - BM;
     if (l < 2) k_of[l] = 4 * chunk;
     if (l < 2 * MB) voff[l] = m0 + row < p.M ? (int)((row * p.as[1] + 4 * chunk) * 4) : kOutOfRange;
-    else voff[l] = col < p.N ? (int)((b_column(p, D, col) * p.bs[2] + 4 * chunk) * 4) : kOutOfRange;
+    else voff[l] = col < p.N ? (int)((b_col(col) * p.bs[2] + 4 * chunk) * 4) : kOutOfRange;
   }
   const uint32_t ring = (uint32_t)(uintptr_t)(lds_void_t *)&lds[wk * 2 * kStage];
 #pragma clang diagnostic push
@@ -445,12 +451,16 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
   if (i < steps) step(i, even, odd);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing arrives in the ring any more
 
-  // ---- fold the shares: each wave takes MB NB / WK blocks (or a part of one), and looks whether their sums are finite ----
-  constexpr int kRegs = 16 * MB * NB / WK;  // registers a lane of a wave folds
-  constexpr int kPart = kRegs % 16 == 0 ? 16 : kRegs % 8 == 0 ? 8 : 4;  // ... in parts that lie in one block
-  static_assert(kRegs % kPart == 0, "whole parts");
-  float sum[kRegs];
+  // ---- fold the shares, four columns of a row a thread, and look whether the sums are finite ----
+  // Through LDS in rows, so that a wave stores whole rows of c: as a lane holds them, a column each, they are stores of 64 to 128
+  // bytes a row, 2.2 to 4.4 us of a launch. us a layer, before and now: 700 rows, hidden 2048, 32 heads of 64 111.1 and 108.7 (32 KV heads
+  // 178.8 and 173.5), 2 x 1000 rows, 12 heads of 128 302 and 283, 4 x 400 rows, 16 heads of 96 167 and 160, with biases 144.8 and 137.8
+  constexpr int Q = BM * BN / 1024;  // fours of a thread
+  if ((int)threadIdx.x < BN) bias_s[threadIdx.x] = bias;
+  floatx4_t sum[Q];
+  bool redone = false;
   for (int pass = 0;; pass++) {
+    redone = pass > 0;
     const float unscale = pass ? 1.f : kPieceUnscale * kPieceUnscale;
     if (pass) {
       // the workgroup's block again with the fp32 product, the operands straight from memory
@@ -462,7 +472,7 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
       for (int i = 0; i < MB + NB; i++) {
         const int row = 32 * i + n, col = n0 + row - BM;
         if (i < MB) off[i] = m0 + row < p.M ? (int)(row * p.as[1] * 4) : -1;
-        else off[i] = col < p.N ? (int)(b_column(p, D, col) * p.bs[2] * 4) : -1;
+        else off[i] = col < p.N ? (int)(b_col(col) * p.bs[2] * 4) : -1;
       }
       for (int i = 0; i < 2 * steps; i++) {
         const int k = 16 * (wk + WK * (i >> 1)) + 8 * (i & 1) + 4 * h;
@@ -479,31 +489,65 @@ __global__ __launch_bounds__(256, 1) void matmul_split_kernel(MatmulArgs args, C
       }
     }
     __syncthreads();
+    float *w = &lds[wk * kShare + 4 * h * LDC + n];
 #pragma unroll
-    for (int q = 0; q < 4 * MB * NB; q++) {
-      const floatx16_t &x = acc[q / 4 / NB][q / 4 % NB];
-      *reinterpret_cast<floatx4_t *>(&lds[wk * kShare + q * 256 + 4 * lane]) = (floatx4_t){x[4 * (q & 3)], x[4 * (q & 3) + 1], x[4 * (q & 3) + 2], x[4 * (q & 3) + 3]};
-    }
+    for (int r = 0; r < MB; r++)
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) w[(32 * r + 8 * (i >> 2) + (i & 3)) * LDC + 32 * j] = acc[r][j][i];
     __syncthreads();
     float finite = 0.f;
 #pragma unroll
-    for (int q = 0; q < kRegs / 4; q++) {
-      const float *s = &lds[(wk * (kRegs / 4) + q) * 256 + 4 * lane];
+    for (int q = 0; q < Q; q++) {
+      const int at = threadIdx.x + 256 * q;
+      const float *s = &lds[at / (BN / 4) * LDC + at % (BN / 4) * 4];
       floatx4_t x = *reinterpret_cast<const floatx4_t *>(s);
 #pragma unroll
-      for (int w = 1; w < WK; w++) x += *reinterpret_cast<const floatx4_t *>(s + w * kShare);
+      for (int o = 1; o < WK; o++) x += *reinterpret_cast<const floatx4_t *>(s + o * kShare);
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        sum[4 * q + e] = x[e] * unscale;
-        finite = fmaf(x[e], 0.f, finite);
-      }
+      for (int e = 0; e < 4; e++) finite = fmaf(x[e], 0.f, finite);
+      sum[q] = x * unscale;
     }
     if (pass || !__syncthreads_or(finite != 0.f || finite != finite)) break;
   }
+  auto place = [&](int m, int j) -> int64_t {
+    if (!p.heads) return ((int64_t)batch * p.M + m) * p.N + j;
+    const int b = (uint32_t)m / p.by_seq, head = (uint32_t)j / p.by_D;  // c[b, head, s, d], rows m = b S + s
+    return (((int64_t)b * p.heads + head) * p.seq + (m - b * p.seq)) * D + (j - head * D);
+  };
+  if (!p.c_vec) {  // columns that do not come in fours: element by element, from the shares in LDS
+    const float unscale = redone ? 1.f : kPieceUnscale * kPieceUnscale;
+#pragma unroll 1
+    for (int at = threadIdx.x; at < BM * BN; at += 256) {
+      const int m = m0 + at / BN, j = n0 + at % BN;
+      if (m >= p.M || j >= p.N) continue;
+      const float *s = &lds[at / BN * LDC + at % BN];
+      float x = s[0];
 #pragma unroll
-  for (int r = 0; r < kRegs; r += kPart) {
-    const int block = (wk * kRegs + r) / 16;
-    store_block<kPart>(p, sum + r, m0 + 32 * (block / NB) + (wk * kRegs + r) % 16 * 2, n0 + 32 * (block % NB) + n, h, batch);
+      for (int o = 1; o < WK; o++) x += s[o * kShare];
+      x = x * unscale + bias_s[at % BN];
+      const int64_t off = place(m, j);
+      if (p.c_dtype == LMH_F32) reinterpret_cast<float *>(p.c)[off] = x;
+      else if (p.c_dtype == LMH_F16) reinterpret_cast<_Float16 *>(p.c)[off] = (_Float16)x;
+      else reinterpret_cast<uint16_t *>(p.c)[off] = f32_to_bf16_bits(x);
+    }
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int at = threadIdx.x + 256 * q, m = m0 + at / (BN / 4), j = n0 + at % (BN / 4) * 4;
+    if (m >= p.M || j >= p.N) continue;
+    const floatx4_t x = sum[q] + *reinterpret_cast<const floatx4_t *>(&bias_s[j - n0]);
+    const int64_t off = place(m, j);
+    if (p.c_dtype == LMH_F32) {
+      *reinterpret_cast<floatx4_t *>(reinterpret_cast<float *>(p.c) + off) = x;
+      continue;
+    }
+    uint16_t y[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) y[e] = p.c_dtype == LMH_F16 ? __builtin_bit_cast(uint16_t, (_Float16)x[e]) : f32_to_bf16_bits(x[e]);
+    *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.c) + off) = make_uint2((uint32_t)y[0] | (uint32_t)y[1] << 16, (uint32_t)y[2] | (uint32_t)y[3] << 16);
   }
 }
 
@@ -536,6 +580,15 @@ template <int MB, int NB>
 int launch_split_form(MatmulArgs &args, int n, hipStream_t stream, const CopyManyArgs &fed, int n_copies) {
   const int64_t tiles = number_tiles(args, n, 32 * MB, 32 * NB);
   if (tiles < 0) return fail(LMH_E_UNSUPPORTED, "matmul: too many tiles");
+  for (int i = 0; i < n; i++) {
+    MatmulProblem &p = args.p[i];
+    const int D = p.heads ? p.N / p.heads : 1;
+    p.by_m_tiles = fast_div((p.M + 32 * MB - 1) / (32 * MB));
+    p.by_n_tiles = fast_div((p.N + 32 * NB - 1) / (32 * NB));
+    p.by_D = fast_div(D);
+    p.by_seq = fast_div(p.heads ? p.seq : 1);
+    p.c_vec = p.N % 4 == 0 && (!p.heads || D % 4 == 0) && (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
+  }
   hipLaunchKernelGGL((matmul_split_kernel<MB, NB>), dim3((unsigned)((tiles + 7) / 8 * 8 + n_copies)), dim3(256), 0, stream, args, fed, n_copies);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;

@@ -258,3 +258,21 @@ def test_a_product_left_to_a_small_element(lm, hip, oracle, M, K, N):
         assert (np.abs(a - b) <= 2.0 ** -22 * np.abs(b)).all(), small[i]
         a, b = got[21:, 40 + i], want[21:, 40 + i]
         assert (np.abs(a - b) <= 2.0 ** -22 * np.abs(b)).all(), small[i]
+
+
+@pytest.mark.parametrize("M,K,N,dtype", [(700, 2048, 2560, "f32"), (701, 2052, 2000, "bf16"), (590, 580, 1156, "f16")])
+def test_products_on_pieces_into_results_of_any_alignment(lm, hip, oracle, M, K, N, dtype):
+    """Results that begin between 16-byte addresses are stored column by column: the bits of the aligned ones, nothing beside them."""
+    x, w, bv = oracle.gen_normal((1, M, K), 38000), oracle.gen_normal((N, K), 38100, 1.0 / np.sqrt(K)), oracle.gen_normal((N,), 38200)
+    dx, dw, db = (lm.to_device(a, hip) for a in (x, w, bv))
+    out, wide = lm.HipArray((1, M, N), dtype, hip), lm.HipArray((M * N + 8,), dtype, hip).fill_bytes(0xff)
+    p = (lm.binding.MatmulParams * 1)()
+    assert _low(lm).fill_matmul(p[0], out, dx, dw, transposed=True, bias=db)
+    lm.binding.matmul(p, 1)
+    esz = 4 if dtype == "f32" else 2
+    p[0].c = wide.ptr + 3 * esz
+    lm.binding.matmul(p, 1)
+    got = wide.to_host()
+    np.testing.assert_array_equal(got[3:3 + M * N].reshape(1, M, N), out.to_host())
+    assert np.isnan(got[:3]).all() and np.isnan(got[3 + M * N:]).all()  # (0xffff is a NaN in every type)
+    assert rel_err(out.to_host(), x.astype(np.float64) @ w.astype(np.float64).T + bv) <= {"f32": 2e-6, "f16": 5e-4, "bf16": 4e-3}[dtype]
