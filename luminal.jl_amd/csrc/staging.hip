@@ -81,13 +81,23 @@ __global__ __launch_bounds__(256) void upload_kernel(UploadArgs a) {
   }
 }
 
-// n values of any type -> fp32 in pinned host memory, four per thread and step
+// n values of any type -> fp32 in pinned host memory, four per thread and step. (32-bit ones too: a copy of the runtime's begins 10 us
+// after the kernel in front of it. execute() of 2 MB of results 292 -> 280 us, of 256 KB 76.9 -> 72.9.)
 __global__ __launch_bounds__(256) void download_kernel(float *dst, const void *src, int64_t n, int dtype) {
   for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += (int64_t)gridDim.x * 1024) {
     float f[4];
+    const bool words = dtype == LMH_F32;
+    if (words && i + 4 <= n && ((uintptr_t)src & 15) == 0) {
+      *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(reinterpret_cast<const float *>(src) + i);
+      continue;
+    }
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       if (i + e >= n) break;
+      if (words) {
+        f[e] = reinterpret_cast<const float *>(src)[i + e];
+        continue;
+      }
       const uint16_t h = reinterpret_cast<const uint16_t *>(src)[i + e];
       f[e] = dtype == LMH_F16 ? (float)__builtin_bit_cast(_Float16, h) : bf16_bits_to_f32(h);
     }
@@ -221,9 +231,17 @@ int launch_upload(const UploadItem *items, int n, hipStream_t stream) {
 }
 
 int launch_download(float *dst, const void *src, int64_t n, int dtype, hipStream_t stream) {
-  if (dtype == LMH_F32) {
-    LMH_HIP_TRY(hipMemcpyAsync(dst, src, (size_t)n * 4, hipMemcpyDeviceToHost, stream));
-    return LMH_OK;
+  if (dtype == LMH_F32) {  // the runtime's copy takes memory that a kernel does not reach: of the host's but not pinned, of another GPU
+    hipPointerAttribute_t to, from;
+    int dev = 0;
+    const bool reached = ((uintptr_t)dst & 15) == 0 && ((uintptr_t)src & 3) == 0 && hipGetDevice(&dev) == hipSuccess &&
+                         hipPointerGetAttributes(&to, dst) == hipSuccess && to.type == hipMemoryTypeHost &&
+                         hipPointerGetAttributes(&from, src) == hipSuccess && from.type == hipMemoryTypeDevice && from.device == dev;
+    if (!reached) {
+      (void)hipGetLastError();
+      LMH_HIP_TRY(hipMemcpyAsync(dst, src, (size_t)n * 4, hipMemcpyDeviceToHost, stream));
+      return LMH_OK;
+    }
   }
   const int64_t blocks = (n + 1023) / 1024;
   hipLaunchKernelGGL(download_kernel, dim3((unsigned)(blocks > 1024 ? 1024 : blocks)), dim3(256), 0, stream, dst, src, n, dtype);

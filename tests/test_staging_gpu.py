@@ -1,5 +1,6 @@
 """Host arrays to the device and back through pinned memory: lengths around the staging pieces (16 KB per workgroup, 256 KB for
 a call's first piece, 1 MB slots, 8 of them before one is used again), conversions bit for bit numpy's, streams and threads."""
+import ctypes
 import threading
 
 import numpy as np
@@ -76,3 +77,23 @@ def test_results_stay_theirs_and_the_pools_are_given_back(lm, hip):
         np.testing.assert_array_equal(a.to_host(), np.arange(5000, dtype=np.float32))
     finally:
         pool.most = most
+
+
+@pytest.mark.parametrize("n,src_at,dst_at", [(1, 0, 0), (4097, 1, 0), (4098, 0, 1), (300001, 3, 2), (300001, 0, 0)])
+def test_fp32_downloads_of_any_alignment(lm, hip, oracle, n, src_at, dst_at):
+    """By a kernel where the ends are aligned and pinned, otherwise by the runtime: into pinned memory at any float, and into pageable."""
+    b = lm.binding
+    x = oracle.gen_normal((n + 8,), 43000 + n)
+    x[src_at] = np.float32(1e-45)  # the smallest subnormal stays what it is
+    dev = lm.to_device(x, hip)
+    ptr = b.host_alloc(4 * (n + 8))
+    pinned = np.frombuffer((ctypes.c_char * (4 * (n + 8))).from_address(ptr), np.float32)
+    pageable = np.empty(n + 8, np.float32)
+    for to, at in ((pinned, ptr), (pageable, pageable.ctypes.data)):
+        to[:] = -7
+        b.download(at + 4 * dst_at, dev.ptr + 4 * src_at, n, b.LMH_F32)
+        b.sync()
+        np.testing.assert_array_equal(to[dst_at:dst_at + n], x[src_at:src_at + n])
+        assert (to[:dst_at] == -7).all() and (to[dst_at + n:] == -7).all()
+    del pinned, to
+    b.host_free(ptr)
