@@ -299,13 +299,15 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
     for (int j = 0; j < VR; j++) vreg[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(v_rsrc, vr_voff[j], soff, 0));
   };
   auto post_top = [&](int slot) {
-    u16x2_t all = {0, 0};
+    // (four at a time: a packed maximum that waits for the one before it costs two instructions)
+    u16x2_t part[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
 #pragma unroll
     for (int j = 0; j < VR; j++) {
       const uint32_t w[4] = {vreg[j].x, vreg[j].y, vreg[j].z, vreg[j].w};
 #pragma unroll
-      for (int e = 0; e < 4; e++) all = __builtin_elementwise_max(all, __builtin_bit_cast(u16x2_t, w[e] & 0x7fff7fffu));
+      for (int e = 0; e < 4; e++) part[e] = __builtin_elementwise_max(part[e], __builtin_bit_cast(u16x2_t, w[e] & 0x7fff7fffu));
     }
+    const u16x2_t all = __builtin_elementwise_max(__builtin_elementwise_max(part[0], part[1]), __builtin_elementwise_max(part[2], part[3]));
     uint32_t m = max((uint32_t)all[0], (uint32_t)all[1]);
     v_special = m >= 0x7f80u;
     if (v_special) {
