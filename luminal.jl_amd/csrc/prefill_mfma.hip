@@ -402,13 +402,15 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
         for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[kb][i]);
       return max_over_wave_halves(mx);
     };
+    // (With the lane's end taken once, as below, these forms are slower: bf16 S=1500 D=256 41.0 us instead of 40.0.)
     auto mask = [&](int k0, floatx16_t (&s)[NKB]) __attribute__((always_inline)) {
-      const int end = (CAUSAL ? min(n_keys, qi + 1) : n_keys) - k0 - 4 * g;  // of the keys that the lane's query sees
 #pragma unroll
       for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
-        for (int i = 0; i < 16; i++)
-          if (kb * 32 + 8 * (i >> 2) + (i & 3) >= end) s[kb][i] = -INFINITY;
+        for (int i = 0; i < 16; i++) {
+          const int key = k0 + kb * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
+          if (key >= n_keys || (CAUSAL && key > qi)) s[kb][i] = -INFINITY;
+        }
     };
     const int kg0 = wave_u / RG * BW, q_lo = q0 + wave_u % RG * 32, q_hi = q_lo + 31;  // (the branches below are the wave's)
     auto masked = [&](int k0) __attribute__((always_inline)) { return (k0 + BW > n_keys) || (CAUSAL && k0 + BW - 1 > q_lo); };
