@@ -156,10 +156,18 @@ __device__ __forceinline__ void attend_block(floatx4_t (&sacc)[2], int key0, int
   }
 }
 
+// What the split kernel divides by in front of its first load. Five divisions of 25 to 40 instructions, one behind the other, went with
+// it, and with the branches around the loads of q the wait for all of them: steps of fp16 B=4 L=4096 D=128 17.5 -> 16.7 us, bf16 B=1 L=8192
+// 16.0 -> 15.2, decodes of B=4 L=4096 16.3 -> 16.0, B=64 L=512 ragged 16.8 -> 16.3.
+struct DecodeDeal {
+  int32_t group, g_chunks;  // query heads of a KV head, and in slices of 16
+  FastDiv by_chunk, by_g_chunks, by_grid;
+};
+
 template <typename MT, int D, bool COLUMNS>
-__global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, int g_chunks) {
+__global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeDeal deal, DecodeArgs a) {
+  request_arg(deal.group);
   request_args(a);
-  request_arg(g_chunks);
   using vec8 = typename MT::vec8;
   constexpr int KS = D / 32;             // k-steps of S^T = K Q^T
   constexpr int DB = D / 16;             // 16-row blocks of O^T
@@ -180,14 +188,14 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int n = lane & 15, g = lane >> 4;
-  const int group = a.Hq / a.Hkv;
+  const int group = deal.group, g_chunks = deal.g_chunks;
   const int kv_slots = a.Hkv * g_chunks;  // (kv head, slice of <= 16 group members) pairs
 
   // ---- this workgroup's share of the (b, kv slot, chunk) units ----
   // s_pref = exclusive prefix sum of the chunks per sequence. Without kv_len it is a closed form; with it, the
   // first wave scans 64 sequences at a time with lane shifts (a serial loop over B = 64 by one thread was 3 us).
   if (!a.kv_len) {
-    const int per_seq = (a.Lmax + a.chunk - 1) / a.chunk;
+    const int per_seq = (int)((uint32_t)(a.Lmax + a.chunk - 1) / deal.by_chunk);
     for (int i = tid; i <= a.B; i += kWaves * 64) {
       s_pref[i] = i * per_seq;
       if (i < a.B) s_len[i] = a.Lmax;
@@ -200,7 +208,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
       if (i < a.B) {
         const int len = min(max(a.kv_len[i], 0), a.Lmax);
         s_len[i] = len;
-        v = (len + a.chunk - 1) / a.chunk;
+        v = (int)((uint32_t)(len + a.chunk - 1) / deal.by_chunk);
       }
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
@@ -217,7 +225,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
   // the other kernel): the first total % grid workgroups take one unit more. 64-bit divisions are ~100 scalar
   // instructions each on this hardware, and five of them stood between a workgroup's start and its first load.
   const uint32_t total_units = (uint32_t)s_pref[a.B] * (uint32_t)kv_slots;
-  const uint32_t share = total_units / gridDim.x, extra = total_units % gridDim.x;
+  const uint32_t share = total_units / deal.by_grid, extra = total_units - share * gridDim.x;
   uint32_t u = blockIdx.x * share + min((uint32_t)blockIdx.x, extra);
   const uint32_t u_end = u + share + (blockIdx.x < extra ? 1u : 0u);
 
@@ -253,11 +261,11 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
     const int n_chunks = s_pref[b + 1] - s_pref[b];
     const uint32_t rem = u - (uint32_t)s_pref[b] * (uint32_t)kv_slots;
     const int slot_id = (int)(rem / (uint32_t)n_chunks);
-    const int c0 = (int)(rem % (uint32_t)n_chunks);
+    const int c0 = (int)rem - slot_id * n_chunks;
     const int c1 = (int)min((uint32_t)n_chunks, c0 + (u_end - u));
     u += (uint32_t)(c1 - c0);
-    const int kvh = slot_id / g_chunks;
-    const int g0 = (slot_id % g_chunks) * 16;  // first group member handled here
+    const int kvh = (int)((uint32_t)slot_id / deal.by_g_chunks);
+    const int g0 = (slot_id - kvh * g_chunks) * 16;  // first group member handled here
     const int n_heads = min(16, group - g0);
     const int L = s_len[b];
     const int start = c0 * a.chunk;
@@ -265,7 +273,8 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
     const int split = c0;
 
 
-  // Q^T fragments (B operand): lane (head n, g) holds q[head][32*ks + 8*g .. +7]; zero for padding heads
+  // Q^T fragments (B operand): lane (head n, g) holds q[head][32*ks + 8*g .. +7], the first head's for padding columns, which nothing
+  // reads (no branch: with one, the wait for q is a wait for all loads)
   vec8 qreg[KS];
   const int copy = COLUMNS ? n / n_heads : 0;
   {
@@ -274,11 +283,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
     const int hq = q_head_of(kvh, head_ok ? g0 + head : 0, a.Hq, a.Hkv, a.head_map);
     const uint16_t *qp = reinterpret_cast<const uint16_t *>(a.q) + b * a.qs[0] + hq * a.qs[1];
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      uint4 raw = make_uint4(0, 0, 0, 0);
-      if (head_ok) raw = *reinterpret_cast<const uint4 *>(qp + 32 * ks + 8 * g);
-      qreg[ks] = __builtin_bit_cast(vec8, raw);
-    }
+    for (int ks = 0; ks < KS; ks++) qreg[ks] = __builtin_bit_cast(vec8, *reinterpret_cast<const uint4 *>(qp + 32 * ks + 8 * g));
   }
 
   const uint16_t *kbase = reinterpret_cast<const uint16_t *>(a.k) + b * a.ks[0] + kvh * a.ks[1];
@@ -328,7 +333,11 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
     if (a.q_rope) {
       float sn[(D + 127) / 128], cs[(D + 127) / 128];
 #pragma unroll
-      for (int i = 0; i < (D + 127) / 128; i++) sincos_angle((float)L * rope_inv_freq(64 * i + lane, D, a.rope_log2_base), &sn[i], &cs[i]);
+      for (int i = 0; i < (D + 127) / 128; i++) {
+        int j = 64 * i + lane;
+        asm volatile("" : "+v"(j));  // (the frequency stays here and is not evaluated in front of everything, also where nothing rotates)
+        sincos_angle((float)L * rope_inv_freq(j, D, a.rope_log2_base), &sn[i], &cs[i]);
+      }
       auto from = [&](const float *x, int j0, int j) { return __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (j0 % 64 + j), __float_as_int(x[j0 / 64]))); };
       if (!a.rope_interleaved) {
         if constexpr (KS % 2 == 0) {
@@ -357,7 +366,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a, 
     }
   };
   const int n_blocks = (end - start + kBlk - 1) / kBlk;
-  if (wave < n_blocks) load_tile(start + wave * kBlk);
+  load_tile(wave < n_blocks ? start + wave * kBlk : end);  // (behind the end: zeros, without a branch)
   rotate_q();  // (after the first loads are on their way: the rotation is in front of the first score)
 
   for (int blk = wave; blk < n_blocks; blk += kWaves) {
@@ -698,7 +707,8 @@ int launch_form(const DecodeArgs &a, hipStream_t stream) {
   const int64_t max_units = (int64_t)a.B * a.Hkv * g_chunks * a.num_splits;
   if (max_units >= (int64_t(1) << 31)) return fail(LMH_E_UNSUPPORTED, "MFMA decode: %lld units do not fit 32 bits", (long long)max_units);
   const int n_wgs = (int)(max_units < wgs_per_device ? max_units : wgs_per_device);
-  hipLaunchKernelGGL((decode_mfma_kernel<MT, D, COLUMNS>), dim3(n_wgs), dim3(kWaves * 64), 0, stream, a, g_chunks);
+  const DecodeDeal deal = {group, g_chunks, fast_div(a.chunk), fast_div(g_chunks), fast_div(n_wgs)};
+  hipLaunchKernelGGL((decode_mfma_kernel<MT, D, COLUMNS>), dim3(n_wgs), dim3(kWaves * 64), 0, stream, deal, a);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
 }
