@@ -323,10 +323,26 @@ __device__ __forceinline__ void merge_row(const DecodeArgs &a, int hq, int b) {
   // the partial rows), each about as long as the arithmetic of the whole kernel. The rows of the first slots do
   // not depend on the others: they are requested first, and travel while the statistics are reduced. Rows of
   // slots that turn out not to exist or to be empty are unset memory and are discarded unread below.
+  // So is the new row, whose place in memory does not depend on the length either (asked for where each part is used, its value behind
+  // everything else, steps of bf16 B=1 L=8192 D=128 took 14.2 us instead of 13.9, B=16 L=4096 46.4 instead of 45.9).
+  const int kvh = STEP ? kv_head_of(hq, a.Hq, a.Hkv, a.head_map) : 0;
+  const int64_t new_row = ((int64_t)b * a.Hkv + kvh) * a.D;
+  const raw *v_new_row = reinterpret_cast<const raw *>(a.v_new) + new_row;
+  // element d of the query and of the new key, with the partner that the rotation pairs it with, and of the new value
+  struct Fresh { raw q, q_pair, k, k_pair, v; };
+  auto partner = [&](int d) { return !a.q_rope ? d : a.rope_interleaved ? d ^ 1 : d < a.D / 2 ? d + a.D / 2 : d - a.D / 2; };
+  auto fetch_new = [&](int d) {
+    const raw *q_row = reinterpret_cast<const raw *>(a.q) + b * a.qs[0] + hq * a.qs[1];
+    const raw *k_row = reinterpret_cast<const raw *>(a.k_new) + new_row;
+    return Fresh{q_row[d], q_row[partner(d)], k_row[d], k_row[partner(d)], v_new_row[d]};
+  };
+  const int first_d = min(tid, a.D - 1);
+  Fresh fresh = {};
+  if (STEP) fresh = fetch_new(first_d);
   float pre[kMergePrefetch];
   const int n_pre = min(a.num_splits, kMergePrefetch);
 #pragma unroll
-  for (int u = 0; u < kMergePrefetch; u++) pre[u] = (u < n_pre && tid < a.D) ? po[(int64_t)u * a.D + tid] : 0.f;
+  for (int u = 0; u < kMergePrefetch; u++) pre[u] = po[(int64_t)min(u, n_pre - 1) * a.D + first_d];
 
   int L = a.kv_len ? a.kv_len[b] : a.Lmax;
   L = min(max(L, 0), a.Lmax);
@@ -336,27 +352,29 @@ __device__ __forceinline__ void merge_row(const DecodeArgs &a, int hq, int b) {
   const float2 ml_first = tid < n ? ml[tid] : make_float2(-INFINITY, 0.f);
   // the new row: its score in log2 units, and (first query head of the KV head only) its place in the caches
   float m_new = -INFINITY;
-  const raw *v_new_row = nullptr;
-  if (STEP && L < a.Lmax) {
-    const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
+  const bool appends = STEP && L < a.Lmax;
+  if (appends) {
     const bool writer = q_head_of(kvh, 0, a.Hq, a.Hkv, a.head_map) == hq;
-    const raw *q_row = reinterpret_cast<const raw *>(a.q) + b * a.qs[0] + hq * a.qs[1];
-    const raw *k_new_row = reinterpret_cast<const raw *>(a.k_new) + ((int64_t)b * a.Hkv + kvh) * a.D;
-    v_new_row = reinterpret_cast<const raw *>(a.v_new) + ((int64_t)b * a.Hkv + kvh) * a.D;
     raw *k_dst = const_cast<raw *>(reinterpret_cast<const raw *>(a.k)) + b * a.ks[0] + kvh * a.ks[1] + (int64_t)L * a.ks[2];
     raw *v_dst = const_cast<raw *>(reinterpret_cast<const raw *>(a.v)) + b * a.vs[0] + kvh * a.vs[1] + (int64_t)L * a.vs[2];
-    auto ld = [](raw x) { return E::ld(x); };
     float dot = 0.f;
     for (int d = tid; d < a.D; d += kMergeThreads) {
-      raw qr = q_row[d], kr = k_new_row[d];
-      if (a.q_rope) {
-        qr = E::st(rope_element(q_row, d, a.D, (float)L, a.rope_log2_base, a.rope_interleaved != 0, ld));
-        kr = E::st(rope_element(k_new_row, d, a.D, (float)L, a.rope_log2_base, a.rope_interleaved != 0, ld));
+      const Fresh x = d == tid ? fresh : fetch_new(d);
+      raw qr = x.q, kr = x.k;
+      if (a.q_rope) {  // (rope_element of both, with one sine)
+        const bool first = a.rope_interleaved ? d % 2 == 0 : d < a.D / 2;
+        const int j = a.rope_interleaved ? d / 2 : first ? d : d - a.D / 2;
+        float sn, cs, o0, o1;
+        sincos_angle((float)L * rope_inv_freq(j, a.D, a.rope_log2_base), &sn, &cs);
+        rope_rotate(E::ld(first ? x.q : x.q_pair), E::ld(first ? x.q_pair : x.q), sn, cs, &o0, &o1);
+        qr = E::st(first ? o0 : o1);
+        rope_rotate(E::ld(first ? x.k : x.k_pair), E::ld(first ? x.k_pair : x.k), sn, cs, &o0, &o1);
+        kr = E::st(first ? o0 : o1);
       }
       dot += E::ld(qr) * E::ld(kr);
       if (writer) {
         k_dst[d] = kr;
-        v_dst[d] = v_new_row[d];
+        v_dst[d] = x.v;
       }
     }
 #pragma unroll
@@ -408,7 +426,7 @@ __device__ __forceinline__ void merge_row(const DecodeArgs &a, int hq, int b) {
     if (full >> (tid & 63) & 1) full_s[n_full + __builtin_popcountll(full & ((uint64_t(1) << (tid & 63)) - 1))] = (uint16_t)s;
     n_full += __builtin_popcountll(full);
   }
-  const float w_new = (STEP && v_new_row) ? __builtin_amdgcn_exp2f(m_new - M) : 0.f;  // the new row's sum is 1
+  const float w_new = appends ? __builtin_amdgcn_exp2f(m_new - M) : 0.f;  // the new row's sum is 1
   lsum += w_new;
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
 
@@ -453,7 +471,7 @@ __device__ __forceinline__ void merge_row(const DecodeArgs &a, int hq, int b) {
       acc[0] += w != 0.f ? x * w : 0.f;
     }
     float o = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-    if (STEP && v_new_row) o += w_new * E::ld(v_new_row[d]);
+    if (appends) o += w_new * E::ld(d == tid ? fresh.v : v_new_row[d]);
     if (a.out_f32) reinterpret_cast<float *>(a.out)[off + d] = o * inv;
     else reinterpret_cast<raw *>(a.out)[off + d] = E::st(o * inv);
   }
