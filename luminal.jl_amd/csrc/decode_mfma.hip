@@ -247,8 +247,10 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeDeal dea
   const int k_frag_off = n * LDK + 8 * g;                             // + 16*hb*LDK + 32*ks
   const int v_frag_off = (4 * g + (n >> 2)) * LDV + 4 * (n & 3);      // + 16*hb*LDV + 16*db
 
-  while (u < u_end) {
-    // segment = the maximal run of units of one (b, kv slot) inside [u, u_end)
+  // A segment = the maximal run of units of one (b, kv slot) inside [u, u_end).
+  struct Segment { int b, kvh, g0, n_heads, c0, c1, L, start, end, n_blocks; };
+  auto next_segment = [&]() {
+    Segment s;
     // largest b with s_pref[b] * kv_slots <= u, 64 sequences at a time (halving the range, one LDS read after the other, and
     // kv_len[b] from memory once more, stood in front of a segment's first load: steps of B=16 L=4096 D=128 50.3 -> 49.8 us, decodes of
     // B=64 L=512 ragged 18.6 -> 17.9, L=3000 93.5 -> 91.9)
@@ -257,51 +259,31 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeDeal dea
       const int i = base + lane;
       b += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i < a.B && (uint32_t)s_pref[i] * (uint32_t)kv_slots <= u));
     }
-    b = __builtin_amdgcn_readfirstlane(b);
+    s.b = b = __builtin_amdgcn_readfirstlane(b);
     const int n_chunks = s_pref[b + 1] - s_pref[b];
     const uint32_t rem = u - (uint32_t)s_pref[b] * (uint32_t)kv_slots;
     const int slot_id = (int)(rem / (uint32_t)n_chunks);
-    const int c0 = (int)rem - slot_id * n_chunks;
-    const int c1 = (int)min((uint32_t)n_chunks, c0 + (u_end - u));
-    u += (uint32_t)(c1 - c0);
-    const int kvh = (int)((uint32_t)slot_id / deal.by_g_chunks);
-    const int g0 = (slot_id - kvh * g_chunks) * 16;  // first group member handled here
-    const int n_heads = min(16, group - g0);
-    const int L = s_len[b];
-    const int start = c0 * a.chunk;
-    const int end = min(L, c1 * a.chunk);
-    const int split = c0;
-
+    s.c0 = (int)rem - slot_id * n_chunks;
+    s.c1 = (int)min((uint32_t)n_chunks, s.c0 + (u_end - u));
+    u += (uint32_t)(s.c1 - s.c0);
+    s.kvh = (int)((uint32_t)slot_id / deal.by_g_chunks);
+    s.g0 = (slot_id - s.kvh * g_chunks) * 16;  // first group member handled here
+    s.n_heads = min(16, group - s.g0);
+    s.L = s_len[b];
+    s.start = s.c0 * a.chunk;
+    s.end = min(s.L, s.c1 * a.chunk);
+    s.n_blocks = (s.end - s.start + kBlk - 1) / kBlk;
+    return s;
+  };
 
   // Q^T fragments (B operand): lane (head n, g) holds q[head][32*ks + 8*g .. +7], the first head's for padding columns, which nothing
   // reads (no branch: with one, the wait for q is a wait for all loads)
   vec8 qreg[KS];
-  const int copy = COLUMNS ? n / n_heads : 0;
-  {
-    const int head = n - copy * n_heads;
-    const bool head_ok = COLUMNS ? copy < MT::kPieces : n < n_heads;
-    const int hq = q_head_of(kvh, head_ok ? g0 + head : 0, a.Hq, a.Hkv, a.head_map);
-    const uint16_t *qp = reinterpret_cast<const uint16_t *>(a.q) + b * a.qs[0] + hq * a.qs[1];
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) qreg[ks] = __builtin_bit_cast(vec8, *reinterpret_cast<const uint4 *>(qp + 32 * ks + 8 * g));
-  }
-
-  const uint16_t *kbase = reinterpret_cast<const uint16_t *>(a.k) + b * a.ks[0] + kvh * a.ks[1];
-  const uint16_t *vbase = reinterpret_cast<const uint16_t *>(a.v) + b * a.vs[0] + kvh * a.vs[1];
-
-  floatx4_t oacc[DB];
-#pragma unroll
-  for (int db = 0; db < DB; db++) oacc[db] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-  float m_i = -INFINITY;  // running max of the scores of head n in log2 units, as the weights have it (same in the 4 lanes of a head)
-  float l_i = 0.f;        // this lane's share of the running sum
-
+  int copy;
   // Raw buffer descriptors over the valid rows [0, end) of this (b, kv head) slice: a load past `end` returns zeros
   // without a branch, so the loads of a block are NL back-to-back instructions (address = lane-invariant offset +
   // scalar block offset). Non-temporal, like every cache stream of this library.
-  const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t *>(kbase), 0, __builtin_amdgcn_readfirstlane(end * k_row_bytes), 0x00020000);
-  const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t *>(vbase), 0, __builtin_amdgcn_readfirstlane(end * v_row_bytes), 0x00020000);
+  __amdgpu_buffer_rsrc_t k_rsrc, v_rsrc;
   uint4 kreg[NL], vreg[NL];
   auto load_tile = [&](int key0) {
     const int k_soff = __builtin_amdgcn_readfirstlane(key0 * k_row_bytes);
@@ -322,7 +304,23 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeDeal dea
     }
   };
 
-  auto rotate_q = [&]() {
+  // q and the wave's first block of a segment on their way
+  auto begin = [&](const Segment &s) {
+    copy = COLUMNS ? n / s.n_heads : 0;
+    const int head = n - copy * s.n_heads;
+    const bool head_ok = COLUMNS ? copy < MT::kPieces : n < s.n_heads;
+    const int hq = q_head_of(s.kvh, head_ok ? s.g0 + head : 0, a.Hq, a.Hkv, a.head_map);
+    const uint16_t *qp = reinterpret_cast<const uint16_t *>(a.q) + s.b * a.qs[0] + hq * a.qs[1];
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) qreg[ks] = __builtin_bit_cast(vec8, *reinterpret_cast<const uint4 *>(qp + 32 * ks + 8 * g));
+    const uint16_t *kbase = reinterpret_cast<const uint16_t *>(a.k) + s.b * a.ks[0] + s.kvh * a.ks[1];
+    const uint16_t *vbase = reinterpret_cast<const uint16_t *>(a.v) + s.b * a.vs[0] + s.kvh * a.vs[1];
+    k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(kbase), 0, __builtin_amdgcn_readfirstlane(s.end * k_row_bytes), 0x00020000);
+    v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(vbase), 0, __builtin_amdgcn_readfirstlane(s.end * v_row_bytes), 0x00020000);
+    load_tile(wave < s.n_blocks ? s.start + wave * kBlk : s.end);  // (behind the end: zeros, without a branch)
+  };
+
+  auto rotate_q = [&](int L) {
     // lmh_decode_step: this step's query is rotated at the position of the row the step appends, kv_len[b], as it is
     // loaded (apply_rotary_embeddings on the queries, reference src/NN.jl:356). Lane (n, g) holds elements
     // 32 ks + 8 g + e: the partner j + D/2 sits in fragment ks + KS/2 of the same lane when KS is even (the launcher
@@ -365,16 +363,27 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeDeal dea
       }
     }
   };
-  const int n_blocks = (end - start + kBlk - 1) / kBlk;
-  load_tile(wave < n_blocks ? start + wave * kBlk : end);  // (behind the end: zeros, without a branch)
-  rotate_q();  // (after the first loads are on their way: the rotation is in front of the first score)
 
-  for (int blk = wave; blk < n_blocks; blk += kWaves) {
-    const int key0 = start + blk * kBlk;
+  Segment seg = {};
+  bool more = u < u_end;
+  if (more) {
+    seg = next_segment();
+    begin(seg);
+  }
+  while (more) {
+  rotate_q(seg.L);  // (after the first loads are on their way: the rotation is in front of the first score)
+  floatx4_t oacc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; db++) oacc[db] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  float m_i = -INFINITY;  // running max of the scores of head n in log2 units, as the weights have it (same in the 4 lanes of a head)
+  float l_i = 0.f;        // this lane's share of the running sum
+
+  for (int blk = wave; blk < seg.n_blocks; blk += kWaves) {
+    const int key0 = seg.start + blk * kBlk;
     wave_lds_fence();  // the previous block's fragment reads precede these writes
     store_tile();
     wave_lds_fence();
-    if (blk + kWaves < n_blocks) load_tile(key0 + kWaves * kBlk);  // in flight during the math below
+    if (blk + kWaves < seg.n_blocks) load_tile(key0 + kWaves * kBlk);  // in flight during the math below
 
     // ---- S^T = K Q^T for the two 16-key halves ----
     floatx4_t sacc[2];
@@ -387,7 +396,16 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeDeal dea
         sacc[hb] = MT::mfma(kf, qreg[ks], sacc[hb]);
       }
     }
-    attend_block<MT, D, COLUMNS, DB % 8 == 0 ? 8 : DB, LDV>(sacc, key0, end, g, copy, c, Vs + v_frag_off, 0, m_i, l_i, oacc);
+    attend_block<MT, D, COLUMNS, DB % 8 == 0 ? 8 : DB, LDV>(sacc, key0, seg.end, g, copy, c, Vs + v_frag_off, 0, m_i, l_i, oacc);
+  }
+
+  // The next segment's first blocks travel while this one's sums are folded (asked for behind them: decodes of B=64 H=32/8 L=3000 ragged
+  // D=128 88.9 us instead of 87.4, B=100 L=1000 52.8 instead of 52.0, B=64 L=2000 D=64 28.8 instead of 28.4).
+  const int b = seg.b, kvh = seg.kvh, g0 = seg.g0, n_heads = seg.n_heads, c0 = seg.c0, c1 = seg.c1;
+  more = u < u_end;
+  if (more) {
+    seg = next_segment();
+    begin(seg);
   }
 
   // ---- merge the 4 waves, then write the split partial (or the final output) ----
@@ -431,7 +449,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeDeal dea
       if (a.out_f32) reinterpret_cast<float *>(a.out)[off] = o / lsum;
       else reinterpret_cast<uint16_t *>(a.out)[off] = MT::cvt_bits(o / lsum);
     } else {
-      const int64_t row = ((int64_t)b * a.Hq + hq) * a.num_splits + split;
+      const int64_t row = ((int64_t)b * a.Hq + hq) * a.num_splits + c0;
       a.ws_o[row * D + d] = o;
       if (d == 0) {
         a.ws_ml[row * 2 + 0] = M;
@@ -450,7 +468,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeDeal dea
     }
   }
   __syncthreads();  // the merge buffers are tile memory again in the next segment
-  }  // while (u < u_end)
+  }  // while (more)
 
   // A sequence without keys has no unit. With several splits the merge kernel writes its zeros; with one split
   // nothing else would write its output rows.
