@@ -510,12 +510,17 @@ __global__ __launch_bounds__(64 * pair_waves<D>()) void decode_pair_kernel(Decod
   constexpr int LDQ = D + 8;
   constexpr int kTile = NW * 2 * kBlk * D * 2, LDO = D + 4, kMerge = NW * 16 * LDO * 4;
   __shared__ __attribute__((aligned(16))) unsigned char smem[kTile > kMerge ? kTile : kMerge];  // K and V tiles, then the waves' sums
-  __shared__ __attribute__((aligned(16))) raw q_s[16 * LDQ], k_s[D];
+  __shared__ __attribute__((aligned(16))) raw q_s[16 * LDQ], k_s[D], v_s[D], row_s[NW][D];
   __shared__ float sm_m[NW * 16], sm_l[NW * 16], sm_f[NW * 16], new_s[16], total_s[16], new_w[16];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
   const int b = blockIdx.z, kvh = blockIdx.x, g0 = 16 * blockIdx.y, n_heads = min(16, group - g0);
+  // (a scalar load, which is not counted with the loads of the tiles, and no branch, which would wait for it; without kv_len any word)
+  typedef const __attribute__((address_space(4))) int32_t constant_int_t;
+  const int length = *(constant_int_t *)(a.kv_len ? (uintptr_t)(a.kv_len + b) : (uintptr_t)a.q);
+  const int head0 = a.head_map == LMH_HEADMAP_BLOCKED ? kvh * group + g0 : kvh + a.Hkv * g0, head_step = a.head_map == LMH_HEADMAP_BLOCKED ? 1 : a.Hkv;
+  auto head_at = [&](int h) { return head0 + h * head_step; };  // q_head_of
 
   // ---- tiles: global memory -> LDS directly, in whole rows (see prefill_mfma.hip for the asm). Load r of a block fetches its chunks
   // r * 64 .. + 63; the descriptor ends with the cache, past it zeros arrive. The first block is fetched without waiting for kv_len:
@@ -525,73 +530,89 @@ __global__ __launch_bounds__(64 * pair_waves<D>()) void decode_pair_kernel(Decod
   typedef __attribute__((address_space(3))) void lds_void_t;
   constexpr int kSwizzle = CPR == 8 ? 7 : CPR % 16 == 0 ? 15 : 0, kSwizzleV = kSwizzle & ~1;
   const int k_row_bytes = (int)(a.ks[2] * 2), v_row_bytes = (int)(a.vs[2] * 2);
-  auto make_desc = [&](const void *base, int64_t offset, int row_bytes) {
+  auto make_desc = [](const void *base, int64_t offset, int bytes) {
     const uint64_t p = (uint64_t)base + 2 * offset;
     i32x4_t d;
     d[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)p);
     d[1] = __builtin_amdgcn_readfirstlane((int)((p >> 32) & 0xffff));
-    d[2] = __builtin_amdgcn_readfirstlane(a.Lmax * row_bytes);
+    d[2] = __builtin_amdgcn_readfirstlane(bytes);
     d[3] = 0x00020000;
     return d;
   };
-  const i32x4_t k_desc = make_desc(a.k, b * a.ks[0] + kvh * a.ks[1], k_row_bytes), v_desc = make_desc(a.v, b * a.vs[0] + kvh * a.vs[1], v_row_bytes);
+  const i32x4_t k_desc = make_desc(a.k, b * a.ks[0] + kvh * a.ks[1], a.Lmax * k_row_bytes), v_desc = make_desc(a.v, b * a.vs[0] + kvh * a.vs[1], a.Lmax * v_row_bytes);
+  // (where a load is whole rows, its lanes' rows are the first load's and a scalar more: no product each)
+  constexpr bool kWhole = 64 % CPR == 0;
+  constexpr int kRows = kWhole ? 64 / CPR : 0;
   int k_voff[NL], v_voff[NL];
 #pragma unroll
   for (int r = 0; r < NL; r++) {
-    const int id = r * 64 + lane, row = id / CPR, col = id % CPR;
-    k_voff[r] = (int)((row * a.ks[2] + (col ^ (row & kSwizzle)) * 8) * 2);
-    v_voff[r] = (int)((row * a.vs[2] + (col ^ (2 * row & kSwizzleV)) * 8) * 2);
+    const int id = kWhole ? lane : r * 64 + lane, row = id / CPR, col = id % CPR, at = row + kRows * r;
+    k_voff[r] = row * k_row_bytes + ((col ^ (at & kSwizzle)) * 16 + kRows * r * k_row_bytes);
+    v_voff[r] = row * v_row_bytes + ((col ^ (2 * at & kSwizzleV)) * 16 + kRows * r * v_row_bytes);
   }
   const uint32_t k_lds = (uint32_t)(uintptr_t)(lds_void_t *)smem + wave * (2 * kBlk * D * 2), v_lds = k_lds + kBlk * D * 2;
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 is a reserved register; it is only written here
-  auto load = [](i32x4_t desc, uint32_t lds, const int (&voff)[NL], int soff) __attribute__((always_inline)) {
-#pragma unroll
-    for (int r = 0; r < NL; r++)
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
-                   :: "s"(lds + r * 1024), "v"(voff[r]), "s"(desc), "s"(soff) : "memory", "m0");
+  auto load_1k = [](i32x4_t desc, uint32_t lds, int voff, int soff) __attribute__((always_inline)) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" :: "s"(lds), "v"(voff), "s"(desc), "s"(soff) : "memory", "m0");
   };
 #pragma clang diagnostic pop
+  auto load = [&](i32x4_t desc, uint32_t lds, const int (&voff)[NL], int soff) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < NL; r++) load_1k(desc, lds + r * 1024, voff[r], soff);
+  };
   auto load_k = [&](int key0) __attribute__((always_inline)) { load(k_desc, k_lds, k_voff, key0 * k_row_bytes); };
   auto load_v = [&](int key0) __attribute__((always_inline)) { load(v_desc, v_lds, v_voff, key0 * v_row_bytes); };
+
+  // ---- q and, for a step, its new key, rotated at position L and rounded to the element type, and the new value, through LDS: a
+  // wave per row, whose elements arrive in front of the wave's keys. (Loaded behind those they were waited for with the keys and then
+  // once more: with the branches of the merge below that was 8.4 us for a step of 512 keys, H=32/8 D=128, which takes 7.5, and 7.2 for a
+  // decode of 322 keys, which takes 6.7.) ----
+  const int rows = n_heads + (a.step ? 2 : 0);
+  const int64_t new_row = ((int64_t)b * a.Hkv + kvh) * D;
+  auto row_at = [&](int h) {
+    const void *base = h < n_heads ? a.q : h == n_heads ? a.k_new : a.v_new;
+    return reinterpret_cast<const raw *>(base) + (h < n_heads ? b * a.qs[0] + head_at(h) * a.qs[1] : new_row);
+  };
+  bool own_direct = false;
+  const int own = NW - 1 - wave;  // (the last waves are the first to be left without keys)
+  if (own < rows) {
+    const raw *from = row_at(own);
+    own_direct = ((uint64_t)from & 15) == 0;
+    if (own_direct && lane < CPR) load_1k(make_desc(from, 0, D * 2), (uint32_t)(uintptr_t)(lds_void_t *)row_s[wave], lane * 16, 0);
+  }
   if (wave * kBlk < a.Lmax) {
     load_k(wave * kBlk);
     load_v(wave * kBlk);
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * NL) : "memory");  // the row is in LDS
+  } else {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
-  int L = a.kv_len ? a.kv_len[b] : a.Lmax;
-  L = min(max(L, 0), a.Lmax);
+  const int L = a.kv_len ? min(max(length, 0), a.Lmax) : a.Lmax;
   const int n_blocks = (L + kBlk - 1) / kBlk;
-
-  // ---- q and, for a step, its new row, rotated at position L and rounded to the element type, through LDS ----
   const bool append = a.step && L < a.Lmax;
-  const raw *v_new = reinterpret_cast<const raw *>(a.v_new) + ((int64_t)b * a.Hkv + kvh) * D;
-  {
-    const raw *k_new = reinterpret_cast<const raw *>(a.k_new) + ((int64_t)b * a.Hkv + kvh) * D;
-    raw *k_dst = const_cast<raw *>(reinterpret_cast<const raw *>(a.k)) + b * a.ks[0] + kvh * a.ks[1] + (int64_t)L * a.ks[2];
-    raw *v_dst = const_cast<raw *>(reinterpret_cast<const raw *>(a.v)) + b * a.vs[0] + kvh * a.vs[1] + (int64_t)L * a.vs[2];
-    const bool writer = g0 == 0;
-    for (int i = tid; i < (n_heads + (append ? 1 : 0)) * (D / 2); i += NT) {
-      const int h = i / (D / 2), j = i % (D / 2);
+  auto place = [&](int h, auto element) __attribute__((always_inline)) {
+    raw *to = h < n_heads ? q_s + h * LDQ : h == n_heads ? k_s : v_s;
+#pragma unroll 1
+    for (int j = lane; j < D / 2; j += 64) {
       const int d0 = a.rope_interleaved ? 2 * j : j, d1 = a.rope_interleaved ? 2 * j + 1 : j + D / 2;
-      const bool is_q = h < n_heads;
-      const raw *src = is_q ? reinterpret_cast<const raw *>(a.q) + b * a.qs[0] + q_head_of(kvh, g0 + (is_q ? h : 0), a.Hq, a.Hkv, a.head_map) * a.qs[1] : k_new;
-      raw x0 = src[d0], x1 = src[d1];
-      if (a.q_rope) {
+      raw x0 = element(d0), x1 = element(d1);
+      if (a.q_rope && h <= n_heads) {
         float o0, o1;
         rope_pair(E::ld(x0), E::ld(x1), (float)L, j, D, a.rope_log2_base, &o0, &o1);
         x0 = E::st(o0);
         x1 = E::st(o1);
       }
-      raw *dst = is_q ? q_s + h * LDQ : k_s;
-      dst[d0] = x0;
-      dst[d1] = x1;
-      if (!is_q && writer) {
-        k_dst[d0] = x0;
-        k_dst[d1] = x1;
-        v_dst[d0] = v_new[d0];
-        v_dst[d1] = v_new[d1];
-      }
+      to[d0] = x0;
+      to[d1] = x1;
     }
+  };
+  const int n_rows = n_heads + (append ? 2 : 0);
+  if (own_direct && own < n_rows) place(own, [&](int d) { return row_s[wave][d]; });
+#pragma unroll 1
+  for (int h = own_direct ? own + NW : own; h < n_rows; h += NW) {
+    const raw *from = row_at(h);
+    place(h, [&](int d) { return from[d]; });
   }
   __syncthreads();
   const int copy = !COLUMNS ? 0 : (n >= n_heads) + (n >= 2 * n_heads) + (MT::kPieces > 2 && n >= 3 * n_heads), head = n - copy * n_heads;
@@ -661,9 +682,9 @@ __global__ __launch_bounds__(64 * pair_waves<D>()) void decode_pair_kernel(Decod
   const int used = min(NW, n_blocks);
   {
     const float m_new = append && head_ok ? new_s[head] : -INFINITY;
-    float M = m_new;
+    float M = m_new, tops[NW];
 #pragma unroll
-    for (int w = 0; w < NW; w++) M = fmaxf(M, sm_m[w * 16 + n]);
+    for (int w = 0; w < NW; w++) M = fmaxf(M, tops[w] = sm_m[w * 16 + n]);
     if (wave < used) {
       if (g == 0) sm_f[wave * 16 + n] = __builtin_amdgcn_exp2f(m_i - M);
 #pragma unroll
@@ -674,32 +695,46 @@ __global__ __launch_bounds__(64 * pair_waves<D>()) void decode_pair_kernel(Decod
     if (wave == NW - 1 && g == 0 && n < n_heads) {
       const float w_new = append ? __builtin_amdgcn_exp2f(m_new - M) : 0.f;  // the new row's sum is 1
       float part[4] = {0.f, 0.f, 0.f, 0.f};  // (four shorter sums are rounded less than one)
+      // (waves without keys add zeros; branches around them, here and below, would make a round trip to LDS of each)
 #pragma unroll
-      for (int w = 0; w < NW; w++)
-        if (w < used) part[w & 3] += sm_l[w * 16 + n] * __builtin_amdgcn_exp2f(sm_m[w * 16 + n] - M);
+      for (int w = 0; w < NW; w++) part[w & 3] += sm_l[w * 16 + n] * __builtin_amdgcn_exp2f(tops[w] - M);
       total_s[n] = used == 0 && !append ? 1.f : (part[0] + part[1]) + (part[2] + part[3]) + w_new;  // no key: zeros
       new_w[n] = w_new;
     }
   }
   __syncthreads();
+  // the new row's place in the caches (in front of the keys, the wait for them would be one for these stores)
+  if (append && g0 == 0) {
+    raw *k_dst = const_cast<raw *>(reinterpret_cast<const raw *>(a.k)) + b * a.ks[0] + kvh * a.ks[1] + (int64_t)L * a.ks[2];
+    raw *v_dst = const_cast<raw *>(reinterpret_cast<const raw *>(a.v)) + b * a.vs[0] + kvh * a.vs[1] + (int64_t)L * a.vs[2];
+    for (int d = tid; d < D; d += NT) {
+      k_dst[d] = k_s[d];
+      v_dst[d] = v_s[d];
+    }
+  }
   for (int idx = tid; idx < n_heads * D; idx += NT) {
     const int h = idx / D, d = idx % D;
     float part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < NW; w++) {
-      if (w >= used) break;
-      float x = sm_o[(w * 16 + h) * LDO + d];
-      if constexpr (COLUMNS) {
-        float rest = sm_o[(w * 16 + (MT::kPieces - 1) * n_heads + h) * LDO + d];
-        if (MT::kPieces == 3) rest += sm_o[(w * 16 + n_heads + h) * LDO + d];
-        x += rest;
+    for (int w0 = 0; w0 < NW; w0 += 4) {
+      if (w0 >= used) break;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int w = w0 + u;
+        float x = sm_o[(w * 16 + h) * LDO + d];
+        if constexpr (COLUMNS) {
+          float rest = sm_o[(w * 16 + (MT::kPieces - 1) * n_heads + h) * LDO + d];
+          if (MT::kPieces == 3) rest += sm_o[(w * 16 + n_heads + h) * LDO + d];
+          x += rest;
+        }
+        x *= sm_f[w * 16 + h];
+        part[u] += w < used ? x : 0.f;  // (what lies in LDS for waves without keys is read and thrown away)
       }
-      part[w & 3] += x * sm_f[w * 16 + h];
     }
     float o = (part[0] + part[1]) + (part[2] + part[3]);
-    if (append) o += new_w[h] * E::ld(v_new[d]);
+    if (append) o += new_w[h] * E::ld(v_s[d]);
     const float out = o / total_s[h];
-    const int64_t off = b * a.os[0] + q_head_of(kvh, g0 + h, a.Hq, a.Hkv, a.head_map) * a.os[1] + d;
+    const int64_t off = b * a.os[0] + head_at(h) * a.os[1] + d;
     if (a.out_f32) reinterpret_cast<float *>(a.out)[off] = out;
     else reinterpret_cast<uint16_t *>(a.out)[off] = MT::cvt_bits(out);
   }

@@ -71,3 +71,25 @@ def test_short_step(lm, hip, oracle, D, Lmax, group, dtype):
     assert rel_err(one[0], two[0]) <= 2e-6
     np.testing.assert_array_equal(one[1], two[1])
     np.testing.assert_array_equal(one[2], two[2])
+
+
+@pytest.mark.parametrize("D,group,dtype", [(64, 3, "f16"), (128, 4, "bf16"), (128, 16, "f16"), (256, 2, "bf16")])
+def test_new_rows_off_alignment(lm, hip, oracle, D, group, dtype):
+    """New rows that do not lie on 16 bytes are loaded element by element: the same bits as of rows that do."""
+    pos = np.array([0, 37, 200], np.int32)
+    B, Hkv = len(pos), 2
+    q, kn, vn, kc, vc = step_inputs(oracle, B, Hkv * group, Hkv, 250, D, dtype, 43000 + D + group)
+
+    def step(shift):
+        dq, dkc, dvc = lm.to_device(np.ascontiguousarray(q[:, :, 0]), hip, dtype), lm.to_device(kc, hip, dtype), lm.to_device(vc, hip, dtype)
+        news = []
+        for x in (kn, vn):
+            whole = lm.to_device(np.concatenate([np.zeros(shift, np.float32), x.reshape(-1)]), hip, dtype)
+            part = whole.view(whole.shape)
+            part.shape, part.nbytes, part.ptr = x.shape, 2 * x.size, whole.ptr + 2 * shift
+            news.append(part)
+        out = lm.execute_op(lm.DecodeStepOp(lm.default_scale(D), 0, 0, "f32", 10000.0, False), dq, dkc, dvc, *news, lm.to_device(pos, hip))[0]
+        return out.to_host(), dkc.to_host(), dvc.to_host()
+
+    for a, b in zip(step(0), step(1)):
+        np.testing.assert_array_equal(a, b)
