@@ -103,16 +103,20 @@ __device__ inline void rotate_q_fragments_with_table(typename MT::vec8 (&qreg)[D
 // WPS: waves per SIMD the register budget is set for (3 x 4 waves, 2 x 8 waves or 1 x 8 waves per CU).
 template <int D, int NW> constexpr int default_wps() { return D > 128 ? 1 : D > 96 ? 2 : NW == 8 ? 4 : 3; }
 // AHEAD: the loop that is a tile ahead with its scores, for one wave per SIMD.
-template <typename MT, int D, bool CAUSAL, int KSPLIT, int NW, int WPS, bool AHEAD>
+// HEADS = 2: the waves' second half takes the same rows of another query head of the KV head, so that a tile is staged, and in bf16 rewritten
+// as fp16, once for both, in row tiles half as high as NW waves of one head have. B=3 H=32/8 S=1337 D=128 causal fp16 61.2 -> 57.4 us, bf16
+// 70.5 -> 67.0 (ragged 65.8 -> 64.0), a prompt of B=4 T=777 fp16 54.9 -> 51.8.
+template <typename MT, int D, bool CAUSAL, int KSPLIT, int NW, int WPS, bool AHEAD, int HEADS = 1>
 __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, PrefillArgs a, QueryCopy queries) {
   request_args(a);
   request_args(deal);
   using vec8 = typename MT::vec8;
-  constexpr int BM = 32 * NW / KSPLIT;  // query rows per workgroup
+  constexpr int BM = 32 * NW / KSPLIT / HEADS;  // query rows per workgroup
   // keys per staged tile: 64; 128 where one workgroup has the CU to itself and LDS and registers allow (half the
   // barriers and per-tile bookkeeping: 114.2 -> 111.9 us on B=1 H=32 S=4096 causal)
   constexpr int BT = (NW == 8 && WPS == 2 && D <= 96 && KSPLIT == 1) ? 2 * BN : BN;
   constexpr int RG = NW / KSPLIT;   // waves (32-row groups) per key group
+  constexpr int RH = RG / HEADS;    // ... and of a head
   constexpr int NKB = BT / 32 / KSPLIT;   // 32-key blocks a wave takes per tile
   constexpr int BW = 32 * NKB;      // ... in keys
   constexpr int KS = D / 16;       // k-steps of the S^T product
@@ -136,7 +140,12 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   // ---- which (b, hq, query tile) this workgroup owns ----
   int bh, tile_rank;
   if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, &bh, &tile_rank)) return;
-  const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
+  const int b = (int)((uint32_t)bh / deal.hq);
+  int hq = bh - b * (a.Hq / HEADS), hq_step = 0;  // the (first) query head; with HEADS = 2 the waves' second half takes another one
+  if constexpr (HEADS == 2) {  // hq counts the pairs of heads of one KV head
+    hq_step = a.head_map == LMH_HEADMAP_BLOCKED ? 1 : a.Hkv;
+    hq = a.head_map == LMH_HEADMAP_BLOCKED ? 2 * hq : hq + hq / a.Hkv * a.Hkv;
+  }
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
   // Causal rows grow with the query index: long rows are issued first so that the short ones fill
   // the tail of the launch. (Pairing tile r with tile n-1-r in one workgroup equalises the work but
@@ -148,7 +157,8 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   const int lane = tid & 63, wave = tid >> 6;
   const int n = lane & 31, g = lane >> 5;
   const int kg = wave / RG;  // key group of this wave (always 0 when KSPLIT == 1)
-  const int wave_q_lo = q0 + (wave % RG) * 32;
+  const int wave_q_lo = q0 + (wave % RH) * 32;
+  const int own_hq = HEADS == 1 ? hq : hq + __builtin_amdgcn_readfirstlane(wave % RG / RH) * hq_step;
   const int wave_q_hi = wave_q_lo + 31;
   const int qi = wave_q_lo + n;
 
@@ -158,7 +168,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   if (CAUSAL) k_end = min(k_end, q0 + BM);
   const int n_kv_tiles = (k_end + BT - 1) / BT;
 
-  const uint16_t *qp = reinterpret_cast<const uint16_t *>(a.q) + b * a.qs[0] + hq * a.qs[1];
+  const uint16_t *qp = reinterpret_cast<const uint16_t *>(a.q) + b * a.qs[0] + own_hq * a.qs[1];
   const uint16_t *kp = reinterpret_cast<const uint16_t *>(a.k) + b * a.ks[0] + kvh * a.ks[1];
   const uint16_t *vp = reinterpret_cast<const uint16_t *>(a.v) + b * a.vs[0] + kvh * a.vs[1];
 
@@ -412,7 +422,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
           if (key >= n_keys || (CAUSAL && key > qi)) s[kb][i] = -INFINITY;
         }
     };
-    const int kg0 = wave_u / RG * BW, q_lo = q0 + wave_u % RG * 32, q_hi = q_lo + 31;  // (the branches below are the wave's)
+    const int kg0 = wave_u / RG * BW, q_lo = q0 + wave_u % RH * 32, q_hi = q_lo + 31;  // (the branches below are the wave's)
     auto masked = [&](int k0) __attribute__((always_inline)) { return (k0 + BW > n_keys) || (CAUSAL && k0 + BW - 1 > q_lo); };
     // tiles in which a key of this wave's share is before its diagonal and the last key
     const int n_live = ((CAUSAL ? min(k_end, q_hi + 1) : k_end) - kg0 + BT - 1) / BT;
@@ -731,8 +741,11 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   // workgroup has the CU (D=256, 1500 rows: 1 % slower without a copy to make). ----
   auto store_queries = [&]() {
     const int first = max(q0, 0);
-    const int64_t at = ((int64_t)(b * a.Hq + hq) * a.Sq + first) * a.D * 2;
-    copy_span<64 * NW, (D / 16 + KSPLIT - 1) / KSPLIT>((char *)queries.dst + at, (const char *)queries.src + at, (min(q0 + BM, a.Sq) - first) * a.D * 2, wave_u);
+#pragma unroll
+    for (int h = 0; h < HEADS; h++) {
+      const int64_t at = ((int64_t)(b * a.Hq + hq + h * hq_step) * a.Sq + first) * a.D * 2;
+      copy_span<64 * NW, (D / 16 + KSPLIT - 1) / KSPLIT>((char *)queries.dst + at, (const char *)queries.src + at, (min(q0 + BM, a.Sq) - first) * a.D * 2, wave_u);
+    }
   };
   if (CAUSAL && KSPLIT > 1 && D <= 128 && queries.dst) store_queries();  // (before its second key group's waves end)
 
@@ -805,7 +818,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   const float l_tot = sum_over_wave_halves(l_i);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if ((uint32_t)qi < (uint32_t)a.Sq) {
-    const int64_t off = b * a.os[0] + hq * a.os[1] + (int64_t)qi * a.os[2];
+    const int64_t off = b * a.os[0] + own_hq * a.os[1] + (int64_t)qi * a.os[2];
     store_out_rows<MT, DB>(oacc, inv, a.out, off, g, a.D, a.out_f32);
   }
   if (CAUSAL && KSPLIT == 1 && D <= 128 && queries.dst) store_queries();
@@ -1474,22 +1487,23 @@ int launch_pair(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stre
 template <typename MT, bool V16, int KSPLIT> struct base_policy { using type = MT; };
 template <> struct base_policy<MfmaBF16, true, 1> { using type = MfmaBF16V16; };
 
-template <typename MT0, bool V16, int D, int KSPLIT, int NW, int WPS = default_wps<D, NW>(), bool AHEAD = false>
+template <typename MT0, bool V16, int D, int KSPLIT, int NW, int WPS = default_wps<D, NW>(), bool AHEAD = false, int HEADS = 1>
 int launch_split(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream) {
   using MT = typename base_policy<MT0, V16, KSPLIT>::type;
-  constexpr int BM = 32 * NW / KSPLIT;
+  constexpr int BM = 32 * NW / KSPLIT / HEADS;
   const int n_q_tiles = (a.Sq + BM - 1) / BM;
-  const int64_t wgs = deal_grid((int64_t)a.B * a.Hq, n_q_tiles);
+  const int64_t wgs = deal_grid((int64_t)a.B * a.Hq / HEADS, n_q_tiles);
   const int rc = check_grid(wgs, 64 * NW);
   if (rc != LMH_OK) return rc;
   dim3 grid((uint32_t)wgs), block(64 * NW);
-  if (plan_only("prefill_mfma_kernel<%s, D=%d, %s, key groups=%d, waves=%d, waves per SIMD=%d> workgroups=%u%s%s", MT::kName, D,
-                a.causal ? "causal" : "full", KSPLIT, NW, WPS, grid.x, MT::kConvertV ? ", V as fp16" : "", AHEAD ? ", a tile ahead" : ""))
+  if (plan_only("prefill_mfma_kernel<%s, D=%d, %s, key groups=%d, waves=%d, waves per SIMD=%d> workgroups=%u%s%s%s", MT::kName, D,
+                a.causal ? "causal" : "full", KSPLIT, NW / HEADS, WPS, (uint32_t)deal_grid((int64_t)a.B * a.Hq, n_q_tiles),
+                HEADS == 2 ? ", joined two by two" : "", MT::kConvertV ? ", V as fp16" : "", AHEAD ? ", a tile ahead" : ""))  // (waves and workgroups of a head)
     return LMH_OK;
-  const Deal deal = make_deal(a.B, a.Hq, n_q_tiles, a.causal ? 4 * WPS / NW : 0, device_cu_count());
+  const Deal deal = make_deal(a.B, a.Hq / HEADS, n_q_tiles, a.causal ? 4 * WPS / NW : 0, device_cu_count());
   if (a.causal)
-    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS, AHEAD>), grid, block, 0, stream, deal, a, queries);
-  else
+    hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, true, KSPLIT, NW, WPS, AHEAD, HEADS>), grid, block, 0, stream, deal, a, queries);
+  else if constexpr (HEADS == 1)
     hipLaunchKernelGGL((prefill_mfma_kernel<MT, D, false, KSPLIT, NW, WPS, AHEAD>), grid, block, 0, stream, deal, a, queries);
   LMH_HIP_TRY(hipGetLastError());
   return LMH_OK;
@@ -1623,6 +1637,16 @@ inline double form_cost(const FormCost &f, const PrefillArgs &a, int form, int p
   return f.fixed + sqrt(sqrt(longest * longest * longest * longest + mean * mean * mean * mean)) + f.per_wg * wgs;
 }
 
+// Whether a causal launch of 128-row workgroups at head dim 128 takes two query heads of one KV head in eight waves instead (HEADS = 2
+// below). By 230 launches of drawn sizes, both ways timed on each (104 to 128 elements, 1 to 64 heads, 200 to 4096 rows): from 1.5 to 2.1
+// of the doubled workgroups per CU, of at least eight row tiles (bf16) or five (fp16), it takes 0.89 to 0.98 of the time, 0.93 on average,
+// the worst 1.00. Up to 1.5 per CU 1.05 on average (0.92 to 1.12: the longest workgroup decides, and is longer), beyond 2.1 0.93 to 1.1, with
+// fewer row tiles 0.94 to 1.1 (the two smaller workgroups of a CU are at different places of their tiles).
+inline bool two_heads_ahead(const PrefillArgs &a, bool v16, int n_cus) {
+  const int64_t tiles = (a.Sq + 127) / 128, wgs = (int64_t)a.B * a.Hq / 2 * tiles;
+  return a.causal && a.Hq / a.Hkv % 2 == 0 && tiles >= (v16 ? 8 : 5) && 2 * wgs > 3 * n_cus && 10 * wgs <= 21 * n_cus;
+}
+
 // Launch the cheapest form, in favour of the one that the rules by size chose. bf16 launches whose weights are head + remainder
 // by those rules stay so: V as fp16 goes with weights of 11 bits.
 template <typename MT, int D, bool V16>
@@ -1656,6 +1680,7 @@ int launch_cheapest(const PrefillArgs &a, const QueryCopy &queries, int by_size,
         if (best == kRows256Pair) return launch_split<MT, V, D, 1, 8>(a, queries, stream);
     } else if constexpr (!MT::kSplitP || V) {
       if (best == kRows256) return launch_split<MT, V, D, 1, 8>(a, queries, stream);
+      if (best == kRows128 && two_heads_ahead(a, V, n_cus)) return launch_split<MT, V, D, 1, 8, 2, false, 2>(a, queries, stream);
     }
     return launch_split<MT, V, D, 1, 4>(a, queries, stream);
   };
