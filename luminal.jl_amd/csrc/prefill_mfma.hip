@@ -1488,7 +1488,7 @@ template <typename MT, bool V16, int KSPLIT> struct base_policy { using type = M
 template <> struct base_policy<MfmaBF16, true, 1> { using type = MfmaBF16V16; };
 
 template <typename MT0, bool V16, int D, int KSPLIT, int NW, int WPS = default_wps<D, NW>(), bool AHEAD = false, int HEADS = 1>
-int launch_split(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream) {
+int launch_split(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream, bool joined = false) {  // joined: named as the workgroups of one head that it joins
   using MT = typename base_policy<MT0, V16, KSPLIT>::type;
   constexpr int BM = 32 * NW / KSPLIT / HEADS;
   const int n_q_tiles = (a.Sq + BM - 1) / BM;
@@ -1497,8 +1497,8 @@ int launch_split(const PrefillArgs &a, const QueryCopy &queries, hipStream_t str
   if (rc != LMH_OK) return rc;
   dim3 grid((uint32_t)wgs), block(64 * NW);
   if (plan_only("prefill_mfma_kernel<%s, D=%d, %s, key groups=%d, waves=%d, waves per SIMD=%d> workgroups=%u%s%s%s", MT::kName, D,
-                a.causal ? "causal" : "full", KSPLIT, NW / HEADS, WPS, (uint32_t)deal_grid((int64_t)a.B * a.Hq, n_q_tiles),
-                HEADS == 2 ? ", joined two by two" : "", MT::kConvertV ? ", V as fp16" : "", AHEAD ? ", a tile ahead" : ""))  // (waves and workgroups of a head)
+                a.causal ? "causal" : "full", KSPLIT, joined ? NW / 2 : NW, WPS, joined ? (uint32_t)deal_grid((int64_t)a.B * a.Hq, n_q_tiles) : grid.x,
+                joined ? ", joined two by two" : HEADS == 2 ? ", two heads each" : "", MT::kConvertV ? ", V as fp16" : "", AHEAD ? ", a tile ahead" : ""))
     return LMH_OK;
   const Deal deal = make_deal(a.B, a.Hq / HEADS, n_q_tiles, a.causal ? 4 * WPS / NW : 0, device_cu_count());
   if (a.causal)
@@ -1637,14 +1637,13 @@ inline double form_cost(const FormCost &f, const PrefillArgs &a, int form, int p
   return f.fixed + sqrt(sqrt(longest * longest * longest * longest + mean * mean * mean * mean)) + f.per_wg * wgs;
 }
 
-// Whether a causal launch of 128-row workgroups at head dim 128 takes two query heads of one KV head in eight waves instead (HEADS = 2
-// below). By 230 launches of drawn sizes, both ways timed on each (104 to 128 elements, 1 to 64 heads, 200 to 4096 rows): from 1.5 to 2.1
+// Whether a causal launch of 128-row workgroups at head dim 128 takes two query heads of one KV head in eight waves instead (HEADS = 2). By 230 launches of drawn sizes, both ways timed on each (104 to 128 elements, 1 to 64 heads, 200 to 4096 rows): from 1.5 to 2.1
 // of the doubled workgroups per CU, of at least eight row tiles (bf16) or five (fp16), it takes 0.89 to 0.98 of the time, 0.93 on average,
 // the worst 1.00. Up to 1.5 per CU 1.05 on average (0.92 to 1.12: the longest workgroup decides, and is longer), beyond 2.1 0.93 to 1.1, with
 // fewer row tiles 0.94 to 1.1 (the two smaller workgroups of a CU are at different places of their tiles).
 inline bool two_heads_ahead(const PrefillArgs &a, bool v16, int n_cus) {
   const int64_t tiles = (a.Sq + 127) / 128, wgs = (int64_t)a.B * a.Hq / 2 * tiles;
-  return a.causal && a.Hq / a.Hkv % 2 == 0 && tiles >= (v16 ? 8 : 5) && 2 * wgs > 3 * n_cus && 10 * wgs <= 21 * n_cus;
+  return tiles >= (v16 ? 8 : 5) && 2 * wgs > 3 * n_cus && 10 * wgs <= 21 * n_cus;
 }
 
 // Launch the cheapest form, in favour of the one that the rules by size chose. bf16 launches whose weights are head + remainder
@@ -1674,13 +1673,21 @@ int launch_cheapest(const PrefillArgs &a, const QueryCopy &queries, int by_size,
   auto launch = [&](auto with_v) {
     constexpr bool V = decltype(with_v)::value;
     if (best == kKeysSplit64) return launch_split<MT, V, D, 2, 4>(a, queries, stream);
+    // Causal launches that eight waves of 256 rows would serve take two query heads of a KV head instead, 128 rows of each: as much shared,
+    // and half a tile less on the diagonal and past the last row. 128 drawn launches of 256 to 8192 rows, time against 256 rows: head dim
+    // 128 0.96 on average (0.88 to 1.01), up to 96 two workgroups on a CU 0.98 (0.90 to 1.01), one 0.98 in bf16 (0.94 to 1.01); one in fp16
+    // 1.00 (to 1.02), which stays.
+    const bool two = a.causal && a.Hq / a.Hkv % 2 == 0;
     if constexpr (D <= 96) {
+      if constexpr (MT::kSplitP)
+        if (best == kRows256 && two) return launch_split<MT, V, D, 1, 8, 2, false, 2>(a, queries, stream);
       if (best == kRows256) return launch_split<MT, V, D, 1, 8, 2>(a, queries, stream);
       if constexpr (!(D == 96 && V))  // (its registers spill at four waves per SIMD)
-        if (best == kRows256Pair) return launch_split<MT, V, D, 1, 8>(a, queries, stream);
+        if (best == kRows256Pair) return two ? launch_split<MT, V, D, 1, 8, 4, false, 2>(a, queries, stream) : launch_split<MT, V, D, 1, 8>(a, queries, stream);
     } else if constexpr (!MT::kSplitP || V) {
+      if (best == kRows256 ? two : best == kRows128 && two && two_heads_ahead(a, V, n_cus))
+        return launch_split<MT, V, D, 1, 8, 2, false, 2>(a, queries, stream, best == kRows128);
       if (best == kRows256) return launch_split<MT, V, D, 1, 8>(a, queries, stream);
-      if (best == kRows128 && two_heads_ahead(a, V, n_cus)) return launch_split<MT, V, D, 1, 8, 2, false, 2>(a, queries, stream);
     }
     return launch_split<MT, V, D, 1, 4>(a, queries, stream);
   };

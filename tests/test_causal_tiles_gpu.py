@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
     (1, 3, 1, 65, 65, 64, "f16", "key groups=2, waves=4"), (2, 5, 5, 191, 191, 80, "bf16", "key groups=2, waves=4"),
     (2, 32, 4, 1151, 1151, 128, "f16", "key groups=1, waves=4"), (6, 32, 8, 833, 833, 64, "f16", "key groups=1, waves=4"),
     (2, 32, 8, 1100, 900, 128, "bf16", "key groups=1, waves=4"), (2, 64, 8, 1153, 1153, 96, "f16", "waves=8, waves per SIMD=4"),
-    (2, 32, 8, 2177, 2177, 128, "bf16", "waves=8, waves per SIMD=2> workgroups=576, V as fp16"), (2, 32, 8, 2177, 2177, 128, "f16", "waves=8, waves per SIMD=2"),
+    (2, 32, 8, 2177, 2177, 128, "bf16", "waves=8, waves per SIMD=2> workgroups=576, two heads each, V as fp16"), (2, 32, 8, 2177, 2177, 128, "f16", "waves=8, waves per SIMD=2"),
     (4, 33, 3, 300, 511, 256, "bf16", "waves=8"), (1, 128, 16, 833, 833, 96, "f16", "pair_kernel"), (3, 85, 5, 385, 1000, 64, "f16", "pair_kernel"),
     (2, 20, 4, 577, 577, 64, "f32", "prefill_f32_split_kernel<D=64, causal, key groups=2> rows=64"),
     (1, 32, 8, 1217, 1217, 96, "f32", "prefill_f32_split_kernel<D=96, causal, key groups=2> rows=128"),

@@ -1,4 +1,4 @@
-"""Causal launches at head dim 128 whose workgroups take two query heads of one KV head: both head maps, groups of two to eight heads,
+"""Causal launches whose workgroups take two query heads of one KV head: both head maps, groups of two to eight heads,
 ragged row tiles and lengths, head dims below the tiling, against softmax in 64 bits."""
 import numpy as np
 import pytest
@@ -16,7 +16,9 @@ def attend(lm, hip, q, k, v, dtype, head_map, kv_len):
 
 @pytest.mark.parametrize("B,Hkv,G,S,D,dtype,ragged", [(10, 2, 4, 1300, 128, "f16", False), (12, 2, 2, 2049, 128, "bf16", True),
                                                       (5, 3, 6, 1153, 104, "bf16", False), (9, 4, 4, 769, 112, "f16", True),
-                                                      (13, 4, 2, 1030, 128, "bf16", False), (13, 2, 8, 513, 120, "f16", False)])
+                                                      (13, 4, 2, 1030, 128, "bf16", False), (13, 2, 8, 513, 120, "f16", False),
+                                                      (16, 4, 2, 1024, 128, "bf16", True), (7, 4, 2, 1994, 64, "bf16", False), (10, 4, 4, 1024, 64, "bf16", True),
+                                                      (15, 3, 8, 434, 96, "f16", False), (8, 5, 4, 1792, 96, "bf16", False), (5, 3, 8, 2310, 80, "bf16", True)])
 def test_two_heads_of_a_workgroup(lm, hip, oracle, B, Hkv, G, S, D, dtype, ragged):
     H = Hkv * G
     q, k, v = (oracle.round_to(oracle.gen_normal((B, h, S, D), 51000 + S + i), dtype) for i, h in enumerate((H, Hkv, Hkv)))
@@ -25,7 +27,8 @@ def test_two_heads_of_a_workgroup(lm, hip, oracle, B, Hkv, G, S, D, dtype, ragge
         lens[0], lens[1] = S, 0
     rows = [0, 1, 31, 32, 127, 128, 129, S // 2, S - 130, S - 1]
     for head_map in (0, 1):
-        assert "joined two by two" in lm.flash_attention_plan(q.shape, k.shape, dtype, True)
+        plan = lm.flash_attention_plan(q.shape, k.shape, dtype, True)
+        assert "joined two by two" in plan or "two heads each" in plan
         got = attend(lm, hip, q, k, v, dtype, head_map, lens)
         for b in (0, 1, B - 1):
             n = S if lens is None else int(lens[b])
