@@ -216,7 +216,7 @@ size_t lmh_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lm
 int32_t lmh_decode_auto_splits(int32_t B, int32_t Hkv, int32_t Lmax);
 int lmh_decode_attn(const lmh_decode_params *p);
 
-/* ---- one decode step of a cached attention layer in two launches: append + attend.
+/* ---- one decode step of a cached attention layer in one or two launches: append + attend.
  * Replaces, for one layer, what decode_step! does with the self-attention caches (reference
  * src/Whisper.jl:761-801: feed the caches in, run whisper_self_attn_cached :584-620, take the rebuilt caches
  * out) and the rotary embedding of this step's q and k in front of it (src/NN.jl:356-358).
@@ -227,7 +227,8 @@ int lmh_decode_attn(const lmh_decode_params *p);
  *     and x->v_new; out = attention of q over rows 0 .. kv_len[b] inclusive. q itself is not modified.
  *   - num_splits == 0 takes up to lmh_decode_step_splits(); an explicit count must be >= 2; the workspace is
  *     lmh_decode_workspace_bytes(..., that count).
- * The first launch is the split kernel of lmh_decode_attn over the old rows, rotating q as it loads it; the second
+ * Short walks with an open count take one launch, a workgroup per (sequence, KV head) pair, and no workspace. Otherwise the first
+ * launch is the split kernel of lmh_decode_attn over the old rows, rotating q as it loads it; the second
  * merges the partials, adds the new row from k_new / v_new and stores it into the caches, so the separate append
  * launch (lmh_kv_append) disappears. fp16 / bf16 on the matrix-core decode kernel only (head dims 64, 128, 256;
  * 96 with the interleaved pairing); anything else returns LMH_E_UNSUPPORTED and the caller uses

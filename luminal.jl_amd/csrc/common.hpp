@@ -72,7 +72,7 @@ struct DecodeArgs {
   float *ws_o;    // [B][Hq][num_splits][D] un-normalised partial outputs
   float *ws_ml;   // [B][Hq][num_splits][2] (running max in log2 units, partial sum)
   // lmh_decode_step: the split kernel attends the kv_len[b] rows already in the cache with q rotated as it is loaded;
-  // the merge kernel adds row kv_len[b] from k_new / v_new (K rotated) and writes it into the caches.
+  // the merge kernel adds row kv_len[b] from k_new / v_new (K rotated) and writes it into the caches. Short steps do it all in one.
   int32_t step;             // 0: plain decode attention
   int32_t q_rope;           // rotate q (and k_new) at position kv_len[b]
   int32_t rope_interleaved;

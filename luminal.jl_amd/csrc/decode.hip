@@ -483,8 +483,7 @@ __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(DecodeArgs 
   merge_row<E, STEP>(a, blockIdx.x, blockIdx.y);
 }
 // ... of a step whose operands lie in the caller's arrays: further workgroups copy those into the graph's buffers, which nothing
-// else in the step waits for (bf16 steps of B=1 H=32/8 L=512 D=128: 15.3 us with the copy in front, 12.6 here; B=16 L=4096: 53.5
-// and 50.3).
+// else in the step waits for (bf16 steps of B=16 H=32/8 L=4096 D=128: 53.5 us with the copy in front, 50.3 here).
 template <typename E>
 __global__ __launch_bounds__(kMergeThreads) void decode_merge_fed_kernel(DecodeArgs a, CopyManyArgs fed, int n_copies) {
   request_args(a);

@@ -802,7 +802,7 @@ bool decode_mfma_rope_ok(int D, int interleaved) { return interleaved || (D / 32
 // Whether a pair's whole walk in one workgroup (decode_pair_kernel, with one split) is the fastest form. By 12 000 launches, both ways
 // timed on each (1 to 640 pairs, 64 to 4096 keys, D = 64 to 256): where it is taken steps take 0.66 of the two launches' time and
 // decodes 0.85 of the split kernel's, on average; the worst 1.06 (steps) and 1.1 (ragged decodes of 128 pairs). us, steps, D = 128 bf16,
-// H=32/8: L=128 12.8 -> 6.2 (what the host takes for a call), L=512 12.8 -> 8.0, L=1024 13.0 -> 10.3 (L=1500 13.6 -> 15), B=16 L=512 16.1
+// H=32/8: L=128 12.8 -> 6.2 (what the host takes for a call), L=512 12.8 -> 8.0 (7.5 since), L=1024 13.0 -> 10.3 (L=1500 13.6 -> 15), B=16 L=512 16.1
 // -> 10.8, B=32 L=512 20.7 -> 14.5; decodes L=512 10.6 -> 7.3 (L=1024 11.9 -> 12.1), D=64 B=1 L=700 9.1 -> 6.7 (L=1500 9.5 -> 10.2). Few pairs:
 // as long as one CU's walk is not longer than the merge launch and what more CUs gain. From 112 pairs on the CUs are at work either way,
 // and the walk may be longer: D=128 128 pairs L=2048 a step 0.95, a decode 0.98, ragged 1.1. More pairs than CUs go round in rounds.

@@ -387,7 +387,7 @@ class DecodeAttentionOp(Op):
 
 
 class DecodeStepOp(Op):
-    """One decode step of a cached attention layer as ONE node and two launches (lmh_decode_step): inputs
+    """One decode step of a cached attention layer as ONE node and one or two launches (lmh_decode_step): inputs
     (q (B,Hq,D), k_cache, v_cache, k_new (B,Hkv,1,D), v_new, pos int32[B]); output 0 is the attention result over rows
     0 .. pos[b] inclusive, outputs 1 and 2 are the caches themselves with row pos[b] written (K rotated when rope_base
     is set; q is rotated inside the kernel and left as it was). What decode_step! and whisper_self_attn_cached do for
@@ -825,7 +825,7 @@ def cached_self_attention_core(q, k_new, v_new, k_cache, v_cache, pos, kv_len, r
     k_cache, v_cache)."""
     g = q.graph_ref
     if fused and len(q.shape) == 4 and q.shape[2] == 1 and decode_step_supported(g.dtypes[q.id], q.shape[-1], rope_base is not None):
-        # one node, two launches: the split kernel rotates q as it loads it, the merge launch adds and stores the new row
+        # one node, two launches (one for short walks): the split kernel rotates q as it loads it, the merge adds and stores the new row
         # (`kv_len` is not needed: the step attends rows 0 .. pos[b])
         q3 = GraphTensor(q.id, (q.shape[0], q.shape[1], q.shape[3]), g, q.index)
         return decode_step(q3, k_cache, v_cache, k_new, v_new, pos, scale=scale, head_map=head_map, num_splits=num_splits,

@@ -321,7 +321,7 @@ execute_op(op::DecodeAttentionOp, q::HipArray, kc::HipArray, vc::HipArray, kv_le
     execute_op!(similar(q), op, q, kc, vc, kv_len)
 
 # ------------------------------------------------------------------------------------------
-# DecodeStepOp: one decode step of a cached attention layer as one node and two launches (lmh_decode_step): what
+# DecodeStepOp: one decode step of a cached attention layer as one node and one or two launches (lmh_decode_step): what
 # decode_step! and whisper_self_attn_cached do for one layer (src/Whisper.jl:761-801, :584-620) with the rotary embedding
 # of src/NN.jl:356-358. Inputs (q, k_cache, v_cache, k_new, v_new, pos); the value of the node is the attention result
 # over rows 0 .. pos[b] inclusive; the caches are updated in place (row pos[b]; K rotated when rope_base is set); q is
@@ -540,7 +540,7 @@ function cached_self_attention_core!(out::HipArray{TO,3}, q::HipArray{T,4}, k_ne
                                      head_map::Int32=HEADMAP_INTERLEAVED, fused::Bool=false) where {TO,T}
     size(q, 3) == 1 || error("cached attention takes one query token per sequence")
     if fused && decode_step_supported(T, size(q, 4); rope=(rope_base !== nothing))
-        # two launches instead of three: the split kernel rotates q as it loads it, the merge launch adds and stores the new row
+        # two launches (one for short walks) instead of three: the split kernel rotates q, the merge adds and stores the new row
         s = isnothing(scale) ? 1.0f0 / sqrt(Float32(size(q, 4))) : Float32(scale)
         q3 = HipArray{T,3}(q.ptr, (size(q, 1), size(q, 2), size(q, 4)), q)
         return execute_op!(out, DecodeStepOp(s, head_map, Float32(something(rope_base, 0.0f0))), q3, kc, vc, k_new, v_new, pos)
