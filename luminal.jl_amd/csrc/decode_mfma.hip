@@ -804,12 +804,15 @@ bool decode_mfma_rope_ok(int D, int interleaved) { return interleaved || (D / 32
 // decodes 0.85 of the split kernel's, on average; the worst 1.06 (steps) and 1.1 (ragged decodes of 128 pairs). us, steps, D = 128 bf16,
 // H=32/8: L=128 12.8 -> 6.2 (what the host takes for a call), L=512 12.8 -> 8.0 (7.5 since), L=1024 13.0 -> 10.3 (L=1500 13.6 -> 15), B=16 L=512 16.1
 // -> 10.8, B=32 L=512 20.7 -> 14.5; decodes L=512 10.6 -> 7.3 (L=1024 11.9 -> 12.1), D=64 B=1 L=700 9.1 -> 6.7 (L=1500 9.5 -> 10.2). Few pairs:
-// as long as one CU's walk is not longer than the merge launch and what more CUs gain. From 112 pairs on the CUs are at work either way,
+// as long as one CU's walk is not longer than the merge launch and what more CUs gain. That line was drawn again when both
+// forms had become faster, pair / split: steps D=128 B=6 H=8 L=1084 9.1 / 11.3, B=12 Hkv=1 L=1200 9.9 / 10.9, B=9 Hkv=4 L=1373 13.8 / 12.2, D=256 L=509 12.5 /
+// 14.3, L=532 17.2 / 16.4, D=64 L=1575 9.7 / 10.3, L=2526 16.6 / 12.5; decodes D=64 B=22 Hkv=2 L=1367 9.4 / 10.5, L=2040 10.2 / 10.2, D=96 B=17 L=1172 8.3 /
+// 9.1, B=3 H=20 L=1197 11.5 / 10.5, D=128 B=3 L=750 8.6 / 10.4, B=5 H=64/16 L=1137 14.4 / 13.3. From 112 pairs on the CUs are at work either way,
 // and the walk may be longer: D=128 128 pairs L=2048 a step 0.95, a decode 0.98, ragged 1.1. More pairs than CUs go round in rounds.
 bool decode_by_pairs(const DecodeArgs &a) {
   const int64_t cus = device_cu_count(), pairs = (int64_t)a.B * a.Hkv * ((a.Hq / a.Hkv + 15) / 16), walk = (int64_t)a.Lmax * a.D;
   const bool many = pairs * 16 >= cus * 7;
-  if (!many) return walk <= (a.step ? (a.D > 96 ? 110000 : 90000) : (a.D > 96 ? 95000 : 78000));
+  if (!many) return walk <= (a.step ? (a.D > 128 ? 125000 : a.D > 96 ? 140000 : 105000) : (a.D > 96 ? 125000 : 100000));
   if (!a.step) return walk <= 160000 && pairs <= cus && (a.D > 64 || pairs * 5 <= cus * 4);
   const int64_t rounds = (pairs + cus - 1) / cus;
   return walk <= (rounds == 1 || pairs * 20 >= rounds * cus * 17 ? 262144 : 50000);

@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 CASES = [  # D, Lmax, group, dtype
     (64, 1100, 1, "f16"), (64, 513, 5, "bf16"), (64, 40, 9, "f16"), (96, 700, 4, "bf16"), (96, 385, 8, "f16"), (96, 130, 17, "bf16"),
     (128, 260, 4, "bf16"), (128, 700, 6, "bf16"), (128, 512, 8, "f16"), (128, 33, 20, "f16"), (256, 350, 2, "f16"), (256, 129, 7, "bf16"),
+    (64, 1560, 3, "f16"), (96, 1040, 2, "bf16"), (128, 976, 4, "f16"), (256, 488, 1, "bf16"),  # the longest walks of few pairs
 ]
 
 
