@@ -94,3 +94,22 @@ def test_new_rows_off_alignment(lm, hip, oracle, D, group, dtype):
 
     for a, b in zip(step(0), step(1)):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("B,Hkv,G,L,D,dtype,step", [(50, 4, 2, 2250, 128, "bf16", False), (33, 7, 1, 1100, 256, "f16", False), (28, 8, 1, 4600, 64, "f16", False),
+                                                    (45, 8, 2, 1300, 128, "f16", True), (36, 8, 1, 660, 256, "bf16", True)])
+def test_long_walks_of_many_pairs(lm, hip, oracle, B, Hkv, G, L, D, dtype, step):
+    """Nearly a pair per CU, or steps whose last round of pairs is part full, at the longest walks that still take one launch."""
+    q, kn, vn, kc, vc = step_inputs(oracle, B, Hkv * G, Hkv, L, D, dtype, 44000 + L)
+    lens = np.random.default_rng(L).integers(1, L, size=B).astype(np.int32)
+    lens[:3] = (L - 1, 1, 0)
+    if step:
+        got, kc_after, vc_after = run_step(lm, hip, q, kn, vn, kc, vc, lens, dtype, True, False)
+        want, _, _ = expected(oracle, q, kn, vn, kc, vc, lens, dtype, True, False, 0)
+        np.testing.assert_array_equal(vc_after[0, :, L - 1], vn[0, :, 0])
+        assert rel_err(got, want) <= TOL[dtype]
+    else:
+        got = run_decode(lm, hip, q[:, :, 0], kc, vc, dtype, kv_len=lens, out_dtype="f32")
+        some = lens > 0
+        want = oracle.decode_attn(q[some][:, :, 0], kc[some], vc[some], kv_len=lens[some], nthreads=16)
+        assert rel_err(got[some], want) <= TOL[dtype] and not got[~some].any()
