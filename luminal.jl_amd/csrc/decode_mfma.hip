@@ -809,16 +809,20 @@ bool decode_mfma_rope_ok(int D, int interleaved) { return interleaved || (D / 32
 // 14.3, L=532 17.2 / 16.4, D=64 L=1575 9.7 / 10.3, L=2526 16.6 / 12.5; decodes D=64 B=22 Hkv=2 L=1367 9.4 / 10.5, L=2040 10.2 / 10.2, D=96 B=17 L=1172 8.3 /
 // 9.1, B=3 H=20 L=1197 11.5 / 10.5, D=128 B=3 L=750 8.6 / 10.4, B=5 H=64/16 L=1137 14.4 / 13.3. From 112 pairs on the CUs are at work either way,
 // and the walk may be longer: D=128 128 pairs L=2048 a step 0.95, a decode 0.98, ragged 1.1. More pairs than CUs go round in rounds.
-// Decodes of 195 to 256 pairs, walks of 160 to 300 thousand elements, 22 launches: 0.86 of the split kernel's time on average, 0.77 to 0.98, D=64 on all CUs
-// 1.04 (B=56 Hkv=4 L=1493 D=128 31.5 -> 26.8); of 112 pairs that long 1.27. Steps of D=128 and 256 whose last round of two or three is part full, walks of 50 to 170 thousand, 15
-// launches: 0.80 on average, the worst 1.00 (B=50 L=760 ragged 33.7 -> 23.6), beyond that up to 1.04; D=64 0.80 to 1.08, which stays.
+// On 192 to 256 CUs a pair each, 42 launches: decodes of walks of 160 to 450 thousand elements 0.87 of the split kernel's time on average, 0.77 to 0.98 (B=56
+// Hkv=4 L=1493 D=128 31.5 -> 26.8; D=64 on all CUs 1.04; beyond, 0.94 to 1.10), steps of 262 to 500 thousand 0.81 to 0.94 (B=24 H=64/8 L=2106 D=256 82.9 -> 67.0).
+// Of 112 pairs that long 1.16 to 1.5. Steps of two or three rounds: the last nearly full, up to 300 thousand, 0.81 to 0.98; part full, D=128 and 256, 50 to 170
+// thousand 0.80 on average, the worst 1.00 (B=50 L=760 ragged 33.7 -> 23.6), beyond that up to 1.04; D=64 0.80 to 1.08, which stays. Decodes of two or three rounds 0.78
+// to 1.2, which stay.
 bool decode_by_pairs(const DecodeArgs &a) {
   const int64_t cus = device_cu_count(), pairs = (int64_t)a.B * a.Hkv * ((a.Hq / a.Hkv + 15) / 16), walk = (int64_t)a.Lmax * a.D;
   const bool many = pairs * 16 >= cus * 7;
   if (!many) return walk <= (a.step ? (a.D > 128 ? 125000 : a.D > 96 ? 140000 : 105000) : (a.D > 96 ? 125000 : 100000));
-  if (!a.step) return pairs <= cus && walk <= (pairs * 4 >= cus * 3 ? 300000 : 160000) && (a.D > 64 || pairs * 20 <= cus * 19);
+  const bool nearly_all = pairs * 4 >= cus * 3;
+  if (!a.step) return pairs <= cus && walk <= (nearly_all ? 450000 : 160000) && (a.D > 64 || pairs * 20 <= cus * 19);
   const int64_t rounds = (pairs + cus - 1) / cus;
-  return walk <= (rounds == 1 || pairs * 20 >= rounds * cus * 17 ? 262144 : a.D > 96 ? 170000 : 50000);
+  if (rounds == 1) return walk <= (nearly_all ? 500000 : 262144);
+  return walk <= (pairs * 20 >= rounds * cus * 17 ? 300000 : a.D > 96 ? 170000 : 50000);
 }
 
 bool decode_mfma_supported(int dtype, int D, int B) {
