@@ -1488,7 +1488,7 @@ template <typename MT, bool V16, int KSPLIT> struct base_policy { using type = M
 template <> struct base_policy<MfmaBF16, true, 1> { using type = MfmaBF16V16; };
 
 template <typename MT0, bool V16, int D, int KSPLIT, int NW, int WPS = default_wps<D, NW>(), bool AHEAD = false, int HEADS = 1>
-int launch_split(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream, bool joined = false) {  // joined: named as the workgroups of one head that it joins
+int launch_split(const PrefillArgs &a, const QueryCopy &queries, hipStream_t stream) {
   using MT = typename base_policy<MT0, V16, KSPLIT>::type;
   constexpr int BM = 32 * NW / KSPLIT / HEADS;
   const int n_q_tiles = (a.Sq + BM - 1) / BM;
@@ -1497,8 +1497,7 @@ int launch_split(const PrefillArgs &a, const QueryCopy &queries, hipStream_t str
   if (rc != LMH_OK) return rc;
   dim3 grid((uint32_t)wgs), block(64 * NW);
   if (plan_only("prefill_mfma_kernel<%s, D=%d, %s, key groups=%d, waves=%d, waves per SIMD=%d> workgroups=%u%s%s%s", MT::kName, D,
-                a.causal ? "causal" : "full", KSPLIT, joined ? NW / 2 : NW, WPS, joined ? (uint32_t)deal_grid((int64_t)a.B * a.Hq, n_q_tiles) : grid.x,
-                joined ? ", joined two by two" : HEADS == 2 ? ", two heads each" : "", MT::kConvertV ? ", V as fp16" : "", AHEAD ? ", a tile ahead" : ""))
+                a.causal ? "causal" : "full", KSPLIT, NW, WPS, grid.x, HEADS == 2 ? ", two heads each" : "", MT::kConvertV ? ", V as fp16" : "", AHEAD ? ", a tile ahead" : ""))
     return LMH_OK;
   const Deal deal = make_deal(a.B, a.Hq / HEADS, n_q_tiles, a.causal ? 4 * WPS / NW : 0, device_cu_count());
   if (a.causal)
@@ -1686,7 +1685,7 @@ int launch_cheapest(const PrefillArgs &a, const QueryCopy &queries, int by_size,
         if (best == kRows256Pair) return two ? launch_split<MT, V, D, 1, 8, 4, false, 2>(a, queries, stream) : launch_split<MT, V, D, 1, 8>(a, queries, stream);
     } else if constexpr (!MT::kSplitP || V) {
       if (best == kRows256 ? two : best == kRows128 && two && two_heads_ahead(a, V, n_cus))
-        return launch_split<MT, V, D, 1, 8, 2, false, 2>(a, queries, stream, best == kRows128);
+        return launch_split<MT, V, D, 1, 8, 2, false, 2>(a, queries, stream);
       if (best == kRows256) return launch_split<MT, V, D, 1, 8>(a, queries, stream);
     }
     return launch_split<MT, V, D, 1, 4>(a, queries, stream);

@@ -203,8 +203,10 @@ def test_kernel_plan_of_the_benchmark_configurations(lm):
     assert "key groups=2, waves=4" in plan((4, 20, 448, 64), (4, 20, 1500, 64), "f16", True)
     # 64 heads: two 64-row workgroups per CU already balance
     assert "prefill_mfma_kernel<f16, D=64, full, key groups=2" in plan((4, 16, 448, 64), (4, 16, 1500, 64), "f16", False)
-    # a last tile of 9 rows: 128-row workgroups walk fewer tiles than 256-row ones
-    assert "key groups=1, waves=4, waves per SIMD=2> workgroups=896" in plan((4, 32, 777, 128), (4, 8, 777, 128), "f16", True)
+    # seven row tiles of 128 rows walk fewer key tiles than four of 256; an even group goes two heads to a workgroup, eight waves on
+    # half as many workgroups
+    assert plan((4, 33, 777, 128), (4, 11, 777, 128), "f16", True).endswith("key groups=1, waves=4, waves per SIMD=2> workgroups=928")
+    assert plan((4, 32, 777, 128), (4, 8, 777, 128), "f16", True).endswith("key groups=1, waves=8, waves per SIMD=2> workgroups=448, two heads each")
     # weights that are head + remainder by the rules for the length stay so, whatever V as fp16 would cost
     assert not plan((11, 32, 843, 96), (11, 8, 843, 96), "bf16", False).endswith("V as fp16")
     # head dims the matrix-core kernels do not tile, unaligned scale

@@ -141,7 +141,8 @@ def test_blocks_of_32_rotate_their_queries_in_registers(lm, hip, oracle, Hq, Sk,
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,dtype,form", [
     (13, 6, 6, 730, 730, 64, False, "f16", "key groups=1, waves=8, waves per SIMD=2>"), (10, 20, 20, 408, 65, 80, False, "f16", "key groups=1, waves=8, waves per SIMD=4>"),
     (1, 19, 19, 3000, 100, 120, False, "f16", "key groups=1, waves=4, waves per SIMD=2>"), (2, 16, 4, 777, 777, 128, True, "f16", "key groups=2, waves=4"),
-    (4, 32, 8, 777, 777, 128, True, "f16", "key groups=1, waves=4"), (5, 20, 20, 115, 67, 64, False, "f16", "key groups=2, waves=4"),
+    (4, 33, 11, 777, 777, 128, True, "f16", "key groups=1, waves=4, waves per SIMD=2> workgroups=928"),
+    (4, 32, 8, 777, 777, 128, True, "f16", "key groups=1, waves=8, waves per SIMD=2> workgroups=448, two heads each"), (5, 20, 20, 115, 67, 64, False, "f16", "key groups=2, waves=4"),
     (5, 16, 16, 119, 119, 80, True, "bf16", "key groups=2, waves=4"), (6, 16, 4, 431, 431, 72, True, "bf16", "key groups=2, waves=4"),
     (3, 33, 11, 1285, 1285, 128, True, "bf16", "waves=4, waves per SIMD=2> workgroups=1096, V as fp16"),
 ])

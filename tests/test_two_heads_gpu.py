@@ -28,7 +28,7 @@ def test_two_heads_of_a_workgroup(lm, hip, oracle, B, Hkv, G, S, D, dtype, ragge
     rows = [0, 1, 31, 32, 127, 128, 129, S // 2, S - 130, S - 1]
     for head_map in (0, 1):
         plan = lm.flash_attention_plan(q.shape, k.shape, dtype, True)
-        assert "joined two by two" in plan or "two heads each" in plan
+        assert "waves=8" in plan and "two heads each" in plan
         got = attend(lm, hip, q, k, v, dtype, head_map, lens)
         for b in (0, 1, B - 1):
             n = S if lens is None else int(lens[b])
