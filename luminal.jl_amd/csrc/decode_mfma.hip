@@ -484,8 +484,8 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeDeal dea
   }
 }
 
-// A (b, kv head slice) pair's whole walk in one workgroup, for launches of few keys and at most about one pair per CU: no partials
-// in memory and no second launch. What bounds these launches is latency: the kernel's chain of round trips and barriers, and the start
+// A (b, kv head slice) pair's whole walk in one workgroup, for the launches that decode_by_pairs names: no partials in memory and no
+// second launch. What bounds these launches is latency: the kernel's chain of round trips and barriers, and the start
 // of a second kernel behind it. So as many waves as LDS holds take a 32-key block each (256 keys at once at D = 128), straight into LDS
 // in whole rows (K into the MFMA's layout, 16 rows x 64 bytes a load, reads every line twice: a step of 512 keys 12.6 us, 10.5 this
 // way), and q, which every wave needs, is rotated once by the whole workgroup. Bank conflicts of the sums' rows and of V's transposing
@@ -799,30 +799,39 @@ int launch_for_type(const DecodeArgs &a, const CopyManyArgs *fed, int n_copies, 
 // The query rotation of lmh_decode_step happens in registers: the partner of every element must be in the same lane.
 bool decode_mfma_rope_ok(int D, int interleaved) { return interleaved || (D / 32) % 2 == 0; }
 
-// Whether a pair's whole walk in one workgroup (decode_pair_kernel, with one split) is the fastest form. By 12 000 launches, both ways
-// timed on each (1 to 640 pairs, 64 to 4096 keys, D = 64 to 256): where it is taken steps take 0.66 of the two launches' time and
-// decodes 0.85 of the split kernel's, on average; the worst 1.06 (steps) and 1.1 (ragged decodes of 128 pairs). us, steps, D = 128 bf16,
-// H=32/8: L=128 12.8 -> 6.2 (what the host takes for a call), L=512 12.8 -> 8.0 (7.5 since), L=1024 13.0 -> 10.3 (L=1500 13.6 -> 15), B=16 L=512 16.1
-// -> 10.8, B=32 L=512 20.7 -> 14.5; decodes L=512 10.6 -> 7.3 (L=1024 11.9 -> 12.1), D=64 B=1 L=700 9.1 -> 6.7 (L=1500 9.5 -> 10.2). Few pairs:
-// as long as one CU's walk is not longer than the merge launch and what more CUs gain. That line was drawn again when both
-// forms had become faster, pair / split: steps D=128 B=6 H=8 L=1084 9.1 / 11.3, B=12 Hkv=1 L=1200 9.9 / 10.9, B=9 Hkv=4 L=1373 13.8 / 12.2, D=256 L=509 12.5 /
-// 14.3, L=532 17.2 / 16.4, D=64 L=1575 9.7 / 10.3, L=2526 16.6 / 12.5; decodes D=64 B=22 Hkv=2 L=1367 9.4 / 10.5, L=2040 10.2 / 10.2, D=96 B=17 L=1172 8.3 /
-// 9.1, B=3 H=20 L=1197 11.5 / 10.5, D=128 B=3 L=750 8.6 / 10.4, B=5 H=64/16 L=1137 14.4 / 13.3. From 112 pairs on the CUs are at work either way,
-// and the walk may be longer: D=128 128 pairs L=2048 a step 0.95, a decode 0.98, ragged 1.1. More pairs than CUs go round in rounds.
-// On 192 to 256 CUs a pair each, 42 launches: decodes of walks of 160 to 450 thousand elements 0.87 of the split kernel's time on average, 0.77 to 0.98 (B=56
-// Hkv=4 L=1493 D=128 31.5 -> 26.8; D=64 on all CUs 1.04; beyond, 0.94 to 1.10), steps of 262 to 500 thousand 0.81 to 0.94 (B=24 H=64/8 L=2106 D=256 82.9 -> 67.0).
-// Of 112 pairs that long 1.16 to 1.5. Steps of two or three rounds: the last nearly full, up to 300 thousand, 0.81 to 0.98; part full, D=128 and 256, 50 to 170
-// thousand 0.80 on average, the worst 1.00 (B=50 L=760 ragged 33.7 -> 23.6), beyond that up to 1.04; D=64 0.80 to 1.08, which stays. Decodes of two or three rounds 0.78
-// to 1.2, which stay.
+// Whether a pair's whole walk in one workgroup (decode_pair_kernel, with one split) is taken. A launch of it lasts as long as its longest
+// pair, and the host knows the caches' length, not the sequences': of lengths that differ, one long sequence may stand beside many short
+// ones, whose keys the split kernel deals to all CUs. So wherever lengths are given (steps always) the line lies where one sequence
+// as long as the cache beside others of one key takes no longer than it did in the two launches before this kernel (1.03 of them at
+// most). Measured on 8300 launches (G = 1 to 20, D = 64 to 256, 2 to 8192 pairs; all lengths full, uniform below the cache's, one full
+// beside sixteenths, one full beside single keys), time against the split kernel (and the merge) of today, full / uniform / one
+// beside single keys:
+//   steps, few pairs: D=64 59 thousand elements a walk 1.03 / 0.94 / 1.00, 80 thousand 1.13 / 1.07 / 1.10; D=128 80 0.97 / 0.93 / 0.96, 103 1.12 /
+//     1.09 / 1.10; D=256 89 0.86 / 0.83 / 0.83, 123 1.07 / 0.97 / 1.04. On three eighths of the CUs and more the walk may be longer, D=128 112 to
+//     192 pairs 123 thousand 0.86 / 0.75 / 1.26, 160 0.90 / 0.90 / 1.45; D=128 and 256 on nearly all CUs, 160 0.83 / 0.74 / 1.24
+//   steps of several rounds: D=128 768 pairs 30 thousand 0.83 / 0.74 / 0.93, 167 0.91 / 0.81 / 0.98 and 8192 pairs 0.90 / 0.85 / 0.93, 289 up to 1.58 in
+//     the third; D=256 512 pairs 289 0.92 / 0.87 / 1.24. D=64 480 pairs 16 thousand 0.91 / 0.99 / 1.15, 30 1.33 in the third; 1024 pairs 16
+//     1.13 / 1.14 / 1.32, 8192 pairs of 64 keys 1.31 all full: a workgroup has the CU, its prologue and fold nothing beside them
+//   decodes: 16 pairs D=64 40 thousand 0.96 / 0.92 / 0.94, 80 1.23 / 1.21 / 1.22; D=128 59 0.98, 103 1.21; D=256 89 0.94, 103 1.16. From half the
+//     CUs on the split kernel takes walks up to 131 thousand in one split too: D=64 and 96 1.02 to 1.09 of its time, D=128 and 256 0.96 to 1.04
+//   decodes without lengths (all as long as the cache), 112 to 256 pairs: 0.73 to 0.97 of two launches up to 160 thousand, from three quarters
+//     of the CUs on 0.82 to 0.96 up to 440. With lengths 300 thousand on 256 pairs took 1.32, D=64 on 224 1.93 (one beside sixteenths).
 bool decode_by_pairs(const DecodeArgs &a) {
   const int64_t cus = device_cu_count(), pairs = (int64_t)a.B * a.Hkv * ((a.Hq / a.Hkv + 15) / 16), walk = (int64_t)a.Lmax * a.D;
-  const bool many = pairs * 16 >= cus * 7;
-  if (!many) return walk <= (a.step ? (a.D > 128 ? 125000 : a.D > 96 ? 140000 : 105000) : (a.D > 96 ? 125000 : 100000));
-  const bool nearly_all = pairs * 4 >= cus * 3;
-  if (!a.step) return pairs <= cus && walk <= (nearly_all ? 450000 : 160000) && (a.D > 64 || pairs * 20 <= cus * 19);
-  const int64_t rounds = (pairs + cus - 1) / cus;
-  if (rounds == 1) return walk <= (nearly_all ? 500000 : 262144);
-  return walk <= (pairs * 20 >= rounds * cus * 17 ? 300000 : a.D > 96 ? 170000 : 50000);
+  const int d = a.D > 128 ? 3 : a.D > 96 ? 2 : a.D > 64 ? 1 : 0;
+  const bool many = pairs * 8 >= cus * 3;
+  if (a.step) {
+    constexpr int32_t kFew[4] = {65536, 81920, 81920, 98304}, kMany[4] = {85000, 100000, 125000, 180000}, kAll[4] = {85000, 100000, 160000, 250000};
+    if (pairs <= cus) return walk <= (pairs * 8 >= cus * 7 ? kAll : many ? kMany : kFew)[d];
+    const int64_t rounds = (pairs + cus - 1) / cus;
+    if (d >= 2) return walk <= (d == 3 && pairs * 20 >= rounds * cus * 17 ? 300000 : 170000);
+    return rounds <= 4 && walk <= (rounds <= 2 ? (d ? 30000 : 16384) : (d ? 12288 : 8192));
+  }
+  constexpr int32_t kFew[4] = {65536, 73728, 81920, 98304}, kMany[4] = {65536, 73728, 105000, 140000};
+  if (d < 2 && pairs * 2 >= cus && walk <= 131072) return false;
+  if (pairs > cus || (d == 0 && pairs * 20 > cus * 19)) return false;
+  if (!a.kv_len && pairs * 16 >= cus * 7) return walk <= (pairs * 4 >= cus * 3 ? 450000 : 160000);
+  return walk <= (many ? kMany : kFew)[d];
 }
 
 bool decode_mfma_supported(int dtype, int D, int B) {

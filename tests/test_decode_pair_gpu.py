@@ -1,6 +1,6 @@
 """Short walks of decode attention and of decode steps, one workgroup per (sequence, KV head) pair: lengths at the edges of a wave's
 32 keys and of a round of all waves (128 to 512 keys), caches whose rows past the length are NaN, every head dim and the group sizes
-at which the pieces of the weights stop being columns of one product. Against the oracle, and steps against append + attend."""
+at which the pieces of the weights stop being columns of one product; which launches take it. Against the oracle, and steps against append + attend."""
 import numpy as np
 import pytest
 
@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 CASES = [  # D, Lmax, group, dtype
     (64, 1100, 1, "f16"), (64, 513, 5, "bf16"), (64, 40, 9, "f16"), (96, 700, 4, "bf16"), (96, 385, 8, "f16"), (96, 130, 17, "bf16"),
     (128, 260, 4, "bf16"), (128, 700, 6, "bf16"), (128, 512, 8, "f16"), (128, 33, 20, "f16"), (256, 350, 2, "f16"), (256, 129, 7, "bf16"),
-    (64, 1560, 3, "f16"), (96, 1040, 2, "bf16"), (128, 976, 4, "f16"), (256, 488, 1, "bf16"),  # the longest walks of few pairs
+    (64, 1560, 3, "f16"), (96, 1040, 2, "bf16"), (128, 976, 4, "f16"), (256, 488, 1, "bf16"),
+    (64, 1024, 2, "bf16"), (96, 768, 3, "f16"), (128, 640, 5, "f16"), (256, 384, 3, "bf16"),  # the longest walks of few pairs in one launch
 ]
 
 
@@ -96,20 +97,60 @@ def test_new_rows_off_alignment(lm, hip, oracle, D, group, dtype):
         np.testing.assert_array_equal(a, b)
 
 
-@pytest.mark.parametrize("B,Hkv,G,L,D,dtype,step", [(50, 4, 2, 2250, 128, "bf16", False), (33, 7, 1, 1100, 256, "f16", False), (28, 8, 1, 4600, 64, "f16", False),
-                                                    (45, 8, 2, 1300, 128, "f16", True), (36, 8, 1, 660, 256, "bf16", True)])
-def test_long_walks_of_many_pairs(lm, hip, oracle, B, Hkv, G, L, D, dtype, step):
-    """Nearly a pair per CU, or steps whose last round of pairs is part full, at the longest walks that still take one launch."""
+def launches(lm, hip, call):
+    """How many launches a decode or a step takes: one leaves the scratch for the partial results as it is."""
+    scratch = lm.host._workspaces
+    at = scratch.get(1 << 25, hip)[0]
+    scratch.buf.fill_bytes(0xff)
+    result = call()
+    assert scratch.buf.ptr == at
+    return result, 1 if np.isnan(scratch.buf.to_host()).all() else 2
+
+
+@pytest.mark.parametrize("B,Hkv,G,L,D,dtype,step,ragged,expected_launches", [
+    (50, 4, 2, 2250, 128, "bf16", False, True, 2), (33, 7, 1, 1100, 256, "f16", False, True, 2), (28, 8, 1, 4600, 64, "f16", False, True, 2),
+    (50, 4, 2, 3515, 128, "bf16", False, False, 1), (32, 8, 1, 820, 128, "f16", False, True, 1), (24, 5, 2, 546, 256, "bf16", False, True, 1),
+    (45, 8, 2, 1300, 128, "f16", True, True, 1), (36, 8, 1, 660, 256, "bf16", True, True, 1), (32, 8, 2, 1250, 128, "bf16", True, True, 1),
+    (28, 8, 1, 976, 256, "f16", True, True, 1), (30, 8, 1, 1328, 64, "bf16", True, True, 1), (24, 8, 1, 1041, 96, "f16", True, True, 1),
+    (55, 8, 1, 1171, 256, "bf16", True, True, 1), (40, 8, 3, 256, 64, "f16", True, True, 1), (50, 8, 1, 312, 96, "bf16", True, True, 1),
+    (100, 8, 1, 128, 96, "f16", True, True, 1)])
+def test_long_walks_of_many_pairs(lm, hip, oracle, B, Hkv, G, L, D, dtype, step, ragged, expected_launches):
+    """A good part of the CUs with a pair each, or several rounds of pairs, at the longest walks that still take one launch, and decodes beyond them."""
     q, kn, vn, kc, vc = step_inputs(oracle, B, Hkv * G, Hkv, L, D, dtype, 44000 + L)
     lens = np.random.default_rng(L).integers(1, L, size=B).astype(np.int32)
     lens[:3] = (L - 1, 1, 0)
     if step:
-        got, kc_after, vc_after = run_step(lm, hip, q, kn, vn, kc, vc, lens, dtype, True, False)
-        want, _, _ = expected(oracle, q, kn, vn, kc, vc, lens, dtype, True, False, 0)
+        rope = D != 96
+        (got, kc_after, vc_after), n = launches(lm, hip, lambda: run_step(lm, hip, q, kn, vn, kc, vc, lens, dtype, rope, False))
+        want, _, _ = expected(oracle, q, kn, vn, kc, vc, lens, dtype, rope, False, 0)
         np.testing.assert_array_equal(vc_after[0, :, L - 1], vn[0, :, 0])
         assert rel_err(got, want) <= TOL[dtype]
     else:
-        got = run_decode(lm, hip, q[:, :, 0], kc, vc, dtype, kv_len=lens, out_dtype="f32")
-        some = lens > 0
-        want = oracle.decode_attn(q[some][:, :, 0], kc[some], vc[some], kv_len=lens[some], nthreads=16)
+        kv_len = lens if ragged else None
+        got, n = launches(lm, hip, lambda: run_decode(lm, hip, q[:, :, 0], kc, vc, dtype, kv_len=kv_len, out_dtype="f32"))
+        some = lens > 0 if ragged else lens >= 0
+        want = oracle.decode_attn(q[some][:, :, 0], kc[some], vc[some], kv_len=lens[some] if ragged else None, nthreads=16)
         assert rel_err(got[some], want) <= TOL[dtype] and not got[~some].any()
+    assert n == expected_launches
+
+
+@pytest.mark.parametrize("B,Hkv,G,D,step,ragged,L,longer", [  # the longest walk in one launch (None: no walk is), and one beyond it
+    (1, 8, 4, 64, True, True, 1024, 1032), (2, 8, 4, 96, True, True, 853, 864), (1, 8, 4, 128, True, True, 640, 648), (4, 8, 2, 256, True, True, 384, 392),
+    (12, 8, 4, 128, True, True, 976, 1000), (32, 8, 4, 128, True, True, 1250, 1256), (32, 8, 2, 256, True, True, 976, 980),
+    (64, 8, 4, 128, True, True, 1328, 1336), (64, 8, 2, 256, True, True, 1168, 1176), (64, 8, 4, 64, True, True, 256, 264),
+    (128, 8, 1, 64, True, True, 128, 136), (1024, 8, 1, 64, True, True, None, 64), (256, 8, 4, 96, True, True, None, 64),
+    (1, 8, 4, 64, False, True, 1024, 1032), (1, 8, 4, 128, False, True, 640, 648), (64, 4, 4, 128, False, False, 3515, 3520),
+    (64, 4, 4, 128, False, True, 820, 3437), (28, 8, 1, 64, False, True, 2048, 2500)])
+def test_walks_of_one_launch(lm, hip, B, Hkv, G, D, step, ragged, L, longer):
+    """Caches whose lengths may differ go to one workgroup a pair only as far as one long sequence does not hold the others up."""
+    for n_keys, want in ((L, 1), (longer, 2)):
+        if n_keys is None:
+            continue
+        q, kn, vn = (lm.HipArray(shape, "f16", hip).fill_bytes(0) for shape in ((B, Hkv * G, D), (B, Hkv, 1, D), (B, Hkv, 1, D)))
+        kc, vc = (lm.HipArray((B, Hkv, n_keys, D), "f16", hip).fill_bytes(0) for _ in range(2))
+        lens = lm.to_device(np.full(B, n_keys - 1, np.int32), hip)
+        if step:
+            call = lambda: lm.execute_op(lm.DecodeStepOp(lm.default_scale(D), 0, 0, "f32", None, False), q, kc, vc, kn, vn, lens)
+        else:
+            call = lambda: lm.execute_op(lm.DecodeAttentionOp(lm.default_scale(D), 0, 0), q, kc, vc, *([lens] if ragged else []))
+        assert launches(lm, hip, call)[1] == want, n_keys
