@@ -1558,9 +1558,8 @@ int launch_wide(const PrefillArgs &a, int wgs_per_head, int n_waves, int mixed, 
 // The forms of prefill_mfma_kernel and what a launch of each costs.
 //
 // A launch lasts as long as its busiest CU, and where the sizes leave a last row tile or a last round nearly empty the forms
-// differ by up to 60 %: B=4 H=32 S=777 D=128 causal fp16 has four row tiles of 256 with 9 rows in the last (46.8 us) or seven of
-// 128 (40.2); B=1 H=16 S=4501 D=96 causal bf16 one and a half rounds of 128-row workgroups (173 us) or 1.1 rounds of 256-row
-// ones (106). The thresholds of launch_for_d were measured at powers of two. Hence an estimate from the launch's own tiles, in us:
+// differ by up to 60 %: B=1 H=16 S=4501 D=96 causal bf16 is one and a half rounds of 128-row workgroups (173 us) or 1.1 rounds of
+// 256-row ones (106). The thresholds of launch_for_d were measured at powers of two. Hence an estimate from the launch's tiles, in us:
 //   fixed + longest row tile x alone       while every CU has at most one workgroup, or
 //   the mean over the CUs x shared         when several share it (causal; the fourth powers blend the two), or
 //   whole rounds of equal workgroups       (no mask), + per_wg for every workgroup that a CU starts.
@@ -1569,6 +1568,9 @@ int launch_wide(const PrefillArgs &a, int wgs_per_head, int n_waves, int mixed, 
 // of powers of two, with every form timed on each: rms 5 to 13 %. The form of the rules by size is therefore left only for one
 // that is estimated 8 % cheaper: 337 of those launches change their form, 296 of them gain more than 5 %, two lose more than 5 %
 // (13 and 14 us), all 1916 together gain 2.5 % (with a margin of 4 % 2.9 %, and ten lose).
+// The fit was made when causal tiles began at row 0, every workgroup took one head and 16-bit results were stored 8 bytes at a time, and the
+// tiles are still counted so: the constants go with that count. Tiles counted as they are dealt now (causal_shift, two heads), with the
+// constants as they are, change the form of 168 of 4000 drawn causal launches, to 0.75 to 1.44 of the time, 0.99 on average and half of them to more.
 enum Form { kKeysSplit64, kRows128, kRows256, kRows256Pair };  // rows per workgroup; Pair: two 256-row workgroups on a CU
 struct FormCost {
   float fixed, alone, per_wg, shared[2];  // shared by two and by three workgroups; with one per CU: in a later round
