@@ -227,10 +227,10 @@ int lmh_decode_attn(const lmh_decode_params *p);
  *     and x->v_new; out = attention of q over rows 0 .. kv_len[b] inclusive. q itself is not modified.
  *   - num_splits == 0 takes up to lmh_decode_step_splits(); an explicit count must be >= 2; the workspace is
  *     lmh_decode_workspace_bytes(..., that count).
- * Short walks, and longer ones of nearly a pair per CU, with an open count take one launch, a workgroup per (sequence, KV head) pair,
- * and no workspace. Otherwise the first
- * launch is the split kernel of lmh_decode_attn over the old rows, rotating q as it loads it; the second
- * merges the partials, adds the new row from k_new / v_new and stores it into the caches, so the separate append
+ * Short walks with an open count take one launch, a workgroup per (sequence, KV head) pair, which leaves the workspace as it is; which
+ * walks are short depends on the sizes and on the device, so the workspace of lmh_decode_step_splits() is asked for all the same
+ * (LMH_E_WORKSPACE without it). Otherwise the first launch is the split kernel of lmh_decode_attn over the old rows, rotating q as it
+ * loads it; the second merges the partials, adds the new row from k_new / v_new and stores it into the caches, so the separate append
  * launch (lmh_kv_append) disappears. fp16 / bf16 on the matrix-core decode kernel only (head dims 64, 128, 256;
  * 96 with the interleaved pairing); anything else returns LMH_E_UNSUPPORTED and the caller uses
  * lmh_kv_append + lmh_decode_attn. The caller advances kv_len afterwards. */

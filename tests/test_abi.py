@@ -119,6 +119,21 @@ def test_decode_argument_errors(lm, kw, code):
     assert "lmh_decode_attn" in str(e.value)
 
 
+@pytest.mark.parametrize("Lmax", [128, 512, 4096])
+def test_a_step_asks_for_its_workspace_whatever_it_launches(lm, Lmax):
+    """Also where an open count ends in one launch that has no partials: what a caller has to hand over follows from the sizes alone."""
+    b = lm.binding
+    x = b.DecodeStepExtra()
+    x.k_new, x.v_new = 0x6000, 0x7000
+    need = b.decode_workspace_bytes(2, 8, 2, Lmax, 128, b.decode_step_splits(2, 2, Lmax))
+    for ws, size in ((0, 0), (0x5000, need - 1)):
+        with pytest.raises(lm.LuminalHipError) as e:
+            b.decode_step(_dec(lm, Lmax=Lmax, kv_len=0x8000, num_splits=0, workspace=ws, workspace_bytes=size), x)
+        assert e.value.code == b.LMH_E_WORKSPACE and "workspace of %d bytes" % need in str(e.value)
+    header = " ".join(open(os.path.join(ROOT, "include", "luminal_hip.h")).read().replace("*", " ").split())
+    assert "(LMH_E_WORKSPACE without it)" in header and "and no workspace. Otherwise" not in header
+
+
 def test_decode_workspace_and_split_heuristic(lm):
     b = lm.binding
     assert b.decode_workspace_bytes(2, 8, 2, 1024, 128, 1) == 0
