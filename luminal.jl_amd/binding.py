@@ -335,7 +335,7 @@ def decode_attn(params):
 
 
 def decode_step(params, extra):
-    """lmh_decode_step: append this step's K / V rows and attend, in two launches."""
+    """lmh_decode_step: append this step's K / V rows and attend, in one or two launches."""
     check(load().lmh_decode_step(ctypes.byref(params), ctypes.byref(extra)))
 
 

@@ -505,26 +505,23 @@ size_t lmh_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lm
 
 // Where the caller leaves the split count to the library, the matrix-core kernel takes fewer than lmh_decode_auto_splits where
 // that is faster (us with that count and with this one, D = 128 bf16 unless named; 190 sizes timed):
-//   * one, so that the merge launch and the partials drop out, where a workgroup walks a whole sequence in the time of that
-//     launch, or where the pairs fill the CUs and the walk is short beside the whole launch: B=1 Hkv=8 L=200 12.8 -> 9.2 and
-//     L=512 11.8 -> 11.2 (L=1024 12.1 -> 15.7; D=64 L=512 9.4 -> 7.9, L=1000 9.4 -> 10.5, with 96 pairs 13.4 -> 11.8), B=16
-//     L=1024 20.8 -> 18.7 (L=2100 33.5 -> 32.3, ragged 26.0 -> 28.8), B=64 L=512 ragged 35.1 -> 24.0, L=2100 92 -> 90 (L=4096
-//     169.6 -> 167.6, ragged 121.0 -> 120.6: within what cards differ by); the longer walks only where the last round of pairs
-//     is nearly full (B=81 Hkv=4 L=3522 D=64 54.5 -> 58.6);
+//   * one, so that the merge launch and the partials drop out, where a workgroup of a kernel of its own walks a whole pair
+//     (decode_by_pairs, steps as well), or where the pairs fill the CUs and the walk is short beside the whole launch: B=16 L=1024 20.8
+//     -> 18.7 (L=2100 33.5 -> 32.3, ragged 26.0 -> 28.8), B=64 L=512 ragged 35.1 -> 24.0, L=2100 92 -> 90 (L=4096 169.6 -> 167.6,
+//     ragged 121.0 -> 120.6: within what cards differ by); the longer walks only where the last round of pairs is nearly full
+//     (B=81 Hkv=4 L=3522 D=64 54.5 -> 58.6);
 //   * one unit per CU for few pairs, in chunks long enough for the merge: B=4 Hkv=8 L=2100 19.3 -> 16.0, L=8192 ragged
 //     28.4 -> 24.0, B=1 L=8192 19.0 -> 16.4, L=32768 41.4 -> 29.9. From 128 pairs on more units balance ragged batches better
 //     (B=16 L=4096 ragged 38.5 with 16, 39.9 with 2).
-// Shorter walks take one launch of a workgroup per pair, steps as well (decode_by_pairs). Other steps keep their two launches and with
-// them two splits at least; there, few are no better than more.
+// Other steps keep their two launches and with them two splits at least; there, few are no better than more.
 // The sums are the same fp32 sums in another order, and no less exact for it (the kernel adds a block's share once and holds the
 // weights in full): against 64 bits (2-norm, fp32 results) B=4 Hkv=8 L=512 D=128 bf16 1.57e-7 with four splits and 1.55e-7 with
 // one, D=64 fp16 1.56e-7 and 1.51e-7, B=1 L=32768 D=64 fp16 2.31e-7 with 256 and 2.13e-7 with 32.
 static int32_t decode_splits(const DecodeArgs &a, int32_t most) {
   const int64_t cus = device_cu_count(), pairs = (int64_t)a.B * a.Hkv * ((a.Hq / a.Hkv + 15) / 16), walk = (int64_t)a.Lmax * a.D;
-  const bool full = pairs * 20 >= (pairs + cus - 1) / cus * cus * 17;
-  const bool one = (walk <= 65536 && (a.Lmax <= 512 || pairs * 8 >= cus * 3)) || (walk <= 131072 && pairs >= cus / 2) || (walk <= 262144 && pairs >= cus && full);
   if (decode_by_pairs(a)) return 1;
-  if (one && !a.step) return 1;
+  const bool full = pairs * 20 >= (pairs + cus - 1) / cus * cus * 17;
+  if (!a.step && ((walk <= 131072 && pairs * 2 >= cus) || (walk <= 262144 && pairs >= cus && full))) return 1;
   const int64_t per_pair = cus / pairs;
   if (per_pair < 4 || per_pair * pairs * 8 < cus * 7) return most;
   const int64_t chunk = std::min(std::max(a.Lmax / 1024 * 64, 128), 512);

@@ -46,10 +46,8 @@ __device__ inline float load_as_f32(const void *p, int64_t i, int dtype) {
 // (the reference's column-major reshape of hidden into (heads, D) makes the head index the fast one).
 __device__ inline int b_column(const MatmulProblem &p, int D, int j) { return p.heads ? j / D + p.heads * (j % D) : j; }
 
-// Store R registers a lane of a wave's 32 x 32 block, R / 4 rows of it in fours: lane (n, h) holds column j, register i row
-// mw + 8 (i / 4) + 4 h + i % 4.
-template <int R, typename Acc>
-__device__ inline void store_block(const MatmulProblem &p, const Acc &acc, int mw, int j, int h, int batch) {
+// Store a wave's 32 x 32 block: lane (n, h) holds column j, register i row mw + 8 (i / 4) + 4 h + i % 4.
+__device__ inline void store_block(const MatmulProblem &p, const floatx16_t &acc, int mw, int j, int h, int batch) {
   if (j >= p.N || mw >= p.M) return;
   const int D = p.heads ? p.N / p.heads : 1;
   const float bias = p.bias ? load_as_f32(p.bias, b_column(p, D, j), p.bias_dtype) : 0.f;
@@ -69,7 +67,7 @@ __device__ inline void store_block(const MatmulProblem &p, const Acc &acc, int m
   }
   auto store_rows = [&](auto store) {
 #pragma unroll
-    for (int i = 0; i < R; i++) {
+    for (int i = 0; i < 16; i++) {
       const int r = 8 * (i >> 2) + 4 * h + (i & 3);
       if (mw + r >= p.M) break;  // rows ascend with i
       int64_t off = base + (int64_t)r * row_step;
@@ -278,7 +276,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void matmul_f32_kernel(Matmul
     }
   }
 
-  store_block<16>(p, acc, m0 + 32 * wm, n0 + 32 * wn + n, h, batch);
+  store_block(p, acc, m0 + 32 * wm, n0 + 32 * wn + n, h, batch);
 }
 
 // The same products for fp32 operands that are contiguous along the contraction, on the bf16 matrix pipe (16 times the rate).

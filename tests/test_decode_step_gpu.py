@@ -1,6 +1,6 @@
-"""lmh_decode_step: one decode step of a cached attention layer in two launches — the split kernel over the rows
-already in the caches with q rotated as it is loaded, then the merge launch that adds the new row from k_new / v_new
-and stores it (K rotated) into the caches. Checked through the C ABI against the CPU oracle (rope, cache append, decode
+"""lmh_decode_step: one decode step of a cached attention layer, short walks in one launch, others in two — the split kernel
+over the rows already in the caches with q rotated as it is loaded, then the merge launch that adds the new row from k_new /
+v_new and stores it (K rotated) into the caches. Checked through the C ABI against the CPU oracle (rope, cache append, decode
 attention: reference src/NN.jl:253-303, src/Whisper.jl:552-570, :584-620) and against the library's own three-launch
 path (lmh_kv_append + lmh_decode_attn)."""
 import numpy as np
