@@ -106,10 +106,11 @@ def test_decode_step_equals_append_then_attend(lm, hip, oracle, dtype):
     assert rel_err(got, out.to_host()) <= 2e-6
 
 
-def test_decode_step_graph_steps_through_positions(lm, hip, oracle):
+@pytest.mark.parametrize("Lmax,launches", [(512, 1), (1500, 2)])
+def test_decode_step_graph_steps_through_positions(lm, hip, oracle, Lmax, launches):
     """cached_self_attention_core(fused=True) is one node; one compiled graph serves every position, and the caches it
     holds afterwards are the rotated K and the raw V of all steps (as in the two-node form)."""
-    B, Hq, Hkv, S, D, Lmax, dtype = 2, 8, 2, 20, 64, 512, "f16"
+    B, Hq, Hkv, S, D, dtype = 2, 8, 2, 20, 64, "f16"
     q = oracle.round_to(oracle.gen_normal((B, Hq, S, D), 16600), dtype)
     k = oracle.round_to(oracle.gen_normal((B, Hkv, S, D), 16601), dtype)
     v = oracle.round_to(oracle.gen_normal((B, Hkv, S, D), 16602), dtype)
@@ -125,9 +126,12 @@ def test_decode_step_graph_steps_through_positions(lm, hip, oracle):
     for t in range(S):
         if t == 3:
             cg.capture()  # the step can be recorded like the two-node form
+        if t:
+            cg.workspaces.buf.fill_bytes(0xff)
         res = cg({tq.id: np.ascontiguousarray(q[:, :, t:t + 1]), tkn.id: np.ascontiguousarray(k[:, :, t:t + 1]),
                   tvn.id: np.ascontiguousarray(v[:, :, t:t + 1]), tpos.id: np.full(B, t, np.int32)})
         assert rel_err(res[out.id][0].to_host(), want[:, :, t]) <= TOL[dtype], t
+        assert t == 0 or np.isnan(cg.workspaces.buf.to_host()).all() == (launches == 1)  # (one launch has no partials)
     cg.release()
     assert rel_err(res[out.id][1].to_host()[:, :, :S], oracle.round_to(oracle.rope(k), dtype)) <= 8e-3
     np.testing.assert_array_equal(res[out.id][2].to_host()[:, :, :S], v)
@@ -150,13 +154,15 @@ def test_decode_step_refuses_what_it_cannot_take(lm, hip, oracle):
     assert isinstance(g.nodes[out.id].op, lm.DecodeAttentionOp)
 
 
-@pytest.mark.parametrize("dtype,B,Hq,Hkv,T,L,D,rope", [
-    ("bf16", 1, 4, 4, 1, 64, 64, True), ("f16", 5, 32, 2, 1, 700, 128, True), ("f16", 2, 12, 4, 1, 300, 96, True),  # steps; the last in two nodes
-    ("f32", 3, 6, 2, 1, 130, 64, True),  # ... that rotates the queries in place
-    ("f16", 2, 8, 2, 33, 64, 128, True), ("bf16", 1, 6, 3, 777, 800, 64, True), ("f16", 1, 8, 2, 300, 333, 256, False),  # prompts
-    ("f16", 3, 16, 16, 513, 600, 96, True), ("bf16", 2, 4, 1, 130, 200, 80, False), ("f16", 2, 4, 4, 16, 40, 80, True),
-    ("f32", 2, 4, 2, 257, 300, 64, False)])
-def test_operands_taken_from_the_callers_arrays(lm, hip, dtype, B, Hq, Hkv, T, L, D, rope):
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,T,L,D,rope,launches", [
+    ("bf16", 1, 4, 4, 1, 64, 64, True, 1), ("f16", 5, 32, 2, 1, 700, 128, True, 2), ("f16", 2, 12, 4, 1, 300, 96, True, None),  # steps; the last in two nodes
+    ("f16", 5, 32, 2, 1, 600, 128, True, 1), ("bf16", 3, 12, 4, 1, 500, 96, False, 1), ("f16", 2, 8, 4, 1, 300, 256, True, 1),
+    ("f16", 3, 32, 8, 1, 3000, 128, True, 2), ("bf16", 2, 8, 4, 1, 900, 256, True, 2), ("bf16", 2, 12, 4, 1, 1100, 96, False, 2),
+    ("f32", 3, 6, 2, 1, 130, 64, True, None),  # ... that rotates the queries in place
+    ("f16", 2, 8, 2, 33, 64, 128, True, None), ("bf16", 1, 6, 3, 777, 800, 64, True, None), ("f16", 1, 8, 2, 300, 333, 256, False, None),  # prompts
+    ("f16", 3, 16, 16, 513, 600, 96, True, None), ("bf16", 2, 4, 1, 130, 200, 80, False, None), ("f16", 2, 4, 4, 16, 40, 80, True, None),
+    ("f32", 2, 4, 2, 257, 300, 64, False, None)])
+def test_operands_taken_from_the_callers_arrays(lm, hip, dtype, B, Hq, Hkv, T, L, D, rope, launches):
     """A call of a compiled graph leaves the same memory behind whether its inputs are copied in front of the launches or read
     where they lie: the result, the caches and the graph's copies of the inputs, bit for bit. Also with inputs that rule
     the second out (a misaligned array, the graph's own result or cache as input) and with some left out."""
@@ -201,6 +207,13 @@ def test_operands_taken_from_the_callers_arrays(lm, hip, dtype, B, Hq, Hkv, T, L
     same = array(tkn)
     call({tkn.id: same, tvn.id: same, tq.id: lambda cg: result(cg).view(tq.shape)})
     call({tkc.id: array(tkc), tvn.id: array(tvn), tkn.id: lambda cg: cg.results[tvn.id]})
+    if launches:  # a step of one launch has no partials: their scratch stays as it is
+        fresh = {tq.id: array(tq), tkn.id: array(tkn), tvn.id: array(tvn), **at}
+        for cg in (fed, plain):
+            cg.workspaces.buf.fill_bytes(0xff)
+            cg(fresh)
+            lm.binding.sync()
+            assert np.isnan(cg.workspaces.buf.to_host()).all() == (launches == 1)
     if Hq * T <= Hkv * L:
         inside = lambda cg: (lambda v: (setattr(v, "shape", tq.shape), setattr(v, "nbytes", cg.results[tq.id].nbytes), v)[2])(cg.results[tvc.id].view(tvc.shape))
         call({tq.id: inside, tkn.id: array(tkn)})
