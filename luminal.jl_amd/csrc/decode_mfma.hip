@@ -33,6 +33,7 @@
 // chunk (the other chunk slots of the run get an "empty" marker the merge kernel skips).
 // Split-KV partial layout and the merge kernel are shared with decode.hip.
 #include <algorithm>
+#include <utility>
 
 #include "common.hpp"
 #include "copy.hpp"
@@ -799,6 +800,19 @@ int launch_for_type(const DecodeArgs &a, const CopyManyArgs *fed, int n_copies, 
 // The query rotation of lmh_decode_step happens in registers: the partner of every element must be in the same lane.
 bool decode_mfma_rope_ok(int D, int interleaved) { return interleaved || (D / 32) % 2 == 0; }
 
+// Whether no two rows of a cache with these strides (batch, KV head, row) have an element in common.
+static bool rows_apart(const int64_t (&stride)[3], const DecodeArgs &a) {
+  std::pair<int64_t, int64_t> dims[3] = {{stride[0], a.B}, {stride[1], a.Hkv}, {stride[2], a.Lmax}};
+  std::sort(dims, dims + 3);
+  int64_t span = a.D;  // of what lies inside of a step along the next dimension
+  for (const auto &[step, n] : dims) {
+    if (n == 1) continue;
+    if (step < span) return false;
+    span += (n - 1) * step;
+  }
+  return true;
+}
+
 // Whether a pair's whole walk in one workgroup (decode_pair_kernel, with one split) is taken. A launch of it lasts as long as its longest
 // pair, and the host knows the caches' length, not the sequences': of lengths that differ, one long sequence may stand beside many short
 // ones, whose keys the split kernel deals to all CUs. So wherever lengths are given (steps always) the line lies where one sequence
@@ -816,7 +830,10 @@ bool decode_mfma_rope_ok(int D, int interleaved) { return interleaved || (D / 32
 //     CUs on the split kernel takes walks up to 131 thousand in one split too: D=64 and 96 1.02 to 1.09 of its time, D=128 and 256 0.96 to 1.04
 //   decodes without lengths (all as long as the cache), 112 to 256 pairs: 0.73 to 0.97 of two launches up to 160 thousand, from three quarters
 //     of the CUs on 0.82 to 0.96 up to 440. With lengths 300 thousand on 256 pairs took 1.32, D=64 on 224 1.93 (one beside sixteenths).
+//
+// A step whose sequences share rows of a cache (windows of one buffer) stays on two launches: there every row is read before one is written.
 bool decode_by_pairs(const DecodeArgs &a) {
+  if (a.step && !(rows_apart(a.ks, a) && rows_apart(a.vs, a))) return false;
   const int64_t cus = device_cu_count(), pairs = (int64_t)a.B * a.Hkv * ((a.Hq / a.Hkv + 15) / 16), walk = (int64_t)a.Lmax * a.D;
   const int d = a.D > 128 ? 3 : a.D > 96 ? 2 : a.D > 64 ? 1 : 0;
   const bool many = pairs * 8 >= cus * 3;

@@ -97,6 +97,38 @@ def test_new_rows_off_alignment(lm, hip, oracle, D, group, dtype):
         np.testing.assert_array_equal(a, b)
 
 
+def test_steps_over_windows_of_one_buffer(lm, hip, oracle):
+    """Sequences whose caches overlap attend the rows as they were before the step: a row that one of them writes may be another one's
+    old row, so all are read before the first is written. Each writes another row of the buffer here."""
+    B, Hq, Lmax, D, dtype = 6, 4, 96, 128, "f16"
+    buf_k, buf_v = (oracle.round_to(oracle.gen_normal((Lmax + 8 * B, D), 45000 + i), dtype) for i in range(2))
+    q, kn, vn = (oracle.round_to(oracle.gen_normal((B, h, D), 45010 + h + i), dtype) for i, h in enumerate((Hq, 1, 1)))
+    pos = np.array([80, 61, 48, 31, 22, 5], np.int32)  # rows 80, 69, 64, 55, 54 and 45 of the buffer
+    at = 8 * np.arange(B) + pos
+    assert len(set(at)) == B
+    dk, dv, dq, dkn, dvn = (lm.to_device(x, hip, dtype) for x in (buf_k, buf_v, q, kn, vn))
+    out, dpos = lm.HipArray((B, Hq, D), "f32", hip), lm.to_device(pos, hip)
+    b = lm.binding
+    p, x = b.DecodeParams(), b.DecodeStepExtra()
+    p.out, p.q, p.k_cache, p.v_cache, p.kv_len = out.ptr, dq.ptr, dk.ptr, dv.ptr, dpos.ptr
+    p.B, p.Hq, p.Hkv, p.Lmax, p.D = B, Hq, 1, Lmax, D
+    for s in (p.k_stride, p.v_stride):
+        s[0], s[1], s[2] = 8 * D, D, D
+    p.dtype, p.scale, p.out_f32 = b.DTYPE_CODES[dtype], lm.default_scale(D), 1
+    x.k_new, x.v_new = dkn.ptr, dvn.ptr
+    need = b.decode_workspace_bytes(B, Hq, 1, Lmax, D, b.decode_step_splits(B, 1, Lmax))
+    scratch = lm.HipArray((need // 4,), "f32", hip).fill_bytes(0xff)
+    p.workspace, p.workspace_bytes = scratch.ptr, need
+    b.decode_step(p, x)
+    k, v = (np.stack([w[8 * i:8 * i + Lmax] for i in range(B)])[:, None] for w in (buf_k, buf_v))
+    want, _, _ = expected(oracle, q[:, :, None], kn[:, :, None], vn[:, :, None], k, v, pos, dtype, False, False, 0)
+    assert rel_err(out.to_host(), want) <= TOL[dtype]
+    buf_k[at], buf_v[at] = kn[:, 0], vn[:, 0]
+    np.testing.assert_array_equal(dk.to_host(), buf_k)
+    np.testing.assert_array_equal(dv.to_host(), buf_v)
+    assert not np.isnan(scratch.to_host()).all()  # two launches
+
+
 def launches(lm, hip, call):
     """How many launches a decode or a step takes: one leaves the scratch for the partial results as it is."""
     scratch = lm.host._workspaces
