@@ -128,6 +128,12 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   using pvec8 = typename MT::pvec8;
   constexpr int LDK = D + kPadK;   // LDS row strides in elements
   constexpr int LDV = D + pad_v<D>();
+  // Forms whose loop takes every register there is: what the masks and the stores need is made where they are, for what is held over the
+  // loop goes to memory in front of it and comes back behind it, with a wait for every load. us before 16-byte stores and masks of one
+  // compare, with both and now: 12 x 16 heads Sq=3300 Sk=20 D=96 bf16 69.7, 61.5, 52.8 (fp32 results 105.8, 110.8, 92.9), 6 x 32 Sq=2019 Sk=138
+  // 64.3, 62.2, 54.7, 14 x 20 Sq=1813 Sk=500 D=80 169.0, 173.0, 164.6, V as fp16 15 x 32 Sq=323 Sk=1393 175.6, 175.2, 160.9, causal 15 x 32/8
+  // S=709 D=72 96.4, 96.5, 92.5; fp16 7 x 32/8 Sq=3000 Sk=60 fp32 results 100.0, 113.1, 99.7.
+  constexpr bool TIGHT = D == 96 && (WPS == 4 || (CV && !CAUSAL));
 
   __shared__ __attribute__((aligned(16))) uint16_t Ks2[2][BT * LDK];  // double-buffered tiles
   __shared__ __attribute__((aligned(16))) uint16_t Vs2[2][BT * LDV];
@@ -630,11 +636,14 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
     const bool need_mask = (k0 + BW > n_keys) || (CAUSAL && k0 + BW - 1 > wave_q_lo);
     if (need_mask) {
       const int end = (CAUSAL ? min(n_keys, qi + 1) : n_keys) - k0 - 4 * g;  // of the keys that the lane's query sees
+      constexpr bool kTwoCompares = TIGHT && (MT::kSplitP || !CAUSAL);  // (`end` is a register over the loop)
 #pragma unroll
       for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
-        for (int i = 0; i < 16; i++)
-          if (kb * 32 + 8 * (i >> 2) + (i & 3) >= end) sacc[kb][i] = -INFINITY;
+        for (int i = 0; i < 16; i++) {
+          const int at = kb * 32 + 8 * (i >> 2) + (i & 3), key = k0 + at + 4 * g;
+          if (kTwoCompares ? key >= n_keys || (CAUSAL && key > qi) : at >= end) sacc[kb][i] = -INFINITY;
+        }
     }
 
     // ---- online softmax; all statistics are per lane (one query column) ----
@@ -817,9 +826,17 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   // ---- epilogue: out[qi][d] = O^T[d][qi] / l ----
   const float l_tot = sum_over_wave_halves(l_i);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if ((uint32_t)qi < (uint32_t)a.Sq) {
-    const int64_t off = b * a.os[0] + own_hq * a.os[1] + (int64_t)qi * a.os[2];
-    store_out_rows<MT, DB>(oacc, inv, a.out, off, g, a.D, a.out_f32);
+  int row = qi, half = g;
+  if (TIGHT && !CAUSAL) {  // (the row and its place from the lane's number, so that no register holds them until here)
+    const int own_lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+    row = q0 + wave_u % RH * 32 + (own_lane & 31);
+    half = own_lane >> 5;
+  } else if (TIGHT) {
+    asm volatile("" : "+v"(half));  // (or the offsets 16 j + 8 g of Q's loads are kept for the stores)
+  }
+  if ((uint32_t)row < (uint32_t)a.Sq) {
+    const int64_t off = b * a.os[0] + own_hq * a.os[1] + (int64_t)row * a.os[2];
+    store_out_rows<MT, DB>(oacc, inv, a.out, off, half, a.D, a.out_f32);
   }
   if (CAUSAL && KSPLIT == 1 && D <= 128 && queries.dst) store_queries();
 }
