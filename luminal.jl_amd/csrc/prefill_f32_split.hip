@@ -52,7 +52,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   const int b = (int)((uint32_t)bh / deal.hq), hq = bh - b * a.Hq;
   const int kvh = kv_head_of(hq, a.Hq, a.Hkv, a.head_map);
   const int q_tile = CAUSAL ? (deal.tiles - 1 - tile_rank) : tile_rank;
-  const int q0 = q_tile * BM - (CAUSAL && BM > BT ? causal_shift(deal.tiles, BM, a.Sq, BT) : 0);
+  const int q0 = q_tile * BM - (CAUSAL ? causal_shift(deal.tiles, BM, a.Sq, BT) : 0);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -157,7 +157,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void prefill_mfma_kernel(Deal deal, P
   // the tail of the launch. (Pairing tile r with tile n-1-r in one workgroup equalises the work but
   // halves the number of workgroups; measured 15 % slower on the S = 4096 workload.)
   const int q_tile = CAUSAL ? (deal.tiles - 1 - tile_rank) : tile_rank;
-  const int q0 = q_tile * BM - (CAUSAL && BM > BT ? causal_shift(deal.tiles, BM, a.Sq, BT) : 0);
+  const int q0 = q_tile * BM - (CAUSAL ? causal_shift(deal.tiles, BM, a.Sq, BT) : 0);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
