@@ -57,7 +57,9 @@ __host__ __device__ inline bool deal_tile(const Deal &t, int x, int i, int *head
 // Rows by which the row tiles of a causal launch begin before row 0. Where they do not fill the rows, the rows that a tile lacks
 // are those of the first one, whose keys are few, and not of the last one, which walks all of them whether it has one row or
 // all: S=777 in tiles of 128 rows is 49 key tiles of 64 a head in place of 55, S=1337 121 in place of 131. The shift is a multiple
-// of the key tile (a power of two), so that every tile's diagonal lies where it would without one; rows before row 0 see no key.
+// of the key tile (a power of two), so that every tile's diagonal lies where it would without one; rows before row 0 see no key. Where a
+// row tile is no higher than a key tile the shift is zero; left out there, the fp16 and bf16 kernels of two key groups took longer: fp16 B=1 H=6 S=2143
+// D=128 31.6 -> 32.6 us, H=12 S=1524 24.5 -> 25.1, bf16 H=8 S=1584 28.8 -> 29.1 (B=7 H=8/4 S=1994 D=64 52.4 -> 52.1).
 __host__ __device__ inline int causal_shift(int tiles, int rows, int Sq, int key_tile) {
   return (int)(((uint32_t)tiles * (uint32_t)rows - (uint32_t)Sq) & ~(uint32_t)(key_tile - 1));
 }

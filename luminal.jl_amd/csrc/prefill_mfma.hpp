@@ -151,8 +151,9 @@ __device__ inline void store_out_rows(const floatx16_t (&oacc)[DB], float inv, v
   if (out_f32) {
     // A head dim that fills its tiling is stored without a branch around each store. With the branches and the 16-bit stores below launches of
     // few keys took longer than with 8-byte 16-bit stores, whose fp32 part has the same instructions; us, as it was then, with the branches and
-    // now: B=11 H=8 Sq=6985 D=64 fp16 Sk=64 44.8, 46.5, 44.5; bf16 ragged Sk=30 44.1, 46.6, 44.6, all 30 keys 46.4, 50.3, 48.8 (what is left
-    // of that one has no cause that is known); fp16 B=5 H=8 Sq=4096 Sk=100 D=96 25.1, 25.7, 25.1; B=8 H=32/8 S=512 D=64 27.5, 28.0, 27.4.
+    // now: B=11 H=8 Sq=6985 D=64 fp16 Sk=64 44.8, 46.5, 44.5; bf16 ragged Sk=30 44.1, 46.6, 44.6, all 30 keys 46.4, 50.3, 48.8 (with masks of
+    // two compares 47.2, but other launches without a causal mask 0.5 to 1 % longer); fp16 B=5 H=8 Sq=4096 Sk=100 D=96 25.1, 25.7, 25.1; B=8 H=32/8
+    // S=512 D=64 27.5, 28.0, 27.4.
     float *op32 = reinterpret_cast<float *>(out) + row_off + 4 * g;
     auto group = [&](int db, int i4) {
       *reinterpret_cast<float4 *>(op32 + 32 * db + 8 * i4) = make_float4(oacc[db][4 * i4 + 0] * inv, oacc[db][4 * i4 + 1] * inv,
