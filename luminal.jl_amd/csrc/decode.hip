@@ -416,16 +416,19 @@ __device__ __forceinline__ void merge_row(const DecodeArgs &a, int hq, int b) {
   for (int w = 0; w < kMergeThreads / 64; w++) lsum += red_l[w];
   // Most slots behind the prefetched ones are empty where a workgroup walks several chunks of a sequence (a slot per chunk, one
   // row per run of them): their rows are not read (B=64 H=32/8 up to 32768 keys D=128, 64 slots: the whole call 849.7 -> 842.2 us). Up to
-  // twice as many slots as are prefetched, all of them are fetched as they come (B=1 L=32768, 32 slots, none empty: 29.0, skipping 30.4).
+  // twice as many slots as are prefetched, and where more than half hold something, all of them are fetched as they come, whose
+  // addresses wait for nothing (B=1 L=32768, 32 slots, none empty: 29.0, skipping 30.4; B=2 H=32/4 L=26420 D=80, 207 of them: 37.5 and 44.7).
   const int n_lds = min(n, kMergeMaxSlots), n_p = min(n_lds, n_pre) & ~3;
-  const bool skip = n_lds > 2 * kMergePrefetch;
+  const bool counted = n_lds > 2 * kMergePrefetch;
   int n_full = 0;
-  for (int base = n_p; skip && base < n_lds; base += 64) {  // (every wave finds the same ones)
+  for (int base = n_p; counted && base < n_lds; base += 64) {  // (every wave finds the same ones)
     const int s = base + (tid & 63);
     const uint64_t full = __builtin_amdgcn_ballot_w64(s < n_lds && w_s[s] != 0.f);
     if (full >> (tid & 63) & 1) full_s[n_full + __builtin_popcountll(full & ((uint64_t(1) << (tid & 63)) - 1))] = (uint16_t)s;
     n_full += __builtin_popcountll(full);
   }
+  const bool skip = counted && 2 * n_full <= n_lds - n_p;
+  if (!skip) n_full = 0;
   const float w_new = appends ? __builtin_amdgcn_exp2f(m_new - M) : 0.f;  // the new row's sum is 1
   lsum += w_new;
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;

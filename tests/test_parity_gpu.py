@@ -1035,6 +1035,18 @@ def test_decode_random_shapes_and_options(lm, hip, oracle, seed):
                                                    lens=None if lens is None else lens.tolist())
 
 
+@pytest.mark.parametrize("dtype,B,Hkv,D", [("f32", 2, 2, 64), ("bf16", 3, 2, 80), ("f16", 1, 4, 128), ("bf16", 2, 8, 128), ("f16", 3, 8, 64), ("bf16", 8, 8, 64)])
+def test_merge_of_many_slots(lm, hip, oracle, dtype, B, Hkv, D):
+    """More slots than the merge prefetches twice, all of them with a partial result (the first three), about half (two chunks of a
+    sequence a workgroup, or three), and few; sequences that fill the cache, a part of it and a few chunks."""
+    L, splits = 70 * 64, 70
+    q, k, v = inputs(oracle, (B, 2 * Hkv, D), (B, Hkv, L, D), dtype, 9970 + B + D)
+    lens = np.linspace(L, 33 * 64 + 5, B).astype(np.int32)
+    lens[B - 1] = 100 if B > 3 else lens[B - 1]
+    got = run_decode(lm, hip, q, k, v, dtype, kv_len=lens, num_splits=splits, out_dtype="f32")
+    assert rel_err(got, oracle.decode_attn(q, k, v, kv_len=lens, nthreads=NT)) <= TOL[dtype]
+
+
 @pytest.mark.parametrize("dtype,D,group,L", [
     ("bf16", 128, 1, 512), ("bf16", 128, 4, 200), ("bf16", 64, 5, 512), ("bf16", 96, 6, 500), ("bf16", 256, 17, 300),
     ("f16", 64, 1, 512), ("f16", 128, 3, 200), ("f16", 96, 8, 500), ("f16", 64, 9, 512), ("f16", 256, 33, 300), ("f16", 64, 4, 20000),
