@@ -816,18 +816,23 @@ static bool rows_apart(const int64_t (&stride)[3], const DecodeArgs &a) {
 // Whether a pair's whole walk in one workgroup (decode_pair_kernel, with one split) is taken. A launch of it lasts as long as its longest
 // pair, and the host knows the caches' length, not the sequences': of lengths that differ, one long sequence may stand beside many short
 // ones, whose keys the split kernel deals to all CUs. So wherever lengths are given (steps always) the line lies where one sequence
-// as long as the cache beside others of one key takes no longer than it did in the two launches before this kernel (1.03 of them at
-// most). Measured on 8300 launches (G = 1 to 20, D = 64 to 256, 2 to 8192 pairs; all lengths full, uniform below the cache's, one full
-// beside sixteenths, one full beside single keys), time against the split kernel (and the merge) of today, full / uniform / one
-// beside single keys:
-//   steps, few pairs: D=64 59 thousand elements a walk 1.03 / 0.94 / 1.00, 80 thousand 1.13 / 1.07 / 1.10; D=128 80 0.97 / 0.93 / 0.96, 103 1.12 /
-//     1.09 / 1.10; D=256 89 0.86 / 0.83 / 0.83, 123 1.07 / 0.97 / 1.04. On three eighths of the CUs and more the walk may be longer, D=128 112 to
-//     192 pairs 123 thousand 0.86 / 0.75 / 1.26, 160 0.90 / 0.90 / 1.45; D=128 and 256 on nearly all CUs, 160 0.83 / 0.74 / 1.24
-//   steps of several rounds: D=128 768 pairs 30 thousand 0.83 / 0.74 / 0.93, 167 0.91 / 0.81 / 0.98 and 8192 pairs 0.90 / 0.85 / 0.93, 289 up to 1.58 in
-//     the third; D=256 512 pairs 289 0.92 / 0.87 / 1.24. D=64 480 pairs 16 thousand 0.91 / 0.99 / 1.15, 30 1.33 in the third; 1024 pairs 16
-//     1.13 / 1.14 / 1.32, 8192 pairs of 64 keys 1.31 all full: a workgroup has the CU, its prologue and fold nothing beside them
-//   decodes: 16 pairs D=64 40 thousand 0.96 / 0.92 / 0.94, 80 1.23 / 1.21 / 1.22; D=128 59 0.98, 103 1.21; D=256 89 0.94, 103 1.16. From half the
-//     CUs on the split kernel takes walks up to 131 thousand in one split too: D=64 and 96 1.02 to 1.09 of its time, D=128 and 256 0.96 to 1.04
+// as long as the cache beside others of one key takes no longer than it did in the two launches before this kernel, and where the others gain.
+// Measured on 2150 calls one behind the other, host and launches together (G = 1 to 4, D = 64 to 256, 2 to 2048 pairs), time against the split
+// kernel (and the merge) of today with all lengths full / uniform in the upper three quarters / one full beside single keys, and the last
+// also against the two launches before this kernel:
+//   steps, few pairs: D=64 80 thousand elements a walk 0.76 to 0.90 / 0.73 to 0.88 / 0.87 to 0.91, 110 0.88 to 1.07 / 0.72 to 0.96 / 0.97 to 1.08;
+//     D=128 110 0.70 to 0.96 / 0.54 to 0.82 / 0.81 to 0.94, 130 up to 1.11; D=256 130 0.78 to 0.91 / 0.60 to 0.86 / 0.78 to 0.91, 150 up to 1.05
+//   steps on three eighths of the CUs and more: D=64 85 0.73 to 0.80 / 0.72 to 0.82 / 1.03 to 1.09 (0.85 to 0.90), 110 (0.99 to 1.08); D=128
+//     140 0.76 to 0.87 / 0.65 to 0.87 / 1.00 to 1.29 (0.80 to 1.03), 180 from seven eighths on 0.84 to 0.87 / 0.78 to 0.81 / 1.23 to 1.30 (0.95 to 0.99), on fewer (0.92
+//     to 1.21); D=256 180 0.73 to 0.92 / 0.68 to 0.85 / 0.87 to 1.18 (0.72 to 0.96), 250 from seven eighths on (0.93), on fewer (1.14 to 1.17)
+//   steps of several rounds: D=128 170 0.86 to 1.01 / 0.78 to 1.02 / 0.93 to 1.39 (0.80 to 1.05), 300 (up to 1.32); D=256 300 nearly full rounds 0.91 to
+//     0.93 / 0.74 to 0.92 / 0.77 to 1.32 (0.73 to 1.10); two rounds D=64 and 96 50 0.78 to 0.98 / 0.85 to 0.97 / 1.08 to 1.28 (0.87 to 1.01), 100 (up to 1.14); three
+//     rounds D=64 8 0.86 / 0.82 / 0.91, 16 1.07 / 1.09 / 1.28, D=96 16 0.95 / 0.96 / 1.16 (0.94), 50 (1.29); four D=64 8 1.20, D=96 8 0.93, 16 1.23: a workgroup has the
+//     CU, its prologue and fold nothing beside them
+//   decodes, few pairs: D=64 80 0.83 to 0.94 / 0.77 to 0.90 / 0.88 to 0.94, 95 0.94 to 1.07; D=96 95 0.86 to 1.03; D=128 110 0.75 to 1.02 / 0.70 to 0.91 / 0.91 to 1.07, 130 0.95 to
+//     1.19; D=256 95 0.79 to 0.86 / 0.59 to 0.82 / 0.80 to 0.85, 110 0.87 to 1.09. On three eighths of the CUs and more D=64 85 0.88 / 0.88 / 1.12 (0.92), 110
+//     (1.20); D=128 110 0.78 to 0.99 / 0.88 to 0.99 / 1.00 to 1.17 (0.82 to 0.95), 140 (up to 1.17); D=256 140 0.77 to 0.94 / 0.76 to 0.96 / 0.98 to 1.29 (0.77 to 0.95), 180 (up to
+//     1.10). From half the CUs on the split kernel takes walks up to 131 thousand in one split too: D=64 and 96 0.96 to 1.08, D=128 and 256 0.91 to 1.01
 //   decodes without lengths (all as long as the cache), 112 to 256 pairs: 0.73 to 0.97 of two launches up to 160 thousand, from three quarters
 //     of the CUs on 0.82 to 0.96 up to 440. With lengths 300 thousand on 256 pairs took 1.32, D=64 on 224 1.93 (one beside sixteenths).
 //
@@ -838,13 +843,13 @@ bool decode_by_pairs(const DecodeArgs &a) {
   const int d = a.D > 128 ? 3 : a.D > 96 ? 2 : a.D > 64 ? 1 : 0;
   const bool many = pairs * 8 >= cus * 3;
   if (a.step) {
-    constexpr int32_t kFew[4] = {65536, 81920, 81920, 98304}, kMany[4] = {85000, 100000, 125000, 180000}, kAll[4] = {85000, 100000, 160000, 250000};
+    constexpr int32_t kFew[4] = {100000, 100000, 120000, 140000}, kMany[4] = {100000, 100000, 140000, 200000}, kAll[4] = {100000, 100000, 180000, 280000};
     if (pairs <= cus) return walk <= (pairs * 8 >= cus * 7 ? kAll : many ? kMany : kFew)[d];
     const int64_t rounds = (pairs + cus - 1) / cus;
     if (d >= 2) return walk <= (d == 3 && pairs * 20 >= rounds * cus * 17 ? 300000 : 170000);
-    return rounds <= 4 && walk <= (rounds <= 2 ? (d ? 30000 : 16384) : (d ? 12288 : 8192));
+    return walk <= (rounds == 2 ? 50000 : rounds == 3 ? (d ? 16384 : 8192) : rounds == 4 && d ? 8192 : 0);
   }
-  constexpr int32_t kFew[4] = {65536, 73728, 81920, 98304}, kMany[4] = {65536, 73728, 105000, 140000};
+  constexpr int32_t kFew[4] = {90000, 92000, 110000, 105000}, kMany[4] = {90000, 92000, 110000, 150000};
   if (d < 2 && pairs * 2 >= cus && walk <= 131072) return false;
   if (pairs > cus || (d == 0 && pairs * 20 > cus * 19)) return false;
   if (!a.kv_len && pairs * 16 >= cus * 7) return walk <= (pairs * 4 >= cus * 3 ? 450000 : 160000);

@@ -14,7 +14,8 @@ CASES = [  # D, Lmax, group, dtype
     (64, 1100, 1, "f16"), (64, 513, 5, "bf16"), (64, 40, 9, "f16"), (96, 700, 4, "bf16"), (96, 385, 8, "f16"), (96, 130, 17, "bf16"),
     (128, 260, 4, "bf16"), (128, 700, 6, "bf16"), (128, 512, 8, "f16"), (128, 33, 20, "f16"), (256, 350, 2, "f16"), (256, 129, 7, "bf16"),
     (64, 1560, 3, "f16"), (96, 1040, 2, "bf16"), (128, 976, 4, "f16"), (256, 488, 1, "bf16"),
-    (64, 1024, 2, "bf16"), (96, 768, 3, "f16"), (128, 640, 5, "f16"), (256, 384, 3, "bf16"),  # the longest walks of few pairs in one launch
+    (64, 1406, 2, "bf16"), (96, 958, 3, "f16"), (128, 859, 5, "f16"), (256, 410, 3, "bf16"),  # the longest walks of few pairs in one launch, decodes
+    (64, 1562, 2, "f16"), (96, 1041, 3, "bf16"), (128, 937, 5, "bf16"), (256, 546, 3, "f16"),  # ... and steps
 ]
 
 
@@ -141,11 +142,11 @@ def launches(lm, hip, call):
 
 @pytest.mark.parametrize("B,Hkv,G,L,D,dtype,step,ragged,expected_launches", [
     (50, 4, 2, 2250, 128, "bf16", False, True, 2), (33, 7, 1, 1100, 256, "f16", False, True, 2), (28, 8, 1, 4600, 64, "f16", False, True, 2),
-    (50, 4, 2, 3515, 128, "bf16", False, False, 1), (32, 8, 1, 820, 128, "f16", False, True, 1), (24, 5, 2, 546, 256, "bf16", False, True, 1),
-    (45, 8, 2, 1300, 128, "f16", True, True, 1), (36, 8, 1, 660, 256, "bf16", True, True, 1), (32, 8, 2, 1250, 128, "bf16", True, True, 1),
-    (28, 8, 1, 976, 256, "f16", True, True, 1), (30, 8, 1, 1328, 64, "bf16", True, True, 1), (24, 8, 1, 1041, 96, "f16", True, True, 1),
-    (55, 8, 1, 1171, 256, "bf16", True, True, 1), (40, 8, 3, 256, 64, "f16", True, True, 1), (50, 8, 1, 312, 96, "bf16", True, True, 1),
-    (100, 8, 1, 128, 96, "f16", True, True, 1)])
+    (50, 4, 2, 3515, 128, "bf16", False, False, 1), (32, 8, 1, 859, 128, "f16", False, True, 1), (24, 5, 2, 585, 256, "bf16", False, True, 1),
+    (45, 8, 2, 1300, 128, "f16", True, True, 1), (36, 8, 1, 660, 256, "bf16", True, True, 1), (32, 8, 2, 1406, 128, "bf16", True, True, 1),
+    (28, 8, 1, 1093, 256, "f16", True, True, 1), (30, 8, 1, 1562, 64, "bf16", True, True, 1), (24, 8, 1, 1041, 96, "f16", True, True, 1),
+    (55, 8, 1, 1171, 256, "bf16", True, True, 1), (40, 8, 3, 781, 64, "f16", True, True, 1), (50, 8, 1, 520, 96, "bf16", True, True, 1),
+    (80, 8, 1, 170, 96, "f16", True, True, 1), (100, 8, 1, 85, 96, "f16", True, True, 1)])
 def test_long_walks_of_many_pairs(lm, hip, oracle, B, Hkv, G, L, D, dtype, step, ragged, expected_launches):
     """A good part of the CUs with a pair each, or several rounds of pairs, at the longest walks that still take one launch, and decodes beyond them."""
     q, kn, vn, kc, vc = step_inputs(oracle, B, Hkv * G, Hkv, L, D, dtype, 44000 + L)
@@ -167,12 +168,13 @@ def test_long_walks_of_many_pairs(lm, hip, oracle, B, Hkv, G, L, D, dtype, step,
 
 
 @pytest.mark.parametrize("B,Hkv,G,D,step,ragged,L,longer", [  # the longest walk in one launch (None: no walk is), and one beyond it
-    (1, 8, 4, 64, True, True, 1024, 1032), (2, 8, 4, 96, True, True, 853, 864), (1, 8, 4, 128, True, True, 640, 648), (4, 8, 2, 256, True, True, 384, 392),
-    (12, 8, 4, 128, True, True, 976, 1000), (32, 8, 4, 128, True, True, 1250, 1256), (32, 8, 2, 256, True, True, 976, 980),
-    (64, 8, 4, 128, True, True, 1328, 1336), (64, 8, 2, 256, True, True, 1168, 1176), (64, 8, 4, 64, True, True, 256, 264),
-    (128, 8, 1, 64, True, True, 128, 136), (1024, 8, 1, 64, True, True, None, 64), (256, 8, 4, 96, True, True, None, 64),
-    (1, 8, 4, 64, False, True, 1024, 1032), (1, 8, 4, 128, False, True, 640, 648), (64, 4, 4, 128, False, False, 3515, 3520),
-    (64, 4, 4, 128, False, True, 820, 3437), (28, 8, 1, 64, False, True, 2048, 2500)])
+    (1, 8, 4, 64, True, True, 1562, 1568), (2, 8, 4, 96, True, True, 1041, 1048), (1, 8, 4, 128, True, True, 937, 944), (4, 8, 2, 256, True, True, 546, 552),
+    (12, 8, 4, 128, True, True, 1093, 1100), (12, 8, 2, 256, True, True, 781, 784), (32, 8, 4, 128, True, True, 1406, 1408), (32, 8, 2, 256, True, True, 1093, 1096),
+    (64, 8, 4, 128, True, True, 1328, 1336), (64, 8, 2, 256, True, True, 1168, 1176), (64, 8, 4, 64, True, True, 781, 784),
+    (96, 8, 1, 64, True, True, 128, 136), (96, 8, 1, 96, True, True, 170, 176), (128, 8, 1, 96, True, True, 85, 88), (128, 8, 1, 64, True, True, None, 64),
+    (1024, 8, 1, 64, True, True, None, 64), (256, 8, 4, 96, True, True, None, 64),
+    (1, 8, 4, 64, False, True, 1406, 1408), (2, 8, 4, 96, False, True, 958, 960), (1, 8, 4, 128, False, True, 859, 864), (1, 8, 2, 256, False, True, 410, 416),
+    (12, 8, 2, 256, False, True, 585, 592), (64, 4, 4, 128, False, False, 3515, 3520), (64, 4, 4, 128, False, True, 859, 3437), (28, 8, 1, 64, False, True, 2048, 2500)])
 def test_walks_of_one_launch(lm, hip, B, Hkv, G, D, step, ragged, L, longer):
     """Caches whose lengths may differ go to one workgroup a pair only as far as one long sequence does not hold the others up."""
     for n_keys, want in ((L, 1), (longer, 2)):
