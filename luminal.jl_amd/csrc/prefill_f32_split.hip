@@ -94,12 +94,14 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   // Rounds of whole rows (HALF): one offset a tensor, and what a round adds is the same for every lane.
   constexpr int kRoundRows = HALF ? NT / DC : 0, kRoundsK = HALF ? BT / (NT / DC) : 0;
   static_assert(!HALF || (NT % DC == 0 && BT % (NT / DC) == 0), "whole rows a round");
+  auto round_bytes = [&](int r, int64_t stride) { return (uint32_t)min((int64_t)r * kRoundRows * stride * 4, (int64_t)kOutOfRange); };
   int voff[HALF ? 2 : R], lds_off[HALF ? 2 : R];
 #pragma unroll
   for (int r = 0; r < (HALF ? 2 : R); r++) {
     const int q = tid + r * (HALF ? BT * DC : NT), c = q % (BT * DC), row = c / DC, col = c % DC;
     const bool is_v = q >= BT * DC;
-    voff[r] = q < kChunks && 8 * col < a.D ? (int)((row * (is_v ? a.vs[2] : a.ks[2]) + 8 * col) * 4) : kOutOfRange - 16;
+    const int64_t at = (row * (is_v ? a.vs[2] : a.ks[2]) + 8 * col) * 4;
+    voff[r] = q < kChunks && 8 * col < a.D ? (int)(HALF ? min(at, (int64_t)kOutOfRange - 16) : at) : kOutOfRange - 16;
     lds_off[r] = is_v ? kPlanesK * kPlaneK + row * LDV + 8 * col : row * LDK + 8 * col;
   }
   floatx4_t x[R][2];
@@ -113,7 +115,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
       if constexpr (HALF) {
         const bool is_v = r >= kRoundsK;
         // (the round's rows are part of the vector offset: a scalar one beyond the last key defeats the range check)
-        const int off = voff[is_v] + (r - (is_v ? kRoundsK : 0)) * kRoundRows * (int)(is_v ? a.vs[2] : a.ks[2]) * 4;
+        // (unsigned: a column that is not there, kOutOfRange, and a round's bytes together stay below 2^32)
+        const uint32_t off = (uint32_t)voff[is_v] + round_bytes(r - (is_v ? kRoundsK : 0), is_v ? a.vs[2] : a.ks[2]);
 #pragma unroll
         for (int e = 0; e < 2; e++)
           x[r][e] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(is_v ? v_rsrc : k_rsrc, off + 16 * e, kt * (is_v ? v_tile_bytes : k_tile_bytes), 0));
