@@ -31,16 +31,6 @@ constexpr int kWaves = 4;
 constexpr int kUnroll = 4;  // key steps per wave per iteration
 constexpr float kLog2e = 1.4426950408889634f;
 
-// v_mov_b32_dpp with a compile-time lane pattern; the compiler folds it into the consuming VALU op.
-template <int CTRL>
-__device__ inline float dpp(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
-}
-constexpr int kDppXor1 = 0xB1;        // quad_perm [1,0,3,2]
-constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
-constexpr int kDppHalfMirror = 0x141; // lane i <- lane 7-i of its 8-lane half row
-constexpr int kDppMirror = 0x140;     // lane i <- lane 15-i of its 16-lane row
-
 // All-reduce (sum) over the LPK adjacent lanes that share a key. Up to 16 lanes this is pure DPP
 // (no LDS round trip): after the two quad steps every lane of a quad holds the quad sum, so the
 // mirror patterns, which pair quad 0 with 1 (and 2 with 3), then half row 0 with 1, finish it.

@@ -50,6 +50,23 @@ __device__ inline float sum_over_wave_rows(float x) {
   return sum_over_wave_halves(a + b);
 }
 
+// v_mov_b32_dpp with a compile-time lane pattern; the compiler folds it into the consuming VALU op.
+template <int CTRL>
+__device__ inline float dpp(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+constexpr int kDppXor1 = 0xB1;        // quad_perm [1,0,3,2]
+constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
+constexpr int kDppHalfMirror = 0x141; // lane i <- lane 7-i of its 8-lane half row
+constexpr int kDppMirror = 0x140;     // lane i <- lane 15-i of its 16-lane row
+// max over a row of 16 lanes, on every lane of it
+__device__ inline float max_over_row(float x) {
+  x = fmaxf(x, dpp<kDppXor1>(x));
+  x = fmaxf(x, dpp<kDppXor2>(x));
+  x = fmaxf(x, dpp<kDppHalfMirror>(x));
+  return fmaxf(x, dpp<kDppMirror>(x));
+}
+
 __device__ inline float bf16_bits_to_f32(uint32_t bits16) { return __uint_as_float(bits16 << 16); }
 
 // round-to-nearest-even, NaN kept quiet: v_cvt_pk_bf16_f32, the same bits as the integer rounding it replaces for every

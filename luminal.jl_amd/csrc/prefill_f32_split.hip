@@ -21,9 +21,13 @@
 // accumulators of their own, lo lo left out, and two planes of K instead of three. What is lost weighs less than what the fp32 product
 // rounds (2-norm against 64 bits, that product and this kernel): 4.6e-7 and 1.7e-7 (S = 2048 D = 128 causal), 5.7e-7 and 2.0e-7 (S = 1024),
 // 5.6e-7 and 2.0e-7 (S = 1023 D = 112). Below it, against three bf16 pieces, it would weigh 0.05 to 0.2 more than nothing (S = 1023 D = 80
-// 1.83e-7 and 1.90e-7, S = 2048 D = 64 causal 1.35e-7 and 1.52e-7), so these stay. us, the fp32 product and this kernel: B=1 H=32/8 S=4096
-// D=128 causal 1067 and 599, H=16 S=2048 178 and 127, B=2 H=12 S=1023 D=112 115 and 66, B=8 H=16 S=300 D=128 causal 46.7 and 34.8. One tile of
-// 64 keys is in LDS at a time; with K's next one beside it, and both split beside the MFMAs, it took 594 and 132 us, in another order
+// 1.83e-7 and 1.90e-7, S = 2048 D = 64 causal 1.35e-7 and 1.52e-7), so these stay. The pieces are taken relative to a power of two, each query's
+// own and that of the largest key so far, so what they lack is small beside what is there at any magnitude (S = 1024 causal, queries of 1e3 and keys of 1e-5:
+// 1.6e-7 with the fp32 product, 0.7e-7; 3e3 and 1: 2.7e-5 and 1.1e-5). What still goes to the fp32 product: infinities and NaN, scores beyond 2^30, and walks whose
+// largest key leaves so little of the others that bits of their scores would be lost (from about 2^20 on). That takes three times as long as
+// the fp32 product's own kernel (S = 4096 1070 and 3370 us, B=8 H=16 S=300 47 and 159); until the pieces were relative, values of 1e3 took it too,
+// and normal ones up to 2 % less. us, the fp32 product and this kernel: B=1 H=32/8 S=4096 D=128 causal 1068 and 602, H=16 S=2048 177 and 129,
+// B=2 H=12 S=1023 D=112 115 and 75, B=8 H=16 S=300 D=128 causal 47.4 and 37.0. One tile of 64 keys is in LDS at a time; with K's next one beside it, and both split beside the MFMAs, it took 594 and 132 us, in another order
 // 634 and 133.
 #include <math.h>
 
@@ -59,6 +63,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   constexpr int NBUF = 4 * kTile <= 160 * 1024 && NW == 8 ? 2 : 1;
   __shared__ __attribute__((aligned(16))) uint16_t planes[NBUF * kTile];
   __shared__ int redo;
+  __shared__ int key_top;  // HALF: exponent of the largest key so far
 
   int bh, tile_rank;
   if (!deal_tile(deal, blockIdx.x & 7, blockIdx.x >> 3, &bh, &tile_rank)) return;
@@ -105,7 +110,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
     lds_off[r] = is_v ? kPlanesK * kPlaneK + row * LDV + 8 * col : row * LDK + 8 * col;
   }
   floatx4_t x[R][2];
-  float top = 0.f;  // the largest magnitude among this thread's values of Q and K (and a part of V's)
+  float top = 0.f;  // the largest magnitude among this thread's values of Q and K (and a part of V's); HALF: of the K in its registers
   auto is_v_wave = [&](int r) { return wave * 64 + r * NT >= BT * DC; };  // (a wave's 64 chunks are K's or V's: 8 D is a multiple of 64)
   auto fetch = [&](int kt, int first, int last) {  // rounds first .. last - 1
 #pragma unroll
@@ -133,6 +138,17 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
     for (int e = 0; e < 4; e++) so_far = fmaxf(fmaxf(fabsf(lo[e]), fabsf(hi[e])), so_far);
     return so_far;
   };
+  // HALF: Q and K are split relative to a power of two, a row's own of Q and that of the largest key so far of K, so that what two
+  // pieces do not hold is small beside what is there, whatever the magnitude (half_up, half_down).
+  int key_exp = kHalfLeast;
+  auto note_top = [&]() {  // ahead of the barrier in front of split_tile; grows a few times in a walk
+    float t = 0.f;
+#pragma unroll
+    for (int r = 0; r < kRoundsK; r++) t = top_of(x[r][0], x[r][1], t);
+    if (__builtin_amdgcn_ballot_w64(half_exponent(t) > key_exp) == 0) return;
+    const int wave_exp = __builtin_amdgcn_readfirstlane(half_exponent(max_over_wave_rows(max_over_row(t))));
+    if (lane == 0) atomicMax(&key_top, wave_exp);
+  };
   auto split_tile = [&](int buf) {
 #pragma unroll
     for (int r = 0; r < R; r++) {
@@ -145,8 +161,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
 #pragma unroll
           for (int i = 0; i < 3; i++) *reinterpret_cast<bf16x8_t *>(to + i * kPlaneV) = f.p[i];
         } else {
-          top = top_of(x[r][0], x[r][1], top);
-          const HalfPieces f = split_half_8(x[r][0], x[r][1]);
+          const HalfPieces f = split_half_8(x[r][0], x[r][1], half_up(key_exp));
           *reinterpret_cast<half8_t *>(to) = f.hi;
           *reinterpret_cast<half8_t *>(to + kPlaneK) = f.lo;
         }
@@ -162,13 +177,13 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
     }
   };
   if (n_kv_tiles > 0) fetch(0, 0, R);
+  if (tid == 0) redo = 0, key_top = kHalfLeast;
   if (D % 32 != 0) {  // columns of the last block of O^T that no chunk fills
     for (int i = tid; i < NBUF * 3 * BT * (32 * DB - D); i += NT) {
       const int row = i / (32 * DB - D), col = i % (32 * DB - D), plane = row / BT;
       planes[plane / 3 * kTile + kPlanesK * kPlaneK + plane % 3 * kPlaneV + row % BT * LDV + D + col] = 0;
     }
   }
-  if (tid == 0) redo = 0;
 
   // ---- Q: lane (n, g) holds q[qi][16 ks + 8 g .. + 7] ----
   floatx4_t q[KS][2];
@@ -213,10 +228,14 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   const float unit = HALF ? __int_as_float(__float_as_int(c) & 0x7f800000) : c, grow = 1.f / unit;
   std::conditional_t<HALF, HalfPieces, Pieces> qf[KS];
   load_q();
+  if (HALF) __syncthreads();  // (key_top is there)
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) top = top_of(q[ks][0], q[ks][1], top);
+  const int q_exp = half_exponent(max_over_wave_halves(top) * (c * grow));
+  const float row_unit = unit * half_down(q_exp);  // of a score whose K is as it came
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) {
-    top = top_of(q[ks][0], q[ks][1], top);
-    if constexpr (HALF) qf[ks] = split_half_8(q[ks][0], q[ks][1], c * grow, fmaf(a.scale, kLog2eRest, fmaf(a.scale, kLog2e, -c)) * grow);
+    if constexpr (HALF) qf[ks] = split_half_8(q[ks][0], q[ks][1], c * grow * half_up(q_exp), fmaf(a.scale, kLog2eRest, fmaf(a.scale, kLog2e, -c)) * grow * half_up(q_exp));
     else qf[ks] = split_8(q[ks][0], q[ks][1]);
   }
 
@@ -232,23 +251,37 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   };
   clear();
   const int last_key = (CAUSAL ? min(qi, n_keys - 1) : n_keys - 1) - 4 * g;  // that the lane's row sees, less the lane's own offset
-  // Mask, running max, weights and their sum; register i of block kb is key k0 + 32 kb + 8 (i / 4) + 4 g + i % 4.
-  auto soften = [&](auto &s, int blocks, int k0, float unit, const auto &exponent) {  // (of a weight, from its score)
+  // Mask, running max, weights and their sum; register i of block kb is key k0 + 32 kb + 8 (i / 4) + 4 g + i % 4. `unit` is what a score is in log2
+  // units; the running max is a score, HALF: one in log2 units. `exponent` is that of a weight, from its score. HALF: what the smaller products
+  // add to a score is masked as well (it may be NaN), and counts in the max of large scores only (`whole`), where it could move a weight by more
+  // than its exponent holds.
+  auto soften = [&](auto &s, auto &small, int blocks, int k0, float unit, const auto &exponent, const auto &whole) {
     if (k0 + 32 * blocks > n_keys || (CAUSAL && k0 + 32 * blocks - 1 > wave_q_lo)) {
 #pragma unroll
       for (int kb = 0; kb < blocks; kb++)
 #pragma unroll
         for (int i = 0; i < 16; i++) {
           const int key = k0 + 32 * kb + 8 * (i >> 2) + (i & 3);
-          if (HALF ? key > last_key : key + 4 * g >= n_keys || (CAUSAL && key + 4 * g > qi)) s[kb][i] = -INFINITY;
+          if (HALF ? key > last_key : key + 4 * g >= n_keys || (CAUSAL && key + 4 * g > qi)) {
+            if (HALF) small[kb][i] = 0.f;
+            s[kb][i] = -INFINITY;
+          }
         }
     }
-    float mx = s[0][0];
+    auto top_score = [&](const auto &score) {
+      float mx = score(0, 0);
 #pragma unroll
-    for (int kb = 0; kb < blocks; kb++)
+      for (int kb = 0; kb < blocks; kb++)
 #pragma unroll
-      for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[kb][i]);
-    mx = max_over_wave_halves(mx);
+        for (int i = 0; i < 16; i++) mx = fmaxf(mx, score(kb, i));
+      return max_over_wave_halves(mx);
+    };
+    float mx = top_score([&](int kb, int i) { return s[kb][i]; });
+    if (HALF) {
+      mx *= unit;
+      if (__builtin_amdgcn_ballot_w64(fabsf(mx) > 1024.f) != 0) mx = top_score(whole) * unit;
+      unit = 1.f;
+    }
     if (__builtin_amdgcn_ballot_w64((mx - m_i) * unit > kLazyRescale) != 0) {
       const float m_new = fmaxf(m_i, mx);
       const float alpha = m_i == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_i - m_new) * unit);
@@ -287,8 +320,10 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   }
   for (int kt = 0; kt < n_kv_tiles; kt++) {
     const int buf = NBUF == 2 ? kt & 1 : 0;
+    if constexpr (HALF) note_top();
     __syncthreads();  // everyone is done with tile kt - 1 (and, with two tiles, tile kt is in LDS)
     if (NBUF == 1) {
+      if constexpr (HALF) key_exp = __builtin_amdgcn_readfirstlane(key_top);
       split_tile(0);
       if (kt + 1 < n_kv_tiles) fetch(kt + 1, 0, HALF ? kRoundsK : R);
       __syncthreads();  // tile kt is in LDS
@@ -344,13 +379,16 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
     }
     prepare_next();
     if constexpr (HALF) {
-      soften(s, NKB, k0, unit, [&](int kb, int i, float mc) { return fmaf(small[kb][i], unit * (1.f / kHalfGap), fmaf(s[kb][i], unit, -mc)); });
+      const float by = row_unit * half_down(key_exp);
+      soften(s, small, NKB, k0, by, [&](int kb, int i, float mc) { return fmaf(small[kb][i], by * (1.f / kHalfGap), fmaf(s[kb][i], by, -mc)); },
+             [&](int kb, int i) { return fmaf(small[kb][i], 1.f / kHalfGap, s[kb][i]); });
     } else {
 #pragma unroll
       for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
         for (int i = 0; i < 16; i++) s[kb][i] += small[kb][i];
-      soften(s, NKB, k0, c, [&](int kb, int i, float mc) { return s[kb][i] * c - mc; });
+      auto score = [&](int kb, int i) { return s[kb][i]; };
+      soften(s, small, NKB, k0, c, [&](int kb, int i, float mc) { return s[kb][i] * c - mc; }, score);
     }
     Pieces pf[NKB][2];
 #pragma unroll
@@ -394,8 +432,10 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
 
   // ---- values that pieces do not hold, anywhere in the workgroup: its rows again with the fp32 product ----
   // (up to here the lost bits of Q and K move a scaled score by less than 2^-37)
-  // (two pieces: what Q and K lack of 2^-36 each moves one by less than 2^-22)
-  const bool held = HALF ? top < 0x1p14f && top * unit * (float)a.D <= 0x1p14f && unit > 0x1p-100f && unit < 0x1p100f : fmaxf(top, 1.f) * a.scale <= 0x1p80f;
+  // (two pieces: what Q and K lack of 2^-36 of 2^15 each, D times, moves one by less than 2^-22, or than half an fp32 unit of the row's
+  // largest score, which the sum of its products is rounded to anyway)
+  const bool held = HALF ? row_unit * half_down(key_exp) * (16.f * D) <= fmaxf(4.f, fabsf(m_i) - kLazyRescale) && unit > 0x1p-30f && unit < 0x1p30f
+                         : fmaxf(top, 1.f) * a.scale <= 0x1p80f;
   float finite = 0.f;
 #pragma unroll
   for (int db = 0; db < DB; db++)
@@ -425,7 +465,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
 #pragma unroll
           for (int i = 0; i < 4; i++) s[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[i], q[ks][e][i], s[0], 0, 0, 0);
         }
-      soften(s, 1, k0, c, [&](int, int i, float mc) { return s[0][i] * c - mc; });
+      auto score = [&](int, int i) { return s[0][i]; };
+      soften(s, s, 1, k0, c, [&](int, int i, float mc) { return s[0][i] * c - mc; }, score);
       auto v_at = [&](int key, int db) { return key < n_keys && 32 * db + n < a.D ? vp[(int64_t)key * a.vs[2] + 32 * db + n] : 0.f; };
       if (!CAUSAL || k0 + 31 <= wave_q_lo) {
 #pragma unroll
@@ -454,7 +495,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
     constexpr int NF = DB * 16 + 2;
     static_assert(RW * NF * 64 * 4 <= (int)sizeof(planes), "the partial results fit the planes");
     float *xch = reinterpret_cast<float *>(planes) + (wave % RW) * (NF * 64) + lane;
-    const float in_c = redo ? c : unit;  // (what the max is a multiple of)
+    const float in_c = HALF ? 1.f : c;  // (what the max is a multiple of)
     if (kg > 0) {
       xch[0] = m_i;
       xch[64] = l_i;

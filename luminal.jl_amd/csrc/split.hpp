@@ -49,6 +49,12 @@ struct HalfPieces {
   half8_t hi, lo;
 };
 constexpr float kHalfGap = 2048.f;
+// Values whose largest is `top`, in [2^14, 2^15) at its exponent: times half_up, and what comes of them times half_down. What is all below 2^-30 is
+// left smaller. Infinities stay infinite.
+constexpr int kHalfLeast = 97;  // biased exponent of 2^-30
+__device__ inline int half_exponent(float top) { return max((int)(__float_as_uint(top) >> 23), kHalfLeast); }
+__device__ inline float half_up(int exponent) { return __uint_as_float((uint32_t)(268 - exponent) << 23); }
+__device__ inline float half_down(int exponent) { return __uint_as_float((uint32_t)(exponent - 14) << 23); }
 
 __device__ inline uint32_t round_half2(float a, float b) {
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -70,8 +76,9 @@ __device__ inline HalfPieces split_half_8(const floatx4_t &x0, const floatx4_t &
   }
   return {__builtin_bit_cast(half8_t, make_uint4(hi[0], hi[1], hi[2], hi[3])), __builtin_bit_cast(half8_t, make_uint4(lo[0], lo[1], lo[2], lo[3]))};
 }
-__device__ inline HalfPieces split_half_8(const floatx4_t &x0, const floatx4_t &x1) {
-  return split_half_8(x0, x1, [](float x) { return x; }, [](float x, float h) { return fmaf(h, -kHalfGap, x * kHalfGap); });
+// x times a power of two.
+__device__ inline HalfPieces split_half_8(const floatx4_t &x0, const floatx4_t &x1, float up) {
+  return split_half_8(x0, x1, [=](float x) { return x * up; }, [=](float x, float h) { return fmaf(h, -kHalfGap, x * (up * kHalfGap)); });
 }
 // The same of x (by + rest): hi is the rounded product, and what the rounding leaves of the exact one goes to lo.
 __device__ inline HalfPieces split_half_8(const floatx4_t &x0, const floatx4_t &x1, float by, float rest) {

@@ -1,5 +1,7 @@
 """fp32 flash attention of head dims 104 to 128 on pieces of 16 bits (queries and keys as two fp16 pieces): row and key tiles with remainders,
 head dims that do not fill the tiling, ragged keys, rotated queries, and values that the pieces do not hold."""
+import time
+
 import numpy as np
 import pytest
 
@@ -82,3 +84,76 @@ def test_large_logits(lm, hip, oracle):
     got = run(lm, hip, q, k, v, "f32", False)
     # |s| below 60 in natural units comes with 128 products of at most 2^-22 of 30 each: 1e-4 at worst, a hundredth of it in the mean
     assert rel_err(got, oracle.flash_attn(q, k, v, nthreads=NT)) <= 1e-5
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D", [128, 112])
+def test_magnitudes_stay_on_the_pieces(lm, hip, oracle, causal, D):
+    """Powers of two taken from the keys and given to the queries, and the other way, leave every bit: both are split relative to their own
+    magnitude, and none of these goes to the fp32 product, whose sums are others."""
+    q, k, v = inputs(oracle, (1, 40, 700, D), (1, 8, 700, D), "f32", 52500 + D)
+    assert "prefill_f32_split_kernel" in plan(lm, q, k, "f32", causal, False)
+    want = run(lm, hip, q, k, v, "f32", causal)
+    for by in (-27, -17, -10, 7, 12, 27):
+        got = run(lm, hip, q * np.float32(2.0 ** by), k * np.float32(2.0 ** -by), v, "f32", causal)
+        np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("q_mul,k_mul", [(1e3, 1e-5), (1.0, 3e3), (2e3, 1.0), (300.0, 300.0)])
+def test_error_at_large_and_small_magnitudes(lm, hip, oracle, q_mul, k_mul):
+    """No further from 64 bits than scores that one fp32 product after the other is added to (the softmax in 64 bits), with half as much again for
+    the weights' and the result's own roundings where scores are so small that those count (3e-7 as above)."""
+    q, k, v = inputs(oracle, (1, 40, 600, 128), (1, 8, 600, 128), "f32", 52600)
+    q, k = q * np.float32(q_mul), k * np.float32(k_mul)
+    assert "prefill_f32_split_kernel" in plan(lm, q, k, "f32", False, False)
+    got = run(lm, hip, q, k, v, "f32", False)[0, :8].astype(np.float64)
+    scale = np.float32(lm.default_scale(128))
+    chain = np.zeros((8, 600, 600), np.float32)
+    for d in range(128):
+        chain += q[0, :8, :, d, None] * k[0, :, None, :, d]
+    exact = q[0, :8].astype(np.float64) @ np.swapaxes(k[0].astype(np.float64), 1, 2)
+
+    def attend(s):
+        s = s * np.float64(scale)
+        w = np.exp(s - s.max(-1, keepdims=True))
+        return (w / w.sum(-1, keepdims=True)) @ v[0].astype(np.float64)
+    want = attend(exact)
+    size = np.linalg.norm(want)
+    assert np.linalg.norm(got - want) <= max(1.5 * np.linalg.norm(attend(chain.astype(np.float64)) - want), 3e-7 * size)
+
+
+@pytest.mark.parametrize("by,most", [(2.0 ** 14, 3e-7), (2.0 ** 24, 7e-7), (2.0 ** 40, 7e-7)])  # (the pieces' error, and the fp32 product's, as above)
+def test_one_large_key_among_small_ones(lm, hip, oracle, by, most):
+    """The queries that turn away from it weigh the others as if it were not there: where the pieces would lose bits of those, fp32 takes over."""
+    q, k, v = inputs(oracle, (1, 40, 700, 128), (1, 8, 700, 128), "f32", 52700)
+    k[0, :, 70] *= np.float32(by)
+    assert "prefill_f32_split_kernel" in plan(lm, q, k, "f32", False, False)
+    got = run(lm, hip, q, k, v, "f32", False)
+    away = np.einsum("hsd,hd->hs", q[0, :8].astype(np.float64), k[0, :, 70].astype(np.float64)) < 0
+    s = q[0, :8].astype(np.float64) @ np.swapaxes(k[0].astype(np.float64), 1, 2) * np.float64(np.float32(lm.default_scale(128)))
+    w = np.exp(s - s.max(-1, keepdims=True))
+    want = (w / w.sum(-1, keepdims=True)) @ v[0].astype(np.float64)
+    assert away.sum() > 1000
+    assert np.linalg.norm((got[0, :8] - want)[away]) <= most * np.linalg.norm(want[away])
+
+
+def test_large_values_take_no_longer(lm, hip, oracle):
+    """Rows that go to the fp32 product as well take five times as long: queries and keys in the thousands do not."""
+    q, k, v = inputs(oracle, (1, 32, 1024, 128), (1, 8, 1024, 128), "f32", 52800)
+    op = lm.FlashAttentionOp(lm.default_scale(128), False)
+
+    def best(mul):
+        dq, dk, dv = (lm.to_device(x, hip, "f32") for x in (q * np.float32(mul), k * np.float32(mul), v))
+        out = lm.HipArray(q.shape, "f32", hip)
+        times = []
+        for _ in range(8):
+            lm.binding.sync()
+            at = time.perf_counter()
+            for _ in range(5):
+                lm.host.execute_op_inplace(out, op, dq, dk, dv)
+            lm.binding.sync()
+            times.append(time.perf_counter() - at)
+        return min(times)
+    usual = best(1.0)
+    for mul in (100.0, 1e3, 5e3):
+        assert best(mul) < 2 * usual
