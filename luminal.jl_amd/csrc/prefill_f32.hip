@@ -375,40 +375,56 @@ int launch_for_d(const PrefillArgs &a, hipStream_t stream) {
     }
     const bool many = tiles(128) >= 4 * n_cus;
     const double c128 = form_cost<D, 8, 1, 2>(a, 0.96);
-    // In pieces (prefill_f32_split.hip), up to head dim 128: by the time that the cost of the form here stands for, in us (a part
+    // In pieces (prefill_f32_split.hip), up to head dim 96: by the time that the cost of the form here stands for, in us (a part
     // per launch, a part per key of the walk; fitted to 240 launches of drawn sizes, rms 2 to 13 %). Of 330 such launches 159 go
     // over, none loses more than 4 %, and together the 330 gain 12 %: B=2 H=12 S=1023 D=80 without a mask 76 -> 57 us, B=1 H=32
     // S=2048 D=96 380 -> 255, causal 214 -> 150, B=1 H=48 S=1100 D=64 causal 79 -> 58. The small launches stay because their waves
     // walk the keys alone (B=1 H=6 S=846 D=96 causal), and without a mask what the pieces would take less than 14.5 us for, where
     // the fit overrates the forms here: D=72 to 96 on up to 170 keys 4 to 14 us here, up to 2 times that there (H=12 502 x 167
     // D=72 13.5 and 14.0), while above it 55 of 60 drawn launches of up to 340 keys gain (20 x 300 x 119 D=80, B=4, 28.9 -> 21.2) and
-    // the worst loses 7 % (H=4 1981 x 163 D=96, B=2, 16.3 and 17.5). Of 220 launches of head dims 104, 112 and 128, in 128 rows only, 136
-    // go over: 20 % off all 220 together, the worst loses 3 % (B=3 H=8 1328 x 508 D=128 77.9 and 80.0); the others are up to twice as fast here
-    // (B=3 H=2 S=1137 D=128 causal, 54 workgroups of 128 rows, 37.6 and 72.5). Without a mask one round of two key tiles stays, 17.5 us by the
-    // estimate (H=8 470 x 67 D=128, B=8, 21.2 and 19.7), and 9 of the 10 above it that are estimated below 40 gain 4 to 31 %; and where two key groups
-    // of 64 rows take a round, up to 320 keys come out even (B=3 H=7 S=640 D=128, 256 / 320 / 512 keys: 25.1 / 31.2 / 42.9 here, 25.2 / 29.7 / 39.0 there).
-    auto pieces = [&](double here, int *form) {
-      constexpr double fit[7][2][2] = {{{6.6, 0.0178}, {4.3, 0.0197}}, {{6.1, 0.0249}, {5.1, 0.0277}}, {{5.6, 0.0352}, {5.7, 0.0351}},
-                                       {{7.5, 0.0419}, {6.4, 0.0451}}, {{6.2, 0.0527}, {8.6, 0.0505}},
-                                       {{10.4, 0.0591}, {8.7, 0.0562}}, {{9.9, 0.0707}, {12.1, 0.0629}}};  // D = 32, 48, 64, 80, 96, 112, 128
-      const auto &f = fit[D == 128 ? 6 : D / 16 - 2][a.causal != 0];
+    // the worst loses 7 % (H=4 1981 x 163 D=96, B=2, 16.3 and 17.5).
+    // Above it, up to head dim 128, the same by a fit of each form's own (2300 launches, rms 2 to 11 %): where its cost stands for a time by one fit for all, an
+    // error of 20 % counts for more than what the pieces gain on a launch of one round (B=8 H=12 S=189 D=128 causal 18.7 here and 22.6 in pieces, H=32 S=305,
+    // B=2, 26.2 and 30.5). Of 2000 other drawn launches of head dims 104 to 128 (24 to 6000 workgroups, a third with lengths) 1168 go over: 29 % off all of
+    // them together, 18 lose more than 5 %, the worst 11 % (B=9 H=8 S=219 without a mask, with lengths, 22.5 and 25.3); by one fit 55 lost that, up to 19 %.
+    // Causal launches of one round are closest. Below 18 us by the estimate, a round of two key tiles, the other costs of a launch decide: they stay.
+    enum Here { kC128, kC64, kC32, kC32x2, kC16, kF128, kF64 };
+    auto pieces = [&](double here, Here which, int *form) {
       const double split = prefill_f32_split_cost(a, form);
-      if (D > 96 && f64 < f128 && a.Sk <= 320) return false;
-      return (a.causal || split >= (D > 96 ? 18.0 : 14.5)) && split < 0.95 * (f[0] + f[1] * here);
+      if constexpr (D > 96) {
+        constexpr double fit[2][2][7][2] = {  // [D = 112, 128][causal][Here]
+            {{{6.7, 0.0577}, {5.7, 0.0621}, {6.6, 0.0550}, {4.9, 0.0674}, {3.7, 0.0723}, {}, {}},
+             {{11.4, 0.0550}, {11.8, 0.0545}, {10.7, 0.0530}, {8.1, 0.0599}, {6.0, 0.0636}, {}, {}}},
+            {{{6.7, 0.0701}, {6.7, 0.0701}, {7.6, 0.0640}, {5.5, 0.0756}, {4.4, 0.0812}, {7.6, 0.0681}, {6.6, 0.0654}},
+             {{16.2, 0.0614}, {19.1, 0.0590}, {11.7, 0.0604}, {7.6, 0.0709}, {5.7, 0.0768}, {}, {}}}};
+        const auto &f = fit[D == 128][a.causal != 0][which];
+        const bool close = D == 128 && a.causal && tiles(128) <= n_cus;
+        return split >= 18.0 && split < (close ? 0.92 : 0.96) * (f[0] + f[1] * here);
+      } else {
+        constexpr double fit[5][2][2] = {{{6.6, 0.0178}, {4.3, 0.0197}}, {{6.1, 0.0249}, {5.1, 0.0277}}, {{5.6, 0.0352}, {5.7, 0.0351}},
+                                         {{7.5, 0.0419}, {6.4, 0.0451}}, {{6.2, 0.0527}, {8.6, 0.0505}}};  // D = 32, 48, 64, 80, 96
+        const auto &f = fit[D / 16 - 2][a.causal != 0];
+        return (a.causal || split >= 14.5) && split < 0.95 * (f[0] + f[1] * here);
+      }
     };
     int split_form = 0;
-    if (many && pieces(kFull && !a.causal ? f128 : c128, &split_form)) return launch_prefill_f32_split(a, split_form, stream);
+    if (many && (kFull && !a.causal ? pieces(f128, kF128, &split_form) : pieces(c128, kC128, &split_form))) return launch_prefill_f32_split(a, split_form, stream);
     if (many) return kFull && !a.causal ? launch_prefill_f32_full(a, 1, stream) : launch_form<D, 8, 1, 2>(a, stream);
     const bool few32 = tiles(32) <= (a.causal ? 2 : 1) * n_cus, few16 = tiles(16) <= 2 * n_cus;
     const double c64 = form_cost<D, 4, 1, 2>(a, 1.0), c32 = form_cost<D, 2, 2, 1>(a, w32),
                  c32x2 = form_cost<D, 2, 2, 2>(a, few32 ? 1.0 : D <= 64 ? 1.15 : 1.4), c16 = form_cost<D, 1, 4, 1>(a, few16 ? 1.2 : D <= 64 ? 1.5 : 1.8);
     const double best = fmin(fmin(c128, c64), fmin(fmin(c32, c32x2), c16));
-    if (pieces(fmin(best, fmin(f128, f64)), &split_form)) return launch_prefill_f32_split(a, split_form, stream);
-    if (fmin(f128, f64) < best) return launch_prefill_f32_full(a, f64 < f128 ? 2 : 1, stream);
-    if (best == c128) return launch_form<D, 8, 1, 2>(a, stream);
-    if (best == c64) return launch_form<D, 4, 1, 2>(a, stream);
-    if (best == c32) return launch_form<D, 2, 2, 1>(a, stream);
-    if (best == c32x2) return launch_form<D, 2, 2, 2>(a, stream);
+    const Here which = fmin(f128, f64) < best ? (f64 < f128 ? kF64 : kF128) : best == c128 ? kC128 : best == c64 ? kC64 : best == c32 ? kC32 : best == c32x2 ? kC32x2 : kC16;
+    if (pieces(fmin(best, fmin(f128, f64)), which, &split_form)) return launch_prefill_f32_split(a, split_form, stream);
+    switch (which) {
+      case kF128: return launch_prefill_f32_full(a, 1, stream);
+      case kF64: return launch_prefill_f32_full(a, 2, stream);
+      case kC128: return launch_form<D, 8, 1, 2>(a, stream);
+      case kC64: return launch_form<D, 4, 1, 2>(a, stream);
+      case kC32: return launch_form<D, 2, 2, 1>(a, stream);
+      case kC32x2: return launch_form<D, 2, 2, 2>(a, stream);
+      case kC16: break;
+    }
     return launch_form<D, 1, 4, 1>(a, stream);
   }
 }

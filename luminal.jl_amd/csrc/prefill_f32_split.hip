@@ -557,20 +557,32 @@ int launch_for_d(const PrefillArgs &a, int form, hipStream_t stream) {
 
 }  // namespace
 
-// Estimated microseconds of the cheapest form (0: 64 rows, two workgroups on a CU; 1: 128 rows, the only one above head dim 96; 2: 256 rows), from the launch's own
+// Estimated microseconds of the cheapest form (0: 64 rows, two workgroups on a CU; 1: 128 rows; 2: 256 rows), from the launch's own
 // tiles as in prefill_mfma.hip: without a mask whole rounds, causal the longest workgroup and the mean over the CUs. Fitted to 330
 // launches of drawn sizes, rms 3 to 10 %.
 double prefill_f32_split_cost(const PrefillArgs &a, int *form) {
   struct Cost { double fixed, alone, per_wg, shared; };  // a tile of 64 keys in a CU's only workgroup, and in one of several
-  static const Cost costs[4][3][2] = {  // [head dims up to 64, 80, 96, 128][form][causal]
+  const int64_t cus = device_cu_count(), heads = (int64_t)a.B * a.Hq, row_tiles = (a.Sk + 63) / 64;
+  if (a.D > 96) {  // in 128 rows only; fitted to 2300 launches, rms 4 to 8 %
+    static const Cost wide[2][2] = {{{-0.68, 3.68, 9.29, 3.97}, {1.13, 3.44, 8.35, 4.30}}, {{-0.68, 3.70, 10.75, 4.06}, {0.89, 3.48, 9.58, 4.52}}};  // [up to 112, 128][causal]
+    const Cost &c = wide[a.D > 112][a.causal != 0];
+    const int64_t n = (a.Sq + 127) / 128, rounds = (heads * n + cus - 1) / cus;
+    *form = 1;
+    if (!a.causal) return c.fixed + row_tiles * (rounds <= 1 ? c.alone : c.shared * rounds) + c.per_wg * rounds;
+    // the last workgroup of a head ends at its last row, the others 128 rows apart (causal_shift): of `diagonal` key tiles, two less each, `all` walk every key
+    const int64_t diagonal = (a.Sq + 63) / 64, all = std::min(n, std::max<int64_t>(0, (diagonal - row_tiles + 1) / 2));
+    const double longest = (double)std::min(row_tiles, diagonal) * c.alone;
+    if (rounds <= 1) return c.fixed + longest + c.per_wg;
+    const double mean = (double)heads * (all * row_tiles + (n - all) * (diagonal - (n - 1 + all))) / cus * c.shared;
+    return c.fixed + sqrt(sqrt(longest * longest * longest * longest + mean * mean * mean * mean)) + c.per_wg * (heads * n) / cus;
+  }
+  static const Cost costs[3][3][2] = {  // [head dims up to 64, 80, 96][form][causal]
       {{{3.3, 1.89, 1.8, 1.33}, {3.6, 1.86, 1.8, 1.40}}, {{1.3, 2.26, 5.7, 0.}, {1.5, 2.13, 6.4, 2.47}}, {{0., 4.26, 8.4, 0.}, {0., 3.98, 8.4, 4.13}}},
       {{{2.6, 2.61, 2.4, 1.76}, {3.3, 2.51, 2.7, 1.85}}, {{0., 3.00, 7.0, 0.}, {0., 2.86, 8.0, 3.28}}, {{0., 4.96, 10.3, 0.}, {0., 4.46, 10.1, 5.47}}},
-      {{{0.2, 3.36, 5.0, 2.28}, {2.3, 3.17, 5.5, 2.19}}, {{0., 3.30, 8.9, 0.}, {0., 3.03, 10.3, 3.44}}, {{0., 6.3, 11.6, 0.}, {0., 5.73, 10.0, 6.74}}},
-      {{}, {{0., 3.82, 9.9, 0.}, {5.4, 3.49, 4.0, 4.63}}, {}}};  // (220 launches of head dims 104, 112 and 128, rms 6 and 10 %)
-  const int64_t cus = device_cu_count(), heads = (int64_t)a.B * a.Hq, row_tiles = (a.Sk + 63) / 64;
+      {{{0.2, 3.36, 5.0, 2.28}, {2.3, 3.17, 5.5, 2.19}}, {{0., 3.30, 8.9, 0.}, {0., 3.03, 10.3, 3.44}}, {{0., 6.3, 11.6, 0.}, {0., 5.73, 10.0, 6.74}}}};
   double least = INFINITY;
-  for (int f = a.D > 96 ? 1 : 0; f < (a.D > 96 ? 2 : 3); f++) {
-    const Cost &c = costs[a.D <= 64 ? 0 : a.D <= 80 ? 1 : a.D <= 96 ? 2 : 3][f][a.causal != 0];
+  for (int f = 0; f < 3; f++) {
+    const Cost &c = costs[a.D <= 64 ? 0 : a.D <= 80 ? 1 : 2][f][a.causal != 0];
     const int64_t step = int64_t(1) << f, n = (a.Sq + 64 * step - 1) / (64 * step), rounds = (heads * n + cus - 1) / cus;
     double t;
     if (!a.causal) {
