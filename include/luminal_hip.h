@@ -216,6 +216,10 @@ size_t lmh_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lm
 int32_t lmh_decode_auto_splits(int32_t B, int32_t Hkv, int32_t Lmax);
 int lmh_decode_attn(const lmh_decode_params *p);
 
+/* Which kernel lmh_decode_attn would launch for `p`, in how many splits, as text in `plan`, as lmh_flash_attn_plan does for flash attention:
+ * nothing is launched and no tensor is touched; the workspace counts with its size. */
+int lmh_decode_plan(const lmh_decode_params *p, char *plan, size_t plan_bytes);
+
 /* ---- one decode step of a cached attention layer in one or two launches: append + attend.
  * Replaces, for one layer, what decode_step! does with the self-attention caches (reference
  * src/Whisper.jl:761-801: feed the caches in, run whisper_self_attn_cached :584-620, take the rebuilt caches

@@ -24,7 +24,7 @@ EXPORTS = [
     "lmh_version", "lmh_measurement_build", "lmh_last_error", "lmh_device_count", "lmh_init", "lmh_device_name", "lmh_malloc", "lmh_free",
     "lmh_memset", "lmh_memcpy_h2d", "lmh_memcpy_d2h", "lmh_memcpy_d2d", "lmh_sync", "lmh_event_create",
     "lmh_event_destroy", "lmh_event_record", "lmh_event_elapsed_ms", "lmh_flash_attn_fwd",
-    "lmh_decode_workspace_bytes", "lmh_decode_auto_splits", "lmh_decode_attn", "lmh_flash_attn_plan", "lmh_rope",
+    "lmh_decode_workspace_bytes", "lmh_decode_auto_splits", "lmh_decode_attn", "lmh_flash_attn_plan", "lmh_decode_plan", "lmh_rope",
     "lmh_kv_append", "lmh_stream_create", "lmh_stream_destroy", "lmh_graph_capture_begin", "lmh_graph_capture_end",
     "lmh_graph_launch", "lmh_graph_destroy", "lmh_static_scratch_bytes", "lmh_decode_static_splits",
     "lmh_decode_attn_static", "lmh_decode_step_splits", "lmh_decode_step", "lmh_matmul", "lmh_map", "lmh_copy_many", "lmh_decode_step_fed", "lmh_kv_append_fed", "lmh_matmul_fed",
@@ -179,6 +179,8 @@ def load():
     L.lmh_decode_static_splits.argtypes = [ctypes.c_int32] * 5
     L.lmh_flash_attn_plan.argtypes = [ctypes.POINTER(AttnParams), ctypes.c_char_p, ctypes.c_size_t]
     L.lmh_flash_attn_plan.restype = ctypes.c_int
+    L.lmh_decode_plan.argtypes = [ctypes.POINTER(DecodeParams), ctypes.c_char_p, ctypes.c_size_t]
+    L.lmh_decode_plan.restype = ctypes.c_int
     L.lmh_rope.argtypes = [ctypes.POINTER(RopeParams)]
     L.lmh_kv_append.argtypes = [ctypes.POINTER(KvAppendParams)]
     L.lmh_stream_create.argtypes = [ctypes.POINTER(vp)]
@@ -440,6 +442,13 @@ def flash_attn_plan(params):
     """Text naming the kernel lmh_flash_attn_fwd would launch for `params`; launches nothing."""
     buf = ctypes.create_string_buffer(256)
     check(load().lmh_flash_attn_plan(ctypes.byref(params), buf, len(buf)))
+    return buf.value.decode()
+
+
+def decode_plan(params):
+    """Text naming the kernel lmh_decode_attn would launch for `params`; launches nothing."""
+    buf = ctypes.create_string_buffer(256)
+    check(load().lmh_decode_plan(ctypes.byref(params), buf, len(buf)))
     return buf.value.decode()
 
 

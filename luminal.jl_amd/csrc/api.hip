@@ -632,6 +632,16 @@ int lmh_decode_attn(const lmh_decode_params *p) {
   return decode_launch(p, "lmh_decode_attn", splits, p->workspace, p->workspace_bytes, p->num_splits == 0);
 }
 
+int lmh_decode_plan(const lmh_decode_params *p, char *plan, size_t plan_bytes) {
+  if (!plan || plan_bytes < 2) return fail(LMH_E_NULL, "lmh_decode_plan: no room for the description");
+  plan[0] = 0;
+  g_plan_buf = plan;
+  g_plan_bytes = plan_bytes;
+  const int rc = lmh_decode_attn(p);
+  g_plan_buf = nullptr;
+  return rc;
+}
+
 int32_t lmh_decode_step_splits(int32_t B, int32_t Hkv, int32_t Lmax) {
   const int32_t s = lmh_decode_auto_splits(B, Hkv, Lmax);
   return s == 0 ? 0 : (s < 2 ? 2 : s);  // the merge launch always runs: it is what adds the new row

@@ -19,7 +19,7 @@ int device_cu_count();
 int hip_fail(hipError_t e, const char *what);
 // LMH_OK, or the error of a launch whose threads a grid cannot number.
 int check_grid(int64_t workgroups, int threads);
-// While a plan query (lmh_flash_attn_plan) runs on this thread, a launcher that calls this with the description of
+// While a plan query (lmh_flash_attn_plan, lmh_decode_plan) runs on this thread, a launcher that calls this with the description of
 // the kernel it has chosen gets `true` back and must return LMH_OK without launching.
 bool plan_only(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 

@@ -561,6 +561,9 @@ int launch_for_lpk(const DecodeArgs &a, hipStream_t stream) {
   const int64_t cus = device_cu_count();
   const bool wide = a.num_splits == 1 ? f.units <= cus && 2 * a.Lmax > 7 * f.keys && f.heads * E::kVec < 32 && one_split(f, a.Lmax, E::kVec, cus)
                                       : few_units(f, a.Lmax, cus) && f.units * a.num_splits <= cus;
+  if (plan_only("decode_split_kernel<%s, lanes a key=%d, heads=%d, waves=%d> splits=%d", E::kName, LPK, f.heads, wide && f.heads <= 4 ? wide_waves(f.heads, E::kVec) : kWaves,
+                a.num_splits))
+    return LMH_OK;
   auto launch = [&](auto heads) {
     constexpr int G = decltype(heads)::value, W = wide_waves(G, E::kVec);
     const int g_chunks = (a.Hq / a.Hkv + G - 1) / G;
@@ -613,6 +616,9 @@ int launch_decode(const DecodeArgs &a, int dtype, hipStream_t stream, CopyManyAr
   // (the matrix-core kernel deals its (b, kv head slice, chunk) units in 32-bit arithmetic)
   const int64_t mfma_units = (int64_t)a.B * a.Hkv * ((a.Hq / a.Hkv + 15) / 16) * a.num_splits;
   if (decode_mfma_takes(a, dtype) && mfma_units < (int64_t(1) << 31)) {
+    if (plan_only("decode_%s_kernel<%s, D=%d> splits=%d", a.num_splits == 1 && (a.step || decode_by_pairs(a)) ? "pair" : "mfma", dtype == LMH_F16 ? F16::kName : BF16::kName, a.D,
+                  a.num_splits))
+      return LMH_OK;
     const int n_copies = n_fed ? (int)number_copy_blocks(*fed, n_fed) : 0;
     const int rc = launch_decode_mfma_split(a, dtype, stream, fed, n_copies);
     if (rc != LMH_OK || a.num_splits == 1) return rc;

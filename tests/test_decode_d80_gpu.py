@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from conftest import TOL, rel_err
+from test_decode_valu_gpu import plan
 from test_parity_gpu import inputs, run_decode
 
 pytestmark = pytest.mark.gpu
@@ -45,3 +46,13 @@ def test_infinite_values(lm, hip, oracle, dtype, splits):
     w[1, 0, 7, 3] = np.nan
     got = run_decode(lm, hip, q, k, w, dtype, num_splits=splits)
     assert np.isnan(got[1, ::2, 3]).all() and np.isnan(got).sum() == 8
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("B,Hq,Hkv,L,form", [
+    (2, 3, 1, 161, "decode_mfma_kernel"), (1, 6, 1, 700, "decode_mfma_kernel"), (70, 8, 8, 385, "decode_mfma_kernel"), (9, 48, 6, 153, "decode_mfma_kernel"),
+    (2, 3, 1, 160, "decode_split_kernel"), (4, 4, 2, 31, "decode_split_kernel"), (70, 8, 8, 383, "decode_split_kernel"), (1030, 3, 1, 170, "decode_split_kernel")])
+def test_which_kernel(lm, hip, dtype, B, Hq, Hkv, L, form):
+    """The lines of the choice, whatever the count of splits; batches that the persistent kernel does not take stay off it."""
+    for splits in (0, 3):
+        assert plan(lm, dtype, B, Hq, Hkv, L, 80, splits).startswith(form)

@@ -230,7 +230,9 @@ def test_operands_taken_from_the_callers_arrays(lm, hip, dtype, B, Hq, Hkv, T, L
     ("f16", 4, 64, 8, 897, 900, 128, "D=128, causal, key groups=1, waves=8, waves per SIMD=2>"),
     ("bf16", 2, 64, 8, 2101, 2200, 64, "D=64, causal, key groups=1, waves=8, waves per SIMD=4>"),
     ("bf16", 1, 64, 8, 2100, 2100, 96, "D=96, causal, key groups=1, waves=8, waves per SIMD=2>"),
-    ("bf16", 2, 64, 8, 2177, 2300, 128, "D=128, causal, key groups=1, waves=8, waves per SIMD=2>")])
+    ("bf16", 2, 64, 8, 2177, 2300, 128, "D=128, causal, key groups=1, waves=8, waves per SIMD=2>"),
+    ("f16", 1, 4, 4, 2175, 2300, 128, "D=128, causal, key groups=4, waves=8,"), ("bf16", 1, 5, 5, 2113, 2200, 96, "D=96, causal, key groups=4, waves=8,"),  # few workgroups
+    ("f16", 1, 3, 3, 1537, 1600, 64, "D=64, causal, key groups=8, waves=8,")])
 def test_queries_stored_by_the_forms_of_large_prompts(lm, hip, dtype, B, Hq, Hkv, T, L, D, form):
     """The attention launch of a prompt stores the graph's copy of the queries: every row of it in the 256-row and paired-tile forms
     too, whose last tile is partly filled, and the result is the one of queries that were copied in front of the launch."""

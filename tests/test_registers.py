@@ -52,3 +52,15 @@ def test_loops_at_the_register_limit(spilled, policy, causal, waves, per_simd, h
     form = "19prefill_mfma_kernelINS0_%sELi96ELb%dELi1ELi%dELi%dELb0ELi%dE" % (policy, causal, waves, per_simd, heads)
     sizes = [size for name, size in spilled.items() if form in name and not name.endswith(".kd")]
     assert len(sizes) == 1 and sizes[0] <= most
+
+
+@pytest.mark.parametrize("kernel,most", [
+    ("24prefill_f32_split_kernelILi128ELb0ELi8ELi2E", 0), ("24prefill_f32_split_kernelILi128ELb1ELi8ELi2E", 128),  # 48 in the loop, the others where rows are taken again
+    ("19prefill_mfma_kernelINS0_7MfmaF16ELi256ELb0ELi4ELi8E", 20), ("19prefill_mfma_kernelINS0_7MfmaF16ELi256ELb1ELi4ELi8E", 0),
+    ("19prefill_mfma_kernelINS0_7MfmaF16ELi192ELb1ELi4ELi8E", 0), ("19prefill_mfma_kernelINS0_8MfmaBF16ELi128ELb1ELi4ELi8E", 0),
+    ("19prefill_mfma_kernelINS0_8MfmaBF16ELi64ELb1ELi8ELi8E", 0), ("18decode_mfma_kernelINS0_10Mfma16BF16ELi80ELb0E", 0),
+    ("18decode_mfma_kernelINS0_13Mfma16F16FullELi80ELb0E", 0)])
+def test_two_waves_per_simd_and_key_groups(spilled, kernel, most):
+    """Present values, as ceilings."""
+    sizes = [size for name, size in spilled.items() if kernel in name and not name.endswith(".kd")]
+    assert len(sizes) == 1 and sizes[0] <= most
