@@ -1999,7 +1999,9 @@ int launch_for_d(const PrefillArgs &a, const QueryCopy &queries, hipStream_t str
 // 64 in 2.1 to 2.4; folding four groups costs it 3 to 5 us a workgroup. fp16, us in the form of before and in it: 16 heads 548 x 5273 D=160 88.1 and 64.7, H=6
 // S=2255 causal 42.6 and 32.7, H=2 S=6502 D=192 causal 109.8 and 82.5, H=1 S=5850 D=256 causal 108.3 and 89.0, H=3 S=2389 51.0 and 45.1, H=6 110 x 2476
 // 52.9 and 46.9. Fitted to 64 launches of 500 to 8192 keys that one or two of the others were best for: 29 go over, none loses more than 2.6 % (H=2 S=1739 D=256
-// 22.4 and 24.1 stays). bf16, with twice the second products, comes out even (H=8 S=3130 D=256 causal 71.4 and 73.3, 16/8 heads S=1500 45.7 and 52.3). With the
+// 22.4 and 24.1 stays). Launches of more workgroups than CUs, whose K and V the 64-row tiles read more often, go over from 15 % on (H=6 S=7218 D=256
+// causal with lengths 144.5 and 168.5, B=5 H=4 S=961 D=192 causal 22.0 and 24.7, 160 heads 252 x 4832 D=176 242 and 354 stay): of 3000 drawn launches 527 go over,
+// 1.17 times as fast in the geometric mean, none loses more than 5 %; from 0 % on 611 did, 13 of them lost that, up to 30 %. bf16, with twice the second products, comes out even (H=8 S=3130 D=256 causal 71.4 and 73.3, 16/8 heads S=1500 45.7 and 52.3). With the
 // second half's waves a barrier behind, so that one half's softmax stands beside the other's second product, it took 2 to 10 % longer (H=3 3451 keys D=160
 // 45.4 and 48.1): the phases are as long as the fetches then.
 // B=1 H=32 S=4096 D=256 causal fp16 takes 292 us = 940 TFLOP/s (363 with 128 rows on four waves as the only form).
@@ -2024,7 +2026,7 @@ int launch_wide_heads(const PrefillArgs &a, const QueryCopy &queries, hipStream_
   }
   const double rows64 = cost(64, 1., 5.), rows128 = cost(128, 1.4, 5.), eight = cost(128, 1.2, 6.);
   if constexpr (!MT::kSplitP)
-    if (cost(64, 0.68, D <= 192 ? 9. : 15., 2) < std::min(rows64, std::min(rows128, eight))) return launch_split<MT, false, D, 4, 8, 2>(a, queries, stream);
+    if (cost(64, 0.68, D <= 192 ? 9. : 15., 2) < (heads * ((a.Sq + 63) / 64) > cus ? 0.85 : 1.) * std::min(rows64, std::min(rows128, eight))) return launch_split<MT, false, D, 4, 8, 2>(a, queries, stream);
   if (rows64 <= std::min(rows128, eight)) return launch_split<MT, false, D, 2, 4, 1, true>(a, queries, stream);
   if (rows128 < 0.98 * eight) return launch_split<MT, false, D, 1, 4, 1, true>(a, queries, stream);
   return launch_split<MT, false, D, 2, 8, 2>(a, queries, stream);

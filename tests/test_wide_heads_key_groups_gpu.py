@@ -46,3 +46,10 @@ def test_lines_of_the_choice(lm, oracle):
     assert FORM in name(1, 2, 2400, 256) and FORM in name(1, 2, 1200, 160)
     for call in [(1, 2, 1500, 256), (1, 2, 600, 160), (1, 2, 2400, 256, "bf16"), (4, 16, 2400, 256)]:
         assert FORM not in name(*call)
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk,D,causal", [(1, 6, 7218, 7218, 256, True), (5, 4, 961, 961, 192, True), (3, 6, 1148, 1148, 192, True), (5, 32, 252, 4832, 176, False),
+                                                (14, 4, 674, 6304, 208, False)])
+def test_launches_of_more_workgroups_than_cus_stay(lm, B, H, Sq, Sk, D, causal):
+    name = lm.flash_attention_plan((B, H, Sq, D), (B, H, Sk, D), "f16", causal)
+    assert FORM not in name, name
