@@ -926,11 +926,12 @@ bool decode_mfma_supported(int dtype, int D, int B) {
 }
 
 // Whether a call's rows go to the split kernel here: the head dims above, and 80 where it is ahead of the vector ALUs. Those are busy with
-// the products from three query heads a KV head on: us there and here, fp16 and bf16, B=33 64/8 heads L=682 40.5 and 10.3, B=31 64/8 L=12366 262 and
-// 99, B=34 8/1 L=5052 45.1 and 15.4, B=57 16/4 L=1315 27.5 and 14.9, B=7 4/1 L=3337 13.0 and 10.7; walks of up to 160 keys of up to four heads stay (B=13
-// 32/8 L=152 9.2 and 9.9). Of two heads it takes the longer walks (B=1 40/20 L=12138 26.6 and 18.5, B=11 12/6 L=1269 11.1 and 10.5; B=7 12/6 L=484 8.9 and
-// 9.3) and what goes round (B=113 12/6 L=498 24.4 and 15.9; not more than four times: B=120 64/32 L=231 33.2 and 37.9), of one likewise (Hkv=12 L=3681 10.6
-// and 9.8, B=37 Hkv=16 L=1487 41.2 and 33.8; B=2 Hkv=20 L=2714 10.8 and 11.7).
+// the products from three query heads a KV head on: us there and here, bf16, every sequence Lmax long, B=33 64/8 heads L=682 49.3 and 15.4, B=31 64/8 L=12366 409
+// and 162 (981 MB; with lengths from a quarter of it up 293 and 113), B=34 8/1 L=5052 44.7 and 16.3, B=57 16/4 L=1315 34.0 and 18.3, B=7 4/1 L=3337 12.7 and 10.7;
+// walks of up to 160 keys of up to four heads stay (B=13 32/8 L=152 8.7 and 10.2). Of two heads it takes the longer walks (B=1 40/20 L=12138 26.3 and 17.2, B=11
+// 12/6 L=1269 12.2 and 11.1; B=7 12/6 L=484 9.0 and 9.2) and what goes round (B=113 12/6 L=498 26.1 and 19.9; not more than four times: B=120 64/32 L=231 48.7
+// and 47.6, with lengths 36.4 and 41.5). Of one it takes what goes round, for the lengths' sake (fp16 B=50 Hkv=12 L=844 30.7 and 29.4, with lengths 28.2 and 21.6,
+// B=37 Hkv=16 L=1487 50.0 and 49.4, 41.6 and 39.2); a round or less comes out even, and behind with lengths (bf16 B=2 Hkv=20 L=2714 12.4 and 12.0, 9.4 and 11.2).
 bool decode_mfma_takes(const DecodeArgs &a, int dtype) {
   if (!a.mfma_ok) return false;
   if (decode_mfma_supported(dtype, a.D, a.B)) return true;

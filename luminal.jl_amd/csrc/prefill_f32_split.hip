@@ -16,9 +16,11 @@
 // Bound: the bf16 matrix pipe at the clock it gets, then the vector ALUs beside it. S = 1023 D = 80, 57 us: 36 with two of the six
 // products, 52 without splitting K and V, 57 without splitting P (measurement variants).
 //
-// Head dims above 96 (HALF): the pieces of Q do not fit two waves per SIMD in three times 16 bits (160 bytes of spills: B=1 H=16 S=2048 D=128
-// causal 178 us, as with the fp32 product). Q and K are two fp16 pieces there, 22 to 24 bits: three products for one in S^T, hi lo and lo hi in
-// accumulators of their own, lo lo left out, and two planes of K instead of three. What is lost weighs less than what the fp32 product
+// Head dims above 96 (HALF): three bf16 pieces of Q and K, with 160 bytes a lane in memory beside the registers of two waves per SIMD, are as fast as
+// the fp32 product (B=1 H=16 S=2048 D=128 causal 178 us). Q and K are two fp16 pieces there, 22 to 24 bits: three products for one in S^T, hi lo and lo hi in
+// accumulators of their own, lo lo left out (Ootomo and Yokota, "Recovering single precision accuracy from Tensor Cores while surpassing the FP32 theoretical
+// peak performance", 2022), and two planes of K instead of three. The gain is half the products of S^T and a plane less; the causal kernel keeps 128 bytes in
+// memory still, 48 of them V's on its way through the loop, the one without a mask none. What is lost weighs less than what the fp32 product
 // rounds (2-norm against 64 bits, that product and this kernel): 4.6e-7 and 1.7e-7 (S = 2048 D = 128 causal), 5.7e-7 and 2.0e-7 (S = 1024),
 // 5.6e-7 and 2.0e-7 (S = 1023 D = 112). Below it, against three bf16 pieces, it would weigh 0.05 to 0.2 more than nothing (S = 1023 D = 80
 // 1.83e-7 and 1.90e-7, S = 2048 D = 64 causal 1.35e-7 and 1.52e-7), so these stay. The pieces are taken relative to a power of two, each query's
@@ -26,9 +28,9 @@
 // 1.6e-7 with the fp32 product, 0.7e-7; 3e3 and 1: 2.7e-5 and 1.1e-5). What still goes to the fp32 product: infinities and NaN, scores beyond 2^30, and walks whose
 // largest key leaves so little of the others that bits of their scores would be lost (from about 2^20 on). That takes three times as long as
 // the fp32 product's own kernel (S = 4096 1070 and 3370 us, B=8 H=16 S=300 47 and 159); until the pieces were relative, values of 1e3 took it too,
-// and normal ones up to 2 % less. us, the fp32 product and this kernel: B=1 H=32/8 S=4096 D=128 causal 1068 and 602, H=16 S=2048 177 and 129,
-// B=2 H=12 S=1023 D=112 115 and 75, B=8 H=16 S=300 D=128 causal 47.4 and 37.0. One tile of 64 keys is in LDS at a time; with K's next one beside it, and both split beside the MFMAs, it took 594 and 132 us, in another order
-// 634 and 133.
+// and normal ones up to 2 % less. us, the fp32 product and this kernel: B=1 H=32/8 S=4096 D=128 causal 1068 and 591, H=16 S=2048 177 and 128,
+// B=2 H=12 S=1023 D=112 115 and 69, B=8 H=16 S=300 D=128 causal 46.9 and 35.2. One tile of 64 keys
+// is in LDS at a time; with K's next one beside it, and both split beside the MFMAs, the first two took 594 and 132 us, in another order 634 and 133.
 #include <math.h>
 
 #include <algorithm>

@@ -103,8 +103,8 @@ __device__ inline void rotate_q_fragments_with_table(typename MT::vec8 (&qreg)[D
 // wave, a fetch, two products and a softmax per tile (0.46 us for a tile of 64 keys at head dim 64 in two key groups, where its MFMAs
 // take 0.1), so a tile is four or eight groups of 32 keys, and a wave walks a quarter or an eighth of the keys. 64 rows on eight waves,
 // at head dims up to 64 also 32 rows on four or, with tiles of 256 keys, on eight, which no CU holds more than once. The groups are
-// folded two by two. fp16, us in two groups and here: 1 x 2 heads 988 x 7818 D=128 97.9 and 73.1, B=6 H=1 S=1295 D=64 14.0 and 9.7, H=4
-// S=4066 D=40 causal 35.3 and 23.1, H=3 S=3910 D=64 causal 34.1 and 19.6, 24 x 7127 keys of 18 rows 59.8 and 28.3; bf16 H=8 S=3169 D=64
+// folded two by two. fp16, us in two groups and here: 1 x 2 heads 988 x 7818 D=128 97.6 and 72.1, B=6 H=1 S=1295 D=64 causal 14.1 and 10.3, H=4
+// S=4066 D=40 causal 35.4 and 23.5, H=3 S=3910 D=64 causal 33.9 and 19.8, 24 x 7127 keys of 18 rows 57.6 and 29.9; bf16 H=8 S=3169 D=64
 // causal 38.3 and 30.5. (32 rows on four waves at head dims 96 and 128: 0 to 25 % behind 64 rows on eight, one wave per SIMD.)
 // The second launch bound is waves per SIMD.
 // WPS: waves per SIMD the register budget is set for (3 x 4 waves, 2 x 8 waves or 1 x 8 waves per CU).
