@@ -537,18 +537,19 @@ SplitForm split_form(const DecodeArgs &a, int vec) {
   f.wide_keys = f.keys / kWaves * wide_waves(f.heads, vec);
   return f;
 }
-// Walks so short that one workgroup takes all of a unit's keys in less time than the merge launch adds: us with the partials and without, every
-// sequence Lmax long, fp32 B=2 Hkv=16 L=182 D=128 10.9 and 6.7, B=4 Hkv=12 L=242 10.5 and 7.3, L=460 D=64 32 heads of 2 9.0 and 7.1, fp16 B=20 Hkv=4 L=174 D=80 10.4
-// and 6.0, bf16 B=5 Hkv=20 L=529 9.7 and 8.7. A CU fetches 65 bytes a ns, so it ends where the wide workgroup has two and a half iterations of 64 or
-// 128 KB to walk, three and a half from half the CUs on (fp32 L=858 D=64 176 units 16.0 and 13.7); with two heads in 16 bits after two (fp16 B=2 12/6 heads
-// L=575 D=72 9.2 and 10.1, B=6 16/8 L=554 D=80 10.0 and 10.4), with four and more the arithmetic counts as well (fp32 B=12 32/8 heads L=535 D=128 17.4
-// and 23.6, B=4 64/8 L=256 D=96 19.2 and 19.5). More units than CUs go round in four waves: fp32 B=54 Hkv=8 L=152 D=64 13.1 and 7.1, fp16 B=21 64/32
-// heads L=183 D=80 16.9 and 10.4, fp32 B=11 Hkv=32 L=446 D=64 16.6 and 13.7. So do walks of up to three and a half iterations of four waves (bf16 B=3 24/12
-// heads L=83 D=80 5.3, on sixteen waves 6.4; fp32 B=9 48/12 heads L=117 D=128 10.2 and 8.5).
+// Walks so short that one workgroup takes all of a unit's keys in less time than the merge launch adds: us with the partials and without, every sequence Lmax
+// long, fp32 B=2 Hkv=16 L=182 D=128 10.9 and 6.7, B=4 Hkv=12 L=242 10.5 and 7.3, L=460 D=64 32 heads of 2 9.0 and 7.1, fp16 B=20 Hkv=4 L=174 D=80 10.4 and 6.0,
+// bf16 B=5 Hkv=20 L=529 9.7 and 8.7. A CU fetches 65 bytes a ns, so it ends where the wide workgroup has two and a half iterations of 64 or 128 KB to walk,
+// three and a half from half the CUs on (fp32 L=858 D=64 176 units 16.0 and 13.7); with two heads in 16 bits, short rows and up to a fifth of the CUs after two
+// (fp16 B=2 12/6 heads L=575 D=72 9.2 and 10.1, B=17 2/1 L=520 9.8 and 10.9; B=50 2/1 L=258 D=192 13.5 and 10.8), with four and more the arithmetic counts as
+// well (fp32 B=12 32/8 heads L=535 D=128 17.4 and 23.6, B=4 64/8 L=256 D=96 19.2 and 19.5). More units than CUs go round in four waves: fp32 B=54 Hkv=8 L=152
+// D=64 13.1 and 7.1, fp16 B=21 64/32 heads L=183 D=80 16.9 and 10.4, fp32 B=11 Hkv=32 L=446 D=64 16.6 and 13.7. So do walks of up to three and a half
+// iterations of four waves (bf16 B=3 24/12 heads L=83 D=80 5.3, on sixteen waves 6.4; fp32 B=9 48/12 heads L=117 D=128 10.2 and 8.5).
 bool one_split(const SplitForm &f, int Lmax, int vec, int64_t cus) {
   if (f.units > cus) return Lmax <= (f.heads <= 2 ? 448 : 256);
   if (f.heads * vec >= 32) return Lmax * 5 <= f.wide_keys * 6;
-  return f.heads > 2 || 2 * f.units < cus ? Lmax * 5 <= f.wide_keys * (f.heads == 2 && vec == 8 ? 10 : 12) : Lmax * 5 <= f.wide_keys * 17;
+  if (f.heads == 2 && vec == 8 && f.lanes <= 16 && 5 * f.units <= cus) return Lmax <= f.wide_keys * 2;
+  return f.heads > 2 || 2 * f.units < cus ? Lmax * 5 <= f.wide_keys * 12 : Lmax * 5 <= f.wide_keys * 17;
 }
 // Few units and long walks: a wide workgroup a CU, and with it fewer partials (bf16 B=2 Hkv=1 L=29834 D=80 25.4 -> 16.4 us, fp16 B=3 Hkv=2 L=18681 24.3 ->
 // 13.5, B=3 Hkv=4 L=24282 30.3 -> 19.8, fp32 B=2 8/4 heads L=11136 D=128 24.7 -> 20.8; 24 to 32 units come out even). 94 drawn ones of full length are

@@ -49,7 +49,8 @@ def plan(lm, dtype, B, Hq, Hkv, L, D, num_splits=0):
     ("bf16", 6, 24, 6, 75, 160, "lanes a key=32, heads=4, waves=4> splits=1"), ("f32", 40, 8, 8, 152, 64, "lanes a key=16, heads=1, waves=4> splits=1"),
     ("f32", 2, 12, 6, 151, 256, "lanes a key=64, heads=2, waves=16> splits=1"), ("f32", 7, 36, 3, 201, 32, "lanes a key=8, heads=8, waves=4> splits=1"),
     # two heads, longer than two iterations of sixteen waves: partials
-    ("f16", 2, 12, 6, 575, 72, "lanes a key=16, heads=2, waves=4> splits=5"), ("bf16", 6, 16, 8, 512, 80, "lanes a key=16, heads=2, waves=16> splits=1"),
+    ("f16", 2, 12, 6, 575, 72, "lanes a key=16, heads=2, waves=4> splits=5"), ("bf16", 8, 16, 8, 613, 72, "lanes a key=16, heads=2, waves=16> splits=1"),
+    ("f16", 50, 2, 1, 258, 192, "lanes a key=32, heads=2, waves=16> splits=1"),
     # few units: a wide workgroup a CU
     ("f16", 1, 4, 1, 30001, 112, "lanes a key=16, heads=4, waves=8> splits="), ("bf16", 3, 3, 1, 16385, 200, "lanes a key=32, heads=4, waves=8> splits="),
     ("bf16", 1, 2, 2, 29834, 80, "lanes a key=16, heads=1, waves=16> splits="), ("f32", 6, 1, 1, 11075, 64, "lanes a key=16, heads=1, waves=16> splits="),
