@@ -435,8 +435,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_f32_split_kernel(Deal deal
   // ---- values that pieces do not hold, anywhere in the workgroup: its rows again with the fp32 product ----
   // (up to here the lost bits of Q and K move a scaled score by less than 2^-37)
   // (two pieces: what Q and K lack of 2^-36 of 2^15 each, D times, moves one by less than 2^-22, or than half an fp32 unit of the row's
-  // largest score, which the sum of its products is rounded to anyway)
-  const bool held = HALF ? row_unit * half_down(key_exp) * (16.f * D) <= fmaxf(4.f, fabsf(m_i) - kLazyRescale) && unit > 0x1p-30f && unit < 0x1p30f
+  // largest score, which the sum of its products is rounded to anyway; below 2^-38 the units of small queries and keys would be subnormal)
+  const bool held = HALF ? row_unit * half_down(key_exp) * (16.f * D) <= fmaxf(4.f, fabsf(m_i) - kLazyRescale) && unit >= 0x1p-38f && unit < 0x1p100f
                          : fmaxf(top, 1.f) * a.scale <= 0x1p80f;
   float finite = 0.f;
 #pragma unroll

@@ -261,3 +261,21 @@ def test_plain_c_client_builds_against_the_public_header(tmp_path):
     res = subprocess.run([binary], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert "libluminal_hip version" in res.stdout, res.stdout
     assert res.returncode in (0, 77), res.stdout
+
+
+def test_decode_plan_validates_as_the_launch_does(lm):
+    """No room for the text, and what lmh_decode_attn refuses, come back as errors; nothing is launched."""
+    b = lm.binding
+    p = b.DecodeParams()
+    p.out = p.q = p.k_cache = p.v_cache = p.workspace = 4096
+    p.B, p.Hq, p.Hkv, p.Lmax, p.D, p.dtype, p.scale, p.workspace_bytes = 1, 8, 2, 4096, 128, b.DTYPE_CODES["bf16"], 0.1, 1 << 40
+    assert b.decode_plan(p).startswith("decode_mfma_kernel<bf16, D=128> splits=")
+    assert b.load().lmh_decode_plan(ctypes.byref(p), None, 0) == b.LMH_E_NULL
+    p.workspace_bytes = 16
+    with pytest.raises(lm.LuminalHipError) as e:
+        b.decode_plan(p)
+    assert e.value.code == b.LMH_E_WORKSPACE
+    p.D = 260
+    with pytest.raises(lm.LuminalHipError) as e:
+        b.decode_plan(p)
+    assert e.value.code == b.LMH_E_UNSUPPORTED

@@ -99,6 +99,18 @@ def test_magnitudes_stay_on_the_pieces(lm, hip, oracle, causal, D):
         np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("q_by,k_by", [(34, 0), (10, 24), (-20, -20), (-24, 0)])
+def test_scales_stay_on_the_pieces(lm, hip, oracle, q_by, k_by):
+    """The same with the power of two in the scale."""
+    q, k, v = inputs(oracle, (1, 40, 520, 128), (1, 8, 520, 128), "f32", 52550)
+    assert "prefill_f32_split_kernel" in plan(lm, q, k, "f32", False, False)
+    want = run(lm, hip, q, k, v, "f32", False)
+    dq, dk, dv = (lm.to_device(x, hip, "f32") for x in (q * np.float32(2.0 ** q_by), k * np.float32(2.0 ** k_by), v))
+    out = lm.HipArray(q.shape, "f32", hip)
+    lm.host.execute_op_inplace(out, lm.FlashAttentionOp(float(np.float32(lm.default_scale(128)) * np.float32(2.0 ** -(q_by + k_by))), False), dq, dk, dv)
+    np.testing.assert_array_equal(out.to_host(), want)
+
+
 @pytest.mark.parametrize("q_mul,k_mul", [(1e3, 1e-5), (1.0, 3e3), (2e3, 1.0), (300.0, 300.0)])
 def test_error_at_large_and_small_magnitudes(lm, hip, oracle, q_mul, k_mul):
     """No further from 64 bits than scores that one fp32 product after the other is added to (the softmax in 64 bits), with half as much again for
